@@ -203,6 +203,16 @@ int tgis_rmsnorm_residual(const void* x, const void* residual, const void* weigh
 int tgis_rmsnorm_residual_partial(const float* slabs, int num_slabs, int64_t slab_ld, const void* bias,
                                   const void* residual, const void* weight, void* y, int64_t ldy, void* res_out,
                                   int64_t rows, int64_t hidden, float eps, int dtype, void* stream);
+/* RMSNorm in front of an act-order int4 GEMM: y leaves gathered, y[m][k] = normed[m][perm[k]] (perm int32 [hidden]), so that the
+ * GEMM takes it like an operand of a matrix without act-order (perm = NULL).  The input is x, or (x NULL) split-K slabs (+ xbias). */
+int tgis_rmsnorm_residual_gather(const void* x, const float* slabs, int num_slabs, int64_t slab_ld, const void* xbias,
+                                 const void* residual, const void* weight, const int32_t* perm, void* y, int64_t ldy,
+                                 void* res_out, int64_t rows, int64_t hidden, float eps, int dtype, void* stream);
+/* out[m][k] = x[m][perm[k]] for a two-byte activation x [M, in_cols] (row stride ldx); perm int32 [K], entries outside
+ * [0, in_cols) give 0 (padded act-order row shards).  ldo: row stride of out (a multiple of 8), or TGIS_LD_FRAGMENTS
+ * (M <= 64, K % 64 == 0).  What an act-order int4 GEMM's operand is passed through when no norm in front of it can gather. */
+int tgis_gather_columns(const void* x, int64_t ldx, const int32_t* perm, void* out, int64_t ldo, int64_t M, int64_t in_cols,
+                        int64_t K, void* stream);
 int tgis_layernorm_residual(const void* x, const void* residual, const void* weight, const void* bias,
                             void* y, void* res_out, int64_t rows, int64_t hidden, float eps,
                             int dtype, void* stream);

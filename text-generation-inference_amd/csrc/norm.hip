@@ -31,10 +31,12 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
                                                   const T* __restrict__ weight, const T* __restrict__ bias,
                                                   T* y, T* res_out, int hidden,
                                                   float eps, const float* __restrict__ slabs, int S, int64_t slab_ld,
-                                                  const T* __restrict__ xbias, int y_frag) {
+                                                  const T* __restrict__ xbias, int y_frag,
+                                                  const int32_t* __restrict__ perm) {
     using V8 = typename VecT<T>::x8;
     constexpr int MAXV = MAX_HIDDEN / (NT * 8);
     __shared__ float sh[NT / 64];
+    extern __shared__ __attribute__((aligned(16))) unsigned char norm_row[];  // the normed row, only where perm is given
     const int64_t row = blockIdx.x;
     const T* xr = PARTIAL ? nullptr : x + row * hidden;
     const T* rr = residual ? residual + row * hidden : nullptr;
@@ -42,6 +44,12 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
     V8 wvs[MAXV], bvs[MAXV];  // weight / bias: asked for with the inputs, not after the row reductions
     const int nchunk = hidden >> 3;  // hidden % 8 == 0
     float s1 = 0.f, s2 = 0.f;
+    int src[8];  // where this thread's first gathered columns come from: asked for with the inputs too
+    const bool src_early = RMS && perm && (int)threadIdx.x < nchunk;
+    if (src_early) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) src[e] = perm[threadIdx.x * 8 + e];
+    }
 #pragma unroll
     for (int it = 0; it < MAXV; ++it) {
         int c = threadIdx.x + it * NT;
@@ -128,6 +136,29 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
                 for (int e = 0; e < 8; ++e) o[e] = from_f32<T>((v[it][e] - mean) * rstd * to_f32(wv[e]));
             }
             // y_frag (RMSNorm in front of an int4 decode GEMM): 32-row fragment order, xf_off in common.h
+            if (RMS && perm)
+                st16(reinterpret_cast<T*>(norm_row) + c * 8, o);
+            else
+                st16(y + (y_frag ? xf_off(row, c * 8, hidden) : row * hidden + c * 8), o);
+        }
+    }
+    // perm (in front of an act-order int4 GEMM): the normed row leaves gathered, y[k] = row[perm[k]].  The row goes through LDS: a
+    // two-byte read per element at a random place is a few cycles per wave there (11 x 4096: 4.8 us with and without; 6.2 us when
+    // the indices were only asked for after the reductions).
+    if (RMS && perm) {
+        __syncthreads();
+        const T* nr = reinterpret_cast<const T*>(norm_row);
+        for (int c = threadIdx.x; c < nchunk; c += NT) {
+            if (c >= NT) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) src[e] = perm[c * 8 + e];
+            }
+            V8 o;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool in = (unsigned)src[e] < (unsigned)hidden;
+                o[e] = in ? nr[in ? src[e] : 0] : (T)0.f;
+            }
             st16(y + (y_frag ? xf_off(row, c * 8, hidden) : row * hidden + c * 8), o);
         }
     }
@@ -137,7 +168,7 @@ template <bool RMS>
 static int launch_norm(const void* x, const void* residual, const void* weight, const void* bias, void* y,
                        void* res_out, int64_t rows, int64_t hidden, float eps, int dtype, void* stream,
                        const float* slabs = nullptr, int S = 0, int64_t slab_ld = 0, const void* xbias = nullptr,
-                       int64_t ldy = 0) {
+                       int64_t ldy = 0, const int32_t* perm = nullptr) {
     TGIS_CHECK_ARG((x || slabs) && weight && y, "norm: null tensor");
     TGIS_CHECK_ARG(!slabs || (S >= 1 && slab_ld >= hidden && slab_ld % 4 == 0),
                    "norm: partial input needs a slab row stride >= hidden");
@@ -152,16 +183,17 @@ static int launch_norm(const void* x, const void* residual, const void* weight, 
     hipStream_t st = (hipStream_t)stream;
     TgisTimedScope timed(TGIS_OP_NORM, st);
     const bool wide = rows <= 64 && hidden >= 2048;
+    const size_t lds = perm ? (size_t)hidden * 2 : 0;
 #define TGIS_NORM_LAUNCH(T, P)                                                                                   \
     do {                                                                                                         \
         if (wide)                                                                                                \
-            hipLaunchKernelGGL((norm_kernel<T, RMS, P, 512>), dim3((unsigned)rows), dim3(512), 0, st, (const T*)x, \
+            hipLaunchKernelGGL((norm_kernel<T, RMS, P, 512>), dim3((unsigned)rows), dim3(512), lds, st, (const T*)x, \
                                (const T*)residual, (const T*)weight, (const T*)bias, (T*)y, (T*)res_out,         \
-                               (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag);                    \
+                               (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag, perm);                    \
         else                                                                                                     \
-            hipLaunchKernelGGL((norm_kernel<T, RMS, P, 256>), dim3((unsigned)rows), dim3(256), 0, st, (const T*)x, \
+            hipLaunchKernelGGL((norm_kernel<T, RMS, P, 256>), dim3((unsigned)rows), dim3(256), lds, st, (const T*)x, \
                                (const T*)residual, (const T*)weight, (const T*)bias, (T*)y, (T*)res_out,         \
-                               (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag);                    \
+                               (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag, perm);                    \
     } while (0)
     if (dtype == TGIS_F16) {
         if (slabs) TGIS_NORM_LAUNCH(f16, true); else TGIS_NORM_LAUNCH(f16, false);
@@ -188,6 +220,15 @@ extern "C" int tgis_rmsnorm_residual_partial(const float* slabs, int num_slabs, 
     TGIS_CHECK_ARG(slabs, "tgis_rmsnorm_residual_partial: null slabs");
     return launch_norm<true>(nullptr, residual, weight, nullptr, y, res_out, rows, hidden, eps, dtype, stream, slabs,
                              num_slabs, slab_ld, bias, ldy);
+}
+
+extern "C" int tgis_rmsnorm_residual_gather(const void* x, const float* slabs, int num_slabs, int64_t slab_ld, const void* xbias,
+                                            const void* residual, const void* weight, const int32_t* perm, void* y, int64_t ldy,
+                                            void* res_out, int64_t rows, int64_t hidden, float eps, int dtype, void* stream) {
+    TGIS_CHECK_ARG(perm, "tgis_rmsnorm_residual_gather: null permutation");
+    TGIS_CHECK_ARG(!x != !slabs, "tgis_rmsnorm_residual_gather: the input is either a tensor or split-K slabs");
+    return launch_norm<true>(x, residual, weight, nullptr, y, res_out, rows, hidden, eps, dtype, stream, slabs, num_slabs, slab_ld,
+                             xbias, ldy, perm);
 }
 
 extern "C" int tgis_layernorm_residual_partial(const float* slabs, int num_slabs, int64_t slab_ld, const void* xbias,

@@ -84,10 +84,11 @@ class KVArgs:
 # measured slower than the launches they replace: experiments/README.md is their ledger.)
 
 
-def frag_rows(linear, rows: int, kv: "KVArgs", act: int = 0) -> bool:
-    """Decode step of <= 64 rows in front of an int4 linear that takes its operand in fragment order (native.FragAct)."""
+def frag_rows(linear, rows: int, kv: "KVArgs", act: int = 0, gathers: bool = False) -> bool:
+    """Decode step of <= 64 rows in front of an int4 linear that takes its operand in fragment order (native.FragAct); gathers: the
+    producer can write an act-order matrix's column order."""
     return (kv.max_q_len == 1 and not kv.fresh_prefill and rows <= 64 and hasattr(linear, "wants_fragments")
-            and linear.wants_fragments(rows, act))
+            and linear.wants_fragments(rows, act, gathers))
 
 
 class LlamaRMSNorm:
@@ -95,9 +96,12 @@ class LlamaRMSNorm:
         self.weight = weights.get_tensor(f"{prefix}.weight").contiguous()
         self.variance_epsilon = eps
 
-    def forward(self, hidden_states, residual=None, frag: bool = False):
+    def forward(self, hidden_states, residual=None, frag: bool = False, perm=None):
         # returns (normed, res) like the reference; res is hidden_states itself when residual is None
-        # frag: the normed activation leaves in fragment order (native.FragAct) for the int4 GEMM behind it
+        # frag: the normed activation leaves in fragment order (native.FragAct) for the int4 GEMM behind it; perm: its columns
+        # leave in that (act-order) GEMM's order
+        if perm is not None:
+            return native.rmsnorm_residual(hidden_states, residual, self.weight, self.variance_epsilon, frag=frag, perm=perm)
         return native.rmsnorm_residual(hidden_states, residual, self.weight, self.variance_epsilon, frag=frag)
 
     __call__ = forward
@@ -145,21 +149,22 @@ class FlashLlamaAttention:
         if hasattr(self.query_key_value.linear, "rope_heads"):
             self.query_key_value.linear.rope_heads = (self.num_heads, self.num_key_value_heads, self.head_size)
 
-    def project_qkv(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs):
-        """qkv GEMM, rotation of q and k in place, k and v scattered to their page slots (reference :251-268,282)."""
+    def project_qkv(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False):
+        """qkv GEMM, rotation of q and k in place, k and v scattered to their page slots (reference :251-268,282).
+        gathered: hidden_states' columns are in the order of an act-order qkv weight."""
         H, Hkv, D = self.num_heads, self.num_key_value_heads, self.head_size
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         lin = self.query_key_value.linear
         rope_w = getattr(lin, "rope_handle", None)
         if isinstance(hidden_states, native.FragAct) or (
                 rope_w is not None and kv.slots is not None and not kv.fresh_prefill and kv.max_q_len == 1
-                and hidden_states.shape[0] <= 64 and cos.shape[1] * 2 == D
+                and (gathered or getattr(lin, "perm", None) is None) and hidden_states.shape[0] <= 64 and cos.shape[1] * 2 == D
                 and native.rope_gemm_ok(hidden_states.shape[0], rope_w, D)):
             # one launch: GEMM + rotary embedding + cache write (native.gptq_gemm_rope / native.dense_gemm_rope)
             fused = native.gptq_gemm_rope if isinstance(rope_w, native.GptqWeight) else native.dense_gemm_rope
             return fused(hidden_states, rope_w, lin.bias, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D)
         # [T, (H + 2 Hkv) D]; at decode sizes the split-K sum of the GPTQ GEMM is finished inside the rope kernel
-        qkv = self.query_key_value(hidden_states, partial=True)
+        qkv = self.query_key_value(hidden_states, partial=True, **({"gathered": True} if gathered else {}))
         if kv.fresh_prefill and not isinstance(qkv, native.Partial):
             return native.rope_kv_write_prefill(qkv, cos, sin, position_ids, cu_seqlens_q, kv.block_tables, k_pool, v_pool,
                                                 kv.max_q_len, H, Hkv, D, D)
@@ -184,8 +189,8 @@ class FlashLlamaAttention:
                           attn_output, B, H, Hkv, D, kv.max_q_len, kv.max_ctx, self.softmax_scale, kv.num_splits, ws)
         return attn_output
 
-    def forward(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs):
-        qkv = self.project_qkv(hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id, kv)
+    def forward(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False):
+        qkv = self.project_qkv(hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id, kv, gathered)
         attn_output = self.attend(qkv, cu_seqlens_q, layer_id, kv)
         # may be a native.Partial: the following fused add+RMSNorm finishes the split-K sum
         return self.o_proj(attn_output, partial=True)
@@ -209,15 +214,28 @@ class LlamaMLP:
         if self.fused_epilogue:
             self.gate_up_proj.linear.gate_up = True
 
-    def forward(self, hidden_states):
+    def post_init(self):
+        """An act-order down projection wants its operand's columns in its own order: the gate and up columns that produce
+        them are re-ordered once, and nothing is gathered per step."""
+        down, gate_up = self.down_proj.linear, self.gate_up_proj.linear
+        if not self.fused_epilogue or not hasattr(down, "order_columns") or not hasattr(gate_up, "order_columns"):
+            return
+        if gate_up.q_handle is None and down.perm is not None and down.height == self.intermediate_size:
+            order = down.perm
+            if bool((order >= 0).all()):
+                gate_up.order_columns(torch.cat([order, order + self.intermediate_size]))
+                down.take_ordered_input()
+
+    def forward(self, hidden_states, gathered: bool = False):
+        kw = {"gathered": True} if gathered else {}
         if self.fused_epilogue:
             if isinstance(hidden_states, native.FragAct):  # decode: SiLU * up leaves in the layout down_proj reads
                 rows = hidden_states.shape[0]
                 act = self.gate_up_proj(hidden_states, out_frag=self.down_proj.linear.wants_fragments(rows))
                 return self.down_proj(act, partial=True)
-            act = self.gate_up_proj(hidden_states)  # [T, I], already silu(gate) * up
+            act = self.gate_up_proj(hidden_states, **kw)  # [T, I], already silu(gate) * up
             return self.down_proj(act, partial=True)
-        gate_up_states = self.gate_up_proj(hidden_states)  # [T, 2, I]
+        gate_up_states = self.gate_up_proj(hidden_states, **kw)  # [T, 2, I]
         return self.down_proj(gate_up_states, act=1, partial=True)
 
     __call__ = forward
@@ -237,15 +255,17 @@ class FlashLlamaLayer:
     def forward(self, hidden_states, residual, cos, sin, position_ids, cu_seqlens_q, kv: KVArgs):
         rows = hidden_states.shape[0]
         att = self.self_attn
-        # decode steps of <= 32 rows hand the int4 GEMMs their operands in fragment order (native.FragAct): the qkv + rotary
-        # launch when it serves the step, the MLP when the SiLU * up epilogue does
+        # decode steps of <= 64 rows hand the int4 GEMMs their operands in fragment order (native.FragAct): the qkv + rotary
+        # launch when it serves the step, the MLP when the SiLU * up epilogue does; the norms gather for act-order weights
+        qkv_perm = getattr(att.query_key_value.linear, "perm", None)
         qkv_frag = (kv.slots is not None and cos.shape[1] * 2 == att.head_size
-                    and frag_rows(att.query_key_value.linear, rows, kv, act=3))
-        normed_hidden_states, res = self.input_layernorm(hidden_states, residual, frag=qkv_frag)
-        attn_output = att(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv)
-        mlp_frag = self.mlp.fused_epilogue and frag_rows(self.mlp.gate_up_proj.linear, rows, kv, act=2)
-        normed_attn_res_output, attn_res = self.post_attention_layernorm(attn_output, res, frag=mlp_frag)
-        mlp_output = self.mlp(normed_attn_res_output)
+                    and frag_rows(att.query_key_value.linear, rows, kv, act=3, gathers=True))
+        normed_hidden_states, res = self.input_layernorm(hidden_states, residual, frag=qkv_frag, perm=qkv_perm)
+        attn_output = att(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv, qkv_perm is not None)
+        mlp_perm = getattr(self.mlp.gate_up_proj.linear, "perm", None)
+        mlp_frag = self.mlp.fused_epilogue and frag_rows(self.mlp.gate_up_proj.linear, rows, kv, act=2, gathers=True)
+        normed_attn_res_output, attn_res = self.post_attention_layernorm(attn_output, res, frag=mlp_frag, perm=mlp_perm)
+        mlp_output = self.mlp(normed_attn_res_output, mlp_perm is not None)
         return mlp_output, attn_res
 
     __call__ = forward
@@ -301,6 +321,8 @@ class FlashLlamaForCausalLM:
 
     def post_init(self):
         """Repack every GPTQ linear for the kernels (the reference does this in serve(), server.py:334-358)."""
+        for layer in self.model.layers:
+            layer.mlp.post_init()
         for lin in self.gptq_linears:
             if lin.q_handle is None:
                 lin.post_init()

@@ -6,6 +6,7 @@ utils/layers.py:361,403-404, utils/gptq/exllamav2.py:7) this module loads one C-
 passes raw device pointers, sizes and the current HIP stream.  There is no CPU or eager-torch fallback:
 if the library is missing or a call fails, an exception is raised.
 """
+import copy
 import ctypes
 import os
 from typing import Optional
@@ -66,6 +67,9 @@ SIGNATURES = {
     "tgis_rmsnorm_residual": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_f, _c_int, _vp]),
     "tgis_rmsnorm_residual_partial": (_c_int, [_vp, _c_int, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_f,
                                                _c_int, _vp]),
+    "tgis_rmsnorm_residual_gather": (_c_int, [_vp, _vp, _c_int, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_f,
+                                              _c_int, _vp]),
+    "tgis_gather_columns": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_layernorm_residual": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_f, _c_int, _vp]),
     "tgis_layernorm_residual_partial": (_c_int, [_vp, _c_int, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64,
                                                  _c_f, _c_int, _vp]),
@@ -401,6 +405,14 @@ class GptqWeight:
             self.perm = explicit.to(dev, torch.int32).contiguous()
         torch.cuda.current_stream().synchronize()  # qweight/qzeros/scales may be freed by the caller
 
+    def in_order(self) -> "GptqWeight":
+        """The same image for operands whose columns are gathered with `perm` already (gather_columns, rmsnorm_residual)."""
+        if self.perm is None:
+            return self
+        w = copy.copy(self)
+        w.perm, w.in_features, w.partial_plan = None, self.K, {}
+        return w
+
     def workspace_bytes(self, M: int) -> int:
         return load_library().tgis_gptq_gemm_workspace_bytes(M, self.K, self.N)
 
@@ -443,6 +455,22 @@ def gptq_gemm(x, w: GptqWeight, ws: Workspace, bias=None, act: int = 0, out=None
                                           out.stride(0), M, w.K, w.N, w.groups, act, ws.ptr, ws.nbytes, _stream()),
         "tgis_gptq_gemm_f16")
     return out
+
+
+def gather_columns(x: torch.Tensor, perm: torch.Tensor, frag: bool = False):
+    """x[:, perm] of a two-byte activation, zeros where perm is outside x; frag (rows <= 64, f16): as a FragAct."""
+    assert x.dim() == 2 and x.stride(1) == 1 and x.element_size() == 2
+    assert perm.dtype == torch.int32 and perm.is_contiguous()
+    M, K = x.shape[0], perm.numel()
+    if frag:
+        res = FragAct.empty(M, K, x.device)
+        optr, ldo = _ptr(res.buf), LD_FRAGMENTS
+    else:
+        res = torch.empty((M, K), dtype=x.dtype, device=x.device)
+        optr, ldo = _ptr(res), K
+    _check(load_library().tgis_gather_columns(_ptr(x), x.stride(0) if M > 1 else x.shape[1], _ptr(perm), optr, ldo, M, x.shape[1], K,
+                                              _stream()), "tgis_gather_columns")
+    return res
 
 
 class Partial:
@@ -628,9 +656,10 @@ def clear_error() -> None:
 
 
 # ---- norms --------------------------------------------------------------------------------------------
-def rmsnorm_residual(x, residual, weight, eps: float, y=None, res_out=None, frag: bool = False):
+def rmsnorm_residual(x, residual, weight, eps: float, y=None, res_out=None, frag: bool = False, perm=None):
     """(y, res) = fused add + RMSNorm; mirrors LlamaRMSNorm.forward (flash_llama_modeling.py:113-152).
-    frag (rows <= 32, f16): y is returned as a FragAct, the layout the int4 GEMM behind the norm reads."""
+    frag (rows <= 32, f16): y is returned as a FragAct, the layout the int4 GEMM behind the norm reads.
+    perm (int32 [hidden]): y's columns leave gathered with it, as the act-order int4 GEMM behind the norm wants them."""
     rows, hidden = x.shape
     yf = None
     if frag:
@@ -639,6 +668,21 @@ def rmsnorm_residual(x, residual, weight, eps: float, y=None, res_out=None, frag
         y, ldy = yf.buf, LD_FRAGMENTS
     else:
         ldy = hidden
+    if perm is not None:
+        assert perm.dtype == torch.int32 and perm.numel() == hidden and perm.is_contiguous()
+        part = isinstance(x, Partial)
+        assert part or (x.dim() == 2 and x.is_contiguous())
+        if y is None:
+            y = torch.empty((rows, hidden), dtype=x.dtype, device=x.device)
+        if res_out is None:
+            res_out = x if residual is None and not part else torch.empty((rows, hidden), dtype=x.dtype, device=x.device)
+        _check(
+            load_library().tgis_rmsnorm_residual_gather(
+                None if part else _ptr(x), _ptr(x.slabs) if part else None, x.S if part else 0, x.ld if part else 0,
+                _ptr(x.bias) if part else None, _ptr(residual), _ptr(weight), _ptr(perm), _ptr(y), ldy,
+                _ptr(res_out) if res_out is not x else None, rows, hidden, float(eps), dtype_code(x.dtype), _stream()),
+            "tgis_rmsnorm_residual_gather")
+        return (yf if frag else y), res_out
     if isinstance(x, Partial):
         if y is None:
             y = torch.empty((rows, hidden), dtype=x.dtype, device=x.device)

@@ -152,17 +152,48 @@ class Ex4bitLinearV2:
         # native.gptq_gemm_rope, the decode launch that rotates q / k and writes the cache in its epilogue
         self.rope_heads = None
         self.rope_handle: Optional[native.GptqWeight] = None
+        self._perm: Optional[torch.Tensor] = None  # see `perm`
         self._fused = {}  # act -> rows up to which the library's fused kernels are used
 
     def post_init(self):
-        self.q_handle = native.GptqWeight(self.qweight, self.qzeros, self.scales, self.g_idx, self.bits,
-                                          self.groupsize, gate_up=self.gate_up)
+        handle = native.GptqWeight(self.qweight, self.qzeros, self.scales, self.g_idx, self.bits, self.groupsize,
+                                   gate_up=self.gate_up)
+        # act-order: the operand is gathered once, in front of the GEMM, and every kernel takes the matrix as if it had no
+        # act-order (7B, 11 rows: the four GEMMs of a layer and the rotary launch 163 us when the GEMMs gather while they stage their operand,
+        # 48 us with one gather launch in front of o_proj and the norms gathering for qkv and gate_up)
+        self._perm = handle.perm
+        self.q_handle = handle if handle.perm is None else handle.in_order()
         if self.rope_heads is not None and FUSED_ROPE_GEMM:
             H, Hkv, D = self.rope_heads
-            if self.q_handle.perm is None and any(native.gptq_rope_ok(m, self.q_handle, D) for m in (1, 32, 64)):
-                self.rope_handle = native.GptqWeight(self.qweight, self.qzeros, self.scales, None, self.bits,
-                                                     self.groupsize, rope=(D, H + Hkv))
+            if any(native.gptq_rope_ok(m, self.q_handle, D) for m in (1, 32, 64)):
+                rope = native.GptqWeight(self.qweight, self.qzeros, self.scales, self.g_idx if self._perm is not None else None,
+                                         self.bits, self.groupsize, rope=(D, H + Hkv))
+                self.rope_handle = rope if rope.perm is None else rope.in_order()
         self.qweight = self.qzeros = self.scales = None  # the prepared image replaces them
+
+    @property
+    def perm(self) -> Optional[torch.Tensor]:
+        """Columns of the activation in the order the image wants them (int32, -1 = a zero column), None = as they are.  A
+        producer that can gather (native.rmsnorm_residual) passes `gathered=True` on to forward."""
+        if self.q_handle is None:
+            self.post_init()
+        return self._perm
+
+    def order_columns(self, order: torch.Tensor):
+        """Before post_init: re-order the output columns, y[:, i] = old y[:, order[i]]."""
+        assert self.q_handle is None
+        order = order.to(self.device).long()
+        self.qweight = self.qweight.index_select(1, order)
+        self.scales = self.scales.index_select(1, order)
+        shifts = 4 * torch.arange(8, dtype=torch.int32, device=self.device)
+        zeros = ((self.qzeros[:, :, None] >> shifts) & 15).view(self.qzeros.shape[0], -1).index_select(1, order)
+        self.qzeros = (zeros.view(self.qzeros.shape[0], -1, 8) << shifts).sum(-1, dtype=torch.int32)
+        if self.bias is not None:
+            self.bias = self.bias.index_select(0, order)
+
+    def take_ordered_input(self):
+        """From now on the activation arrives in the image's order (its producer's columns were re-ordered to match)."""
+        self._perm = None
 
     def _fused_rows(self, act: int) -> int:
         got = self._fused.get(act)
@@ -179,21 +210,27 @@ class Ex4bitLinearV2:
                                                              device=self.device)
         return buf
 
-    def wants_fragments(self, rows: int, act: int = 0) -> bool:
+    def wants_fragments(self, rows: int, act: int = 0, gathers: bool = False) -> bool:
         """Should the producer of this linear's operand write it in fragment order (native.FragAct) for `rows` decode
-        rows?  act: 0 plain / partial, 2 the SiLU * up image, 3 the rope image (the fused qkv + rotary launch)."""
-        if self.q_handle is None:
-            self.post_init()
+        rows?  act: 0 plain / partial, 2 the SiLU * up image, 3 the rope image (the fused qkv + rotary launch).  An act-order
+        matrix asks for it only of a producer that can gather the columns (`gathers`)."""
+        if self.perm is not None and not gathers:
+            return False
         if act == 2 and not self.gate_up:
             act = 0
         w = self.rope_handle if act == 3 else self.q_handle
         return w is not None and rows <= 64 and native.gptq_fragments_ok(rows, w, act)
 
-    def forward(self, x, act: int = 0, partial: bool = False, out_frag: bool = False):
+    def forward(self, x, act: int = 0, partial: bool = False, out_frag: bool = False, gathered: bool = False):
         """partial=True (decode-sized M only): return native.Partial — the consumer kernel finishes the split-K sum.
-        x may be a native.FragAct (decode, <= 32 rows; see wants_fragments); out_frag: the SiLU * up output leaves as one."""
-        if self.q_handle is None:
-            self.post_init()
+        x may be a native.FragAct (decode, <= 64 rows; see wants_fragments); out_frag: the SiLU * up output leaves as one.
+        gathered: x is in the order of `perm` already (a FragAct always is)."""
+        if self.perm is not None and not gathered and not isinstance(x, native.FragAct):
+            if act:
+                x, act = native.act_mul(x, self.height), 0
+            rows = x.shape[0]
+            x = native.gather_columns(x, self._perm, frag=1 <= rows <= 64 and native.gptq_fragments_ok(
+                rows, self.q_handle, 2 if self.gate_up else 0))
         if isinstance(x, native.FragAct):
             if self.gate_up:
                 return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias, act=2, out_frag=out_frag)
@@ -215,13 +252,7 @@ class Ex4bitLinearV2:
         return self._large_m(x)
 
     def _large_m(self, x: torch.Tensor) -> torch.Tensor:
-        """prefill-sized M: dequantise once into scratch, then a library GEMM (exllamav2.py:87 "M > 50")."""
-        if self.q_handle.perm is not None:
-            perm = self.q_handle.perm.long()
-            if self.q_handle.in_features != self.q_handle.K:  # padded shard: index -1 reads a zero column
-                x = torch.nn.functional.pad(x, (0, 1))
-                perm = torch.where(perm < 0, torch.full_like(perm, x.shape[1] - 1), perm)
-            x = x.index_select(1, perm)
+        """prefill-sized M: dequantise once into scratch, then a library GEMM (exllamav2.py:87 "M > 50"); x in image order."""
         w = self._dequant_scratch()
         native._check(native.load_library().tgis_gptq_dequant_f16(
             self.q_handle.image.data_ptr(), w.data_ptr(), self.height, self.width, self.q_handle.groups,
