@@ -1,0 +1,80 @@
+"""-m gpu: the recurrence of csrc/wkv.hip in chunks of 16 tokens and token by token, against its definition in float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def definition(r, k, v, gate, logw, u, gain, S, eps):
+    """One sequence: r, k, v, gate, logw [T, H, d], u [H, d], gain [H, d], S [H, d, d] -> (out [T, H, d], S)."""
+    out = torch.empty_like(v)
+    for t in range(r.shape[0]):
+        kv = k[t][:, :, None] * v[t][:, None, :]
+        o = torch.einsum("hi,hij->hj", r[t], S + u[:, :, None] * kv)
+        S = logw[t].exp()[:, :, None] * S + kv
+        out[t] = o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * gain * torch.nn.functional.silu(gate[t])
+    return out, S
+
+
+# dims: every template width, padded ones, one that is not a multiple of 4; pad: rows that are not aligned groups of four
+@pytest.mark.parametrize("d,pad", [(64, 0), (64, 2), (32, 0), (8, 0), (48, 0), (128, 0), (100, 0), (18, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scan_in_chunks(gpu_device, d, pad, dtype):
+    from tgis_amd import native
+
+    H, W, eps = 3, 40, 1e-4
+    lens = [1, 4, 5, 16, 17, 31, 48, 50]  # both ways of walking, whole and ragged chunks
+    fresh = [i % 3 == 0 for i in range(len(lens))]
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(d)
+    r, k, v, gate = ((torch.randn(T, H, d, generator=g) * s).to(dtype) for s in (0.5, 0.5, 1.0, 1.0))
+    # decays near one, ordinary, and so strong that their products underflow
+    logw = -torch.exp(torch.randn(T, H, d, generator=g) * 1.5 - 1.0)
+    logw[torch.rand(T, H, d, generator=g) < 0.05] = -60.0
+    u, gain = torch.randn(H, d, generator=g) * 0.3, torch.rand(H, d, generator=g) + 0.5
+    state = torch.randn(B + 1, H, d, d, generator=g)
+    h, shift = torch.randn(T, W, generator=g), torch.zeros(B + 1, W)
+    slots = torch.randperm(B, generator=g).to(torch.int32)
+    cu = torch.tensor([0] + lens).cumsum(0)
+    pos = torch.cat([torch.arange(n) + (0 if f else 7) for n, f in zip(lens, fresh)]).to(torch.int32)
+    dev = lambda t: t.to(gpu_device)
+    rows = lambda t: torch.nn.functional.pad(t.reshape(T, H * d), (0, pad)).to(gpu_device)[:, :H * d]
+    st, sh = dev(state).clone(), dev(shift)
+    got = native.wkv_scan(rows(r), rows(k), rows(v), rows(gate), dev(logw.reshape(T, -1)), dev(u.reshape(-1)), dev(gain.reshape(-1)),
+                          st, sh, dev(h), dev(slots), dev(cu.to(torch.int32)), dev(pos), H, d, eps).double().cpu().view(T, H, d)
+    for b, (n, f) in enumerate(zip(lens, fresh)):
+        a, e = int(cu[b]), int(cu[b + 1])
+        S0 = torch.zeros(H, d, d, dtype=torch.float64) if f else state[int(slots[b])].double()
+        want, S = definition(*(t[a:e].double() for t in (r, k, v, gate, logw)), u.double(), gain.double(), S0, eps)
+        # fp32 sums of up to d + 16 terms of either sign and products of up to 16 decays: some tens of roundings (2e-7 each at the
+        # most, relative to the row's size), and exp's own error; two-byte outputs add their rounding (2 ** -9 of the value)
+        size = want.square().mean(-1, keepdim=True).sqrt()
+        tol = 2e-5 * size + (0.0 if dtype == torch.float32 else 2.0 ** -8 * want.abs())
+        assert ((got[a:e] - want).abs() <= tol).all(), (n, float(((got[a:e] - want).abs() / size).max()))
+        got_S = st[int(slots[b])].double().cpu()
+        assert (got_S - S).abs().max() <= 1e-5 * S.abs().max(), n
+        assert torch.equal(sh[int(slots[b])].cpu(), h[e - 1])
+    assert torch.equal(st[B].cpu(), state[B])
+
+
+@pytest.mark.parametrize("W", [40, 1024, 1030])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_token_shift_and_decay(gpu_device, W, dtype):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(W)
+    lens, T = [1, 1100], 1101
+    h, shift, mu = torch.randn(T, W, generator=g), torch.randn(3, W, generator=g), torch.rand(5, W, generator=g)
+    pos = torch.cat([torch.tensor([9]), torch.arange(1100)]).to(torch.int32)
+    dev = lambda t: t.to(gpu_device)
+    got = native.token_shift_mix(dev(h), dev(shift), dev(torch.tensor([2, 0], dtype=torch.int32)),
+                                 dev(torch.tensor([0, 1, T], dtype=torch.int32)), dev(pos), dev(mu), dtype).cpu()
+    before = torch.cat([shift[2:3], torch.zeros(1, W), h[1:-1]])
+    want = h[None] + (before - h)[None] * mu[:, None]
+    tol = 1e-6 if dtype == torch.float32 else 2.0 ** -10
+    assert ((got.float() - want).abs() <= tol * (1 + want.abs())).all()
+    for T2 in (3, 1024, 1101):  # single tokens, whole and ragged groups of tokens per workgroup
+        a, w2t, w0 = torch.randn(T2, 24, generator=g).to(dtype), torch.randn(24, W, generator=g) * 0.2, torch.randn(W, generator=g)
+        lw = native.wkv_decay(dev(a), dev(w2t), dev(w0)).cpu().double()
+        z = w0.double() + torch.tanh(a.double()) @ w2t.double()
+        assert ((lw + z.exp()).abs() <= 1e-5 * (1 + z.exp())).all()

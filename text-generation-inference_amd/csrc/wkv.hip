@@ -6,6 +6,8 @@
 // State per slot: S[head][key channel][value channel] (fp32) and the last token's mixer input (fp32).  A sequence whose
 // step starts at position 0 starts from zeros whatever its slot held before: slots need no clearing when they change hands.
 #include "common.h"
+#include <type_traits>
+#include "wave_dpp.h"
 
 namespace {
 
@@ -20,40 +22,65 @@ __device__ __forceinline__ int seq_of_token(const int32_t* __restrict__ cu_q, in
     return lo;
 }
 
-// one workgroup per token; out[s][t][c], s < NM
-template <typename T>
+// grid (token, block of 256 x VEC columns); out[s][t][c], s < NM.  Bound by its writes (one fp32 row in, NM two-byte rows out): VEC 4
+// stores 8 or 16 bytes per thread (4096 x 2048, five mixes: 47 -> 29 us), 1 is for widths that are not multiples of 4.
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void token_shift_mix_kernel(const float* __restrict__ h, const float* __restrict__ shift_state,
                                                               const int32_t* __restrict__ state_slots, const int32_t* __restrict__ cu_q,
                                                               const int32_t* __restrict__ positions, int B, const float* __restrict__ mu,
                                                               int NM, T* __restrict__ out, int64_t Ttot, int64_t W) {
+    typedef float F __attribute__((ext_vector_type(VEC)));
+    typedef T TV __attribute__((ext_vector_type(VEC)));
     const int t = blockIdx.x;
+    const int64_t c = ((int64_t)blockIdx.y * blockDim.x + threadIdx.x) * VEC;
+    if (c >= W) return;
     const int b = seq_of_token(cu_q, B, t);
     const bool first = t == cu_q[b];
     const bool fresh = first && positions[t] == 0;
     const float* prev = first ? shift_state + (int64_t)state_slots[b] * W : h + (int64_t)(t - 1) * W;
-    const float* cur = h + (int64_t)t * W;
-    // grid (token, 256-column block): one element per thread, so that a decode step's few tokens still fill the chip
-    const int64_t c = (int64_t)blockIdx.y * blockDim.x + threadIdx.x;
-    if (c >= W) return;
-    const float x = cur[c];
-    const float d = (fresh ? 0.f : prev[c]) - x;
-    for (int s = 0; s < NM; ++s) out[((int64_t)s * Ttot + t) * W + c] = (T)(x + d * mu[(int64_t)s * W + c]);
+    const F x = *reinterpret_cast<const F*>(h + (int64_t)t * W + c);
+    F d = *reinterpret_cast<const F*>(prev + c);
+    if (fresh) d = F(0.f);
+    d -= x;
+    for (int s = 0; s < NM; ++s) {
+        const F m = x + d * *reinterpret_cast<const F*>(mu + (int64_t)s * W + c);
+        TV o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o[e] = (T)m[e];
+        *reinterpret_cast<TV*>(out + ((int64_t)s * Ttot + t) * W + c) = o;
+    }
 }
 
-// grid (token, 256-channel block): logw[t][c] = -exp(w0[c] + sum_r tanh(a[t][r]) * w2t[r][c])
-template <typename T>
+// grid (TB tokens, 256-channel block): logw[t][c] = -exp(w0[c] + sum_r tanh(a[t][r]) * w2t[r][c])
+// TB tokens share a read of w2t's columns: with one token per workgroup a 4 x 1024-token step reads the 512 KiB matrix 4096 times from
+// L2 (rank 64, 4096 x 2048: 79 -> 39 us).  TB 8 from 1024 tokens on; below, single tokens keep the chip filled.
+template <typename T, int TB>
 __global__ __launch_bounds__(256) void wkv_decay_kernel(const T* __restrict__ a, int64_t ld_a, const float* __restrict__ w2t,
-                                                        const float* __restrict__ w0, float* __restrict__ logw, int R, int64_t C) {
-    extern __shared__ float th[];
-    const int64_t t = blockIdx.x;
-    for (int r = threadIdx.x; r < R; r += blockDim.x) th[r] = tanhf(ldf(a + t * ld_a + r));
+                                                        const float* __restrict__ w0, float* __restrict__ logw, int R, int64_t C,
+                                                        int64_t Ttot) {
+    extern __shared__ float th[];  // [R][TB]
+    const int64_t t0 = (int64_t)blockIdx.x * TB;
+    const int n = (int)min((int64_t)TB, Ttot - t0);
+    for (int i = threadIdx.x; i < R * TB; i += blockDim.x) {
+        const int t = i / R, rr = i - t * R;
+        th[rr * TB + t] = t < n ? tanhf(ldf(a + (t0 + t) * ld_a + rr)) : 0.f;
+    }
     __syncthreads();
     const int64_t c = (int64_t)blockIdx.y * blockDim.x + threadIdx.x;
     if (c >= C) return;
-    float z = w0[c];
-#pragma unroll 8
-    for (int r = 0; r < R; ++r) z += th[r] * w2t[(int64_t)r * C + c];
-    logw[t * C + c] = -expf(z);
+    float z[TB];
+    const float z0 = w0[c];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) z[t] = z0;
+#pragma unroll 16
+    for (int rr = 0; rr < R; ++rr) {
+        const float w = w2t[(int64_t)rr * C + c];
+#pragma unroll
+        for (int t = 0; t < TB; ++t) z[t] += th[rr * TB + t] * w;
+    }
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+        if (t < n) logw[(t0 + t) * C + c] = -expf(z[t]);
 }
 
 // One workgroup per (sequence, head) = four thread groups: thread (q, j) owns value channel j and keeps the rows
@@ -182,11 +209,355 @@ __global__ __launch_bounds__((DMAX < 64 ? 64 : DMAX) * IS) void wkv_scan_kernel(
     }
 }
 
+// The same recurrence 16 tokens at a time, for head widths that are multiples of 4 and rows of aligned groups of four elements.
+//
+// A token-by-token scan is a serial chain of 0.7 us per token at d = 64 (LDS round trips and 80 dependent-ish vector instructions), on
+// one workgroup per (sequence, head).  Over a chunk the state is only needed twice,
+//   O = R' S0 + A V          R'_t = r_t * prod_{x < t} w_x          A[t][s] = sum_i r_t[i] k_s[i] prod_{s < x < t} w_x[i], A[t][t] = r u k
+//   S = diag(E) S0 + K'^T V  E = prod_x w_x                         K'_s = k_s * prod_{x > s} w_x
+// four products that go through the fp32 matrix instruction (16x16x4), 36 of them per wave and chunk at d = 64.
+//   * Half of the waves ("makers") stage chunk c + 1 and form its A, R', K' and E while the other half ("holders") run chunk c's
+//     products and finish its output: only the holders' part is a chain from chunk to chunk.
+//   * The state stays in the holders' accumulators from chunk to chunk: holder w has columns 16 w .. 16 w + 15, register r of tile
+//     `it` in lane l is row 16 it + 4 (l / 16) + r, which is also the B operand of a k-step over the rows {16 it + 4 q + r, q = 0 .. 3}.
+//   * Decays are only ever multiplied, in the order of time (a thread per (token, four channels) walks the chunk and keeps its key's
+//     decayed value), never divided or formed as differences of logarithms: products that underflow do so as in the scan, and the
+//     error is the scan's.  A's sums over channels are a reduce-scatter over the token's lanes, 15 moves for 16 sums.
+// A sequence that brings fewer than TOKENWISE tokens (decode) is bound by reading and writing its state: it is walked token by token
+// with the state spread over all threads in 16-byte pieces.
+// 4 x 1024 tokens, 32 heads of 64, bf16: 697 us for the token-by-token scan, 409 us with one set of waves doing both halves' work, 162 us
+// in this form (2.5 us per chunk: the makers' walk through the chunk, 21 vector instructions per token, is the longer half).
+constexpr int CHUNK = 16;
+constexpr int TOKENWISE = 5;
+
+template <typename T, int D>
+__global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
+    const T* __restrict__ r, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ gate, int64_t ld,
+    const float* __restrict__ logw, const float* __restrict__ u, const float* __restrict__ gain, float* __restrict__ state,
+    float* __restrict__ shift_state, const float* __restrict__ h, int64_t W, const int32_t* __restrict__ state_slots,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions, T* __restrict__ out, int64_t ld_out, int H, int d,
+    float eps) {
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    constexpr int NT = 8 * D, NH = NT / 2;  // threads, threads per half
+    constexpr int L = D / 4;     // lanes per token
+    constexpr int NI = D / 16;   // row tiles of the state
+    constexpr int PRE = D > 64 ? 2 : 8;  // (1024 threads have half the registers)
+    constexpr int SV = D + 16;   // row stride of operands read as [4 rows][16 columns]: four rows cover the 64 banks
+    constexpr int SR = D + 4;    // row stride of operands read as [16 rows][4 columns]
+    __shared__ __attribute__((aligned(16))) float rr[CHUNK][D], ww[CHUNK][D], oo[CHUNK][SR];
+    struct Operands {
+        float vv[2][CHUNK][SV], kd[2][CHUNK][SV], rp[2][CHUNK][SR], aa[2][CHUNK][CHUNK + 4], ee[2][D];
+    };
+    __shared__ __attribute__((aligned(16))) Operands sm;
+    auto &vv = sm.vv, &kd = sm.kd;
+    auto &rp = sm.rp;
+    auto &aa = sm.aa;
+    auto &ee = sm.ee;
+    const int b = blockIdx.x, head = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int t0 = cu_q[b], t1 = cu_q[b + 1];
+    if (t1 <= t0) return;
+    const int64_t slot = state_slots[b];
+    const bool fresh = positions[t0] == 0;
+    const int64_t col0 = (int64_t)head * d, C = (int64_t)H * d;
+    float* Sg = state + ((slot * H + head) * d) * (int64_t)d;  // [i][j]
+    const int half_tid = tid % NH;
+    const int s = half_tid / L, c4 = (half_tid % L) * 4;  // token s of a chunk, channels c4 .. c4 + 3
+    const bool mine = c4 < d;
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    auto raw4 = [&](const T* p, int t) -> T4 { return *reinterpret_cast<const T4*>(p + (int64_t)t * ld + col0 + c4); };
+    auto wide4 = [](T4 x) -> f32x4 { return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; };
+    auto row4 = [&](const T* p, int t) -> f32x4 { return wide4(raw4(p, t)); };
+    T4 none;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) none[e] = (T)0.f;
+    f32x4 g4 = zero4;
+    if (mine) g4 = *reinterpret_cast<const f32x4*>(gain + col0 + c4);
+    // per-head unit norm, gain, gate of token t (o4: its four channels; threads of the token's lanes together)
+    auto finish = [&](f32x4 o4, f32x4 gt, int t, bool live) {
+        float ss = o4[0] * o4[0] + o4[1] * o4[1] + o4[2] * o4[2] + o4[3] * o4[3];
+        ss = sum_neighbours<(L < 16 ? L : 16)>(live ? ss : 0.f);
+        if (L > 16) ss += __shfl_xor(ss, 16, 64);
+        if (live && mine) {
+            const float rinv = 1.0f / sqrtf(ss / (float)d + eps);
+            T4 res;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) res[e] = (T)(o4[e] * rinv * g4[e] * (gt[e] / (1.f + expf(-gt[e]))));
+            *reinterpret_cast<T4*>(out + (int64_t)t * ld_out + col0 + c4) = res;
+        }
+    };
+    if (head == 0) {
+        const float* last = h + (int64_t)(t1 - 1) * W;
+        float* dst = shift_state + slot * W;
+        for (int64_t c = tid; c < W; c += NT) dst[c] = last[c];
+    }
+
+    if (t1 - t0 < TOKENWISE) {
+        constexpr int RG = NT / L, RPT = D / RG;  // row groups, rows per thread: rows rg, rg + RG, ...
+        const int n = t1 - t0, rg = tid / L;
+        float(*parts)[TOKENWISE - 1][D] = reinterpret_cast<float(*)[TOKENWISE - 1][D]>(&sm);  // [waves][token][column]
+        static_assert(sizeof(float) * (NT / 64) * (TOKENWISE - 1) * D <= sizeof(sm.vv) + sizeof(sm.kd), "the waves' parts of the output");
+        f32x4 St[RPT];
+#pragma unroll
+        for (int x = 0; x < RPT; ++x) {
+            const int i = rg + x * RG;
+            St[x] = (!fresh && mine && i < d) ? *reinterpret_cast<const f32x4*>(Sg + (int64_t)i * d + c4) : zero4;
+        }
+        const f32x4 u4 = mine ? *reinterpret_cast<const f32x4*>(u + col0 + c4) : zero4;
+        f32x4 vt[TOKENWISE - 1];
+#pragma unroll
+        for (int t = 0; t < TOKENWISE - 1; ++t) vt[t] = (mine && t < n) ? row4(v, t0 + t) : zero4;
+        f32x4 gt = zero4;
+        if (tid < NH && s < n && mine) gt = row4(gate, t0 + s);
+        if (tid < NH && s < n) {
+            f32x4 rc = zero4, kc = zero4, wc = zero4;
+            if (mine) {
+                rc = row4(r, t0 + s);
+                kc = row4(k, t0 + s);
+                wc = *reinterpret_cast<const f32x4*>(logw + (int64_t)(t0 + s) * C + col0 + c4);
+            }
+            float diag = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                diag += rc[e] * u4[e] * kc[e];
+                wc[e] = expf(wc[e]);
+            }
+            *reinterpret_cast<f32x4*>(&rr[s][c4]) = rc;
+            *reinterpret_cast<f32x4*>(&ww[s][c4]) = wc;
+            *reinterpret_cast<f32x4*>(&rp[0][s][c4]) = kc;
+            diag = sum_neighbours<(L < 16 ? L : 16)>(diag);
+            if (L > 16) diag += __shfl_xor(diag, 16, 64);
+            if (half_tid % L == 0) aa[0][s][0] = diag;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TOKENWISE - 1; ++t) {
+            if (t >= n) break;
+            f32x4 o4 = zero4;
+#pragma unroll
+            for (int x = 0; x < RPT; ++x) {
+                const int i = rg + x * RG;
+                const float ri = rr[t][i], wi = ww[t][i], ki = rp[0][t][i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o4[e] += ri * St[x][e];
+                    St[x][e] = wi * St[x][e] + ki * vt[t][e];
+                }
+            }
+            // the wave's row groups, then (below) the waves
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (L <= 8) o4[e] += __shfl_xor(o4[e], 8, 64);
+                if (L <= 16) o4[e] += __shfl_xor(o4[e], 16, 64);
+                o4[e] += __shfl_xor(o4[e], 32, 64);
+            }
+            if (lane < L) *reinterpret_cast<f32x4*>(&parts[tid >> 6][t][c4]) = o4;
+        }
+#pragma unroll
+        for (int x = 0; x < RPT; ++x) {
+            const int i = rg + x * RG;
+            if (mine && i < d) *reinterpret_cast<f32x4*>(Sg + (int64_t)i * d + c4) = St[x];
+        }
+        __syncthreads();
+        if (tid < NH) {
+            f32x4 o4 = zero4;
+            if (s < n && mine) {
+                const f32x4 vs = row4(v, t0 + s);
+                const float diag = aa[0][s][0];
+#pragma unroll
+                for (int w = 0; w < NT / 64; ++w) o4 += *reinterpret_cast<const f32x4*>(&parts[w][s][c4]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o4[e] += diag * vs[e];
+            }
+            finish(o4, gt, t0 + s, s < n);
+        }
+        return;
+    }
+
+    const int wave = __builtin_amdgcn_readfirstlane(half_tid >> 6);
+    const int chunks = (t1 - t0 + CHUNK - 1) / CHUNK;
+    if (tid < NH) {  // ---- makers ----
+        const int s_lo = wave * (64 / L), s_hi = s_lo + 64 / L - 1;
+        const f32x4 u4 = mine ? *reinterpret_cast<const f32x4*>(u + col0 + c4) : zero4;
+        T4 pr, pk, pv;  // as loaded: widening them here would wait for them here
+        f32x4 pw;
+        auto fetch = [&](int c) {
+            const int t = t0 + c * CHUNK + s;
+            pr = pk = pv = none;  // tokens past the end and padded channels: no key, no decay
+            pw = zero4;
+            if (mine && t < t1) {
+                pr = raw4(r, t);
+                pk = raw4(k, t);
+                pv = raw4(v, t);
+                pw = *reinterpret_cast<const f32x4*>(logw + (int64_t)t * C + col0 + c4);
+            }
+        };
+        fetch(0);
+        for (int c = 0; c <= chunks; ++c) {  // holders are one chunk behind
+            const int buf = c & 1;
+            const f32x4 rc = wide4(pr), kc = wide4(pk);
+            float diag = 0.f;
+            if (c < chunks) {
+                f32x4 wc;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    wc[e] = expf(pw[e]);
+                    diag += rc[e] * u4[e] * kc[e];
+                }
+                *reinterpret_cast<f32x4*>(&rr[s][c4]) = rc;
+                *reinterpret_cast<f32x4*>(&ww[s][c4]) = wc;
+                *reinterpret_cast<f32x4*>(&vv[buf][s][c4]) = wide4(pv);
+            }
+            __syncthreads();
+            if (c < chunks) {
+                if (c + 1 < chunks) fetch(c + 1);
+                int own = s;  // (opaque: sixteen hoisted comparison masks would not fit the scalar registers)
+                asm volatile("" : "+v"(own));
+                float p[CHUNK];
+                f32x4 x = zero4, y = {1.f, 1.f, 1.f, 1.f}, rd = zero4;
+#pragma unroll
+                for (int th = 0; th < CHUNK; th += PRE) {
+                    f32x4 w4[PRE], r4[PRE];  // all LDS reads of PRE tokens in flight together
+#pragma unroll
+                    for (int t = 0; t < PRE; ++t) {
+                        w4[t] = *reinterpret_cast<const f32x4*>(&ww[th + t][c4]);
+                        r4[t] = *reinterpret_cast<const f32x4*>(&rr[th + t][c4]);
+                    }
+#pragma unroll
+                    for (int t = 0; t < PRE; ++t) {
+                        const int tt = th + t;
+                        p[tt] = 0.f;
+                        if (tt > s_hi) {  // x: the key of token s as token tt sees it
+                            p[tt] = r4[t][0] * x[0] + r4[t][1] * x[1] + r4[t][2] * x[2] + r4[t][3] * x[3];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) x[e] *= w4[t][e];
+                        } else {          // y: the decay of everything in front of token tt
+                            if (tt >= s_lo) {
+                                const bool at = tt == own;
+                                const float q = r4[t][0] * x[0] + r4[t][1] * x[1] + r4[t][2] * x[2] + r4[t][3] * x[3];
+                                p[tt] = at ? diag : q;
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    x[e] = at ? kc[e] : x[e] * w4[t][e];
+                                    rd[e] = at ? rc[e] * y[e] : rd[e];
+                                }
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) y[e] *= w4[t][e];
+                        }
+                    }
+                }
+                if (s == CHUNK - 1) *reinterpret_cast<f32x4*>(&ee[buf][c4]) = y;
+                *reinterpret_cast<f32x4*>(&rp[buf][s][c4]) = rd;
+                *reinterpret_cast<f32x4*>(&kd[buf][s][c4]) = x;
+                // sums over the token's lanes: a lane passes on the half of its sums that its partner keeps
+                auto halve = [&](auto ctrl, auto width_, int bit) {
+                    constexpr int width = decltype(width_)::value;
+                    const bool upper = (lane & bit) != 0;
+#pragma unroll
+                    for (int i = 0; i < width; ++i) {
+                        const float keep = upper ? p[width + i] : p[i], pass = upper ? p[i] : p[width + i];
+                        p[i] = keep + moved<decltype(ctrl)::value>(0.f, pass);
+                    }
+                };
+                constexpr int W0 = L >= 16 ? 8 : 16;
+                using std::integral_constant;
+                if constexpr (L >= 16) halve(integral_constant<int, 0x140>{}, integral_constant<int, 8>{}, 8);  // lane 15 - i of the row
+                halve(integral_constant<int, 0x141>{}, integral_constant<int, W0 / 2>{}, 4);                    // lane 7 - i of the half row
+                halve(integral_constant<int, 0x1B>{}, integral_constant<int, W0 / 4>{}, 2);                     // lane 3 - i of the quad
+                halve(integral_constant<int, 0xB1>{}, integral_constant<int, W0 / 8>{}, 1);                     // lane ^ 1
+                if (L > 16) p[0] += __shfl_xor(p[0], 16, 64);
+                if (L >= 16) {
+                    aa[buf][lane & 15][s] = p[0];
+                } else {
+                    aa[buf][2 * (lane & 7)][s] = p[0];
+                    aa[buf][2 * (lane & 7) + 1][s] = p[1];
+                }
+            }
+            __syncthreads();
+        }
+        return;
+    }
+
+    // ---- holders ----
+    const int lq = lane >> 4, lc = lane & 15, j = 16 * wave + lc;
+    f32x4 S[NI];
+#pragma unroll
+    for (int it = 0; it < NI; ++it)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = 16 * it + 4 * lq + e;
+            S[it][e] = (!fresh && i < d && j < d) ? Sg[(int64_t)i * d + j] : 0.f;
+        }
+    __syncthreads();
+    __syncthreads();  // the makers' first chunk
+    for (int c = 0; c < chunks; ++c) {
+        const int buf = c & 1, t = t0 + c * CHUNK + s;
+        T4 gt = none;
+        if (mine && t < t1) gt = raw4(gate, t);
+        float vb[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) vb[ks] = vv[buf][4 * ks + lq][j];
+        f32x4 o0 = zero4, o1 = zero4;
+#pragma unroll
+        for (int it = 0; it < NI; ++it) {
+            const f32x4 a4 = *reinterpret_cast<const f32x4*>(&rp[buf][lc][16 * it + 4 * lq]);
+            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[0], S[it][0], o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[1], S[it][1], o1, 0, 0, 0);
+            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[2], S[it][2], o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[3], S[it][3], o1, 0, 0, 0);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ks += 2) {
+            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[buf][lc][4 * ks + lq], vb[ks], o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[buf][lc][4 * ks + 4 + lq], vb[ks + 1], o1, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oo[4 * lq + e][j] = o0[e] + o1[e];
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < NI; ++it) {
+            S[it] *= *reinterpret_cast<const f32x4*>(&ee[buf][16 * it + 4 * lq]);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                S[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[buf][4 * ks + lq][16 * it + lc], vb[ks], S[it], 0, 0, 0);
+        }
+        finish(*reinterpret_cast<const f32x4*>(&oo[s][c4]), wide4(gt), t, t < t1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int it = 0; it < NI; ++it)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = 16 * it + 4 * lq + e;
+            if (i < d && j < d) Sg[(int64_t)i * d + j] = S[it][e];
+        }
+}
+
 template <typename T>
 int launch_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw, const float* u,
                 const float* gain, float* state, float* shift_state, const float* h, int64_t W, const int32_t* slots,
                 const int32_t* cu_q, const int32_t* positions, void* out, int64_t ld_out, int B, int H, int d, float eps,
                 hipStream_t st) {
+    // the chunked form takes rows in groups of four elements (any head width that is a multiple of 4, aligned tensors)
+    const size_t quad = 4 * sizeof(T);
+    auto rows_of_four = [&](const void* p, int64_t stride) { return (uintptr_t)p % quad == 0 && stride % 4 == 0; };
+    if (d % 4 == 0 && rows_of_four(r, ld) && rows_of_four(k, ld) && rows_of_four(v, ld) && rows_of_four(gate, ld) &&
+        rows_of_four(out, ld_out) && (uintptr_t)logw % 16 == 0 && (uintptr_t)u % 16 == 0 && (uintptr_t)gain % 16 == 0 &&
+        (uintptr_t)state % 16 == 0) {
+#define TGIS_WKV_CHUNKS(DM)                                                                                                    \
+    hipLaunchKernelGGL((wkv_chunk_kernel<T, DM>), dim3((unsigned)B, (unsigned)H), dim3(8 * DM), 0, st, (const T*)r, (const T*)k, \
+                       (const T*)v, (const T*)gate, ld, logw, u, gain, state, shift_state, h, W, slots, cu_q, positions, (T*)out, \
+                       ld_out, H, d, eps)
+        if (d <= 32)
+            TGIS_WKV_CHUNKS(32);
+        else if (d <= 64)
+            TGIS_WKV_CHUNKS(64);
+        else
+            TGIS_WKV_CHUNKS(128);
+#undef TGIS_WKV_CHUNKS
+        return 0;
+    }
 #define TGIS_WKV_LAUNCH(DM)                                                                                               \
     hipLaunchKernelGGL((wkv_scan_kernel<T, DM>), dim3((unsigned)B, (unsigned)H), dim3((DM < 64 ? 64 : DM) * IS), 0, st, (const T*)r, \
                        (const T*)k, (const T*)v, (const T*)gate, ld, logw, u, gain, state, shift_state, h, W, slots, cu_q,    \
@@ -212,12 +583,25 @@ extern "C" int tgis_token_shift_mix(const float* h, const float* shift_state, co
     TGIS_CHECK_ARG(B >= 1 && num_mixes >= 1 && W >= 1 && dtype3(dtype), "tgis_token_shift_mix: bad arguments");
     if (T == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
+    const bool vec = W % 4 == 0 && (uintptr_t)h % 16 == 0 && (uintptr_t)shift_state % 16 == 0 && (uintptr_t)mu % 16 == 0 &&
+                     (uintptr_t)out % (dtype == TGIS_F32 ? 16 : 8) == 0;
+    const dim3 grid((unsigned)T, (unsigned)cdiv64(W, vec ? 1024 : 256));
+#define TGIS_SHIFT(TT)                                                                                                             \
+    do {                                                                                                                           \
+        if (vec)                                                                                                                   \
+            hipLaunchKernelGGL((token_shift_mix_kernel<TT, 4>), grid, dim3(256), 0, st, h, shift_state, state_slots, cu_seqlens_q, \
+                               positions, (int)B, mu, num_mixes, (TT*)out, T, W);                                                  \
+        else                                                                                                                       \
+            hipLaunchKernelGGL((token_shift_mix_kernel<TT, 1>), grid, dim3(256), 0, st, h, shift_state, state_slots, cu_seqlens_q, \
+                               positions, (int)B, mu, num_mixes, (TT*)out, T, W);                                                  \
+    } while (0)
     if (dtype == TGIS_F16)
-        hipLaunchKernelGGL(token_shift_mix_kernel<f16>, dim3((unsigned)T, (unsigned)cdiv64(W, 256)), dim3(256), 0, st, h, shift_state, state_slots, cu_seqlens_q, positions, (int)B, mu, num_mixes, (f16*)out, T, W);
+        TGIS_SHIFT(f16);
     else if (dtype == TGIS_BF16)
-        hipLaunchKernelGGL(token_shift_mix_kernel<bf16>, dim3((unsigned)T, (unsigned)cdiv64(W, 256)), dim3(256), 0, st, h, shift_state, state_slots, cu_seqlens_q, positions, (int)B, mu, num_mixes, (bf16*)out, T, W);
+        TGIS_SHIFT(bf16);
     else
-        hipLaunchKernelGGL(token_shift_mix_kernel<float>, dim3((unsigned)T, (unsigned)cdiv64(W, 256)), dim3(256), 0, st, h, shift_state, state_slots, cu_seqlens_q, positions, (int)B, mu, num_mixes, (float*)out, T, W);
+        TGIS_SHIFT(float);
+#undef TGIS_SHIFT
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
@@ -227,13 +611,23 @@ extern "C" int tgis_wkv_decay(const void* a, int64_t ld_a, const float* w2t, con
     TGIS_CHECK_ARG(a && w2t && w0 && logw && rank >= 1 && rank <= 8192 && C >= 1 && C <= 65535 * 256 && ld_a >= rank && dtype3(dtype), "tgis_wkv_decay: bad arguments");
     if (T == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    const size_t lds = (size_t)rank * sizeof(float);
+    const int tb = T >= 1024 && rank <= 512 ? 8 : 1;
+    const size_t lds = (size_t)rank * tb * sizeof(float);
+    const dim3 grid((unsigned)cdiv64(T, tb), (unsigned)cdiv64(C, 256));
+#define TGIS_DECAY(TT)                                                                                                              \
+    do {                                                                                                                            \
+        if (tb == 8)                                                                                                                \
+            hipLaunchKernelGGL((wkv_decay_kernel<TT, 8>), grid, dim3(256), lds, st, (const TT*)a, ld_a, w2t, w0, logw, rank, C, T); \
+        else                                                                                                                        \
+            hipLaunchKernelGGL((wkv_decay_kernel<TT, 1>), grid, dim3(256), lds, st, (const TT*)a, ld_a, w2t, w0, logw, rank, C, T); \
+    } while (0)
     if (dtype == TGIS_F16)
-        hipLaunchKernelGGL(wkv_decay_kernel<f16>, dim3((unsigned)T, (unsigned)cdiv64(C, 256)), dim3(256), lds, st, (const f16*)a, ld_a, w2t, w0, logw, rank, C);
+        TGIS_DECAY(f16);
     else if (dtype == TGIS_BF16)
-        hipLaunchKernelGGL(wkv_decay_kernel<bf16>, dim3((unsigned)T, (unsigned)cdiv64(C, 256)), dim3(256), lds, st, (const bf16*)a, ld_a, w2t, w0, logw, rank, C);
+        TGIS_DECAY(bf16);
     else
-        hipLaunchKernelGGL(wkv_decay_kernel<float>, dim3((unsigned)T, (unsigned)cdiv64(C, 256)), dim3(256), lds, st, (const float*)a, ld_a, w2t, w0, logw, rank, C);
+        TGIS_DECAY(float);
+#undef TGIS_DECAY
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
