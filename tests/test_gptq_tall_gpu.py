@@ -1,0 +1,60 @@
+"""-m gpu: the int4 GEMM at prefill sizes (csrc/gptq_tall.hip): every tile shape, unsplit tiles, tiles split over k, ragged edges."""
+import pytest
+import torch
+
+from oracle import ops_ref
+
+pytestmark = pytest.mark.gpu
+
+
+# K: one step, fewer and more steps than the ring of buffers, a whole number of rings; N: one tile, ragged and several column blocks
+@pytest.mark.parametrize("K,N,groupsize", [(64, 32, 64), (192, 288, 64), (320, 512, 64), (1024, 1120, 128), (1152, 96, 1152)])
+@pytest.mark.parametrize("M", [129, 161, 300])
+@pytest.mark.parametrize("act", [0, 2])
+def test_every_plan(gpu_device, K, N, groupsize, M, act, monkeypatch):
+    from tgis_amd import native
+
+    qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, groupsize, seed=K + N)
+    w = native.GptqWeight(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), 4, groupsize, gate_up=act == 2)
+    g = torch.Generator().manual_seed(M)
+    x, bias = torch.randn(M, K, generator=g).half(), (torch.randn(N, generator=g) * 0.1).half()
+    ws = native.Workspace(64 << 20, gpu_device)
+    y = x.double() @ ops_ref.gptq_dequant(qw, qz, sc, gi, groupsize).half().double() + bias.double()
+    # a rounding of an fp32 sum to f16 (2 ** -11 of it) plus the sum's own order; before the activation that order may turn the
+    # rounding of gate or up the other way (2 ** -10 of either, so 3 * 2 ** -10 of the product)
+    ulp = 2.0 ** -10
+    want, tol = y, ulp * y.abs() + 1e-5
+    if act == 2:
+        gate, up = y.half()[:, :N // 2], y.half()[:, N // 2:]
+        want = (torch.nn.functional.silu(gate.float()).half().float() * up.float()).half().double()
+        tol = 3 * ulp * (gate.double() * up.double()).abs() + 1e-5
+    cols = want.shape[1]
+    # (a launch that splits needs at least one k64-step per split)
+    plans = [None] + [f"{b},{t},{s}" for b in (2, 3, 4) for t in (1, 2) for s in (1, 2, 5) if s == 1 or K // 64 >= 2 * s]
+    for plan in plans:
+        if plan is None:
+            monkeypatch.delenv("TGIS_TALL_PLAN", raising=False)
+        else:
+            monkeypatch.setenv("TGIS_TALL_PLAN", plan)
+        for pad in (0, 3):  # rows of the output that take 16-byte stores, and rows that do not
+            wide = torch.full((M, cols + pad), 7.0, dtype=torch.float16, device=gpu_device)
+            native.gptq_gemm(x.to(gpu_device), w, ws, bias=bias.to(gpu_device), act=act, out=wide[:, :cols])
+            err = (wide[:, :cols].double().cpu() - want).abs()
+            assert (err <= tol).all(), (plan, pad, float((err - tol).max()))
+            assert (wide[:, cols:] == 7.0).all()
+
+
+def test_linear_takes_whole_sums_past_128_rows(gpu_device):
+    """129 .. 256 rows: the linear returns a finished tensor where 64-row passes left slabs to the consumer."""
+    from tgis_amd import native
+    from tgis_amd.utils.layers import Ex4bitLinearV2
+
+    qw, qz, sc, gi = ops_ref.make_gptq_tensors(256, 128, 128, seed=3)
+    lin = Ex4bitLinearV2(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), None, 4, 128)
+    for M in (128, 129, 256):
+        x = torch.randn(M, 256, generator=torch.Generator().manual_seed(M)).half()
+        got = lin(x.to(gpu_device), partial=True)
+        assert isinstance(got, native.Partial) == (M == 128)
+        if M > 128:
+            want = x.double() @ ops_ref.gptq_dequant(qw, qz, sc, gi, 128).half().double()
+            assert ((got.double().cpu() - want).abs() <= 2.0 ** -10 * want.abs() + 1e-5).all()

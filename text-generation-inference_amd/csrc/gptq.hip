@@ -20,6 +20,7 @@
 #include <type_traits>
 #include "gptq_gemm_body.h"
 #include "gptq_wide_body.h"
+#include "gptq_tall.h"
 
 namespace {
 
@@ -110,211 +111,6 @@ template <int CT, int ACT, bool OUTF, int MR>
 __global__ __launch_bounds__(64 * gptq::WIDE_WK) void gptq_wide_kernel(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     gptq::gptq_wide_unit<CT, ACT, OUTF, MR>(a, smem);
-}
-
-// ---- "tall" kernel: 64 < M (decode batches beyond 32 rows, add-on prefills of up to a few thousand tokens) --------
-// The streaming kernel above re-streams and re-dequantises the weights once per 32 (64) rows; the library path
-// (dequantise the whole matrix to a scratch copy, then hipBLASLt) only pays off for very tall M.  In between, one block
-// keeps BM = 32 BMR rows of x in LDS per 128-k chunk and each of its four waves owns one 32-column tile: a wave loads
-// 1 KiB of the same prepared image per k64-step, dequantises it ONCE into four MFMA B fragments and applies them to
-// all BMR row blocks (BMR x 4 MFMAs 32x32x16 per 52 dequantisation instructions: MFMA-bound from BMR = 2).  No scratch
-// copy of W, no second pass over the weights, same epilogues (bias, SiLU * up on the interleaved gate/up image,
-// split-K slabs in the 32-row units the consumers expect).
-constexpr int TKC = 128;       // k per x chunk (2 k64-steps)
-constexpr int TRS = TKC + 8;   // LDS row stride in halves (+16 B: conflict-free ds_read_b128 of A fragments)
-
-// TW = 32-column tiles per wave.  With one tile every MFMA needs its own 1 KiB A fragment from LDS: eight resident waves x
-// one ds_read_b128 per 32-cycle MFMA is the whole LDS bandwidth of the CU.  With two tiles an A fragment feeds two MFMAs
-// (256-column blocks, half the LDS traffic per flop); the kernel is held to 256 registers so that two blocks still share
-// a CU.
-template <int BMR, int ACT, int TW>
-__global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(GemmArgs a) {
-    constexpr int BM = 32 * BMR;
-    constexpr int NJ = BM * 16 / 256;  // 16-byte x pieces per thread and chunk
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    f16* xs = reinterpret_cast<f16*>(smem);  // [2][BM][TRS]
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int m0 = blockIdx.y * BM;
-    const int mrows = min(BM, a.M - m0);
-    const int split = blockIdx.z;
-    const int nt_raw0 = (blockIdx.x * 4 + w) * TW;
-    const int ksteps = a.K >> 6;                     // K % 64 == 0 (host)
-    const int per = a.KR >> 6;                       // k64-steps per split (multiple of 2)
-    const int ks0 = split * per, ks1 = min(ksteps, ks0 + per);
-    const int nchunks = (ks1 - ks0 + 1) >> 1;        // block-uniform
-
-    const char* wtile[TW];
-    const char* sztile[TW];
-#pragma unroll
-    for (int t = 0; t < TW; ++t) {
-        const int nt = min(nt_raw0 + t, a.NT - 1);
-        wtile[t] = reinterpret_cast<const char*>(a.prep) + (int64_t)nt * a.KS * 1024;
-        sztile[t] = reinterpret_cast<const char*>(a.prep + a.offB) + (int64_t)nt * a.G * 128;
-    }
-    const uint32_t woff = lane * 16, szoff = (lane & 31) * 4;
-    auto sz_at = [&](int t, int ks) -> uint32_t {
-        const int g = min(ks >> a.spg_shift, a.G - 1);
-        const char* p = sztile[t] + (int64_t)g * 128;
-        PIN_SGPR(p);
-        const uint32_t v = *(const GLOBAL_AS uint32_t*)(p + szoff);
-        return ks < ks1 ? v : 0u;  // steps past the split's range add zeros
-    };
-    auto w_at = [&](int t, int ks) -> u32x4 {
-        const char* p = wtile[t] + (int64_t)min(ks, ksteps - 1) * 1024;
-        PIN_SGPR(p);
-        return __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(p + woff));
-    };
-
-    // x staging: piece p = tid + 256 j -> row p / 16, 8-element column (p % 16) * 8 of the chunk
-    const f16* xbase = a.x + (int64_t)m0 * a.ldx;
-    f16x8 xg[NJ];
-    uint32_t rowoff[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) rowoff[j] = (uint32_t)(min((tid + 256 * j) >> 4, mrows - 1) * (int)a.ldx * 2);
-    const int scol = (tid & 15) * 8;
-    auto stage_load = [&](int chunk) {
-        const int kc = min((ks0 << 6) + chunk * TKC + scol, a.K - 8);
-        const char* xb = reinterpret_cast<const char*>(xbase);
-        PIN_SGPR(xb);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) xg[j] = *(const GLOBAL_AS f16x8*)(xb + rowoff[j] + (uint32_t)kc * 2);
-    };
-    auto stage_store = [&](int buf) {
-        f16* dst = xs + buf * (BM * TRS) + (tid >> 4) * TRS + scol;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) st16(dst + j * 16 * TRS, xg[j]);
-    };
-
-    uint32_t EXr = 0x64006400u, M0r = 0x000F000Fu, M1r = 0x00F000F0u;
-    asm volatile("" : "+v"(EXr));
-    asm volatile("" : "+s"(M0r), "+s"(M1r));
-    f32x16 acc[TW][BMR];
-#pragma unroll
-    for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int rb = 0; rb < BMR; ++rb) acc[t][rb] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int xoff = (lane & 31) * TRS + (lane >> 5) * 32;
-
-    stage_load(0);
-    u32x4 wq[TW][4];
-    uint32_t szr[TW][4];
-#pragma unroll
-    for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) szr[t][s] = sz_at(t, ks0 + s);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int t = 0; t < TW; ++t) wq[t][s] = w_at(t, ks0 + s);
-    stage_store(0);
-    __syncthreads();
-
-    // one chunk = 2 k64-steps in ring slots SB, SB + 1; the slots are refilled in place two chunks ahead
-    auto chunk_body = [&](const int chunk, auto sb_tag) {
-        constexpr int SB = decltype(sb_tag)::value;
-        const bool more = chunk + 1 < nchunks;  // block-uniform
-        if (more) stage_load(chunk + 1);
-        uint32_t szn[TW][2];
-#pragma unroll
-        for (int t = 0; t < TW; ++t)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) szn[t][s2] = sz_at(t, ks0 + chunk * 2 + s2 + 4);
-        const f16* xbuf = xs + (chunk & 1) * (BM * TRS) + xoff;
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            const int ks = ks0 + chunk * 2 + s2;
-            f16x8 b[TW][4];
-#pragma unroll
-            for (int t = 0; t < TW; ++t) {
-                const u32x4 cur = wq[t][SB + s2];
-                const f16x2 szh = __builtin_bit_cast(f16x2, szr[t][SB + s2]);
-                const f16 zc1 = szh[1];
-                const f16 zd1 = (f16)960.f - zc1;
-                const f16x2 zc = {zc1, zc1}, zd = {zd1, zd1}, sc = {szh[0], szh[0]};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    b[t][i] = gptq::dequant8(cur[i], zc, zd, sc, EXr, M0r, M1r);
-                }
-                wq[t][SB + s2] = w_at(t, ks + 4);
-            }
-            const f16* xk = xbuf + s2 * 64;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int rb = 0; rb < BMR; ++rb) {
-                    const f16x8 av = ld16<f16x8>(xk + rb * (32 * TRS) + i * 8);
-#pragma unroll
-                    for (int t = 0; t < TW; ++t) acc[t][rb] = mfma32(av, b[t][i], acc[t][rb]);
-                }
-        }
-#pragma unroll
-        for (int t = 0; t < TW; ++t)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) szr[t][SB + s2] = szn[t][s2];
-        if (more) stage_store((chunk + 1) & 1);
-        __syncthreads();
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using I2 = std::integral_constant<int, 2>;
-    int chunk = 0;
-    for (; chunk + 1 < nchunks; chunk += 2) {
-        chunk_body(chunk, I0{});
-        chunk_body(chunk + 1, I2{});
-    }
-    if (chunk < nchunks) chunk_body(chunk, I0{});
-
-    // ---- epilogue: lane holds rows m = 32 rb + (r&3) + 8 (r>>2) + 4 (lane>>5) of column n = nt * 32 + (lane & 31) ----
-    const int c = lane & 31;
-#pragma unroll
-    for (int t = 0; t < TW; ++t) {
-    const int nt = nt_raw0 + t;
-    if (nt >= a.NT) break;
-    if (ACT == 2) {
-        const int half = a.N >> 1;
-        const int j = nt * 16 + (c & 15);
-        const int nsrc = (c < 16) ? j : half + j;
-        const float bv = a.bias ? (float)a.bias[nsrc] : 0.f;
-#pragma unroll
-        for (int rb = 0; rb < BMR; ++rb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float mine = (float)(f16)(acc[t][rb][r] + bv);
-                const float other = __shfl_xor(mine, 16, 64);
-                const int m = rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                if (c < 16 && m < mrows) {
-                    const float sl = mine / (1.f + __expf(-mine));
-                    a.out[(int64_t)(m0 + m) * a.ldo + j] = (f16)((float)(f16)sl * other);
-                }
-            }
-        continue;
-    }
-    const int n = nt * 32 + c;
-    if (a.S == 1 && !a.partial) {
-        const float bv = a.bias ? (float)a.bias[n] : 0.f;
-#pragma unroll
-        for (int rb = 0; rb < BMR; ++rb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                if (m < mrows) a.out[(int64_t)(m0 + m) * a.ldo + n] = (f16)(acc[t][rb][r] + bv);
-            }
-    } else {
-        // slabs in 32-row units [unit][S][32][NP], unit = row / 32 (what norm / rope / the reduce kernel index)
-        const int64_t np = (int64_t)a.NT * 32;
-#pragma unroll
-        for (int rb = 0; rb < BMR; ++rb) {
-            const int unit = blockIdx.y * BMR + rb;
-            if (unit * 32 >= a.M) continue;
-            float* sl = a.slabs + ((int64_t)(unit * a.S + split) * 32) * np + n;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                sl[(int64_t)m * np] = acc[t][rb][r];
-            }
-        }
-    }
-    }
 }
 
 // Sum the S split-K slabs in fixed order (deterministic) and emit f16 (+bias): thread = (row, 4 columns).
@@ -465,128 +261,18 @@ extern "C" int tgis_gptq_prepare(const int32_t* qweight, const int32_t* qzeros, 
     return TGIS_OK;
 }
 
-// ---- tall kernel: when, and how it is cut ---------------------------------------------------------------------------
-// Rows from which the tall kernel replaces the 64-row streaming passes, and up to which it replaces dequantise + library
-// GEMM.  tools/tall_sweep.py on MI355X, cfg3 shapes (profiles/r02_tall_sweep.log; us, tall / passes / library incl. its
-// dequantisation): gate_up M=256 75 / 82 / 172, M=512 132 / 164 / 206, M=1024 235 / - / 304, M=2048 437 / - / 508, M=3072
-// 640 / - / 659, M=4096 814 / - / 871; qkv M=512 81 / 82 / 100, M=1024 133 / - / 138, M=2048 227 / - / 230, M=3072 339 / -
-// / 331, M=4096 423 / - / 381; the four GEMMs of a layer together: M=2048 954 / - / 1027, M=3072 1444 / - / 1373, M=4096
-// 1752 / - / 1713, M=8192 3441 / - / 3056.  Up to 256 rows the passes (with their deferred split-K sums) stay; from 257 to
-// 3072 rows the tall kernel runs at 0.65-0.9 PFLOP/s without a scratch copy of W; above, hipBLASLt on the dequantised
-// copy (1.1-1.2 PFLOP/s) wins by a few per cent and more.  Two 32-column tiles per wave (an A fragment from LDS feeds two
-// MFMAs; 1.0 PFLOP/s at M >= 4096) once 384 blocks of 256 columns remain; one tile per wave below.
-static int64_t tall_min_m() {
-    static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 257;
-    return v;
-}
-static int64_t tall_max_m() {
-    static const int64_t v = getenv("TGIS_TALL_MAX_M") ? atoll(getenv("TGIS_TALL_MAX_M")) : 3072;
-    return v;
-}
-static bool tall_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act) {
-    if (M < tall_min_m() || perm != nullptr || act == 1 || K % 64 != 0) return false;
-    const int64_t gs = K / groups, spg = gs / 64;
-    return groups == 1 || (gs % 64 == 0 && (spg & (spg - 1)) == 0);
-}
-struct TallPlan {
-    int BMR, S, KR, TW;
-};
-static TallPlan plan_tall(int64_t M, int64_t K, int64_t N, int act) {
-    TallPlan t;
-    t.BMR = M > 64 ? 4 : 2;
-    // two tiles per wave (256-column blocks) once that still leaves every CU a few blocks
-    t.TW = (t.BMR == 4 && cdiv64(cdiv64(N, 32), 8) * cdiv64(M, 128) >= 384) ? 2 : 1;
-    if (const char* e = getenv("TGIS_TALL_TW")) t.TW = (atoi(e) == 2 && t.BMR == 4) ? 2 : 1;
-    const int64_t blocks = cdiv64(cdiv64(N, 32), 4 * t.TW) * cdiv64(M, 32 * t.BMR);
-    const int64_t kchunks = cdiv64(K, TKC);
-    int64_t S = 1;
-    if (act != 2 && blocks < 384) S = std::min<int64_t>(std::min<int64_t>(kchunks, 16), cdiv64(512, blocks));
-    if (const char* e = getenv("TGIS_TALL_SPLITS")) S = std::max<int64_t>(1, std::min<int64_t>(kchunks, atoll(e)));
-    if (act == 2) S = 1;
-    int64_t per = cdiv64(kchunks, S);
-    while (S > 1 && (S - 1) * per >= kchunks) --S;
-    t.S = (int)S;
-    t.KR = (int)(per * TKC);
-    return t;
-}
-static int64_t tall_slab_bytes(int64_t M, int64_t N, int S) { return (int64_t)cdiv64(M, 32) * S * 32 * cdiv64(N, 32) * 32 * 4; }
-
-static int launch_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo,
-                       int64_t M, int64_t K, int64_t N, int64_t groups, int act, float* slabs, int partial,
-                       const TallPlan& tp, hipStream_t st) {
-    PrepLayout p = prep_layout(K, N, groups);
-    const int64_t gs = K / groups, spg = gs / 64;
-    GemmArgs a;
-    a.x = (const f16*)x;
-    a.ldx = ldx;
-    a.prep = (const uint8_t*)prepared;
-    a.offB = p.offB;
-    a.bias = partial ? nullptr : (const f16*)bias;
-    a.perm = nullptr;
-    a.out = (f16*)out;
-    a.ldo = ldo;
-    a.M = (int)M;
-    a.K = (int)K;
-    a.N = (int)N;
-    a.G = (int)groups;
-    a.gs = (int)gs;
-    a.KR = tp.KR;
-    a.S = tp.S;
-    a.NT = (int)p.NT;
-    a.KS = (int)p.KS;
-    a.slabs = slabs;
-    a.partial = partial;
-    a.spg_shift = 30;
-    a.positions = a.slots = nullptr;
-    a.cosb = a.sinb = nullptr;
-    a.kpool = a.vpool = nullptr;
-    a.rH = a.rHkv = a.rD = 0;
-    if (groups > 1)
-        for (a.spg_shift = 0; (1 << a.spg_shift) < spg; ++a.spg_shift) {}
-    const int BM = 32 * tp.BMR;
-    TGIS_CHECK_ARG(cdiv64(M, BM) <= 65535, "tgis_gptq_gemm: M too large for one launch");
-    dim3 grid((unsigned)cdiv64(p.NT, 4 * tp.TW), (unsigned)cdiv64(M, BM), (unsigned)tp.S);
-    const size_t lds = (size_t)2 * BM * TRS * sizeof(f16);
-#define TGIS_TALL(B, A, W)                                                                                     \
-    do {                                                                                                      \
-        static bool attr = false;                                                                             \
-        if (!attr) {                                                                                          \
-            TGIS_CHECK_HIP(hipFuncSetAttribute((const void*)gptq_gemm_tall_kernel<B, A, W>,                   \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 128 * TRS * 2)); \
-            attr = true;                                                                                      \
-        }                                                                                                     \
-        hipLaunchKernelGGL((gptq_gemm_tall_kernel<B, A, W>), grid, dim3(256), lds, st, a);                    \
-    } while (0)
-    if (tp.BMR == 4 && tp.TW == 2) {
-        if (act == 2) TGIS_TALL(4, 2, 2); else TGIS_TALL(4, 0, 2);
-    } else if (tp.BMR == 4) {
-        if (act == 2) TGIS_TALL(4, 2, 1); else TGIS_TALL(4, 0, 1);
-    } else {
-        if (act == 2) TGIS_TALL(2, 2, 1); else TGIS_TALL(2, 0, 1);
-    }
-#undef TGIS_TALL
-    TGIS_CHECK_LAUNCH();
-    if (!partial && tp.S > 1) {
-        const int NP = (int)p.NT * 32;
-        dim3 rgrid((unsigned)cdiv64((int64_t)32 * (NP / 4), 256), (unsigned)cdiv64(M, 32));
-        hipLaunchKernelGGL(splitk_reduce_f16_kernel, rgrid, dim3(256), 0, st, slabs, (const f16*)bias, (f16*)out, ldo,
-                           (int)M, (int)N, NP, tp.S);
-        TGIS_CHECK_LAUNCH();
-    }
-    return TGIS_OK;
-}
-
 extern "C" int64_t tgis_gptq_gemm_fused_rows(int64_t K, int64_t groups, int act_order, int act) {
     if (K <= 0 || groups <= 0 || K % groups) return 0;
     static const int32_t some_perm = 0;
-    return tall_ok(tall_min_m(), K, groups, act_order ? &some_perm : nullptr, act) ? std::max<int64_t>(256, tall_max_m()) : 256;
+    return gptq::tall_ok(gptq::tall_min_m(act), K, groups, act_order ? &some_perm : nullptr, act) ? std::max<int64_t>(256, gptq::tall_max_m()) : 256;
 }
 
 extern "C" int64_t tgis_gptq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     GemmPlan pl = plan_gemm(K, N, 0, M);
     int64_t need = 4096 + slab_bytes(M, N, pl.S);
     if (M <= 64 && K % 64 == 0) need = std::max(need, 4096 + slab_bytes(M, N, gptq::wide_max_splits(K, N)));
-    if (M >= tall_min_m() && K % 64 == 0) need = std::max(need, 4096 + tall_slab_bytes(M, N, plan_tall(M, K, N, 0).S));
+    if (M >= gptq::tall_min_m(2) && K % 64 == 0)
+        need = std::max(need, 4096 + gptq::tall_workspace_bytes(M, K, N));
     return need;
 }
 
@@ -810,14 +496,12 @@ extern "C" int tgis_gptq_gemm_f16(const void* x, int64_t ldx, const void* prepar
                            (float*)((uint8_t*)workspace + 4096), 0, wp, st);
     }
     TGIS_CHECK_ARG(ldo != TGIS_LD_FRAGMENTS, "tgis_gptq_gemm_f16: a fragment-order output needs a fragment-order activation");
-    if (tall_ok(M, K, groups, perm, act)) {
-        const TallPlan tp = plan_tall(M, K, N, act);
-        const int64_t need_t = 4096 + (tp.S > 1 ? tall_slab_bytes(M, N, tp.S) : 0);
+    if (gptq::tall_ok(M, K, groups, perm, act)) {
+        const int64_t need_t = 4096 + gptq::tall_workspace_bytes(M, K, N);
         TGIS_CHECK_ARG(workspace && workspace_bytes >= need_t, "tgis_gptq_gemm_f16: workspace too small (%ld < %ld)",
                        (long)workspace_bytes, (long)need_t);
         TgisTimedScope timed(TGIS_OP_GPTQ_GEMM, st);
-        return launch_tall(x, ldx, prepared, bias, out, ldo, M, K, N, groups, act, (float*)((uint8_t*)workspace + 4096), 0,
-                           tp, st);
+        return gptq::launch_tall(x, ldx, prepared, bias, out, ldo, M, K, N, groups, act, (float*)((uint8_t*)workspace + 4096), st);
     }
     GemmPlan pl = plan_gemm(K, N, act, M);
     TGIS_CHECK_ARG(cdiv64(M, 32) <= 65535, "tgis_gptq_gemm_f16: M too large for one launch");
@@ -906,7 +590,7 @@ extern "C" int64_t tgis_gptq_gemm_partial_bytes(int64_t M, int64_t K, int64_t N)
     int64_t need = cdiv64(std::max<int64_t>(M, 1), 64) * 2 * pl.S * 32 * cdiv64(N, 32) * 32 * 4;
     if (M <= 64 && K % 64 == 0)  // the fragment-order kernel's plan may split further
         need = std::max<int64_t>(need, (int64_t)2 * gptq::wide_max_splits(K, N) * 32 * cdiv64(N, 32) * 32 * 4);
-    if (M >= tall_min_m() && K % 64 == 0) need = std::max(need, tall_slab_bytes(M, N, plan_tall(M, K, N, 0).S));
+    if (M >= 257 && K % 64 == 0) need = std::max(need, gptq::tall_slab_bytes(M, N, gptq::tall_partial_splits(M, K, N)));
     return need;
 }
 
@@ -934,14 +618,13 @@ extern "C" int tgis_gptq_gemm_f16_partial(const void* x, int64_t ldx, const void
     if (rc != TGIS_OK) return rc;
     TGIS_CHECK_ARG(M >= 1 && cdiv64(M, 32) <= 65535, "tgis_gptq_gemm_f16_partial: bad M");
     TGIS_CHECK_ARG(act != 2, "tgis_gptq_gemm_f16_partial: act=2 cannot be deferred");
-    if (tall_ok(M, K, groups, perm, act)) {
-        const TallPlan tp = plan_tall(M, K, N, act);
-        TGIS_CHECK_ARG(slabs && slabs_bytes >= tall_slab_bytes(M, N, tp.S),
-                       "tgis_gptq_gemm_f16_partial: slab buffer too small");
-        if (num_slabs) *num_slabs = tp.S;
+    if (gptq::tall_partial_ok(M, K, groups, perm, act)) {
+        const int S = gptq::tall_partial_splits(M, K, N);
+        TGIS_CHECK_ARG(slabs && slabs_bytes >= gptq::tall_slab_bytes(M, N, S), "tgis_gptq_gemm_f16_partial: slab buffer too small");
+        if (num_slabs) *num_slabs = S;
         if (slab_ld) *slab_ld = cdiv64(N, 32) * 32;
         TgisTimedScope timed(TGIS_OP_GPTQ_GEMM, (hipStream_t)stream);
-        return launch_tall(x, ldx, prepared, nullptr, nullptr, 0, M, K, N, groups, act, slabs, 1, tp, (hipStream_t)stream);
+        return gptq::launch_tall_partial(x, ldx, prepared, M, K, N, groups, slabs, (hipStream_t)stream);
     }
     GemmPlan pl = plan_gemm(K, N, 0, M);
     if (ldx == TGIS_LD_FRAGMENTS) {

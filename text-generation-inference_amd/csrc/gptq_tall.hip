@@ -1,0 +1,505 @@
+// The int4 GEMM at prefill sizes: more rows than the streaming kernels of gptq_gemm_body.h / gptq_wide_body.h take in one pass.
+//
+// Those re-stream and re-dequantise the weights once per 32 (64) rows; the library path (dequantise the whole matrix to a scratch copy,
+// then hipBLASLt) pays for the copy.  In between, one block keeps BM = 32 BMR rows of x in LDS and each of its four waves owns TW
+// 32-column tiles: a wave loads 1 KiB of the prepared image per k64-step and tile, dequantises it ONCE into four MFMA B fragments and
+// applies them to all BMR row blocks.  No scratch copy of W, no second pass over the weights, SiLU * up in the epilogue.
+//
+// Rows of x go to LDS by direct loads, 64 k at a time, three steps ahead, into a ring of four buffers: no registers, no stores, and one
+// barrier per step (32 MFMAs per wave at TW 2), behind which the NEXT step's x is complete too, so that its first fragments are read
+// before the barrier.  A buffer row is 128 bytes; its 16-byte pieces are stored at piece ^ (row & 7) (each lane of the load asks for the
+// piece that belongs at its place), so that fragment reads of 32 rows meet no bank twice.  Inside a step the four 16-k slices are
+// pipelined: while slice i is multiplied, slice i + 1 is dequantised and its A fragments are read.
+//
+// Bound: the matrix cores, which this card's power holds to about 1.5 PFLOP/s on random data whatever feeds them (a bare MFMA loop), and
+// the dequantisation's share of that power.  A 128 x 256 tile of 4096 k takes 51 us alone on a CU, 65 on a full chip (1.05 PFLOP/s; 68
+// and 65 when x went through registers, every fragment was read where it was needed and a chunk of 128 k had one barrier); several
+// blocks on a CU only share its matrix cores, so that the plan below weighs whole rounds of 256 CUs.  7B layer, 765 rows: qkv 112 -> 81,
+// o 51 -> 35, gate_up 202 -> 144, down 110 -> 82 us.
+#include <stdlib.h>
+#include <algorithm>
+#include <type_traits>
+#include "common.h"
+#include "gptq_gemm_body.h"
+#include "gptq_tall.h"
+
+namespace {
+
+using gptq::PrepLayout;
+using gptq::prep_layout;
+
+struct TallArgs {
+    const f16* x;
+    int64_t ldx;
+    const uint8_t* prep;
+    int64_t offB;
+    const f16* bias;
+    f16* out;
+    int64_t ldo;
+    int M, K, N, NT, KS, G, spg_shift;
+    int tile0, col_blocks;  // this launch: tiles tile0 + blockIdx.x, column blocks fastest
+    int per, S;             // k64-steps per split, splits (blockIdx.y)
+    int mode;               // 0: finished output; 1: fp32 tiles [blockIdx.x][split][BM][BN] in `scratch`; 2: fp32 slabs in 32-row units
+    int vec;                // rows of `out` take 16-byte stores
+    float* scratch;
+};
+
+constexpr int TALL_RING = 4;  // k64-steps of weights in flight per wave, and buffers of x
+
+// 1 KiB of x: lane l's 16 bytes at base + off go to LDS byte `lds` + 16 l
+__device__ __forceinline__ void tall_x_to_lds(const char* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+
+template <int BMR, int ACT, int TW>
+__global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
+    constexpr int BM = 32 * BMR;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [TALL_RING][BM][128 bytes]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = a.tile0 + blockIdx.x, col_block = tile % a.col_blocks, row_block = tile / a.col_blocks;
+    const int m0 = row_block * BM;
+    const int mrows = min(BM, a.M - m0);
+    const int split = blockIdx.y;
+    const int nt_raw0 = (col_block * 4 + w) * TW;
+    const int ksteps = a.K >> 6;                                         // K % 64 == 0 (host)
+    const int ks0 = split * a.per, n = min(ksteps, ks0 + a.per) - ks0;   // n >= 1 (host)
+
+    const char* wtile[TW];
+    const char* sztile[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+        const int nt = min(nt_raw0 + t, a.NT - 1);
+        wtile[t] = reinterpret_cast<const char*>(a.prep) + (int64_t)nt * a.KS * 1024;
+        sztile[t] = reinterpret_cast<const char*>(a.prep + a.offB) + (int64_t)nt * a.G * 128;
+    }
+    const uint32_t woff = lane * 16, szoff = (lane & 31) * 4;
+    auto sz_at = [&](int t, int ks) -> uint32_t {
+        const char* p = sztile[t] + (int64_t)min(ks >> a.spg_shift, a.G - 1) * 128;
+        PIN_SGPR(p);
+        return *(const GLOBAL_AS uint32_t*)(p + szoff);
+    };
+    auto w_at = [&](int t, int ks) -> u32x4 {
+        const char* p = wtile[t] + (int64_t)min(ks, ksteps - 1) * 1024;
+        PIN_SGPR(p);
+        return __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(p + woff));
+    };
+
+    // x: load j of wave w brings rows 8 (4 j + w) .. + 7 (rows past M: the last one, never stored)
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    uint32_t rowoff[BMR];
+#pragma unroll
+    for (int j = 0; j < BMR; ++j)
+        rowoff[j] = (uint32_t)(min(8 * (4 * j + w) + (lane >> 3), mrows - 1) * (int)a.ldx * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+    const char* xbase = reinterpret_cast<const char*>(a.x + (int64_t)m0 * a.ldx);
+    auto x_load = [&](int step, int buf) {
+        const char* xb = xbase + (int64_t)min(ks0 + step, ksteps - 1) * 128;
+        PIN_SGPR(xb);
+#pragma unroll
+        for (int j = 0; j < BMR; ++j)
+            tall_x_to_lds(xb, rowoff[j], __builtin_amdgcn_readfirstlane(lds0 + buf * (BM * 128) + (4 * j + w) * 1024));
+    };
+
+    uint32_t EXr = 0x64006400u, M0r = 0x000F000Fu, M1r = 0x00F000F0u;
+    asm volatile("" : "+v"(EXr));
+    asm volatile("" : "+s"(M0r), "+s"(M1r));
+    f32x16 acc[TW][BMR];
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int rb = 0; rb < BMR; ++rb) acc[t][rb] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    // A fragment of slice i, row block rb: row 32 rb + lane % 32, piece i + 4 (lane / 32)
+    uint32_t apos[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) apos[i] = (uint32_t)((lane & 31) * 128 + ((i + 4 * (lane >> 5)) ^ (lane & 7)) * 16);
+
+    x_load(0, 0);
+    x_load(1, 1);
+    x_load(2, 2);
+    u32x4 wq[TALL_RING][TW];
+    uint32_t szr[TALL_RING][TW];
+#pragma unroll
+    for (int s = 0; s < TALL_RING; ++s)
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            szr[s][t] = sz_at(t, ks0 + s);
+            wq[s][t] = w_at(t, ks0 + s);
+        }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+
+    f16x8 b[2][TW], av[2][BMR];
+    auto dequant = [&](f16x8 (&dst)[TW], const u32x4 (&q)[TW], const uint32_t (&sz)[TW], int i) {
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const f16x2 szh = __builtin_bit_cast(f16x2, sz[t]);
+            const f16 zd1 = (f16)960.f - szh[1];
+            dst[t] = gptq::dequant8(q[t][i], f16x2{szh[1], szh[1]}, f16x2{zd1, zd1}, f16x2{szh[0], szh[0]}, EXr, M0r, M1r);
+        }
+    };
+    auto read_a = [&](f16x8 (&dst)[BMR], int buf, int i) {
+#pragma unroll
+        for (int rb = 0; rb < BMR; ++rb) dst[rb] = ld16<f16x8>(smem + buf * (BM * 128) + rb * 4096 + apos[i]);
+    };
+    read_a(av[0], 0, 0);
+    dequant(b[0], wq[0], szr[0], 0);
+    auto step = [&](int s, auto slot_) {
+        constexpr int SL = decltype(slot_)::value;
+        constexpr int NX = (SL + 1) % TALL_RING;
+        x_load(s + 3, (SL + 3) % TALL_RING);  // everyone is done with that buffer since the barrier of the step before
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            read_a(av[(i + 1) & 1], i < 3 ? SL : NX, (i + 1) & 3);
+            __builtin_amdgcn_sched_barrier(0);
+            if (i == 3) {
+#pragma unroll
+                for (int t = 0; t < TW; ++t) {
+                    wq[SL][t] = w_at(t, ks0 + s + TALL_RING);
+                    szr[SL][t] = sz_at(t, ks0 + s + TALL_RING);
+                }
+                dequant(b[0], wq[NX], szr[NX], 0);
+            } else {
+                dequant(b[(i + 1) & 1], wq[SL], szr[SL], i + 1);
+            }
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int t = 0; t < TW; ++t) acc[t][rb] = mfma32(av[i & 1][rb], b[i & 1][t], acc[t][rb]);
+            // a slice's 13 TW dequantisation instructions between its BMR TW products
+#pragma unroll
+            for (int g = 0; g < BMR * TW; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (13 * TW + BMR * TW - 1) / (BMR * TW), 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the x loads of step s + 2 were issued a step ago: behind them this wave has asked for that step's 2 TW weights and scales
+        // and for everything of this step
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BMR + 4 * TW) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    for (int s = 0;;) {
+        step(s, std::integral_constant<int, 0>{});
+        if (++s == n) break;
+        step(s, std::integral_constant<int, 1>{});
+        if (++s == n) break;
+        step(s, std::integral_constant<int, 2>{});
+        if (++s == n) break;
+        step(s, std::integral_constant<int, 3>{});
+        if (++s == n) break;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
+
+    // ---- epilogue: lane holds rows m = 32 rb + (r & 3) + 8 (r >> 2) + 4 (lane >> 5) of column nt * 32 + (lane & 31) -----------
+    const int c = lane & 31;
+    auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
+    constexpr int BN = 128 * TW;
+    if (a.mode == 1) {
+        float* dst = a.scratch + ((int64_t)blockIdx.x * a.S + split) * (BM * BN) + w * (32 * TW) + c;
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(rb, r) * BN + t * 32] = acc[t][rb][r];
+        return;
+    }
+    if (a.mode == 2) {
+        const int64_t np = (int64_t)a.NT * 32;
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const int nt = nt_raw0 + t;
+            if (nt >= a.NT) break;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb) {
+                const int unit = row_block * BMR + rb;
+                if (unit * 32 >= a.M) continue;
+                float* sl = a.scratch + ((int64_t)(unit * a.S + split) * 32) * np + nt * 32 + c;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sl[(int64_t)(row_of(rb, r) - rb * 32) * np] = acc[t][rb][r];
+            }
+        }
+        return;
+    }
+    // finished: the tile goes through LDS so that rows leave in 16-byte pieces, 512 (256 with SiLU * up) contiguous bytes a row
+    constexpr int BO = ACT == 2 ? BN / 2 : BN, OS = BO + 8;
+    const int n_out = ACT == 2 ? a.N >> 1 : a.N, n0 = col_block * BO;
+    __syncthreads();
+    f16* tile_out = reinterpret_cast<f16*>(smem);  // [BM][OS]
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+        const int nt = min(nt_raw0 + t, a.NT - 1);
+        if (ACT == 2) {
+            // Lanes 0 - 15 of a half wave hold gate columns, 16 - 31 the matching up columns.  Swapping those rows of lanes between two
+            // accumulator rows gives every lane a (gate, up) pair: the lower lanes that of row r, the upper ones that of row r + 1.
+            const int half = a.N >> 1, j = nt * 16 + (c & 15);
+            const float bv = a.bias ? (float)a.bias[c < 16 ? j : half + j] : 0.f;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; r += 2) {
+                    const uint32_t v0 = __builtin_bit_cast(uint32_t, (float)(f16)(acc[t][rb][r] + bv));
+                    const uint32_t v1 = __builtin_bit_cast(uint32_t, (float)(f16)(acc[t][rb][r + 1] + bv));
+                    const auto p = __builtin_amdgcn_permlane16_swap(v0, v1, false, false);
+                    const uint32_t g0 = p[0], u0 = p[1];  // (a bit cast of a vector's element itself reads element 0)
+                    const float gate = __builtin_bit_cast(float, g0), up = __builtin_bit_cast(float, u0);
+                    const float sl = gate / (1.f + __expf(-gate));
+                    tile_out[(row_of(rb, r) + (c >> 4)) * OS + (w * TW + t) * 16 + (c & 15)] = (f16)((float)(f16)sl * up);
+                }
+        } else {
+            const float bv = a.bias ? (float)a.bias[nt * 32 + c] : 0.f;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) tile_out[row_of(rb, r) * OS + (w * TW + t) * 32 + c] = (f16)(acc[t][rb][r] + bv);
+        }
+    }
+    __syncthreads();
+    constexpr int PIECES = BO / 8;
+    for (int p = tid; p < mrows * PIECES; p += 256) {
+        const int m = p / PIECES, col = (p % PIECES) * 8;
+        if (n0 + col >= n_out) continue;  // (outputs come in whole groups of 16 columns)
+        const f16x8 v = *reinterpret_cast<const f16x8*>(tile_out + m * OS + col);
+        f16* o = a.out + (int64_t)(m0 + m) * a.ldo + n0 + col;
+        if (a.vec) {
+            st16(o, v);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = v[e];
+        }
+    }
+}
+
+// The tiles that were split over k: sum of a tile's S fp32 parts in fixed order, then what the kernel above does with an unsplit tile.
+// grid (four-column groups of a tile / 256, tiles); ACT 2: four (gate, up) pairs.
+template <int BM, int BN, int ACT>
+__global__ __launch_bounds__(256) void tall_finish_kernel(TallArgs a) {
+    constexpr int PER_ROW = ACT == 2 ? BN / 8 : BN / 4;
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    const int m = idx / PER_ROW, g = idx % PER_ROW;
+    const int tile = a.tile0 + blockIdx.y, col_block = tile % a.col_blocks, row = (tile / a.col_blocks) * BM + m;
+    if (m >= BM || row >= a.M) return;
+    const float* src = a.scratch + (int64_t)blockIdx.y * a.S * (BM * BN) + m * BN;
+    auto part_sum = [&](int col) {
+        f32x4 v = {0, 0, 0, 0};
+        for (int s = 0; s < a.S; ++s) v += *reinterpret_cast<const f32x4*>(src + (int64_t)s * (BM * BN) + col);
+        return v;
+    };
+    if (ACT == 2) {
+        const int t = g >> 2, c = (g & 3) * 4, j = (col_block * (BN / 32) + t) * 16 + c, half = a.N >> 1;
+        if (j >= half) return;
+        const f32x4 gate = part_sum(t * 32 + c), up = part_sum(t * 32 + 16 + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float mine = (float)(f16)(gate[e] + (a.bias ? (float)a.bias[j + e] : 0.f));
+            const float other = (float)(f16)(up[e] + (a.bias ? (float)a.bias[half + j + e] : 0.f));
+            a.out[(int64_t)row * a.ldo + j + e] = (f16)((float)(f16)(mine / (1.f + __expf(-mine))) * other);
+        }
+    } else {
+        const int n = col_block * BN + g * 4;
+        if (n >= a.N) return;
+        const f32x4 v = part_sum(g * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a.out[(int64_t)row * a.ldo + n + e] = (f16)(v[e] + (a.bias ? (float)a.bias[n + e] : 0.f));
+    }
+}
+
+// ---- how a GEMM is cut ----------------------------------------------------------------------------------------------------------
+constexpr int CUS = 256;
+constexpr int TKC = 2;  // k64-steps: granularity of the deferred form's splits
+
+struct TallPlan {
+    int BMR, TW;
+    int col_blocks, tiles;  // tiles of BM x 128 TW
+    int whole;              // leading tiles that are not split
+    int S, per;             // the others: splits, k64-steps per split
+};
+
+// us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip (several blocks on each; clocks drop under
+// the matrix cores' load).  Fitted to launches of 26 - 560 us at the 7B shapes, 260 - 3072 rows; the plans the model picks are within 8 %
+// of the best of the nine that were timed at each size.
+struct TallCost {
+    double alone, busy;
+};
+constexpr TallCost TALL_COST[3][2] = {{{0.39, 0.314}, {0.53, 0.64}}, {{0.45, 0.434}, {0.625, 0.82}}, {{0.50, 0.57}, {0.735, 0.99}}};
+
+// Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k.  One size does not do: 765 rows of
+// a 7B gate_up are 516 tiles of 128 x 256, two rounds and four tiles, which take a third round (187 us; 161 with the four split in
+// eight); a 7B qkv at that size is 768 tiles of 96 x 128, three whole rounds (86 us against 101 for 288 of 128 x 256).
+TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
+    const int64_t steps = K / 64, NT = cdiv64(N, 32);
+    TallPlan best{};
+    double best_us = 1e30;
+    for (int BMR = 2; BMR <= 4; ++BMR)
+        for (int TW = 1; TW <= 2; ++TW) {
+            const TallCost c = TALL_COST[BMR - 2][TW - 1];
+            const int64_t cb = cdiv64(NT, 4 * TW), tiles = cb * cdiv64(M, 32 * BMR), rounds = tiles / CUS, rest = tiles % CUS;
+            const double alone = 4.0 + steps * c.alone, busy = 1.5 + steps * c.busy, share = (double)rest / CUS;
+            for (int S = 1; S <= 16; ++S) {
+                const int64_t per = cdiv64(steps, S);
+                if (S > 1 && (rest == 0 || rest * S > CUS || per < 4)) break;
+                if ((S - 1) * per >= steps) continue;  // an empty last split
+                double us = rounds * busy;
+                if (S > 1)  // the splits, their fp32 tiles written and read, and the launch that adds them
+                    us += 4.0 + per * c.alone + 8.0 + 2.0 * rest * S * (32 * BMR) * (128 * TW) * 4 / 4e6;
+                else if (rounds == 0)
+                    us = alone + std::max(0.0, busy - alone) * share;
+                else
+                    us = std::max(alone, us + (rest ? busy * (0.55 + 0.45 * share) : 0.0));
+                if (us < best_us) {
+                    best_us = us;
+                    best = {BMR, TW, (int)cb, (int)tiles, (int)(S > 1 ? tiles - rest : tiles), S, (int)per};
+                }
+            }
+        }
+    if (const char* e = getenv("TGIS_TALL_PLAN")) {  // tuning hook: "BMR,TW,S" (S splits all tiles past the last whole round)
+        int b = 0, t = 0, S = 0;
+        if (sscanf(e, "%d,%d,%d", &b, &t, &S) == 3 && b >= 2 && b <= 4 && t >= 1 && t <= 2 && S >= 1 && S <= 16) {
+            const int64_t cb = cdiv64(NT, 4 * t), tiles = cb * cdiv64(M, 32 * b), per = cdiv64(steps, S);
+            if ((S - 1) * per < steps) best = {b, t, (int)cb, (int)tiles, (int)(S > 1 ? tiles - tiles % CUS : tiles), S, (int)per};
+        }
+    }
+    return best;
+}
+
+int64_t plan_scratch(const TallPlan& p) {
+    return p.whole < p.tiles ? (int64_t)(p.tiles - p.whole) * p.S * (32 * p.BMR) * (128 * p.TW) * 4 : 0;
+}
+
+template <int BMR, int ACT, int TW>
+int launch_blocks(const TallArgs& a, int tiles, int S, hipStream_t st) {
+    constexpr size_t ring = (size_t)TALL_RING * (32 * BMR) * 128, rows = (size_t)(32 * BMR) * ((ACT == 2 ? 64 : 128) * TW + 8) * 2;
+    constexpr size_t lds = ring > rows ? ring : rows;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gptq_gemm_tall_kernel<BMR, ACT, TW>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    TGIS_CHECK_HIP(attr);
+    hipLaunchKernelGGL((gptq_gemm_tall_kernel<BMR, ACT, TW>), dim3((unsigned)tiles, (unsigned)S), dim3(256), lds, st, a);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+template <int ACT>
+int launch_shape(const TallPlan& p, const TallArgs& a, int tiles, int S, hipStream_t st) {
+    switch (p.BMR * 10 + p.TW) {
+        case 21: return launch_blocks<2, ACT, 1>(a, tiles, S, st);
+        case 22: return launch_blocks<2, ACT, 2>(a, tiles, S, st);
+        case 31: return launch_blocks<3, ACT, 1>(a, tiles, S, st);
+        case 32: return launch_blocks<3, ACT, 2>(a, tiles, S, st);
+        case 41: return launch_blocks<4, ACT, 1>(a, tiles, S, st);
+        default: return launch_blocks<4, ACT, 2>(a, tiles, S, st);
+    }
+}
+
+template <int ACT>
+int launch_finish(const TallPlan& p, const TallArgs& a, int tiles, hipStream_t st) {
+#define TGIS_TALL_FINISH(B, W)                                                                                                         \
+    hipLaunchKernelGGL((tall_finish_kernel<32 * B, 128 * W, ACT>),                                                                     \
+                       dim3((unsigned)cdiv64((int64_t)32 * B * (128 * W) / (ACT == 2 ? 8 : 4), 256), (unsigned)tiles), dim3(256), 0, st, a)
+    switch (p.BMR * 10 + p.TW) {
+        case 21: TGIS_TALL_FINISH(2, 1); break;
+        case 22: TGIS_TALL_FINISH(2, 2); break;
+        case 31: TGIS_TALL_FINISH(3, 1); break;
+        case 32: TGIS_TALL_FINISH(3, 2); break;
+        case 41: TGIS_TALL_FINISH(4, 1); break;
+        default: TGIS_TALL_FINISH(4, 2); break;
+    }
+#undef TGIS_TALL_FINISH
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+TallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, int64_t K, int64_t N, int64_t groups, float* scratch) {
+    const PrepLayout p = prep_layout(K, N, groups);
+    const int64_t spg = K / groups / 64;
+    TallArgs a{};
+    a.x = (const f16*)x;
+    a.ldx = ldx;
+    a.prep = (const uint8_t*)prepared;
+    a.offB = p.offB;
+    a.M = (int)M;
+    a.K = (int)K;
+    a.N = (int)N;
+    a.NT = (int)p.NT;
+    a.KS = (int)p.KS;
+    a.G = (int)groups;
+    a.spg_shift = 30;
+    if (groups > 1)
+        for (a.spg_shift = 0; (1 << a.spg_shift) < spg; ++a.spg_shift) {}
+    a.scratch = scratch;
+    return a;
+}
+
+}  // namespace
+
+// Rows from which it replaces the 64-row streaming passes, and up to which it replaces dequantise + library GEMM (us, passes / tall):
+//   act 2:  7B gate_up 96 rows 46 / 37, 128 rows 47 / 40, 192 rows 69 / 49; 70B gate_up 96 rows 176 / 105, 256 rows 364 / 232
+//   act 0:  7B qkv 128 rows 26 / 32, 192 rows 47 / 36; o 128 rows 15 / 17, 192 rows 19 / 20; down 128 rows 27 / 25, 192 rows 43 / 32;
+//           70B down 128 rows 81 / 71, 256 rows 151 / 124
+// (library with its dequantisation / tall, the four GEMMs of a 7B layer) 3072 rows 1296 / 1159, 6000 rows 2418 / 2184, 8192 rows
+// 2979 / 2993, 16128 rows 5542 / 5947: past 8192 rows hipBLASLt's 256 x 256 tiles, free of dequantisation, win (1.28 against 1.13 PFLOP/s).
+int64_t gptq::tall_min_m(int act) {
+    static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 0;
+    return v ? v : act == 2 ? 65 : 129;
+}
+int64_t gptq::tall_max_m() {
+    static const int64_t v = getenv("TGIS_TALL_MAX_M") ? atoll(getenv("TGIS_TALL_MAX_M")) : 8192;
+    return v;
+}
+bool gptq::tall_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act) {
+    if (M < tall_min_m(act) || perm != nullptr || act == 1 || K % 64 != 0) return false;
+    const int64_t gs = K / groups, spg = gs / 64;
+    return groups == 1 || (gs % 64 == 0 && (spg & (spg - 1)) == 0);
+}
+bool gptq::tall_partial_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act) {
+    return M >= 257 && act == 0 && tall_ok(M, K, groups, perm, act);
+}
+int64_t gptq::tall_workspace_bytes(int64_t M, int64_t K, int64_t N) { return plan_scratch(plan_tall(M, K, N)); }
+
+int gptq::launch_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo, int64_t M, int64_t K,
+                      int64_t N, int64_t groups, int act, float* scratch, hipStream_t st) {
+    const TallPlan p = plan_tall(M, K, N);
+    TallArgs a = tall_args(x, ldx, prepared, M, K, N, groups, scratch);
+    a.bias = (const f16*)bias;
+    a.out = (f16*)out;
+    a.ldo = ldo;
+    a.vec = ldo % 8 == 0 && (uintptr_t)out % 16 == 0;
+    a.col_blocks = p.col_blocks;
+    a.per = (int)(K / 64);
+    a.S = 1;
+    if (p.whole > 0) {
+        const int rc = act == 2 ? launch_shape<2>(p, a, p.whole, 1, st) : launch_shape<0>(p, a, p.whole, 1, st);
+        if (rc != TGIS_OK) return rc;
+    }
+    if (p.whole < p.tiles) {
+        a.tile0 = p.whole;
+        a.per = p.per;
+        a.S = p.S;
+        a.mode = 1;
+        const int rc = launch_shape<0>(p, a, p.tiles - p.whole, p.S, st);  // (fp32 tiles: the same for both activations)
+        if (rc != TGIS_OK) return rc;
+        return act == 2 ? launch_finish<2>(p, a, p.tiles - p.whole, st) : launch_finish<0>(p, a, p.tiles - p.whole, st);
+    }
+    return TGIS_OK;
+}
+
+// The deferred form: every tile split alike, so that a consumer can sum the slabs by rows.
+int gptq::tall_partial_splits(int64_t M, int64_t K, int64_t N) {
+    const int64_t blocks = cdiv64(cdiv64(N, 32), 4) * cdiv64(M, 128), chunks = cdiv64(K / 64, TKC);
+    int64_t S = blocks < 384 ? std::min<int64_t>(std::min<int64_t>(chunks, 16), cdiv64(512, blocks)) : 1;
+    const int64_t per = cdiv64(chunks, S);
+    while (S > 1 && (S - 1) * per >= chunks) --S;
+    return (int)S;
+}
+int64_t gptq::tall_slab_bytes(int64_t M, int64_t N, int S) { return cdiv64(M, 32) * S * 32 * cdiv64(N, 32) * 32 * 4; }
+
+int gptq::launch_tall_partial(const void* x, int64_t ldx, const void* prepared, int64_t M, int64_t K, int64_t N, int64_t groups,
+                              float* slabs, hipStream_t st) {
+    TallArgs a = tall_args(x, ldx, prepared, M, K, N, groups, slabs);
+    const int64_t chunks = cdiv64(K / 64, TKC);
+    a.S = tall_partial_splits(M, K, N);
+    a.per = (int)(cdiv64(chunks, a.S) * TKC);
+    a.mode = 2;
+    a.col_blocks = (int)cdiv64(a.NT, 4);
+    return launch_blocks<4, 0, 1>(a, (int)(a.col_blocks * cdiv64(M, 128)), a.S, st);
+}

@@ -243,7 +243,8 @@ class Ex4bitLinearV2:
             if x.shape[0] <= self._fused_rows(2):
                 return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias, act=2)
             return native.act_mul(self._large_m(x), self.width // 2)
-        if partial and x.shape[0] <= native.PARTIAL_MAX_M and DEFER_REDUCE:
+        # past 128 rows the tall kernel finishes its own sums sooner than a consumer adds the slabs of 64-row passes
+        if partial and x.shape[0] <= (128 if self._fused_rows(act) > 256 else native.PARTIAL_MAX_M) and DEFER_REDUCE:
             return native.gptq_gemm_partial(x, self.q_handle, bias=self.bias, act=act)
         if x.shape[0] <= self._fused_rows(act):
             return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias, act=act)

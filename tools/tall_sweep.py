@@ -1,4 +1,4 @@
-"""GPTQ linear at M > 64: the tall fused kernel (default rule, one and two column tiles per wave) vs the 64-row streaming
+"""GPTQ linear at M > 64: the tall fused kernel (the plan it chooses, 128-row tiles of 128 and 256 columns) vs the 64-row streaming
 passes (TGIS_TALL_MIN_M=huge) vs dequantise + library GEMM, cfg3 shapes.  GPU time per call from a captured graph.  GPU box only."""
 import os
 import subprocess
@@ -34,8 +34,8 @@ for (K, N, act) in [(4096, 12288, 0), (4096, 4096, 0), (4096, 22016, 2), (11008,
         print(f"{mode:7s} K={K:5d} N={N:5d} act={act} M={M:5d}: {t*1e6:9.1f} us  {2*M*K*N/t/1e12:7.1f} TFLOP/s", flush=True)
 '''
 ms = sys.argv[1] if len(sys.argv) > 1 else "96,128,256,512,1024,2048,4096"
-for mode, env in (("tall", {"TGIS_TALL_MAX_M": "1000000"}), ("tall/1", {"TGIS_TALL_MAX_M": "1000000", "TGIS_TALL_TW": "1"}),
-                  ("tall/2", {"TGIS_TALL_MAX_M": "1000000", "TGIS_TALL_TW": "2"}),
+for mode, env in (("tall", {"TGIS_TALL_MAX_M": "1000000"}), ("tall/1", {"TGIS_TALL_MAX_M": "1000000", "TGIS_TALL_PLAN": "4,1,1"}),
+                  ("tall/2", {"TGIS_TALL_MAX_M": "1000000", "TGIS_TALL_PLAN": "4,2,1"}),
                   ("passes", {"TGIS_TALL_MIN_M": "1000000"}), ("lib", {"TGIS_TALL_MAX_M": "0"})):
     e = dict(os.environ, **env)
     m = ms if mode != "passes" else ",".join(x for x in ms.split(",") if int(x) <= 512)
