@@ -75,6 +75,109 @@ __device__ __forceinline__ T finish_out(float v, int gelu, float p0 = 0.f, float
     return t;
 }
 
+// The epilogue of accumulator registers [r0, r0 + NR) of tile nt, their k-sums complete in `fin` (rslot, rcos, rsin: ACT 3 only).
+template <typename T, int ACT, int MR, int NR, int RM, int RN>
+__device__ __forceinline__ void dense_finish(const DenseArgs& a, const float (&fin)[MR][NR], const int r0, const int nt, const int split,
+                                             const int mslab, const int m0, const int mrows, const int lane,
+                                             const int32_t (&rslot)[RM][RN], const T (&rcos)[RM][RN], const T (&rsin)[RM][RN]) {
+    const int c = lane & 31;
+    auto row_of = [&](int j) {
+        const int r = r0 + j;
+        return (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
+    };
+    if (ACT == 3) {
+        // rope image: a tile of a q / k head holds dims [16 t, 16 t + 16) in lanes c < 16 and their rotation partners
+        // rD/2 + [16 t, ..) in lanes c + 16; v heads keep 32 consecutive dims.  Sum (+ bias) rounded to T, rotated in
+        // fp32 (the arithmetic of rope_kv_kernel), q to `out`, k / v into their cache pages.  Host guarantees S == 1.
+        const int per = a.rD >> 5;
+        const int head = nt / per, tt = nt - head * per;
+        const bool roth = head < a.rH + a.rHkv;
+        const int d = roth ? ((c < 16) ? 16 * tt + c : (a.rD >> 1) + 16 * tt + (c - 16)) : 32 * tt + c;
+        const int col = head * a.rD + d;
+        const float bv = a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[col]) : 0.f;
+        T* kpool = reinterpret_cast<T*>(a.kpool);
+        T* vpool = reinterpret_cast<T*>(a.vpool);
+#pragma unroll
+        for (int mr = 0; mr < MR; ++mr)
+#pragma unroll
+            for (int j = 0; j < NR; ++j) {
+                const int m = mr * 32 + row_of(j);
+                const float mine = to_f32(from_f32<T>(fin[mr][j] + bv));
+                float o = mine;
+                if (roth) {
+                    const float other = __shfl_xor(mine, 16, 64);
+                    const float cf = to_f32(rcos[mr][j]), sf = to_f32(rsin[mr][j]);
+                    o = (c < 16) ? mine * cf - other * sf : other * sf + mine * cf;
+                }
+                const T oh = from_f32<T>(o);
+                if (m < mrows) {
+                    if (head < a.rH) {
+                        reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + col] = oh;
+                    } else {
+                        const int page = rslot[mr][j] >> 5, tok = rslot[mr][j] & 31;
+                        if (roth)
+                            kpool[((int64_t)page * a.rHkv + (head - a.rH)) * 32 * a.rD + k_off(tok, d, a.rD)] = oh;
+                        else
+                            vpool[((int64_t)page * a.rHkv + (head - a.rH - a.rHkv)) * 32 * a.rD + v_off(tok, d, a.rD)] = oh;
+                    }
+                }
+            }
+        return;
+    }
+    const int n = nt * 32 + c;
+    if (ACT == 2) {
+        const int half = a.N >> 1;
+        const int j2 = nt * 16 + (c & 15);
+        const int nsrc = (c < 16) ? j2 : half + j2;
+        const float bv = (a.bias && j2 < half) ? to_f32(reinterpret_cast<const T*>(a.bias)[nsrc]) : 0.f;
+#pragma unroll
+        for (int mr = 0; mr < MR; ++mr)
+#pragma unroll
+            for (int j = 0; j < NR; ++j) {
+                const float mine = to_f32(from_f32<T>(fin[mr][j] + bv));
+                const float other = __shfl_xor(mine, 16, 64);
+                const int m = mr * 32 + row_of(j);
+                if (c < 16 && j2 < half && m < mrows) {
+                    if (a.glu_limit > 0.f) {
+                        const float g = fminf(mine, a.glu_limit);
+                        const float u = fminf(fmaxf(other, -a.glu_limit), a.glu_limit);
+                        reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + j2] =
+                            from_f32<T>(g / (1.f + __expf(-a.glu_alpha * g)) * (u + 1.f));
+                    } else {
+                        float sl = mine / (1.f + __expf(-mine));
+                        reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + j2] =
+                            from_f32<T>(to_f32(from_f32<T>(sl)) * other);
+                    }
+                }
+            }
+        return;
+    }
+    if (a.S == 1 && !a.partial) {
+        if (n >= a.N) return;
+        const float bv = a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[n]) : 0.f;
+#pragma unroll
+        for (int mr = 0; mr < MR; ++mr)
+#pragma unroll
+            for (int j = 0; j < NR; ++j) {
+                const int m = mr * 32 + row_of(j);
+                if (m >= mrows) continue;
+                if (a.out_f32)
+                    reinterpret_cast<float*>(a.out)[(int64_t)(m0 + m) * a.ldo + n] = fin[mr][j] + bv;
+                else
+                    reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + n] =
+                        a.gelu == 4 ? gated_lookup_out<T>(fin[mr][j] + bv, m0 + m, n, a.row_ids, a.row_table, a.row_table_ld, a.row_col0, a.row_table_rows)
+                                    : finish_out<T>(fin[mr][j] + bv, a.gelu, a.act_p0, a.act_p1);
+            }
+    } else {
+#pragma unroll
+        for (int mr = 0; mr < MR; ++mr) {
+            float* sl = a.slabs + ((int64_t)((mslab * MR + mr) * a.S + split) * 32) * (a.NT * 32) + n;
+#pragma unroll
+            for (int j = 0; j < NR; ++j) sl[(int64_t)row_of(j) * (a.NT * 32)] = fin[mr][j];
+        }
+    }
+}
+
 // Same structure as gptq_gemm_unit without the dequantisation: a unit of TN*WK waves owns 32*TN columns x KR rows; wave
 // (tile wn, k-part wk) streams its tile's fragments over its own k-range (4 KiB per k64-step, two steps in flight,
 // refilled in place), each k-part group double-buffers 32x256 chunks of x through LDS and paces itself with an LDS
@@ -299,102 +402,7 @@ __device__ __forceinline__ void dense_gemm_unit(const DenseArgs& a, const int nt
                     }
                 }
             }
-        const int c = lane & 31;
-        auto row_of = [&](int j) {
-            const int r = wk * NR + j;
-            return (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-        };
-        if (ACT == 3) {
-            // rope image: a tile of a q / k head holds dims [16 t, 16 t + 16) in lanes c < 16 and their rotation partners
-            // rD/2 + [16 t, ..) in lanes c + 16; v heads keep 32 consecutive dims.  Sum (+ bias) rounded to T, rotated in
-            // fp32 (the arithmetic of rope_kv_kernel), q to `out`, k / v into their cache pages.  Host guarantees S == 1.
-            const int per = a.rD >> 5;
-            const int head = nt / per, tt = nt - head * per;
-            const bool roth = head < a.rH + a.rHkv;
-            const int d = roth ? ((c < 16) ? 16 * tt + c : (a.rD >> 1) + 16 * tt + (c - 16)) : 32 * tt + c;
-            const int col = head * a.rD + d;
-            const float bv = a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[col]) : 0.f;
-            T* kpool = reinterpret_cast<T*>(a.kpool);
-            T* vpool = reinterpret_cast<T*>(a.vpool);
-#pragma unroll
-            for (int mr = 0; mr < MR; ++mr)
-#pragma unroll
-                for (int j = 0; j < NR; ++j) {
-                    const int m = mr * 32 + row_of(j);
-                    const float mine = to_f32(from_f32<T>(fin[mr][j] + bv));
-                    float o = mine;
-                    if (roth) {
-                        const float other = __shfl_xor(mine, 16, 64);
-                        const float cf = to_f32(rcos[mr][j]), sf = to_f32(rsin[mr][j]);
-                        o = (c < 16) ? mine * cf - other * sf : other * sf + mine * cf;
-                    }
-                    const T oh = from_f32<T>(o);
-                    if (m < mrows) {
-                        if (head < a.rH) {
-                            reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + col] = oh;
-                        } else {
-                            const int page = rslot[mr][j] >> 5, tok = rslot[mr][j] & 31;
-                            if (roth)
-                                kpool[((int64_t)page * a.rHkv + (head - a.rH)) * 32 * a.rD + k_off(tok, d, a.rD)] = oh;
-                            else
-                                vpool[((int64_t)page * a.rHkv + (head - a.rH - a.rHkv)) * 32 * a.rD + v_off(tok, d, a.rD)] = oh;
-                        }
-                    }
-                }
-            return;
-        }
-        const int n = nt * 32 + c;
-        if (ACT == 2) {
-            const int half = a.N >> 1;
-            const int j2 = nt * 16 + (c & 15);
-            const int nsrc = (c < 16) ? j2 : half + j2;
-            const float bv = (a.bias && j2 < half) ? to_f32(reinterpret_cast<const T*>(a.bias)[nsrc]) : 0.f;
-#pragma unroll
-            for (int mr = 0; mr < MR; ++mr)
-#pragma unroll
-                for (int j = 0; j < NR; ++j) {
-                    const float mine = to_f32(from_f32<T>(fin[mr][j] + bv));
-                    const float other = __shfl_xor(mine, 16, 64);
-                    const int m = mr * 32 + row_of(j);
-                    if (c < 16 && j2 < half && m < mrows) {
-                        if (a.glu_limit > 0.f) {
-                            const float g = fminf(mine, a.glu_limit);
-                            const float u = fminf(fmaxf(other, -a.glu_limit), a.glu_limit);
-                            reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + j2] =
-                                from_f32<T>(g / (1.f + __expf(-a.glu_alpha * g)) * (u + 1.f));
-                        } else {
-                            float sl = mine / (1.f + __expf(-mine));
-                            reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + j2] =
-                                from_f32<T>(to_f32(from_f32<T>(sl)) * other);
-                        }
-                    }
-                }
-            return;
-        }
-        if (a.S == 1 && !a.partial) {
-            if (n >= a.N) return;
-            const float bv = a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[n]) : 0.f;
-#pragma unroll
-            for (int mr = 0; mr < MR; ++mr)
-#pragma unroll
-                for (int j = 0; j < NR; ++j) {
-                    const int m = mr * 32 + row_of(j);
-                    if (m >= mrows) continue;
-                    if (a.out_f32)
-                        reinterpret_cast<float*>(a.out)[(int64_t)(m0 + m) * a.ldo + n] = fin[mr][j] + bv;
-                    else
-                        reinterpret_cast<T*>(a.out)[(int64_t)(m0 + m) * a.ldo + n] =
-                            a.gelu == 4 ? gated_lookup_out<T>(fin[mr][j] + bv, m0 + m, n, a.row_ids, a.row_table, a.row_table_ld, a.row_col0, a.row_table_rows)
-                                        : finish_out<T>(fin[mr][j] + bv, a.gelu, a.act_p0, a.act_p1);
-                }
-        } else {
-#pragma unroll
-            for (int mr = 0; mr < MR; ++mr) {
-                float* sl = a.slabs + ((int64_t)((mslab * MR + mr) * a.S + split) * 32) * (a.NT * 32) + n;
-#pragma unroll
-                for (int j = 0; j < NR; ++j) sl[(int64_t)row_of(j) * (a.NT * 32)] = fin[mr][j];
-            }
-        }
+        dense_finish<T, ACT, MR, NR>(a, fin, wk * NR, nt, split, mslab, m0, mrows, lane, rslot, rcos, rsin);
         return;
     }
 }

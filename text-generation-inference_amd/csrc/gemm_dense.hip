@@ -9,6 +9,7 @@
 #include <type_traits>
 #include "common.h"
 #include "dense_gemm_body.h"
+#include "dense_wide_body.h"
 
 namespace {
 
@@ -57,6 +58,22 @@ using dense::DRS;
 using dense::plan_dense;
 using dense::dense_slab_bytes;
 
+// Where the kernel that asks for everything at once (dense_wide_body.h; WK = WIDE_WAVES in the plan) replaces the streaming one, for
+// outputs that leave finished (us, bf16, weights cold; streaming / this one):
+//   * act 0 of heads (512 tiles and more) at up to 16 rows, where an extra trip to memory shows: 4096 x 32000 at 1 / 11 rows 47.7 / 42.4,
+//     47.5 / 45.0; 2048 x 32000 at 16 rows 26.7 / 24.8; 6144 x 49152 at 1 row 106 / 96 (32 rows: 107 / 106 - 116)
+//   * act 2 at 33 - 64 rows of small models: 2048 x 11264 at 47 rows 18.0 / 15.0 (6144 x 24576 at 64 rows: 61 / 74)
+// A projection whose streaming plan splits k stays with it, so that it sums in the same order whether it leaves finished or as slabs
+// (2048 x 2048 at 16 rows: finished 7.5 / 5.9, as slabs 4.2 / 5.5).
+static DensePlan plan_finished(int64_t K, int64_t N, int64_t M, int act) {
+    const DensePlan stream = plan_dense(K, N, M, act);
+    if (M < 1 || M > 64 || K % 64 != 0) return stream;
+    const int64_t tiles = cdiv64(N, 32);
+    const DensePlan wide1{(int)K, 1, dense::WIDE_WAVES, 1, 1}, wide2{(int)K, 1, dense::WIDE_WAVES, 2, M > 32 ? 2 : 1};
+    if (act == 2) return M > 32 && K <= 2048 ? wide2 : stream;
+    return act != 0 || tiles < 512 || M > 16 ? stream : (K <= 2048 || M <= 4) ? wide1 : wide2;
+}
+
 // One workgroup = one unit of dense_gemm_body.h (block-wide barriers, plain loads and stores).
 template <typename T, int TN, int WK, int ACT, int MR, bool R16 = false>
 __global__ __launch_bounds__(64 * TN * WK) void dense_gemm_kernel(DenseArgs a) {
@@ -64,6 +81,11 @@ __global__ __launch_bounds__(64 * TN * WK) void dense_gemm_kernel(DenseArgs a) {
     dense::dense_gemm_unit<T, TN, WK, ACT, MR, R16>(a, blockIdx.x, blockIdx.y, blockIdx.z, smem);
 }
 
+template <typename T, int TN, int ACT, int MR, bool R16, int Q>
+__global__ __launch_bounds__(64 * dense::WIDE_WAVES) void dense_wide_kernel(DenseArgs a, int rows_lds) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    dense::dense_wide_unit<T, TN, ACT, MR, R16, Q>(a, blockIdx.x, blockIdx.y, blockIdx.z, rows_lds, smem);
+}
 
 // Sum the S split-K slabs in fixed order and emit the output (+bias); thread = (row, 4 columns).
 template <typename T>
@@ -119,11 +141,32 @@ static int launch_dense_variant(int mr, dim3 grid, size_t lds, hipStream_t st, c
     return launch_dense_one<T, TN, WK, ACT, 1>(grid, lds, st, a);
 }
 
+template <typename T, int TN, int ACT, int MR, bool R16, int Q>
+static int launch_wide(const DenseArgs& a, hipStream_t st) {
+    static const hipError_t attr = hipFuncSetAttribute((const void*)dense_wide_kernel<T, TN, ACT, MR, R16, Q>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    TGIS_CHECK_HIP(attr);
+    dim3 grid((unsigned)cdiv64(a.NT, TN), (unsigned)a.S, (unsigned)cdiv64(a.M, 32 * MR));
+    hipLaunchKernelGGL((dense_wide_kernel<T, TN, ACT, MR, R16, Q>), grid, dim3(64 * dense::WIDE_WAVES),
+                       dense::wide_lds_bytes(a.M, a.KR, TN, MR, R16, Q), st, a, dense::wide_rows_lds(a.M, MR));
+    return TGIS_OK;
+}
+// (the row counts and tiles per wave that plan_finished and plan_dense_rope choose)
+template <typename T>
+static int launch_wide_plan(const DenseArgs& a, int TN, int act, hipStream_t st) {
+    if (act == 3) return launch_wide<T, 1, 3, 1, true, 4>(a, st);
+    if (act == 2) return launch_wide<T, 2, 2, 2, false, 1>(a, st);
+    return TN == 2 ? launch_wide<T, 2, 0, 1, true, 4>(a, st) : launch_wide<T, 1, 0, 1, true, 4>(a, st);
+}
+
 template <typename T>
 static int launch_dense(const DenseArgs& a, const DensePlan& pl, int act, int64_t mslabs32, hipStream_t st) {
     dim3 grid((unsigned)cdiv64(a.NT, pl.TN), (unsigned)pl.S, (unsigned)cdiv64(mslabs32, pl.MR));
     const size_t lds = (size_t)pl.WK * 2 * 32 * pl.MR * DRS * sizeof(T) + 64;
     int rc = TGIS_EINVAL;
+    if (pl.WK == dense::WIDE_WAVES) {
+        rc = launch_wide_plan<T>(a, pl.TN, act, st);
+    } else {
 #define TGIS_DENSE_CASE(T_, W_)                                                        \
     if (pl.TN == T_ && pl.WK == W_)                                                    \
         rc = act == 3   ? launch_dense_variant<T, T_, W_, 3>(pl.MR, grid, lds, st, a)                                           \
@@ -138,6 +181,7 @@ static int launch_dense(const DenseArgs& a, const DensePlan& pl, int act, int64_
     TGIS_DENSE_CASE(4, 2);
     TGIS_DENSE_CASE(4, 4);
 #undef TGIS_DENSE_CASE
+    }
     if (rc != TGIS_OK) {
         tgis_set_error("tgis_dense_gemm: no kernel for plan TN=%d WK=%d", pl.TN, pl.WK);
         return rc;
@@ -244,7 +288,7 @@ extern "C" int tgis_dense_gemm(const void* x, int64_t ldx, const void* prepared,
     hipStream_t st = (hipStream_t)stream;
     const int gelu = act == 4 ? 1 : act == 5 ? 2 : 0;  // GELU of the finished sum: epilogue (unsplit) or split-K reduce
     if (gelu) act = 0;
-    DensePlan pl = plan_dense(K, N, M, act);
+    DensePlan pl = plan_finished(K, N, M, act);
     TGIS_CHECK_ARG(act != 2 || (!out_f32 && pl.S == 1), "tgis_dense_gemm: act 2 writes the model dtype, unsplit");
     TGIS_CHECK_ARG(!gelu || !out_f32, "tgis_dense_gemm: act 4 / 5 (GELU) write the model dtype");
     const int64_t need = tgis_dense_gemm_workspace_bytes(M, K, N);
@@ -267,7 +311,7 @@ extern "C" int tgis_dense_gemm_clamped_glu(const void* x, int64_t ldx, const voi
     TGIS_CHECK_ARG(out && limit > 0.f, "tgis_dense_gemm_clamped_glu: needs an output and a positive limit");
     if (M == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    DensePlan pl = plan_dense(K, N, M, 2);
+    DensePlan pl = plan_finished(K, N, M, 2);
     TGIS_CHECK_ARG(pl.S == 1, "tgis_dense_gemm_clamped_glu: the epilogue needs the unsplit plan");
     const int64_t need = tgis_dense_gemm_workspace_bytes(M, K, N);
     TGIS_CHECK_ARG(workspace && workspace_bytes >= need, "tgis_dense_gemm_clamped_glu: workspace too small (%ld < %ld)",
@@ -291,7 +335,7 @@ extern "C" int tgis_dense_gemm_xielu(const void* x, int64_t ldx, const void* pre
     TGIS_CHECK_ARG(out, "tgis_dense_gemm_xielu: null out");
     if (M == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    DensePlan pl = plan_dense(K, N, M, 0);
+    DensePlan pl = plan_finished(K, N, M, 0);
     const int64_t need = tgis_dense_gemm_workspace_bytes(M, K, N);
     TGIS_CHECK_ARG(workspace && workspace_bytes >= need, "tgis_dense_gemm_xielu: workspace too small (%ld < %ld)",
                    (long)workspace_bytes, (long)need);
@@ -313,7 +357,7 @@ extern "C" int tgis_dense_gemm_relu2(const void* x, int64_t ldx, const void* pre
     TGIS_CHECK_ARG(out, "tgis_dense_gemm_relu2: null out");
     if (M == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    DensePlan pl = plan_dense(K, N, M, 0);
+    DensePlan pl = plan_finished(K, N, M, 0);
     const int64_t need = tgis_dense_gemm_workspace_bytes(M, K, N);
     TGIS_CHECK_ARG(workspace && workspace_bytes >= need, "tgis_dense_gemm_relu2: workspace too small (%ld < %ld)", (long)workspace_bytes, (long)need);
     TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
@@ -334,7 +378,7 @@ extern "C" int tgis_dense_gemm_gelu_lookup(const void* x, int64_t ldx, const voi
     TGIS_CHECK_ARG(out && ids && table && col0 >= 0 && ld_table >= col0 + N && vocab > 0, "tgis_dense_gemm_gelu_lookup: bad arguments");
     if (M == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    DensePlan pl = plan_dense(K, N, M, 0);
+    DensePlan pl = plan_finished(K, N, M, 0);
     const int64_t need = tgis_dense_gemm_workspace_bytes(M, K, N);
     TGIS_CHECK_ARG(workspace && workspace_bytes >= need, "tgis_dense_gemm_gelu_lookup: workspace too small (%ld < %ld)",
                    (long)workspace_bytes, (long)need);
@@ -356,7 +400,13 @@ extern "C" int tgis_dense_gemm_gelu_lookup(const void* x, int64_t ldx, const voi
 static DensePlan plan_dense_rope(int64_t K, int64_t N, int64_t M) {
     DensePlan pl = plan_dense(K, N, M, 2);
     const int64_t tiles = cdiv64(N, 32);
-    if (M <= 32 && pl.WK == 4 && cdiv64(tiles, pl.TN) < 128) pl.TN = 1;
+    if (M <= 32 && pl.WK == 4 && cdiv64(tiles, pl.TN) < 128) {
+        pl.TN = 1;
+        // Up to 16 rows and K = 4096 every operand byte of a workgroup fits in flight at once (dense_wide_body.h): 2048 x 2560 at 1 / 8 / 16
+        // rows 6.3 -> 5.5, 6.7 -> 5.9, 6.9 -> 6.5 us; at 24 rows 7.7 / 7.4 and at 32 7.7 / 7.8; 4096 x 3072 at 8 rows 10.8 -> 9.5, at 32
+        // 12.4 / 13.1; 5120 x 3072 at 16 rows 13.6 / 14.4.
+        if (M <= 16 && K % 64 == 0 && K <= 4096) pl = {(int)K, 1, dense::WIDE_WAVES, 1, 1};
+    }
     return pl;
 }
 
