@@ -699,6 +699,12 @@ int tgis_moe_choose(const float* logits, int64_t T, int E, int k, int groups, in
 int tgis_relu2(const void* in, int64_t ld_in, void* out, int64_t ld_out, int64_t rows, int64_t C, int dtype, void* stream);
 int tgis_dense_gemm_relu2(const void* x, int64_t ldx, const void* prepared, void* out, int64_t ldo, int64_t M, int64_t K,
                           int64_t N, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* `groups` products in one launch: rows [g N_group, (g + 1) N_group) of one stacked weight (a plain image; the last group takes the rows
+ * that are left) times an input of their own, x + g x_group elements; out + g out_group elements takes group g's columns from 0 on.
+ * M <= 64, K a multiple of 64, N_group of 32, x_group of 8. */
+int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo, int64_t out_group,
+                           int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups, int dtype, void* stream);
 /* Matrix memory with exponential gates per (sequence, head), tokens in order (the running maximum m starts at 0):
  *   i = cap tanh((z_i + i_bias) / cap);  f = ln sigmoid(cap tanh((z_f + f_bias) / cap));  m' = max(f + m, i);
  *   S <- e^(f + m - m') S + e^(i - m') k v^T;  n likewise with k;  o = c S^T q / (max(|c n . q|, e^-m') + read_eps), c = q_scale;

@@ -86,3 +86,35 @@ def test_rope(gpu_device, K, H, Hkv, D, M):
     for a, b in ((q0[:, :H * D], q1[:, :H * D]), (pools[0], pools[2]), (pools[1], pools[3])):
         diff = (a.float() - b.float()).abs()
         assert float(diff.max()) <= scale and float((diff > 0).float().mean()) < 0.05
+
+
+# groups: one, and several with a last one that is whole / one ragged tile / several tiles
+@pytest.mark.parametrize("K,n_group,N,G", [(64, 32, 20, 1), (448, 96, 288, 3), (576, 64, 150, 3), (2048, 512, 2048 + 64, 5), (4160, 64, 4 * 64 + 33, 5)])
+@pytest.mark.parametrize("M", [1, 8, 15, 16, 17, 32, 33, 64])
+def test_groups(gpu_device, K, n_group, N, G, M):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(K + N + M)
+    dtype = torch.bfloat16 if M & 1 else torch.float16
+    eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    x, wt = torch.randn(G, M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) * 0.05).to(dtype)
+    w = native.DenseWeight(wt.to(gpu_device))
+    out = torch.full((G, M, n_group + 8), 7.0, dtype=dtype, device=gpu_device)
+    native.dense_gemm_groups(x.to(gpu_device), w, n_group, out)
+    for i in range(G):
+        rows = wt[i * n_group:(i + 1) * n_group]
+        want = x[i].double() @ rows.double().t()
+        assert ((out[i, :, :len(rows)].double().cpu() - want).abs() <= _bound(x[i], rows, eps)(want)).all(), i
+        assert (out[i, :, len(rows):] == 7.0).all()
+        # a group as a weight of its own
+        part = w.rows(i * n_group, len(rows))
+        y = native.dense_gemm(x[i].to(gpu_device), part, native.Workspace(part.workspace_bytes(M), gpu_device))
+        assert ((y.double().cpu() - want).abs() <= _bound(x[i], rows, eps)(want)).all(), i
+
+
+def test_groups_refuses(gpu_device):
+    from tgis_amd import native
+
+    w = native.DenseWeight(torch.zeros(96, 72, dtype=torch.float16, device=gpu_device))
+    with pytest.raises(RuntimeError, match="multiple of 64"):
+        native.dense_gemm_groups(torch.zeros(3, 4, 72, dtype=torch.float16, device=gpu_device), w, 32, torch.zeros(3, 4, 32, dtype=torch.float16, device=gpu_device))

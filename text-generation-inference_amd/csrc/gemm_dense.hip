@@ -87,6 +87,20 @@ __global__ __launch_bounds__(64 * dense::WIDE_WAVES) void dense_wide_kernel(Dens
     dense::dense_wide_unit<T, TN, ACT, MR, R16, Q>(a, blockIdx.x, blockIdx.y, blockIdx.z, rows_lds, smem);
 }
 
+// Several inputs, each with weight rows of its own, stacked in one image: group g = tiles [g tiles, (g + 1) tiles), the last one what is left.
+template <typename T, int MR, bool R16, int Q>
+__global__ __launch_bounds__(64 * dense::WIDE_WAVES) void dense_groups_kernel(DenseArgs a, int rows_lds, int tiles, int groups, int64_t x_group,
+                                                                              int64_t out_group) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int g = min((int)blockIdx.x / tiles, groups - 1), first = g * tiles;
+    a.x = reinterpret_cast<const T*>(a.x) + g * x_group;
+    a.out = reinterpret_cast<T*>(a.out) + g * out_group;
+    a.prep += (int64_t)first * a.KS * 4096;
+    a.N = g + 1 < groups ? tiles * 32 : a.N - first * 32;
+    a.NT = (a.N + 31) >> 5;
+    dense::dense_wide_unit<T, 1, 0, MR, R16, Q>(a, blockIdx.x - first, 0, 0, rows_lds, smem);
+}
+
 // Sum the S split-K slabs in fixed order and emit the output (+bias); thread = (row, 4 columns).
 template <typename T>
 __global__ __launch_bounds__(256) void dense_splitk_reduce_kernel(const float* __restrict__ slabs,
@@ -392,6 +406,45 @@ extern "C" int tgis_dense_gemm_gelu_lookup(const void* x, int64_t ldx, const voi
     a.row_col0 = col0;
     a.row_table_rows = vocab;
     return dtype == TGIS_F16 ? launch_dense<f16>(a, pl, 0, cdiv64(M, 32), st) : launch_dense<bf16>(a, pl, 0, cdiv64(M, 32), st);
+}
+
+// ---- several projections of different inputs in one launch --------------------------------------------
+// At decode sizes a 2048 x 2048 projection is bounded by its own start: 5.4 us + 3.4 us of reduce launch for 8.4 MB.  Four of them and a
+// 64-column fifth side by side are enough tiles for every CU with k unsplit (bf16, us, five launches and their reduces / this one): 1 row
+// 33.8 / 9.5, 8 rows 36.2 / 10.2, 16 rows 36.2 / 11.1, 32 rows 38.0 / 14.7, 64 rows 46.5 / 20.7.
+template <typename T, int MR, bool R16, int Q>
+static int launch_groups(const DenseArgs& a, int groups, int tiles, int64_t x_group, int64_t out_group, hipStream_t st) {
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void*)dense_groups_kernel<T, MR, R16, Q>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    TGIS_CHECK_HIP(attr);
+    hipLaunchKernelGGL((dense_groups_kernel<T, MR, R16, Q>), dim3((unsigned)a.NT), dim3(64 * dense::WIDE_WAVES),
+                       dense::wide_lds_bytes(a.M, a.KR, 1, MR, R16, Q), st, a, dense::wide_rows_lds(a.M, MR), tiles, groups, x_group, out_group);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+template <typename T>
+static int launch_groups_rows(const DenseArgs& a, int groups, int tiles, int64_t x_group, int64_t out_group, hipStream_t st) {
+    if (a.M <= 16) return launch_groups<T, 1, true, 4>(a, groups, tiles, x_group, out_group, st);
+    return a.M <= 32 ? launch_groups<T, 1, false, 2>(a, groups, tiles, x_group, out_group, st)
+                     : launch_groups<T, 2, false, 1>(a, groups, tiles, x_group, out_group, st);
+}
+
+extern "C" int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo,
+                                      int64_t out_group, int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups, int dtype,
+                                      void* stream) {
+    int rc = dense_check(x, ldx, prepared, M, K, N, dtype, 0);
+    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(out && M <= 64 && K % 64 == 0 && x_group % 8 == 0, "tgis_dense_gemm_groups: up to 64 rows, K a multiple of 64");
+    TGIS_CHECK_ARG(N_group > 0 && N_group % 32 == 0 && groups >= 1 && N > (groups - 1) * N_group && N <= groups * N_group,
+                   "tgis_dense_gemm_groups: %ld columns do not make %ld groups of up to %ld", (long)N, (long)groups, (long)N_group);
+    if (M == 0) return TGIS_OK;
+    hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
+    DenseArgs a;
+    dense_fill(a, x, ldx, prepared, nullptr, out, ldo, M, K, N, 0, nullptr, 0, {(int)K, 1, dense::WIDE_WAVES, 1, M > 32 ? 2 : 1});
+    const int tiles = (int)(N_group / 32);
+    return dtype == TGIS_F16 ? launch_groups_rows<f16>(a, (int)groups, tiles, x_group, out_group, st)
+                             : launch_groups_rows<bf16>(a, (int)groups, tiles, x_group, out_group, st);
 }
 
 // ---- qkv projection with the rotary embedding and the cache write in its epilogue (dense weights) ---------------------

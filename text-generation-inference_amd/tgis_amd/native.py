@@ -183,6 +183,7 @@ SIGNATURES = {
     "tgis_narrow_product": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_int, _c_i64, _c_int, _vp]),
     "tgis_moe_choose": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_f, _vp, _vp, _vp]),
     "tgis_relu2": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
     "tgis_matrix_memory": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _vp, _c_i64, _vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp,
                                     _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_f, _c_f, _c_f, _c_int, _c_int, _vp]),
@@ -596,6 +597,28 @@ class DenseWeight:
 
     def workspace_bytes(self, M: int) -> int:
         return load_library().tgis_dense_gemm_workspace_bytes(M, self.K, self.N)
+
+    def rows(self, first: int, n: int) -> "DenseWeight":
+        """Weight rows [first, first + n) of a plain image, as a weight of their own that shares its memory (first a multiple of a tile)."""
+        assert not self.flags and first % 32 == 0 and 0 <= first and n > 0 and first + n <= self.N
+        part = object.__new__(DenseWeight)
+        part.N, part.K, part.dtype, part.flags = n, self.K, self.dtype, 0
+        part.image = self.image[first // 32 * ((self.K + 63) // 64) * 4096:]
+        return part
+
+
+GROUPS_MAX_M = 64
+
+
+def dense_gemm_groups(x: torch.Tensor, w: DenseWeight, n_group: int, out: torch.Tensor) -> torch.Tensor:
+    """out[g] = x[g] @ (rows [g n_group, (g + 1) n_group) of w)^T in one launch; x [G, M, K], out [G, M, >= n_group].  The last group has
+    the rows that are left and writes that many columns."""
+    G, M, K = x.shape
+    assert x.dtype == w.dtype == out.dtype and not w.flags and K == w.K and M <= GROUPS_MAX_M and x.stride(2) == out.stride(2) == 1
+    assert out.shape[:2] == (G, M) and out.shape[2] >= n_group and (G - 1) * n_group < w.N <= G * n_group
+    _check(load_library().tgis_dense_gemm_groups(_ptr(x), x.stride(1), x.stride(0), _ptr(w.image), _ptr(out), out.stride(1), out.stride(0), M, K,
+                                                 n_group, w.N, G, dtype_code(w.dtype), _stream()), "tgis_dense_gemm_groups")
+    return out
 
 
 def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f32: bool = False, act: int = 0,

@@ -6,6 +6,7 @@ Mirrors utils/layers.py of the reference: `FastLinear` (:104-111), the `get_line
 `PositionRotaryEmbedding` (:406-490); `Ex4bitLinearV2` mirrors utils/gptq/exllamav2.py:100-144.
 Every forward runs a kernel of libtgis_hip.so (decode-sized M) or, for prefill-sized M, a library GEMM
 on the same device; there is no CPU path."""
+import copy
 import math
 from typing import List, Optional
 
@@ -53,6 +54,14 @@ class FastLinear:
         self._gate_up = False
         self._rope_heads = None
         self.rope_handle: Optional[native.DenseWeight] = None
+
+    def rows(self, first: int, n: int) -> "FastLinear":
+        """Output columns [first, first + n) as a projection of their own on the same weight and image (first a multiple of 32)."""
+        assert self.bias is None and not self._gate_up and self._rope_heads is None
+        part = copy.copy(self)
+        part.weight, part.out_features = self.weight[first:first + n], n
+        part.prepared = self.prepared.rows(first, n) if self.streams else None
+        return part
 
     @property
     def gate_up(self) -> bool:

@@ -124,8 +124,16 @@ class WkvMixer:
         self.layer_id = layer_id
         self.H, self.d, self.eps = heads, dim, float(eps)
         self.mu = torch.stack([_f32(weights.get_tensor(f"{prefix}.mu.{s}")) for s in self.MIXES]).contiguous()
-        self.proj = [load_linear(weights, f"{prefix}.{s}") for s in ("r", "k", "v", "g")]
-        self.w1 = load_linear(weights, f"{prefix}.w1")
+        names, HD, rank = [f"{prefix}.{s}" for s in ("r", "k", "v", "g", "w1")], heads * dim, weights.get_tensor(f"{prefix}.w1").shape[0]
+        # decode-sized steps take the five projections, each of its own mix, in one launch on one stacked image
+        self.stacked = None
+        if HD % 32 == 0 and rank <= HD:
+            stacked = load_stacked_linear(weights, names)
+            self.proj, self.w1 = [stacked.rows(i * HD, HD) for i in range(4)], stacked.rows(4 * HD, rank)
+            if stacked.streams and stacked.in_features % 64 == 0:
+                self.stacked = stacked.prepared
+        else:
+            self.proj, self.w1 = [load_linear(weights, n) for n in names[:4]], load_linear(weights, names[4])
         self.w2t = _f32(weights.get_tensor(f"{prefix}.w2")).t().contiguous()  # [rank, H d]
         self.w0 = _f32(weights.get_tensor(f"{prefix}.w0"))
         self.u = _f32(weights.get_tensor(f"{prefix}.u")).reshape(-1)
@@ -140,10 +148,15 @@ class WkvMixer:
         mixes = native.token_shift_mix(h32, shift, step.state_slots, step.cu_seqlens_q, position_ids, self.mu, dtype)
         T = h32.shape[0]
         HD = self.H * self.d
-        rkvg = torch.empty((4, T, HD), dtype=dtype, device=h32.device)
-        for i, lin in enumerate(self.proj):
-            lin(mixes[i], out=rkvg[i])
-        logw = native.wkv_decay(self.w1(mixes[4]), self.w2t, self.w0)
+        rkvg = torch.empty((5, T, HD), dtype=dtype, device=h32.device)
+        if self.stacked is not None and T <= native.GROUPS_MAX_M:
+            native.dense_gemm_groups(mixes, self.stacked, HD, rkvg)
+            low = rkvg[4, :, :self.w1.out_features]
+        else:
+            for i, lin in enumerate(self.proj):
+                lin(mixes[i], out=rkvg[i])
+            low = self.w1(mixes[4])
+        logw = native.wkv_decay(low, self.w2t, self.w0)
         out = native.wkv_scan(rkvg[0], rkvg[1], rkvg[2], rkvg[3], logw, self.u, self.gain, state, shift, h32, step.state_slots,
                               step.cu_seqlens_q, position_ids, self.H, self.d, self.eps)
         return self.o(out, partial=self.defer)
