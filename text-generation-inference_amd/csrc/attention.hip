@@ -516,25 +516,6 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     }
 }
 
-static int next_pow2(int v) {
-    int p = 1;
-    while (p < v) p <<= 1;
-    return p;
-}
-
-struct AttnGeom {
-    int G, Gc, Gp, TQ, HC;
-};
-static AttnGeom geom(int H, int Hkv) {
-    AttnGeom g;
-    g.G = H / Hkv;
-    g.Gc = std::min(g.G, 16);
-    g.HC = (g.G + 15) / 16;
-    g.Gp = next_pow2(g.Gc);
-    g.TQ = 16 / g.Gp;
-    return g;
-}
-
 // Decode with fewer than 256 (sequence, kv head) groups: blocks of 8 waves that share one group's keys page by page
 // (and merge through LDS) instead of more key splits merged across blocks.
 static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && groups < 256; }
@@ -612,7 +593,7 @@ static int launch_attn(const AttnArgs& a, dim3 grid, int64_t total_q, hipStream_
 
 extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len, int64_t max_ctx) {
     if (B <= 0 || Hkv <= 0 || H <= 0 || H % Hkv != 0 || max_q_len != 1) return 1;  // splits: decode only
-    AttnGeom g = geom(H, Hkv);
+    AttnGeom g = attn_geom(H, Hkv);
     int64_t q_tiles = cdiv64(max_q_len, g.TQ);
     const int ch = chunks_per_block(g.HC, max_q_len);
     int64_t base = B * Hkv * cdiv64(g.HC, ch) * q_tiles;
@@ -656,7 +637,7 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
 
 // records of the fused combine: [group = (sequence, kv head, chunk block)][chunk][16 columns][split]
 static int64_t fused_records(int64_t B, int H, int Hkv, int num_splits) {
-    AttnGeom g = geom(H, Hkv);
+    AttnGeom g = attn_geom(H, Hkv);
     const int ch = chunks_per_block(g.HC, 1);
     return B * Hkv * cdiv64(g.HC, ch) * ch * 16 * num_splits;
 }
@@ -800,7 +781,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     (void)max_ctx;
     if (B == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    AttnGeom g = geom(H, Hkv);
+    AttnGeom g = attn_geom(H, Hkv);
     AttnArgs a;
     a.q = q;
     a.ld_q = ld_q;
@@ -812,15 +793,8 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     a.cu_q = cu_seqlens_q;
     a.out = out;
     a.out_frag = ld_out == TGIS_LD_FRAGMENTS;
-    a.H = H;
-    a.Hkv = Hkv;
-    a.G = g.G;
-    a.Gc = g.Gc;
-    a.Gp = g.Gp;
-    a.Gp_shift = 0;
-    while ((1 << a.Gp_shift) < g.Gp) ++a.Gp_shift;
-    a.TQ = g.TQ;
-    a.HC = g.HC;
+    a.ld_out = (int64_t)H * D;
+    attn_set_geom(a, H, Hkv, g);
     const int ch = chunks_per_block(g.HC, max_q_len);
     a.HCB = (g.HC + ch - 1) / ch;
     a.NS = num_splits;
@@ -849,7 +823,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     // long q (prefill): blocks of 128 columns that stage each K/V page once in LDS (attention_prefill.hip)
     if (num_splits == 1 && max_q_len * g.Gp > 64 && !getenv("TGIS_ATTN_NO_PREFILL_KERNEL")) {
         TgisTimedScope timed(TGIS_OP_ATTN, st);
-        return tgis_launch_attn_prefill(a, B, Hkv, D, max_q_len, dtype, st);
+        return tgis_launch_attn_prefill(a, B, Hkv, D, max_q_len, dtype, false, st);
     }
     int64_t q_tiles = cdiv64(max_q_len, g.TQ);
     TGIS_CHECK_ARG(q_tiles <= 2147483647LL && (int64_t)Hkv * a.HCB <= 65535 && B * num_splits <= 65535,

@@ -12,6 +12,7 @@ struct AttnArgs {
     const int32_t* ctx_lens;
     const int32_t* cu_q;
     void* out;
+    int64_t ld_out;  // prefill kernel: elements between two tokens' rows of `out`
     int out_frag;  // 1: out is [<= 32 tokens, H * D] in 32-row fragment order (xf_off in common.h), else row-major
     int H, Hkv, G, Gc, Gp, TQ, HC, NS;
     int Gp_shift;  // Gp is a power of two: column -> (q token, head of the group) by shift and mask, not by division
@@ -25,5 +26,31 @@ struct AttnArgs {
 
 constexpr float NEG_BIG = -1.0e30f;
 
-// prefill kernel launcher (attention_prefill.hip); `a` carries the geometry filled in by tgis_attn_paged
-int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, hipStream_t st);
+// How the heads of a kv group become MFMA columns: chunks of up to 16 heads, padded to a power of two, TQ q tokens per 16 columns.
+struct AttnGeom {
+    int G, Gc, Gp, TQ, HC;
+};
+static inline AttnGeom attn_geom(int H, int Hkv) {
+    AttnGeom g;
+    g.G = H / Hkv;
+    g.Gc = g.G < 16 ? g.G : 16;
+    g.HC = (g.G + 15) / 16;
+    for (g.Gp = 1; g.Gp < g.Gc;) g.Gp *= 2;
+    g.TQ = 16 / g.Gp;
+    return g;
+}
+static inline void attn_set_geom(AttnArgs& a, int H, int Hkv, const AttnGeom& g) {
+    a.H = H;
+    a.Hkv = Hkv;
+    a.G = g.G;
+    a.Gc = g.Gc;
+    a.Gp = g.Gp;
+    a.Gp_shift = 0;
+    while ((1 << a.Gp_shift) < g.Gp) ++a.Gp_shift;
+    a.TQ = g.TQ;
+    a.HC = g.HC;
+}
+
+// prefill kernel launcher (attention_prefill.hip): q, pools, tables, out, scale and geometry of `a`; D 64 or 128; rows: the page layout
+// of attn_varlen.hip
+int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st);

@@ -13,6 +13,7 @@
 #include <stdlib.h>
 #include <algorithm>
 #include <type_traits>
+#include "attention_args.h"
 #include "common.h"
 #include "wave_dpp.h"
 
@@ -80,6 +81,10 @@ __device__ __forceinline__ int first_visible(const AttnExt& e, int pos) {
 }
 // key j of a query at position pos whose window / block starts at lo
 __device__ __forceinline__ bool key_visible(const AttnExt& e, int key, int pos, int lo) { return key <= pos && (key >= lo || key < e.keep_first); }
+// nothing beside causal softmax attention
+static inline bool plain(const AttnExt& e) {
+    return !e.r1 && !e.chunk && !e.gate && !e.window && !e.keep_first && !e.sink && e.out_scale == 1.f && e.softcap == 0.f && !e.turns;
+}
 // The pages (or 64-key chunks) a walk visits: the first `nkeep` units hold kept first positions, then it continues at unit `u0`.
 __device__ __forceinline__ int kept_units(const AttnExt& e, int u0, int unit) { return min((e.keep_first + unit - 1) / unit, u0); }
 __device__ __forceinline__ int walk_unit(int i, int nkeep, int u0) { return i < nkeep ? i : u0 + (i - nkeep); }
@@ -1289,6 +1294,28 @@ void launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void*
             (void)hipFuncSetAttribute((const void*)attn_varlen_mfma_kernel<T, DK16, DVT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     } else {
         gx = (unsigned)cdiv64(cdiv64(max_q_len * R, 32), nw);
+        // Plain causal attention at the widths of the paged prefill kernel runs there (attention_prefill.hip: pages by direct loads,
+        // softmax and products of neighbouring pages overlapped).  us, staged or direct
+        // below / there: 4 x 1024 tokens, 32 heads on 4, dk 64: 173 / 47; 32 on 32, dk 128: 255 / 93; 4 x 300, 32 on 8, dk 128: 40 / 20;
+        // 24 x 60, dk 64: 12.7 / 9.9; 16 x 30: 9.3 / 9.4.
+        if (plain(ext) && dk == dv && (dk == 64 || dk == 128) && (int64_t)B * G * cdiv64(R, 16) * cdiv64(max_q_len, 8) <= 2147483647LL &&
+            (int64_t)G * cdiv64(R, 16) <= 65535) {
+            AttnArgs a{};
+            a.q = q;
+            a.ld_q = ldq;
+            a.kpool = k_pool;
+            a.vpool = v_pool;
+            a.bt = bt;
+            a.max_pages = bt_ld;
+            a.ctx_lens = ctx_lens;
+            a.cu_q = cu_q;
+            a.out = out;
+            a.ld_out = ld_out;
+            a.scale_log2 = scale * 1.4426950408889634f;
+            attn_set_geom(a, H, G, attn_geom(H, G));
+            (void)tgis_launch_attn_prefill(a, B, G, dk, max_q_len, std::is_same<T, f16>::value ? TGIS_F16 : TGIS_BF16, true, st);
+            return;
+        }
         // Measured (4 x 1024-token prompts): staging wins for narrow heads (dk 64 / dv 64, R 8: 2.96 ms against 3.20 for 22 layers)
         // and loses for wide ones (dk 128 / dv 128, MHA: 10.4 against 8.4 ms for 32 layers: two barriers per page and one LDS
         // buffer cost more than the second trip to L1 saves), so wide heads keep taking their fragments straight from L2 / L1.
