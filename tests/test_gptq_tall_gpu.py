@@ -58,3 +58,21 @@ def test_linear_takes_whole_sums_past_128_rows(gpu_device):
         if M > 128:
             want = x.double() @ ops_ref.gptq_dequant(qw, qz, sc, gi, 128).half().double()
             assert ((got.double().cpu() - want).abs() <= 2.0 ** -10 * want.abs() + 1e-5).all()
+
+
+# K: half a k64-step, whole ones, a ragged last; N: one tile, a block of eight and ragged ones; groups shorter than a step
+@pytest.mark.parametrize("K,N,groupsize", [(32, 32, 32), (96, 288, 32), (256, 256, 128), (320, 544, 64), (160, 1024, 160)])
+@pytest.mark.parametrize("image", ["plain", "gate_up", "rope"])
+def test_dequant_bits(gpu_device, K, N, groupsize, image):
+    """The image back to [K, N]: the bits of the reference formula, from each column order, into aligned and unaligned memory."""
+    from tgis_amd import native
+
+    qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, groupsize, seed=K + N)
+    kind = {"gate_up": {"gate_up": True}, "rope": {"rope": (32, max(1, N // 32 - 1))}}.get(image, {})
+    w = native.GptqWeight(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), 4, groupsize, **kind)
+    want = ops_ref.gptq_dequant(qw, qz, sc, gi, groupsize).half()
+    assert torch.equal(native.gptq_dequant(w).cpu(), want)
+    buf = torch.full((K * N + 2,), 7.0, dtype=torch.float16, device=gpu_device)
+    lib = native.load_library()
+    assert lib.tgis_gptq_dequant_f16(w.image.data_ptr(), buf.data_ptr() + 2, K, N, w.groups, w.flags, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(buf[1:-1].view(K, N).cpu(), want) and buf[0] == 7.0 and buf[-1] == 7.0

@@ -180,27 +180,48 @@ int gptq::reduce_slabs(const float* slabs, const f16* bias, f16* out, int64_t ld
 
 namespace {
 
-__global__ void gptq_dequant_kernel(const uint8_t* __restrict__ prep, int64_t offB, f16* __restrict__ wout,
-                                    int K, int N, int G, int gs, int NT, int KS, int flags) {
-    // one thread per prepared int32 (8 k of one column)
-    int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)NT * KS * 256) return;
-    int i = idx & 3;
-    int l = (idx >> 2) & 63;
-    int64_t ks = (idx >> 8) % KS;
-    int64_t nt = (idx >> 8) / KS;
-    int n = (int)col_src(nt, l & 31, N, flags);
-    int k0 = (ks * 8 + (l >> 5) * 4 + i) * 8;
-    if (n >= N || k0 >= K) return;
-    uint32_t q = reinterpret_cast<const uint32_t*>(prep)[idx];
-    int g = min(k0 / gs, G - 1);
-    f16x2 szh = __builtin_bit_cast(f16x2, reinterpret_cast<const uint32_t*>(prep + offB)[(nt * G + g) * 32 + (l & 31)]);
-    float s = (float)szh[0];
-    float z = (float)szh[1] - 1024.f;
+// The image back to [K][N] f16.  A workgroup takes one k64-step of eight neighbouring tiles: a KiB per tile straight from the image, 32 k
+// of a column per lane, and through LDS, so that rows leave in 16-byte pieces, 512 contiguous bytes of a plain image (256 + 256 of a
+// gate | up one).  Bound by the bytes: one 2-byte store per value and lane it was bound by its stores (7B, us before / now: qkv 4096 x 12288 34 / 22, gate_up
+// 4096 x 22016 88 / 37, down 11008 x 4096 33 / 21).
+constexpr int DQ_TILES = 8, DQ_ROW = DQ_TILES * 32 + 8;
+__global__ __launch_bounds__(256) void gptq_dequant_kernel(const uint8_t* __restrict__ prep, int64_t offB, f16* __restrict__ wout, int K,
+                                                           int N, int G, int gs, int NT, int KS, int flags, int vec) {
+    __shared__ __attribute__((aligned(16))) f16 tile[64 * DQ_ROW];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int ksteps = (K + 63) >> 6, ks = blockIdx.x % ksteps, nt0 = blockIdx.x / ksteps * DQ_TILES;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        float v = ((float)((q >> (4 * j)) & 15u) - z) * s;
-        wout[(int64_t)(k0 + nib_src(j)) * N + n] = (f16)v;
+    for (int r = 0; r < DQ_TILES / 4; ++r) {
+        const int t = r * 4 + w, nt = nt0 + t;
+        if (nt >= NT) break;
+        const u32x4 q = *reinterpret_cast<const u32x4*>(prep + (((int64_t)nt * KS + ks) * 64 + lane) * 16);
+        const uint32_t* sz = reinterpret_cast<const uint32_t*>(prep + offB) + (int64_t)nt * G * 32 + (lane & 31);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int kk = (lane >> 5) * 32 + i * 8;
+            const uint32_t word = sz[min((ks * 64 + kk) / gs, G - 1) * 32];
+            const f16x2 szh = __builtin_bit_cast(f16x2, word);
+            const float s = (float)szh[0], z = (float)szh[1] - 1024.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                tile[(kk + nib_src(j)) * DQ_ROW + t * 32 + (lane & 31)] = (f16)(((float)((q[i] >> (4 * j)) & 15u) - z) * s);
+        }
+    }
+    __syncthreads();
+    for (int p = tid; p < 64 * DQ_TILES * 4; p += 256) {
+        // piece of a row: 8 columns of a tile; in images with pairs the first halves of the eight tiles, then the second ones
+        const int k = p / (DQ_TILES * 4), at = p % (DQ_TILES * 4);
+        const int t = flags & 3 ? (at >> 1) % DQ_TILES : at >> 2;
+        const int c = flags & 3 ? at / (DQ_TILES * 2) * 16 + (at & 1) * 8 : (at & 3) * 8;
+        if (nt0 + t >= NT || ks * 64 + k >= K) continue;
+        const f16x8 v = *reinterpret_cast<const f16x8*>(tile + k * DQ_ROW + t * 32 + c);
+        f16* o = wout + (int64_t)(ks * 64 + k) * N + col_src(nt0 + t, c, N, flags);
+        if (vec) {
+            st16(o, v);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = v[e];
+        }
     }
 }
 
@@ -668,10 +689,9 @@ extern "C" int tgis_gptq_dequant_f16(const void* prepared, void* w_out, int64_t 
     TGIS_CHECK_ARG(prepared && w_out && K > 0 && N > 0 && groups > 0 && K % groups == 0,
                    "tgis_gptq_dequant_f16: bad arguments");
     PrepLayout p = prep_layout(K, N, groups);
-    int64_t total = p.NT * p.KS * 256;
-    hipLaunchKernelGGL(gptq_dequant_kernel, dim3((unsigned)cdiv64(total, 256)), dim3(256), 0, (hipStream_t)stream,
-                       (const uint8_t*)prepared, p.offB, (f16*)w_out, (int)K, (int)N, (int)groups,
-                       (int)(K / groups), (int)p.NT, (int)p.KS, flags);
+    hipLaunchKernelGGL(gptq_dequant_kernel, dim3((unsigned)(cdiv64(p.NT, DQ_TILES) * cdiv64(K, 64))), dim3(256), 0, (hipStream_t)stream,
+                       (const uint8_t*)prepared, p.offB, (f16*)w_out, (int)K, (int)N, (int)groups, (int)(K / groups), (int)p.NT, (int)p.KS,
+                       flags, ((uintptr_t)w_out & 15) == 0 && N % 8 == 0);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
