@@ -168,7 +168,7 @@ static int launch_wide(const DenseArgs& a, hipStream_t st) {
 // (the row counts and tiles per wave that plan_finished and plan_dense_rope choose)
 template <typename T>
 static int launch_wide_plan(const DenseArgs& a, int TN, int act, hipStream_t st) {
-    if (act == 3) return launch_wide<T, 1, 3, 1, true, 4>(a, st);
+    if (act == 3) return a.M <= 16 ? launch_wide<T, 1, 3, 1, true, 4>(a, st) : launch_wide<T, 1, 3, 2, false, 1>(a, st);
     if (act == 2) return launch_wide<T, 2, 2, 2, false, 1>(a, st);
     return TN == 2 ? launch_wide<T, 2, 0, 1, true, 4>(a, st) : launch_wide<T, 1, 0, 1, true, 4>(a, st);
 }
@@ -460,6 +460,10 @@ static DensePlan plan_dense_rope(int64_t K, int64_t N, int64_t M) {
         // 12.4 / 13.1; 5120 x 3072 at 16 rows 13.6 / 14.4.
         if (M <= 16 && K % 64 == 0 && K <= 4096) pl = {(int)K, 1, dense::WIDE_WAVES, 1, 1};
     }
+    // 33 - 64 rows of small models (against the slab form and a rotary launch behind it): 2048 x 2560 at 33 / 47 / 64 rows 10.7 -> 9.1,
+    // 10.9 -> 9.9, 11.2 -> 11.0; 2048 x 6144 13.6 -> 11.3, 14.4 -> 13.0; 1024 x 3072 9.4 -> 7.5, 9.6 -> 8.7; but 4096 x 3072 14.0 / 14.8,
+    // 14.5 / 18.1, 4096 x 12288 27 / 32: a block's x outgrows what its few columns need.
+    if (M > 32 && M <= 64 && K % 64 == 0 && K <= 2048 && tiles >= 64 && tiles <= 256) pl = {(int)K, 1, dense::WIDE_WAVES, 1, 2};
     return pl;
 }
 

@@ -145,7 +145,7 @@ class FlashLlamaAttention:
             bias=config.attention_bias)
         self.o_proj = TensorParallelRowLinear.load(config, prefix=f"{prefix}.o_proj", weights=weights,
                                                    bias=config.attention_bias)
-        # int4 qkv: decode steps of up to 32 rows rotate q / k and write the cache in the GEMM epilogue
+        # steps of up to 64 rows (where native.rope_gemm_ok) rotate q / k and write the cache in the GEMM epilogue, prompts included
         if hasattr(self.query_key_value.linear, "rope_heads"):
             self.query_key_value.linear.rope_heads = (self.num_heads, self.num_key_value_heads, self.head_size)
 
@@ -157,7 +157,7 @@ class FlashLlamaAttention:
         lin = self.query_key_value.linear
         rope_w = getattr(lin, "rope_handle", None)
         if isinstance(hidden_states, native.FragAct) or (
-                rope_w is not None and kv.slots is not None and not kv.fresh_prefill and kv.max_q_len == 1
+                rope_w is not None and kv.slots is not None
                 and (gathered or getattr(lin, "perm", None) is None) and hidden_states.shape[0] <= 64 and cos.shape[1] * 2 == D
                 and native.rope_gemm_ok(hidden_states.shape[0], rope_w, D)):
             # one launch: GEMM + rotary embedding + cache write (native.gptq_gemm_rope / native.dense_gemm_rope)
