@@ -249,13 +249,14 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _stream():
-    """hipStream_t of torch's current stream.  The raw getter skips the Stream object that
-    torch.cuda.current_stream() builds (a third of the host time of an eager decode step went there)."""
+    """hipStream_t of torch's current stream.  The raw getters skip the Stream object that torch.cuda.current_stream() builds and the
+    checks of torch.cuda.current_device() (a tensor on the device is there already): 0.9 -> 0.3 us per launch."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_device())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -584,6 +585,7 @@ class DenseWeight:
         assert weight.dim() == 2
         self.N, self.K = weight.shape
         self.dtype = weight.dtype
+        self.plans = {}  # rows -> scratch bytes / (slab bytes, S, ld) of the slab form, asked from the library once
         self.flags = 1 if gate_up else 0
         if rope is not None:  # (D, rotated heads): the image of a fused qkv projection for dense_gemm_rope
             assert not gate_up
@@ -596,13 +598,16 @@ class DenseWeight:
         torch.cuda.current_stream().synchronize()
 
     def workspace_bytes(self, M: int) -> int:
-        return load_library().tgis_dense_gemm_workspace_bytes(M, self.K, self.N)
+        got = self.plans.get(M)
+        if got is None:
+            got = self.plans[M] = load_library().tgis_dense_gemm_workspace_bytes(M, self.K, self.N)
+        return got
 
     def rows(self, first: int, n: int) -> "DenseWeight":
         """Weight rows [first, first + n) of a plain image, as a weight of their own that shares its memory (first a multiple of a tile)."""
         assert not self.flags and first % 32 == 0 and 0 <= first and n > 0 and first + n <= self.N
         part = object.__new__(DenseWeight)
-        part.N, part.K, part.dtype, part.flags = n, self.K, self.dtype, 0
+        part.N, part.K, part.dtype, part.flags, part.plans = n, self.K, self.dtype, 0, {}
         part.image = self.image[first // 32 * ((self.K + 63) // 64) * 4096:]
         return part
 
@@ -641,16 +646,18 @@ def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f3
 def dense_gemm_partial(x: torch.Tensor, w: DenseWeight, bias=None, act: int = 0) -> Partial:
     """Launch the dense GEMM but leave the split-K reduce (and bias) to the consumer kernel."""
     assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[0] <= PARTIAL_MAX_M
-    lib = load_library()
-    nbytes = lib.tgis_dense_gemm_partial_bytes(x.shape[0], w.K, w.N)
+    lib, M = load_library(), x.shape[0]
+    plan = w.plans.get(("slabs", M))
+    nbytes = plan[0] if plan is not None else lib.tgis_dense_gemm_partial_bytes(M, w.K, w.N)
     slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
-    S = _c_int()
-    ld = _c_i64()
+    S, ld = (None, None) if plan is not None else (_c_int(), _c_i64())
     _check(
-        lib.tgis_dense_gemm_partial(_ptr(x), x.stride(0), _ptr(w.image), x.shape[0], w.K, w.N, dtype_code(w.dtype), act,
-                                    _ptr(slabs), nbytes, ctypes.byref(S), ctypes.byref(ld), _stream()),
+        lib.tgis_dense_gemm_partial(_ptr(x), x.stride(0), _ptr(w.image), M, w.K, w.N, dtype_code(w.dtype), act, _ptr(slabs), nbytes,
+                                    None if S is None else ctypes.byref(S), None if ld is None else ctypes.byref(ld), _stream()),
         "tgis_dense_gemm_partial")
-    p = Partial(slabs, S.value, ld.value, x.shape[0], w.N, bias)
+    if plan is None:
+        plan = w.plans[("slabs", M)] = (nbytes, S.value, ld.value)
+    p = Partial(slabs, plan[1], plan[2], M, w.N, bias)
     p.dtype = w.dtype
     return p
 
