@@ -60,6 +60,36 @@ __device__ __forceinline__ uint32_t order_key(float x) {  // unsigned order == f
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+__device__ __forceinline__ float from_order_key(uint32_t k) {  // the float it is the key of
+    return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
+}
+
+// The bin of a 256-bin histogram that holds the `want`-th entry from above, and how many of its entries are wanted.  Called by one wave;
+// lane l sums bins 4 l .. + 3.  (Entry by entry it was a chain of up to 255 LDS reads: 8 us a pass.)
+__device__ __forceinline__ void bin_from_above(const int* hist, int want, int lane, uint32_t* out) {
+    int h[4], mine = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mine += h[e] = hist[lane * 4 + e];
+    int above = mine;  // entries in bins of this lane and those above it
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+        const int v = __shfl_down(above, o, 64);
+        above += lane + o < 64 ? v : 0;
+    }
+    int left = want - (above - mine);  // wanted below the bins of the lanes above
+    if (left > 0 && (left <= mine || lane == 0)) {
+        int bin = 3;
+#pragma unroll
+        for (int e = 3; e > 0; --e)
+            if (bin == e && h[e] < left) {
+                left -= h[e];
+                bin = e - 1;
+            }
+        out[0] = (uint32_t)(lane * 4 + bin);
+        out[1] = (uint32_t)left;
+    }
+}
+
 struct Block {
     float* fbuf;   // [NW]
     int* ibuf;     // [NW]
@@ -115,8 +145,8 @@ struct Block {
 
 __device__ __forceinline__ void philox_round(uint32_t (&c)[4], uint32_t k0, uint32_t k1) {
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
-    uint32_t hi0 = __umulhi(M0, c[0]), lo0 = M0 * c[0];
-    uint32_t hi1 = __umulhi(M1, c[2]), lo1 = M1 * c[2];
+    const uint64_t p0 = (uint64_t)M0 * c[0], p1 = (uint64_t)M1 * c[2];  // one multiplication each for both halves
+    const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0, hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
     uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
     c[0] = n0;
     c[1] = lo1;
@@ -326,6 +356,9 @@ __global__ __launch_bounds__(NT) void warp_sample_kernel(SampleArgs a) {
 // registers; the probabilities of the top-p / typical-p searches are computed once per search instead of once per bit.
 // Same per-thread element order, same expressions, same block reductions: bit-identical to warp_sample_kernel, which stays
 // for larger vocabularies.  (The global form re-read the 128 KB row from L2 ~80 times: 0.4 ms per step at V = 32000.)
+// One CU per row, so bound by its vector units and by the chain of reductions.  V = 32000, us, with 32 row masks and keys made anew for
+// every bit (82 registers in memory) and the histogram read bin by bin / now: greedy 26 / 17, a draw 51 / 38, top-k 50 64 / 37, top-p 0.9
+// 89 / 54, both and a draw 132 / 78, repetition penalty 36 / 21, everything 190 / 129.
 template <int NPT>
 __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
     __shared__ float fbuf[NW];
@@ -351,19 +384,28 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
         return x;
     };
     float x[NPT];
+    // Elements of this thread.  Each loop compares with a copy of its own (opaque): 32 row masks kept for all loops would not fit.
+    const int mine = (V - tid + NT - 1) / NT;
+    auto own_count = [&] {
+        int n = mine;
+        asm volatile("" : "+v"(n));
+        return n;
+    };
     const float pen = a.rep_penalty ? a.rep_penalty[b] : 1.0f;
     const bool scatter = pen != 1.0f && a.input_ids;
+    const int own1 = own_count();
 #pragma unroll
     for (int j = 0; j < NPT; ++j) {
         const int i = tid + j * NT;
-        x[j] = i < V ? adjusted(i) / T : NEG_INF;
+        x[j] = j < own1 ? adjusted(i) / T : NEG_INF;
     }
     if (scatter) {
         // the penalised entries go through the row in memory (any thread may hit any id), then come back into registers
+        const int own2 = own_count();
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
             const int i = tid + j * NT;
-            if (i < V) s[i] = x[j];
+            if (j < own2) s[i] = x[j];
         }
         __syncthreads();
         const int64_t* ids = a.input_ids + (int64_t)b * a.ld_ids;
@@ -375,10 +417,11 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
             s[id] = v / T;
         }
         __syncthreads();
+        const int own3 = own_count();
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
             const int i = tid + j * NT;
-            if (i < V) x[j] = s[i];
+            if (j < own3) x[j] = s[i];
         }
     }
 
@@ -391,23 +434,16 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
         for (int shift = 24; shift >= 0; shift -= 8) {
             for (int i = tid; i < 256; i += NT) hist[i] = 0;
             __syncthreads();
+            const int own4 = own_count();
 #pragma unroll
             for (int j = 0; j < NPT; ++j) {
-                if (tid + j * NT < V) {
+                if (j < own4) {
                     uint32_t key = order_key(x[j]);
                     if ((key & known) == prefix) atomicAdd(&hist[(key >> shift) & 255], 1);
                 }
             }
             __syncthreads();
-            if (tid == 0) {
-                int bin = 255, left = want;
-                for (; bin > 0; --bin) {
-                    if (hist[bin] >= left) break;
-                    left -= hist[bin];
-                }
-                bc[0] = (uint32_t)bin;
-                bc[1] = (uint32_t)left;
-            }
+            if (tid < 64) bin_from_above(hist, want, tid, bc);
             __syncthreads();
             prefix |= bc[0] << shift;
             known |= 255u << shift;
@@ -427,31 +463,34 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
         for (int j = 0; j < NPT; ++j) m = fmaxf(m, x[j]);
         m = blk.max(m);
         float z = 0.f;
+        const int own5 = own_count();
 #pragma unroll
         for (int j = 0; j < NPT; ++j)
-            if (tid + j * NT < V) z += expf(x[j] - m);
+            if (j < own5) z += expf(x[j] - m);
         z = blk.sum(z);
         const float inv_z = 1.0f / z;
-        float p[NPT];  // (the keys are three operations away from x: recomputed per bit, the registers go to p)
+        float p[NPT];
+        uint32_t key[NPT];  // in x's place: a bit of the search is a comparison, a selection and an addition per element
+        const int own6 = own_count();
 #pragma unroll
-        for (int j = 0; j < NPT; ++j) p[j] = tid + j * NT < V ? expf(x[j] - m) * inv_z : 0.f;
+        for (int j = 0; j < NPT; ++j) {
+            p[j] = j < own6 ? expf(x[j] - m) * inv_z : 0.f;
+            key[j] = order_key(x[j]);
+            asm volatile("" : "+v"(key[j]));  // (kept, not made again from x for every bit)
+        }
         uint32_t t = 0;
 #pragma unroll 1
         for (int bit = 31; bit >= 0; --bit) {
             const uint32_t cand = t | (1u << bit);
             float acc = 0.f;
-            uint32_t zb = 0;
-            asm volatile("" : "+v"(zb));  // an opaque zero: keeps the 32 keys from being hoisted out of the bit loop (registers)
 #pragma unroll
-            for (int j = 0; j < NPT; ++j)
-                if (order_key(__uint_as_float(__float_as_uint(x[j]) | zb)) <= cand) acc += p[j];  // p is 0 beyond the row
+            for (int j = 0; j < NPT; ++j) acc += key[j] <= cand ? p[j] : 0.f;  // p is 0 beyond the row
             if (blk.sum(acc) <= cut) t = cand;
         }
         const uint32_t top = order_key(m);  // min_tokens_to_keep = 1
         if (t >= top) t = top - 1;
 #pragma unroll
-        for (int j = 0; j < NPT; ++j)
-            if (order_key(x[j]) <= t) x[j] = NEG_INF;
+        for (int j = 0; j < NPT; ++j) x[j] = key[j] <= t ? NEG_INF : from_order_key(key[j]);
     }
 
     // ---- typical-p ------------------------------------------------------------------------------------------------
@@ -462,15 +501,17 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
         for (int j = 0; j < NPT; ++j) m = fmaxf(m, x[j]);
         m = blk.max(m);
         float z = 0.f;
+        const int own7 = own_count();
 #pragma unroll
         for (int j = 0; j < NPT; ++j)
-            if (tid + j * NT < V) z += expf(x[j] - m);
+            if (j < own7) z += expf(x[j] - m);
         z = blk.sum(z);
         const float log_z = m + logf(z), inv_z = 1.0f / z;
         float h = 0.f;
+        const int own8 = own_count();
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
-            if (tid + j * NT < V && x[j] != NEG_INF) {  // nansum: 0 * -inf terms are skipped
+            if (j < own8 && x[j] != NEG_INF) {  // nansum: 0 * -inf terms are skipped
                 float lp = x[j] - log_z;
                 h -= expf(lp) * lp;
             }
@@ -478,8 +519,9 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
         const float ent = blk.sum(h);
         auto dist_key = [&](float v) { return __float_as_uint(fabsf((log_z - v) - ent)); };  // >= 0: bits are ordered
         float p[NPT];
+        const int own9 = own_count();
 #pragma unroll
-        for (int j = 0; j < NPT; ++j) p[j] = tid + j * NT < V ? expf(x[j] - m) * inv_z : 0.f;
+        for (int j = 0; j < NPT; ++j) p[j] = j < own9 ? expf(x[j] - m) * inv_z : 0.f;
         uint32_t u = 0;
 #pragma unroll 1
         for (int bit = 31; bit >= 0; --bit) {
@@ -498,19 +540,21 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
     }
 
     // the warped scores are an output (top-n tokens and ranks read them); the chosen score is read back from them
+    const int own10 = own_count();
 #pragma unroll
     for (int j = 0; j < NPT; ++j) {
         const int i = tid + j * NT;
-        if (i < V) s[i] = x[j];
+        if (j < own10) s[i] = x[j];
     }
 
     // ---- choice + log-softmax of the warped scores at the chosen id ----------------------------------------------
     float m = NEG_INF;
     int mi = 0x7fffffff;
+    const int own11 = own_count();
 #pragma unroll
     for (int j = 0; j < NPT; ++j) {
         const int i = tid + j * NT;
-        if (i < V && (x[j] > m || (x[j] == m && i < mi))) {
+        if (j < own11 && (x[j] > m || (x[j] == m && i < mi))) {
             m = x[j];
             mi = i;
         }
@@ -518,9 +562,10 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
     blk.argmax(m, mi);
     if (mi >= V) mi = 0;  // a row of NaNs: no comparison ever succeeded
     float z = 0.f;
+    const int own12 = own_count();
 #pragma unroll
     for (int j = 0; j < NPT; ++j)
-        if (tid + j * NT < V) z += expf(x[j] - m);
+        if (j < own12) z += expf(x[j] - m);
     z = blk.sum(z);
     const float log_z = m + logf(z);
     int chosen = mi;
@@ -529,10 +574,12 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
         const uint64_t seed = a.rng[2 * b], offset = a.rng[2 * b + 1];
         float best = NEG_INF;
         int bi = 0x7fffffff;
+        const int own13 = own_count();
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
+            __builtin_amdgcn_sched_barrier(0);  // (one element's generator after another's: 32 of them side by side do not fit)
             const int i = tid + j * NT;
-            if (i >= V || x[j] == NEG_INF) continue;
+            if (j >= own13 || x[j] == NEG_INF) continue;
             float uu = ((float)philox_u32(seed, offset, (uint32_t)i) + 0.5f) * 2.3283064365386963e-10f;  // (0, 1]
             uu = fminf(uu, 0.99999994f);
             float g = (x[j] - m) - logf(-logf(uu));  // log(p_i / E_i) up to a constant
