@@ -26,7 +26,10 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
 // x either as a model-dtype tensor, or (PARTIAL) as S fp32 split-K slabs [S][32][slab_ld] whose sum (+xbias) is
 // rounded to the model dtype first — bit-identical to running the split-K reduce kernel and then this one.
 // NT threads per row: 256 in general, 512 for decode-sized batches (few rows: latency matters, not occupancy)
-template <typename T, bool RMS, bool PARTIAL, int NT>
+// ITERS: 8-element chunks per thread (the row in registers, the loops unrolled).  A decode step's norm is one round trip to memory and the
+// fetch of its own code, so a row gets the shortest form it fits (us before / now: 1040 x 4096 8.0 / 6.6,
+// 64 x 8192 in slabs of 4 7.75 / 7.64, 32 x 4096 4.09 / 4.03).  PERM: `perm` is given.
+template <typename T, bool RMS, bool PARTIAL, int NT, int ITERS, bool PERM>
 __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
                                                   const T* __restrict__ weight, const T* __restrict__ bias,
                                                   T* y, T* res_out, int hidden,
@@ -34,7 +37,7 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
                                                   const T* __restrict__ xbias, int y_frag,
                                                   const int32_t* __restrict__ perm) {
     using V8 = typename VecT<T>::x8;
-    constexpr int MAXV = MAX_HIDDEN / (NT * 8);
+    constexpr int MAXV = ITERS;
     __shared__ float sh[NT / 64];
     extern __shared__ __attribute__((aligned(16))) unsigned char norm_row[];  // the normed row, only where perm is given
     const int64_t row = blockIdx.x;
@@ -45,8 +48,7 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
     const int nchunk = hidden >> 3;  // hidden % 8 == 0
     float s1 = 0.f, s2 = 0.f;
     int src[8];  // where this thread's first gathered columns come from: asked for with the inputs too
-    const bool src_early = RMS && perm && (int)threadIdx.x < nchunk;
-    if (src_early) {
+    if (PERM && (int)threadIdx.x < nchunk) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) src[e] = perm[threadIdx.x * 8 + e];
     }
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
                 for (int e = 0; e < 8; ++e) o[e] = from_f32<T>((v[it][e] - mean) * rstd * to_f32(wv[e]));
             }
             // y_frag (RMSNorm in front of an int4 decode GEMM): 32-row fragment order, xf_off in common.h
-            if (RMS && perm)
+            if (PERM)
                 st16(reinterpret_cast<T*>(norm_row) + c * 8, o);
             else
                 st16(y + (y_frag ? xf_off(row, c * 8, hidden) : row * hidden + c * 8), o);
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
     // perm (in front of an act-order int4 GEMM): the normed row leaves gathered, y[k] = row[perm[k]].  The row goes through LDS: a
     // two-byte read per element at a random place is a few cycles per wave there (11 x 4096: 4.8 us with and without; 6.2 us when
     // the indices were only asked for after the reductions).
-    if (RMS && perm) {
+    if (PERM) {
         __syncthreads();
         const T* nr = reinterpret_cast<const T*>(norm_row);
         for (int c = threadIdx.x; c < nchunk; c += NT) {
@@ -184,16 +186,27 @@ static int launch_norm(const void* x, const void* residual, const void* weight, 
     TgisTimedScope timed(TGIS_OP_NORM, st);
     const bool wide = rows <= 64 && hidden >= 2048;
     const size_t lds = perm ? (size_t)hidden * 2 : 0;
-#define TGIS_NORM_LAUNCH(T, P)                                                                                   \
-    do {                                                                                                         \
-        if (wide)                                                                                                \
-            hipLaunchKernelGGL((norm_kernel<T, RMS, P, 512>), dim3((unsigned)rows), dim3(512), lds, st, (const T*)x, \
-                               (const T*)residual, (const T*)weight, (const T*)bias, (T*)y, (T*)res_out,         \
-                               (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag, perm);                    \
-        else                                                                                                     \
-            hipLaunchKernelGGL((norm_kernel<T, RMS, P, 256>), dim3((unsigned)rows), dim3(256), lds, st, (const T*)x, \
-                               (const T*)residual, (const T*)weight, (const T*)bias, (T*)y, (T*)res_out,         \
-                               (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag, perm);                    \
+#define TGIS_NORM_FORM(T, P, N, I, G)                                                                                                  \
+    hipLaunchKernelGGL((norm_kernel<T, RMS, P, N, I, G>), dim3((unsigned)rows), dim3(N), lds, st, (const T*)x, (const T*)residual,       \
+                       (const T*)weight, (const T*)bias, (T*)y, (T*)res_out, (int)hidden, eps, slabs, S, slab_ld, (const T*)xbias, y_frag, perm)
+#define TGIS_NORM_ROWS(T, P, N, I)                                                                                                     \
+    do {                                                                                                                               \
+        if constexpr (RMS) {                                                                                                           \
+            if (perm) {                                                                                                                \
+                TGIS_NORM_FORM(T, P, N, I, true);                                                                                      \
+                break;                                                                                                                 \
+            }                                                                                                                          \
+        }                                                                                                                              \
+        TGIS_NORM_FORM(T, P, N, I, false);                                                                                             \
+    } while (0)
+#define TGIS_NORM_LAUNCH(T, P)                                                                                                         \
+    do {                                                                                                                               \
+        if (wide && hidden <= 4096) TGIS_NORM_ROWS(T, P, 512, 1);                                                                      \
+        else if (wide && hidden <= 8192) TGIS_NORM_ROWS(T, P, 512, 2);                                                                 \
+        else if (wide) TGIS_NORM_ROWS(T, P, 512, MAX_HIDDEN / 4096);                                                                   \
+        else if (hidden <= 4096) TGIS_NORM_ROWS(T, P, 256, 2);                                                                         \
+        else if (hidden <= 8192) TGIS_NORM_ROWS(T, P, 256, 4);                                                                         \
+        else TGIS_NORM_ROWS(T, P, 256, MAX_HIDDEN / 2048);                                                                             \
     } while (0)
     if (dtype == TGIS_F16) {
         if (slabs) TGIS_NORM_LAUNCH(f16, true); else TGIS_NORM_LAUNCH(f16, false);
@@ -201,6 +214,8 @@ static int launch_norm(const void* x, const void* residual, const void* weight, 
         if (slabs) TGIS_NORM_LAUNCH(bf16, true); else TGIS_NORM_LAUNCH(bf16, false);
     }
 #undef TGIS_NORM_LAUNCH
+#undef TGIS_NORM_ROWS
+#undef TGIS_NORM_FORM
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
