@@ -399,6 +399,13 @@ int tgis_wkv_scan(const void* r, const void* k, const void* v, const void* gate,
                   const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
                   int64_t ld_out, int64_t B, int H, int d, float eps, int dtype, void* stream);
 
+/* tgis_wkv_decay of low [T, >= rank] (row stride ld_low) and tgis_wkv_scan in one launch, for steps in which sequences bring single
+ * tokens (any number works, one after another).  d a multiple of 4 up to 128, rank <= 1024; rows of r, k, v, gate and out are groups of
+ * four aligned elements, u, gain and state 16-byte aligned. */
+int tgis_wkv_step(const void* r, const void* k, const void* v, const void* gate, const void* low, int64_t ld, int64_t ld_low,
+                  const float* w2t, const float* w0, int rank, const float* u, const float* gain, float* state, float* shift_state,
+                  const float* h, int64_t W, const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
+                  int64_t ld_out, int64_t B, int H, int d, float eps, int dtype, void* stream);
 /* Mixture of experts, no host round trip.  Pairs p = t * k + j.  Rows of the grouped GEMMs live in tiles of tile_rows (32 or 128)
  * rows, one expert per tile; tgis_moe_row_capacity rows always suffice.  tgis_moe_tile_rows names the tile_rows a mixture of n_pairs
  * pairs over E experts of W -> ff -> W should use (128: long steps, f16 / bf16, inner widths that are multiples of 32). */

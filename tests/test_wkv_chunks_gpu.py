@@ -78,3 +78,49 @@ def test_token_shift_and_decay(gpu_device, W, dtype):
         lw = native.wkv_decay(dev(a), dev(w2t), dev(w0)).cpu().double()
         z = w0.double() + torch.tanh(a.double()) @ w2t.double()
         assert ((lw + z.exp()).abs() <= 1e-5 * (1 + z.exp())).all()
+
+
+# ranks: one, fewer than a thread's first load, exactly those, more; lens: single tokens, none, and a few one after another
+@pytest.mark.parametrize("d,rank", [(64, 64), (64, 5), (32, 1), (8, 70), (48, 200), (128, 32), (100, 129)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_step_with_its_decay(gpu_device, d, rank, dtype):
+    from tgis_amd import native
+
+    H, W, eps = 3, 300, 1e-4
+    lens = [1, 0, 1, 3, 1, 1]
+    fresh = [False, True, True, False, False, True]
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(d + rank)
+    r, k, v, gate = ((torch.randn(T, H, d, generator=g) * s).to(dtype) for s in (0.5, 0.5, 1.0, 1.0))
+    low = torch.randn(T, rank, generator=g).to(dtype)
+    w2t, w0 = torch.randn(rank, H * d, generator=g) * 0.3 * rank ** -0.5, torch.randn(H * d, generator=g) - 1.0
+    logw = -torch.exp(w0.double() + torch.tanh(low.double()) @ w2t.double()).view(T, H, d)
+    u, gain = torch.randn(H, d, generator=g) * 0.3, torch.rand(H, d, generator=g) + 0.5
+    state = torch.randn(B + 1, H, d, d, generator=g)
+    state[1::2, :, :, 0] = float("nan")  # what a fresh sequence's slot holds must not matter
+    slots = torch.tensor([0, 3, 1, 2, 4, 5], dtype=torch.int32)
+    fresh = [int(s) % 2 == 1 for s in slots]
+    h, shift = torch.randn(T, W, generator=g), torch.zeros(B + 1, W)
+    cu = torch.tensor([0] + lens).cumsum(0)
+    pos = torch.cat([torch.arange(n) + (0 if f else 7) for n, f in zip(lens, fresh)]).to(torch.int32)
+    dev = lambda t: t.to(gpu_device)
+    rows = lambda t: torch.nn.functional.pad(t.reshape(T, H * d), (0, 4)).to(gpu_device)[:, :H * d]
+    st, sh = dev(state).clone(), dev(shift)
+    got = native.wkv_step(rows(r), rows(k), rows(v), rows(gate), torch.nn.functional.pad(dev(low), (0, 3))[:, :rank], dev(w2t), dev(w0),
+                          dev(u.reshape(-1)), dev(gain.reshape(-1)), st, sh, dev(h), dev(slots), dev(cu.to(torch.int32)), dev(pos), H, d,
+                          eps).double().cpu().view(T, H, d)
+    for b, (n, f) in enumerate(zip(lens, fresh)):
+        a, e, slot = int(cu[b]), int(cu[b + 1]), int(slots[b])
+        if n == 0:
+            assert torch.equal(st[slot].cpu().nan_to_num(), state[slot].nan_to_num()) and not sh[slot].any()
+            continue
+        S0 = torch.zeros(H, d, d, dtype=torch.float64) if f else state[slot].double()
+        want, S = definition(*(t[a:e].double() for t in (r, k, v, gate, logw)), u.double(), gain.double(), S0, eps)
+        size = want.square().mean(-1, keepdim=True).sqrt()
+        # as above; the decay's exponent adds the fp32 sum of `rank` terms (2e-7 of its size per term at the most)
+        tol = 4e-5 * size + (0.0 if dtype == torch.float32 else 2.0 ** -8 * want.abs())
+        assert ((got[a:e] - want).abs() <= tol).all(), (b, float(((got[a:e] - want).abs() / size).max()))
+        got_S = st[slot].double().cpu()
+        assert (got_S - S).abs().max() <= 2e-5 * S.abs().max(), b
+        assert torch.equal(sh[slot].cpu(), h[e - 1])
+    assert torch.equal(st[B].cpu(), state[B])

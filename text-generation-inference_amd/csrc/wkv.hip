@@ -534,6 +534,143 @@ __global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
         }
 }
 
+// A decode step: the log-decay's second factor and the recurrence of the few tokens a sequence brings, in one launch.
+//
+// Bound by a chain of trips to memory (which sequence, its state and its rows, their answers) and the state's bytes; in the chunk kernel
+// above a single token paid for that kernel's size, 52 KiB of LDS and eight waves with three barriers' worth of staging, and the decay for
+// a launch of its own.  Here the state, the token's rows and the decay's weights are asked for together, each thread loads the rows of
+// r, k and u that its state rows need, and the waves meet three times.  24 sequences, 32 heads of 64, rank 64, us: 18.0 + 4.9 / 10.5.
+constexpr int STEP_THREADS = 256, STEP_WAVES = STEP_THREADS / 64, STEP_MAX_RANK = 1024;
+
+template <typename T, int D>
+__global__ __launch_bounds__(STEP_THREADS) void wkv_step_kernel(
+    const T* __restrict__ r, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ gate, const T* __restrict__ low,
+    int64_t ld, int64_t ld_low, const float* __restrict__ w2t, const float* __restrict__ w0, int R, const float* __restrict__ u,
+    const float* __restrict__ gain, float* __restrict__ state, float* __restrict__ shift_state, const float* __restrict__ h, int64_t W,
+    const int32_t* __restrict__ state_slots, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions, T* __restrict__ out,
+    int64_t ld_out, int H, int d, float eps) {
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    constexpr int L = D / 4, RG = STEP_THREADS / L, RPT = D / RG;  // lanes per state row, row groups, (neighbouring) rows per thread
+    constexpr int P = STEP_THREADS / D, EARLY = 16;                // parts of the decay's sum; weights a thread asks for at once
+    static_assert(RPT % 4 == 0, "rows of a thread come in fours");
+    __shared__ float th[STEP_MAX_RANK], part[P][D], bonus_of[STEP_WAVES];
+    __shared__ __attribute__((aligned(16))) float ww[D], o_of[STEP_WAVES][D];
+    const int b = blockIdx.x, head = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int t0 = cu_q[b], t1 = cu_q[b + 1];
+    const int64_t slot = state_slots[b];
+    if (t1 <= t0) return;
+    const int64_t col0 = (int64_t)head * d, C = (int64_t)H * d;
+    float* Sg = state + ((slot * H + head) * d) * (int64_t)d;  // [i][j]
+    const int c4 = (tid % L) * 4, i0 = tid / L * RPT;
+    const bool mine = c4 < d;
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    f32x4 St[RPT], u4[RPT / 4], r4[RPT / 4], k4[RPT / 4];
+#pragma unroll
+    for (int x = 0; x < RPT; ++x) St[x] = (mine && i0 + x < d) ? *reinterpret_cast<const f32x4*>(Sg + (int64_t)(i0 + x) * d + c4) : zero4;
+    auto wide4 = [](T4 x) -> f32x4 { return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; };
+    auto rows4 = [&](const T* p, int t, f32x4 (&dst)[RPT / 4]) {
+#pragma unroll
+        for (int y = 0; y < RPT / 4; ++y)
+            dst[y] = i0 + 4 * y < d ? wide4(*reinterpret_cast<const T4*>(p + (int64_t)t * ld + col0 + i0 + 4 * y)) : zero4;
+    };
+#pragma unroll
+    for (int y = 0; y < RPT / 4; ++y) u4[y] = i0 + 4 * y < d ? *reinterpret_cast<const f32x4*>(u + col0 + i0 + 4 * y) : zero4;
+    const f32x4 g4 = mine ? *reinterpret_cast<const f32x4*>(gain + col0 + c4) : zero4;
+    const int zc = tid % D, zp = tid / D, per = (R + P - 1) / P, za = zp * per, ze = min(R, za + per);  // this thread's part of the decay
+    float wz[EARLY];
+#pragma unroll
+    for (int e = 0; e < EARLY; ++e) wz[e] = (zc < d && za + e < ze) ? w2t[(int64_t)(za + e) * C + col0 + zc] : 0.f;
+    const float z0 = zc < d ? w0[col0 + zc] : 0.f;
+    if (positions[t0] == 0) {
+#pragma unroll
+        for (int x = 0; x < RPT; ++x) St[x] = zero4;
+    }
+    for (int t = t0; t < t1; ++t) {
+        rows4(r, t, r4);
+        rows4(k, t, k4);
+        f32x4 v4 = zero4, gt = zero4;
+        if (mine) {
+            v4 = wide4(*reinterpret_cast<const T4*>(v + (int64_t)t * ld + col0 + c4));
+            gt = wide4(*reinterpret_cast<const T4*>(gate + (int64_t)t * ld + col0 + c4));
+        }
+        for (int i = tid; i < R; i += STEP_THREADS) th[i] = tanhf((float)low[(int64_t)t * ld_low + i]);
+        __syncthreads();
+        float z = 0.f;
+#pragma unroll
+        for (int e = 0; e < EARLY; ++e) z += (za + e < ze ? th[za + e] : 0.f) * wz[e];
+        for (int i = za + EARLY; i < ze; ++i) z += zc < d ? th[i] * w2t[(int64_t)i * C + col0 + zc] : 0.f;
+        part[zp][zc] = z;
+        __syncthreads();
+        if (zp == 0) {
+            z = z0;
+#pragma unroll
+            for (int p = 0; p < P; ++p) z += part[p][zc];
+            ww[zc] = expf(-expf(z));
+        }
+        __syncthreads();
+        f32x4 o = zero4;
+        float bonus = 0.f;
+#pragma unroll
+        for (int y = 0; y < RPT / 4; ++y) {
+            const f32x4 w4 = *reinterpret_cast<const f32x4*>(&ww[i0 + 4 * y]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                f32x4& S = St[4 * y + e];
+                bonus += r4[y][e] * u4[y][e] * k4[y][e];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    o[c] += r4[y][e] * S[c];
+                    S[c] = w4[e] * S[c] + k4[y][e] * v4[c];
+                }
+            }
+        }
+#pragma unroll
+        for (int far = L; far < 64; far *= 2) {
+            bonus += __shfl_xor(bonus, far, 64);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o[c] += __shfl_xor(o[c], far, 64);
+        }
+        if (lane < L) *reinterpret_cast<f32x4*>(&o_of[wave][c4]) = o;
+        if (lane == 0) bonus_of[wave] = bonus;
+        __syncthreads();
+        if (wave == 0) {  // (its lanes past the first L repeat them)
+            o = zero4;
+            bonus = 0.f;
+#pragma unroll
+            for (int p = 0; p < STEP_WAVES; ++p) {
+                o += *reinterpret_cast<const f32x4*>(&o_of[p][c4]);
+                bonus += bonus_of[p];
+            }
+            float ss = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                o[c] += bonus * v4[c];
+                ss += o[c] * o[c];
+            }
+            ss = sum_neighbours<16>(ss);
+            if (L > 16) ss += __shfl_xor(ss, 16, 64);
+            if (lane < L && mine) {
+                const float rinv = 1.0f / sqrtf(ss / (float)d + eps);
+                T4 res;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) res[e] = (T)(o[e] * rinv * g4[e] * (gt[e] / (1.f + expf(-gt[e]))));
+                *reinterpret_cast<T4*>(out + (int64_t)t * ld_out + col0 + c4) = res;
+            }
+        }
+    }
+    if (mine) {
+#pragma unroll
+        for (int x = 0; x < RPT; ++x)
+            if (i0 + x < d) *reinterpret_cast<f32x4*>(Sg + (int64_t)(i0 + x) * d + c4) = St[x];
+    }
+    if (head == 0) {
+        const float* last = h + (int64_t)(t1 - 1) * W;
+        float* dst = shift_state + slot * W;
+        for (int64_t c = tid; c < W; c += STEP_THREADS) dst[c] = last[c];
+    }
+}
+
 template <typename T>
 int launch_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw, const float* u,
                 const float* gain, float* state, float* shift_state, const float* h, int64_t W, const int32_t* slots,
@@ -649,6 +786,41 @@ extern "C" int tgis_wkv_scan(const void* r, const void* k, const void* v, const 
         launch_scan<bf16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, st);
     else
         launch_scan<float>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, st);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+// rows of groups of four aligned elements, as the chunk form wants them; d <= 128, rank <= STEP_MAX_RANK
+extern "C" int tgis_wkv_step(const void* r, const void* k, const void* v, const void* gate, const void* low, int64_t ld, int64_t ld_low,
+                             const float* w2t, const float* w0, int rank, const float* u, const float* gain, float* state,
+                             float* shift_state, const float* h, int64_t W, const int32_t* state_slots, const int32_t* cu_seqlens_q,
+                             const int32_t* positions, void* out, int64_t ld_out, int64_t B, int H, int d, float eps, int dtype,
+                             void* stream) {
+    TGIS_CHECK_ARG(r && k && v && gate && low && w2t && w0 && u && gain && state && shift_state && h && state_slots && cu_seqlens_q &&
+                       positions && out,
+                   "tgis_wkv_step: null tensor");
+    TGIS_CHECK_ARG(B >= 1 && H >= 1 && H <= 65535 && d >= 4 && d <= 128 && d % 4 == 0 && rank >= 1 && rank <= STEP_MAX_RANK,
+                   "tgis_wkv_step: head width %d (multiples of 4 up to 128), rank %d (up to %d)", d, rank, STEP_MAX_RANK);
+    const uintptr_t four = dtype == TGIS_F32 ? 16 : 8;
+    TGIS_CHECK_ARG(dtype3(dtype) && ld >= (int64_t)H * d && ld_out >= (int64_t)H * d && ld_low >= rank && ld % 4 == 0 && ld_out % 4 == 0 &&
+                       ((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)gate | (uintptr_t)out) % four == 0 &&
+                       ((uintptr_t)u | (uintptr_t)gain | (uintptr_t)state) % 16 == 0 && W >= 1,
+                   "tgis_wkv_step: rows must be groups of four aligned elements");
+    hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_SCAN, st);
+#define TGIS_STEP(TT, DM)                                                                                                             \
+    hipLaunchKernelGGL((wkv_step_kernel<TT, DM>), dim3((unsigned)B, (unsigned)H), dim3(STEP_THREADS), 0, st, (const TT*)r, (const TT*)k, \
+                       (const TT*)v, (const TT*)gate, (const TT*)low, ld, ld_low, w2t, w0, rank, u, gain, state, shift_state, h, W,     \
+                       state_slots, cu_seqlens_q, positions, (TT*)out, ld_out, H, d, eps)
+#define TGIS_STEP_WIDTH(TT) do { if (d <= 64) TGIS_STEP(TT, 64); else TGIS_STEP(TT, 128); } while (0)
+    if (dtype == TGIS_F16)
+        TGIS_STEP_WIDTH(f16);
+    else if (dtype == TGIS_BF16)
+        TGIS_STEP_WIDTH(bf16);
+    else
+        TGIS_STEP_WIDTH(float);
+#undef TGIS_STEP_WIDTH
+#undef TGIS_STEP
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }

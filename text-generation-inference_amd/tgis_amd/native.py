@@ -106,6 +106,8 @@ SIGNATURES = {
                                   _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_int, _vp]),
     "tgis_token_shift_mix": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_int, _vp, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_wkv_decay": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_int, _c_i64, _c_int, _vp]),
+    "tgis_wkv_step": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _vp, _vp, _c_int, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp,
+                               _c_i64, _c_i64, _c_int, _c_int, _c_f, _c_int, _vp]),
     "tgis_wkv_scan": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64,
                                _c_i64, _c_int, _c_int, _c_f, _c_int, _vp]),
     "tgis_moe_row_capacity": (_c_i64, [_c_i64, _c_i64, _c_int]),
@@ -1080,6 +1082,23 @@ def wkv_scan(r, k, v, gate, logw, u, gain, state, shift_state, h, state_slots, c
         _f32(shift_state, "shift_state"), _f32(h, "h"), h.shape[1], _i32(state_slots, "state_slots"),
         _i32(cu_seqlens_q, "cu_seqlens_q"), _i32(positions, "positions"), _ptr(out), out.stride(0), state_slots.shape[0], H, d,
         float(eps), dtype_code3(r.dtype), _stream()), "tgis_wkv_scan")
+    return out
+
+
+WKV_STEP_MAX_RANK = 1024
+
+
+def wkv_step(r, k, v, gate, low, w2t, w0, u, gain, state, shift_state, h, state_slots, cu_seqlens_q, positions, H: int, d: int, eps: float):
+    """wkv_scan with the decay made from low [T, rank] on the way (wkv_decay): the form for steps of single tokens.  d % 4 == 0."""
+    T, ld = r.shape[0], r.stride(0)
+    assert all(t.stride(0) == ld and t.stride(1) == 1 and t.dtype == r.dtype for t in (k, v, gate))
+    assert low.dtype == r.dtype and low.stride(1) == 1 and low.shape == (T, w2t.shape[0]) and w2t.shape[1] == H * d
+    out = torch.empty((T, H * d), dtype=r.dtype, device=r.device)
+    _check(load_library().tgis_wkv_step(
+        _ptr(r), _ptr(k), _ptr(v), _ptr(gate), _ptr(low), ld, low.stride(0), _f32(w2t, "w2t"), _f32(w0, "w0"), w2t.shape[0], _f32(u, "u"),
+        _f32(gain, "gain"), _f32(state, "state"), _f32(shift_state, "shift_state"), _f32(h, "h"), h.shape[1], _i32(state_slots, "state_slots"),
+        _i32(cu_seqlens_q, "cu_seqlens_q"), _i32(positions, "positions"), _ptr(out), out.stride(0), state_slots.shape[0], H, d, float(eps),
+        dtype_code3(r.dtype), _stream()), "tgis_wkv_step")
     return out
 
 
