@@ -80,15 +80,31 @@ template <typename V> __device__ __forceinline__ void st16(void* p, V v) {
     *reinterpret_cast<V*>(p) = v;
 }
 
+// Sum / maximum over the 64 lanes of a wave, in every lane: v (+) v of lane ^ 32, ^ 16, ^ 8, ^ 4, ^ 2, ^ 1, by register moves (six trips
+// through LDS with __shfl_xor, the same bits).  Lane ^ 4 is a rotation of the row by 4: lanes l and l ^ 8 are alike by then.
+template <int CTRL> __device__ __forceinline__ float row_moved(float v) {
+    const int x = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, CTRL, 0xF, 0xF, false));
+}
+template <typename F> __device__ __forceinline__ float wave_reduce(float v, F op) {
+    const uint32_t x = __builtin_bit_cast(uint32_t, v);
+    const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    const uint32_t h0 = h[0], h1 = h[1];
+    v = op(__builtin_bit_cast(float, h0), __builtin_bit_cast(float, h1));
+    const uint32_t y = __builtin_bit_cast(uint32_t, v);
+    const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+    const uint32_t q0 = q[0], q1 = q[1];
+    v = op(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
+    v = op(v, row_moved<0x128>(v));  // rotated by 8
+    v = op(v, row_moved<0x124>(v));  // by 4
+    v = op(v, row_moved<0x4E>(v));   // lane ^ 2
+    return op(v, row_moved<0xB1>(v));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 
 // Sum of S split-K slabs for 8 consecutive columns: all loads of a bucket are issued before the first add (a

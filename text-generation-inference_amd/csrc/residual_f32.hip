@@ -163,17 +163,7 @@ __global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, 
     __shared__ float red[16];
     const int64_t row = blockIdx.x;
     f32x4 xv[NV], dv[NV], pw[NV], qw[NV];
-    if (S > 0) {  // slabs: ld_delta is the slab row stride
-        const float* sp = reinterpret_cast<const float*>(delta) + ((row >> 5) * S * 32 + (row & 31)) * ld_delta;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
-            f32x4 acc = {};
-            if (c < E)
-                for (int sidx = 0; sidx < S; ++sidx) acc += Vec4<float>::ld(sp + (int64_t)sidx * 32 * ld_delta + c);
-            dv[i] = acc;
-        }
-    }
+    // everything is asked for at once: behind the slabs' sum, the residual and the gains were a second trip to memory
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
@@ -182,6 +172,26 @@ __global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, 
         if (S == 0) dv[i] = (in && delta) ? Vec4<TD>::ld(delta + row * ld_delta + c) : f32x4{};
         pw[i] = (in && delta) ? (post_w ? Vec4<float>::ld(post_w + c) + post_add : f32x4{1.f, 1.f, 1.f, 1.f}) : f32x4{};
         qw[i] = in ? (pre_w ? Vec4<float>::ld(pre_w + c) + pre_add : f32x4{1.f, 1.f, 1.f, 1.f}) : f32x4{};
+    }
+    if (S > 0) {  // slabs: ld_delta is the slab row stride; SLABS of them in flight, added in their order
+        constexpr int SLABS = 8;
+        const float* sp = reinterpret_cast<const float*>(delta) + ((row >> 5) * S * 32 + (row & 31)) * ld_delta;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
+            f32x4 acc = {};
+            if (c < E)
+                for (int s0 = 0; s0 < S; s0 += SLABS) {
+                    f32x4 part[SLABS];
+#pragma unroll
+                    for (int e = 0; e < SLABS; ++e)
+                        part[e] = s0 + e < S ? Vec4<float>::ld(sp + (int64_t)(s0 + e) * 32 * ld_delta + c) : f32x4{};
+#pragma unroll
+                    for (int e = 0; e < SLABS; ++e)
+                        if (s0 + e < S) acc += part[e];
+                }
+            dv[i] = acc;
+        }
     }
     if (delta) {
         float rinv_d = post_scale;
