@@ -16,7 +16,7 @@ struct AttnArgs {
     int H, Hkv, G, Gc, Gp, TQ, HC, NS;
     int Gp_shift;  // Gp is a power of two: column -> (q token, head of the group) by shift and mask, not by division
     int HCB;  // decode kernel: blocks per kv head along the 16-head chunks (HC / chunks per block)
-    int xcd_remap;  // decode kernel, HCB > 1: the chunk blocks of a (sequence, split, kv head) group run on one XCD
+    int xcd_remap;  // decode kernel, HCB > 1: the chunk blocks of a (sequence, split, kv head) group run on one XCD; prefill: its tiles
     float scale_log2;
     float* ws_o;   // [total_q][H][NS][D]        (fused combine: [group][chunk][16 columns][NS][D])
     float* ws_ml;  // [total_q][H][NS][2]        (fused combine: [group][chunk][16 columns][NS][4], {m, l, -, -})

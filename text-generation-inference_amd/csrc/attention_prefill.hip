@@ -63,22 +63,17 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, c = lane >> 4;
     // long (late) tiles first: the causal triangle's tail is short ones.  The tiles of a (sequence, kv head, chunk) read the same pages:
-    // where those groups come in eights, each keeps to one XCD (blocks are dealt to the eight in turn), whose L2 then holds them.
-    const int tiles = gridDim.x, heads = gridDim.y;
-    int qt, group;
-    {
-        const int id = blockIdx.x + tiles * (blockIdx.y + heads * blockIdx.z);
-        if ((heads * gridDim.z) % 8 == 0) {
-            qt = (id >> 3) % tiles;
-            group = (id >> 3) / tiles * 8 + (id & 7);
-        } else {
-            qt = id % tiles;
-            group = id / tiles;
-        }
-        qt = tiles - 1 - qt;
+    // where those groups come in eights (xcd_remap), each keeps to one XCD (blocks are dealt to the eight in turn), whose L2 then holds them.
+    int qt = blockIdx.x, head_block = blockIdx.y, b = blockIdx.z;
+    if (a.xcd_remap) {
+        const int tiles = gridDim.x, heads = gridDim.y, id = blockIdx.x + tiles * (blockIdx.y + heads * blockIdx.z);
+        const int group = (id >> 3) / tiles * 8 + (id & 7);
+        qt = (id >> 3) % tiles;
+        head_block = group % heads;
+        b = group / heads;
     }
-    const int hk = (group % heads) / a.HC, hc = (group % heads) % a.HC;
-    const int b = group / heads;
+    qt = gridDim.x - 1 - qt;
+    const int hk = head_block / a.HC, hc = head_block % a.HC;
 
     const int q0 = a.cu_q[b], q_len = a.cu_q[b + 1] - q0;
     const int TQB = a.TQ * 4 * CG;  // q tokens of the block's tile (128 columns)
@@ -314,11 +309,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
 int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st) {
     const int TQB = a.TQ * 8;
     const int64_t q_tiles = cdiv64(max_q_len, TQB);
-    TGIS_CHECK_ARG(q_tiles <= 2147483647LL && (int64_t)Hkv * a.HC <= 65535 && B <= 65535 && q_tiles * Hkv * a.HC * B <= 2147483647LL,
-                   "tgis_attn_paged: grid too large");
+    TGIS_CHECK_ARG(q_tiles <= 2147483647LL && (int64_t)Hkv * a.HC <= 65535 && B <= 65535, "tgis_attn_paged: grid too large");
+    AttnArgs dealt = a;
+    dealt.xcd_remap = (int64_t)Hkv * a.HC * B % 8 == 0 && (double)q_tiles * Hkv * a.HC * B <= 2147483647.0;
     dim3 grid((unsigned)q_tiles, (unsigned)(Hkv * a.HC), (unsigned)B);
     const size_t lds = (size_t)PREFILL_RING * 2 * 32 * D * 2;  // buffers of (K page + V page)
-#define TGIS_PREFILL_LAUNCH(T, DD, R) hipLaunchKernelGGL((attn_prefill_kernel<T, DD, R>), grid, dim3(256), lds, st, a)
+#define TGIS_PREFILL_LAUNCH(T, DD, R) hipLaunchKernelGGL((attn_prefill_kernel<T, DD, R>), grid, dim3(256), lds, st, dealt)
 #define TGIS_PREFILL_WIDTH(T, R) do { if (D == 128) TGIS_PREFILL_LAUNCH(T, 128, R); else TGIS_PREFILL_LAUNCH(T, 64, R); } while (0)
     if (dtype == TGIS_F16) {
         if (rows) TGIS_PREFILL_WIDTH(f16, true); else TGIS_PREFILL_WIDTH(f16, false);

@@ -1298,8 +1298,7 @@ void launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void*
         // softmax and products of neighbouring pages overlapped).  us, staged or direct
         // below / there: 4 x 1024 tokens, 32 heads on 4, dk 64: 173 / 47; 32 on 32, dk 128: 255 / 93; 4 x 300, 32 on 8, dk 128: 40 / 20;
         // 24 x 60, dk 64: 12.7 / 9.9; 16 x 30: 9.3 / 9.4.
-        if (plain(ext) && dk == dv && (dk == 64 || dk == 128) && (int64_t)B * G * cdiv64(R, 16) * cdiv64(max_q_len, 8) <= 2147483647LL &&
-            (int64_t)G * cdiv64(R, 16) <= 65535) {
+        if (plain(ext) && dk == dv && (dk == 64 || dk == 128) && (int64_t)G * cdiv64(R, 16) <= 65535) {
             AttnArgs a{};
             a.q = q;
             a.ld_q = ldq;
