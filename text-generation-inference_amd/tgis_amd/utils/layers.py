@@ -154,6 +154,7 @@ class Ex4bitLinearV2:
         # (no device check here: native.GptqWeight refuses tensors that are not on the GPU — server.py:290-291)
         assert self.height % 32 == 0 and self.width % 32 == 0
         self.q_handle: Optional[native.GptqWeight] = None
+        self.ordered: Optional[native.GptqWeight] = None  # the same image for operands in its own order: what the kernels run on
         # set by LlamaMLP on the fused [gate | up] projection: SiLU(gate)*up runs in the GEMM epilogue
         self.gate_up = False
         # set by FlashLlamaAttention on the fused qkv projection: (H, Hkv, D) of this shard -> post_init also builds the
@@ -171,10 +172,10 @@ class Ex4bitLinearV2:
         # act-order (7B, 11 rows: the four GEMMs of a layer and the rotary launch 163 us when the GEMMs gather while they stage their operand,
         # 48 us with one gather launch in front of o_proj and the norms gathering for qkv and gate_up)
         self._perm = handle.perm
-        self.q_handle = handle if handle.perm is None else handle.in_order()
+        self.q_handle, self.ordered = handle, handle.in_order()
         if self.rope_heads is not None and FUSED_ROPE_GEMM:
             H, Hkv, D = self.rope_heads
-            if any(native.gptq_rope_ok(m, self.q_handle, D) for m in (1, 32, 64)):
+            if any(native.gptq_rope_ok(m, self.ordered, D) for m in (1, 32, 64)):
                 rope = native.GptqWeight(self.qweight, self.qzeros, self.scales, self.g_idx if self._perm is not None else None,
                                          self.bits, self.groupsize, rope=(D, H + Hkv))
                 self.rope_handle = rope if rope.perm is None else rope.in_order()
@@ -207,7 +208,7 @@ class Ex4bitLinearV2:
     def _fused_rows(self, act: int) -> int:
         got = self._fused.get(act)
         if got is None:
-            got = self._fused[act] = self.q_handle.fused_rows(act)
+            got = self._fused[act] = self.ordered.fused_rows(act)
         return got
 
     def _dequant_scratch(self) -> torch.Tensor:
@@ -227,7 +228,7 @@ class Ex4bitLinearV2:
             return False
         if act == 2 and not self.gate_up:
             act = 0
-        w = self.rope_handle if act == 3 else self.q_handle
+        w = self.rope_handle if act == 3 else self.ordered
         return w is not None and rows <= 64 and native.gptq_fragments_ok(rows, w, act)
 
     def forward(self, x, act: int = 0, partial: bool = False, out_frag: bool = False, gathered: bool = False):
@@ -239,24 +240,24 @@ class Ex4bitLinearV2:
                 x, act = native.act_mul(x, self.height), 0
             rows = x.shape[0]
             x = native.gather_columns(x, self._perm, frag=1 <= rows <= 64 and native.gptq_fragments_ok(
-                rows, self.q_handle, 2 if self.gate_up else 0))
+                rows, self.ordered, 2 if self.gate_up else 0))
         if isinstance(x, native.FragAct):
             if self.gate_up:
-                return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias, act=2, out_frag=out_frag)
+                return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=2, out_frag=out_frag)
             assert act == 0
             if partial and DEFER_REDUCE:
-                return native.gptq_gemm_partial(x, self.q_handle, bias=self.bias)
-            return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias)
+                return native.gptq_gemm_partial(x, self.ordered, bias=self.bias)
+            return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias)
         if self.gate_up:
             # output is the activated [M, I] tensor
             if x.shape[0] <= self._fused_rows(2):
-                return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias, act=2)
+                return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=2)
             return native.act_mul(self._large_m(x), self.width // 2)
         # past 128 rows the tall kernel finishes its own sums sooner than a consumer adds the slabs of 64-row passes
         if partial and x.shape[0] <= (128 if self._fused_rows(act) > 256 else native.PARTIAL_MAX_M) and DEFER_REDUCE:
-            return native.gptq_gemm_partial(x, self.q_handle, bias=self.bias, act=act)
+            return native.gptq_gemm_partial(x, self.ordered, bias=self.bias, act=act)
         if x.shape[0] <= self._fused_rows(act):
-            return native.gptq_gemm(x, self.q_handle, workspace(x.device), bias=self.bias, act=act)
+            return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=act)
         if act:
             x = native.act_mul(x, self.height)
         return self._large_m(x)
@@ -265,8 +266,8 @@ class Ex4bitLinearV2:
         """prefill-sized M: dequantise once into scratch, then a library GEMM (exllamav2.py:87 "M > 50"); x in image order."""
         w = self._dequant_scratch()
         native._check(native.load_library().tgis_gptq_dequant_f16(
-            self.q_handle.image.data_ptr(), w.data_ptr(), self.height, self.width, self.q_handle.groups,
-            self.q_handle.flags, native._stream()), "tgis_gptq_dequant_f16")
+            self.ordered.image.data_ptr(), w.data_ptr(), self.height, self.width, self.ordered.groups,
+            self.ordered.flags, native._stream()), "tgis_gptq_dequant_f16")
         out = torch.matmul(x, w)
         if self.bias is not None:
             out.add_(self.bias)
