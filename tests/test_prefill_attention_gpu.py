@@ -49,10 +49,12 @@ def _oracle(q, k, v, scale):
 @pytest.mark.parametrize("H,G,D,dtype", [(8, 8, 128, torch.float16), (6, 2, 64, torch.bfloat16), (8, 1, 64, torch.float16), (16, 1, 128, torch.bfloat16),
                                          (20, 1, 128, torch.float16), (16, 8, 64, torch.bfloat16)])
 @pytest.mark.parametrize("layout", ["fragments", "rows"])
+@pytest.mark.parametrize("groups_per_wave", ["1", "2"])
 @pytest.mark.parametrize("runs", [((65, 65),), ((127, 127), (1, 40)), ((128, 128), (129, 129), (31, 32)), ((33, 97), (300, 300), (2, 2)), ((161, 500),)])
-def test_against_float64(gpu_device, H, G, D, dtype, layout, runs):
+def test_against_float64(gpu_device, H, G, D, dtype, layout, groups_per_wave, runs, monkeypatch):
     from tgis_amd import native
 
+    monkeypatch.setenv("TGIS_PREFILL_CG", groups_per_wave)
     g = torch.Generator().manual_seed(H * D + len(runs))
     q = [torch.randn(n, H, D, generator=g).to(dtype) for n, _ in runs]
     k = [(2 * torch.randn(c, G, D, generator=g)).to(dtype) for _, c in runs]
@@ -82,10 +84,12 @@ def test_against_float64(gpu_device, H, G, D, dtype, layout, runs):
             assert (err <= tol).all(), (scale, b, float((err - tol).max()))
 
 
-def test_large_and_missing_scores(gpu_device):
+@pytest.mark.parametrize("groups_per_wave", ["1", "2"])
+def test_large_and_missing_scores(gpu_device, groups_per_wave, monkeypatch):
     """Scores of every size: a maximum that moves late, keys whose scores are -inf, a row that sees one key."""
     from tgis_amd import native
 
+    monkeypatch.setenv("TGIS_PREFILL_CG", groups_per_wave)
     H = G = 8
     n, D = 200, 64
     g = torch.Generator().manual_seed(5)

@@ -3,7 +3,7 @@
 // what changes is who reads K/V.  In attn_paged_kernel every wave loads the fragments of a page for its own 16
 // columns, which is right for decode (one pass over the cache) and wasteful for prefill, where the same page is needed
 // by every q tile of the sequence: measured 100-180 TFLOP/s, bound by L1 fragment traffic.  Here a block of 4 waves
-// owns 128 columns (32 per wave, two 16-column groups), brings each 32-token page to LDS once and every wave takes its
+// owns 128 columns (32 per wave, two 16-column groups; half of that where prompts are few), brings each 32-token page to LDS once and every wave takes its
 // K / V^T fragments from there, each fragment read feeding two MFMAs.
 //
 // Pages go to LDS by direct loads, three ahead of the one that is multiplied, in a ring of four: no registers, no
@@ -50,12 +50,12 @@ constexpr int PREFILL_RING = 4;  // pages in LDS
 
 // ROWS: the "rows" pages of attn_varlen.hip (keys token-major, values channel-major) instead of those of kv_layout.h.  There the token
 // that a score row stands for is chosen so that the probabilities a lane holds are eight neighbours of a value row.
-template <typename T, int D, bool ROWS>
+// CG: 16-column groups per wave (2; 1 where that leaves the chip idle, see the launcher).
+template <typename T, int D, bool ROWS, int CG>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
     using V8 = typename VecT<T>::x8;
     constexpr int KS = D / 32;  // k-steps of the QK^T MFMA
     constexpr int NB = D / 16;  // 16-row blocks of O^T
-    constexpr int CG = 2;       // 16-column groups per wave
     constexpr int PAGE_ELEMS = 32 * D;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     T* lds = reinterpret_cast<T*>(smem);  // [PREFILL_RING][K page | V page]
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
     const int hk = head_block / a.HC, hc = head_block % a.HC;
 
     const int q0 = a.cu_q[b], q_len = a.cu_q[b + 1] - q0;
-    const int TQB = a.TQ * 4 * CG;  // q tokens of the block's tile (128 columns)
+    const int TQB = a.TQ * 4 * CG;  // q tokens of the block's tile (64 CG columns)
     const int t0 = qt * TQB;
     if (t0 >= q_len) return;
     const int ctx = a.ctx_lens[b];
@@ -227,10 +227,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x100, 2 * KS, 0);  // K's fragments, then products of scores among the exponentials
         __builtin_amdgcn_sched_group_barrier(0x402, 8, 0);
 #pragma unroll
-        for (int g = 0; g < 4 * KS; ++g) {
+        for (int g = 0; g < 2 * CG * KS; ++g) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x402, 80 / (4 * KS), 0);
-            if (g >= 2 * KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, 20 / KS, 0);
+            if (g >= 2 * (CG - 1) * KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -307,14 +307,25 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
 }  // namespace
 
 int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st) {
-    const int TQB = a.TQ * 8;
-    const int64_t q_tiles = cdiv64(max_q_len, TQB);
-    TGIS_CHECK_ARG(q_tiles <= 2147483647LL && (int64_t)Hkv * a.HC <= 65535 && B <= 65535, "tgis_attn_paged: grid too large");
+    TGIS_CHECK_ARG(cdiv64(max_q_len, a.TQ * 4) <= 2147483647LL && (int64_t)Hkv * a.HC <= 65535 && B <= 65535, "tgis_attn_paged: grid too large");
+    const int64_t groups = (int64_t)Hkv * a.HC * B;
+    // Tiles of 128 columns, or of 64 where those would be fewer than the 512 that are resident at once (us, 128 / 64): 1 x 100 tokens, 32
+    // heads of 128: 8.5 / 6.3; 1 x 1000 30.8 / 27.7; 1 x 512, 64 heads on 8: 19.1 / 15.7; 1 x 1500, 32 on 4, D 64: 40 / 30; 3 x 433, 32
+    // heads: 24.7 / 23.5; from 512 on: 4 x 433 24.4 / 26.2, 8 x 200 17.2 / 19.4, 16 x 1008 300 / 337.
+    int cg = groups * cdiv64(max_q_len, a.TQ * 8) < 512 ? 1 : 2;
+    if (const char* e = getenv("TGIS_PREFILL_CG")) cg = atoi(e) == 1 ? 1 : 2;  // tuning and test hook
+    const int64_t q_tiles = cdiv64(max_q_len, a.TQ * 4 * cg);
     AttnArgs dealt = a;
-    dealt.xcd_remap = (int64_t)Hkv * a.HC * B % 8 == 0 && (double)q_tiles * Hkv * a.HC * B <= 2147483647.0;
+    dealt.xcd_remap = groups % 8 == 0 && (double)q_tiles * groups <= 2147483647.0;
     dim3 grid((unsigned)q_tiles, (unsigned)(Hkv * a.HC), (unsigned)B);
     const size_t lds = (size_t)PREFILL_RING * 2 * 32 * D * 2;  // buffers of (K page + V page)
-#define TGIS_PREFILL_LAUNCH(T, DD, R) hipLaunchKernelGGL((attn_prefill_kernel<T, DD, R>), grid, dim3(256), lds, st, dealt)
+#define TGIS_PREFILL_LAUNCH(T, DD, R)                                                                             \
+    do {                                                                                                          \
+        if (cg == 1)                                                                                              \
+            hipLaunchKernelGGL((attn_prefill_kernel<T, DD, R, 1>), grid, dim3(256), lds, st, dealt);              \
+        else                                                                                                      \
+            hipLaunchKernelGGL((attn_prefill_kernel<T, DD, R, 2>), grid, dim3(256), lds, st, dealt);              \
+    } while (0)
 #define TGIS_PREFILL_WIDTH(T, R) do { if (D == 128) TGIS_PREFILL_LAUNCH(T, 128, R); else TGIS_PREFILL_LAUNCH(T, 64, R); } while (0)
     if (dtype == TGIS_F16) {
         if (rows) TGIS_PREFILL_WIDTH(f16, true); else TGIS_PREFILL_WIDTH(f16, false);
