@@ -124,3 +124,40 @@ def test_step_with_its_decay(gpu_device, d, rank, dtype):
         assert (got_S - S).abs().max() <= 2e-5 * S.abs().max(), b
         assert torch.equal(sh[slot].cpu(), h[e - 1])
     assert torch.equal(st[B].cpu(), state[B])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_values_that_are_not_finite_stay_with_later_tokens(gpu_device, dtype, bad):
+    """Prompts of several chunks, one value channel of one token not finite: every token in front of it keeps its output, every one from
+    it on loses its own, as when the tokens are walked one by one."""
+    from tgis_amd import native
+
+    H, d, W, eps = 2, 64, 40, 1e-4
+    lens, at = [40, 33, 20], [25, 16, 18]  # inside a chunk, its first token, a ragged last chunk
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(3)
+    r, k, v, gate = (torch.randn(T, H, d, generator=g).to(dtype) for _ in range(4))
+    logw = -torch.exp(torch.randn(T, H, d, generator=g) - 1.0)
+    u, gain = torch.randn(H, d, generator=g) * 0.3, torch.rand(H, d, generator=g) + 0.5
+    cu = torch.tensor([0] + lens).cumsum(0)
+    pos = torch.cat([torch.arange(n) for n in lens]).to(torch.int32)
+    dev = lambda t: t.to(gpu_device)
+    rows = lambda t: dev(t.reshape(T, H * d))
+
+    def scan(v):
+        return native.wkv_scan(rows(r), rows(k), rows(v), rows(gate), rows(logw), dev(u.reshape(-1)), dev(gain.reshape(-1)),
+                               torch.zeros(B, H, d, d, device=gpu_device), torch.zeros(B, W, device=gpu_device), torch.zeros(T, W, device=gpu_device),
+                               dev(torch.arange(B, dtype=torch.int32)), dev(cu.int()), dev(pos), H, d, eps).float().cpu().view(T, H, d)
+
+    clean = scan(v)
+    for b, s in enumerate(at):
+        v[int(cu[b]) + s, 0, 7] = bad
+    got = scan(v)
+    # (the sums of a token in a chunk with such a value are added in another order: fp32 roundings, then the output's)
+    tol = 2e-5 + (0.0 if dtype == torch.float32 else 2.0 ** -7)
+    for b, s in enumerate(at):
+        a, e = int(cu[b]), int(cu[b + 1])
+        assert ((got[a:a + s] - clean[a:a + s]).abs() <= tol * (1 + clean[a:a + s].abs())).all(), b
+        assert not got[a + s:e, 0, 7].isfinite().any(), b
+        assert torch.equal(got[a:e, 1], clean[a:e, 1]), b  # the other head

@@ -498,19 +498,29 @@ __global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
         float vb[4];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) vb[ks] = vv[buf][4 * ks + lq][j];
-        f32x4 o0 = zero4, o1 = zero4;
+        f32x4 s0 = zero4, s1 = zero4;
 #pragma unroll
         for (int it = 0; it < NI; ++it) {
             const f32x4 a4 = *reinterpret_cast<const f32x4*>(&rp[buf][lc][16 * it + 4 * lq]);
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[0], S[it][0], o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[1], S[it][1], o1, 0, 0, 0);
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[2], S[it][2], o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[3], S[it][3], o1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[0], S[it][0], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[1], S[it][1], s1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[2], S[it][2], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[3], S[it][3], s1, 0, 0, 0);
         }
+        f32x4 o0 = s0, o1 = s1;
 #pragma unroll
         for (int ks = 0; ks < 4; ks += 2) {
             o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[buf][lc][4 * ks + lq], vb[ks], o0, 0, 0, 0);
             o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(aa[buf][lc][4 * ks + 4 + lq], vb[ks + 1], o1, 0, 0, 0);
+        }
+        // A is zero past its diagonal, but 0 times a value that is not finite is no zero: such a value shows in every row of its column.
+        // Then each token adds up only the values that it sees, and those in front of it stay what they are token by token.
+        if (__builtin_amdgcn_ballot_w64(!(fabsf(o0[0] + o1[0]) < __builtin_inff())) != 0) {
+            o0 = s0;
+            o1 = s1;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                for (int x = 0; x <= 4 * lq + e; ++x) o0[e] += aa[buf][4 * lq + e][x] * vv[buf][x][j];
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) oo[4 * lq + e][j] = o0[e] + o1[e];
