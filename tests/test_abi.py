@@ -67,6 +67,20 @@ def test_argument_validation_needs_no_gpu():
     lib.tgis_clear_error()
 
 
+def test_a_refused_launch_is_reported():
+    """tgis_attn_varlen passes on what the kernel it chose refuses: a run too long for any grid, seen before anything is launched."""
+    import ctypes
+
+    from tgis_amd import native
+
+    lib = native.load_library()
+    p, run = ctypes.c_void_p(4096), 1 << 40
+    for dtype in (0, 1):
+        rc = lib.tgis_attn_varlen(p, 512, p, p, p, 4, p, p, 1, p, 512, 100, run, 100, 8, 8, 64, 64, 0.125, 0, dtype, None)
+        assert rc == -1 and b"grid too large" in lib.tgis_last_error()
+    lib.tgis_clear_error()
+
+
 def test_integration_doc_names_only_declared_entry_points():
     """INTEGRATION.md is what a maintainer binds from: outside its 'NOT in this ABI any more' section every tgis_* call it
     names must be declared in include/tgis_hip.h (three rows pointed at entry points that had moved out)."""

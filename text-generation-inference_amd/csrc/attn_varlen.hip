@@ -1260,9 +1260,9 @@ __global__ __launch_bounds__(256) void latent_norm_write_kernel(T* __restrict__ 
 }
 
 template <typename T, int DK16, int DVT>
-void launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void* v_pool, const int32_t* bt, int64_t bt_ld,
-                     const int32_t* ctx_lens, const int32_t* cu_q, int B, void* out, int64_t ld_out, int64_t max_q_len, int H, int G,
-                     int dk, int dv, float scale, int64_t max_ctx, AttnExt ext, hipStream_t st) {
+int launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void* v_pool, const int32_t* bt, int64_t bt_ld,
+                    const int32_t* ctx_lens, const int32_t* cu_q, int B, void* out, int64_t ld_out, int64_t max_q_len, int H, int G,
+                    int dk, int dv, float scale, int64_t max_ctx, AttnExt ext, hipStream_t st) {
     const int R = H / G;
     const bool split = max_q_len * R <= 32;
     // a windowed query walks its window's pages and the kept first ones, whatever the context
@@ -1312,8 +1312,7 @@ void launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void*
             a.ld_out = ld_out;
             a.scale_log2 = scale * 1.4426950408889634f;
             attn_set_geom(a, H, G, attn_geom(H, G));
-            (void)tgis_launch_attn_prefill(a, B, G, dk, max_q_len, std::is_same<T, f16>::value ? TGIS_F16 : TGIS_BF16, true, st);
-            return;
+            return tgis_launch_attn_prefill(a, B, G, dk, max_q_len, std::is_same<T, f16>::value ? TGIS_F16 : TGIS_BF16, true, st);
         }
         // Measured (4 x 1024-token prompts): staging wins for narrow heads (dk 64 / dv 64, R 8: 2.96 ms against 3.20 for 22 layers)
         // and loses for wide ones (dk 128 / dv 128, MHA: 10.4 against 8.4 ms for 32 layers: two barriers per page and one LDS
@@ -1326,7 +1325,7 @@ void launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void*
             hipLaunchKernelGGL((attn_varlen_staged_kernel<T, DK16, DVT>), dim3(gx, (unsigned)G, (unsigned)B), dim3(256), 0, st,
                                (const T*)q, ldq, (const T*)k_pool, (const T*)v_pool, bt, bt_ld, ctx_lens, cu_q, (T*)out, ld_out, H, G,
                                dk, dv, scale, ext);
-            return;
+            return TGIS_OK;
         }
     }
     hipLaunchKernelGGL((attn_varlen_mfma_kernel<T, DK16, DVT>), dim3(gx, (unsigned)G, (unsigned)B), dim3(64 * nw), lds, st,
@@ -1335,33 +1334,32 @@ void launch_mfma_one(const void* q, int64_t ldq, const void* k_pool, const void*
     if (key_splits > 1)
         hipLaunchKernelGGL(attn_combine_splits_kernel<T>, dim3((unsigned)ext.partial_tokens, (unsigned)H), dim3(64), 0, st, ext.partial,
                            key_splits, ext.partial_tokens, H, dv, (T*)out, ld_out, ext);
+    return TGIS_OK;
 }
 
 template <typename T, int DK16>
-void launch_mfma_dv(const void* q, int64_t ldq, const void* k_pool, const void* v_pool, const int32_t* bt, int64_t bt_ld,
-                    const int32_t* ctx_lens, const int32_t* cu_q, int B, void* out, int64_t ld_out, int64_t max_q_len, int H, int G,
-                    int dk, int dv, float scale, int64_t max_ctx, AttnExt ext, hipStream_t st) {
+int launch_mfma_dv(const void* q, int64_t ldq, const void* k_pool, const void* v_pool, const int32_t* bt, int64_t bt_ld,
+                   const int32_t* ctx_lens, const int32_t* cu_q, int B, void* out, int64_t ld_out, int64_t max_q_len, int H, int G,
+                   int dk, int dv, float scale, int64_t max_ctx, AttnExt ext, hipStream_t st) {
     const int nvt = dv / 32;
     if (nvt <= 1)
-        launch_mfma_one<T, DK16, 1>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
-    else if (nvt <= 2)
-        launch_mfma_one<T, DK16, 2>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
-    else if (nvt <= 4)
-        launch_mfma_one<T, DK16, 4>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
-    else
-        launch_mfma_one<T, DK16, 8>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+        return launch_mfma_one<T, DK16, 1>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+    if (nvt <= 2)
+        return launch_mfma_one<T, DK16, 2>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+    if (nvt <= 4)
+        return launch_mfma_one<T, DK16, 4>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+    return launch_mfma_one<T, DK16, 8>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
 }
 
 template <typename T>
-void launch_mfma(const void* q, int64_t ldq, const void* k_pool, const void* v_pool, const int32_t* bt, int64_t bt_ld,
-                 const int32_t* ctx_lens, const int32_t* cu_q, int B, void* out, int64_t ld_out, int64_t max_q_len, int H, int G, int dk,
-                 int dv, float scale, int64_t max_ctx, AttnExt ext, hipStream_t st) {
+int launch_mfma(const void* q, int64_t ldq, const void* k_pool, const void* v_pool, const int32_t* bt, int64_t bt_ld,
+                const int32_t* ctx_lens, const int32_t* cu_q, int B, void* out, int64_t ld_out, int64_t max_q_len, int H, int G, int dk,
+                int dv, float scale, int64_t max_ctx, AttnExt ext, hipStream_t st) {
     if (dk <= 64)
-        launch_mfma_dv<T, 4>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
-    else if (dk <= 128)
-        launch_mfma_dv<T, 8>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
-    else
-        launch_mfma_dv<T, 16>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+        return launch_mfma_dv<T, 4>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+    if (dk <= 128)
+        return launch_mfma_dv<T, 8>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+    return launch_mfma_dv<T, 16>(q, ldq, k_pool, v_pool, bt, bt_ld, ctx_lens, cu_q, B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
 }
 
 template <typename T>
@@ -1436,10 +1434,10 @@ static int attn_varlen_impl(const void* q, int64_t ldq, const void* k_pool, cons
                          B <= 65535 && G <= 65535;
     TGIS_CHECK_ARG(impl != 2 || mfma_ok, "tgis_attn_varlen: the matrix-core kernel needs a two-byte dtype, dk %% 16 == 0, dv %% 32 == 0, both <= 256, aligned operands");
     if (mfma_ok && impl != 1) {
-        if (dtype == TGIS_F16)
-            launch_mfma<f16>(q, ldq, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, (int)B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
-        else
-            launch_mfma<bf16>(q, ldq, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, (int)B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+        const int rc =
+            dtype == TGIS_F16 ? launch_mfma<f16>(q, ldq, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, (int)B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st)
+                              : launch_mfma<bf16>(q, ldq, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, (int)B, out, ld_out, max_q_len, H, G, dk, dv, scale, max_ctx, ext, st);
+        if (rc != TGIS_OK) return rc;
         TGIS_CHECK_LAUNCH();
         return TGIS_OK;
     }
