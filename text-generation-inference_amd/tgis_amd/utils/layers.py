@@ -172,7 +172,7 @@ class Ex4bitLinearV2:
         # act-order (7B, 11 rows: the four GEMMs of a layer and the rotary launch 163 us when the GEMMs gather while they stage their operand,
         # 48 us with one gather launch in front of o_proj and the norms gathering for qkv and gate_up)
         self._perm = handle.perm
-        self.q_handle, self.ordered = handle, handle.in_order()
+        self.q_handle, self.ordered = handle, handle if self._perm is None else handle.in_order()
         if self.rope_heads is not None and FUSED_ROPE_GEMM:
             H, Hkv, D = self.rope_heads
             if any(native.gptq_rope_ok(m, self.ordered, D) for m in (1, 32, 64)):
