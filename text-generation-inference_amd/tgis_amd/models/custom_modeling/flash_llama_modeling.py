@@ -145,7 +145,7 @@ class FlashLlamaAttention:
             bias=config.attention_bias)
         self.o_proj = TensorParallelRowLinear.load(config, prefix=f"{prefix}.o_proj", weights=weights,
                                                    bias=config.attention_bias)
-        # steps of up to 64 rows (where native.rope_gemm_ok) rotate q / k and write the cache in the GEMM epilogue, prompts included
+        # steps of up to 64 rows (where native.rope_gemm_ok) rotate q / k and write the cache in the GEMM epilogue, prompts where that pays
         if hasattr(self.query_key_value.linear, "rope_heads"):
             self.query_key_value.linear.rope_heads = (self.num_heads, self.num_key_value_heads, self.head_size)
 
@@ -156,10 +156,12 @@ class FlashLlamaAttention:
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         lin = self.query_key_value.linear
         rope_w = getattr(lin, "rope_handle", None)
+        decode = kv.max_q_len == 1 and not kv.fresh_prefill
         if isinstance(hidden_states, native.FragAct) or (
                 rope_w is not None and kv.slots is not None
                 and (gathered or getattr(lin, "perm", None) is None) and hidden_states.shape[0] <= 64 and cos.shape[1] * 2 == D
-                and native.rope_gemm_ok(hidden_states.shape[0], rope_w, D)):
+                and native.rope_gemm_ok(hidden_states.shape[0], rope_w, D)
+                and (decode or native.rope_gemm_pays_for_prompts(hidden_states.shape[0], rope_w))):
             # one launch: GEMM + rotary embedding + cache write (native.gptq_gemm_rope / native.dense_gemm_rope)
             fused = native.gptq_gemm_rope if isinstance(rope_w, native.GptqWeight) else native.dense_gemm_rope
             return fused(hidden_states, rope_w, lin.bias, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D)

@@ -545,6 +545,16 @@ def rope_gemm_ok(M: int, w, D: int) -> bool:
     return got
 
 
+def rope_gemm_pays_for_prompts(M: int, w) -> bool:
+    """Whether a prompt's rows, which arrive row-major, should take the fused launch too.  rope_gemm_ok answers for decode steps, whose int4
+    operands are in fragment order; the row-major int4 kernel keeps the whole k range in blocks of two tiles and more, and past 32 rows
+    a block takes in twice the activation.  us, fused row-major / split GEMM and a rotary launch: 4096 x 12288 at 1, 32, 33, 64 rows 12.7 /
+    14.5, 12.8 / 15.7, 25.7 / 18.9, 27.2 / 21.4; 1024 x 3072 5.5 / 6.6, 6.2 / 7.7, 11.3 / 8.7, 12.4 / 9.1; 3072 x 9216 at 32 10.8 / 12.6;
+    8192 x 24576 30.6 / 34.9; with fewer columns the split wins: 8192 x 10240 at 1, 32, 33, 64 rows 20.6 / 19.1, 20.1 / 19.8, 41.9 / 24.5,
+    43.5 / 26.9; 4096 x 6144 at 1, 32 rows 11.6 / 10.9, 12.0 / 11.9; 6144 x 8192 15.3 / 14.0, 16.0 / 15.6; 3072 x 5120 9.6 / 9.1, 10.4 / 9.9."""
+    return not isinstance(w, GptqWeight) or (M <= 32 and w.N >= 2 * w.K)
+
+
 def gptq_gemm_rope(x: torch.Tensor, w: GptqWeight, bias, cos, sin, positions, slots, k_pool, v_pool, H: int, Hkv: int,
                    D: int, out=None) -> torch.Tensor:
     """qkv projection + rotary embedding + cache write in one launch (decode, M <= 64; `w` is the rope image of the fused
