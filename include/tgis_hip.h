@@ -707,6 +707,9 @@ int tgis_relu2(const void* in, int64_t ld_in, void* out, int64_t ld_out, int64_t
 int tgis_dense_gemm_relu2(const void* x, int64_t ldx, const void* prepared, void* out, int64_t ldo, int64_t M, int64_t K,
                           int64_t N, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* 1 where a finished product (act 0, or 2: SiLU * up) runs in the form that has its whole operand in flight at once, 0 where it streams
+ * (a host-side query; results differ by the order of fp32 sums alone). */
+int tgis_dense_gemm_whole_operand(int64_t M, int64_t K, int64_t N, int act);
 /* `groups` products in one launch: rows [g N_group, (g + 1) N_group) of one stacked weight (a plain image; the last group takes the rows
  * that are left) times an input of their own, x + g x_group elements; out + g out_group elements takes group g's columns from 0 on.
  * M <= 64, K a multiple of 64, N_group of 32, x_group of 8. */

@@ -41,7 +41,8 @@ def test_finished(gpu_device, K, N, M):
     assert ((y.double().cpu() - want).abs() <= eps * want.abs() + 1.13 * bound(plain) + 1e-3 * eps).all()  # |gelu'| <= 1.13
 
 
-@pytest.mark.parametrize("K,I", [(64, 16), (576, 48), (2048, 208), (2112, 64)])
+# (and the sizes between which the form with the whole operand in flight runs: 256 to 512 tiles, the last ones ragged)
+@pytest.mark.parametrize("K,I", [(64, 16), (576, 48), (2048, 208), (2112, 64), (1152, 4080), (1152, 4096), (2048, 8176), (2048, 8192), (1984, 5600)])
 @pytest.mark.parametrize("M", [32, 33, 47, 64])
 def test_gate_up(gpu_device, K, I, M):
     from tgis_amd import native

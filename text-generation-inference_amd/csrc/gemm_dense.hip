@@ -62,7 +62,11 @@ using dense::dense_slab_bytes;
 // outputs that leave finished (us, bf16, weights cold; streaming / this one):
 //   * act 0 of heads (512 tiles and more) at up to 16 rows, where an extra trip to memory shows: 4096 x 32000 at 1 / 11 rows 47.7 / 42.4,
 //     47.5 / 45.0; 2048 x 32000 at 16 rows 26.7 / 24.8; 6144 x 49152 at 1 row 106 / 96 (32 rows: 107 / 106 - 116)
-//   * act 2 at 33 - 64 rows of small models: 2048 x 11264 at 47 rows 18.0 / 15.0 (6144 x 24576 at 64 rows: 61 / 74)
+//   * act 2 at 33 - 64 rows of small models, where the chip holds a block of every two tiles at once and the streaming form has its widest
+//     blocks: 2048 x 8192 at 33 / 64 rows 16.7 / 13.0, 18.4 / 14.8; 2048 x 11264 19.1 / 15.2, 20.7 / 17.0; 2048 x 16384 20.9 / 18.5, 22.7 /
+//     20.1; 1152 x 8192 13.1 / 11.1, 14.3 / 12.5; 1152 x 16384 15.6 / 14.3, 17.1 / 15.5.  Outside: 2048 x 8128 13.6 / 12.9, 14.6 / 14.8; 2048 x
+//     5632 13.4 / 14.0, 14.0 / 14.3; 2048 x 16448 20.8 / 26.5, 22.7 / 29.9; 1024 x 16384 12.3 / 12.9, 13.3 / 13.7; 256 x 24576 8.0 / 13.1
+//     (6144 x 24576 at 64 rows: 61 / 74)
 // A projection whose streaming plan splits k stays with it, so that it sums in the same order whether it leaves finished or as slabs
 // (2048 x 2048 at 16 rows: finished 7.5 / 5.9, as slabs 4.2 / 5.5).
 static DensePlan plan_finished(int64_t K, int64_t N, int64_t M, int act) {
@@ -70,7 +74,7 @@ static DensePlan plan_finished(int64_t K, int64_t N, int64_t M, int act) {
     if (M < 1 || M > 64 || K % 64 != 0) return stream;
     const int64_t tiles = cdiv64(N, 32);
     const DensePlan wide1{(int)K, 1, dense::WIDE_WAVES, 1, 1}, wide2{(int)K, 1, dense::WIDE_WAVES, 2, M > 32 ? 2 : 1};
-    if (act == 2) return M > 32 && K <= 2048 ? wide2 : stream;
+    if (act == 2) return M > 32 && K >= 1152 && K <= 2048 && tiles >= 256 && tiles <= 512 ? wide2 : stream;
     return act != 0 || tiles < 512 || M > 16 ? stream : (K <= 2048 || M <= 4) ? wide1 : wide2;
 }
 
@@ -406,6 +410,12 @@ extern "C" int tgis_dense_gemm_gelu_lookup(const void* x, int64_t ldx, const voi
     a.row_col0 = col0;
     a.row_table_rows = vocab;
     return dtype == TGIS_F16 ? launch_dense<f16>(a, pl, 0, cdiv64(M, 32), st) : launch_dense<bf16>(a, pl, 0, cdiv64(M, 32), st);
+}
+
+// Does the kernel that asks for everything at once serve this finished product?  (a size query)
+extern "C" int tgis_dense_gemm_whole_operand(int64_t M, int64_t K, int64_t N, int act) {
+    if (K <= 0 || N <= 0 || (act != 0 && act != 2)) return 0;
+    return plan_finished(K, N, M, act).WK == dense::WIDE_WAVES ? 1 : 0;
 }
 
 // ---- several projections of different inputs in one launch --------------------------------------------

@@ -185,6 +185,7 @@ SIGNATURES = {
     "tgis_narrow_product": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_int, _c_i64, _c_int, _vp]),
     "tgis_moe_choose": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_f, _vp, _vp, _vp]),
     "tgis_relu2": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_gemm_whole_operand": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
     "tgis_matrix_memory": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _vp, _c_i64, _vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp,
