@@ -11,7 +11,8 @@ def _bound(x, w, eps):
 
 
 # K: fewer steps than waves, a ragged last round of steps, one phase exactly, several phases; N: one ragged tile, several, a head (512+)
-@pytest.mark.parametrize("K,N", [(64, 40), (448, 96), (576, 128), (2048, 2048), (2048, 100), (4160, 4128), (6144, 4096), (320, 16400), (4160, 16400)])
+@pytest.mark.parametrize("K,N", [(64, 40), (448, 96), (576, 128), (2048, 2048), (2048, 100), (4160, 4128), (6144, 4096), (320, 16400), (4160, 16400),
+                                 (1280, 16384), (4160, 16384), (2112, 40960)])
 @pytest.mark.parametrize("M", [1, 2, 5, 15, 16, 17, 31, 32, 33, 47, 64, 65])
 def test_finished(gpu_device, K, N, M):
     from tgis_amd import native

@@ -12,3 +12,16 @@ def test_dense_gate_up(M, K, N, whole):
     from tgis_amd import native
 
     assert native.load_library().tgis_dense_gemm_whole_operand(M, K, N, 2) == whole
+
+
+# one-tile blocks (two to a CU) and two-tile blocks (one to a CU), each with a last round that is full enough and one that is not
+@pytest.mark.parametrize("M,K,N,whole", [
+    (1, 4096, 32000, 1), (16, 2048, 32000, 1), (4, 8192, 32000, 1), (1, 6144, 49152, 1), (17, 2048, 32000, 0), (16, 2048, 16352, 0),
+    (1, 512, 32000, 0), (1, 1216, 32000, 0), (1, 1280, 32000, 1), (1, 5120, 20480, 0), (16, 1792, 20480, 0), (1, 5120, 24576, 1),
+    (11, 4096, 32000, 1), (5, 4096, 24576, 0), (16, 4096, 50304, 0), (16, 4096, 49152, 1), (11, 5120, 40960, 1), (11, 5120, 32000, 0),
+    (11, 3072, 32000, 0), (11, 3072, 16384, 1), (11, 8192, 128256, 1), (1, 4100, 32000, 0),
+])
+def test_dense_head(M, K, N, whole):
+    from tgis_amd import native
+
+    assert native.load_library().tgis_dense_gemm_whole_operand(M, K, N, 0) == whole

@@ -60,8 +60,12 @@ using dense::dense_slab_bytes;
 
 // Where the kernel that asks for everything at once (dense_wide_body.h; WK = WIDE_WAVES in the plan) replaces the streaming one, for
 // outputs that leave finished (us, bf16, weights cold; streaming / this one):
-//   * act 0 of heads (512 tiles and more) at up to 16 rows, where an extra trip to memory shows: 4096 x 32000 at 1 / 11 rows 47.7 / 42.4,
-//     47.5 / 45.0; 2048 x 32000 at 16 rows 26.7 / 24.8; 6144 x 49152 at 1 row 106 / 96 (32 rows: 107 / 106 - 116)
+//   * act 0 of heads (512 tiles and more) at up to 16 rows and K >= 1280 (below, a wave's ring is emptier than full: 512 x 32000 at 1 row 8.0 /
+//     11.8, 1024 x 24576 11.1 / 12.1), where blocks fill their last round.  One-tile blocks (K <= 2048, or up to 4 rows), two to a CU:
+//     4096 x 32000 at 1 row 47.4 / 41.2; 2048 x 32000 at 16 rows 26.8 / 24.0; 6144 x 49152 at 1 row 106 / 96; with a last round a quarter
+//     full 5120 x 20480 at 1 row 35.3 / 36.7, 1792 x 20480 at 16 rows 15.3 / 16.0.  Two-tile blocks, one to a CU: 4096 x 32000 at 11 rows
+//     47.9 / 44.8, 6144 x 49152 107 / 98; with a half-full round among two 4096 x 24576 at 11 rows 33.4 / 37.5, among
+//     three or with a last phase of x half full 4096 x 50304 at 16 rows 72.7 / 77.0, 3072 x 32000 34.6 / 36.4, 5120 x 32000 53.8 / 55.5
 //   * act 2 at 33 - 64 rows of small models, where the chip holds a block of every two tiles at once and the streaming form has its widest
 //     blocks: 2048 x 8192 at 33 / 64 rows 16.7 / 13.0, 18.4 / 14.8; 2048 x 11264 19.1 / 15.2, 20.7 / 17.0; 2048 x 16384 20.9 / 18.5, 22.7 /
 //     20.1; 1152 x 8192 13.1 / 11.1, 14.3 / 12.5; 1152 x 16384 15.6 / 14.3, 17.1 / 15.5.  Outside: 2048 x 8128 13.6 / 12.9, 14.6 / 14.8; 2048 x
@@ -75,7 +79,11 @@ static DensePlan plan_finished(int64_t K, int64_t N, int64_t M, int act) {
     const int64_t tiles = cdiv64(N, 32);
     const DensePlan wide1{(int)K, 1, dense::WIDE_WAVES, 1, 1}, wide2{(int)K, 1, dense::WIDE_WAVES, 2, M > 32 ? 2 : 1};
     if (act == 2) return M > 32 && K >= 1152 && K <= 2048 && tiles >= 256 && tiles <= 512 ? wide2 : stream;
-    return act != 0 || tiles < 512 || M > 16 ? stream : (K <= 2048 || M <= 4) ? wide1 : wide2;
+    if (act != 0 || tiles < 512 || M > 16 || K < 1280) return stream;
+    if (K <= 2048 || M <= 4) return 10 * tiles >= 7 * 512 * cdiv64(tiles, 512) ? wide1 : stream;
+    const int64_t blocks = cdiv64(tiles, 2), rounds = cdiv64(blocks, 256), slots = 256 * rounds;
+    const bool full = rounds >= 3 ? 10 * blocks >= 8 * slots : (blocks == slots || (K % 2048 == 0 && 100 * blocks >= 95 * slots));
+    return full ? wide2 : stream;
 }
 
 // One workgroup = one unit of dense_gemm_body.h (block-wide barriers, plain loads and stores).
