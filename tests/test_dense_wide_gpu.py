@@ -66,7 +66,8 @@ def test_gate_up(gpu_device, K, I, M):
 
 @pytest.mark.parametrize("K,H,Hkv,D,M", [(*shape, M) for shape in [(1088, 48, 8, 32), (2048, 32, 4, 64), (2112, 16, 4, 128), (4096, 16, 8, 64),
                                                                    (4160, 16, 8, 64)] for M in (1, 2, 15, 16, 17)]
-                         + [(*shape, M) for shape in [(64, 48, 8, 32), (1088, 48, 8, 32), (2048, 32, 4, 64)] for M in (33, 47, 63, 64)])
+                         + [(*shape, M) for shape in [(64, 48, 8, 32), (1088, 48, 8, 32), (2048, 32, 4, 64)] for M in (33, 47, 63, 64)]
+                         + [(*shape, M) for shape in [(1024, 32, 8, 64), (3072, 24, 8, 128)] for M in (8, 9, 16)])
 def test_rope(gpu_device, K, H, Hkv, D, M):
     """Against the plain image's GEMM followed by the rotary launch: the two differ by the order of their fp32 sums alone."""
     from tgis_amd import native

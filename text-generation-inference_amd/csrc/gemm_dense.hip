@@ -475,8 +475,9 @@ static DensePlan plan_dense_rope(int64_t K, int64_t N, int64_t M) {
         pl.TN = 1;
         // Up to 16 rows and K = 4096 every operand byte of a workgroup fits in flight at once (dense_wide_body.h): 2048 x 2560 at 1 / 8 / 16
         // rows 6.3 -> 5.5, 6.7 -> 5.9, 6.9 -> 6.5 us; at 24 rows 7.7 / 7.4 and at 32 7.7 / 7.8; 4096 x 3072 at 8 rows 10.8 -> 9.5, at 32
-        // 12.4 / 13.1; 5120 x 3072 at 16 rows 13.6 / 14.4.
-        if (M <= 16 && K % 64 == 0 && K <= 4096) pl = {(int)K, 1, dense::WIDE_WAVES, 1, 1};
+        // 12.4 / 13.1; 5120 x 3072 at 16 rows 13.6 / 14.4.  Where K suits the streaming form's four k-parts and half of a phase of x here is
+        // past the range, the larger batches stay there: 1024 x 3072 at 8 / 16 rows 5.2 / 5.2, 5.3 / 5.6; 3072 x 5120 9.2 / 9.0, 9.6 / 10.0.
+        if (M <= 16 && K % 64 == 0 && K <= 4096 && (M <= 8 || K % 1024 != 0 || K % 2048 == 0)) pl = {(int)K, 1, dense::WIDE_WAVES, 1, 1};
     }
     // 33 - 64 rows of small models (against the slab form and a rotary launch behind it): 2048 x 2560 at 33 / 47 / 64 rows 10.7 -> 9.1,
     // 10.9 -> 9.9, 11.2 -> 11.0; 2048 x 6144 13.6 -> 11.3, 14.4 -> 13.0; 1024 x 3072 9.4 -> 7.5, 9.6 -> 8.7; but 4096 x 3072 14.0 / 14.8,
