@@ -25,3 +25,19 @@ def test_dense_head(M, K, N, whole):
     from tgis_amd import native
 
     assert native.load_library().tgis_dense_gemm_whole_operand(M, K, N, 0) == whole
+
+
+# up to 256 rows: matrices whose 64-row passes are done first, and those where the tall kernel is; above, it always serves
+@pytest.mark.parametrize("M,K,N,act,whole", [
+    (128, 4096, 12288, 0, 0), (129, 4096, 12288, 0, 1), (256, 4096, 12288, 0, 1), (129, 2048, 2560, 0, 0), (256, 2048, 2560, 0, 0),
+    (257, 2048, 2560, 0, 1), (192, 1024, 1024, 0, 0), (192, 3072, 5120, 0, 0), (256, 3072, 5120, 0, 1), (192, 2048, 6144, 0, 1),
+    (256, 4096, 4096, 0, 0), (129, 11008, 4096, 0, 1), (129, 256, 128, 0, 1), (64, 4096, 22016, 2, 0), (65, 4096, 22016, 2, 1),
+    (128, 2048, 11264, 2, 0), (129, 2048, 11264, 2, 1), (96, 1024, 5632, 2, 0), (300, 1024, 5632, 2, 1), (300, 4096, 4096, 1, 0),
+])
+def test_int4_tall(M, K, N, act, whole):
+    from tgis_amd import native
+
+    lib = native.load_library()
+    assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 128, 0, act) == whole
+    assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 128, 1, act) == 0  # act-order
+    assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 32, 0, act) == 0   # groups shorter than a k64-step

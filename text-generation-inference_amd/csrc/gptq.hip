@@ -284,8 +284,13 @@ extern "C" int tgis_gptq_prepare(const int32_t* qweight, const int32_t* qzeros, 
 
 extern "C" int64_t tgis_gptq_gemm_fused_rows(int64_t K, int64_t groups, int act_order, int act) {
     if (K <= 0 || groups <= 0 || K % groups) return 0;
-    static const int32_t some_perm = 0;
-    return gptq::tall_ok(gptq::tall_min_m(act), K, groups, act_order ? &some_perm : nullptr, act) ? std::max<int64_t>(256, gptq::tall_max_m()) : 256;
+    return gptq::tall_serves(K, groups, act_order != 0, act) ? std::max<int64_t>(256, gptq::tall_max_m()) : 256;
+}
+
+// Does tgis_gptq_gemm_f16 finish its sums by itself at M rows?  (the tall kernel; else 64-row passes and, where they split, their reduce)
+extern "C" int tgis_gptq_gemm_whole_sums(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act) {
+    if (M < 1 || K <= 0 || N <= 0 || groups <= 0 || K % groups) return 0;
+    return gptq::tall_ok(M, K, N, groups, act_order != 0, act) ? 1 : 0;
 }
 
 extern "C" int64_t tgis_gptq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
@@ -517,7 +522,7 @@ extern "C" int tgis_gptq_gemm_f16(const void* x, int64_t ldx, const void* prepar
                            (float*)((uint8_t*)workspace + 4096), 0, wp, st);
     }
     TGIS_CHECK_ARG(ldo != TGIS_LD_FRAGMENTS, "tgis_gptq_gemm_f16: a fragment-order output needs a fragment-order activation");
-    if (gptq::tall_ok(M, K, groups, perm, act)) {
+    if (gptq::tall_ok(M, K, N, groups, perm != nullptr, act)) {
         const int64_t need_t = 4096 + gptq::tall_workspace_bytes(M, K, N);
         TGIS_CHECK_ARG(workspace && workspace_bytes >= need_t, "tgis_gptq_gemm_f16: workspace too small (%ld < %ld)",
                        (long)workspace_bytes, (long)need_t);

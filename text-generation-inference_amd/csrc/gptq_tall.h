@@ -5,9 +5,10 @@
 
 namespace gptq {
 
-// Does the tall kernel run this GEMM?  (from tall_min_m() rows; K in whole k64-steps, groups of 64 * 2^n rows, no act-order
-// permutation, act 0 or 2)
-bool tall_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act);
+// Can the tall kernel run this GEMM?  (K in whole k64-steps, groups of 64 * 2^n rows, no act-order permutation, act 0 or 2)
+bool tall_serves(int64_t K, int64_t groups, bool act_order, int act);
+// ... and does it, at M rows?  (from tall_min_m(); up to 256 rows where the streaming passes would take longer)
+bool tall_ok(int64_t M, int64_t K, int64_t N, int64_t groups, bool act_order, int act);
 // ... and its deferred form?  (up to 256 rows the streaming passes leave fewer and smaller slabs)
 bool tall_partial_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act);
 int64_t tall_min_m(int act);

@@ -314,6 +314,7 @@ struct TallPlan {
     int col_blocks, tiles;  // tiles of BM x 128 TW
     int whole;              // leading tiles that are not split
     int S, per;             // the others: splits, k64-steps per split
+    double us;              // what the model below expects
 };
 
 // us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip (several blocks on each; clocks drop under
@@ -349,7 +350,7 @@ TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
                     us = std::max(alone, us + (rest ? busy * (0.55 + 0.45 * share) : 0.0));
                 if (us < best_us) {
                     best_us = us;
-                    best = {BMR, TW, (int)cb, (int)tiles, (int)(S > 1 ? tiles - rest : tiles), S, (int)per};
+                    best = {BMR, TW, (int)cb, (int)tiles, (int)(S > 1 ? tiles - rest : tiles), S, (int)per, us};
                 }
             }
         }
@@ -357,7 +358,7 @@ TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
         int b = 0, t = 0, S = 0;
         if (sscanf(e, "%d,%d,%d", &b, &t, &S) == 3 && b >= 2 && b <= 4 && t >= 1 && t <= 2 && S >= 1 && S <= 16) {
             const int64_t cb = cdiv64(NT, 4 * t), tiles = cb * cdiv64(M, 32 * b), per = cdiv64(steps, S);
-            if ((S - 1) * per < steps) best = {b, t, (int)cb, (int)tiles, (int)(S > 1 ? tiles - tiles % CUS : tiles), S, (int)per};
+            if ((S - 1) * per < steps) best = {b, t, (int)cb, (int)tiles, (int)(S > 1 ? tiles - tiles % CUS : tiles), S, (int)per, 0.0};
         }
     }
     return best;
@@ -432,12 +433,11 @@ TallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, 
 
 }  // namespace
 
-// Rows from which it replaces the 64-row streaming passes, and up to which it replaces dequantise + library GEMM (us, passes / tall):
-//   act 2:  7B gate_up 96 rows 46 / 37, 128 rows 47 / 40, 192 rows 69 / 49; 70B gate_up 96 rows 176 / 105, 256 rows 364 / 232
-//   act 0:  7B qkv 128 rows 26 / 32, 192 rows 47 / 36; o 128 rows 15 / 17, 192 rows 19 / 20; down 128 rows 27 / 25, 192 rows 43 / 32;
-//           70B down 128 rows 81 / 71, 256 rows 151 / 124
-// (library with its dequantisation / tall, the four GEMMs of a 7B layer) 3072 rows 1296 / 1159, 6000 rows 2418 / 2184, 8192 rows
+// Rows from which it may replace the 64-row streaming passes, and up to which it replaces dequantise + library GEMM:
+// (library with its dequantisation / tall, us, the four GEMMs of a 7B layer) 3072 rows 1296 / 1159, 6000 rows 2418 / 2184, 8192 rows
 // 2979 / 2993, 16128 rows 5542 / 5947: past 8192 rows hipBLASLt's 256 x 256 tiles, free of dequantisation, win (1.28 against 1.13 PFLOP/s).
+// (Over 30 shapes the library takes 1.07 - 1.21 times as long at each of 4096, 5000, 6144, 7168 and 8192 rows; 5120 x 15360 is the
+// shape it serves best: 752 / 778 at 5000 rows, 1166 / 1228 at 8192.)
 int64_t gptq::tall_min_m(int act) {
     static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 0;
     return v ? v : act == 2 ? 65 : 129;
@@ -446,13 +446,34 @@ int64_t gptq::tall_max_m() {
     static const int64_t v = getenv("TGIS_TALL_MAX_M") ? atoll(getenv("TGIS_TALL_MAX_M")) : 8192;
     return v;
 }
-bool gptq::tall_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act) {
-    if (M < tall_min_m(act) || perm != nullptr || act == 1 || K % 64 != 0) return false;
+bool gptq::tall_serves(int64_t K, int64_t groups, bool act_order, int act) {
+    if (act_order || act == 1 || K % 64 != 0 || groups <= 0) return false;
     const int64_t gs = K / groups, spg = gs / 64;
     return groups == 1 || (gs % 64 == 0 && (spg & (spg - 1)) == 0);
 }
+// Up to 256 rows the passes take k in parallel (k-parts, splits) where a tile here walks it alone, so it depends on the matrix which of
+// the two is done first.  us, the passes with the launch that adds their slabs / this kernel with a norm behind it (act 2: either alone):
+//   act 0:  2048 x 2560 at 129 / 256 rows 12.1 / 19.4, 15.4 / 19.7; 1024 x 1024 8.1 / 10.5, 8.7 / 11.3; 3072 x 5120 19.9 / 26.1, 32.7 /
+//           26.8; 4096 x 4096 21.9 / 20.6, 23.5 / 25.5; 2048 x 6144 25.1 / 20.0, 26.7 / 20.9; 4096 x 12288 50.4 / 39.6, 51.1 / 44.8;
+//           11008 x 4096 44.1 / 33.1, 45.9 / 38.4; 8192 x 10240 49.6 / 49.4, 87.1 / 59.5
+//   act 2:  2048 x 11264 at 65 / 128 / 129 rows 14.2 / 16.4, 14.3 / 16.7, 24.7 / 20.2; 4096 x 22016 48.3 / 35.8, 47.1 / 40.5, 67.7 / 48.1
+// The passes' time is that of their rounds of 256 blocks, each its chunks of 256 k per k-part (fitted to 30 shapes, within 8 %); the
+// choice is the faster one, or within 2 % of it, at all of these but 1024 x 8192 and 4096 x 2752, where it keeps the passes (up to 1.26).
+static bool pays_below_257_rows(int64_t M, int64_t K, int64_t N, int act) {
+    const gptq::GemmPlan pass = gptq::plan_gemm(K, N, act, M);
+    const double rounds = (double)cdiv64(cdiv64(cdiv64(N, 32), pass.TN) * cdiv64(M, 64) * pass.S, CUS), chunks = pass.KR / 256 / pass.WK;
+    const double passes = act == 2 ? 2.0 + rounds * (2.0 + chunks * (pass.TN == 4 ? 2.65 : 1.9))
+                                   : 5.0 + rounds * (3.0 + chunks * (pass.TN == 4 ? 2.45 : 1.65));
+    const TallPlan p = plan_tall(M, K, N);
+    const bool split = p.whole < p.tiles;  // (the model is 4 us above split plans)
+    return (split ? p.us - (act == 2 ? 4.0 : 3.5) : act == 2 ? p.us + 1.0 : 1.1 * p.us + 2.0) <= passes;
+}
+bool gptq::tall_ok(int64_t M, int64_t K, int64_t N, int64_t groups, bool act_order, int act) {
+    if (M < tall_min_m(act) || !tall_serves(K, groups, act_order, act)) return false;
+    return M > 256 || getenv("TGIS_TALL_MIN_M") || getenv("TGIS_TALL_PLAN") || pays_below_257_rows(M, K, N, act);
+}
 bool gptq::tall_partial_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act) {
-    return M >= 257 && act == 0 && tall_ok(M, K, groups, perm, act);
+    return M >= 257 && act == 0 && tall_serves(K, groups, perm != nullptr, act);
 }
 int64_t gptq::tall_workspace_bytes(int64_t M, int64_t K, int64_t N) { return plan_scratch(plan_tall(M, K, N)); }
 

@@ -21,7 +21,7 @@ import os
 
 # rows up to which the dense weight-streaming MFMA kernel is used (one pass over the weights per 32 / 64 rows); above,
 # hipBLASLt.  GPTQ linears ask the library how far its fused kernels reach (GptqWeight.fused_rows: 64-row streaming passes
-# to 256 rows, then the tall fused kernel to ~3k rows; beyond that dequantise once + hipBLASLt, exllamav2.py:87).
+# to 256 rows, the tall kernel from 65 / 129 rows where it is faster to 8192; beyond that dequantise once + hipBLASLt, exllamav2.py:87).
 SKINNY_MAX_M = int(os.getenv("TGIS_SKINNY_MAX_M", "256"))
 # fuse the split-K reduce of decode-sized GPTQ GEMMs into the consumer kernel (rmsnorm / rope+KV write)
 DEFER_REDUCE = os.getenv("TGIS_DEFER_REDUCE", "true").lower() not in ("0", "false")
@@ -164,6 +164,7 @@ class Ex4bitLinearV2:
         self.rope_handle: Optional[native.GptqWeight] = None
         self._perm: Optional[torch.Tensor] = None  # see `perm`
         self._fused = {}  # act -> rows up to which the library's fused kernels are used
+        self._whole = {}  # (rows, act) -> whether the library finishes the sums by itself
 
     def post_init(self):
         handle = native.GptqWeight(self.qweight, self.qzeros, self.scales, self.g_idx, self.bits, self.groupsize,
@@ -211,6 +212,14 @@ class Ex4bitLinearV2:
             got = self._fused[act] = self.ordered.fused_rows(act)
         return got
 
+    def _whole_sums(self, rows: int, act: int) -> bool:
+        if rows <= 64 or self._fused_rows(act) <= 256:
+            return False
+        got = self._whole.get((rows, act))  # (up to 256 rows: PARTIAL_MAX_M)
+        if got is None:
+            got = self._whole[(rows, act)] = self.ordered.whole_sums(rows, act)
+        return got
+
     def _dequant_scratch(self) -> torch.Tensor:
         key = (str(self.device), self.height, self.width)
         buf = Ex4bitLinearV2._temp_dq.get(key)
@@ -253,8 +262,8 @@ class Ex4bitLinearV2:
             if x.shape[0] <= self._fused_rows(2):
                 return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=2)
             return native.act_mul(self._large_m(x), self.width // 2)
-        # past 128 rows the tall kernel finishes its own sums sooner than a consumer adds the slabs of 64-row passes
-        if partial and x.shape[0] <= (128 if self._fused_rows(act) > 256 else native.PARTIAL_MAX_M) and DEFER_REDUCE:
+        # where the tall kernel finishes its own sums sooner than a consumer adds the slabs of 64-row passes, nothing is deferred
+        if partial and x.shape[0] <= native.PARTIAL_MAX_M and DEFER_REDUCE and not self._whole_sums(x.shape[0], act):
             return native.gptq_gemm_partial(x, self.ordered, bias=self.bias, act=act)
         if x.shape[0] <= self._fused_rows(act):
             return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=act)
