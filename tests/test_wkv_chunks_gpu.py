@@ -161,3 +161,42 @@ def test_values_that_are_not_finite_stay_with_later_tokens(gpu_device, dtype, ba
         assert ((got[a:a + s] - clean[a:a + s]).abs() <= tol * (1 + clean[a:a + s].abs())).all(), b
         assert not got[a + s:e, 0, 7].isfinite().any(), b
         assert torch.equal(got[a:e, 1], clean[a:e, 1]), b  # the other head
+
+
+# heads and ranks on each side of what the step launch is for
+@pytest.mark.parametrize("d,rank,stepped", [(64, 64, True), (64, 65, False), (32, 16, True), (68, 32, False), (128, 64, False)])
+def test_single_tokens_of_a_mixer(gpu_device, monkeypatch, d, rank, stepped):
+    """A decode step of the mixer takes the step launch where it pays, and the decay and the scan elsewhere, with the same result."""
+    from types import SimpleNamespace
+
+    from tgis_amd import native
+    from tgis_amd.utils.mixers import WkvMixer
+
+    H, B = 2, 3
+    W = HD = H * d
+    g = torch.Generator().manual_seed(d + rank)
+    shapes = {**{f"m.mu.{s}": (W,) for s in WkvMixer.MIXES}, **{f"m.{s}": (HD, W) for s in "rkvgo"}, "m.w1": (rank, W), "m.w2": (HD, rank),
+              "m.w0": (HD,), "m.u": (H, d), "m.norm": (HD,)}
+    t = {n: (torch.randn(s, generator=g) * (W ** -0.5 if len(s) == 2 else 0.3)).bfloat16().to(gpu_device) for n, s in shapes.items()}
+    weights = SimpleNamespace(get_tensor=lambda n, **kw: t[n], dtype=torch.bfloat16, device=gpu_device)
+    m = WkvMixer(weights, "m", 0, H, d, 1e-5)
+    state, shift = torch.randn(B, H, d, d, generator=g).to(gpu_device), torch.randn(B, W, generator=g).to(gpu_device)
+    calls = []
+    real = native.wkv_step
+    monkeypatch.setattr(native, "wkv_step", lambda *a: calls.append(1) or real(*a))
+    index = torch.arange(B + 1, dtype=torch.int32, device=gpu_device)
+    h = torch.randn(B, W, generator=g).to(gpu_device)
+    pos = torch.full((B,), 9, dtype=torch.int32, device=gpu_device)
+    out = []
+    for pays in (None, True, False):
+        if pays is not None:
+            monkeypatch.setattr(native, "wkv_step_pays", lambda *a: pays and d % 4 == 0)
+        kept = SimpleNamespace(state=[state.clone()], shift=[shift.clone()])
+        step = SimpleNamespace(state=kept, state_slots=index[:B], cu_seqlens_q=index, max_q_len=1)
+        m.defer = False
+        out.append(torch.cat([m.forward(h, pos, step, torch.bfloat16).float().flatten(), kept.state[0].flatten(), kept.shift[0].flatten()]))
+        assert bool(calls) == (stepped if pays is None else pays)
+        calls.clear()
+    # fp32 sums in other orders, rounded to bf16 once before and once behind the output projection
+    for a in out[1:]:
+        assert ((a - out[0]).abs() <= 2.0 ** -6 * (out[0].abs() + out[0].square().mean().sqrt())).all()

@@ -1104,6 +1104,15 @@ def wkv_scan(r, k, v, gate, logw, u, gain, state, shift_state, h, state_slots, c
 WKV_STEP_MAX_RANK = 1024
 
 
+def wkv_step_pays(d: int, rank: int) -> bool:
+    """Whether single tokens should take wkv_step: it makes the decay again for every (sequence, head), from columns of w2t that the launch
+    of wkv_decay shares, and keeps twice the state rows per thread where heads are wider than 64.  us, decay and scan / step, heads of 64:
+    rank 64 at 1, 24, 256 sequences of 32 heads 7.2 / 6.2, 12.4 / 9.6, 80 / 74; rank 128 of 64 heads 8.5 / 9.4, 26.3 / 25.7, 178 / 248; rank
+    256 9.6 / 12.7, 17.9 / 23.9, 98 / 179; rank 1024 20.7 / 37.9, 44 / 78, 167 / 628.  Heads of 128, rank 64, 16 heads: 8.0 / 10.0, 18.9 /
+    19.0, 136 / 174."""
+    return d % 4 == 0 and d <= 64 and rank <= 64
+
+
 def wkv_step(r, k, v, gate, low, w2t, w0, u, gain, state, shift_state, h, state_slots, cu_seqlens_q, positions, H: int, d: int, eps: float):
     """wkv_scan with the decay made from low [T, rank] on the way (wkv_decay): the form for steps of single tokens.  d % 4 == 0."""
     T, ld = r.shape[0], r.stride(0)

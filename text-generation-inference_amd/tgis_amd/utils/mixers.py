@@ -156,7 +156,7 @@ class WkvMixer:
             for i, lin in enumerate(self.proj):
                 lin(mixes[i], out=rkvg[i])
             low = self.w1(mixes[4])
-        if T == step.state_slots.shape[0] and self.d % 4 == 0 and self.w2t.shape[0] <= native.WKV_STEP_MAX_RANK:  # a token each
+        if T == step.state_slots.shape[0] and native.wkv_step_pays(self.d, self.w2t.shape[0]):  # a token each
             out = native.wkv_step(rkvg[0], rkvg[1], rkvg[2], rkvg[3], low, self.w2t, self.w0, self.u, self.gain, state, shift, h32,
                                   step.state_slots, step.cu_seqlens_q, position_ids, self.H, self.d, self.eps)
             return self.o(out, partial=self.defer)
