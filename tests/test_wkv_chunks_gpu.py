@@ -200,3 +200,36 @@ def test_single_tokens_of_a_mixer(gpu_device, monkeypatch, d, rank, stepped):
     # fp32 sums in other orders, rounded to bf16 once before and once behind the output projection
     for a in out[1:]:
         assert ((a - out[0]).abs() <= 2.0 ** -6 * (out[0].abs() + out[0].square().mean().sqrt())).all()
+
+
+# (heads, sequences, head width): more blocks than a CU holds of the chunk kernel, and not more; runs: the longest that is walked by token, one more
+@pytest.mark.parametrize("H,B,d,by_token", [(8, 40, 64, True), (8, 32, 64, False), (6, 90, 32, True), (6, 40, 32, False), (3, 90, 68, False)])
+@pytest.mark.parametrize("longest", [1, 10, 11, 16, 17, 18])
+def test_scan_of_short_runs(gpu_device, H, B, d, by_token, longest):
+    """Many short runs: the bits of the token-by-token walk where it is chosen (rows that are no groups of four take it always)."""
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(H + B + longest)
+    lens = torch.randint(0, longest + 1, (B,), generator=g)
+    lens[B // 2] = longest
+    T, W = int(lens.sum()), 8
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)]).int().to(gpu_device)
+    rkvg = [torch.randn(T, H * d, generator=g).bfloat16().to(gpu_device) for _ in range(4)]
+    logw = -torch.exp(torch.randn(T, H * d, generator=g) - 1.0).to(gpu_device)
+    u, gain, state = (torch.randn(*s, generator=g).to(gpu_device) for s in ((H * d,), (H * d,), (B, H, d, d)))
+    slots, pos = torch.randperm(B, generator=g).int().to(gpu_device), torch.randint(0, 2, (T,), generator=g).int().to(gpu_device)
+
+    def scan(pad, hint):
+        rows = [torch.nn.functional.pad(t, (0, pad))[:, :H * d] for t in rkvg]
+        st = state.clone()
+        out = native.wkv_scan(*rows, logw, u, gain, st, torch.zeros(B, W, device=gpu_device), torch.zeros(T, W, device=gpu_device), slots, cu, pos, H, d,
+                              1e-5, max_q_len=hint)
+        return out.float(), st
+
+    walked, walked_st = scan(2, 0)
+    got, got_st = scan(0, longest)
+    if by_token and (longest <= 10 or longest == 17):
+        assert torch.equal(got, walked) and torch.equal(got_st, walked_st)
+    # fp32 sums in another order, one rounding to bf16
+    assert ((got - walked).abs() <= 2.0 ** -7 * (walked.abs() + walked.square().mean().sqrt())).all()
+    assert (got_st - walked_st).abs().max() <= 1e-5 * walked_st.abs().max()

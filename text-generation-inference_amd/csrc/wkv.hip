@@ -681,15 +681,25 @@ __global__ __launch_bounds__(STEP_THREADS) void wkv_step_kernel(
     }
 }
 
+// Steps whose longest run has a few tokens, or a few more than a chunk, with more blocks than a CU holds at once (its registers let it hold
+// one of the chunk kernel up to d = 64, two up to 32; four of the token-by-token one), walk their tokens one by one.  us, token by token /
+// chunks, d 64: 24 sequences x 32 heads of 1, 5, 8, 12, 16, 17, 20 tokens 9.9 / 12.2, 12.3 / 17.7, 13.9 / 17.8, 17.5 / 18.0, 20.9 / 19.1, 22.6 /
+// 25.1, 24.6 / 25.2; 32 x 64 heads of 5 29.0 / 41.6; but 8 x 32 heads of 5 9.1 / 8.0.  d 32: 24 x 32 heads of 5, 12, 16, 17, 20 8.1 / 12.2, 11.2 /
+// 12.4, 13.0 / 12.4, 14.2 / 17.1, 15.3 / 16.9; 16 x 32 of 5 7.5 / 7.6.  d 128, 32 x 16 heads of 5: by 1.15 in chunks.
+bool runs_by_token(int64_t blocks, int d, int64_t max_q_len) {
+    if (max_q_len < 1 || d > 64 || blocks <= (d <= 32 ? 512 : 256)) return false;
+    return max_q_len <= CHUNK ? max_q_len <= (d <= 32 ? 12 : 10) : max_q_len <= (d <= 32 ? 20 : 17);
+}
+
 template <typename T>
 int launch_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw, const float* u,
                 const float* gain, float* state, float* shift_state, const float* h, int64_t W, const int32_t* slots,
                 const int32_t* cu_q, const int32_t* positions, void* out, int64_t ld_out, int B, int H, int d, float eps,
-                hipStream_t st) {
+                int64_t max_q_len, hipStream_t st) {
     // the chunked form takes rows in groups of four elements (any head width that is a multiple of 4, aligned tensors)
     const size_t quad = 4 * sizeof(T);
     auto rows_of_four = [&](const void* p, int64_t stride) { return (uintptr_t)p % quad == 0 && stride % 4 == 0; };
-    if (d % 4 == 0 && rows_of_four(r, ld) && rows_of_four(k, ld) && rows_of_four(v, ld) && rows_of_four(gate, ld) &&
+    if (!runs_by_token((int64_t)B * H, d, max_q_len) && d % 4 == 0 && rows_of_four(r, ld) && rows_of_four(k, ld) && rows_of_four(v, ld) && rows_of_four(gate, ld) &&
         rows_of_four(out, ld_out) && (uintptr_t)logw % 16 == 0 && (uintptr_t)u % 16 == 0 && (uintptr_t)gain % 16 == 0 &&
         (uintptr_t)state % 16 == 0) {
 #define TGIS_WKV_CHUNKS(DM)                                                                                                    \
@@ -779,10 +789,10 @@ extern "C" int tgis_wkv_decay(const void* a, int64_t ld_a, const float* w2t, con
     return TGIS_OK;
 }
 
-extern "C" int tgis_wkv_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
-                             const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
-                             const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
-                             int64_t ld_out, int64_t B, int H, int d, float eps, int dtype, void* stream) {
+extern "C" int tgis_wkv_scan_runs(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
+                                  const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
+                                  const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
+                                  int64_t ld_out, int64_t B, int H, int d, float eps, int64_t max_q_len, int dtype, void* stream) {
     TGIS_CHECK_ARG(r && k && v && gate && logw && u && gain && state && shift_state && h && state_slots && cu_seqlens_q &&
                        positions && out,
                    "tgis_wkv_scan: null tensor");
@@ -791,13 +801,21 @@ extern "C" int tgis_wkv_scan(const void* r, const void* k, const void* v, const 
     hipStream_t st = (hipStream_t)stream;
     TgisTimedScope timed(TGIS_OP_SCAN, st);
     if (dtype == TGIS_F16)
-        launch_scan<f16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, st);
+        launch_scan<f16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, max_q_len, st);
     else if (dtype == TGIS_BF16)
-        launch_scan<bf16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, st);
+        launch_scan<bf16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, max_q_len, st);
     else
-        launch_scan<float>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, st);
+        launch_scan<float>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, max_q_len, st);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
+}
+
+extern "C" int tgis_wkv_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
+                             const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
+                             const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
+                             int64_t ld_out, int64_t B, int H, int d, float eps, int dtype, void* stream) {
+    return tgis_wkv_scan_runs(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, B, H,
+                              d, eps, 0, dtype, stream);
 }
 
 // rows of groups of four aligned elements, as the chunk form wants them; d <= 128, rank <= STEP_MAX_RANK

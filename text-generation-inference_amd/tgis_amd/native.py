@@ -111,6 +111,8 @@ SIGNATURES = {
                                _c_i64, _c_i64, _c_int, _c_int, _c_f, _c_int, _vp]),
     "tgis_wkv_scan": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64,
                                _c_i64, _c_int, _c_int, _c_f, _c_int, _vp]),
+    "tgis_wkv_scan_runs": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64,
+                               _c_i64, _c_int, _c_int, _c_f, _c_i64, _c_int, _vp]),
     "tgis_moe_row_capacity": (_c_i64, [_c_i64, _c_i64, _c_int]),
     "tgis_moe_route": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int, _c_int, _vp]),
     "tgis_moe_align": (_c_int, [_vp, _c_i64, _c_int, _vp, _c_i64, _vp, _vp, _vp, _c_int, _vp]),
@@ -1087,17 +1089,19 @@ def wkv_decay(a, w2t, w0):
     return out
 
 
-def wkv_scan(r, k, v, gate, logw, u, gain, state, shift_state, h, state_slots, cu_seqlens_q, positions, H: int, d: int, eps: float):
-    """r / k / v / gate [T, H d] views with one common row stride; returns [T, H d]."""
+def wkv_scan(r, k, v, gate, logw, u, gain, state, shift_state, h, state_slots, cu_seqlens_q, positions, H: int, d: int, eps: float,
+             max_q_len: int = 0):
+    """r / k / v / gate [T, H d] views with one common row stride; returns [T, H d].  max_q_len: the longest run of
+    a sequence in the step, 0 where it is not known."""
     T = r.shape[0]
     ld = r.stride(0)
     assert all(t.stride(0) == ld and t.stride(1) == 1 and t.dtype == r.dtype for t in (k, v, gate))
     out = torch.empty((T, H * d), dtype=r.dtype, device=r.device)
-    _check(load_library().tgis_wkv_scan(
+    _check(load_library().tgis_wkv_scan_runs(
         _ptr(r), _ptr(k), _ptr(v), _ptr(gate), ld, _f32(logw, "logw"), _f32(u, "u"), _f32(gain, "gain"), _f32(state, "state"),
         _f32(shift_state, "shift_state"), _f32(h, "h"), h.shape[1], _i32(state_slots, "state_slots"),
         _i32(cu_seqlens_q, "cu_seqlens_q"), _i32(positions, "positions"), _ptr(out), out.stride(0), state_slots.shape[0], H, d,
-        float(eps), dtype_code3(r.dtype), _stream()), "tgis_wkv_scan")
+        float(eps), int(max_q_len), dtype_code3(r.dtype), _stream()), "tgis_wkv_scan_runs")
     return out
 
 

@@ -162,7 +162,7 @@ class WkvMixer:
             return self.o(out, partial=self.defer)
         logw = native.wkv_decay(low, self.w2t, self.w0)
         out = native.wkv_scan(rkvg[0], rkvg[1], rkvg[2], rkvg[3], logw, self.u, self.gain, state, shift, h32, step.state_slots,
-                              step.cu_seqlens_q, position_ids, self.H, self.d, self.eps)
+                              step.cu_seqlens_q, position_ids, self.H, self.d, self.eps, max_q_len=step.max_q_len)
         return self.o(out, partial=self.defer)
 
 
