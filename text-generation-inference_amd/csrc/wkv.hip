@@ -53,7 +53,8 @@ __global__ __launch_bounds__(256) void token_shift_mix_kernel(const float* __res
 
 // grid (TB tokens, 256-channel block): logw[t][c] = -exp(w0[c] + sum_r tanh(a[t][r]) * w2t[r][c])
 // TB tokens share a read of w2t's columns: with one token per workgroup a 4 x 1024-token step reads the 512 KiB matrix 4096 times from
-// L2 (rank 64, 4096 x 2048: 79 -> 39 us).  TB 8 from 1024 tokens on; below, single tokens keep the chip filled.
+// L2 (rank 64, 4096 x 2048: 79 -> 39 us).  TB 8 from 1024 tokens on where that leaves a workgroup per CU (1024 x 512, rank 64: 7.1 / 7.0; 1024 x
+// 256 5.5 / 6.8); else single tokens keep the chip filled.
 template <typename T, int TB>
 __global__ __launch_bounds__(256) void wkv_decay_kernel(const T* __restrict__ a, int64_t ld_a, const float* __restrict__ w2t,
                                                         const float* __restrict__ w0, float* __restrict__ logw, int R, int64_t C,
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(256) void wkv_decay_kernel(const T* __restrict__ a,
     const int64_t t0 = (int64_t)blockIdx.x * TB;
     const int n = (int)min((int64_t)TB, Ttot - t0);
     for (int i = threadIdx.x; i < R * TB; i += blockDim.x) {
-        const int t = i / R, rr = i - t * R;
+        const int t = TB == 1 ? 0 : i / R, rr = i - t * R;
         th[rr * TB + t] = t < n ? tanhf(ldf(a + (t0 + t) * ld_a + rr)) : 0.f;
     }
     __syncthreads();
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(256) void wkv_decay_kernel(const T* __restrict__ a,
     const float z0 = w0[c];
 #pragma unroll
     for (int t = 0; t < TB; ++t) z[t] = z0;
-#pragma unroll 16
+#pragma unroll (TB == 1 ? 8 : 16)
     for (int rr = 0; rr < R; ++rr) {
         const float w = w2t[(int64_t)rr * C + c];
 #pragma unroll
@@ -768,7 +769,7 @@ extern "C" int tgis_wkv_decay(const void* a, int64_t ld_a, const float* w2t, con
     TGIS_CHECK_ARG(a && w2t && w0 && logw && rank >= 1 && rank <= 8192 && C >= 1 && C <= 65535 * 256 && ld_a >= rank && dtype3(dtype), "tgis_wkv_decay: bad arguments");
     if (T == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    const int tb = T >= 1024 && rank <= 512 ? 8 : 1;
+    const int tb = T >= 1024 && rank <= 512 && cdiv64(T, 8) * cdiv64(C, 256) >= 256 ? 8 : 1;
     const size_t lds = (size_t)rank * tb * sizeof(float);
     const dim3 grid((unsigned)cdiv64(T, tb), (unsigned)cdiv64(C, 256));
 #define TGIS_DECAY(TT)                                                                                                              \
