@@ -23,7 +23,8 @@ __device__ __forceinline__ int seq_of_token(const int32_t* __restrict__ cu_q, in
 }
 
 // grid (token, block of 256 x VEC columns); out[s][t][c], s < NM.  Bound by its writes (one fp32 row in, NM two-byte rows out): VEC 4
-// stores 8 or 16 bytes per thread (4096 x 2048, five mixes: 47 -> 29 us), 1 is for widths that are not multiples of 4.
+// stores 8 or 16 bytes per thread (4096 x 2048, five mixes: 47 -> 29 us), 1 is for widths that are not multiples of 4 and for small steps,
+// where it is more workgroups (us, VEC 1 / 4: 1 x 2048 2.8 / 3.0, 64 x 2048 2.9 / 3.1, 128 x 2048 3.4 / 3.3, 300 x 2048 5.4 / 4.7).
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void token_shift_mix_kernel(const float* __restrict__ h, const float* __restrict__ shift_state,
                                                               const int32_t* __restrict__ state_slots, const int32_t* __restrict__ cu_q,
@@ -741,7 +742,7 @@ extern "C" int tgis_token_shift_mix(const float* h, const float* shift_state, co
     TGIS_CHECK_ARG(B >= 1 && num_mixes >= 1 && W >= 1 && dtype3(dtype), "tgis_token_shift_mix: bad arguments");
     if (T == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
-    const bool vec = W % 4 == 0 && (uintptr_t)h % 16 == 0 && (uintptr_t)shift_state % 16 == 0 && (uintptr_t)mu % 16 == 0 &&
+    const bool vec = T * W >= 196608 && W % 4 == 0 && (uintptr_t)h % 16 == 0 && (uintptr_t)shift_state % 16 == 0 && (uintptr_t)mu % 16 == 0 &&
                      (uintptr_t)out % (dtype == TGIS_F32 ? 16 : 8) == 0;
     const dim3 grid((unsigned)T, (unsigned)cdiv64(W, vec ? 1024 : 256));
 #define TGIS_SHIFT(TT)                                                                                                             \
