@@ -61,7 +61,9 @@ def test_linear_takes_whole_sums_past_128_rows(gpu_device):
 
 
 # K: half a k64-step, whole ones, a ragged last; N: one tile, a block of eight and ragged ones; groups shorter than a step
-@pytest.mark.parametrize("K,N,groupsize", [(32, 32, 32), (96, 288, 32), (256, 256, 128), (320, 544, 64), (160, 1024, 160)])
+# (and a matrix on each side of the 768 blocks of eight tiles)
+@pytest.mark.parametrize("K,N,groupsize", [(32, 32, 32), (96, 288, 32), (256, 256, 128), (320, 544, 64), (160, 1024, 160), (2016, 6112, 32),
+                                           (2048, 5888, 128)])
 @pytest.mark.parametrize("image", ["plain", "gate_up", "rope"])
 def test_dequant_bits(gpu_device, K, N, groupsize, image):
     """The image back to [K, N]: the bits of the reference formula, from each column order, into aligned and unaligned memory."""

@@ -180,20 +180,22 @@ int gptq::reduce_slabs(const float* slabs, const f16* bias, f16* out, int64_t ld
 
 namespace {
 
-// The image back to [K][N] f16.  A workgroup takes one k64-step of eight neighbouring tiles: a KiB per tile straight from the image, 32 k
+// The image back to [K][N] f16.  A workgroup takes one k64-step of DQ_TILES neighbouring tiles: a KiB per tile straight from the image, 32 k
 // of a column per lane, and through LDS, so that rows leave in 16-byte pieces, 512 contiguous bytes of a plain image (256 + 256 of a
 // gate | up one).  Bound by the bytes: one 2-byte store per value and lane it was bound by its stores (7B, us before / now: qkv 4096 x 12288 34 / 22, gate_up
-// 4096 x 22016 88 / 37, down 11008 x 4096 33 / 21).
-constexpr int DQ_TILES = 8, DQ_ROW = DQ_TILES * 32 + 8;
+// 4096 x 22016 88 / 37, down 11008 x 4096 33 / 21).  Eight tiles where that makes three workgroups per CU, two on smaller matrices (us, before /
+// eight / two: 1024 x 1024 3.9 / 5.6 / 4.2, 2048 x 2560 7.0 / 7.3 / 6.2, 2048 x 6144 11.7 / 9.7 / 9.7, 4096 x 4096 14.2 / 11.7 / 12.1).
+template <int DQ_TILES>
 __global__ __launch_bounds__(256) void gptq_dequant_kernel(const uint8_t* __restrict__ prep, int64_t offB, f16* __restrict__ wout, int K,
                                                            int N, int G, int gs, int NT, int KS, int flags, int vec) {
+    constexpr int DQ_ROW = DQ_TILES * 32 + 8;
     __shared__ __attribute__((aligned(16))) f16 tile[64 * DQ_ROW];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int ksteps = (K + 63) >> 6, ks = blockIdx.x % ksteps, nt0 = blockIdx.x / ksteps * DQ_TILES;
 #pragma unroll
-    for (int r = 0; r < DQ_TILES / 4; ++r) {
+    for (int r = 0; r < (DQ_TILES + 3) / 4; ++r) {
         const int t = r * 4 + w, nt = nt0 + t;
-        if (nt >= NT) break;
+        if (t >= DQ_TILES || nt >= NT) break;
         const u32x4 q = *reinterpret_cast<const u32x4*>(prep + (((int64_t)nt * KS + ks) * 64 + lane) * 16);
         const uint32_t* sz = reinterpret_cast<const uint32_t*>(prep + offB) + (int64_t)nt * G * 32 + (lane & 31);
 #pragma unroll
@@ -694,9 +696,13 @@ extern "C" int tgis_gptq_dequant_f16(const void* prepared, void* w_out, int64_t 
     TGIS_CHECK_ARG(prepared && w_out && K > 0 && N > 0 && groups > 0 && K % groups == 0,
                    "tgis_gptq_dequant_f16: bad arguments");
     PrepLayout p = prep_layout(K, N, groups);
-    hipLaunchKernelGGL(gptq_dequant_kernel, dim3((unsigned)(cdiv64(p.NT, DQ_TILES) * cdiv64(K, 64))), dim3(256), 0, (hipStream_t)stream,
-                       (const uint8_t*)prepared, p.offB, (f16*)w_out, (int)K, (int)N, (int)groups, (int)(K / groups), (int)p.NT, (int)p.KS,
-                       flags, ((uintptr_t)w_out & 15) == 0 && N % 8 == 0);
+    const int64_t ksteps = cdiv64(K, 64), blocks = cdiv64(p.NT, 8) * ksteps;
+    const int vec = ((uintptr_t)w_out & 15) == 0 && N % 8 == 0;
+#define TGIS_DEQUANT(TILES)                                                                                                              \
+    hipLaunchKernelGGL((gptq_dequant_kernel<TILES>), dim3((unsigned)(cdiv64(p.NT, TILES) * ksteps)), dim3(256), 0, (hipStream_t)stream, \
+                       (const uint8_t*)prepared, p.offB, (f16*)w_out, (int)K, (int)N, (int)groups, (int)(K / groups), (int)p.NT, (int)p.KS, flags, vec)
+    if (blocks < 768) TGIS_DEQUANT(2); else TGIS_DEQUANT(8);
+#undef TGIS_DEQUANT
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
