@@ -8,17 +8,20 @@ pytestmark = pytest.mark.gpu
 
 
 def _pages(k, v, lens, layout, order):
-    """k, v: per sequence [ctx, G, D] -> pools of 32-token pages dealt in `order`, and the block table."""
+    """k, v: per sequence [ctx, G, D] -> pools of 32-token pages dealt in `order`, and the block table.  What is past a context, the page that
+    no sequence owns and the table entries past a sequence's pages (which name it) hold large values of either sign: a previous owner's."""
     G, D = k[0].shape[1:]
     per = [(n + 31) // 32 for n in lens]
-    kp, vp = torch.zeros(sum(per), G, 32 * D, dtype=k[0].dtype), torch.zeros(sum(per), G, 32 * D, dtype=k[0].dtype)
-    table = torch.zeros(len(lens), max(per), dtype=torch.int32)
+    dice = torch.Generator().manual_seed(len(order))
+    stale = lambda *shape: (60000 * (2 * torch.randint(0, 2, shape, generator=dice) - 1)).to(k[0].dtype)
+    kp, vp = stale(sum(per) + 1, G, 32 * D), stale(sum(per) + 1, G, 32 * D)
+    table = torch.full((len(lens), max(per) + 2), sum(per), dtype=torch.int32)
     it = iter(order)
     for b, n in enumerate(lens):
         for p in range(per[b]):
             page = next(it)
             table[b, p] = page
-            kb, vb = torch.zeros(32, G, D, dtype=kp.dtype), torch.zeros(32, G, D, dtype=kp.dtype)
+            kb, vb = stale(32, G, D), stale(32, G, D)
             m = min(32, n - 32 * p)
             kb[:m], vb[:m] = k[b][32 * p:32 * p + m], v[b][32 * p:32 * p + m]
             kb, vb = kb.transpose(0, 1), vb.transpose(0, 1)  # [G, 32, D]
@@ -28,7 +31,7 @@ def _pages(k, v, lens, layout, order):
                 kp[page] = kb.reshape(G, 2, 16, D // 8, 8).transpose(2, 3).reshape(G, -1)
                 tok = torch.arange(32)
                 col = (tok % 16 // 4) * 8 + tok // 16 * 4 + tok % 4
-                cols = torch.zeros(G, 32, D, dtype=kp.dtype)
+                cols = torch.empty(G, 32, D, dtype=kp.dtype)
                 cols[:, col] = vb
                 vp[page] = cols.reshape(G, 4, 8, D).transpose(2, 3).reshape(G, -1)
     return kp, vp, table
@@ -50,7 +53,7 @@ def _oracle(q, k, v, scale):
                                          (20, 1, 128, torch.float16), (16, 8, 64, torch.bfloat16)])
 @pytest.mark.parametrize("layout", ["fragments", "rows"])
 @pytest.mark.parametrize("groups_per_wave", ["1", "2"])
-@pytest.mark.parametrize("runs", [((65, 65),), ((127, 127), (1, 40)), ((128, 128), (129, 129), (31, 32)), ((33, 97), (300, 300), (2, 2)), ((161, 500),)])
+@pytest.mark.parametrize("runs", [((65, 65),), ((17, 20), (64, 64), (70, 96)), ((127, 127), (1, 40)), ((128, 128), (129, 129), (31, 32)), ((33, 97), (300, 300), (2, 2)), ((161, 500),)])
 def test_against_float64(gpu_device, H, G, D, dtype, layout, groups_per_wave, runs, monkeypatch):
     from tgis_amd import native
 
