@@ -167,8 +167,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
         }
     };
     page_load(page_number(0), 0);
-    page_load(page_number(1), 1);
-    page_load(page_number(2), 2);
+    if (pages > 1) page_load(page_number(1), 1);
+    if (pages > 2) page_load(page_number(2), 2);
     int next = page_number(3);
 
     auto page_barrier = [&](auto later_) {  // all of this wave's loads but the last `later` pages', and after it everyone's
@@ -256,7 +256,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
         }
     };
     f32x4 s0[CG][2], s1[CG][2];
-    page_barrier(std::integral_constant<int, 2>{});
+    if (pages > 2)
+        page_barrier(std::integral_constant<int, 2>{});
+    else if (pages > 1)
+        page_barrier(std::integral_constant<int, 1>{});
+    else
+        page_barrier(std::integral_constant<int, 0>{});
     scores(0, s0);
     maxima(0, s0, std::true_type{});  // (nothing to rescale yet)
     auto arrive = [&](int p) {
@@ -275,7 +280,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
         attend(p + 1, s1, s0, std::false_type{});
     }
     for (const int own_pages = (wave_kmax + 31) >> 5; p < pages; ++p) {
-        arrive(p);
+        if (p + 2 < pages)  // (past the last page nothing is asked for: a short context has few pages to hide that behind)
+            page_barrier(std::integral_constant<int, 1>{});
+        else
+            page_barrier(std::integral_constant<int, 0>{});
+        if (p + 3 < pages) {
+            page_load(next, (p + 3) & 3);
+            next = page_number(p + 4);
+        }
         if (p >= own_pages) continue;
         attend(p, s0, s1, std::true_type{});
 #pragma unroll
