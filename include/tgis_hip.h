@@ -117,7 +117,8 @@ int tgis_gptq_fragments_ok(int64_t M, int64_t K, int64_t N, int64_t groups, int 
 /* out[M,N] f16 = x[M,K] f16 @ dequant(W)[K,N] (+ bias[N] f16 if non-NULL); fp32 accumulate.
  * Fused int4-dequant MFMA kernel for any M (rows are processed in slabs of 32).
  * x row stride ldx, out row stride ldo (elements).  perm (int32 [K] or NULL) gathers x columns
- * for act-order matrices.  act: 0 = none; 1 = x is [M,2K] and the kernel consumes silu(x[:, :K]) * x[:, K:]
+ * for act-order matrices, once per workgroup that reads them: it works, but the faster way is tgis_gather_columns (or a norm that gathers) in
+ * front and perm NULL, which is how this repository's linears call it.  act: 0 = none; 1 = x is [M,2K] and the kernel consumes silu(x[:, :K]) * x[:, K:]
  * while staging it; 2 = the image was prepared with TGIS_GPTQ_GATE_UP and out is [M, N/2] =
  * silu(gate) * up applied in the epilogue (both fuse LlamaMLP's activation, flash_llama_modeling.py:332-335). */
 int tgis_gptq_gemm_f16(const void* x, int64_t ldx, const void* prepared, const void* bias,
@@ -128,7 +129,8 @@ int tgis_gptq_gemm_f16(const void* x, int64_t ldx, const void* prepared, const v
  * `slabs` as fp32 [ceil(M/32)][S][32][ld] (ld = N rounded up to 32, returned in *slab_ld; S in *num_slabs, >= 1) for a
  * consumer that sums them in its prologue (tgis_rmsnorm_residual_partial / tgis_rope_kv_write_partial), which
  * removes the reduce launch.  The consumer rounds the sum (+bias) to f16 first, so results are bit-identical to
- * tgis_gptq_gemm_f16 followed by the plain consumer.  slabs must hold tgis_gptq_gemm_partial_bytes(M,K,N) bytes. */
+ * tgis_gptq_gemm_f16 followed by the plain consumer, where that runs the same 64-row passes (tgis_gptq_gemm_whole_sums 0; elsewhere its sums
+ * are taken in another order).  Meant for the few rows of decode steps and short prompts; any M works.  slabs must hold tgis_gptq_gemm_partial_bytes(M,K,N) bytes. */
 int64_t tgis_gptq_gemm_partial_bytes(int64_t M, int64_t K, int64_t N);
 int tgis_gptq_gemm_f16_partial(const void* x, int64_t ldx, const void* prepared, const int32_t* perm, int64_t M,
                                int64_t K, int64_t N, int64_t groups, int act, float* slabs, int64_t slabs_bytes,

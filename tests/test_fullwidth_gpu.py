@@ -436,8 +436,9 @@ def test_decode_attention_at_workload_context(gpu_device, name, B, H, Hkv, D, ct
                          # two 32-column tiles per wave (256-column blocks): taken once >= 384 such blocks remain
                          [(4096, 12288, 0, 2100), (4096, 22016, 2, 1100), (11008, 4096, 0, 3000), (4096, 4096, 0, 3072)])
 def test_gptq_tall_kernel_matches_oracle(gpu_device, K, N, act, M):
-    """64 < M: the fused tall kernel (one dequantisation per 128 rows, no scratch copy of W) at the cfg3 shapes, every
-    epilogue (plain, split-K + reduce, SiLU * up on the interleaved image, deferred slabs), ragged last row block."""
+    """64 < M: the 64-row passes and the tall kernel (one dequantisation per 64 - 128 rows, no scratch copy of W) at the cfg3 shapes, each
+    where it is chosen, every epilogue (plain, split tiles + finish, SiLU * up on the interleaved image, the passes' deferred slabs), ragged
+    last row block."""
     from tgis_amd import native
 
     qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, 128, seed=K + N + M)

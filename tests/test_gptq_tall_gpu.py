@@ -60,6 +60,27 @@ def test_linear_takes_whole_sums_past_128_rows(gpu_device):
             assert ((got.double().cpu() - want).abs() <= 2.0 ** -10 * want.abs() + 1e-5).all()
 
 
+def test_deferred_sums_at_any_row_count(gpu_device):
+    """The C entry's slabs past the rows that the linears defer."""
+    import ctypes
+
+    from tgis_amd import native
+
+    K, N, M = 512, 224, 300
+    qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, 128, seed=5)
+    w = native.GptqWeight(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), 4, 128)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half().to(gpu_device)
+    lib = native.load_library()
+    slabs = torch.full((lib.tgis_gptq_gemm_partial_bytes(M, K, N) // 4,), float("nan"), device=gpu_device)
+    S, ld = ctypes.c_int(), ctypes.c_int64()
+    assert lib.tgis_gptq_gemm_f16_partial(x.data_ptr(), K, w.image.data_ptr(), None, M, K, N, w.groups, 0, slabs.data_ptr(), slabs.numel() * 4,
+                                          ctypes.byref(S), ctypes.byref(ld), torch.cuda.current_stream().cuda_stream) == 0
+    units = (M + 31) // 32
+    got = slabs[:units * S.value * 32 * ld.value].view(units, S.value, 32, ld.value).sum(1).reshape(-1, ld.value)[:M, :N].double().cpu()
+    want = x.double().cpu() @ ops_ref.gptq_dequant(qw, qz, sc, gi, 128).half().double()
+    assert ((got - want).abs() <= 1e-5 * (1 + want.abs())).all()
+
+
 # K: half a k64-step, whole ones, a ragged last; N: one tile, a block of eight and ragged ones; groups shorter than a step
 # (and a matrix on each side of the 768 blocks of eight tiles)
 @pytest.mark.parametrize("K,N,groupsize", [(32, 32, 32), (96, 288, 32), (256, 256, 128), (320, 544, 64), (160, 1024, 160), (2016, 6112, 32),

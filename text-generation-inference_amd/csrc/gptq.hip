@@ -618,7 +618,6 @@ extern "C" int64_t tgis_gptq_gemm_partial_bytes(int64_t M, int64_t K, int64_t N)
     int64_t need = cdiv64(std::max<int64_t>(M, 1), 64) * 2 * pl.S * 32 * cdiv64(N, 32) * 32 * 4;
     if (M <= 64 && K % 64 == 0)  // the fragment-order kernel's plan may split further
         need = std::max<int64_t>(need, (int64_t)2 * gptq::wide_max_splits(K, N) * 32 * cdiv64(N, 32) * 32 * 4);
-    if (M >= 257 && K % 64 == 0) need = std::max(need, gptq::tall_slab_bytes(M, N, gptq::tall_partial_splits(M, K, N)));
     return need;
 }
 
@@ -646,14 +645,6 @@ extern "C" int tgis_gptq_gemm_f16_partial(const void* x, int64_t ldx, const void
     if (rc != TGIS_OK) return rc;
     TGIS_CHECK_ARG(M >= 1 && cdiv64(M, 32) <= 65535, "tgis_gptq_gemm_f16_partial: bad M");
     TGIS_CHECK_ARG(act != 2, "tgis_gptq_gemm_f16_partial: act=2 cannot be deferred");
-    if (gptq::tall_partial_ok(M, K, groups, perm, act)) {
-        const int S = gptq::tall_partial_splits(M, K, N);
-        TGIS_CHECK_ARG(slabs && slabs_bytes >= gptq::tall_slab_bytes(M, N, S), "tgis_gptq_gemm_f16_partial: slab buffer too small");
-        if (num_slabs) *num_slabs = S;
-        if (slab_ld) *slab_ld = cdiv64(N, 32) * 32;
-        TgisTimedScope timed(TGIS_OP_GPTQ_GEMM, (hipStream_t)stream);
-        return gptq::launch_tall_partial(x, ldx, prepared, M, K, N, groups, slabs, (hipStream_t)stream);
-    }
     GemmPlan pl = plan_gemm(K, N, 0, M);
     if (ldx == TGIS_LD_FRAGMENTS) {
         TGIS_CHECK_ARG(!perm && act == 0, "tgis_gptq_gemm_f16_partial: fragment-order activations: act 0, no act-order");

@@ -39,7 +39,7 @@ struct TallArgs {
     int M, K, N, NT, KS, G, spg_shift;
     int tile0, col_blocks;  // this launch: tiles tile0 + blockIdx.x, column blocks fastest
     int per, S;             // k64-steps per split, splits (blockIdx.y)
-    int mode;               // 0: finished output; 1: fp32 tiles [blockIdx.x][split][BM][BN] in `scratch`; 2: fp32 slabs in 32-row units
+    int part;               // 1: fp32 tiles [blockIdx.x][split][BM][BN] in `scratch` instead of the finished output
     int vec;                // rows of `out` take 16-byte stores
     float* scratch;
 };
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     const int c = lane & 31;
     auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
     constexpr int BN = 128 * TW;
-    if (a.mode == 1) {
+    if (a.part) {
         float* dst = a.scratch + ((int64_t)blockIdx.x * a.S + split) * (BM * BN) + w * (32 * TW) + c;
 #pragma unroll
         for (int t = 0; t < TW; ++t)
@@ -203,23 +203,6 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
             for (int rb = 0; rb < BMR; ++rb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(rb, r) * BN + t * 32] = acc[t][rb][r];
-        return;
-    }
-    if (a.mode == 2) {
-        const int64_t np = (int64_t)a.NT * 32;
-#pragma unroll
-        for (int t = 0; t < TW; ++t) {
-            const int nt = nt_raw0 + t;
-            if (nt >= a.NT) break;
-#pragma unroll
-            for (int rb = 0; rb < BMR; ++rb) {
-                const int unit = row_block * BMR + rb;
-                if (unit * 32 >= a.M) continue;
-                float* sl = a.scratch + ((int64_t)(unit * a.S + split) * 32) * np + nt * 32 + c;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sl[(int64_t)(row_of(rb, r) - rb * 32) * np] = acc[t][rb][r];
-            }
-        }
         return;
     }
     // finished: the tile goes through LDS so that rows leave in 16-byte pieces, 512 (256 with SiLU * up) contiguous bytes a row
@@ -307,7 +290,6 @@ __global__ __launch_bounds__(256) void tall_finish_kernel(TallArgs a) {
 
 // ---- how a GEMM is cut ----------------------------------------------------------------------------------------------------------
 constexpr int CUS = 256;
-constexpr int TKC = 2;  // k64-steps: granularity of the deferred form's splits
 
 struct TallPlan {
     int BMR, TW;
@@ -472,9 +454,6 @@ bool gptq::tall_ok(int64_t M, int64_t K, int64_t N, int64_t groups, bool act_ord
     if (M < tall_min_m(act) || !tall_serves(K, groups, act_order, act)) return false;
     return M > 256 || getenv("TGIS_TALL_MIN_M") || getenv("TGIS_TALL_PLAN") || pays_below_257_rows(M, K, N, act);
 }
-bool gptq::tall_partial_ok(int64_t M, int64_t K, int64_t groups, const int32_t* perm, int act) {
-    return M >= 257 && act == 0 && tall_serves(K, groups, perm != nullptr, act);
-}
 int64_t gptq::tall_workspace_bytes(int64_t M, int64_t K, int64_t N) { return plan_scratch(plan_tall(M, K, N)); }
 
 int gptq::launch_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo, int64_t M, int64_t K,
@@ -496,31 +475,10 @@ int gptq::launch_tall(const void* x, int64_t ldx, const void* prepared, const vo
         a.tile0 = p.whole;
         a.per = p.per;
         a.S = p.S;
-        a.mode = 1;
+        a.part = 1;
         const int rc = launch_shape<0>(p, a, p.tiles - p.whole, p.S, st);  // (fp32 tiles: the same for both activations)
         if (rc != TGIS_OK) return rc;
         return act == 2 ? launch_finish<2>(p, a, p.tiles - p.whole, st) : launch_finish<0>(p, a, p.tiles - p.whole, st);
     }
     return TGIS_OK;
-}
-
-// The deferred form: every tile split alike, so that a consumer can sum the slabs by rows.
-int gptq::tall_partial_splits(int64_t M, int64_t K, int64_t N) {
-    const int64_t blocks = cdiv64(cdiv64(N, 32), 4) * cdiv64(M, 128), chunks = cdiv64(K / 64, TKC);
-    int64_t S = blocks < 384 ? std::min<int64_t>(std::min<int64_t>(chunks, 16), cdiv64(512, blocks)) : 1;
-    const int64_t per = cdiv64(chunks, S);
-    while (S > 1 && (S - 1) * per >= chunks) --S;
-    return (int)S;
-}
-int64_t gptq::tall_slab_bytes(int64_t M, int64_t N, int S) { return cdiv64(M, 32) * S * 32 * cdiv64(N, 32) * 32 * 4; }
-
-int gptq::launch_tall_partial(const void* x, int64_t ldx, const void* prepared, int64_t M, int64_t K, int64_t N, int64_t groups,
-                              float* slabs, hipStream_t st) {
-    TallArgs a = tall_args(x, ldx, prepared, M, K, N, groups, slabs);
-    const int64_t chunks = cdiv64(K / 64, TKC);
-    a.S = tall_partial_splits(M, K, N);
-    a.per = (int)(cdiv64(chunks, a.S) * TKC);
-    a.mode = 2;
-    a.col_blocks = (int)cdiv64(a.NT, 4);
-    return launch_blocks<4, 0, 1>(a, (int)(a.col_blocks * cdiv64(M, 128)), a.S, st);
 }
