@@ -7,9 +7,10 @@ from oracle import ops_ref
 pytestmark = pytest.mark.gpu
 
 
-# K: one step, fewer and more steps than the ring of buffers, a whole number of rings; N: one tile, ragged and several column blocks
-@pytest.mark.parametrize("K,N,groupsize", [(64, 32, 64), (192, 288, 64), (320, 512, 64), (1024, 1120, 128), (1152, 96, 1152)])
-@pytest.mark.parametrize("M", [129, 161, 300])
+# K: one step, fewer and more steps than the ring of buffers, a whole number of rings; N: one tile, ragged and several column blocks; the last
+# size has more tiles than the 256 of a whole round, so that a split plan launches whole tiles and split ones behind them
+@pytest.mark.parametrize("K,N,groupsize,M", [(*shape, M) for shape in [(64, 32, 64), (192, 288, 64), (320, 512, 64), (1024, 1120, 128), (1152, 96, 1152)]
+                                             for M in (129, 161, 300)] + [(320, 4128, 64, 700)])
 @pytest.mark.parametrize("act", [0, 2])
 def test_every_plan(gpu_device, K, N, groupsize, M, act, monkeypatch):
     from tgis_amd import native
@@ -29,8 +30,9 @@ def test_every_plan(gpu_device, K, N, groupsize, M, act, monkeypatch):
         want = (torch.nn.functional.silu(gate.float()).half().float() * up.float()).half().double()
         tol = 3 * ulp * (gate.double() * up.double()).abs() + 1e-5
     cols = want.shape[1]
-    # (a launch that splits needs at least one k64-step per split)
-    plans = [None] + [f"{b},{t},{s}" for b in (2, 3, 4) for t in (1, 2) for s in (1, 2, 5) if s == 1 or K // 64 >= 2 * s]
+    # (the last split needs a k64-step of its own)
+    steps = K // 64
+    plans = [None] + [f"{b},{t},{p}" for b in (2, 3, 4) for t in (1, 2) for p in (1, 2, 5) if (p - 1) * -(-steps // p) < steps]
     for plan in plans:
         if plan is None:
             monkeypatch.delenv("TGIS_TALL_PLAN", raising=False)
