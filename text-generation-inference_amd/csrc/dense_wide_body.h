@@ -2,7 +2,7 @@
 //
 // dense_gemm_unit (dense_gemm_body.h) keeps two k64-steps of weights in flight per wave and passes x through LDS 256 k at a time, so that
 // a narrow projection is a chain of three to five dependent trips to memory: 5 - 11 us for 8 - 46 MB.  Here
-//   * the 8 waves of a block split the block's k range step by step (wave w: steps w, w + 8, ...; the block reads its tiles' weights as
+//   * the 8 waves of a block split the k range step by step (wave w: steps w, w + 8, ...; the block reads its tiles' weights as
 //     dense runs) and each has WIDE_DEPTH steps of TN tiles on their way to its registers from the first instruction on;
 //   * x goes to LDS by direct loads, 512 Q k at a time (a PHASE, one buffer; two buffers where there are several phases): at the widths
 //     of small models the whole k range is one phase, and a wave waits for memory once;
@@ -24,32 +24,29 @@ __device__ __forceinline__ void wide_x_to_lds(const char* base, uint32_t off, ui
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
 
-// Q (1, 2 or 4): k64-steps per wave and phase.  a.KR: k range of a block (a multiple of 64), a.S splits.  rows_lds: rows of x in LDS, even.
+// Q (1, 2 or 4): k64-steps per wave and phase.  A block takes the whole k range and all rows.  rows_lds: rows of x in LDS, even.
 template <typename T, int TN, int ACT, int MR, bool R16, int Q>
-__device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int ntg, const int split, const int mslab, const int rows_lds,
-                                                unsigned char* smem) {
+__device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int ntg, const int rows_lds, unsigned char* smem) {
     static_assert(!R16 || MR == 1, "16-row staging is for single 32-row passes");
     static_assert(WIDE_DEPTH % Q == 0, "phases and the ring stay in step");
     using V8 = typename VecT<T>::x8;
     constexpr int W = WIDE_WAVES, CHUNKS = 2 * Q;  // 256-k chunks per phase
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int m0 = mslab * (32 * MR);
-    const int mrows = min(R16 ? 16 : 32 * MR, a.M - m0);
-    const int ksteps = a.K >> 6;                                                // K % 64 == 0 (host)
-    const int ks0 = split * (a.KR >> 6), n = min(ksteps - ks0, a.KR >> 6);      // n >= 1 (host)
-    const int mine = (n - w + W - 1) / W;                                       // steps of this wave
+    const int mrows = min(R16 ? 16 : 32 * MR, a.M);
+    const int n = a.K >> 6;                // k64-steps; K % 64 == 0, n >= 1 (host)
+    const int mine = (n - w + W - 1) / W;  // steps of this wave
     const int phases = (n + W * Q - 1) / (W * Q);
     const int buf_bytes = CHUNKS * rows_lds * 512;
 
     // x: one load brings two rows of a chunk
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
-    const char* xbase = reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.x) + (int64_t)m0 * a.ldx);
+    const char* xbase = reinterpret_cast<const char*>(a.x);
     const int pairs = rows_lds >> 1;
     auto x_phase = [&](int p) {
         for (int l = w; l < CHUNKS * pairs; l += W) {
             const int chunk = l / pairs, pair = l - chunk * pairs, m = 2 * pair + (lane >> 5);
-            const int k = min((ks0 << 6) + (p * CHUNKS + chunk) * 256 + ((lane & 31) ^ (m & 7)) * 8, a.K - 8);  // (past the range: never read)
+            const int k = min((p * CHUNKS + chunk) * 256 + ((lane & 31) ^ (m & 7)) * 8, a.K - 8);  // (past the range: never read)
             const char* xb = xbase;
             PIN_SGPR(xb);
             wide_x_to_lds(xb, (uint32_t)(min(m, mrows - 1) * (int)a.ldx * 2 + k * 2),
@@ -64,7 +61,7 @@ __device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int nt
     const uint32_t woff = lane * 16;
     V8 wq[WIDE_DEPTH][TN][4];
     auto w_load = [&](int i_, V8 (&dst)[TN][4]) {
-        const int64_t off = (int64_t)min(ks0 + i_ * W + w, ksteps - 1) * 4096;
+        const int64_t off = (int64_t)min(i_ * W + w, n - 1) * 4096;
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
             const char* p = wtile[t] + off;
@@ -84,8 +81,8 @@ __device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int nt
             for (int j = 0; j < NR; ++j) {
                 const int r = w * NR + j;
                 const int m = min(mr * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5), mrows - 1);
-                rpos[mr][j] = a.positions[m0 + m];
-                rslot[mr][j] = a.slots[m0 + m];
+                rpos[mr][j] = a.positions[m];
+                rslot[mr][j] = a.slots[m];
             }
     }
 
@@ -179,14 +176,14 @@ __device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int nt
                 for (int k = 1; k < W; ++k) v += red[(((k * TN + t) * MR + mr) * NREG + w * NR + j) * 64];
                 fin[mr][j] = v;
             }
-        dense_finish<T, ACT, MR, NR>(a, fin, w * NR, ntg * TN + t, split, mslab, m0, mrows, lane, rslot, rcos[t], rsin[t]);
+        dense_finish<T, ACT, MR, NR>(a, fin, w * NR, ntg * TN + t, 0, 0, 0, mrows, lane, rslot, rcos[t], rsin[t]);
     }
 }
 
 // rows of a batch whose x is staged `rows_lds` (even) rows high, and the LDS of a block
 static inline int wide_rows_lds(int64_t M, int MR) { return (int)(std::min<int64_t>(M, 32 * MR) + 1) / 2 * 2; }
-static inline size_t wide_lds_bytes(int64_t M, int64_t KR, int TN, int MR, bool R16, int Q) {
-    const int64_t phases = cdiv64(KR, 512 * Q);
+static inline size_t wide_lds_bytes(int64_t M, int64_t K, int TN, int MR, bool R16, int Q) {
+    const int64_t phases = cdiv64(K, 512 * Q);
     const size_t x = (size_t)std::min<int64_t>(phases, 2) * (2 * Q) * wide_rows_lds(M, MR) * 512;
     return std::max(x, (size_t)WIDE_WAVES * TN * MR * (R16 ? 8 : 16) * 256);
 }

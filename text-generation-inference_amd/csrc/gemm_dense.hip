@@ -96,7 +96,7 @@ __global__ __launch_bounds__(64 * TN * WK) void dense_gemm_kernel(DenseArgs a) {
 template <typename T, int TN, int ACT, int MR, bool R16, int Q>
 __global__ __launch_bounds__(64 * dense::WIDE_WAVES) void dense_wide_kernel(DenseArgs a, int rows_lds) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    dense::dense_wide_unit<T, TN, ACT, MR, R16, Q>(a, blockIdx.x, blockIdx.y, blockIdx.z, rows_lds, smem);
+    dense::dense_wide_unit<T, TN, ACT, MR, R16, Q>(a, blockIdx.x, rows_lds, smem);
 }
 
 // Several inputs, each with weight rows of its own, stacked in one image: group g = tiles [g tiles, (g + 1) tiles), the last one what is left.
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(64 * dense::WIDE_WAVES) void dense_groups_kernel(De
     a.prep += (int64_t)first * a.KS * 4096;
     a.N = g + 1 < groups ? tiles * 32 : a.N - first * 32;
     a.NT = (a.N + 31) >> 5;
-    dense::dense_wide_unit<T, 1, 0, MR, R16, Q>(a, blockIdx.x - first, 0, 0, rows_lds, smem);
+    dense::dense_wide_unit<T, 1, 0, MR, R16, Q>(a, blockIdx.x - first, rows_lds, smem);
 }
 
 // Sum the S split-K slabs in fixed order and emit the output (+bias); thread = (row, 4 columns).
@@ -172,9 +172,8 @@ static int launch_wide(const DenseArgs& a, hipStream_t st) {
     static const hipError_t attr = hipFuncSetAttribute((const void*)dense_wide_kernel<T, TN, ACT, MR, R16, Q>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     TGIS_CHECK_HIP(attr);
-    dim3 grid((unsigned)cdiv64(a.NT, TN), (unsigned)a.S, (unsigned)cdiv64(a.M, 32 * MR));
-    hipLaunchKernelGGL((dense_wide_kernel<T, TN, ACT, MR, R16, Q>), grid, dim3(64 * dense::WIDE_WAVES),
-                       dense::wide_lds_bytes(a.M, a.KR, TN, MR, R16, Q), st, a, dense::wide_rows_lds(a.M, MR));
+    hipLaunchKernelGGL((dense_wide_kernel<T, TN, ACT, MR, R16, Q>), dim3((unsigned)cdiv64(a.NT, TN)), dim3(64 * dense::WIDE_WAVES),
+                       dense::wide_lds_bytes(a.M, a.K, TN, MR, R16, Q), st, a, dense::wide_rows_lds(a.M, MR));
     return TGIS_OK;
 }
 // (the row counts and tiles per wave that plan_finished and plan_dense_rope choose)
@@ -436,7 +435,7 @@ static int launch_groups(const DenseArgs& a, int groups, int tiles, int64_t x_gr
         hipFuncSetAttribute((const void*)dense_groups_kernel<T, MR, R16, Q>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     TGIS_CHECK_HIP(attr);
     hipLaunchKernelGGL((dense_groups_kernel<T, MR, R16, Q>), dim3((unsigned)a.NT), dim3(64 * dense::WIDE_WAVES),
-                       dense::wide_lds_bytes(a.M, a.KR, 1, MR, R16, Q), st, a, dense::wide_rows_lds(a.M, MR), tiles, groups, x_group, out_group);
+                       dense::wide_lds_bytes(a.M, a.K, 1, MR, R16, Q), st, a, dense::wide_rows_lds(a.M, MR), tiles, groups, x_group, out_group);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
