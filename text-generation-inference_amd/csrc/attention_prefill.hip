@@ -31,11 +31,6 @@
 
 namespace {
 
-// 1 KiB: lane l's 16 bytes at base + off go to LDS byte `lds` + 16 l
-__device__ __forceinline__ void page_to_lds(const char* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
-
 // maximum over the four 16-lane rows of a wave, in every lane
 __device__ __forceinline__ float max_over_rows(float v) {
     const auto h = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
@@ -162,8 +157,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + buf * (PAGE_ELEMS * 4) + (i * 4 + w) * 1024);
-            page_to_lds(kp, koff[i], dst);
-            page_to_lds(vp, voff[i], dst + PAGE_ELEMS * 2);
+            kib_to_lds(kp, koff[i], dst);
+            kib_to_lds(vp, voff[i], dst + PAGE_ELEMS * 2);
         }
     };
     page_load(page_number(0), 0);

@@ -80,6 +80,11 @@ template <typename V> __device__ __forceinline__ void st16(void* p, V v) {
     *reinterpret_cast<V*>(p) = v;
 }
 
+// 1 KiB by a direct load: lane l's 16 bytes at base + off go to LDS byte `lds` + 16 l.  The wave waits for it by its vector memory count.
+__device__ __forceinline__ void kib_to_lds(const char* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+
 // Sum / maximum over the 64 lanes of a wave, in every lane: v (+) v of lane ^ 32, ^ 16, ^ 8, ^ 4, ^ 2, ^ 1, by register moves (six trips
 // through LDS with __shfl_xor, the same bits).  Lane ^ 4 is a rotation of the row by 4: lanes l and l ^ 8 are alike by then.
 template <int CTRL> __device__ __forceinline__ float row_moved(float v) {

@@ -19,11 +19,6 @@ namespace dense {
 constexpr int WIDE_WAVES = 8;
 constexpr int WIDE_DEPTH = 4;  // k64-steps in flight per wave
 
-// 1 KiB: lane l's 16 bytes at base + off go to LDS byte `lds` + 16 l
-__device__ __forceinline__ void wide_x_to_lds(const char* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
-
 // Q (1, 2 or 4): k64-steps per wave and phase.  A block takes the whole k range and all rows.  rows_lds: rows of x in LDS, even.
 template <typename T, int TN, int ACT, int MR, bool R16, int Q>
 __device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int ntg, const int rows_lds, unsigned char* smem) {
@@ -49,7 +44,7 @@ __device__ __forceinline__ void dense_wide_unit(const DenseArgs& a, const int nt
             const int k = min((p * CHUNKS + chunk) * 256 + ((lane & 31) ^ (m & 7)) * 8, a.K - 8);  // (past the range: never read)
             const char* xb = xbase;
             PIN_SGPR(xb);
-            wide_x_to_lds(xb, (uint32_t)(min(m, mrows - 1) * (int)a.ldx * 2 + k * 2),
+            kib_to_lds(xb, (uint32_t)(min(m, mrows - 1) * (int)a.ldx * 2 + k * 2),
                           __builtin_amdgcn_readfirstlane(lds0 + (p & 1) * buf_bytes + (chunk * rows_lds + 2 * pair) * 512));
         }
     };

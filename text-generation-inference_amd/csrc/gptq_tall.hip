@@ -46,11 +46,6 @@ struct TallArgs {
 
 constexpr int TALL_RING = 4;  // k64-steps of weights in flight per wave, and buffers of x
 
-// 1 KiB of x: lane l's 16 bytes at base + off go to LDS byte `lds` + 16 l
-__device__ __forceinline__ void tall_x_to_lds(const char* base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
-}
-
 template <int BMR, int ACT, int TW>
 __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     constexpr int BM = 32 * BMR;
@@ -97,7 +92,7 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
         PIN_SGPR(xb);
 #pragma unroll
         for (int j = 0; j < BMR; ++j)
-            tall_x_to_lds(xb, rowoff[j], __builtin_amdgcn_readfirstlane(lds0 + buf * (BM * 128) + (4 * j + w) * 1024));
+            kib_to_lds(xb, rowoff[j], __builtin_amdgcn_readfirstlane(lds0 + buf * (BM * 128) + (4 * j + w) * 1024));
     };
 
     uint32_t EXr = 0x64006400u, M0r = 0x000F000Fu, M1r = 0x00F000F0u;
