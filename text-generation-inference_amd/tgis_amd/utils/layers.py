@@ -25,8 +25,8 @@ import os
 SKINNY_MAX_M = int(os.getenv("TGIS_SKINNY_MAX_M", "256"))
 # fuse the split-K reduce of decode-sized GPTQ GEMMs into the consumer kernel (rmsnorm / rope+KV write)
 DEFER_REDUCE = os.getenv("TGIS_DEFER_REDUCE", "true").lower() not in ("0", "false")
-# decode batches of up to 32 rows: rotary embedding + cache write in the epilogue of the int4 qkv GEMM (one launch
-# instead of GEMM + tgis_rope_kv_write, no split-K slabs).  Costs a second image of the qkv weights.
+# steps of up to 64 rows, prompts where that pays (native.rope_gemm_pays_for_prompts): rotary embedding + cache write in the epilogue of the qkv
+# GEMM (one launch instead of GEMM + tgis_rope_kv_write, no split-K slabs).  Costs a second image of the qkv weights.
 FUSED_ROPE_GEMM = os.getenv("TGIS_FUSED_ROPE_GEMM", "true").lower() not in ("0", "false")
 # GELU applied by the dense decode GEMM that produces its operand (TGIS_FUSED_GELU_GEMM=false: a launch of its own)
 FUSED_GELU_GEMM = os.getenv("TGIS_FUSED_GELU_GEMM", "true").lower() not in ("0", "false")
