@@ -373,6 +373,27 @@ def test_sandwich_norm_takes_split_k_slabs(gpu_device):
         assert torch.allclose(y.double().cpu(), ref.norm_one_plus(x_ref, wn.double().cpu(), 1e-5), atol=2e-3, rtol=1e-3)
 
 
+@pytest.mark.parametrize("E", [64, 2048, 2052, 4096, 4100, 8192])
+@pytest.mark.parametrize("S", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 15])
+def test_sandwich_norm_of_slabs(gpu_device, S, E):
+    """Any number of slabs at the edges of the row forms, padded slab rows, values of other sequences' rows next to them."""
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(S)
+    M, ld = 35, (E + 31) // 32 * 32
+    slabs = torch.randn(2, S, 32, ld, generator=g)
+    part = native.Partial(slabs.cuda(), S, ld, M, E, None)
+    part.dtype = torch.bfloat16
+    x, wb, wn = torch.randn(M, E, generator=g), torch.randn(E, generator=g) * 0.2, torch.randn(E, generator=g) * 0.2
+    xd = x.cuda()
+    y = native.sandwich_norm_f32(xd, part, wb.cuda(), wn.cuda(), 1e-5, torch.float32)
+    delta = slabs.double().sum(1)[:, :, :E].reshape(64, E)[:M]
+    want_x = x.double() + ref.norm_one_plus(delta, wb.double(), 1e-5)
+    # sums of up to 15 and of E values in fp32, then a handful of roundings: 2^-24 of them each
+    assert torch.allclose(xd.cpu().double(), want_x, atol=1e-5, rtol=1e-5)
+    assert torch.allclose(y.cpu().double(), ref.norm_one_plus(want_x, wn.double(), 1e-5), atol=1e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind", ["clamped", "silu"])
 @pytest.mark.parametrize("T", [37, 300])

@@ -155,7 +155,7 @@ __global__ void glu_vec_kernel(const T* __restrict__ in, int64_t ld_in, T* __res
 // number of memory instructions in it is what counts.
 // delta may also arrive as the S fp32 split-K slabs of the GEMM that produced it ([row / 32][S][32][slab_ld], TD = float,
 // `delta` then points at the slabs): their sum is taken here instead of by a reduce launch of its own.
-template <typename TD, typename TY, int NV>
+template <typename TD, typename TY, int NV, bool SLABS>
 __global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, const TD* __restrict__ delta, int64_t ld_delta,
                                                                 const float* __restrict__ post_w, float post_add, float post_scale, float* x_out,
                                                                 const float* __restrict__ pre_w, float pre_add,
@@ -169,29 +169,57 @@ __global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, 
         const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
         const bool in = c < E;
         xv[i] = in ? Vec4<float>::ld(x + row * E + c) : f32x4{};
-        if (S == 0) dv[i] = (in && delta) ? Vec4<TD>::ld(delta + row * ld_delta + c) : f32x4{};
+        if (!SLABS) dv[i] = (in && delta) ? Vec4<TD>::ld(delta + row * ld_delta + c) : f32x4{};
         pw[i] = (in && delta) ? (post_w ? Vec4<float>::ld(post_w + c) + post_add : f32x4{1.f, 1.f, 1.f, 1.f}) : f32x4{};
         qw[i] = in ? (pre_w ? Vec4<float>::ld(pre_w + c) + pre_add : f32x4{1.f, 1.f, 1.f, 1.f}) : f32x4{};
     }
-    if (S > 0) {  // slabs: ld_delta is the slab row stride; SLABS of them in flight, added in their order
-        constexpr int SLABS = 8;
+    if constexpr (SLABS) {  // ld_delta is the slab row stride
         const float* sp = reinterpret_cast<const float*>(delta) + ((row >> 5) * S * 32 + (row & 31)) * ld_delta;
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
-            f32x4 acc = {};
-            if (c < E)
-                for (int s0 = 0; s0 < S; s0 += SLABS) {
-                    f32x4 part[SLABS];
+        for (int i = 0; i < NV; ++i) dv[i] = f32x4{};
+        // slabs s0 .. s0 + n - 1 of all the thread's columns on their way at once, added in their order
+        auto add_slabs = [&](int s0, auto n_) {
+            constexpr int n = decltype(n_)::value;
+            f32x4 part[NV][n];
 #pragma unroll
-                    for (int e = 0; e < SLABS; ++e)
-                        part[e] = s0 + e < S ? Vec4<float>::ld(sp + (int64_t)(s0 + e) * 32 * ld_delta + c) : f32x4{};
+            for (int i = 0; i < NV; ++i) {
+                const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
 #pragma unroll
-                    for (int e = 0; e < SLABS; ++e)
-                        if (s0 + e < S) acc += part[e];
+                for (int e = 0; e < n; ++e) part[i][e] = Vec4<float>::ld(sp + (int64_t)(s0 + e) * 32 * ld_delta + (c < E ? c : 0));
+            }
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
+                f32x4 acc = dv[i];
+#pragma unroll
+                for (int e = 0; e < n; ++e) acc += part[i][e];
+                dv[i] = c < E ? acc : f32x4{};
+            }
+        };
+        // Each number of slabs has loads of its own, and rows without slabs an instance without their registers.  With eight loads under a
+        // condition each, one column group behind the other, wide rows paid for every group (us, 24 rows, slab by slab / that / now: 8192
+        // columns in 1, 2, 4, 12 slabs 5.8 / 7.9 / 5.3, 6.3 / 7.9 / 5.6, 7.2 / 8.0 / 6.1, 10.7 / 10.0 / 7.8; 4096 in 1, 4 4.7 / 5.4 / 4.0,
+        // 5.4 / 5.4 / 4.3; 2048 in 8 4.5 / 3.9 / 3.8).
+        constexpr int AT_ONCE = NV == 4 ? 4 : 8;
+        int s0 = 0;
+        for (; s0 + AT_ONCE <= S; s0 += AT_ONCE) add_slabs(s0, std::integral_constant<int, AT_ONCE>{});
+        if constexpr (AT_ONCE == 8) {
+            if (S - s0 >= 4) {
+                switch (S - s0) {
+                    case 4: add_slabs(s0, std::integral_constant<int, 4>{}); break;
+                    case 5: add_slabs(s0, std::integral_constant<int, 5>{}); break;
+                    case 6: add_slabs(s0, std::integral_constant<int, 6>{}); break;
+                    default: add_slabs(s0, std::integral_constant<int, 7>{});
                 }
-            dv[i] = acc;
+                s0 = S;
+            }
         }
+        if (S - s0 == 3)
+            add_slabs(s0, std::integral_constant<int, 3>{});
+        else if (S - s0 == 2)
+            add_slabs(s0, std::integral_constant<int, 2>{});
+        else if (S - s0 == 1)
+            add_slabs(s0, std::integral_constant<int, 1>{});
     }
     if (delta) {
         float rinv_d = post_scale;
@@ -257,9 +285,19 @@ int launch_sandwich(const float* x, const void* delta, int64_t ld_delta, const f
 #define TGIS_SANDWICH_REG(NPT)                                                                                                  \
     hipLaunchKernelGGL((sandwich_norm_reg_kernel<TD, TY, NPT>), dim3((unsigned)rows), dim3(256), 0, st, x, (const TD*)delta, ld_delta, \
                        post_w, post_add, post_scale, x_out, pre_w, pre_add, (TY*)y, E, eps)
-#define TGIS_SANDWICH_VEC(NV)                                                                                                  \
-    hipLaunchKernelGGL((sandwich_norm_vec_kernel<TD, TY, NV>), dim3((unsigned)rows), dim3(512), 0, st, x, (const TD*)delta, ld_delta, \
+#define TGIS_SANDWICH_FORM(NV, SLABS)                                                                                          \
+    hipLaunchKernelGGL((sandwich_norm_vec_kernel<TD, TY, NV, SLABS>), dim3((unsigned)rows), dim3(512), 0, st, x, (const TD*)delta, ld_delta, \
                        post_w, post_add, post_scale, x_out, pre_w, pre_add, (TY*)y, E, eps, num_slabs)
+#define TGIS_SANDWICH_VEC(NV)                                                                                                  \
+    do {                                                                                                                       \
+        if constexpr (std::is_same<TD, float>::value) {  /* (slabs are fp32) */                                                \
+            if (num_slabs > 0) {                                                                                               \
+                TGIS_SANDWICH_FORM(NV, true);                                                                                  \
+                break;                                                                                                         \
+            }                                                                                                                  \
+        }                                                                                                                      \
+        TGIS_SANDWICH_FORM(NV, false);                                                                                         \
+    } while (0)
     const bool vec_ok = E % 4 == 0 && (!delta || ld_delta % 4 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)x_out % 16 == 0) &&
                         ((uintptr_t)delta % 16 == 0) && ((uintptr_t)y % 16 == 0) && ((uintptr_t)post_w % 16 == 0) &&
                         ((uintptr_t)pre_w % 16 == 0);
@@ -283,6 +321,7 @@ int launch_sandwich(const float* x, const void* delta, int64_t ld_delta, const f
                            post_w, post_add, post_scale, x_out, pre_w, pre_add, (TY*)y, E, eps);
 #undef TGIS_SANDWICH_REG
 #undef TGIS_SANDWICH_VEC
+#undef TGIS_SANDWICH_FORM
     return 0;
 }
 
