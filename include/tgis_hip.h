@@ -95,9 +95,12 @@ int tgis_gptq_prepare(const int32_t* qweight, const int32_t* qzeros, const void*
  * dequantises once with tgis_gptq_dequant_f16 and uses a library GEMM, exllamav2.py:87 "M > 50"): M <= 64 streams the
  * weights once per pass, 64 < M <= 256 in 64-row passes, and — for K % 64 == 0, group size 64 * 2^n, no act-order, act != 1 —
  * a tall kernel (one dequantisation per 64 - 128 rows, 0.9-1.2 PFLOP/s from a few hundred rows, no scratch copy of W) takes over up to
- * 8192 rows: from 257, and from 129 (act 2: 65) where it is done before the passes.  tgis_gptq_gemm_whole_sums: 1 where it does. */
+ * 8192 rows: from 257, and from 129 (act 2: 65) where it is done before the passes.  tgis_gptq_gemm_whole_sums: 1 where it does.
+ * tgis_gptq_gemm_fused_pays: 0 at row counts up to that largest one where dequantising and a library GEMM is the faster way all the same
+ * (some between 3072 and 8192, where 256 x 256 tiles fill their rounds). */
 int64_t tgis_gptq_gemm_fused_rows(int64_t K, int64_t groups, int act_order, int act);
 int tgis_gptq_gemm_whole_sums(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act);
+int tgis_gptq_gemm_fused_pays(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act);
 int64_t tgis_gptq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
 
 /* Activation layout between the decode step's own kernels (round 4).  A leading dimension of TGIS_LD_FRAGMENTS says that a

@@ -41,3 +41,18 @@ def test_int4_tall(M, K, N, act, whole):
     assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 128, 0, act) == whole
     assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 128, 1, act) == 0  # act-order
     assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 32, 0, act) == 0   # groups shorter than a k64-step
+
+
+# past 3072 rows: row counts at which 256 x 256 tiles fill their rounds of 256, or most of a single one over a long k, and others
+@pytest.mark.parametrize("M,K,N,act,pays", [
+    (257, 4096, 12288, 0, 1), (3072, 11008, 4096, 0, 1), (4096, 11008, 4096, 0, 0), (4097, 11008, 4096, 0, 1), (8192, 4096, 12288, 0, 0), (6000, 4096, 12288, 0, 1),
+    (3841, 4096, 4096, 0, 0), (3840, 4096, 4096, 0, 0), (3584, 4096, 4096, 0, 1), (7168, 11008, 4096, 0, 1), (8192, 13824, 5120, 0, 1), (5120, 5632, 2048, 0, 0),
+    (4864, 5632, 2048, 0, 1), (4865, 5632, 2048, 0, 0), (5120, 5056, 2048, 0, 1), (8192, 4096, 22016, 2, 1), (8193, 4096, 22016, 2, 0), (8193, 4096, 4000, 0, 0),
+])
+def test_int4_library(M, K, N, act, pays):
+    from tgis_amd import native
+
+    lib = native.load_library()
+    assert lib.tgis_gptq_gemm_fused_pays(M, K, N, K // 64, 0, act) == pays
+    assert lib.tgis_gptq_gemm_fused_pays(M, K, N, K // 64, 1, act) == 0          # act-order: up to 256 rows alone
+    assert lib.tgis_gptq_gemm_fused_pays(256, K, N, K // 64, 1, act) == 1

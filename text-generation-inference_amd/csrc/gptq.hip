@@ -289,6 +289,12 @@ extern "C" int64_t tgis_gptq_gemm_fused_rows(int64_t K, int64_t groups, int act_
     return gptq::tall_serves(K, groups, act_order != 0, act) ? std::max<int64_t>(256, gptq::tall_max_m()) : 256;
 }
 
+// Is tgis_gptq_gemm_f16 the faster way at M rows, or dequantising once and a library GEMM?  (of the rows that the former reaches)
+extern "C" int tgis_gptq_gemm_fused_pays(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act) {
+    if (M < 1 || K <= 0 || N <= 0 || M > tgis_gptq_gemm_fused_rows(K, groups, act_order, act)) return 0;
+    return M <= 256 || gptq::tall_before_library(M, K, N, act) ? 1 : 0;
+}
+
 // Does tgis_gptq_gemm_f16 finish its sums by itself at M rows?  (the tall kernel; else 64-row passes and, where they split, their reduce)
 extern "C" int tgis_gptq_gemm_whole_sums(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act) {
     if (M < 1 || K <= 0 || N <= 0 || groups <= 0 || K % groups) return 0;

@@ -9,6 +9,8 @@ namespace gptq {
 bool tall_serves(int64_t K, int64_t groups, bool act_order, int act);
 // ... and does it, at M rows?  (from tall_min_m(); up to 256 rows where the streaming passes would take longer)
 bool tall_ok(int64_t M, int64_t K, int64_t N, int64_t groups, bool act_order, int act);
+// ... and is it, where it serves, the faster way than dequantising and a library GEMM?
+bool tall_before_library(int64_t M, int64_t K, int64_t N, int act);
 int64_t tall_min_m(int act);
 int64_t tall_max_m();
 // fp32 scratch of launch_tall

@@ -413,8 +413,6 @@ TallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, 
 // Rows from which it may replace the 64-row streaming passes, and up to which it replaces dequantise + library GEMM:
 // (library with its dequantisation / tall, us, the four GEMMs of a 7B layer) 3072 rows 1296 / 1159, 6000 rows 2418 / 2184, 8192 rows
 // 2979 / 2993, 16128 rows 5542 / 5947: past 8192 rows hipBLASLt's 256 x 256 tiles, free of dequantisation, win (1.28 against 1.13 PFLOP/s).
-// (Over 30 shapes the library takes 1.07 - 1.21 times as long at each of 4096, 5000, 6144, 7168 and 8192 rows; 5120 x 15360 is the
-// shape it serves best: 752 / 778 at 5000 rows, 1166 / 1228 at 8192.)
 int64_t gptq::tall_min_m(int act) {
     static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 0;
     return v ? v : act == 2 ? 65 : 129;
@@ -427,6 +425,23 @@ bool gptq::tall_serves(int64_t K, int64_t groups, bool act_order, int act) {
     if (act_order || act == 1 || K % 64 != 0 || groups <= 0) return false;
     const int64_t gs = K / groups, spg = gs / 64;
     return groups == 1 || (gs % 64 == 0 && (spg & (spg - 1)) == 0);
+}
+// Between 3072 and tall_max_m() rows it depends on how full the library's 256 x 256 tiles leave their rounds of 256.  act 0, us, dequantise
+// and library / this kernel, weights cold:
+//   93 % full and more:  4096 x 12288 at 4096, 8000, 8192 rows 357 / 364, 674 / 720, 676 / 731; 11008 x 4096 at 4096, 8192 312 / 324, 588 / 641;
+//                        5120 x 15360 at 5000, 6000, 8192 672 / 757, 809 / 876, 1065 / 1188; 8192 x 3072 at 5000 222 / 239
+//   less:                4096 x 12288 at 6000, 7168 610 / 537, 647 / 641; 11008 x 4096 at 7168 728 / 581; 8192 x 10240 at 4096, 5000 737 / 608, 801 /
+//                        755; 13824 x 5120 at 4096, 5000, 6000 588 / 542, 836 / 664, 939 / 774
+//   one round, from three fifths on, of long k:  5632 x 2048 at 5000, 6000, 7168 114 / 134, 130 / 136, 151 / 163; 8192 x 3072 at 4096 193 / 215
+//                        (4096 x 4096 at 3500 120 / 118; 5632 x 2048 at 4096, half a round, 99 / 98)
+// Over 17 shapes and 14 row counts this choice is 0.7 % behind the better of the two, either one alone 2.7 % (this kernel) or 5.9 %.
+// With SiLU * up this kernel is within 5 % of the library and its activation launch, or in front (4096 x 22016 at 4096, 8192 rows 794 / 726, 1416 /
+// 1467; 2048 x 11264 209 / 192, 447 / 359).
+bool gptq::tall_before_library(int64_t M, int64_t K, int64_t N, int act) {
+    if (M <= 3072 || act == 2 || getenv("TGIS_TALL_MAX_M")) return M <= tall_max_m();
+    const int64_t tiles = cdiv64(M, 256) * cdiv64(N, 256), slots = cdiv64(tiles, CUS) * CUS;
+    const bool full = 100 * tiles >= 93 * slots, long_round = tiles <= CUS && 10 * tiles > 6 * CUS && K >= 5120;
+    return M <= tall_max_m() && !full && !long_round;
 }
 // Up to 256 rows the passes take k in parallel (k-parts, splits) where a tile here walks it alone, so it depends on the matrix which of
 // the two is done first.  us, the passes with the launch that adds their slabs / this kernel with a norm behind it (act 2: either alone):

@@ -42,6 +42,7 @@ SIGNATURES = {
     "tgis_gptq_prepared_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "tgis_gptq_prepare": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp, _vp]),
     "tgis_gptq_gemm_fused_rows": (_c_i64, [_c_i64, _c_i64, _c_int, _c_int]),
+    "tgis_gptq_gemm_fused_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "tgis_gptq_gemm_whole_sums": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "tgis_gptq_gemm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "tgis_gptq_gemm_f16": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
@@ -427,6 +428,10 @@ class GptqWeight:
     def fused_rows(self, act: int = 0) -> int:
         """Largest M the fused kernels of tgis_gptq_gemm_f16 should be given (beyond: dequantise + library GEMM)."""
         return load_library().tgis_gptq_gemm_fused_rows(self.K, self.groups, int(self.perm is not None), act)
+
+    def fused_pays(self, M: int, act: int = 0) -> bool:
+        """Whether they are the faster way at M rows, too, of those that they reach."""
+        return bool(load_library().tgis_gptq_gemm_fused_pays(M, self.K, self.N, self.groups, int(self.perm is not None), act))
 
     def whole_sums(self, M: int, act: int = 0) -> bool:
         """Whether gptq_gemm finishes its sums by itself at M rows, so that there is nothing for a consumer to add up."""

@@ -21,7 +21,7 @@ import os
 
 # rows up to which the dense weight-streaming MFMA kernel is used (one pass over the weights per 32 / 64 rows); above,
 # hipBLASLt.  GPTQ linears ask the library how far its fused kernels reach (GptqWeight.fused_rows: 64-row streaming passes
-# to 256 rows, the tall kernel from 65 / 129 rows where it is faster to 8192; beyond that dequantise once + hipBLASLt, exllamav2.py:87).
+# to 256 rows, the tall kernel from 65 / 129 rows to 8192 where it is faster; else dequantise once + hipBLASLt, exllamav2.py:87).
 SKINNY_MAX_M = int(os.getenv("TGIS_SKINNY_MAX_M", "256"))
 # fuse the split-K reduce of decode-sized GPTQ GEMMs into the consumer kernel (rmsnorm / rope+KV write)
 DEFER_REDUCE = os.getenv("TGIS_DEFER_REDUCE", "true").lower() not in ("0", "false")
@@ -259,13 +259,13 @@ class Ex4bitLinearV2:
             return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias)
         if self.gate_up:
             # output is the activated [M, I] tensor
-            if x.shape[0] <= self._fused_rows(2):
+            if x.shape[0] <= self._fused_rows(2) and (x.shape[0] <= 256 or self.ordered.fused_pays(x.shape[0], 2)):
                 return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=2)
             return native.act_mul(self._large_m(x), self.width // 2)
         # where the tall kernel finishes its own sums sooner than a consumer adds the slabs of 64-row passes, nothing is deferred
         if partial and x.shape[0] <= native.PARTIAL_MAX_M and DEFER_REDUCE and not self._whole_sums(x.shape[0], act):
             return native.gptq_gemm_partial(x, self.ordered, bias=self.bias, act=act)
-        if x.shape[0] <= self._fused_rows(act):
+        if x.shape[0] <= self._fused_rows(act) and (x.shape[0] <= 256 or self.ordered.fused_pays(x.shape[0], act)):
             return native.gptq_gemm(x, self.ordered, workspace(x.device), bias=self.bias, act=act)
         if act:
             x = native.act_mul(x, self.height)
