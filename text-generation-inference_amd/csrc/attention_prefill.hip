@@ -316,10 +316,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
 int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st) {
     TGIS_CHECK_ARG(cdiv64(max_q_len, a.TQ * 4) <= 2147483647LL && (int64_t)Hkv * a.HC <= 65535 && B <= 65535, "tgis_attn_paged: grid too large");
     const int64_t groups = (int64_t)Hkv * a.HC * B;
-    // Tiles of 128 columns, or of 64 where those would be fewer than the 512 that are resident at once (us, 128 / 64): 1 x 100 tokens, 32
-    // heads of 128: 8.5 / 6.3; 1 x 1000 30.8 / 27.7; 1 x 512, 64 heads on 8: 19.1 / 15.7; 1 x 1500, 32 on 4, D 64: 40 / 30; 3 x 433, 32
-    // heads: 24.7 / 23.5; from 512 on: 4 x 433 24.4 / 26.2, 8 x 200 17.2 / 19.4, 16 x 1008 300 / 337.
-    int cg = groups * cdiv64(max_q_len, a.TQ * 8) < 512 ? 1 : 2;
+    // Tiles of 128 columns, or of 64 where those would leave part of the chip idle: of the 512 blocks that are resident at once a quarter may
+    // be missing at D 128 (us, 128 / 64).  D 128: 1 x 100 tokens, 32 heads 8.5 / 6.3; 1 x 1000 30.8 / 27.7; 1 x 512, 64 heads on 8 19.1 / 15.7;
+    // 375 tiles, 1 x 1000, 48 on 1 43.7 / 31.5; from 384 on 12 x 65, 32 heads 9.6 / 10.8; 48 x 20, 32 on 8 8.0 / 9.6; 12 x 100, 48 on 1 12.9 /
+    // 14.8; 32 x 33 10.7 / 11.1; 8 x 100, 64 on 8 12.8 / 13.8 (4 x 300, 32 heads 18.5 / 16.9; 24 x 20, 64 on 8 9.6 / 8.9); 16 x 1008 300 / 337.
+    // D 64: 1 x 1500, 32 on 4 40 / 30; 24 x 33 6.6 / 5.0; 384 tiles, 32 x 33 6.7 / 5.6; 512, 64 x 33, 16 on 8 6.1 / 6.5.
+    int cg = groups * cdiv64(max_q_len, a.TQ * 8) < (D == 128 ? 384 : 512) ? 1 : 2;
     if (const char* e = getenv("TGIS_PREFILL_CG")) cg = atoi(e) == 1 ? 1 : 2;  // tuning and test hook
     const int64_t q_tiles = cdiv64(max_q_len, a.TQ * 4 * cg);
     AttnArgs dealt = a;
