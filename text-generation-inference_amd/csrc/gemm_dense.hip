@@ -71,6 +71,10 @@ using dense::dense_slab_bytes;
 //     20.1; 1152 x 8192 13.1 / 11.1, 14.3 / 12.5; 1152 x 16384 15.6 / 14.3, 17.1 / 15.5.  Outside: 2048 x 8128 13.6 / 12.9, 14.6 / 14.8; 2048 x
 //     5632 13.4 / 14.0, 14.0 / 14.3; 2048 x 16448 20.8 / 26.5, 22.7 / 29.9; 1024 x 16384 12.3 / 12.9, 13.3 / 13.7; 256 x 24576 8.0 / 13.1
 //     (6144 x 24576 at 64 rows: 61 / 74)
+//   * act 2 at up to 16 rows streams at every size (streaming / blocks of one tile / of two): the one-user and small-model shape is alike in all
+//     three, 2048 x 11264 at 1 / 16 rows 10.5 / 10.6 / 10.5, 10.5 / 11.3 / 10.5, and larger ones lose, 4096 x 22016 at 16 rows 31.3 / 34.4 / 36.7,
+//     5120 x 27648 46.9 / 55.0 / 48.2.  (Narrower ones would gain from one-tile blocks, 2048 x 5632 at 1 / 16 rows 9.2 / 5.9, 8.8 / 6.7, which
+//     are not built for act 2.)
 // A projection whose streaming plan splits k stays with it, so that it sums in the same order whether it leaves finished or as slabs
 // (2048 x 2048 at 16 rows: finished 7.5 / 5.9, as slabs 4.2 / 5.5).
 static DensePlan plan_finished(int64_t K, int64_t N, int64_t M, int act) {
