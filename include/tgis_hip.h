@@ -94,7 +94,7 @@ int tgis_gptq_prepare(const int32_t* qweight, const int32_t* qzeros, const void*
 /* Largest M for which tgis_gptq_gemm_f16 is a fused dequantise + MFMA kernel worth calling (above it the caller
  * dequantises once with tgis_gptq_dequant_f16 and uses a library GEMM, exllamav2.py:87 "M > 50"): M <= 64 streams the
  * weights once per pass, 64 < M <= 256 in 64-row passes, and — for K % 64 == 0, group size 64 * 2^n, no act-order, act != 1 —
- * a tall kernel (one dequantisation per 64 - 128 rows, 0.9-1.2 PFLOP/s from a few hundred rows, no scratch copy of W) takes over up to
+ * a tall kernel (one dequantisation per 64 - 128 rows, 0.5 - 1.0 PFLOP/s at 500 - 1000 rows of a 7B matrix, 1.0 - 1.1 from 2000, no scratch copy of W) takes over up to
  * 8192 rows: from 257, and from 129 (act 2: 65) where it is done before the passes.  tgis_gptq_gemm_whole_sums: 1 where it does.
  * tgis_gptq_gemm_fused_pays: 0 at row counts up to that largest one where dequantising and a library GEMM is the faster way all the same
  * (some between 3072 and 8192, where 256 x 256 tiles fill their rounds). */
