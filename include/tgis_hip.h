@@ -409,6 +409,14 @@ int tgis_wkv_scan_runs(const void* r, const void* k, const void* v, const void* 
                        const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
                        const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
                        int64_t ld_out, int64_t B, int H, int d, float eps, int64_t max_q_len, int dtype, void* stream);
+/* ... given tgis_wkv_scan_workspace(B, H, d, max_q_len) bytes, 16-byte aligned, walks long runs of few (sequence, head) pairs in segments side
+ * by side (0 bytes: such a step is not cut; a null workspace: it is not either). */
+int64_t tgis_wkv_scan_workspace(int64_t B, int H, int d, int64_t max_q_len);
+int tgis_wkv_scan_segments(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
+                           const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
+                           const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
+                           int64_t ld_out, int64_t B, int H, int d, float eps, int64_t max_q_len, void* workspace,
+                           int64_t workspace_bytes, int dtype, void* stream);
 
 /* tgis_wkv_decay of low [T, >= rank] (row stride ld_low) and tgis_wkv_scan in one launch, for steps in which sequences bring single
  * tokens (any number works, one after another).  d a multiple of 4 up to 128, rank <= 1024; rows of r, k, v, gate and out are groups of

@@ -233,3 +233,47 @@ def test_scan_of_short_runs(gpu_device, H, B, d, by_token, longest):
     # fp32 sums in another order, one rounding to bf16
     assert ((got - walked).abs() <= 2.0 ** -7 * (walked.abs() + walked.square().mean().sqrt())).all()
     assert (got_st - walked_st).abs().max() <= 1e-5 * walked_st.abs().max()
+
+
+# longest: fewer tokens than are cut, just enough, a last segment of one token and of whole sub-blocks, more segments than one launch takes
+@pytest.mark.parametrize("d,longest", [(64, 127), (64, 128), (64, 449), (64, 2500), (32, 129), (48, 640), (128, 513), (100, 511)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scan_in_segments(gpu_device, d, longest, dtype):
+    """Long runs beside short ones, cut into segments, against the same step token by token (rows that are no groups of four, no hint)."""
+    from tgis_amd import native
+
+    H, W, eps = 2, 8, 1e-4
+    lens = [longest, 1, min(129, longest), longest // 2, 64]
+    fresh = [False, False, True, True, False]
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(d + longest)
+    r, k, v, gate = ((torch.randn(T, H * d, generator=g) * s).to(dtype) for s in (0.5, 0.5, 1.0, 1.0))
+    # (r, k and u of one sign: r u k of a fresh run's first token is then no sum that cancels, which the unit norm would magnify)
+    rkvg = [t.to(gpu_device) for t in (r.abs(), k.abs(), v, gate)]
+    logw = -torch.exp(torch.randn(T, H * d, generator=g) * 1.5 - 4.0)  # decays that carry a state over hundreds of tokens, some that end it
+    logw[torch.rand(T, H * d, generator=g) < 0.005] = -60.0
+    u, gain = torch.rand(H * d, generator=g) * 0.5, torch.rand(H * d, generator=g) + 0.5
+    state = torch.randn(B + 1, H, d, d, generator=g).to(gpu_device)
+    state[4, :, :, 0] = float("nan")  # slot of the third sequence, which starts anew
+    slots = torch.tensor([2, 0, 4, 1, 5], dtype=torch.int32)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), torch.tensor(lens).cumsum(0)])
+    pos = torch.cat([torch.arange(n) + (0 if f else 7) for n, f in zip(lens, fresh)]).to(torch.int32)
+    h = torch.randn(T, W, generator=g).to(gpu_device)
+    dev = lambda t: t.to(gpu_device)
+
+    def scan(pad, hint):
+        rows = [torch.nn.functional.pad(t, (0, pad))[:, :H * d] for t in rkvg]
+        st, sh = state.clone(), torch.zeros(B + 1, W, device=gpu_device)
+        out = native.wkv_scan(*rows, dev(logw), dev(u), dev(gain), st, sh, h, dev(slots), dev(cu.to(torch.int32)), dev(pos), H, d, eps, max_q_len=hint)
+        return out.double().view(T, H, d), st[slots.long()], sh, st[3]
+
+    assert (native.load_library().tgis_wkv_scan_workspace(B, H, d, longest) > 0) == (longest >= (128 if d <= 64 else 512))
+    want, want_st, want_sh, _ = scan(2, 0)
+    got, got_st, got_sh, spare = scan(0, longest)
+    # fp32 sums of either sign in another order and products of decays in another order (each a few roundings of 6e-8 per factor that
+    # matters: a key is worth less than 1e-3 after some hundreds); two-byte outputs are rounded once on both sides
+    size = want.square().mean(-1, keepdim=True).sqrt()
+    tol = 4e-5 * size + (0.0 if dtype == torch.float32 else 2.0 ** -7 * want.abs())
+    assert ((got - want).abs() <= tol).all(), float(((got - want).abs() / size).max())
+    assert (got_st - want_st).abs().max() <= 2e-5 * want_st.abs().max()
+    assert torch.equal(got_sh, want_sh) and torch.equal(spare, state[3])

@@ -6,6 +6,7 @@
 // State per slot: S[head][key channel][value channel] (fp32) and the last token's mixer input (fp32).  A sequence whose
 // step starts at position 0 starts from zeros whatever its slot held before: slots need no clearing when they change hands.
 #include "common.h"
+#include <algorithm>
 #include <type_traits>
 #include "wave_dpp.h"
 
@@ -228,22 +229,112 @@ __global__ __launch_bounds__((DMAX < 64 ? 64 : DMAX) * IS) void wkv_scan_kernel(
 // A sequence that brings fewer than TOKENWISE tokens (decode) is bound by reading and writing its state: it is walked token by token
 // with the state spread over all threads in 16-byte pieces.
 // 4 x 1024 tokens, 32 heads of 64, bf16: 697 us for the token-by-token scan, 409 us with one set of waves doing both halves' work, 162 us
-// in this form (2.5 us per chunk: the makers' walk through the chunk, 21 vector instructions per token, is the longer half).
+// in this form (2.5 us per chunk: the makers' walk through the chunk, 21 vector instructions per token, is the longer half), 84 us in segments.
 constexpr int CHUNK = 16;
 constexpr int TOKENWISE = 5;
 
+// Long runs on few (sequence, head) pairs are a chain of 2.5 us per 16 tokens on a part of the chip (4 x 1024 tokens, 32 heads: 128 blocks).
+// They are cut into segments that are walked side by side: wkv_segment_kernel forms what each segment
+// but the last adds to the state and the product of its decays, and a segment of wkv_chunk_kernel takes its state from the records of the
+// segments in front of it.  Record 0 of a pair is the state in front of the step (the last segment overwrites its slot), record x + 1 is
+// segment x's: [D][D] and [D] floats.  The last segment of the grid takes all that is left of a run.
+constexpr __host__ __device__ int record_floats(int D) { return D * D + D; }
+__device__ __forceinline__ int segments_of(int tokens, int seg_len, int most) { return min((tokens + seg_len - 1) / seg_len, most); }
+
+// grid (sequence, head, segment): S = sum_s (k_s prod_{x > s} w_x) v_s^T over the segment's tokens, E = prod_x w_x.  SUB tokens at a time,
+// from the last to the first: a thread has one channel of SUB / 4 of them, decays its keys behind each other, and the four groups of a
+// channel meet in LDS; then wave w adds its 16 columns on the fp32 matrix instruction.  Decays are multiplied, as in the chunks.
 template <typename T, int D>
-__global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
+__global__ __launch_bounds__(4 * D) void wkv_segment_kernel(
+    const T* __restrict__ k, const T* __restrict__ v, int64_t ld, const float* __restrict__ logw, const float* __restrict__ state,
+    const int32_t* __restrict__ state_slots, const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions, int H, int d,
+    float* __restrict__ records, int seg_len) {
+    constexpr int SUB = D > 64 ? 32 : 64, PT = SUB / 4, NI = D / 16, SV = D + 16;
+    __shared__ float kd[SUB][SV], vv[SUB][SV], through[4][D];
+    const int b = blockIdx.x, head = blockIdx.y, seg = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int run0 = cu_q[b], run1 = cu_q[b + 1];
+    const int most = gridDim.z + 1;
+    if (seg + 1 >= segments_of(run1 - run0, seg_len, most)) return;
+    float* rec = records + (((int64_t)b * H + head) * most + seg + 1) * record_floats(D);
+    const int64_t col0 = (int64_t)head * d, C = (int64_t)H * d;
+    if (seg == 0) {
+        const float* Sg = state + ((state_slots[b] * (int64_t)H + head) * d) * (int64_t)d;
+        const bool fresh = positions[run0] == 0;
+        for (int x = tid; x < D * D; x += 4 * D) {
+            const int i = x / D, j = x % D;
+            rec[x - record_floats(D)] = (!fresh && i < d && j < d) ? Sg[(int64_t)i * d + j] : 0.f;
+        }
+    }
+    const int t0 = run0 + seg * seg_len;
+    const int ch = tid % D, group = tid / D;
+    const bool mine = ch < d;
+    T pk[PT], pv[PT];
+    float pw[PT];
+    auto fetch = [&](int sub) {
+#pragma unroll
+        for (int x = 0; x < PT; ++x) {
+            const int64_t t = t0 + sub * SUB + group * PT + x;
+            pk[x] = mine ? k[t * ld + col0 + ch] : (T)0.f;
+            pv[x] = mine ? v[t * ld + col0 + ch] : (T)0.f;
+            pw[x] = mine ? logw[t * C + col0 + ch] : 0.f;
+        }
+    };
+    const int lq = lane >> 4, lc = lane & 15, j = 16 * wave + lc;
+    f32x4 S[NI];
+#pragma unroll
+    for (int it = 0; it < NI; ++it) S[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float behind = 1.f;  // the decays of everything behind this part
+    fetch(seg_len / SUB - 1);
+    for (int sub = seg_len / SUB - 1; sub >= 0; --sub) {
+        float key[PT], y = 1.f;
+#pragma unroll
+        for (int x = PT - 1; x >= 0; --x) {
+            key[x] = (float)pk[x] * y;
+            y *= expf(pw[x]);
+        }
+        through[group][ch] = y;
+#pragma unroll
+        for (int x = 0; x < PT; ++x) vv[group * PT + x][ch] = (float)pv[x];
+        __syncthreads();
+        if (sub > 0) fetch(sub - 1);
+        float later = behind;
+#pragma unroll
+        for (int g = 3; g >= 0; --g) {
+            const float z = through[g][ch];
+            if (g > group) later *= z;
+            behind *= z;
+        }
+#pragma unroll
+        for (int x = 0; x < PT; ++x) kd[group * PT + x][ch] = key[x] * later;
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < SUB / 4; ++ks) {
+            const float vb = vv[4 * ks + lq][j];
+#pragma unroll
+            for (int it = 0; it < NI; ++it) S[it] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[4 * ks + lq][16 * it + lc], vb, S[it], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int it = 0; it < NI; ++it)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rec[(16 * it + 4 * lq + e) * D + j] = S[it][e];
+    if (group == 0) rec[D * D + ch] = behind;
+}
+
+template <typename T, int D, bool SEGMENTS>
+__global__ __launch_bounds__(8 * D, SEGMENTS && D == 64 ? 4 : 1) void wkv_chunk_kernel(
     const T* __restrict__ r, const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ gate, int64_t ld,
     const float* __restrict__ logw, const float* __restrict__ u, const float* __restrict__ gain, float* __restrict__ state,
     float* __restrict__ shift_state, const float* __restrict__ h, int64_t W, const int32_t* __restrict__ state_slots,
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions, T* __restrict__ out, int64_t ld_out, int H, int d,
-    float eps) {
+    float eps, const float* __restrict__ records, int seg_len) {
     typedef T T4 __attribute__((ext_vector_type(4)));
     constexpr int NT = 8 * D, NH = NT / 2;  // threads, threads per half
     constexpr int L = D / 4;     // lanes per token
     constexpr int NI = D / 16;   // row tiles of the state
-    constexpr int PRE = D > 64 ? 2 : 8;  // (1024 threads have half the registers)
+    constexpr int PRE = D > 64 || (SEGMENTS && D == 64) ? 2 : 8;  // (1024 threads on a CU have half the registers)
     constexpr int SV = D + 16;   // row stride of operands read as [4 rows][16 columns]: four rows cover the 64 banks
     constexpr int SR = D + 4;    // row stride of operands read as [16 rows][4 columns]
     __shared__ __attribute__((aligned(16))) float rr[CHUNK][D], ww[CHUNK][D], oo[CHUNK][SR];
@@ -257,10 +348,15 @@ __global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
     auto &ee = sm.ee;
     const int b = blockIdx.x, head = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int t0 = cu_q[b], t1 = cu_q[b + 1];
+    int t0 = cu_q[b], t1 = cu_q[b + 1];
     if (t1 <= t0) return;
     const int64_t slot = state_slots[b];
     const bool fresh = positions[t0] == 0;
+    const int segs = SEGMENTS ? segments_of(t1 - t0, seg_len, gridDim.z) : 1, seg = SEGMENTS ? blockIdx.z : 0;
+    if (seg >= segs) return;
+    t0 += seg * seg_len;
+    if (seg + 1 < segs) t1 = t0 + seg_len;
+    const float* rec = SEGMENTS ? records + ((int64_t)b * H + head) * gridDim.z * record_floats(D) : nullptr;
     const int64_t col0 = (int64_t)head * d, C = (int64_t)H * d;
     float* Sg = state + ((slot * H + head) * d) * (int64_t)d;  // [i][j]
     const int half_tid = tid % NH;
@@ -288,13 +384,13 @@ __global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
             *reinterpret_cast<T4*>(out + (int64_t)t * ld_out + col0 + c4) = res;
         }
     };
-    if (head == 0) {
+    if (head == 0 && seg + 1 == segs) {
         const float* last = h + (int64_t)(t1 - 1) * W;
         float* dst = shift_state + slot * W;
         for (int64_t c = tid; c < W; c += NT) dst[c] = last[c];
     }
 
-    if (t1 - t0 < TOKENWISE) {
+    if (!SEGMENTS && t1 - t0 < TOKENWISE) {
         constexpr int RG = NT / L, RPT = D / RG;  // row groups, rows per thread: rows rg, rg + RG, ...
         const int n = t1 - t0, rg = tid / L;
         float(*parts)[TOKENWISE - 1][D] = reinterpret_cast<float(*)[TOKENWISE - 1][D]>(&sm);  // [waves][token][column]
@@ -489,8 +585,22 @@ __global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int i = 16 * it + 4 * lq + e;
-            S[it][e] = (!fresh && i < d && j < d) ? Sg[(int64_t)i * d + j] : 0.f;
+            if (SEGMENTS && segs > 1)
+                S[it][e] = rec[i * D + j];
+            else
+                S[it][e] = (!fresh && i < d && j < d) ? Sg[(int64_t)i * d + j] : 0.f;
         }
+    if (SEGMENTS) {
+        for (int x = 1; x <= seg; ++x) {  // what the segments in front of this one make of the state
+            rec += record_floats(D);
+#pragma unroll
+            for (int it = 0; it < NI; ++it) {
+                const f32x4 e4 = *reinterpret_cast<const f32x4*>(rec + D * D + 16 * it + 4 * lq);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) S[it][e] = e4[e] * S[it][e] + rec[(16 * it + 4 * lq + e) * D + j];
+            }
+        }
+    }
     __syncthreads();
     __syncthreads();  // the makers' first chunk
     for (int c = 0; c < chunks; ++c) {
@@ -537,6 +647,7 @@ __global__ __launch_bounds__(8 * D) void wkv_chunk_kernel(
         finish(*reinterpret_cast<const f32x4*>(&oo[s][c4]), wide4(gt), t, t < t1);
         __syncthreads();
     }
+    if (seg + 1 < segs) return;
 #pragma unroll
     for (int it = 0; it < NI; ++it)
 #pragma unroll
@@ -693,21 +804,48 @@ bool runs_by_token(int64_t blocks, int d, int64_t max_q_len) {
     return max_q_len <= CHUNK ? max_q_len <= (d <= 32 ? 12 : 10) : max_q_len <= (d <= 32 ? 20 : 17);
 }
 
+struct Segments {
+    int count, tokens;
+};
+// As many segments as the chip takes blocks of the chunk kernel at once (two a CU up to d = 64, held to 128 registers there; one above), none
+// shorter than what a block needs to come up.  us, one block per (sequence, head) / segments, bf16: d 64, 32 heads: 4 x 1024 tokens 162 / 84
+// (4 segments; 6 of them 95), 1 x 1024 147 / 37, 1 x 4093 618 / 87, 1 x 256 41 / 25, 4 x 256 42 / 34, 8 x 512 82 / 80, 8 x 1024 160 / 143, 6 x 700
+// 110 / 99; d 32: 4 x 1024, 32 heads 150 / 60; d 128, 16 heads: 4 x 1024 262 / 136 (8 segments 171), 1 x 2048 515 / 162, 8 x 1024 266 / 211.
+Segments segments_for(int64_t blocks, int d, int64_t max_q_len) {
+    const int64_t room = d <= 64 ? 512 : 256, least = d <= 64 ? 64 : 256;
+    const int64_t most = std::min(std::min(room / blocks, max_q_len / least), (int64_t)16);
+    if (most < 2) return {1, 0};
+    const int64_t tokens = cdiv64(cdiv64(max_q_len, most), 64) * 64;
+    return {(int)cdiv64(max_q_len, tokens), (int)tokens};
+}
+
 template <typename T>
 int launch_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw, const float* u,
                 const float* gain, float* state, float* shift_state, const float* h, int64_t W, const int32_t* slots,
                 const int32_t* cu_q, const int32_t* positions, void* out, int64_t ld_out, int B, int H, int d, float eps,
-                int64_t max_q_len, hipStream_t st) {
+                int64_t max_q_len, void* ws, hipStream_t st) {
     // the chunked form takes rows in groups of four elements (any head width that is a multiple of 4, aligned tensors)
     const size_t quad = 4 * sizeof(T);
     auto rows_of_four = [&](const void* p, int64_t stride) { return (uintptr_t)p % quad == 0 && stride % 4 == 0; };
     if (!runs_by_token((int64_t)B * H, d, max_q_len) && d % 4 == 0 && rows_of_four(r, ld) && rows_of_four(k, ld) && rows_of_four(v, ld) && rows_of_four(gate, ld) &&
         rows_of_four(out, ld_out) && (uintptr_t)logw % 16 == 0 && (uintptr_t)u % 16 == 0 && (uintptr_t)gain % 16 == 0 &&
         (uintptr_t)state % 16 == 0) {
-#define TGIS_WKV_CHUNKS(DM)                                                                                                    \
-    hipLaunchKernelGGL((wkv_chunk_kernel<T, DM>), dim3((unsigned)B, (unsigned)H), dim3(8 * DM), 0, st, (const T*)r, (const T*)k, \
-                       (const T*)v, (const T*)gate, ld, logw, u, gain, state, shift_state, h, W, slots, cu_q, positions, (T*)out, \
-                       ld_out, H, d, eps)
+        const Segments cut = segments_for((int64_t)B * H, d, max_q_len);
+        float* records = cut.count > 1 ? (float*)ws : nullptr;
+#define TGIS_WKV_CHUNKS(DM)                                                                                                       \
+    do {                                                                                                                          \
+        if (records) {                                                                                                            \
+            hipLaunchKernelGGL((wkv_segment_kernel<T, DM>), dim3((unsigned)B, (unsigned)H, (unsigned)cut.count - 1), dim3(4 * DM), 0, st, \
+                               (const T*)k, (const T*)v, ld, logw, state, slots, cu_q, positions, H, d, records, cut.tokens);    \
+            hipLaunchKernelGGL((wkv_chunk_kernel<T, DM, true>), dim3((unsigned)B, (unsigned)H, (unsigned)cut.count), dim3(8 * DM), 0, st, \
+                               (const T*)r, (const T*)k, (const T*)v, (const T*)gate, ld, logw, u, gain, state, shift_state, h, W, \
+                               slots, cu_q, positions, (T*)out, ld_out, H, d, eps, records, cut.tokens);                         \
+        } else {                                                                                                                  \
+            hipLaunchKernelGGL((wkv_chunk_kernel<T, DM, false>), dim3((unsigned)B, (unsigned)H), dim3(8 * DM), 0, st, (const T*)r, \
+                               (const T*)k, (const T*)v, (const T*)gate, ld, logw, u, gain, state, shift_state, h, W, slots, cu_q, \
+                               positions, (T*)out, ld_out, H, d, eps, nullptr, 0);                                               \
+        }                                                                                                                         \
+    } while (0)
         if (d <= 32)
             TGIS_WKV_CHUNKS(32);
         else if (d <= 64)
@@ -791,33 +929,54 @@ extern "C" int tgis_wkv_decay(const void* a, int64_t ld_a, const float* w2t, con
     return TGIS_OK;
 }
 
-extern "C" int tgis_wkv_scan_runs(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
-                                  const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
-                                  const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
-                                  int64_t ld_out, int64_t B, int H, int d, float eps, int64_t max_q_len, int dtype, void* stream) {
+extern "C" int64_t tgis_wkv_scan_workspace(int64_t B, int H, int d, int64_t max_q_len) {
+    if (B < 1 || H < 1 || d < 1 || d > 128) return 0;
+    const Segments cut = segments_for(B * H, d, max_q_len);
+    return cut.count > 1 ? B * H * cut.count * record_floats(d <= 32 ? 32 : d <= 64 ? 64 : 128) * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int tgis_wkv_scan_segments(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
+                                      const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
+                                      const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
+                                      int64_t ld_out, int64_t B, int H, int d, float eps, int64_t max_q_len, void* workspace,
+                                      int64_t workspace_bytes, int dtype, void* stream) {
     TGIS_CHECK_ARG(r && k && v && gate && logw && u && gain && state && shift_state && h && state_slots && cu_seqlens_q &&
                        positions && out,
                    "tgis_wkv_scan: null tensor");
     TGIS_CHECK_ARG(B >= 1 && H >= 1 && d >= 1 && d <= 128, "tgis_wkv_scan: head width %d (1 .. 128 supported)", d);
     TGIS_CHECK_ARG(ld >= (int64_t)H * d && ld_out >= (int64_t)H * d && W >= 1 && dtype3(dtype), "tgis_wkv_scan: bad strides or dtype");
+    TGIS_CHECK_ARG(!workspace || ((uintptr_t)workspace % 16 == 0 && workspace_bytes >= tgis_wkv_scan_workspace(B, H, d, max_q_len)),
+                   "tgis_wkv_scan: the workspace must be 16-byte aligned and of tgis_wkv_scan_workspace bytes");
     hipStream_t st = (hipStream_t)stream;
     TgisTimedScope timed(TGIS_OP_SCAN, st);
+#define TGIS_SCAN(TT)                                                                                                                    \
+    launch_scan<TT>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, \
+                    d, eps, max_q_len, workspace, st)
     if (dtype == TGIS_F16)
-        launch_scan<f16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, max_q_len, st);
+        TGIS_SCAN(f16);
     else if (dtype == TGIS_BF16)
-        launch_scan<bf16>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, max_q_len, st);
+        TGIS_SCAN(bf16);
     else
-        launch_scan<float>(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, (int)B, H, d, eps, max_q_len, st);
+        TGIS_SCAN(float);
+#undef TGIS_SCAN
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
+}
+
+extern "C" int tgis_wkv_scan_runs(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
+                                  const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
+                                  const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
+                                  int64_t ld_out, int64_t B, int H, int d, float eps, int64_t max_q_len, int dtype, void* stream) {
+    return tgis_wkv_scan_segments(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out,
+                                  ld_out, B, H, d, eps, max_q_len, nullptr, 0, dtype, stream);
 }
 
 extern "C" int tgis_wkv_scan(const void* r, const void* k, const void* v, const void* gate, int64_t ld, const float* logw,
                              const float* u, const float* gain, float* state, float* shift_state, const float* h, int64_t W,
                              const int32_t* state_slots, const int32_t* cu_seqlens_q, const int32_t* positions, void* out,
                              int64_t ld_out, int64_t B, int H, int d, float eps, int dtype, void* stream) {
-    return tgis_wkv_scan_runs(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out, ld_out, B, H,
-                              d, eps, 0, dtype, stream);
+    return tgis_wkv_scan_segments(r, k, v, gate, ld, logw, u, gain, state, shift_state, h, W, state_slots, cu_seqlens_q, positions, out,
+                                  ld_out, B, H, d, eps, 0, nullptr, 0, dtype, stream);
 }
 
 // rows of groups of four aligned elements, as the chunk form wants them; d <= 128, rank <= STEP_MAX_RANK

@@ -114,6 +114,9 @@ SIGNATURES = {
                                _c_i64, _c_int, _c_int, _c_f, _c_int, _vp]),
     "tgis_wkv_scan_runs": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64,
                                _c_i64, _c_int, _c_int, _c_f, _c_i64, _c_int, _vp]),
+    "tgis_wkv_scan_workspace": (_c_i64, [_c_i64, _c_int, _c_int, _c_i64]),
+    "tgis_wkv_scan_segments": (_c_int, [_vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64,
+                                        _c_i64, _c_int, _c_int, _c_f, _c_i64, _vp, _c_i64, _c_int, _vp]),
     "tgis_moe_row_capacity": (_c_i64, [_c_i64, _c_i64, _c_int]),
     "tgis_moe_route": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int, _c_int, _vp]),
     "tgis_moe_align": (_c_int, [_vp, _c_i64, _c_int, _vp, _c_i64, _vp, _vp, _vp, _c_int, _vp]),
@@ -1102,11 +1105,14 @@ def wkv_scan(r, k, v, gate, logw, u, gain, state, shift_state, h, state_slots, c
     ld = r.stride(0)
     assert all(t.stride(0) == ld and t.stride(1) == 1 and t.dtype == r.dtype for t in (k, v, gate))
     out = torch.empty((T, H * d), dtype=r.dtype, device=r.device)
-    _check(load_library().tgis_wkv_scan_runs(
+    lib, B = load_library(), state_slots.shape[0]
+    room = lib.tgis_wkv_scan_workspace(B, H, d, int(max_q_len)) if T > B else 0  # (single tokens are never cut)
+    ws = torch.empty(room, dtype=torch.uint8, device=r.device) if room else None
+    _check(lib.tgis_wkv_scan_segments(
         _ptr(r), _ptr(k), _ptr(v), _ptr(gate), ld, _f32(logw, "logw"), _f32(u, "u"), _f32(gain, "gain"), _f32(state, "state"),
         _f32(shift_state, "shift_state"), _f32(h, "h"), h.shape[1], _i32(state_slots, "state_slots"),
-        _i32(cu_seqlens_q, "cu_seqlens_q"), _i32(positions, "positions"), _ptr(out), out.stride(0), state_slots.shape[0], H, d,
-        float(eps), int(max_q_len), dtype_code3(r.dtype), _stream()), "tgis_wkv_scan_runs")
+        _i32(cu_seqlens_q, "cu_seqlens_q"), _i32(positions, "positions"), _ptr(out), out.stride(0), B, H, d,
+        float(eps), int(max_q_len), _ptr(ws), room, dtype_code3(r.dtype), _stream()), "tgis_wkv_scan_segments")
     return out
 
 
