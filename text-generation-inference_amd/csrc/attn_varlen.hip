@@ -191,6 +191,48 @@ __global__ __launch_bounds__(256) void qk_norm_kv_write_kernel(
     for (int d = lane; d < dk; d += 64) dst[d] = (T)(ldf(p + d) * rinv * w[d]);
 }
 
+// The norm of q and k alone, for long steps of two-byte models: L lanes take one head of up to 8 L channels with one 16-byte load each, so
+// a wave has 64 / L heads in flight.  Bound by its bytes; with a wave per head (above) a head of 64 was one 128-byte load and a six-step
+// sum per wave, 147 thousand waves for 4096 tokens of 36 heads.  us, with the values' launch, before / now: 512, 1024, 4096 tokens of 36 heads
+// of 64 9.6 / 6.3, 13.9 / 7.1, 38 / 13; 4096 of 40 heads of 128 47 / 23, 18 of 256 30 / 20; 600 of 10 heads of 128 7.0 / 6.1.
+template <typename T, int L>
+__global__ __launch_bounds__(256) void qk_norm_rows_kernel(
+    T* __restrict__ qkv, int64_t ld, const int32_t* __restrict__ positions, const int32_t* __restrict__ slots,
+    const float* __restrict__ qw, const float* __restrict__ kw, float eps, float gain_coef, int gain_every, T* __restrict__ k_pool,
+    int64_t Ttot, int H, int G, int dk) {
+    using V8 = typename VecT<T>::x8;
+    const int64_t item = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
+    const int64_t t = item / (H + G);
+    const int h = (int)(item - t * (H + G)), c = threadIdx.x % L * 8;
+    const bool live = t < Ttot, mine = live && c < dk;  // (lanes without work stay for the sums)
+    T* p = qkv + t * ld + (int64_t)h * dk + c;
+    const V8 x = mine ? *reinterpret_cast<const V8*>(p) : V8{};
+    f32x4 w[2] = {};
+    float gain = 1.f;
+    if (mine) {
+        const float* wp = (h < H ? qw : kw) + c;
+        w[0] = *reinterpret_cast<const f32x4*>(wp);
+        w[1] = *reinterpret_cast<const f32x4*>(wp + 4);
+        if (h < H) {
+            if (gain_every > 0) gain = 1.f + gain_coef * logf((float)((positions[t] + 1) / gain_every) + 1.f);
+        } else {
+            const int slot = slots[t];
+            p = k_pool + (((int64_t)(slot / PAGE) * G + (h - H)) * PAGE + slot % PAGE) * dk + c;
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss += (float)x[e] * (float)x[e];
+    ss = sum_neighbours<(L < 16 ? L : 16)>(ss);
+    if (L > 16) ss += __shfl_xor(ss, 16, 64);
+    const float rinv = 1.0f / sqrtf(ss / (float)dk + eps) * gain;
+    if (!mine) return;
+    V8 y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = (T)((float)x[e] * rinv * w[e / 4][e % 4]);
+    *reinterpret_cast<V8*>(p) = y;
+}
+
 // value column i (of G * dv, dv even) of one token, turned by the token's position: turns [dv / 2] (cos, sin)
 template <typename T> __device__ __forceinline__ float turned_value(const T* __restrict__ vrow, int i, int dv, const float* __restrict__ turns) {
     const float v = (float)vrow[i], o = (float)vrow[i ^ 1];
@@ -1370,9 +1412,27 @@ int launch_prep(void* qkv, int64_t ld, const int32_t* positions, const int32_t* 
     // portions) take the transposing writer, whose stores are whole page rows
     const int v_inline = T_ < 512 ? 1 : 0;
     const int v_blocks = v_inline ? (int)cdiv64((int64_t)G * dv, 1024) : 0;
-    hipLaunchKernelGGL(qk_norm_kv_write_kernel<T>, dim3((unsigned)T_, (unsigned)((H + G + 3) / 4 + v_blocks)), dim3(256), 0, st, (T*)qkv, ld,
-                       positions, slots, qw, kw, eps, gain_coef, gain_every, (const T*)v_first, ld_vf, lam, (T*)k_pool, (T*)v_pool, H, G, dk,
-                       dv, v_inline);
+    bool rows = false;
+    if constexpr (sizeof(T) == 2) {
+        rows = !v_inline && dk % 8 == 0 && dk <= 256 && ld % 8 == 0 && ((uintptr_t)qkv | (uintptr_t)k_pool | (uintptr_t)qw | (uintptr_t)kw) % 16 == 0;
+        if (rows) {
+            const int64_t items = T_ * (H + G);
+#define TGIS_NORM_ROWS(L)                                                                                                                  \
+    hipLaunchKernelGGL((qk_norm_rows_kernel<T, L>), dim3((unsigned)cdiv64(items, 256 / L)), dim3(256), 0, st, (T*)qkv, ld, positions, slots, \
+                       qw, kw, eps, gain_coef, gain_every, (T*)k_pool, T_, H, G, dk)
+            if (dk <= 64)
+                TGIS_NORM_ROWS(8);
+            else if (dk <= 128)
+                TGIS_NORM_ROWS(16);
+            else
+                TGIS_NORM_ROWS(32);
+#undef TGIS_NORM_ROWS
+        }
+    }
+    if (!rows)
+        hipLaunchKernelGGL(qk_norm_kv_write_kernel<T>, dim3((unsigned)T_, (unsigned)((H + G + 3) / 4 + v_blocks)), dim3(256), 0, st, (T*)qkv, ld,
+                           positions, slots, qw, kw, eps, gain_coef, gain_every, (const T*)v_first, ld_vf, lam, (T*)k_pool, (T*)v_pool, H, G, dk,
+                           dv, v_inline);
     if (!v_inline)
         hipLaunchKernelGGL(v_write_kernel<T>, dim3((unsigned)cdiv64(T_, 32), (unsigned)cdiv64((int64_t)G * dv, 64)), dim3(256), 0, st,
                            (const T*)qkv, ld, (int64_t)(H + G) * dk, slots, (const T*)v_first, ld_vf, lam, (T*)v_pool, T_, G, dv, (const float*)nullptr);
