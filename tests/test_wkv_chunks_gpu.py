@@ -80,6 +80,21 @@ def test_token_shift_and_decay(gpu_device, W, dtype):
         assert ((lw + z.exp()).abs() <= 1e-5 * (1 + z.exp())).all()
 
 
+# tokens, channels, rank: whole tiles of 64 x 256 and ragged ones, ranks of one and two blocks of 64 and past them
+@pytest.mark.parametrize("T,W,rank", [(513, 2100, 64), (1000, 1100, 130), (2049, 1536, 67), (3200, 1030, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_decay_in_tiles(gpu_device, T, W, rank, dtype):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(T)
+    a = torch.randn(T, rank + 3, generator=g).to(dtype).to(gpu_device)[:, :rank]
+    w2t, w0 = (torch.randn(rank, W, generator=g) * rank ** -0.5).to(gpu_device), torch.randn(W, generator=g).to(gpu_device)
+    lw = native.wkv_decay(a, w2t, w0).double()
+    z = w0.double() + torch.tanh(a.double()) @ w2t.double()
+    # an fp32 sum of up to 130 terms of size rank ** -0.5 (some ten roundings of 6e-8 of a sum of up to 5), which exp turns into a relative error
+    assert lw.shape == (T, W) and ((lw + z.exp()).abs() <= 1e-5 * z.exp()).all()
+
+
 # ranks: one, fewer than a thread's first load, exactly those, more; lens: single tokens, none, and a few one after another
 @pytest.mark.parametrize("d,rank", [(64, 64), (64, 5), (32, 1), (8, 70), (48, 200), (128, 32), (100, 129)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

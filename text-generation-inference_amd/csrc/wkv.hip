@@ -86,6 +86,68 @@ __global__ __launch_bounds__(256) void wkv_decay_kernel(const T* __restrict__ a,
         if (t < n) logw[(t0 + t) * C + c] = -expf(z[t]);
 }
 
+// The same for long steps as a product on the fp32 matrix instruction (16x16x4): a workgroup has 64 tokens x 256 channels, wave w its
+// channels 32 w .. + 31; 64 ranks at a time, w2t's rows go straight to the B operand and are on their way while tanh(a) is staged in LDS.
+// Eight tokens per read of w2t's columns were bound by those reads from L2 (4096 x 2048, rank 64: 41 us; 23 in this form, of which the
+// matrix instruction needs 7 and the tanh of each of the eight column blocks 2).  Two workgroups a CU: 25 us with one.
+constexpr int DECAY_TOKENS = 64, DECAY_COLS = 256, DECAY_RANKS = 64;
+
+template <typename T>
+__global__ __launch_bounds__(512, 4) void wkv_decay_tiles_kernel(const T* __restrict__ a, int64_t ld_a, const float* __restrict__ w2t,
+                                                              const float* __restrict__ w0, float* __restrict__ logw, int R, int64_t C,
+                                                              int64_t Ttot) {
+    __shared__ float th[DECAY_TOKENS][DECAY_RANKS + 4];
+    constexpr int STEPS = DECAY_RANKS / 4, PER = DECAY_TOKENS / 8;
+    const int64_t t0 = (int64_t)blockIdx.x * DECAY_TOKENS;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lq = lane >> 4, lc = lane & 15;
+    const int64_t c0 = (int64_t)blockIdx.y * DECAY_COLS + wave * 32 + lc;
+    bool in[2];
+    f32x4 z[4][2];
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+        in[ct] = c0 + 16 * ct < C;
+        const float z0 = in[ct] ? w0[c0 + 16 * ct] : 0.f;
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) z[rt][ct] = f32x4{z0, z0, z0, z0};
+    }
+    for (int r0 = 0; r0 < R; r0 += DECAY_RANKS) {
+        float x[PER], b[STEPS][2];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int64_t t = t0 + wave + 8 * i;
+            x[i] = (r0 + lane < R && t < Ttot) ? ldf(a + t * ld_a + r0 + lane) : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < STEPS; ++k)
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct)
+                b[k][ct] = (in[ct] && r0 + 4 * k + lq < R) ? w2t[(int64_t)(r0 + 4 * k + lq) * C + c0 + 16 * ct] : 0.f;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) th[wave + 8 * i][lane] = tanhf(x[i]);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < STEPS; ++k) {
+            if (r0 + 4 * k >= R) break;
+#pragma unroll
+            for (int rt = 0; rt < 4; ++rt) {
+                const float y = th[16 * rt + lc][4 * k + lq];
+#pragma unroll
+                for (int ct = 0; ct < 2; ++ct) z[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, b[k][ct], z[rt][ct], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t t = t0 + 16 * rt + 4 * lq + e;
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct)
+                if (t < Ttot && in[ct]) logw[t * C + c0 + 16 * ct] = -expf(z[rt][ct][e]);
+        }
+}
+
 // One workgroup per (sequence, head) = four thread groups: thread (q, j) owns value channel j and keeps the rows
 // i in [q DQ, (q + 1) DQ) of column j of S in registers (rows of S evolve independently of each other, so the four groups
 // never have to meet inside a token: each leaves its part of o in LDS and the parts are added once per chunk).  Tokens are
@@ -908,6 +970,23 @@ extern "C" int tgis_wkv_decay(const void* a, int64_t ld_a, const float* w2t, con
     TGIS_CHECK_ARG(a && w2t && w0 && logw && rank >= 1 && rank <= 8192 && C >= 1 && C <= 65535 * 256 && ld_a >= rank && dtype3(dtype), "tgis_wkv_decay: bad arguments");
     if (T == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
+    const int64_t tiles = cdiv64(T, DECAY_TOKENS) * cdiv64(C, DECAY_COLS);
+    // us, the forms without tiles / tiles: rank 64, 2048 channels: 512 tokens 13.4 / 12.3, 1024 12.7 / 13.4, 2048 22 / 14.9, 4096 41 / 23, 8192 78 /
+    // 42; 512 x 4096 22 / 13; 4096 x 256 8.3 / 12.4; rank 128: 256 x 4096 23 / 19.5, 1024 x 2048 22 / 20.5; rank 256, 4096 x 2048 138 / 60; rank 16,
+    // 4096 x 4096 26 / 29.  (Below 1024 tokens the other form is a token per workgroup.)
+    if (rank >= 64 && tiles >= (T < 1024 ? 64 : 192) && C <= (int64_t)65535 * DECAY_COLS) {
+        const dim3 cut((unsigned)cdiv64(T, DECAY_TOKENS), (unsigned)cdiv64(C, DECAY_COLS));
+#define TGIS_DECAY(TT) hipLaunchKernelGGL(wkv_decay_tiles_kernel<TT>, cut, dim3(512), 0, st, (const TT*)a, ld_a, w2t, w0, logw, rank, C, T)
+        if (dtype == TGIS_F16)
+            TGIS_DECAY(f16);
+        else if (dtype == TGIS_BF16)
+            TGIS_DECAY(bf16);
+        else
+            TGIS_DECAY(float);
+#undef TGIS_DECAY
+        TGIS_CHECK_LAUNCH();
+        return TGIS_OK;
+    }
     const int tb = T >= 1024 && rank <= 512 && cdiv64(T, 8) * cdiv64(C, 256) >= 256 ? 8 : 1;
     const size_t lds = (size_t)rank * tb * sizeof(float);
     const dim3 grid((unsigned)cdiv64(T, tb), (unsigned)cdiv64(C, 256));
