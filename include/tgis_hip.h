@@ -279,6 +279,12 @@ int tgis_attn_paged(const void* q, int64_t ld_q, const void* k_pool, const void*
                     const int32_t* cu_seqlens_q, void* out, int64_t ld_out, int64_t B, int H, int Hkv, int D,
                     int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
                     void* workspace, int64_t workspace_bytes, void* stream);
+/* ... of a decode step (one token per sequence), written in fragment order with output column k at column out_cols[k] (a permutation of
+ * 0 .. H * D - 1): the order an act-order matrix behind it wants its operand in. */
+int tgis_attn_paged_ordered(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,
+                            int64_t max_pages, const int32_t* ctx_lens, const int32_t* cu_seqlens_q, void* out,
+                            const int32_t* out_cols, int64_t B, int H, int Hkv, int D, int64_t max_ctx, float scale, int dtype,
+                            int num_splits, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---- elementwise --------------------------------------------------------------------------------- */
 /* out[T,I] = act(gate_up[T,0:I]) * gate_up[T,I:2I]; act 1 = SiLU (flash_llama_modeling.py:332-335). */

@@ -96,3 +96,25 @@ def test_linear_gathers_its_operand(gpu_device, M, groupsize):
             part = down(h, partial=True)
             rows = part.slabs.view(-1)[:(M + 31) // 32 * part.S * 32 * part.ld].view(-1, part.S, 32, part.ld).sum(1).reshape(-1, part.ld)
             close(rows[:M, :256], want, tol_out)
+
+
+# unsplit blocks of four and eight waves, splits merged in the launch, the combine launch of multi-chunk blocks; more than 32 rows
+@pytest.mark.parametrize("B,H,Hkv,D,ctx", [(11, 32, 32, 128, 200), (3, 8, 2, 64, 70), (2, 32, 32, 128, 1500), (2, 48, 1, 128, 1500), (40, 16, 4, 128, 90)])
+def test_decode_attention_writes_columns_at_their_places(gpu_device, B, H, Hkv, D, ctx):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(B + ctx)
+    W = (ctx + 31) // 32
+    ctx_lens = torch.randint(1, ctx + 1, (B,), generator=g).int()
+    ctx_lens[0] = ctx
+    k_pool, v_pool = (torch.randn(B * W, Hkv, 32 * D, generator=g).half().to(gpu_device) for _ in range(2))
+    q = torch.randn(B, H * D, generator=g).half().to(gpu_device)
+    tables = torch.randperm(B * W, generator=g).int().view(B, W).to(gpu_device)
+    places = torch.randperm(H * D, generator=g).int().to(gpu_device)
+    splits = native.attn_num_splits(B, Hkv, H, 1, ctx)
+    ws = native.Workspace(max(native.attn_workspace_bytes(B, H, Hkv, D, splits), 256), gpu_device)
+    cu = torch.arange(B + 1, dtype=torch.int32, device=gpu_device)
+    plain, placed = native.FragAct.empty(B, H * D, gpu_device), native.FragAct.empty(B, H * D, gpu_device)
+    for out, cols in ((plain, None), (placed, places)):
+        native.attn_paged(q, H * D, k_pool, v_pool, tables, ctx_lens.to(gpu_device), cu, out, B, H, Hkv, D, 1, ctx, D ** -0.5, splits, ws, out_cols=cols)
+    assert torch.equal(placed.to_rows()[:, places.long()], plain.to_rows())

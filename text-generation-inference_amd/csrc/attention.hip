@@ -37,6 +37,24 @@
 
 namespace {
 
+// Eight neighbouring output columns, k0 .. k0 + 7 of token tok.  With out_cols they go to the places that the act-order matrix behind the
+// launch wants them in, by two-byte stores all over a row: the lines that several XCDs write in parts cost 2.4 us a launch (11 rows of 4096),
+// the gather launch that they replace 4.7 (7B, 11 ragged sequences, the whole step: 2638 -> 2562 us; asking for the places in front of the
+// waves' meeting changes nothing).
+template <typename T>
+__device__ __forceinline__ void store_out(const AttnArgs& a, int64_t tok, int k0, typename VecT<T>::x8 v) {
+    const int64_t K = a.ld_out;  // H * D
+    T* out = reinterpret_cast<T*>(a.out);
+    if (a.out_cols) {
+        int to[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) to[e] = a.out_cols[k0 + e];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) out[xf_off(tok, to[e], K)] = v[e];
+        return;
+    }
+    st16(out + (a.out_frag ? xf_off(tok, k0, K) : tok * K + k0), v);
+}
 
 // NW = waves per workgroup (the key range of a block is dealt page-by-page to its waves)
 // PIPE: two pages of K/V loads in flight per wave (twice the fragment registers)
@@ -342,8 +360,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
             V8 ov;
 #pragma unroll
             for (int e = 0; e < 8; ++e) ov[e] = from_f32<T>(acc[e] * inv);
-            st16(reinterpret_cast<T*>(a.out) + (a.out_frag ? xf_off(tokidx, (int64_t)headj * D + dc * 8, (int64_t)a.H * D)
-                                                           : (tokidx * a.H + headj) * D + dc * 8), ov);
+            store_out<T>(a, tokidx, headj * D + dc * 8, ov);
         } else if (a.counters) {
             // fused combine: the record leaves as 16-byte write-through stores (no other block's record shares a
             // 128-byte line with it: 16 columns x NS x 16 bytes per (group, chunk))
@@ -458,8 +475,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
             for (int e = 0; e < 8; ++e) ov[e] = from_f32<T>(acc[it][e] * inv);
             const int64_t tokidx = q0 + t0 + tqj;
             const int headj = hk * a.G + (hc0 + ch) * 16 + gj;
-            st16(reinterpret_cast<T*>(a.out) + (a.out_frag ? xf_off(tokidx, (int64_t)headj * D + dcs[it] * 8, (int64_t)a.H * D)
-                                                           : (tokidx * a.H + headj) * D + dcs[it] * 8), ov);
+            store_out<T>(a, tokidx, headj * D + dcs[it] * 8, ov);
         }
     }
 }
@@ -471,7 +487,8 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
 template <typename T, int D, int MAXS>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restrict__ ws_o,
                                                            const float* __restrict__ ws_ml, T* __restrict__ out,
-                                                           int NS, int H, int out_frag, int64_t rows) {
+                                                           int NS, int H, int out_frag, const int32_t* __restrict__ out_cols,
+                                                           int64_t rows) {
     const int64_t th = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // tok*H + head
     if (th >= rows) return;
     const int lane = threadIdx.x & 63;
@@ -511,7 +528,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
     for (int i = 0; i < D / 64; ++i) {
-        const int64_t o = out_frag ? xf_off(th / H, (th % H) * D + i * 64 + lane, (int64_t)H * D) : th * D + i * 64 + lane;
+        const int64_t k = (th % H) * D + i * 64 + lane;
+        const int64_t o = out_frag ? xf_off(th / H, out_cols ? out_cols[k] : k, (int64_t)H * D) : th * D + i * 64 + lane;
         out[o] = from_f32<T>(acc[i] * inv);
     }
 }
@@ -580,10 +598,10 @@ static int launch_attn(const AttnArgs& a, dim3 grid, int64_t total_q, hipStream_
         const int64_t rows = total_q * a.H;
         if (a.NS <= 8)
             hipLaunchKernelGGL((attn_combine_kernel<T, D, 8>), dim3((unsigned)cdiv64(rows, 4)), dim3(256), 0, st, a.ws_o,
-                               a.ws_ml, (T*)a.out, a.NS, a.H, a.out_frag, rows);
+                               a.ws_ml, (T*)a.out, a.NS, a.H, a.out_frag, a.out_cols, rows);
         else
             hipLaunchKernelGGL((attn_combine_kernel<T, D, 0>), dim3((unsigned)cdiv64(rows, 4)), dim3(256), 0, st, a.ws_o,
-                               a.ws_ml, (T*)a.out, a.NS, a.H, a.out_frag, rows);
+                               a.ws_ml, (T*)a.out, a.NS, a.H, a.out_frag, a.out_cols, rows);
         TGIS_CHECK_LAUNCH();
     }
     return TGIS_OK;
@@ -763,8 +781,8 @@ struct CounterLease {  // gives the slot back when the launch is in its stream (
 
 static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool,
                            const int32_t* block_tables, int64_t max_pages, const int32_t* ctx_lens,
-                           const int32_t* cu_seqlens_q, void* out, int64_t ld_out, int64_t B, int H, int Hkv, int D,
-                           int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
+                           const int32_t* cu_seqlens_q, void* out, int64_t ld_out, const int32_t* out_cols, int64_t B, int H, int Hkv,
+                           int D, int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
                            void* workspace, int64_t workspace_bytes, void* stream) {
     TGIS_CHECK_ARG(q && k_pool && v_pool && block_tables && ctx_lens && cu_seqlens_q && out,
                    "tgis_attn_paged: null tensor");
@@ -778,6 +796,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
                        (ld_out == TGIS_LD_FRAGMENTS && max_q_len == 1 && B <= 64 && ((int64_t)H * D) % 64 == 0),
                    "tgis_attn_paged: out is [tokens, H * D] contiguous (ld_out = 0 or H * D), or — decode, <= 64 sequences — in "
                    "fragment order (ld_out = TGIS_LD_FRAGMENTS)");
+    TGIS_CHECK_ARG(!out_cols || ld_out == TGIS_LD_FRAGMENTS, "tgis_attn_paged: columns are re-ordered in fragment order only");
     (void)max_ctx;
     if (B == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
@@ -792,6 +811,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     a.ctx_lens = ctx_lens;
     a.cu_q = cu_seqlens_q;
     a.out = out;
+    a.out_cols = out_cols;
     a.out_frag = ld_out == TGIS_LD_FRAGMENTS;
     a.ld_out = (int64_t)H * D;
     attn_set_geom(a, H, Hkv, g);
@@ -859,7 +879,15 @@ extern "C" int tgis_attn_paged(const void* q, int64_t ld_q, const void* k_pool, 
                                const int32_t* cu_seqlens_q, void* out, int64_t ld_out, int64_t B, int H, int Hkv, int D,
                                int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
                                void* workspace, int64_t workspace_bytes, void* stream) {
-    return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, ld_out, B, H, Hkv, D,
+    return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, ld_out, nullptr, B, H, Hkv, D,
                            max_q_len, max_ctx, scale, dtype, num_splits, workspace, workspace_bytes, stream);
 }
 
+extern "C" int tgis_attn_paged_ordered(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,
+                                       int64_t max_pages, const int32_t* ctx_lens, const int32_t* cu_seqlens_q, void* out,
+                                       const int32_t* out_cols, int64_t B, int H, int Hkv, int D, int64_t max_ctx, float scale, int dtype,
+                                       int num_splits, void* workspace, int64_t workspace_bytes, void* stream) {
+    TGIS_CHECK_ARG(out_cols, "tgis_attn_paged_ordered: null order");
+    return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, TGIS_LD_FRAGMENTS, out_cols, B, H,
+                           Hkv, D, 1, max_ctx, scale, dtype, num_splits, workspace, workspace_bytes, stream);
+}

@@ -148,6 +148,7 @@ class FlashLlamaAttention:
         # steps of up to 64 rows (where native.rope_gemm_ok) rotate q / k and write the cache in the GEMM epilogue, prompts where that pays
         if hasattr(self.query_key_value.linear, "rope_heads"):
             self.query_key_value.linear.rope_heads = (self.num_heads, self.num_key_value_heads, self.head_size)
+        self.out_places: Optional[torch.Tensor] = None  # an act-order o_proj's order of the attention's output columns (post_init)
 
     def project_qkv(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False):
         """qkv GEMM, rotation of q and k in place, k and v scattered to their page slots (reference :251-268,282).
@@ -178,7 +179,11 @@ class FlashLlamaAttention:
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         T = qkv.shape[0]
         B = kv.block_tables.shape[0]
-        if frag_rows(self.o_proj.linear, T, kv):  # decode: the o_proj GEMM reads its operand in fragment order
+        # decode: the o_proj GEMM reads its operand in fragment order, an act-order one with its columns in its own
+        places = {}
+        if frag_rows(self.o_proj.linear, T, kv, gathers=self.out_places is not None):
+            if self.out_places is not None:
+                places = {"out_cols": self.out_places}
             attn_output = native.FragAct.empty(T, H * D, qkv.device)
         else:
             attn_output = torch.empty((T, H * D), dtype=qkv.dtype, device=qkv.device)
@@ -188,7 +193,7 @@ class FlashLlamaAttention:
             ws = workspace(qkv.device)
             ws.ensure(native.attn_workspace_bytes(T, H, Hkv, D, kv.num_splits))
         native.attn_paged(qkv, qkv.stride(0), k_pool, v_pool, kv.block_tables, kv.ctx_lens, cu_seqlens_q,
-                          attn_output, B, H, Hkv, D, kv.max_q_len, kv.max_ctx, self.softmax_scale, kv.num_splits, ws)
+                          attn_output, B, H, Hkv, D, kv.max_q_len, kv.max_ctx, self.softmax_scale, kv.num_splits, ws, **places)
         return attn_output
 
     def forward(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False):
@@ -328,6 +333,10 @@ class FlashLlamaForCausalLM:
         for lin in self.gptq_linears:
             if lin.q_handle is None:
                 lin.post_init()
+        for layer in self.model.layers:
+            o_proj = layer.self_attn.o_proj.linear
+            if hasattr(o_proj, "places"):
+                layer.self_attn.out_places = o_proj.places()
 
     def get_input_embeddings(self):
         return self.model.embed_tokens

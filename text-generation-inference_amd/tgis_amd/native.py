@@ -85,6 +85,8 @@ SIGNATURES = {
     "tgis_attn_workspace_bytes": (_c_i64, [_c_i64, _c_int, _c_int, _c_int, _c_int]),
     "tgis_attn_paged": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int,
                                  _c_int, _c_i64, _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
+    "tgis_attn_paged_ordered": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int,
+                                         _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
     "tgis_act_mul": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_int, _c_int, _vp]),
     "tgis_gelu": (_c_int, [_vp, _vp, _c_i64, _c_int, _c_int, _vp]),
     "tgis_embedding": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
@@ -837,9 +839,10 @@ def attn_workspace_bytes(total_q: int, H: int, Hkv: int, D: int, num_splits: int
 
 
 def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_q, out, B: int, H: int, Hkv: int,
-               D: int, max_q_len: int, max_ctx: int, scale: float, num_splits: int, ws: Optional[Workspace]):
+               D: int, max_q_len: int, max_ctx: int, scale: float, num_splits: int, ws: Optional[Workspace],
+               out_cols: Optional[torch.Tensor] = None):
     """q is a (view into a) [T, *] activation whose row stride is ld_q elements; out [T, H*D], or (decode, B <= 32) a
-    FragAct of that shape for the o_proj GEMM."""
+    FragAct of that shape for the o_proj GEMM, with out_cols (int32, a permutation) with its columns at those places."""
     assert block_tables.dtype == torch.int32 and ctx_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
     assert block_tables.is_contiguous()
     if isinstance(out, FragAct):
@@ -849,6 +852,13 @@ def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_
         assert out.is_contiguous()
         optr, ldo = _ptr(out), H * D
     wptr, wbytes = (ws.ptr, ws.nbytes) if ws is not None else (None, 0)
+    if out_cols is not None:
+        assert ldo == LD_FRAGMENTS and out_cols.dtype == torch.int32 and out_cols.is_contiguous() and out_cols.numel() == H * D
+        _check(load_library().tgis_attn_paged_ordered(_ptr(q), ld_q, _ptr(k_pool), _ptr(v_pool), _ptr(block_tables), block_tables.shape[1],
+                                                      _ptr(ctx_lens), _ptr(cu_seqlens_q), optr, _ptr(out_cols), B, H, Hkv, D, max_ctx,
+                                                      float(scale), dtype_code(q.dtype), num_splits, wptr, wbytes, _stream()),
+               "tgis_attn_paged_ordered")
+        return out
     _check(
         load_library().tgis_attn_paged(_ptr(q), ld_q, _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
                                        block_tables.shape[1], _ptr(ctx_lens), _ptr(cu_seqlens_q), optr, ldo, B, H,

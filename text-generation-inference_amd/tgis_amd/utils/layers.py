@@ -190,6 +190,16 @@ class Ex4bitLinearV2:
             self.post_init()
         return self._perm
 
+    def places(self) -> Optional[torch.Tensor]:
+        """Where each column of the activation goes in the image's order (int32): for a producer that writes its columns one by one (decode
+        attention).  None without act-order and where `perm` is no permutation of the columns."""
+        if self.perm is None or self._perm.numel() != self.height:
+            return None
+        order, columns = self._perm.long(), torch.arange(self.height, device=self._perm.device)
+        if not bool((order.sort().values == columns).all()):
+            return None
+        return torch.empty_like(order).scatter_(0, order, columns).to(torch.int32)
+
     def order_columns(self, order: torch.Tensor):
         """Before post_init: re-order the output columns, y[:, i] = old y[:, order[i]]."""
         assert self.q_handle is None
