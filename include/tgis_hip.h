@@ -169,6 +169,26 @@ int tgis_dense_gemm_rope(const void* x, int64_t ldx, const void* prepared, const
 int tgis_gptq_dequant_f16(const void* prepared, void* w_out, int64_t K, int64_t N, int64_t groups,
                           int flags, void* stream);
 
+/* Decode steps of up to 4 rows: dense products that norm their operand themselves and add to the residual stream, which stays in fp32
+ * (h, [M][width], rows back to back) between them.  With norm(h)[k] = T(h[k] * rstd * norm_w[k]), norm_w of the model dtype, and the images of
+ * tgis_dense_prepare:
+ *   tgis_dense_rows_norm_rope   qkv of norm(h), rotated, k and v to their cache slots (as tgis_dense_gemm_rope; the rope image)
+ *   tgis_dense_rows_residual    h[m][n] = T(x W^T)[m][n] + T(h[m][n]) in place, h of width N
+ *   tgis_dense_rows_norm_silu   T(T(silu(T gate)) * T up) of norm(h) (the gate|up image), [M][N / 2]
+ *   tgis_dense_rows_norm_head   fp32 norm(h) W^T
+ * tgis_dense_rows_ok: whether M rows of K columns are served (norm: one of the three that norm; a size query). */
+int tgis_dense_rows_ok(int64_t M, int64_t K, int norm);
+int tgis_dense_rows_norm_rope(const float* h, const void* norm_w, float eps, const void* prepared, const void* bias,
+                              const int32_t* positions, const int32_t* slots, const void* cos, const void* sin, void* q_out, int64_t ldq,
+                              void* k_pool, void* v_pool, int64_t M, int64_t K, int64_t H, int64_t Hkv, int64_t D, int dtype,
+                              void* stream);
+int tgis_dense_rows_residual(const void* x, int64_t ldx, const void* prepared, float* h, int64_t M, int64_t K, int64_t N, int dtype,
+                             void* stream);
+int tgis_dense_rows_norm_silu(const float* h, const void* norm_w, float eps, const void* prepared, void* out, int64_t ldo, int64_t M,
+                              int64_t K, int64_t N, int dtype, void* stream);
+int tgis_dense_rows_norm_head(const float* h, const void* norm_w, float eps, const void* prepared, float* out, int64_t ldo, int64_t M,
+                              int64_t K, int64_t N, int dtype, void* stream);
+
 /* ---- dense skinny GEMM (replaces F.linear / torch.mm at decode sizes, utils/layers.py:110-111,
  *      lm_head utils/layers.py:261) -------------------------------------------------------------- */
 int64_t tgis_dense_prepared_bytes(int64_t N, int64_t K);

@@ -19,6 +19,7 @@ import torch
 
 from tgis_amd import native
 from tgis_amd.utils.layers import (
+    FastLinear,
     PositionRotaryEmbedding,
     TensorParallelColumnLinear,
     TensorParallelEmbedding,
@@ -300,6 +301,23 @@ class FlashLlamaModel:
             self.max_positions = max(max_s, 2 * self.max_positions, declared, 2048)
         return self.layers[0].self_attn.rotary_emb.tables(dtype, device, self.max_positions)
 
+    def forward_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
+        """A decode step of a few rows on the launches of csrc/dense_rows.hip: the residual stream (fp32, [rows, hidden]) in front of the final
+        norm.  Five launches a layer; the values are those of `forward` but for the order of the sums."""
+        h = native.embedding_scaled_f32(input_ids, self.embed_tokens.weight, 1.0)
+        cos, sin = self.rope_tables(self.embed_tokens.weight.dtype, h.device, max_s)
+        for layer in self.layers:
+            att, mlp = layer.self_attn, layer.mlp
+            qkv = native.dense_rows_rope(h, layer.input_layernorm.weight, layer.input_layernorm.variance_epsilon,
+                                         att.query_key_value.linear.rope_handle, att.query_key_value.linear.bias, cos, sin, position_ids, kv.slots,
+                                         kv.cache.k_pool(layer.layer_id), kv.cache.v_pool(layer.layer_id), att.num_heads, att.num_key_value_heads,
+                                         att.head_size)
+            native.dense_rows_residual(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv), att.o_proj.linear.prepared, h)
+            act = native.dense_rows_silu(h, layer.post_attention_layernorm.weight, layer.post_attention_layernorm.variance_epsilon,
+                                         mlp.gate_up_proj.linear.prepared)
+            native.dense_rows_residual(act, mlp.down_proj.linear.prepared, h)
+        return h
+
     def forward(self, input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv: KVArgs):
         if input_ids is not None and inputs_embeds is not None:
             raise ValueError("You cannot specify both input_ids and inputs_embeds at the same time")
@@ -319,6 +337,7 @@ class FlashLlamaForCausalLM:
         self.config = config
         self.model = FlashLlamaModel(config, weights)
         self.lm_head = TensorParallelHead.load(config, prefix="lm_head", weights=weights)
+        self._rows_path = {}
         self.gptq_linears: List = []
         for layer in self.model.layers:
             for lin in (layer.self_attn.query_key_value.linear, layer.self_attn.o_proj.linear,
@@ -338,6 +357,26 @@ class FlashLlamaForCausalLM:
             if hasattr(o_proj, "places"):
                 layer.self_attn.out_places = o_proj.places()
 
+    def rows_path(self, rows: int) -> bool:
+        """Whether a decode step of `rows` rows runs on the launches that norm their operand themselves (FlashLlamaModel.forward_rows)."""
+        got = self._rows_path.get(rows)
+        if got is None:
+            got = self._rows_path[rows] = rows <= native.DENSE_ROWS_MAX_M and self._serves_rows(rows)
+        return got
+
+    def _serves_rows(self, rows: int) -> bool:
+        cfg = self.config
+        plain = lambda lin: isinstance(lin, FastLinear) and lin.streams and lin.bias is None
+        if self.model.tp_world_size != 1 or not plain(self.lm_head.linear) or not native.dense_rows_ok(rows, cfg.hidden_size, True):
+            return False
+        for layer in self.model.layers:
+            qkv, o = layer.self_attn.query_key_value.linear, layer.self_attn.o_proj.linear
+            gate_up, down = layer.mlp.gate_up_proj.linear, layer.mlp.down_proj.linear
+            if not (isinstance(qkv, FastLinear) and qkv.rope_handle is not None and plain(o) and plain(gate_up) and gate_up.gate_up and plain(down)
+                    and native.dense_rows_ok(rows, o.in_features, False) and native.dense_rows_ok(rows, down.in_features, False)):
+                return False
+        return True
+
     def get_input_embeddings(self):
         return self.model.embed_tokens
 
@@ -348,6 +387,10 @@ class FlashLlamaForCausalLM:
     def forward(self, input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds=None, kv: KVArgs = None,
                 lm_head_indices: Optional[torch.Tensor] = None):
         """position_ids int32 [T]; returns fp32 logits [T or len(lm_head_indices), vocab]."""
+        if (kv.max_q_len == 1 and not kv.fresh_prefill and inputs_embeds is None and lm_head_indices is None and kv.slots is not None
+                and self.rows_path(input_ids.shape[0])):
+            h = self.model.forward_rows(input_ids, position_ids, cu_seqlens_q, max_s, kv)
+            return native.dense_rows_head(h, self.model.norm.weight, self.model.norm.variance_epsilon, self.lm_head.linear.prepared)
         hidden_states = self.model(input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv)
         if lm_head_indices is not None:
             hidden_states = hidden_states.index_select(0, lm_head_indices)

@@ -83,6 +83,12 @@ SIGNATURES = {
                                             _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tgis_attn_num_splits": (_c_int, [_c_i64, _c_int, _c_int, _c_i64, _c_i64]),
     "tgis_attn_workspace_bytes": (_c_i64, [_c_i64, _c_int, _c_int, _c_int, _c_int]),
+    "tgis_dense_rows_ok": (_c_int, [_c_i64, _c_i64, _c_int]),
+    "tgis_dense_rows_norm_rope": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64,
+                                           _c_i64, _c_int, _vp]),
+    "tgis_dense_rows_residual": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_rows_norm_silu": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_rows_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_attn_paged": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int,
                                  _c_int, _c_i64, _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
     "tgis_attn_paged_ordered": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int,
@@ -707,6 +713,53 @@ def dense_gemm_rope(x: torch.Tensor, w: DenseWeight, bias, cos, sin, positions, 
                                             _ptr(cos), _ptr(sin), _ptr(out), out.stride(0), _ptr(k_pool), _ptr(v_pool), M,
                                             w.K, w.N, H, Hkv, D, dtype_code(w.dtype), _stream()),
         "tgis_dense_gemm_rope")
+    return out
+
+
+DENSE_ROWS_MAX_M = 4
+
+
+def dense_rows_ok(M: int, K: int, norm: bool) -> bool:
+    return bool(load_library().tgis_dense_rows_ok(M, K, int(norm)))
+
+
+def _rows_stream(h: torch.Tensor, width: int):
+    assert h.dim() == 2 and h.shape[1] == width and h.dtype == torch.float32 and h.is_contiguous()
+    return _ptr(h)
+
+
+def dense_rows_rope(h, norm_w, eps: float, w: DenseWeight, bias, cos, sin, positions, slots, k_pool, v_pool, H: int, Hkv: int, D: int) -> torch.Tensor:
+    """dense_gemm_rope of the normed fp32 stream h [M, K], M <= DENSE_ROWS_MAX_M."""
+    assert w.flags & 2 and w.N == (H + 2 * Hkv) * D and cos.dtype == w.dtype and cos.shape[1] * 2 == D and norm_w.dtype == w.dtype
+    assert positions.dtype == torch.int32 and slots.dtype == torch.int32
+    M = h.shape[0]
+    out = torch.empty((M, w.N), dtype=w.dtype, device=h.device)
+    _check(load_library().tgis_dense_rows_norm_rope(
+        _rows_stream(h, w.K), _ptr(norm_w), float(eps), _ptr(w.image), _ptr(bias), _ptr(positions), _ptr(slots), _ptr(cos), _ptr(sin), _ptr(out),
+        out.stride(0), _ptr(k_pool), _ptr(v_pool), M, w.K, H, Hkv, D, dtype_code(w.dtype), _stream()), "tgis_dense_rows_norm_rope")
+    return out
+
+
+def dense_rows_residual(x, w: DenseWeight, h) -> None:
+    """h += x @ w^T, the product and the stream rounded to the model dtype first (what a fused add + norm behind the product adds)."""
+    assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K and not w.flags and h.shape[0] == x.shape[0]
+    _check(load_library().tgis_dense_rows_residual(_ptr(x), x.stride(0), _ptr(w.image), _rows_stream(h, w.N), x.shape[0], w.K, w.N,
+                                                   dtype_code(w.dtype), _stream()), "tgis_dense_rows_residual")
+
+
+def dense_rows_silu(h, norm_w, eps: float, w: DenseWeight) -> torch.Tensor:
+    assert w.flags & 1 and norm_w.dtype == w.dtype
+    out = torch.empty((h.shape[0], w.N // 2), dtype=w.dtype, device=h.device)
+    _check(load_library().tgis_dense_rows_norm_silu(_rows_stream(h, w.K), _ptr(norm_w), float(eps), _ptr(w.image), _ptr(out), out.stride(0),
+                                                    h.shape[0], w.K, w.N, dtype_code(w.dtype), _stream()), "tgis_dense_rows_norm_silu")
+    return out
+
+
+def dense_rows_head(h, norm_w, eps: float, w: DenseWeight) -> torch.Tensor:
+    assert not w.flags and norm_w.dtype == w.dtype
+    out = torch.empty((h.shape[0], w.N), dtype=torch.float32, device=h.device)
+    _check(load_library().tgis_dense_rows_norm_head(_rows_stream(h, w.K), _ptr(norm_w), float(eps), _ptr(w.image), _ptr(out), out.stride(0),
+                                                    h.shape[0], w.K, w.N, dtype_code(w.dtype), _stream()), "tgis_dense_rows_norm_head")
     return out
 
 
