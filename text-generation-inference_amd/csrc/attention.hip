@@ -37,13 +37,12 @@
 
 namespace {
 
-// Eight neighbouring output columns, k0 .. k0 + 7 of token tok.  With out_cols they go to the places that the act-order matrix behind the
+// Eight neighbouring output columns, k0 .. k0 + 7 of token tok's K.  With out_cols they go to the places that the act-order matrix behind the
 // launch wants them in, by two-byte stores all over a row: the lines that several XCDs write in parts cost 2.4 us a launch (11 rows of 4096),
 // the gather launch that they replace 4.7 (7B, 11 ragged sequences, the whole step: 2638 -> 2562 us; asking for the places in front of the
 // waves' meeting changes nothing).
 template <typename T>
-__device__ __forceinline__ void store_out(const AttnArgs& a, int64_t tok, int k0, typename VecT<T>::x8 v) {
-    const int64_t K = a.ld_out;  // H * D
+__device__ __forceinline__ void store_out(const AttnArgs& a, int64_t tok, int k0, int64_t K, typename VecT<T>::x8 v) {
     T* out = reinterpret_cast<T*>(a.out);
     if (a.out_cols) {
         int to[8];
@@ -360,7 +359,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
             V8 ov;
 #pragma unroll
             for (int e = 0; e < 8; ++e) ov[e] = from_f32<T>(acc[e] * inv);
-            store_out<T>(a, tokidx, headj * D + dc * 8, ov);
+            store_out<T>(a, tokidx, headj * D + dc * 8, (int64_t)a.H * D, ov);
         } else if (a.counters) {
             // fused combine: the record leaves as 16-byte write-through stores (no other block's record shares a
             // 128-byte line with it: 16 columns x NS x 16 bytes per (group, chunk))
@@ -475,7 +474,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
             for (int e = 0; e < 8; ++e) ov[e] = from_f32<T>(acc[it][e] * inv);
             const int64_t tokidx = q0 + t0 + tqj;
             const int headj = hk * a.G + (hc0 + ch) * 16 + gj;
-            store_out<T>(a, tokidx, headj * D + dcs[it] * 8, ov);
+            store_out<T>(a, tokidx, headj * D + dcs[it] * 8, (int64_t)a.H * D, ov);
         }
     }
 }
