@@ -122,7 +122,8 @@ class FlashMQAttention:
                                      hidden_size=config.hidden_size, num_heads=self.num_heads)
         self.c_proj = load_row(config, prefix=f"{prefix}.c_proj", weights=weights, bias=True)
 
-    def forward(self, hidden_states, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs):
+    def forward(self, hidden_states, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, ends_step: Optional[KVArgs] = None):
+        """ends_step: go on with the rows `kv.ends` alone behind the cache write, as this step."""
         H, D = self.num_heads, self.head_size
         # [T, (H + 2) D]: H query heads, then the single k and v heads; at decode sizes the split-K sum is left to
         # the cache-write kernel below (native.Partial)
@@ -133,6 +134,8 @@ class FlashMQAttention:
                                                kv.max_q_len, H, 1, D, D)  # no rotary: page-wise cache write only
         else:
             qkv = native.rope_kv_write(qkv, None, None, None, kv.slots, k_pool, v_pool, H, 1, D, D)  # no rotary
+        if ends_step is not None:
+            qkv, kv, cu_seqlens_q = qkv.index_select(0, kv.ends), ends_step, ends_step.cu_seqlens_q
         T = qkv.shape[0]
         attn_output = torch.empty((T, H * D), dtype=qkv.dtype, device=qkv.device)
         ws = None
@@ -175,9 +178,11 @@ class Block:
         self.attn = FlashMQAttention(prefix=f"{prefix}.attn", config=config, weights=weights)
         self.mlp = MLP(prefix=f"{prefix}.mlp", config=config, weights=weights)
 
-    def forward(self, hidden_states, residual, position_ids, cu_seqlens_q, kv: KVArgs):
+    def forward(self, hidden_states, residual, position_ids, cu_seqlens_q, kv: KVArgs, ends_step: Optional[KVArgs] = None):
         hidden_states, residual = self.ln_1(hidden_states, residual)
-        hidden_states = self.attn(hidden_states, position_ids, cu_seqlens_q, self.layer_id, kv)
+        hidden_states = self.attn(hidden_states, position_ids, cu_seqlens_q, self.layer_id, kv, ends_step)
+        if ends_step is not None:
+            residual = residual.index_select(0, kv.ends)
         hidden_states, residual = self.ln_2(hidden_states, residual)
         return self.mlp(hidden_states), residual
 
@@ -208,8 +213,10 @@ class FlashSantacoderModel:
             # bound now: a replayed seam must keep reducing THIS tensor, not whatever `hidden_states` names later
             collective(lambda t=hidden_states: torch.distributed.all_reduce(t, group=pg))
         residual = None
-        for layer in self.h:
-            hidden_states, residual = layer(hidden_states, residual, position_ids, cu_seqlens_q, kv)
+        # the last layer of a prefill of which only the last tokens' logits are wanted
+        ends_step = kv.at_ends(self.num_heads, 1) if kv.cuts_to_ends(hidden_states.shape[0]) else None
+        for i, layer in enumerate(self.h):
+            hidden_states, residual = layer(hidden_states, residual, position_ids, cu_seqlens_q, kv, ends_step if i + 1 == len(self.h) else None)
         hidden_states, _ = self.ln_f(hidden_states, residual)
         return hidden_states
 
@@ -242,7 +249,7 @@ class FlashSantacoderForCausalLM:
     def forward(self, input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds=None, kv: KVArgs = None,
                 lm_head_indices: Optional[torch.Tensor] = None):
         hidden_states = self.transformer(input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv)
-        if lm_head_indices is not None:
+        if lm_head_indices is not None and not kv.cuts_to_ends(position_ids.shape[0]):
             hidden_states = hidden_states.index_select(0, lm_head_indices)
         return self.lm_head(hidden_states)
 

@@ -708,12 +708,12 @@ class FlashCausalLM(Model):
 
     def ragged_forward(self, input_ids: torch.Tensor, pages: List[List[int]], cached: List[int], new_lens: List[int],
                        state_slots: Optional[List[int]] = None, block_tables: Optional[torch.Tensor] = None,
-                       lm_head_indices: Optional[torch.Tensor] = None, inputs_embeds=None, residual_trace=None):
+                       lm_head_indices: Optional[torch.Tensor] = None, inputs_embeds=None, residual_trace=None, ends_only: bool = False):
         """THE step function: one forward over sequences that already hold `cached[i]` tokens in their pages (and state
         slot) and bring `new_lens[i]` more, concatenated in `input_ids`.  A whole-prompt prefill is cached = 0 everywhere, a
         decode step is new_lens = 1 everywhere; anything between (portions of prompts beside decoded tokens) needs a model
         that supports ragged steps.  Pages for positions < cached + new must be owned already.  Returns fp32 logits of every
-        token, or of `lm_head_indices`."""
+        token, or of `lm_head_indices` (ends_only: those are every sequence's last token, in order)."""
         dev = self.device
         fresh = not any(cached)
         if not fresh and not self.supports_ragged_steps:
@@ -739,7 +739,7 @@ class FlashCausalLM(Model):
             block_tables = there[-1]
         kv = KVArgs(cache=self.kv_cache, block_tables=block_tables, ctx_lens=ctx_t, slots=slots_t,
                     max_q_len=max(new_lens), max_ctx=max(ctx), num_splits=1, fresh_prefill=fresh and FRESH_PREFILL_KV,
-                    state=self.state_cache, cu_seqlens_q=cu_t, residual_trace=residual_trace,
+                    state=self.state_cache, cu_seqlens_q=cu_t, residual_trace=residual_trace, ends=lm_head_indices if ends_only else None,
                     state_slots=there[4] if state_slots is not None else None)
         return self.model.forward(input_ids, position_ids, cu_t, max(ctx), inputs_embeds, kv, lm_head_indices)
 
@@ -787,7 +787,7 @@ class FlashCausalLM(Model):
         chunk = self.prefill_chunk if self.supports_ragged_steps and not self._need_all_logits else 0
         if chunk <= 0 or max(lens) <= chunk or batch.inputs_embeds is not None:
             return self.ragged_forward(batch.input_ids, batch.pages, [0] * len(lens), lens, batch.state_slots,
-                                       batch.block_tables, lm_head_indices, batch.inputs_embeds)
+                                       batch.block_tables, lm_head_indices, batch.inputs_embeds, ends_only=lm_head_indices is not None)
         # portions: every sequence advances by up to `chunk` tokens per forward; finished ones drop out of later forwards.
         # Logits are taken where a sequence's last token is.
         starts = batch.cu_seqlens[:-1].tolist()

@@ -104,16 +104,21 @@ class NormedQKAttention:
         """The value columns of a projected step (what another layer blends with)."""
         return qkv[:, (self.H + self.G) * self.dk:]
 
-    def forward(self, h: torch.Tensor, position_ids, step, v_other: Optional[torch.Tensor] = None):
-        """h [T, W] -> (out [T, W], qkv [T, H dk + G dk + G dv] with q normed in place)."""
+    def forward(self, h: torch.Tensor, position_ids, step, v_other: Optional[torch.Tensor] = None, ends: Optional[torch.Tensor] = None):
+        """h [T, W] -> (out [T, W], qkv [T, H dk + G dk + G dv] with q normed in place).  ends: out for these rows alone, each the last token of a
+        sequence of the step."""
         qkv = self.qkv(h)
         cache = step.cache
         k_pool, v_pool = cache.k_pool(self.layer_id), cache.v_pool(self.layer_id)
         native.qk_norm_kv_write(qkv, position_ids, step.slots, self.q_gain, self.k_gain, self.eps, self.gain_coef,
                                 self.gain_every, v_other if self.v_lambda is not None else None, self.v_lambda, k_pool, v_pool,
                                 self.H, self.G, self.dk, self.dv)
-        att = native.attn_varlen(qkv, k_pool, v_pool, step.block_tables, step.ctx_lens, step.cu_seqlens_q, self.H, self.G,
-                                 self.dk, self.dv, self.scale, max_q_len=step.max_q_len, max_ctx=step.max_ctx)
+        q, cu_q, longest = qkv, step.cu_seqlens_q, step.max_q_len
+        if ends is not None:
+            q, longest = qkv.index_select(0, ends), 1
+            cu_q = torch.arange(ends.shape[0] + 1, dtype=torch.int32, device=ends.device)
+        att = native.attn_varlen(q, k_pool, v_pool, step.block_tables, step.ctx_lens, cu_q, self.H, self.G,
+                                 self.dk, self.dv, self.scale, max_q_len=longest, max_ctx=step.max_ctx)
         return self.o(att, partial=self.defer), qkv
 
 
@@ -141,8 +146,8 @@ class WkvMixer:
         self.o = load_linear(weights, f"{prefix}.o")
         self.defer = can_defer(self.o)
 
-    def forward(self, h32: torch.Tensor, position_ids, step, dtype):
-        """h32 [T, W] fp32 (the normed mixer input, kept in fp32 because it is also the shift state)."""
+    def forward(self, h32: torch.Tensor, position_ids, step, dtype, ends: Optional[torch.Tensor] = None):
+        """h32 [T, W] fp32 (the normed mixer input, kept in fp32 because it is also the shift state).  ends: the output of these rows alone."""
         st = step.state
         state, shift = st.state[self.layer_id], st.shift[self.layer_id]
         mixes = native.token_shift_mix(h32, shift, step.state_slots, step.cu_seqlens_q, position_ids, self.mu, dtype)
@@ -163,7 +168,7 @@ class WkvMixer:
         logw = native.wkv_decay(low, self.w2t, self.w0)
         out = native.wkv_scan(rkvg[0], rkvg[1], rkvg[2], rkvg[3], logw, self.u, self.gain, state, shift, h32, step.state_slots,
                               step.cu_seqlens_q, position_ids, self.H, self.d, self.eps, max_q_len=step.max_q_len)
-        return self.o(out, partial=self.defer)
+        return self.o(out if ends is None else out.index_select(0, ends), partial=self.defer)
 
 
 class GatedUnit:
