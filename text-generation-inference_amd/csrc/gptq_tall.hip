@@ -12,10 +12,9 @@
 // pipelined: while slice i is multiplied, slice i + 1 is dequantised and its A fragments are read.
 //
 // Bound: the matrix cores, which this card's power holds to about 1.5 PFLOP/s on random data whatever feeds them (a bare MFMA loop), and
-// the dequantisation's share of that power.  A 128 x 256 tile of 4096 k takes 51 us alone on a CU, 65 on a full chip (1.05 PFLOP/s; 68
-// and 65 when x went through registers, every fragment was read where it was needed and a chunk of 128 k had one barrier); several
-// blocks on a CU only share its matrix cores, so that the plan below weighs whole rounds of 256 CUs.  7B layer, 765 rows: qkv 112 -> 81,
-// o 51 -> 35, gate_up 202 -> 144, down 110 -> 82 us.
+// the dequantisation's share of that power.  A 128 x 256 tile of 4096 k takes 45 us alone on a CU, 56 on a full chip (1.2 PFLOP/s); several
+// blocks on a CU only share its matrix cores, so that the plan below weighs whole rounds of 256 CUs.  7B layer, 765 rows: qkv 79 -> 77,
+// o 36 -> 32, gate_up 145 -> 138, down 81 -> 74 us with the loop in whole turns of its ring (below); 300 rows 41 -> 38, 28 -> 23, 72, 45 -> 42.
 #include <stdlib.h>
 #include <algorithm>
 #include <type_traits>
@@ -174,15 +173,22 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    for (int s = 0;;) {
-        step(s, std::integral_constant<int, 0>{});
-        if (++s == n) break;
-        step(s, std::integral_constant<int, 1>{});
-        if (++s == n) break;
-        step(s, std::integral_constant<int, 2>{});
-        if (++s == n) break;
-        step(s, std::integral_constant<int, 3>{});
-        if (++s == n) break;
+    // whole turns of the ring, then what is left: with a way out behind every step the compiler sees ways back to the first one from each of
+    // them, and waits there for every load there is
+    using std::integral_constant;
+    int s = 0;
+    for (; s + TALL_RING <= n; s += TALL_RING) {
+        step(s, integral_constant<int, 0>{});
+        step(s + 1, integral_constant<int, 1>{});
+        step(s + 2, integral_constant<int, 2>{});
+        step(s + 3, integral_constant<int, 3>{});
+    }
+    if (s < n) {
+        step(s, integral_constant<int, 0>{});
+        if (s + 1 < n) {
+            step(s + 1, integral_constant<int, 1>{});
+            if (s + 2 < n) step(s + 2, integral_constant<int, 2>{});
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
 
@@ -295,12 +301,12 @@ struct TallPlan {
 };
 
 // us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip (several blocks on each; clocks drop under
-// the matrix cores' load).  Fitted to launches of 26 - 560 us at the 7B shapes, 260 - 3072 rows; the plans the model picks are within 8 %
-// of the best of the nine that were timed at each size.
+// the matrix cores' load).  Fitted to launches of 23 - 400 us at the 7B shapes; over nine matrices and ten row counts from 140 to 3000 the
+// plans that the model picks are 0.6 % behind the best of up to 24 that were timed at each size.
 struct TallCost {
     double alone, busy;
 };
-constexpr TallCost TALL_COST[3][2] = {{{0.39, 0.314}, {0.53, 0.64}}, {{0.45, 0.434}, {0.625, 0.82}}, {{0.50, 0.57}, {0.735, 0.99}}};
+constexpr TallCost TALL_COST[3][2] = {{{0.33, 0.286}, {0.42, 0.50}}, {{0.41, 0.367}, {0.52, 0.70}}, {{0.45, 0.472}, {0.63, 0.85}}};
 
 // Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k.  One size does not do: 765 rows of
 // a 7B gate_up are 516 tiles of 128 x 256, two rounds and four tiles, which take a third round (187 us; 161 with the four split in
@@ -410,9 +416,9 @@ TallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, 
 
 }  // namespace
 
-// Rows from which it may replace the 64-row streaming passes, and up to which it replaces dequantise + library GEMM:
-// (library with its dequantisation / tall, us, the four GEMMs of a 7B layer) 3072 rows 1296 / 1159, 6000 rows 2418 / 2184, 8192 rows
-// 2979 / 2993, 16128 rows 5542 / 5947: past 8192 rows hipBLASLt's 256 x 256 tiles, free of dequantisation, win (1.28 against 1.13 PFLOP/s).
+// Rows from which it may replace the 64-row streaming passes, and up to which it replaces dequantise + library GEMM: (library with its
+// dequantisation / tall, us, the four GEMMs of a 7B layer) 4096 rows 1547 / 1400, 6000 rows 2288 / 2121, 8192 rows 2829 / 2851; at 16128 rows
+// hipBLASLt's 256 x 256 tiles, free of dequantisation, run at 1.35 PFLOP/s against 1.12 - 1.25.
 int64_t gptq::tall_min_m(int act) {
     static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 0;
     return v ? v : act == 2 ? 65 : 129;
@@ -428,15 +434,15 @@ bool gptq::tall_serves(int64_t K, int64_t groups, bool act_order, int act) {
 }
 // Between 3072 and tall_max_m() rows it depends on how full the library's 256 x 256 tiles leave their rounds of 256.  act 0, us, dequantise
 // and library / this kernel, weights cold:
-//   93 % full and more:  4096 x 12288 at 4096, 8000, 8192 rows 357 / 364, 674 / 720, 676 / 731; 11008 x 4096 at 4096, 8192 312 / 324, 588 / 641;
-//                        5120 x 15360 at 5000, 6000, 8192 672 / 757, 809 / 876, 1065 / 1188; 8192 x 3072 at 5000 222 / 239
-//   less:                4096 x 12288 at 6000, 7168 610 / 537, 647 / 641; 11008 x 4096 at 7168 728 / 581; 8192 x 10240 at 4096, 5000 737 / 608, 801 /
-//                        755; 13824 x 5120 at 4096, 5000, 6000 588 / 542, 836 / 664, 939 / 774
-//   one round, from three fifths on, of long k:  5632 x 2048 at 5000, 6000, 7168 114 / 134, 130 / 136, 151 / 163; 8192 x 3072 at 4096 193 / 215
-//                        (4096 x 4096 at 3500 120 / 118; 5632 x 2048 at 4096, half a round, 99 / 98)
-// Over 17 shapes and 14 row counts this choice is 0.7 % behind the better of the two, either one alone 2.7 % (this kernel) or 5.9 %.
-// With SiLU * up this kernel is within 5 % of the library and its activation launch, or in front (4096 x 22016 at 4096, 8192 rows 794 / 726, 1416 /
-// 1467; 2048 x 11264 209 / 192, 447 / 359).
+//   93 % full and more:  5120 x 15360 at 5000, 6000, 8192 655 / 681, 785 / 804, 1043 / 1096; 11008 x 4096 at 4096, 8192 298 / 300, 561 / 590; 8192 x
+//                        10240 at 6000, 8192 822 / 834, 1060 / 1093; 5120 x 15360 at 4096 543 / 540 (but 4096 x 12288 at 4096 367 / 342, 13824 x
+//                        5120 at 6000 926 / 707)
+//   less:                4096 x 12288 at 6000, 7168 609 / 499, 637 / 596; 11008 x 4096 at 7168 732 / 545; 8192 x 10240 at 4096, 5000 744 / 550, 778 /
+//                        704; 13824 x 5120 at 4096, 5000 574 / 491, 838 / 600
+//   one round, from three fifths on, of long k:  5632 x 2048 at 5000, 7168 111 / 112, 143 / 146; 8192 x 3072 at 4096, 5000 183 / 197, 210 / 216
+//                        (4096 x 4096 at 3500 109 / 106; 5632 x 2048 at 4096, half a round, 97 / 87)
+// With SiLU * up this kernel is in front of the library and its activation launch (4096 x 22016 at 4096, 8192 rows 764 / 641, 1389 / 1365; 2048 x
+// 11264 198 / 178, 421 / 333).
 bool gptq::tall_before_library(int64_t M, int64_t K, int64_t N, int act) {
     if (M <= 3072 || act == 2 || getenv("TGIS_TALL_MAX_M")) return M <= tall_max_m();
     const int64_t tiles = cdiv64(M, 256) * cdiv64(N, 256), slots = cdiv64(tiles, CUS) * CUS;
@@ -445,12 +451,14 @@ bool gptq::tall_before_library(int64_t M, int64_t K, int64_t N, int act) {
 }
 // Up to 256 rows the passes take k in parallel (k-parts, splits) where a tile here walks it alone, so it depends on the matrix which of
 // the two is done first.  us, the passes with the launch that adds their slabs / this kernel with a norm behind it (act 2: either alone):
-//   act 0:  2048 x 2560 at 129 / 256 rows 12.1 / 19.4, 15.4 / 19.7; 1024 x 1024 8.1 / 10.5, 8.7 / 11.3; 3072 x 5120 19.9 / 26.1, 32.7 /
-//           26.8; 4096 x 4096 21.9 / 20.6, 23.5 / 25.5; 2048 x 6144 25.1 / 20.0, 26.7 / 20.9; 4096 x 12288 50.4 / 39.6, 51.1 / 44.8;
-//           11008 x 4096 44.1 / 33.1, 45.9 / 38.4; 8192 x 10240 49.6 / 49.4, 87.1 / 59.5
-//   act 2:  2048 x 11264 at 65 / 128 / 129 rows 14.2 / 16.4, 14.3 / 16.7, 24.7 / 20.2; 4096 x 22016 48.3 / 35.8, 47.1 / 40.5, 67.7 / 48.1
-// The passes' time is that of their rounds of 256 blocks, each its chunks of 256 k per k-part (fitted to 30 shapes, within 8 %); the
-// choice is the faster one, or within 2 % of it, at all of these but 1024 x 8192 and 4096 x 2752, where it keeps the passes (up to 1.26).
+//   act 0:  2048 x 2560 at 129 / 256 rows 16.2 / 17.3, 16.7 / 17.2; 3072 x 5120 21.0 / 23.5, 34.4 / 24.6; 4096 x 4096 23.2 / 20.8, 24.7 /
+//           27.8; 2048 x 6144 25.5 / 18.3, 27.5 / 19.4; 4096 x 12288 51.8 / 37.5, 52.4 / 42.4; 11008 x 4096 44.5 / 30.9, 46.6 / 36.9; 8192 x
+//           10240 49.1 / 45.5, 88.9 / 56.2; 28672 x 8192 146 / 98, 162 / 126
+//   act 2:  2048 x 11264 at 65 / 128 / 129 / 256 rows 15.1 / 15.8, 15.1 / 13.7, 26.1 / 17.7, 28.3 / 19.7; 4096 x 22016 45.5 / 31.0, 46.7 / 34.9,
+//           67.5 / 44.9, 74.0 / 55.7; 8192 x 57344 185 / 92, 185 / 121, 272 / 177, 348 / 225; 1024 x 8192 11.9 / 11.4, 13.6 / 9.2, 10.7 / 8.7, 11.3 / 9.0
+// The passes' time is that of their rounds of 256 blocks, each its chunks of 256 k per k-part (fitted to 30 shapes, within 8 %); of the 63
+// (matrix, rows) that were timed three go the slower way by more than 7 %, by up to 2.4 us (4096 x 4096 at 129
+// rows; 2048 x 11264 with SiLU at 96 and 128).
 static bool pays_below_257_rows(int64_t M, int64_t K, int64_t N, int act) {
     const gptq::GemmPlan pass = gptq::plan_gemm(K, N, act, M);
     const double rounds = (double)cdiv64(cdiv64(cdiv64(N, 32), pass.TN) * cdiv64(M, 64) * pass.S, CUS), chunks = pass.KR / 256 / pass.WK;
@@ -458,7 +466,7 @@ static bool pays_below_257_rows(int64_t M, int64_t K, int64_t N, int act) {
                                    : 5.0 + rounds * (3.0 + chunks * (pass.TN == 4 ? 2.45 : 1.65));
     const TallPlan p = plan_tall(M, K, N);
     const bool split = p.whole < p.tiles;  // (the model is 4 us above split plans)
-    return (split ? p.us - (act == 2 ? 4.0 : 3.5) : act == 2 ? p.us + 1.0 : 1.1 * p.us + 2.0) <= passes;
+    return (split ? p.us - (act == 2 ? 4.0 : 3.5) : act == 2 ? 1.1 * p.us - 1.0 : 1.1 * p.us + 1.0) <= passes;
 }
 bool gptq::tall_ok(int64_t M, int64_t K, int64_t N, int64_t groups, bool act_order, int act) {
     if (M < tall_min_m(act) || !tall_serves(K, groups, act_order, act)) return false;
