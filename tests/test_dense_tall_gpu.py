@@ -1,0 +1,117 @@
+"""The dense GEMM of prefills on the prepared image (tgis_dense_tall) against the float64 product: every tile, whole and split over k, at the
+edges of its rows and columns; and the projections that choose it, on both sides of the rule."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}  # half a step of the dtype, of a value's size
+
+
+def _case(M, K, N, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype)
+    bias = torch.randn(N, generator=g).to(dtype)
+    z = x.double() @ w.double().t() + bias.double()
+    # fp32 sums of K products in any order: K half-steps of 2^-24 of the sum of magnitudes
+    acc = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + bias.double().abs())
+    return x, w, bias, z, acc
+
+
+def _expect(z, acc, dtype, act):
+    """(value, bound): the sum may round to either neighbour (2 half-steps), the activation then moves by its slope (at most 1.13) times
+    that, and every rounding behind it adds a half-step (a step where the intermediate is rounded too)."""
+    u = ULP[dtype]
+    r = z.to(dtype).double()
+    dz = 2 * u * r.abs() + acc + 2.0 ** -24
+    if act == 0:
+        return r, dz
+    if act in (4, 5):
+        return torch.nn.functional.gelu(r, approximate="tanh" if act == 5 else "none"), 1.13 * dz + 2 * u * r.abs() + 2.0 ** -24
+    h = z.shape[1] // 2
+    gate, up, dg, du = r[:, :h], r[:, h:], dz[:, :h], dz[:, h:]
+    if act == 2:
+        s = gate * torch.sigmoid(gate)
+        return s * up, 1.1 * dg * up.abs() + s.abs() * du + 4 * u * (s * up).abs() + 2.0 ** -24
+    gc, uc = gate.clamp(max=3.0), up.clamp(-3.0, 3.0)
+    s = gc * torch.sigmoid(1.7 * gc)
+    return s * (uc + 1), 1.1 * dg * (uc + 1).abs() + s.abs() * du + 4 * u * (s * (uc + 1)).abs() + 2.0 ** -24
+
+
+def _check(out, want):
+    value, bound = want
+    off = (out.double().cpu() - value).abs() - bound
+    assert out.shape == value.shape and bool((off <= 0).all()), float(off.max())
+
+
+def _run(M, K, N, dtype, act, plan, monkeypatch, ld_out=None):
+    from tgis_amd import native
+
+    if plan:
+        monkeypatch.setenv("TGIS_DTALL_PLAN", plan)
+    x, w, bias, z, acc = _case(M, K, N, dtype)
+    clamped = act == 3
+    image = native.DenseWeight(w.cuda(), gate_up=act in (2, 3))
+    ws = native.Workspace(64 << 20, torch.device("cuda"))
+    n_out = N // 2 if act in (2, 3) else N
+    out = torch.full((M, ld_out or n_out), 7.0, dtype=dtype, device="cuda")
+    native.dense_tall(x.cuda(), image, ws, bias=bias.cuda(), act=2 if clamped else act, alpha=1.7, limit=3.0 if clamped else 0.0, out=out[:, :n_out])
+    _check(out[:, :n_out], _expect(z, acc, dtype, act))
+    assert bool((out[:, n_out:] == 7.0).all())
+
+
+# tiles of 64 / 96 / 128 x 128 / 256, whole and in 2 and 3 parts; rows and columns one short of, at and past a tile; every remainder of the ring
+@pytest.mark.parametrize("plan,M,K,N", [
+    ("2,1,1", 65, 64, 128), ("2,1,2", 64, 320, 136), ("2,2,1", 129, 128, 257), ("2,2,3", 63, 1152, 520),
+    ("3,1,1", 96, 192, 100), ("3,1,3", 97, 640, 129), ("3,2,2", 191, 448, 256), ("3,2,1", 290, 256, 31),
+    ("4,1,1", 128, 384, 384), ("4,1,2", 127, 1088, 640), ("4,2,1", 257, 448, 300), ("4,2,3", 130, 896, 512),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_plain(plan, M, K, N, dtype, monkeypatch):
+    _run(M, K, N, dtype, 0, plan, monkeypatch, ld_out=N + 8 if M % 2 else None)
+
+
+@pytest.mark.parametrize("plan", ["2,1,1", "2,2,2", "3,1,3", "3,2,1", "4,1,2", "4,2,1"])
+@pytest.mark.parametrize("act", [2, 3, 4, 5])
+def test_activations(plan, act, monkeypatch):
+    for dtype, M, K, N in ((torch.bfloat16, 131, 576, 352), (torch.float16, 98, 320, 544)):
+        _run(M, K, N, dtype, act, plan, monkeypatch)
+
+
+def test_chosen_plans(monkeypatch):
+    # more than a round of 256 tiles with a split rest; several groups of row blocks; a narrow product
+    for M, K, N, act in ((1100, 1024, 5632, 2), (2100, 256, 4224, 2), (700, 512, 64, 0), (300, 6144, 1024, 0)):
+        _run(M, K, N, torch.bfloat16, act, None, monkeypatch)
+
+
+@pytest.mark.parametrize("M,N", [(64, 1024), (65, 1024), (256, 1024), (257, 1024), (257, 992), (300, 2048), (501, 2048)])
+def test_linear_on_both_sides(M, N):
+    from tgis_amd.utils.layers import FastLinear
+
+    K = 512
+    x, w, bias, z, acc = _case(M, K, N, torch.float16, seed=3)
+    lin = FastLinear(w.cuda(), bias.cuda())
+    _check(lin(x.cuda()), _expect(z, acc, torch.float16, 0))
+    _check(lin(x.cuda(), gelu=True), _expect(z, acc, torch.float16, 5))
+    plain = FastLinear(w.cuda(), None)
+    out = torch.empty(M, N, dtype=torch.float16, device="cuda")
+    plain(x.cuda(), out=out)
+    _check(out, _expect(z - bias.double(), acc, torch.float16, 0))
+    lin.gate_up = True
+    _check(lin(x.cuda()), _expect(z, acc, torch.float16, 2))
+
+
+@pytest.mark.parametrize("pad,first", [(1, 0), (8, 1), (4, 0)])
+def test_rows_it_cannot_read(pad, first):
+    """Rows that are not 16-byte aligned go where they went: to the library."""
+    from tgis_amd import native
+    from tgis_amd.utils.layers import FastLinear
+
+    x, w, bias, z, acc = _case(300, 512, 1024, torch.float16, seed=4)
+    wide = torch.zeros(300, 512 + pad, dtype=torch.float16, device="cuda")
+    view = wide[:, first:first + 512]
+    view.copy_(x)
+    lin = FastLinear(w.cuda(), bias.cuda())
+    assert not native.dense_tall_pays(view, lin.prepared) and native.dense_tall_pays(x.cuda(), lin.prepared)
+    _check(lin(view), _expect(z, acc, torch.float16, 0))

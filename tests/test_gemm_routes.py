@@ -56,3 +56,23 @@ def test_int4_library(M, K, N, act, pays):
     assert lib.tgis_gptq_gemm_fused_pays(M, K, N, K // 64, 0, act) == pays
     assert lib.tgis_gptq_gemm_fused_pays(M, K, N, K // 64, 1, act) == 0          # act-order: up to 256 rows alone
     assert lib.tgis_gptq_gemm_fused_pays(256, K, N, K // 64, 1, act) == 1
+
+
+# the dense prefill kernel: from 65 rows on, past 256 where the library's tiles would leave the chip idle or an activation launch is saved
+@pytest.mark.parametrize("M,K,N,act,pays", [
+    (64, 2048, 2048, 0, 0), (65, 2048, 2048, 0, 1), (256, 6144, 24576, 4, 1), (257, 6144, 24576, 4, 0), (1400, 2048, 2048, 0, 1), (1401, 2048, 2048, 0, 0),
+    (500, 2048, 6144, 0, 1), (501, 2048, 6144, 0, 0), (100, 2040, 2048, 0, 0), (100, 2048, 1024, 0, 1), (100, 2048, 1023, 0, 0), (300, 448, 2048, 0, 0), (200, 64, 2048, 0, 1), (512, 4096, 22016, 2, 0), (513, 4096, 22016, 2, 1), (300, 2048, 11264, 2, 1),
+    (8192, 2048, 11264, 2, 1), (8193, 2048, 11264, 2, 0), (100, 2048, 2048, 1, 0), (0, 2048, 2048, 0, 0),
+])
+def test_dense_tall(M, K, N, act, pays):
+    from tgis_amd import native
+
+    assert (native.load_library().tgis_dense_tall_bytes(M, K, N, act) >= 0) == bool(pays)
+
+
+def test_dense_tall_scratch():
+    """Its scratch fits the workspace that projections share, which captured graphs hold the address of."""
+    from tgis_amd import native
+
+    lib = native.load_library()
+    assert max(lib.tgis_dense_tall_bytes(M, K, N, 2) for M in range(65, 1500, 61) for K in (64, 1024, 5632, 24576) for N in (1024, 2048, 6400, 22016)) <= 48 << 20

@@ -1,0 +1,451 @@
+// The dense (f16 / bf16) GEMM of prefills, on the image that the weight-streaming kernel of decode steps reads (tgis_dense_prepare): more rows
+// than that one takes in a pass, and the products for which a library's 256 x 256 tiles leave most of the chip idle or need a launch of
+// their own for the activation.
+//
+// A block of 4 waves owns a tile of 64, 96 or 128 rows x 128 or 256 columns; wave w its columns, TW tiles of 32, whose fragments it loads
+// straight from the image into registers, WR k64-steps ahead: no other wave reads them, so they need no LDS.  x, which all four read, goes to
+// LDS with direct loads, a ring of four k64-steps of 128-byte rows whose 16-byte pieces are permuted (piece ^ row mod 8) so that the fragment
+// reads fill all banks.  One barrier a step; while slice i is multiplied the A fragments of slice i + 1 are read.
+//
+// Bound: the matrix cores from about 1000 rows on (1.05 - 1.2 PFLOP/s), before that the weights' way from HBM and the latency of the blocks'
+// serial chains: hence the choice of tiles, and the split of a last round's tiles over k (plan_tall).  Tiles are walked in groups of 8 row
+// blocks, each XCD its own run of them, so that its L2 serves a tile of weights to 8 blocks: with columns fastest over the whole chip 4096 x
+// 22016 at 4096 rows took 844 us, so 627.
+#include <stdio.h>
+#include <stdlib.h>
+#include <algorithm>
+#include <type_traits>
+#include "common.h"
+#include "dense_gemm_body.h"
+
+namespace {
+
+struct DTallArgs {
+    const void* x;
+    int64_t ldx;
+    const uint8_t* prep;
+    const void* bias;
+    void* out;
+    int64_t ldo;
+    int M, K, N, NT;
+    int gelu;                    // act 0: as DenseArgs::gelu (0, 1, 2)
+    float glu_alpha, glu_limit;  // act 2: as DenseArgs
+    int tile0, col_blocks;  // this launch: tiles tile0 + 0 .. gridDim.x - 1 in the order of tile_at
+    int per, S;             // k64-steps per split, splits (blockIdx.y)
+    int part;               // 1: fp32 tiles [blockIdx.x][split][BM][BN] in `scratch` instead of the finished output
+    int vec;                // rows of `out` take 16-byte stores
+    float* scratch;
+};
+
+constexpr int X_RING = 4;  // buffers of x
+
+template <typename T> __device__ __forceinline__ float act2_of(const DTallArgs& a, float gate, float up) {
+    if (a.glu_limit > 0.f) {
+        const float g = fminf(gate, a.glu_limit), u = fminf(fmaxf(up, -a.glu_limit), a.glu_limit);
+        return g / (1.f + __expf(-a.glu_alpha * g)) * (u + 1.f);
+    }
+    const float sl = gate / (1.f + __expf(-gate));
+    return to_f32(from_f32<T>(sl)) * up;
+}
+
+constexpr int GROUP_ROWS = 8;  // 4 against 8 row blocks: 4096 x 22016 at 4096 rows 634 / 627 us, 6144 x 6400 at 300 45 / 43
+// Block bid of a launch of n -> its tile: XCD x (blocks x, x + 8, ...) takes a run of neighbouring tiles
+__device__ __forceinline__ int xcd_run(int bid, int n) {
+    const int x = bid & 7, q = n >> 3, rem = n & 7;
+    return x * q + min(x, rem) + (bid >> 3);
+}
+// Tile t of rows x cols blocks: groups of GROUP_ROWS row blocks, rows fastest
+__device__ __forceinline__ void tile_at(int t, int rows, int cols, int& row, int& col) {
+    const int per = GROUP_ROWS * cols, g = t / per, in = t - g * per, h = min(GROUP_ROWS, rows - g * GROUP_ROWS);
+    row = g * GROUP_ROWS + in % h;
+    col = in / h;
+}
+
+template <typename T, int BMR, int ACT, int TW>
+__global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
+    using V8 = typename VecT<T>::x8;
+    constexpr int BM = 32 * BMR;
+    constexpr int WR = TW == 2 ? 2 : 4;  // k64-steps of weights in flight per wave
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [X_RING][BM][128 bytes]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int row_block, col_block;
+    tile_at(a.tile0 + xcd_run(blockIdx.x, gridDim.x), (a.M + BM - 1) / BM, a.col_blocks, row_block, col_block);
+    const int m0 = row_block * BM;
+    const int mrows = min(BM, a.M - m0);
+    const int split = blockIdx.y;
+    const int nt_raw0 = (col_block * 4 + w) * TW;
+    const int ksteps = a.K >> 6;                                         // K % 64 == 0 (host)
+    const int ks0 = split * a.per, n = min(ksteps, ks0 + a.per) - ks0;   // n >= 1 (host)
+
+    const char* wtile[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) wtile[t] = reinterpret_cast<const char*>(a.prep) + (int64_t)min(nt_raw0 + t, a.NT - 1) * ksteps * 4096;
+    const uint32_t woff = lane * 16;
+    auto w_at = [&](int t, int ks, int i) -> V8 {
+        const char* p = wtile[t] + (int64_t)min(ks, ksteps - 1) * 4096 + i * 1024;
+        PIN_SGPR(p);
+        return *(const GLOBAL_AS V8*)(p + woff);
+    };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    uint32_t rowoff[BMR];
+#pragma unroll
+    for (int j = 0; j < BMR; ++j)
+        rowoff[j] = (uint32_t)(min(8 * (4 * j + w) + (lane >> 3), mrows - 1) * (int)a.ldx * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+    const char* xbase = reinterpret_cast<const char*>(a.x) + (int64_t)m0 * a.ldx * 2;
+    auto x_load = [&](int step, int buf) {
+        const char* xb = xbase + (int64_t)min(ks0 + step, ksteps - 1) * 128;
+        PIN_SGPR(xb);
+#pragma unroll
+        for (int j = 0; j < BMR; ++j)
+            kib_to_lds(xb, rowoff[j], __builtin_amdgcn_readfirstlane(lds0 + buf * (BM * 128) + (4 * j + w) * 1024));
+    };
+    f32x16 acc[TW][BMR];
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int rb = 0; rb < BMR; ++rb) acc[t][rb] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    uint32_t apos[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) apos[i] = (uint32_t)((lane & 31) * 128 + ((i + 4 * (lane >> 5)) ^ (lane & 7)) * 16);
+
+    x_load(0, 0);
+    x_load(1, 1);
+    x_load(2, 2);
+    V8 wq[WR][TW][4];
+#pragma unroll
+    for (int s = 0; s < WR; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < TW; ++t) wq[s][t][i] = w_at(t, ks0 + s, i);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WR * TW * 4) : "memory");
+    __syncthreads();
+    V8 av[2][BMR];
+    auto read_a = [&](V8 (&dst)[BMR], int buf, int i) {
+#pragma unroll
+        for (int rb = 0; rb < BMR; ++rb) dst[rb] = ld16<V8>(smem + buf * (BM * 128) + rb * 4096 + apos[i]);
+    };
+    read_a(av[0], 0, 0);
+    auto step = [&](int s, auto slot_) {
+        constexpr int SL = decltype(slot_)::value;
+        constexpr int NX = (SL + 1) % X_RING, WS = SL % WR;
+        x_load(s + 3, (SL + 3) % X_RING);  // everyone is done with that buffer since the barrier of the step before
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            read_a(av[(i + 1) & 1], i < 3 ? SL : NX, (i + 1) & 3);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int t = 0; t < TW; ++t) acc[t][rb] = mfma32(av[i & 1][rb], wq[WS][t][i], acc[t][rb]);
+#pragma unroll
+            for (int t = 0; t < TW; ++t) wq[WS][t][i] = w_at(t, ks0 + s + WR, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the x loads of step s + 2 were issued a step ago: behind them are that step's weights and everything of this step
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BMR + 8 * TW) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // whole turns of the ring, then what is left: with a way out behind every step the compiler sees ways back to the first one from each of
+    // them, and waits there for every load there is
+    using std::integral_constant;
+    int s = 0;
+    for (; s + X_RING <= n; s += X_RING) {
+        step(s, integral_constant<int, 0>{});
+        step(s + 1, integral_constant<int, 1>{});
+        step(s + 2, integral_constant<int, 2>{});
+        step(s + 3, integral_constant<int, 3>{});
+    }
+    if (s < n) {
+        step(s, integral_constant<int, 0>{});
+        if (s + 1 < n) {
+            step(s + 1, integral_constant<int, 1>{});
+            if (s + 2 < n) step(s + 2, integral_constant<int, 2>{});
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
+
+    const int c = lane & 31;
+    auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
+    constexpr int BN = 128 * TW;
+    if (a.part) {
+        float* dst = a.scratch + ((int64_t)xcd_run(blockIdx.x, gridDim.x) * a.S + split) * (BM * BN) + w * (32 * TW) + c;
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(rb, r) * BN + t * 32] = acc[t][rb][r];
+        return;
+    }
+    constexpr int BO = ACT == 2 ? BN / 2 : BN, OS = BO + 8;
+    const int n_out = ACT == 2 ? a.N >> 1 : a.N, n0 = col_block * BO;
+    __syncthreads();
+    T* tile_out = reinterpret_cast<T*>(smem);  // [BM][OS]
+    const T* bias = reinterpret_cast<const T*>(a.bias);
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+        const int nt = min(nt_raw0 + t, a.NT - 1);
+        if (ACT == 2) {
+            const int half = a.N >> 1, j = nt * 16 + (c & 15);
+            const float bv = bias ? to_f32(bias[c < 16 ? j : half + j]) : 0.f;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; r += 2) {
+                    const uint32_t v0 = __builtin_bit_cast(uint32_t, to_f32(from_f32<T>(acc[t][rb][r] + bv)));
+                    const uint32_t v1 = __builtin_bit_cast(uint32_t, to_f32(from_f32<T>(acc[t][rb][r + 1] + bv)));
+                    const auto p = __builtin_amdgcn_permlane16_swap(v0, v1, false, false);
+                    const uint32_t g0 = p[0], u0 = p[1];
+                    const float gate = __builtin_bit_cast(float, g0), up = __builtin_bit_cast(float, u0);
+                    tile_out[(row_of(rb, r) + (c >> 4)) * OS + (w * TW + t) * 16 + (c & 15)] = from_f32<T>(act2_of<T>(a, gate, up));
+                }
+        } else {
+            const float bv = bias && nt * 32 + c < a.N ? to_f32(bias[nt * 32 + c]) : 0.f;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    tile_out[row_of(rb, r) * OS + (w * TW + t) * 32 + c] = dense::finish_out<T>(acc[t][rb][r] + bv, a.gelu);
+        }
+    }
+    __syncthreads();
+    constexpr int PIECES = BO / 8;
+    for (int p = tid; p < mrows * PIECES; p += 256) {
+        const int m = p / PIECES, col = (p % PIECES) * 8;
+        if (n0 + col >= n_out) continue;
+        const V8 v = *reinterpret_cast<const V8*>(tile_out + m * OS + col);
+        T* o = reinterpret_cast<T*>(a.out) + (int64_t)(m0 + m) * a.ldo + n0 + col;
+        if (a.vec && n0 + col + 8 <= n_out) {
+            st16(o, v);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (n0 + col + e < n_out) o[e] = v[e];
+        }
+    }
+}
+
+template <typename T, int BM, int BN, int ACT>
+__global__ __launch_bounds__(256) void dense_tall_finish_kernel(DTallArgs a) {
+    constexpr int PER_ROW = ACT == 2 ? BN / 8 : BN / 4;
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    const int m = idx / PER_ROW, g = idx % PER_ROW;
+    int row_block, col_block;
+    tile_at(a.tile0 + blockIdx.y, (a.M + BM - 1) / BM, a.col_blocks, row_block, col_block);
+    const int row = row_block * BM + m;
+    if (m >= BM || row >= a.M) return;
+    const float* src = a.scratch + (int64_t)blockIdx.y * a.S * (BM * BN) + m * BN;
+    auto part_sum = [&](int col) {
+        f32x4 v = {0, 0, 0, 0};
+        for (int s = 0; s < a.S; ++s) v += *reinterpret_cast<const f32x4*>(src + (int64_t)s * (BM * BN) + col);
+        return v;
+    };
+    const T* bias = reinterpret_cast<const T*>(a.bias);
+    T* out = reinterpret_cast<T*>(a.out) + (int64_t)row * a.ldo;
+    if (ACT == 2) {
+        const int t = g >> 2, c = (g & 3) * 4, j = (col_block * (BN / 32) + t) * 16 + c, half = a.N >> 1;
+        if (j >= half) return;
+        const f32x4 gate = part_sum(t * 32 + c), up = part_sum(t * 32 + 16 + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            out[j + e] = from_f32<T>(act2_of<T>(a, to_f32(from_f32<T>(gate[e] + (bias ? to_f32(bias[j + e]) : 0.f))),
+                                                to_f32(from_f32<T>(up[e] + (bias ? to_f32(bias[half + j + e]) : 0.f)))));
+    } else {
+        const int n = col_block * BN + g * 4;
+        const f32x4 v = part_sum(g * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < a.N) out[n + e] = dense::finish_out<T>(v[e] + (bias ? to_f32(bias[n + e]) : 0.f), a.gelu);
+    }
+}
+
+constexpr int CUS = 256;
+
+struct TallPlan {
+    int BMR, TW;            // 32-row blocks and 32-column tiles per wave: a tile of 32 BMR x 128 TW
+    int col_blocks, tiles;
+    int whole;              // tiles of the unsplit launch; the rest is split S ways, `per` k64-steps each
+    int S, per;
+    double us;
+};
+// us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip.  These and the constants of plan_tall are fitted to
+// 300 products of 65 to 4096 rows and 1024 x 1024 to 24576 x 6144, each with up to 42 plans: the estimates are 10 % off, the plans that they
+// pick 1.1 % behind the best.
+struct TallCost {
+    double alone, busy;
+};
+constexpr TallCost TALL_COST[3][2] = {{{0.310, 0.415}, {0.538, 0.795}}, {{0.389, 0.451}, {0.612, 0.840}}, {{0.643, 0.556}, {0.711, 0.988}}};
+constexpr int MAX_PARTS = 384;  // blocks of the split launch: 48 MiB of fp32 tiles
+
+// Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k: 256 rows of 24576 x 6144 are 48 tiles of 128 x
+// 256 that walk 384 steps each (264 us; 95 split in four), 765 rows of 2048 x 11264 352 tiles of 96 x 128 (44 us; 52 in tiles of 128 x 128).
+TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
+    const int64_t steps = K / 64, NT = cdiv64(N, 32);
+    TallPlan best{};
+    double best_us = 1e30;
+    for (int BMR = 2; BMR <= 4; ++BMR)
+        for (int TW = 1; TW <= 2; ++TW) {
+            const TallCost c = TALL_COST[BMR - 2][TW - 1];
+            const int64_t cb = cdiv64(NT, 4 * TW), tiles = cb * cdiv64(M, 32 * BMR), rounds = tiles / CUS, rest = tiles % CUS;
+            const double alone = 1.6 + steps * c.alone, busy = 1.8 + steps * c.busy, share = (double)rest / CUS;
+            for (int S = 1; S <= 12; ++S) {
+                const int64_t per = cdiv64(steps, S);
+                if (S > 1 && (rest == 0 || rest * S > MAX_PARTS || per < 4)) break;
+                if ((S - 1) * per >= steps) continue;
+                double us = rounds * busy;
+                if (S > 1) {
+                    const double fill = (double)(rest * S) / CUS, part = 1.6 + per * c.alone;
+                    us += fill <= 1.0 ? part : std::max(part, (1.8 + per * c.busy) * fill);
+                    us += 4.4 + 2.0 * rest * S * (32 * BMR) * (128 * TW) * 4 / 3.5e6;  // the finish launch, the partial tiles at 3.5 TB/s
+                } else if (rounds == 0) {
+                    us = alone + std::max(0.0, busy - alone) * share;
+                } else {
+                    us = std::max(alone, us + (rest ? busy * (0.51 + 0.49 * share) : 0.0));
+                }
+                if (us < best_us) {
+                    best_us = us;
+                    best = {BMR, TW, (int)cb, (int)tiles, (int)(S > 1 ? tiles - rest : tiles), S, (int)per, us};
+                }
+            }
+        }
+    if (const char* e = getenv("TGIS_DTALL_PLAN")) {
+        int b = 0, t = 0, S = 0;
+        if (sscanf(e, "%d,%d,%d", &b, &t, &S) == 3 && b >= 2 && b <= 4 && t >= 1 && t <= 2 && S >= 1 && S <= 16) {
+            const int64_t cb = cdiv64(NT, 4 * t), tiles = cb * cdiv64(M, 32 * b), per = cdiv64(steps, S);
+            if ((S - 1) * per < steps && (S == 1 || tiles % CUS * S <= MAX_PARTS)) best = {b, t, (int)cb, (int)tiles, (int)(S > 1 ? tiles - tiles % CUS : tiles), S, (int)per, 0.0};
+        }
+    }
+    return best;
+}
+
+int64_t plan_scratch(const TallPlan& p) {
+    return p.whole < p.tiles ? (int64_t)(p.tiles - p.whole) * p.S * (32 * p.BMR) * (128 * p.TW) * 4 : 0;
+}
+
+template <typename T, int BMR, int ACT, int TW>
+int launch_blocks(const DTallArgs& a, int tiles, int S, hipStream_t st) {
+    constexpr size_t ring = (size_t)X_RING * (32 * BMR) * 128, rows = (size_t)(32 * BMR) * ((ACT == 2 ? 64 : 128) * TW + 8) * 2;
+    constexpr size_t lds = ring > rows ? ring : rows;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)dense_tall_kernel<T, BMR, ACT, TW>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    TGIS_CHECK_HIP(attr);
+    hipLaunchKernelGGL((dense_tall_kernel<T, BMR, ACT, TW>), dim3((unsigned)tiles, (unsigned)S), dim3(256), lds, st, a);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+template <typename T, int ACT>
+int launch_shape(const TallPlan& p, const DTallArgs& a, int tiles, int S, hipStream_t st) {
+    switch (p.BMR * 10 + p.TW) {
+        case 21: return launch_blocks<T, 2, ACT, 1>(a, tiles, S, st);
+        case 22: return launch_blocks<T, 2, ACT, 2>(a, tiles, S, st);
+        case 31: return launch_blocks<T, 3, ACT, 1>(a, tiles, S, st);
+        case 32: return launch_blocks<T, 3, ACT, 2>(a, tiles, S, st);
+        case 41: return launch_blocks<T, 4, ACT, 1>(a, tiles, S, st);
+        default: return launch_blocks<T, 4, ACT, 2>(a, tiles, S, st);
+    }
+}
+
+template <typename T, int ACT>
+int launch_finish(const TallPlan& p, const DTallArgs& a, int tiles, hipStream_t st) {
+#define TGIS_TALL_FINISH(B, W)                                                                                                         \
+    hipLaunchKernelGGL((dense_tall_finish_kernel<T, 32 * B, 128 * W, ACT>),                                                            \
+                       dim3((unsigned)cdiv64((int64_t)32 * B * (128 * W) / (ACT == 2 ? 8 : 4), 256), (unsigned)tiles), dim3(256), 0, st, a)
+    switch (p.BMR * 10 + p.TW) {
+        case 21: TGIS_TALL_FINISH(2, 1); break;
+        case 22: TGIS_TALL_FINISH(2, 2); break;
+        case 31: TGIS_TALL_FINISH(3, 1); break;
+        case 32: TGIS_TALL_FINISH(3, 2); break;
+        case 41: TGIS_TALL_FINISH(4, 1); break;
+        default: TGIS_TALL_FINISH(4, 2); break;
+    }
+#undef TGIS_TALL_FINISH
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+template <typename T>
+int run_tall(const TallPlan& p, DTallArgs& a, int act, hipStream_t st) {
+    a.per = a.K / 64;
+    a.S = 1;
+    if (p.whole > 0) {
+        const int rc = act == 2 ? launch_shape<T, 2>(p, a, p.whole, 1, st) : launch_shape<T, 0>(p, a, p.whole, 1, st);
+        if (rc != TGIS_OK) return rc;
+    }
+    if (p.whole < p.tiles) {
+        a.tile0 = p.whole;
+        a.per = p.per;
+        a.S = p.S;
+        a.part = 1;
+        const int rc = launch_shape<T, 0>(p, a, p.tiles - p.whole, p.S, st);
+        if (rc != TGIS_OK) return rc;
+        return act == 2 ? launch_finish<T, 2>(p, a, p.tiles - p.whole, st) : launch_finish<T, 0>(p, a, p.tiles - p.whole, st);
+    }
+    return TGIS_OK;
+}
+}  // namespace
+
+// Is this kernel the faster way?  us, the alternative / this kernel, weights cold, launches back to back.
+// Up to 256 rows the alternative is the weight-streaming kernel, which goes over the weights once per 64 rows (a product below 65 rows stays there):
+//   65 / 128 / 140 / 256 rows: 2048 x 2048 9.9 / 8.9, 10.7 / 9.6, 11.4 / 9.9, 12.4 / 10.9; 1024 x 1024 8.0 / 7.8, 8.2 / 7.9, 8.3 / 7.9, 8.7 / 8.0; 5632 x
+//   2048 14.8 / 12.2, 15.5 / 12.6, 20 / 13.6, 21 / 15; 2048 x 11264 with SiLU 18.6 / 16.3, 18.8 / 18.4, 30 / 20, 36 / 24; 4096 x 12288 33 / 26, 32 / 30,
+//   55 / 34, 65 / 42; 6144 x 24576 98 / 63, 106 / 76, 157 / 88, 195 / 99; 24576 x 6144 109 / 66, 110 / 68, 203 / 84, 219 / 95
+// Above, it is the library, with a launch of its own for the activation.  Its 256 x 256 tiles at 1.2 - 1.45 PFLOP/s win wherever they fill the chip:
+//   act 0 / GELU, 300 / 600 / 1024 / 1400 / 2048 rows: 2048 x 2048 10.7 / 11.6, 13.8 / 12.5, 15.9 / 13.6, 19.0 / 18.2, 21.6 / 23.6; 5632 x 2048 24 / 16, 30 /
+//   25, 37 / 32, 45 / 40, 54 / 54; 6144 x 6400 44 / 42, 64 / 59, 92 / 85, 101 / 115, 139 / 155; 24576 x 6144 200 / 123, 278 / 180, 405 / 320, 621 / 380, 468 /
+//   530; 4096 x 12288 53 / 52, 66 / 68, 93 / 115; 6144 x 24576 118 / 130, 202 / 180, 267 / 264, 386 / 379, 463 / 497; 2048 x 6144 15.6 / 13.8, 22 / 23,
+//   29 / 36: hence bounds on rows x columns, against the depth and at 6.3 million, and on the rows
+//   act 2, 300 / 433 / 600 / 1024 / 2048 / 4096 / 8186 / 16128 rows: 1024 x 5632 14 / 8.4, 17 / 11, 20 / 13, 26 / 18, 44 / 31, 69 / 54; 2048 x 11264 32 / 28, 37 /
+//   30, 39 / 35, 60 / 54, 100 / 90, 187 / 170, 410 / 316, 626 / 620; 4096 x 22016 78 / 86, 95 / 97, 140 / 117, 190 / 177, 440 / 335, 720 / 627, 1260 / 1249,
+//   2294 / 2500
+// Narrow and shallow ones stay where they were: 2048 x 512 at 128 / 300 rows 8.6 / 9.2, 8.2 / 9.0; 64 x 2048 at 600, 1400 rows 4.4 / 5.1, 5.2 / 6.8.
+static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act) {
+    if (M <= 64 || K % 64 != 0 || N < 1024) return false;
+    if (M <= 256) return true;
+    if (act == 2) return M <= 8192 && (M > 512 || K * N <= (32 << 20));
+    return M <= 1400 && K >= 512 && M * N <= std::min<int64_t>(1500 * K, 6300000);
+}
+
+// Bytes of scratch of tgis_dense_tall where it is the faster way to this product, -1 where it is not.
+extern "C" int64_t tgis_dense_tall_bytes(int64_t M, int64_t K, int64_t N, int act) {
+    if (M < 1 || K < 64 || N < 1 || !(act == 0 || act == 2 || act == 4 || act == 5) || !dense_tall_pays(M, K, N, act)) return -1;
+    return plan_scratch(plan_tall(M, K, N));
+}
+
+// out = act(x @ w^T + bias) in the model dtype.  act 0; 4 / 5: GELU (erf / tanh) of the rounded sum; 2: SiLU(gate) * up of a gate | up image
+// (out [M, N / 2]), or with glu_limit > 0 the clamped unit (DenseArgs::glu_limit).
+extern "C" int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo, int64_t M, int64_t K,
+                               int64_t N, int dtype, int act, float glu_alpha, float glu_limit, void* workspace, int64_t workspace_bytes,
+                               void* stream) {
+    TGIS_CHECK_ARG(x && prepared && out && M >= 0 && K >= 64 && K % 64 == 0 && N >= 1, "tgis_dense_tall: bad arguments");
+    TGIS_CHECK_ARG((dtype == TGIS_F16 || dtype == TGIS_BF16) && (act == 0 || act == 2 || act == 4 || act == 5), "tgis_dense_tall: bad dtype or act");
+    TGIS_CHECK_ARG(act != 2 || N % 32 == 0, "tgis_dense_tall: act 2 needs a gate|up image (N / 2 a multiple of 16)");
+    TGIS_CHECK_ARG(ldx >= K && ldx % 8 == 0 && (uintptr_t)x % 16 == 0, "tgis_dense_tall: x rows must be 16-byte aligned");
+    TGIS_CHECK_ARG(ldx < (1ll << 22), "tgis_dense_tall: x rows too far apart");  // a tile's rows are addressed with 31 bits
+    if (M == 0) return TGIS_OK;
+    const TallPlan p = plan_tall(M, K, N);
+    TGIS_CHECK_ARG(plan_scratch(p) == 0 || (workspace && workspace_bytes >= plan_scratch(p)), "tgis_dense_tall: workspace too small");
+    DTallArgs a{};
+    a.x = x;
+    a.ldx = ldx;
+    a.prep = (const uint8_t*)prepared;
+    a.bias = bias;
+    a.out = out;
+    a.ldo = ldo;
+    a.M = (int)M;
+    a.K = (int)K;
+    a.N = (int)N;
+    a.NT = (int)cdiv64(N, 32);
+    a.gelu = act == 4 ? 1 : act == 5 ? 2 : 0;
+    a.glu_alpha = glu_alpha;
+    a.glu_limit = glu_limit;
+    a.vec = ldo % 8 == 0 && (uintptr_t)out % 16 == 0;
+    a.col_blocks = p.col_blocks;
+    a.scratch = (float*)workspace;
+    const hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
+    return dtype == TGIS_F16 ? run_tall<f16>(p, a, act == 2 ? 2 : 0, st) : run_tall<bf16>(p, a, act == 2 ? 2 : 0, st);
+}

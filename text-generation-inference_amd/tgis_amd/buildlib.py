@@ -17,13 +17,14 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-tar
 
 # translation units per family (api.hip: error state / version; elementwise.hip: decode bookkeeping, argmax)
 FAMILY_UNITS = {
-    "lenisun": ["api", "elementwise", "gemm_dense", "residual_f32", "attn_varlen", "attention_prefill", "wkv", "moe", "sampler"],
-    "senadra": ["api", "elementwise", "gemm_dense", "residual_f32", "attn_varlen", "attention_prefill", "head_product", "delta_rule", "sampler"],
-    "mananex": ["api", "elementwise", "gemm_dense", "residual_f32", "attn_varlen", "attention_prefill", "gated_linear_scan", "moe", "sampler"],
-    "tatevik": ["api", "elementwise", "gemm_dense", "residual_f32", "norm_f32", "attn_varlen", "attention_prefill", "attn_mixed_heads", "gated_linear_scan",
-                "selective_scan", "causal_conv", "moe", "sampler"],
-    "gopetar": ["api", "elementwise", "gemm_dense", "residual_f32", "hyper_streams", "attn_varlen", "attention_prefill", "head_product", "min_gru", "moe", "sampler"],
-    "fidatar": ["api", "elementwise", "gemm_dense", "residual_f32", "post_norm", "attn_varlen", "attention_prefill", "matrix_memory", "moe", "sampler"],
+    "lenisun": ["api", "elementwise", "gemm_dense", "dense_tall", "residual_f32", "attn_varlen", "attention_prefill", "wkv", "moe", "sampler"],
+    "senadra": ["api", "elementwise", "gemm_dense", "dense_tall", "residual_f32", "attn_varlen", "attention_prefill", "head_product", "delta_rule", "sampler"],
+    "mananex": ["api", "elementwise", "gemm_dense", "dense_tall", "residual_f32", "attn_varlen", "attention_prefill", "gated_linear_scan", "moe", "sampler"],
+    "tatevik": ["api", "elementwise", "gemm_dense", "dense_tall", "residual_f32", "norm_f32", "attn_varlen", "attention_prefill", "attn_mixed_heads",
+                "gated_linear_scan", "selective_scan", "causal_conv", "moe", "sampler"],
+    "gopetar": ["api", "elementwise", "gemm_dense", "dense_tall", "residual_f32", "hyper_streams", "attn_varlen", "attention_prefill", "head_product",
+                "min_gru", "moe", "sampler"],
+    "fidatar": ["api", "elementwise", "gemm_dense", "dense_tall", "residual_f32", "post_norm", "attn_varlen", "attention_prefill", "matrix_memory", "moe", "sampler"],
 }
 
 

@@ -200,6 +200,8 @@ SIGNATURES = {
     "tgis_narrow_product": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_int, _c_i64, _c_int, _vp]),
     "tgis_moe_choose": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_f, _vp, _vp, _vp]),
     "tgis_relu2": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_tall_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int]),
+    "tgis_dense_tall": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_f, _c_f, _vp, _c_i64, _vp]),
     "tgis_dense_gemm_whole_operand": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
@@ -676,6 +678,31 @@ def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f3
         load_library().tgis_dense_gemm(_ptr(x), x.stride(0), _ptr(w.image), _ptr(bias), _ptr(out), out.stride(0), M,
                                        w.K, w.N, dtype_code(w.dtype), int(out_f32), act, ws.ptr, ws.nbytes,
                                        _stream()), "tgis_dense_gemm")
+    return out
+
+
+DENSE_TALL_MIN_M = 65
+
+
+def dense_tall_pays(x: torch.Tensor, w: DenseWeight, act: int = 0) -> bool:
+    """Is dense_tall the faster way to x @ w^T?  (a size query; x as it reads it)"""
+    M, ld = x.shape[0], x.stride(0)
+    return (M >= DENSE_TALL_MIN_M and x.stride(1) == 1 and ld % 8 == 0 and w.K <= ld < 1 << 22 and x.data_ptr() % 16 == 0
+            and load_library().tgis_dense_tall_bytes(M, w.K, w.N, act) >= 0)
+
+
+def dense_tall(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, act: int = 0, alpha: float = 0.0, limit: float = 0.0, out=None) -> torch.Tensor:
+    """dense_gemm of a prefill's rows; act 0, 4, 5 or 2 (limit > 0: the clamped unit of dense_gemm_clamped_glu)."""
+    assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K
+    assert (act == 2) == bool(w.flags & 1) and not w.flags & 2
+    M = x.shape[0]
+    if out is None:
+        out = torch.empty((M, w.N // 2 if act == 2 else w.N), dtype=w.dtype, device=x.device)
+    lib = load_library()
+    nbytes = lib.tgis_dense_tall_bytes(M, w.K, w.N, act)
+    ws.ensure(4096 + max(nbytes, 0))  # (the first page holds the arrival counters of other launches)
+    _check(lib.tgis_dense_tall(_ptr(x), x.stride(0), _ptr(w.image), _ptr(bias), _ptr(out), out.stride(0), M, w.K, w.N, dtype_code(w.dtype), act,
+                               float(alpha), float(limit), ws.ptr + 4096, ws.nbytes - 4096, _stream()), "tgis_dense_tall")
     return out
 
 

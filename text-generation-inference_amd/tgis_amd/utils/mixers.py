@@ -189,8 +189,8 @@ class GatedUnit:
         self.fused = self.mode == 0 and self.gate_up.streams and self.ff % 16 == 0
         if self.fused:
             self.gate_up.gate_up = True
-        # the clamped form at decode sizes: the same gate | up image with the clamped unit in the epilogue (a second image
-        # of the weight; longer steps take the library GEMM on the checkpoint layout and the activation launch)
+        # the clamped form: the same gate | up image with the clamped unit in the epilogue (a second image of the weight; steps that
+        # neither kernel on it serves take the library GEMM on the checkpoint layout and the activation launch)
         self.clamped_image = None
         if self.mode == 1 and self.gate_up.streams and self.ff % 16 == 0 and self.limit > 0:
             self.clamped_image = native.DenseWeight(self.gate_up.weight, gate_up=True)
@@ -200,6 +200,9 @@ class GatedUnit:
         partial = partial and can_defer(self.down)
         if self.fused:
             return self.down(self.gate_up(h), partial=partial)
+        if self.clamped_image is not None and native.dense_tall_pays(h, self.clamped_image, 2):
+            act = native.dense_tall(h, self.clamped_image, workspace(h.device), bias=self.gate_up.bias, act=2, alpha=self.alpha, limit=self.limit)
+            return self.down(act, partial=partial)
         if self.clamped_image is not None and h.shape[0] <= CLAMPED_EPILOGUE_MAX_M:
             act = native.dense_gemm_clamped_glu(h, self.clamped_image, workspace(h.device), self.alpha, self.limit)
             return self.down(act, partial=partial)
