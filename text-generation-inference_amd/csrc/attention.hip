@@ -44,7 +44,7 @@ namespace {
 template <typename T>
 __device__ __forceinline__ void store_out(const AttnArgs& a, int64_t tok, int k0, int64_t K, typename VecT<T>::x8 v) {
     T* out = reinterpret_cast<T*>(a.out);
-    if (a.out_cols) {
+    if (a.out_frag > 1) {
         int to[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) to[e] = a.out_cols[k0 + e];
@@ -811,7 +811,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     a.cu_q = cu_seqlens_q;
     a.out = out;
     a.out_cols = out_cols;
-    a.out_frag = ld_out == TGIS_LD_FRAGMENTS;
+    a.out_frag = out_cols ? 2 : ld_out == TGIS_LD_FRAGMENTS;
     a.ld_out = (int64_t)H * D;
     attn_set_geom(a, H, Hkv, g);
     const int ch = chunks_per_block(g.HC, max_q_len);

@@ -12,7 +12,7 @@ struct AttnArgs {
     const int32_t* ctx_lens;
     const int32_t* cu_q;
     void* out;
-    int out_frag;  // 1: out is [<= 32 tokens, H * D] in 32-row fragment order (xf_off in common.h), else row-major
+    int out_frag;  // 1: out is [<= 32 tokens, H * D] in 32-row fragment order (xf_off in common.h), 2: with its columns re-ordered; else row-major
     int H, Hkv, G, Gc, Gp, TQ, HC, NS;
     int Gp_shift;  // Gp is a power of two: column -> (q token, head of the group) by shift and mask, not by division
     int HCB;  // decode kernel: blocks per kv head along the 16-head chunks (HC / chunks per block)
@@ -22,7 +22,7 @@ struct AttnArgs {
     float* ws_ml;  // [total_q][H][NS][2]        (fused combine: [group][chunk][16 columns][NS][4], {m, l, -, -})
     unsigned* counters;  // fused combine: per-group arrival counters (zero between launches), or nullptr
     int64_t ld_out;  // prefill kernel: elements between two tokens' rows of `out`
-    const int32_t* out_cols;  // decode, out_frag: output column k is stored as column out_cols[k] (a permutation), or nullptr
+    const int32_t* out_cols;  // out_frag 2: output column k is stored as column out_cols[k] (a permutation)
 };
 
 constexpr float NEG_BIG = -1.0e30f;
