@@ -169,13 +169,18 @@ int tgis_dense_gemm_rope(const void* x, int64_t ldx, const void* prepared, const
 int tgis_gptq_dequant_f16(const void* prepared, void* w_out, int64_t K, int64_t N, int64_t groups,
                           int flags, void* stream);
 
-/* Dense products of prefills on the image of tgis_dense_prepare: out = act(x W^T + bias) in the model dtype, K a multiple of 64, x rows 16-byte
- * aligned.  act 0 none, 4 / 5 GELU (erf / tanh) of the rounded sum, 2 SiLU(gate) * up of the gate|up image ([M][N / 2]; glu_limit > 0: the
+/* Dense products of prefills on the image of tgis_dense_prepare: out = act(x W^T + bias) in the model dtype or, act 0, in fp32; K a multiple of 64, x rows 16-byte aligned.  act 0 none, 4 / 5 GELU (erf / tanh) of the rounded sum, 2 SiLU(gate) * up of the gate|up image ([M][N / 2]; glu_limit > 0: the
  * clamped unit of tgis_dense_gemm_clamped_glu instead).
  * tgis_dense_tall_bytes: the scratch that M rows take where this is the faster way to the product, -1 where it is not (a size query). */
 int64_t tgis_dense_tall_bytes(int64_t M, int64_t K, int64_t N, int act);
 int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo, int64_t M, int64_t K, int64_t N,
-                    int dtype, int act, float glu_alpha, float glu_limit, void* workspace, int64_t workspace_bytes, void* stream);
+                    int dtype, int out_f32, int act, float glu_alpha, float glu_limit, void* workspace, int64_t workspace_bytes, void* stream);
+/* ... left as partial sums, as by tgis_dense_gemm_partial, up to 256 rows (-1 bytes: not the faster way). */
+int64_t tgis_dense_tall_partial_bytes(int64_t M, int64_t K, int64_t N);
+int tgis_dense_tall_partial(const void* x, int64_t ldx, const void* prepared, int64_t M, int64_t K, int64_t N, int dtype, float* slabs,
+                            int64_t slabs_bytes, int* num_slabs, int64_t* slab_ld, void* stream);
+
+#define TGIS_DENSE_TALL_MIN_M 65
 
 /* Decode steps of up to 4 rows: dense products that norm their operand themselves and add to the residual stream, which stays in fp32
  * (h, [M][width], rows back to back) between them.  With norm(h)[k] = T(h[k] * rstd * norm_w[k]), norm_w of the model dtype, and the images of

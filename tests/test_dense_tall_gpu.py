@@ -56,7 +56,7 @@ def _run(M, K, N, dtype, act, plan, monkeypatch, ld_out=None):
     ws = native.Workspace(64 << 20, torch.device("cuda"))
     n_out = N // 2 if act in (2, 3) else N
     out = torch.full((M, ld_out or n_out), 7.0, dtype=dtype, device="cuda")
-    native.dense_tall(x.cuda(), image, ws, bias=bias.cuda(), act=2 if clamped else act, alpha=1.7, limit=3.0 if clamped else 0.0, out=out[:, :n_out])
+    native.dense_tall(x.cuda(), image, ws, 48 << 20, bias=bias.cuda(), act=2 if clamped else act, alpha=1.7, limit=3.0 if clamped else 0.0, out=out[:, :n_out])
     _check(out[:, :n_out], _expect(z, acc, dtype, act))
     assert bool((out[:, n_out:] == 7.0).all())
 
@@ -70,6 +70,24 @@ def _run(M, K, N, dtype, act, plan, monkeypatch, ld_out=None):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_plain(plan, M, K, N, dtype, monkeypatch):
     _run(M, K, N, dtype, 0, plan, monkeypatch, ld_out=N + 8 if M % 2 else None)
+
+
+@pytest.mark.parametrize("plan,M", [("2,1,1", 97), ("2,2,3", 129), ("3,2,2", 190), ("4,2,1", 256), ("4,1,5", 65), (None, 108)])
+def test_fp32_sums(plan, M, monkeypatch):
+    """Without a rounding: the partial sums that a norm finishes, and a head's logits."""
+    from tgis_amd import native
+    from tgis_amd.utils.layers import FastLinear
+
+    K, N = 576, 1100
+    x, w, bias, z, acc = _case(M, K, N, torch.bfloat16, seed=5)
+    lin = FastLinear(w.cuda(), bias.cuda())
+    if plan:
+        monkeypatch.setenv("TGIS_DTALL_PLAN", plan)
+    part = lin(x.cuda(), partial=True)
+    assert isinstance(part, native.Partial) and part.ld == 1120 and part.bias is lin.bias and (plan is None or part.S == int(plan[4]))
+    sums = part.slabs.view(-1, part.S, 32, part.ld).sum(1, dtype=torch.float64).flatten(0, 1)
+    _check(sums[:M, :N], (z - bias.double(), acc))
+    _check(lin(x.cuda(), out_f32=True), (z, acc))
 
 
 @pytest.mark.parametrize("plan", ["2,1,1", "2,2,2", "3,1,3", "3,2,1", "4,1,2", "4,2,1"])
@@ -113,5 +131,5 @@ def test_rows_it_cannot_read(pad, first):
     view = wide[:, first:first + 512]
     view.copy_(x)
     lin = FastLinear(w.cuda(), bias.cuda())
-    assert not native.dense_tall_pays(view, lin.prepared) and native.dense_tall_pays(x.cuda(), lin.prepared)
+    assert lin.tall(view) == -1 and lin.tall(x.cuda()) >= 0
     _check(lin(view), _expect(z, acc, torch.float16, 0))

@@ -32,8 +32,10 @@ struct DTallArgs {
     float glu_alpha, glu_limit;  // act 2: as DenseArgs
     int tile0, col_blocks;  // this launch: tiles tile0 + 0 .. gridDim.x - 1 in the order of tile_at
     int per, S;             // k64-steps per split, splits (blockIdx.y)
-    int part;               // 1: fp32 tiles [blockIdx.x][split][BM][BN] in `scratch` instead of the finished output
+    int part;               // instead of the finished output, fp32 sums in `scratch`: 1 tiles [blockIdx.x][split][BM][BN], 2 slabs [row block of
+                            // 32][split][32][32 NT]
     int vec;                // rows of `out` take 16-byte stores
+    int out_f32;            // act 0: `out` takes the fp32 sums (+ bias)
     float* scratch;
 };
 
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
     const int c = lane & 31;
     auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
     constexpr int BN = 128 * TW;
-    if (a.part) {
+    if (a.part == 1) {
         float* dst = a.scratch + ((int64_t)xcd_run(blockIdx.x, gridDim.x) * a.S + split) * (BM * BN) + w * (32 * TW) + c;
 #pragma unroll
         for (int t = 0; t < TW; ++t)
@@ -178,6 +180,40 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
             for (int rb = 0; rb < BMR; ++rb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(rb, r) * BN + t * 32] = acc[t][rb][r];
+        return;
+    }
+    if (ACT == 0 && a.part == 2) {
+        const int ld = a.NT * 32, blocks = (a.M + 31) >> 5;
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            if (nt_raw0 + t >= a.NT) continue;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb) {
+                const int block = row_block * BMR + rb;
+                if (block >= blocks) continue;
+                float* dst = a.scratch + ((int64_t)block * a.S + split) * 32 * ld + (nt_raw0 + t) * 32 + c;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(0, r) * ld] = acc[t][rb][r];
+            }
+        }
+        return;
+    }
+    if (ACT == 0 && a.out_f32) {
+        const int m_lane = m0 + 4 * (lane >> 5);
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const int n = (nt_raw0 + t) * 32 + c;
+            if (n >= a.N) continue;
+            const float bv = a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[n]) : 0.f;
+            float* dst = reinterpret_cast<float*>(a.out) + n;
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m_lane + rb * 32 + (r & 3) + 8 * (r >> 2);
+                    if (m < a.M) dst[(int64_t)m * a.ldo] = acc[t][rb][r] + bv;
+                }
+        }
         return;
     }
     constexpr int BO = ACT == 2 ? BN / 2 : BN, OS = BO + 8;
@@ -256,6 +292,13 @@ __global__ __launch_bounds__(256) void dense_tall_finish_kernel(DTallArgs a) {
     } else {
         const int n = col_block * BN + g * 4;
         const f32x4 v = part_sum(g * 4);
+        if (a.out_f32) {
+            float* sums = reinterpret_cast<float*>(a.out) + (int64_t)row * a.ldo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < a.N) sums[n + e] = v[e] + (bias ? to_f32(bias[n + e]) : 0.f);
+            return;
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (n + e < a.N) out[n + e] = dense::finish_out<T>(v[e] + (bias ? to_f32(bias[n + e]) : 0.f), a.gelu);
@@ -282,7 +325,7 @@ constexpr int MAX_PARTS = 384;  // blocks of the split launch: 48 MiB of fp32 ti
 
 // Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k: 256 rows of 24576 x 6144 are 48 tiles of 128 x
 // 256 that walk 384 steps each (264 us; 95 split in four), 765 rows of 2048 x 11264 352 tiles of 96 x 128 (44 us; 52 in tiles of 128 x 128).
-TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
+TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
     const int64_t steps = K / 64, NT = cdiv64(N, 32);
     TallPlan best{};
     double best_us = 1e30;
@@ -311,14 +354,67 @@ TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
                 }
             }
         }
-    if (const char* e = getenv("TGIS_DTALL_PLAN")) {
-        int b = 0, t = 0, S = 0;
-        if (sscanf(e, "%d,%d,%d", &b, &t, &S) == 3 && b >= 2 && b <= 4 && t >= 1 && t <= 2 && S >= 1 && S <= 16) {
-            const int64_t cb = cdiv64(NT, 4 * t), tiles = cb * cdiv64(M, 32 * b), per = cdiv64(steps, S);
-            if ((S - 1) * per < steps && (S == 1 || tiles % CUS * S <= MAX_PARTS)) best = {b, t, (int)cb, (int)tiles, (int)(S > 1 ? tiles - tiles % CUS : tiles), S, (int)per, 0.0};
-        }
-    }
     return best;
+}
+
+// ... where the consumer adds the parts: every tile in the same number of them, and no launch behind: completions of two prompts of 54 tokens, 8 hybrid layers
+// of 2048, 2360 -> 2250 us (2145 with the plans kept, below).
+TallPlan make_plan_parts(int64_t M, int64_t K, int64_t N) {
+    const int64_t steps = K / 64, NT = cdiv64(N, 32);
+    TallPlan best{};
+    double best_us = 1e30;
+    for (int BMR = 2; BMR <= 4; ++BMR)
+        for (int TW = 1; TW <= 2; ++TW) {
+            const TallCost c = TALL_COST[BMR - 2][TW - 1];
+            const int64_t cb = cdiv64(NT, 4 * TW), tiles = cb * cdiv64(M, 32 * BMR);
+            for (int S = 1; S <= 8; ++S) {
+                const int64_t per = cdiv64(steps, S);
+                if (S > 1 && per < 4) break;
+                if ((S - 1) * per >= steps) continue;
+                const double fill = (double)(tiles * S) / CUS, alone = 1.6 + per * c.alone, busy = 1.8 + per * c.busy;
+                const double us = (fill <= 1.0 ? alone + std::max(0.0, busy - alone) * fill : std::max(alone, busy * fill)) + 0.3 * (S - 1) +
+                                  2.0 * S * M * N * 4 / 3.5e6;
+                if (us < best_us) {
+                    best_us = us;
+                    best = {BMR, TW, (int)cb, (int)tiles, 0, S, (int)per, us};
+                }
+            }
+        }
+    return best;
+}
+
+// TGIS_DTALL_PLAN=BMR,TW,S: this plan for every product that it fits
+bool plan_from_env(int64_t M, int64_t K, int64_t N, bool parts, TallPlan& p) {
+    const char* e = getenv("TGIS_DTALL_PLAN");
+    int b = 0, t = 0, S = 0;
+    if (!e || sscanf(e, "%d,%d,%d", &b, &t, &S) != 3 || b < 2 || b > 4 || t < 1 || t > 2 || S < 1 || S > 16) return false;
+    const int64_t steps = K / 64, cb = cdiv64(cdiv64(N, 32), 4 * t), tiles = cb * cdiv64(M, 32 * b), per = cdiv64(steps, S);
+    if ((S - 1) * per >= steps || (!parts && S > 1 && tiles % CUS * S > MAX_PARTS)) return false;
+    p = {b, t, (int)cb, (int)tiles, (int)(parts ? 0 : S > 1 ? tiles - tiles % CUS : tiles), S, (int)per, 0.0};
+    return true;
+}
+
+// A plan takes 1 - 2 us to make, a short prompt's launch 4 to prepare: each thread keeps those of the sizes that it asked for last.
+template <TallPlan (*MAKE)(int64_t, int64_t, int64_t)>
+TallPlan kept_plan(int64_t M, int64_t K, int64_t N) {
+    struct Entry {
+        int64_t M, K, N;
+        TallPlan plan;
+    };
+    thread_local Entry kept[64] = {};
+    Entry& e = kept[(M * 5 + K / 64 * 3 + N / 32) % 64];
+    if (e.M != M || e.K != K || e.N != N) e = {M, K, N, MAKE(M, K, N)};
+    return e.plan;
+}
+
+TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
+    TallPlan p;
+    return plan_from_env(M, K, N, false, p) ? p : kept_plan<make_plan_tall>(M, K, N);
+}
+
+TallPlan plan_parts(int64_t M, int64_t K, int64_t N) {
+    TallPlan p;
+    return plan_from_env(M, K, N, true, p) ? p : kept_plan<make_plan_parts>(M, K, N);
 }
 
 int64_t plan_scratch(const TallPlan& p) {
@@ -403,7 +499,7 @@ int run_tall(const TallPlan& p, DTallArgs& a, int act, hipStream_t st) {
 //   2294 / 2500
 // Narrow and shallow ones stay where they were: 2048 x 512 at 128 / 300 rows 8.6 / 9.2, 8.2 / 9.0; 64 x 2048 at 600, 1400 rows 4.4 / 5.1, 5.2 / 6.8.
 static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act) {
-    if (M <= 64 || K % 64 != 0 || N < 1024) return false;
+    if (M < TGIS_DENSE_TALL_MIN_M || K % 64 != 0 || N < 1024) return false;
     if (M <= 256) return true;
     if (act == 2) return M <= 8192 && (M > 512 || K * N <= (32 << 20));
     return M <= 1400 && K >= 512 && M * N <= std::min<int64_t>(1500 * K, 6300000);
@@ -415,37 +511,72 @@ extern "C" int64_t tgis_dense_tall_bytes(int64_t M, int64_t K, int64_t N, int ac
     return plan_scratch(plan_tall(M, K, N));
 }
 
-// out = act(x @ w^T + bias) in the model dtype.  act 0; 4 / 5: GELU (erf / tanh) of the rounded sum; 2: SiLU(gate) * up of a gate | up image
-// (out [M, N / 2]), or with glu_limit > 0 the clamped unit (DenseArgs::glu_limit).
-extern "C" int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo, int64_t M, int64_t K,
-                               int64_t N, int dtype, int act, float glu_alpha, float glu_limit, void* workspace, int64_t workspace_bytes,
-                               void* stream) {
-    TGIS_CHECK_ARG(x && prepared && out && M >= 0 && K >= 64 && K % 64 == 0 && N >= 1, "tgis_dense_tall: bad arguments");
-    TGIS_CHECK_ARG((dtype == TGIS_F16 || dtype == TGIS_BF16) && (act == 0 || act == 2 || act == 4 || act == 5), "tgis_dense_tall: bad dtype or act");
-    TGIS_CHECK_ARG(act != 2 || N % 32 == 0, "tgis_dense_tall: act 2 needs a gate|up image (N / 2 a multiple of 16)");
-    TGIS_CHECK_ARG(ldx >= K && ldx % 8 == 0 && (uintptr_t)x % 16 == 0, "tgis_dense_tall: x rows must be 16-byte aligned");
-    TGIS_CHECK_ARG(ldx < (1ll << 22), "tgis_dense_tall: x rows too far apart");  // a tile's rows are addressed with 31 bits
-    if (M == 0) return TGIS_OK;
-    const TallPlan p = plan_tall(M, K, N);
-    TGIS_CHECK_ARG(plan_scratch(p) == 0 || (workspace && workspace_bytes >= plan_scratch(p)), "tgis_dense_tall: workspace too small");
+static bool rows_ok(const void* x, int64_t ldx, int64_t K) {  // (a tile's rows are addressed with 31 bits)
+    return ldx >= K && ldx % 8 == 0 && (uintptr_t)x % 16 == 0 && ldx < (1ll << 22);
+}
+
+static DTallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, int64_t K, int64_t N, void* scratch) {
     DTallArgs a{};
     a.x = x;
     a.ldx = ldx;
     a.prep = (const uint8_t*)prepared;
-    a.bias = bias;
-    a.out = out;
-    a.ldo = ldo;
     a.M = (int)M;
     a.K = (int)K;
     a.N = (int)N;
     a.NT = (int)cdiv64(N, 32);
+    a.scratch = (float*)scratch;
+    return a;
+}
+
+// out = act(x @ w^T + bias) in the model dtype, or (act 0) in fp32.  act 0; 4 / 5: GELU (erf / tanh) of the rounded sum; 2: SiLU(gate) * up of a gate | up image
+// (out [M, N / 2]), or with glu_limit > 0 the clamped unit (DenseArgs::glu_limit).
+extern "C" int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared, const void* bias, void* out, int64_t ldo, int64_t M, int64_t K,
+                               int64_t N, int dtype, int out_f32, int act, float glu_alpha, float glu_limit, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
+    TGIS_CHECK_ARG(x && prepared && out && M >= 0 && K >= 64 && K % 64 == 0 && N >= 1, "tgis_dense_tall: bad arguments");
+    TGIS_CHECK_ARG((dtype == TGIS_F16 || dtype == TGIS_BF16) && (act == 0 || act == 2 || act == 4 || act == 5), "tgis_dense_tall: bad dtype or act");
+    TGIS_CHECK_ARG(!out_f32 || act == 0, "tgis_dense_tall: activations are written in the model dtype");
+    TGIS_CHECK_ARG(act != 2 || N % 32 == 0, "tgis_dense_tall: act 2 needs a gate|up image (N / 2 a multiple of 16)");
+    TGIS_CHECK_ARG(rows_ok(x, ldx, K), "tgis_dense_tall: x rows must be 16-byte aligned and less than 2^22 elements apart");
+    if (M == 0) return TGIS_OK;
+    const TallPlan p = plan_tall(M, K, N);
+    TGIS_CHECK_ARG(plan_scratch(p) == 0 || (workspace && workspace_bytes >= plan_scratch(p)), "tgis_dense_tall: workspace too small");
+    DTallArgs a = tall_args(x, ldx, prepared, M, K, N, workspace);
+    a.bias = bias;
+    a.out = out;
+    a.ldo = ldo;
     a.gelu = act == 4 ? 1 : act == 5 ? 2 : 0;
     a.glu_alpha = glu_alpha;
     a.glu_limit = glu_limit;
+    a.out_f32 = out_f32;
     a.vec = ldo % 8 == 0 && (uintptr_t)out % 16 == 0;
     a.col_blocks = p.col_blocks;
-    a.scratch = (float*)workspace;
     const hipStream_t st = (hipStream_t)stream;
     TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
     return dtype == TGIS_F16 ? run_tall<f16>(p, a, act == 2 ? 2 : 0, st) : run_tall<bf16>(p, a, act == 2 ? 2 : 0, st);
+}
+
+// The product as fp32 partial sums for the consumers of tgis_dense_gemm_partial's, in the same layout; up to 256 rows.
+extern "C" int64_t tgis_dense_tall_partial_bytes(int64_t M, int64_t K, int64_t N) {
+    if (M > 256 || tgis_dense_tall_bytes(M, K, N, 0) < 0) return -1;
+    return cdiv64(M, 32) * 32 * cdiv64(N, 32) * 32 * 4 * plan_parts(M, K, N).S;
+}
+
+extern "C" int tgis_dense_tall_partial(const void* x, int64_t ldx, const void* prepared, int64_t M, int64_t K, int64_t N, int dtype, float* slabs,
+                                       int64_t slabs_bytes, int* num_slabs, int64_t* slab_ld, void* stream) {
+    TGIS_CHECK_ARG(x && prepared && slabs && M >= 1 && M <= 256 && K >= 64 && K % 64 == 0 && N >= 1, "tgis_dense_tall_partial: bad arguments");
+    TGIS_CHECK_ARG(dtype == TGIS_F16 || dtype == TGIS_BF16, "tgis_dense_tall_partial: bad dtype");
+    TGIS_CHECK_ARG(rows_ok(x, ldx, K), "tgis_dense_tall_partial: x rows must be 16-byte aligned and less than 2^22 elements apart");
+    const TallPlan p = plan_parts(M, K, N);
+    TGIS_CHECK_ARG(slabs_bytes >= cdiv64(M, 32) * 32 * cdiv64(N, 32) * 32 * 4 * p.S, "tgis_dense_tall_partial: slab buffer too small");
+    if (num_slabs) *num_slabs = p.S;
+    if (slab_ld) *slab_ld = cdiv64(N, 32) * 32;
+    DTallArgs a = tall_args(x, ldx, prepared, M, K, N, slabs);
+    a.col_blocks = p.col_blocks;
+    a.per = p.per;
+    a.S = p.S;
+    a.part = 2;
+    const hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
+    return dtype == TGIS_F16 ? launch_shape<f16, 0>(p, a, p.tiles, p.S, st) : launch_shape<bf16, 0>(p, a, p.tiles, p.S, st);
 }

@@ -186,8 +186,10 @@ class FlashLlamaAttention:
             # one launch: GEMM + rotary embedding + cache write (native.gptq_gemm_rope / native.dense_gemm_rope)
             fused = native.gptq_gemm_rope if isinstance(rope_w, native.GptqWeight) else native.dense_gemm_rope
             return fused(hidden_states, rope_w, lin.bias, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D)
-        # [T, (H + 2 Hkv) D]; at decode sizes the split-K sum of the GPTQ GEMM is finished inside the rope kernel
-        qkv = self.query_key_value(hidden_states, partial=True, **({"gathered": True} if gathered else {}))
+        # [T, (H + 2 Hkv) D]; at decode sizes the split-K sum of the GPTQ GEMM is finished inside the rope kernel; whole prompts on the dense
+        # prefill kernel take the finished sum, and with it the page-wise cache writes
+        whole = kv.fresh_prefill and isinstance(lin, FastLinear) and lin.tall(hidden_states) >= 0
+        qkv = self.query_key_value(hidden_states, partial=not whole, **({"gathered": True} if gathered else {}))
         if kv.fresh_prefill and not isinstance(qkv, native.Partial):
             return native.rope_kv_write_prefill(qkv, cos, sin, position_ids, cu_seqlens_q, kv.block_tables, k_pool, v_pool,
                                                 kv.max_q_len, H, Hkv, D, D)

@@ -201,7 +201,9 @@ SIGNATURES = {
     "tgis_moe_choose": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_f, _vp, _vp, _vp]),
     "tgis_relu2": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_tall_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int]),
-    "tgis_dense_tall": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_f, _c_f, _vp, _c_i64, _vp]),
+    "tgis_dense_tall": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_f, _c_f, _vp, _c_i64, _vp]),
+    "tgis_dense_tall_partial_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "tgis_dense_tall_partial": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp, _vp, _vp]),
     "tgis_dense_gemm_whole_operand": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
@@ -681,29 +683,52 @@ def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f3
     return out
 
 
-DENSE_TALL_MIN_M = 65
+DENSE_TALL_MIN_M = 65  # TGIS_DENSE_TALL_MIN_M
 
 
-def dense_tall_pays(x: torch.Tensor, w: DenseWeight, act: int = 0) -> bool:
-    """Is dense_tall the faster way to x @ w^T?  (a size query; x as it reads it)"""
+def dense_tall_bytes(x: torch.Tensor, w: DenseWeight, act: int = 0) -> int:
+    """The scratch of dense_tall where it is the faster way to x @ w^T, -1 where it is not or x is not as it reads it (a size query)."""
     M, ld = x.shape[0], x.stride(0)
-    return (M >= DENSE_TALL_MIN_M and x.stride(1) == 1 and ld % 8 == 0 and w.K <= ld < 1 << 22 and x.data_ptr() % 16 == 0
-            and load_library().tgis_dense_tall_bytes(M, w.K, w.N, act) >= 0)
+    if M < DENSE_TALL_MIN_M or x.stride(1) != 1 or ld % 8 or not w.K <= ld < 1 << 22 or x.data_ptr() % 16:
+        return -1
+    if M > PARTIAL_MAX_M:
+        return load_library().tgis_dense_tall_bytes(M, w.K, w.N, act)
+    got = w.plans.get((M, act))
+    if got is None:
+        got = w.plans[(M, act)] = load_library().tgis_dense_tall_bytes(M, w.K, w.N, act)
+    return got
 
 
-def dense_tall(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, act: int = 0, alpha: float = 0.0, limit: float = 0.0, out=None) -> torch.Tensor:
-    """dense_gemm of a prefill's rows; act 0, 4, 5 or 2 (limit > 0: the clamped unit of dense_gemm_clamped_glu)."""
-    assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K
-    assert (act == 2) == bool(w.flags & 1) and not w.flags & 2
+def dense_tall(x: torch.Tensor, w: DenseWeight, ws: Workspace, nbytes: int, bias=None, act: int = 0, alpha: float = 0.0, limit: float = 0.0,
+               out=None, out_f32: bool = False) -> torch.Tensor:
+    """dense_gemm of a prefill's rows (nbytes: dense_tall_bytes); act 0, 4, 5 or 2 (limit > 0: the clamped unit of dense_gemm_clamped_glu)."""
     M = x.shape[0]
     if out is None:
-        out = torch.empty((M, w.N // 2 if act == 2 else w.N), dtype=w.dtype, device=x.device)
-    lib = load_library()
-    nbytes = lib.tgis_dense_tall_bytes(M, w.K, w.N, act)
-    ws.ensure(4096 + max(nbytes, 0))  # (the first page holds the arrival counters of other launches)
-    _check(lib.tgis_dense_tall(_ptr(x), x.stride(0), _ptr(w.image), _ptr(bias), _ptr(out), out.stride(0), M, w.K, w.N, dtype_code(w.dtype), act,
-                               float(alpha), float(limit), ws.ptr + 4096, ws.nbytes - 4096, _stream()), "tgis_dense_tall")
+        out = torch.empty((M, w.N // 2 if act == 2 else w.N), dtype=torch.float32 if out_f32 else w.dtype, device=x.device)
+    assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K
+    assert (act == 2) == bool(w.flags & 1) and not w.flags & 2
+    ws.ensure(4096 + nbytes)  # (the first page holds the arrival counters of other launches)
+    _check(load_library().tgis_dense_tall(_ptr(x), x.stride(0), _ptr(w.image), _ptr(bias), _ptr(out), out.stride(0), M, w.K, w.N, dtype_code(w.dtype),
+                                          int(out_f32), act, alpha, limit, ws.ptr + 4096, ws.nbytes - 4096, _stream()), "tgis_dense_tall")
     return out
+
+
+def dense_tall_partial(x: torch.Tensor, w: DenseWeight, bias=None) -> Partial:
+    """dense_gemm_partial of up to PARTIAL_MAX_M rows, where dense_tall_bytes says so."""
+    assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K and not w.flags
+    lib, M = load_library(), x.shape[0]
+    plan = w.plans.get(("tall slabs", M))
+    nbytes = plan[0] if plan is not None else lib.tgis_dense_tall_partial_bytes(M, w.K, w.N)
+    slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+    S, ld = (None, None) if plan is not None else (_c_int(), _c_i64())
+    _check(lib.tgis_dense_tall_partial(_ptr(x), x.stride(0), _ptr(w.image), M, w.K, w.N, dtype_code(w.dtype), _ptr(slabs), nbytes,
+                                       None if S is None else ctypes.byref(S), None if ld is None else ctypes.byref(ld), _stream()),
+           "tgis_dense_tall_partial")
+    if plan is None:
+        plan = w.plans[("tall slabs", M)] = (nbytes, S.value, ld.value)
+    p = Partial(slabs, plan[1], plan[2], M, w.N, bias)
+    p.dtype = w.dtype
+    return p
 
 
 def dense_gemm_partial(x: torch.Tensor, w: DenseWeight, bias=None, act: int = 0) -> Partial:

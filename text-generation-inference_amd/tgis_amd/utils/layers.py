@@ -20,7 +20,7 @@ from tgis_amd.utils.graph_segments import collective
 import os
 
 # rows up to which the dense weight-streaming MFMA kernel is used (one pass over the weights per 32 / 64 rows); above,
-# hipBLASLt; from 65 rows on the prefill kernel on the same image where it is faster than either (native.dense_tall_pays).
+# hipBLASLt; from 65 rows on the prefill kernel on the same image where it is faster than either (native.dense_tall_bytes).
 # GPTQ linears ask the library how far its fused kernels reach (GptqWeight.fused_rows: 64-row streaming passes
 # to 256 rows, the tall kernel from 65 / 129 rows to 8192 where it is faster; else dequantise once + hipBLASLt, exllamav2.py:87).
 SKINNY_MAX_M = int(os.getenv("TGIS_SKINNY_MAX_M", "256"))
@@ -94,9 +94,10 @@ class FastLinear:
             if any(native.rope_gemm_ok(m, self.prepared, D) for m in (1, 32, 64)):
                 self.rope_handle = native.DenseWeight(self.weight, rope=(D, H + Hkv))
 
-    def takes_tall(self, x: torch.Tensor, act: int = 0) -> bool:
-        """Does the prefill kernel on the image serve this step, and sooner than the weight-streaming kernel or the library GEMM would?"""
-        return self.streams and x.shape[0] >= native.DENSE_TALL_MIN_M and native.dense_tall_pays(x, self.prepared, act)
+    def tall(self, x: torch.Tensor, act: int = 0) -> int:
+        """The scratch of the prefill kernel on the image where it serves this step, and sooner than the weight-streaming kernel or the library
+        GEMM would; else -1."""
+        return native.dense_tall_bytes(x, self.prepared, act) if x.shape[0] >= native.DENSE_TALL_MIN_M and self.streams else -1
 
     def forward(self, x: torch.Tensor, act: int = 0, out_f32: bool = False, partial: bool = False,
                 gelu: Optional[bool] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -106,8 +107,9 @@ class FastLinear:
         if out is not None:
             # the caller's buffer (a [M, N] view with unit column stride): plain projections only
             assert not act and not out_f32 and not partial and gelu is None and not self._gate_up and self.bias is None
-            if self.takes_tall(x):
-                return native.dense_tall(x, self.prepared, workspace(x.device), out=out)
+            tall = self.tall(x)
+            if tall >= 0:
+                return native.dense_tall(x, self.prepared, workspace(x.device), tall, out=out)
             if self.streams and x.shape[0] <= SKINNY_MAX_M:
                 return native.dense_gemm(x, self.prepared, workspace(x.device), out=out)
             if out.is_contiguous():
@@ -122,21 +124,27 @@ class FastLinear:
             return out.float() if out_f32 else out
         if gelu is not None:
             assert act == 0 and not out_f32 and not partial and not self._gate_up
-            if FUSED_GELU_GEMM and self.takes_tall(x, 5 if gelu else 4):
-                return native.dense_tall(x, self.prepared, workspace(x.device), bias=self.bias, act=5 if gelu else 4)
+            tall = self.tall(x, 5 if gelu else 4) if FUSED_GELU_GEMM else -1
+            if tall >= 0:
+                return native.dense_tall(x, self.prepared, workspace(x.device), tall, bias=self.bias, act=5 if gelu else 4)
             if x.shape[0] <= SKINNY_MAX_M and FUSED_GELU_GEMM:
                 return native.dense_gemm(x, self.prepared, workspace(x.device), bias=self.bias, act=5 if gelu else 4)
             return native.gelu(self.forward(x), gelu)
         if self._gate_up:
             # output is the activated [M, I] tensor
-            if self.takes_tall(x, 2):
-                return native.dense_tall(x, self.prepared, workspace(x.device), bias=self.bias, act=2)
+            tall = self.tall(x, 2)
+            if tall >= 0:
+                return native.dense_tall(x, self.prepared, workspace(x.device), tall, bias=self.bias, act=2)
             if x.shape[0] <= SKINNY_MAX_M:
                 return native.dense_gemm(x, self.prepared, workspace(x.device), bias=self.bias, act=2)
             return native.act_mul(F.linear(x, self.weight, self.bias), self.out_features // 2)
-        if not act and not out_f32 and self.takes_tall(x):
-            return native.dense_tall(x, self.prepared, workspace(x.device), bias=self.bias)
-        if partial and x.shape[0] <= native.PARTIAL_MAX_M and DEFER_REDUCE and not out_f32:
+        defers = partial and x.shape[0] <= native.PARTIAL_MAX_M and DEFER_REDUCE and not out_f32
+        tall = self.tall(x) if not act and (not out_f32 or x.shape[0] <= SKINNY_MAX_M) else -1
+        if tall >= 0:
+            if defers:
+                return native.dense_tall_partial(x, self.prepared, bias=self.bias)
+            return native.dense_tall(x, self.prepared, workspace(x.device), tall, bias=self.bias, out_f32=out_f32)
+        if defers:
             # the split-K sum (and the bias) is finished by the consumer kernel (add+norm / rope): no reduce launch
             return native.dense_gemm_partial(x, self.prepared, bias=self.bias, act=act)
         if x.shape[0] <= SKINNY_MAX_M:

@@ -200,8 +200,9 @@ class GatedUnit:
         partial = partial and can_defer(self.down)
         if self.fused:
             return self.down(self.gate_up(h), partial=partial)
-        if self.clamped_image is not None and native.dense_tall_pays(h, self.clamped_image, 2):
-            act = native.dense_tall(h, self.clamped_image, workspace(h.device), bias=self.gate_up.bias, act=2, alpha=self.alpha, limit=self.limit)
+        tall = native.dense_tall_bytes(h, self.clamped_image, 2) if self.clamped_image is not None else -1
+        if tall >= 0:
+            act = native.dense_tall(h, self.clamped_image, workspace(h.device), tall, bias=self.gate_up.bias, act=2, alpha=self.alpha, limit=self.limit)
             return self.down(act, partial=partial)
         if self.clamped_image is not None and h.shape[0] <= CLAMPED_EPILOGUE_MAX_M:
             act = native.dense_gemm_clamped_glu(h, self.clamped_image, workspace(h.device), self.alpha, self.limit)
