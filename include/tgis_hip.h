@@ -182,6 +182,32 @@ int tgis_dense_tall_partial(const void* x, int64_t ldx, const void* prepared, in
 
 #define TGIS_DENSE_TALL_MIN_M 65
 
+/* The layers of a dense Llama model (no biases but qkv's, one rank) on T rows of prompts: the launches of its forward, one call.  Images as
+ * tgis_dense_prepare makes them; qkv_rope is the rope image, for T < TGIS_DENSE_TALL_MIN_M, where tgis_dense_rope_ok must hold; qkv the plain
+ * one, for more rows, where tgis_dense_tall_bytes of the four products must not be negative. */
+typedef struct {
+    const void *input_norm, *qkv, *qkv_rope, *qkv_bias, *o, *post_norm, *gate_up, *down;
+    void *k_pool, *v_pool;
+} TgisLlamaLayer;
+typedef struct {
+    int64_t T, hidden, inner, B, max_pages, max_q_len, max_ctx;
+    int H, Hkv, D, dtype, fresh; /* fresh: token i of a sequence is cache position i */
+    float eps, scale;
+    const void* x; /* [T][hidden] */
+    const int32_t *positions, *slots, *cu_seqlens, *block_tables, *ctx_lens;
+    const void *cos, *sin;
+    void *y, *res[2];      /* [T][hidden]; the residual stream is left in res[0] */
+    void *qkv, *att, *act; /* [T][(H + 2 Hkv) D], [T][H D], [T][inner] */
+    float* slabs;          /* up to 256 rows: the last product is left here, num_slabs partial sums (tgis_rmsnorm_residual_partial) */
+    int64_t slabs_bytes;
+    void* out;             /* more rows: [T][hidden], the last product (slabs NULL) */
+    void* workspace;
+    int64_t workspace_bytes;
+    int64_t slab_ld;       /* set by the call */
+    int num_slabs;
+} TgisLlamaPrompt;
+int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, TgisLlamaPrompt* prompt, void* stream);
+
 /* Decode steps of up to 4 rows: dense products that norm their operand themselves and add to the residual stream, which stays in fp32
  * (h, [M][width], rows back to back) between them.  With norm(h)[k] = T(h[k] * rstd * norm_w[k]), norm_w of the model dtype, and the images of
  * tgis_dense_prepare:

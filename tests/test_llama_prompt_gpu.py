@@ -1,0 +1,73 @@
+"""-m gpu: a dense Llama model's layers on prompts, launched in one call, against the same launches one by one: the same bits in the logits and in
+the pages; and the models and steps that go on one by one."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def model(dtype, **kw):
+    from oracle.tiny_models import TinyLlamaConfig, tiny_llama_tensors
+    from tgis_amd.inference_engine.synthetic import InferenceEngine
+    from tgis_amd.models.custom_modeling.flash_llama_modeling import LlamaConfig
+    from tgis_amd.models.flash_causal_lm import FlashCausalLM
+    from tgis_amd.testing import SyntheticTokenizer
+
+    quantize = kw.pop("quantize", None)
+    cfg = TinyLlamaConfig(**{**dict(hidden_size=2048, intermediate_size=1024, num_attention_heads=32, num_key_value_heads=4, num_hidden_layers=3), **kw})
+    tensors = {k: v.to(dtype) if v.is_floating_point() else v for k, v in tiny_llama_tensors(cfg, seed=7, quantize=quantize, groupsize=64).items()}
+    config = LlamaConfig(**cfg.to_dict())
+    eng = InferenceEngine(tensors, config, dtype, quantize, tokenizer=SyntheticTokenizer(config.vocab_size), gptq_groupsize=64)
+    return FlashCausalLM("synthetic", None, "synthetic", dtype, quantize, engine=eng, kv_cache_pages=64), config
+
+
+def steps(lm, vocab, lens):
+    """Prompts whole; the logits of every token, of the ends alone, and the pages left."""
+    g = torch.Generator().manual_seed(11)
+    pages = [lm.kv_cache.alloc(n // 32 + 1) for n in lens]
+    last = (torch.tensor(lens).cumsum(0) - 1).cuda()
+    ids = torch.randint(3, vocab, (sum(lens),), generator=g).cuda()
+    for i in range(lm.num_layers):
+        for pool in (lm.kv_cache.k_pool(i), lm.kv_cache.v_pool(i)):
+            pool.zero_()  # (what lies behind a sequence's last token is either left or cleared)
+    with lm.context_manager():
+        out = [lm.ragged_forward(ids, pages, [0] * len(lens), lens),
+               lm.ragged_forward(ids, pages, [0] * len(lens), lens, lm_head_indices=last, ends_only=True)]
+        flat = torch.tensor([p for seq in pages for p in seq])
+        for i in range(lm.num_layers):
+            out += [pool.view(64, -1)[flat.cuda()].clone() for pool in (lm.kv_cache.k_pool(i), lm.kv_cache.v_pool(i))]
+    for p in pages:
+        lm.kv_cache.free(p)
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_same_bits(gpu_device, monkeypatch, dtype):
+    from tgis_amd import native
+    from tgis_amd.models.custom_modeling.flash_llama_modeling import FlashLlamaModel
+
+    lm, cfg = model(dtype)
+    calls, run = [], native.llama_prompt
+    monkeypatch.setattr(native, "llama_prompt", lambda layers, x, *a, **k: calls.append((len(layers), x.shape[0])) or run(layers, x, *a, **k))
+    for lens in ([1], [2], [47], [13, 1, 50], [65], [40, 30], [37, 1, 70, 33], [200, 57]):
+        del calls[:]
+        got = steps(lm, cfg.vocab_size, lens)
+        assert calls[0] == (3, sum(lens)) and calls[1] == (2 if sum(lens) >= 128 else 3, sum(lens)), calls
+        with monkeypatch.context() as m:
+            m.setattr(FlashLlamaModel, "plain_layers", lambda self, *a: [])
+            want = steps(lm, cfg.vocab_size, lens)
+        assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want)), lens
+
+
+@pytest.mark.parametrize("kw,lens", [(dict(quantize="gptq"), [20]), (dict(hidden_size=256, num_attention_heads=4), [70]),
+                                     (dict(), [1500])])
+def test_one_by_one(gpu_device, monkeypatch, kw, lens):
+    """int4 layers, products too narrow for the prefill kernel, rows past its rule."""
+    from tgis_amd import native
+
+    lm, cfg = model(torch.float16, **kw)
+    monkeypatch.setattr(native, "llama_prompt", lambda *a, **k: pytest.fail("served"))
+    pages = [lm.kv_cache.alloc(n // 32 + 1) for n in lens]
+    with lm.context_manager():
+        logits = lm.ragged_forward(torch.full((sum(lens),), 5).cuda(), pages, [0] * len(lens), lens)
+    assert bool(torch.isfinite(logits).all())

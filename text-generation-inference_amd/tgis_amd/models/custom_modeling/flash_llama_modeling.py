@@ -19,12 +19,15 @@ import torch
 
 from tgis_amd import native
 from tgis_amd.utils.layers import (
+    DEFER_REDUCE,
+    SKINNY_MAX_M,
     FastLinear,
     PositionRotaryEmbedding,
     TensorParallelColumnLinear,
     TensorParallelEmbedding,
     TensorParallelHead,
     TensorParallelRowLinear,
+    workspace,
 )
 
 
@@ -353,6 +356,38 @@ class FlashLlamaModel:
             native.dense_rows_residual(act, mlp.down_proj.linear.prepared, h)
         return h
 
+    def plain_layers(self, count: int, x, cos, kv: KVArgs) -> list:
+        """The weights and cache pages of the first `count` layers, as native.llama_prompt takes them, if a step of x's rows is a prompt's and
+        each of its products one that the launches there serve; else nothing."""
+        rows, hidden = x.shape
+        att, mlp = self.layers[0].self_attn, self.layers[0].mlp
+        H, Hkv, D, inner = att.num_heads, att.num_key_value_heads, att.head_size, mlp.intermediate_size
+        if ((kv.max_q_len == 1 and not kv.fresh_prefill) or kv.num_splits != 1 or kv.slots is None or kv.residual_trace is not None or not rows
+                or self.tp_world_size != 1 or cos.shape[1] * 2 != D or not x.is_contiguous()):
+            return []
+        tall = rows >= native.DENSE_TALL_MIN_M
+        shapes = {"qkv": ((H + 2 * Hkv) * D, hidden), "o": (hidden, H * D), "gate_up": (2 * inner, hidden), "down": (hidden, inner)}
+        if tall and not all(native.dense_tall_serves(rows, K, N, 2 if name == "gate_up" else 0) for name, (N, K) in shapes.items()):
+            return []
+        if not tall and not (DEFER_REDUCE and rows <= SKINNY_MAX_M):
+            return []
+        got = []
+        for layer in self.layers[:count]:
+            att, mlp = layer.self_attn, layer.mlp
+            lin = {"qkv": att.query_key_value.linear, "o": att.o_proj.linear, "gate_up": mlp.gate_up_proj.linear, "down": mlp.down_proj.linear}
+            for name, (N, K) in shapes.items():
+                w = lin[name]
+                if not (isinstance(w, FastLinear) and w.streams and (w.out_features, w.in_features) == (N, K) and w.weight.dtype == x.dtype
+                        and w.gate_up == (name == "gate_up") and (w.bias is None or name == "qkv")):
+                    return []
+            qkv = lin["qkv"]
+            if not tall and (qkv.rope_handle is None or not native.rope_gemm_ok(rows, qkv.rope_handle, D)):
+                return []
+            got.append((layer.input_layernorm.weight, qkv.prepared.image, None if qkv.rope_handle is None else qkv.rope_handle.image, qkv.bias,
+                        lin["o"].prepared.image, layer.post_attention_layernorm.weight, lin["gate_up"].prepared.image, lin["down"].prepared.image,
+                        kv.cache.k_pool(layer.layer_id), kv.cache.v_pool(layer.layer_id)))
+        return got
+
     def forward(self, input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv: KVArgs):
         if input_ids is not None and inputs_embeds is not None:
             raise ValueError("You cannot specify both input_ids and inputs_embeds at the same time")
@@ -360,7 +395,14 @@ class FlashLlamaModel:
         cos, sin = self.rope_tables(hidden_states.dtype, hidden_states.device, max_s)
         residual = None
         whole = len(self.layers) - kv.cuts_to_ends(hidden_states.shape[0])
-        for layer in self.layers[:whole]:
+        plain = self.plain_layers(whole, hidden_states, cos, kv)
+        if plain:
+            att = self.layers[0].self_attn
+            hidden_states, residual = native.llama_prompt(
+                plain, hidden_states, workspace(hidden_states.device), position_ids, kv.slots, cu_seqlens_q, kv.block_tables, kv.ctx_lens, cos, sin,
+                att.num_heads, att.num_key_value_heads, att.head_size, self.layers[0].mlp.intermediate_size, kv.max_q_len, kv.max_ctx,
+                kv.fresh_prefill, self.layers[0].input_layernorm.variance_epsilon, att.softmax_scale)
+        for layer in self.layers[len(plain):whole]:
             hidden_states, residual = layer(hidden_states, residual, cos, sin, position_ids, cu_seqlens_q, kv)
         for layer in self.layers[whole:]:
             hidden_states, residual = layer.forward_ends(hidden_states, residual, cos, sin, position_ids, cu_seqlens_q, kv)

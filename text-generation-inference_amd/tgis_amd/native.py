@@ -204,6 +204,7 @@ SIGNATURES = {
     "tgis_dense_tall": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_f, _c_f, _vp, _c_i64, _vp]),
     "tgis_dense_tall_partial_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "tgis_dense_tall_partial": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp, _vp, _vp]),
+    "tgis_llama_prompt": (_c_int, [_vp, _c_int, _vp, _vp]),
     "tgis_dense_gemm_whole_operand": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
@@ -686,6 +687,10 @@ def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f3
 DENSE_TALL_MIN_M = 65  # TGIS_DENSE_TALL_MIN_M
 
 
+def dense_tall_serves(M: int, K: int, N: int, act: int = 0) -> bool:
+    return load_library().tgis_dense_tall_bytes(M, K, N, act) >= 0
+
+
 def dense_tall_bytes(x: torch.Tensor, w: DenseWeight, act: int = 0) -> int:
     """The scratch of dense_tall where it is the faster way to x @ w^T, -1 where it is not or x is not as it reads it (a size query)."""
     M, ld = x.shape[0], x.stride(0)
@@ -813,6 +818,55 @@ def dense_rows_head(h, norm_w, eps: float, w: DenseWeight) -> torch.Tensor:
     _check(load_library().tgis_dense_rows_norm_head(_rows_stream(h, w.K), _ptr(norm_w), float(eps), _ptr(w.image), _ptr(out), out.stride(0),
                                                     h.shape[0], w.K, w.N, dtype_code(w.dtype), _stream()), "tgis_dense_rows_norm_head")
     return out
+
+
+LLAMA_LAYER_POINTERS = ("input_norm", "qkv", "qkv_rope", "qkv_bias", "o", "post_norm", "gate_up", "down", "k_pool", "v_pool")
+
+
+class _LlamaPrompt(ctypes.Structure):
+    _fields_ = ([(n, _c_i64) for n in ("T", "hidden", "inner", "B", "max_pages", "max_q_len", "max_ctx")]
+                + [(n, _c_int) for n in ("H", "Hkv", "D", "dtype", "fresh")] + [("eps", _c_f), ("scale", _c_f), ("x", _vp)]
+                + [(n, _vp) for n in ("positions", "slots", "cu_seqlens", "block_tables", "ctx_lens", "cos", "sin", "y", "res0", "res1", "qkv", "att", "act", "slabs")]
+                + [("slabs_bytes", _c_i64), ("out", _vp), ("workspace", _vp), ("workspace_bytes", _c_i64), ("slab_ld", _c_i64), ("num_slabs", _c_int)])
+
+
+def llama_prompt(layers, x, ws: Workspace, positions, slots, cu_seqlens, block_tables, ctx_lens, cos, sin, H: int, Hkv: int, D: int, inner: int,
+                 max_q_len: int, max_ctx: int, fresh: bool, eps: float, scale: float):
+    """The layers of a dense Llama model on a prompt's rows in one call; layers: LLAMA_LAYER_POINTERS of each (DenseWeight images, tensors or
+    None).  Returns what the last layer returns: (hidden states, a Partial up to PARTIAL_MAX_M rows, and the residual stream)."""
+    lib = load_library()
+    T, hidden = x.shape
+    assert x.is_contiguous() and block_tables.is_contiguous() and cos.shape[1] * 2 == D and cos.dtype == x.dtype
+    assert all(t.dtype == torch.int32 for t in (positions, slots, cu_seqlens, block_tables, ctx_lens))
+    pointers = [None if t is None else t.data_ptr() for layer in layers for t in layer]
+    table = (_vp * len(pointers))(*pointers)
+    tall = T >= DENSE_TALL_MIN_M
+    qkv_cols = (H + 2 * Hkv) * D
+    new = lambda cols: torch.empty((T, cols), dtype=x.dtype, device=x.device)
+    y, res0, res1, qkv, att, act = new(hidden), new(hidden), new(hidden), new(qkv_cols), new(H * D), new(inner)
+    out = slabs = None
+    nbytes = 0
+    if tall:
+        if T <= PARTIAL_MAX_M:
+            nbytes = max(lib.tgis_dense_tall_partial_bytes(T, K, hidden) for K in (H * D, inner))
+        else:
+            out = new(hidden)
+        ws.ensure(4096 + max(lib.tgis_dense_tall_bytes(T, K, N, a) for K, N, a in
+                             ((hidden, qkv_cols, 0), (H * D, hidden, 0), (hidden, 2 * inner, 2), (inner, hidden, 0))))
+    else:
+        nbytes = max(lib.tgis_dense_gemm_partial_bytes(T, K, hidden) for K in (H * D, inner))
+        ws.ensure(lib.tgis_dense_gemm_workspace_bytes(T, hidden, 2 * inner))
+    if out is None:
+        slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+    p = _LlamaPrompt(T, hidden, inner, block_tables.shape[0], block_tables.shape[1], max_q_len, max_ctx, H, Hkv, D, dtype_code(x.dtype), int(fresh),
+                     eps, scale, _ptr(x), _ptr(positions), _ptr(slots), _ptr(cu_seqlens), _ptr(block_tables), _ptr(ctx_lens), _ptr(cos), _ptr(sin),
+                     _ptr(y), _ptr(res0), _ptr(res1), _ptr(qkv), _ptr(att), _ptr(act), _ptr(slabs), nbytes, _ptr(out), ws.ptr, ws.nbytes)
+    _check(lib.tgis_llama_prompt(table, len(layers), ctypes.byref(p), _stream()), "tgis_llama_prompt")
+    if out is not None:
+        return out, res0
+    last = Partial(slabs, p.num_slabs, p.slab_ld, T, hidden, None)
+    last.dtype = x.dtype
+    return last, res0
 
 
 def clear_error() -> None:
