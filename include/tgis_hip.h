@@ -443,6 +443,12 @@ int tgis_qk_norm_kv_write(void* qkv, int64_t ld, const int32_t* positions, const
                           const float* k_gain, float eps, float gain_coef, int gain_every, const void* v_first,
                           int64_t ld_v_first, const float* v_lambda, void* k_pool, void* v_pool, int64_t T, int H, int G,
                           int dk, int dv, int dtype, void* stream);
+/* ... of a projection without a bias that was left as partial sums (tgis_dense_gemm_partial); two-byte dtypes, dk even and <= 256.  qkv receives
+ * their sum in the model dtype, the q heads normed. */
+int tgis_qk_norm_kv_write_partial(const float* slabs, int num_slabs, int64_t slab_ld, void* qkv, int64_t ld, const int32_t* positions,
+                                  const int32_t* slots, const float* q_gain, const float* k_gain, float eps, float gain_coef, int gain_every,
+                                  const void* v_first, int64_t ld_v_first, const float* v_lambda, void* k_pool, void* v_pool, int64_t T,
+                                  int H, int G, int dk, int dv, int dtype, void* stream);
 /* out[t][h][:] = softmax_j(scale q[t][h] . k[j]) v[j] over keys j <= the token's position, fp32 scores and weights;
  * query head h reads kv head h / (H / G).  max_q_len / max_ctx: upper bounds of a sequence's run in this step and of
  * ctx_lens (launch shaping only).  impl 0: the matrix-core kernel where it applies (two-byte dtype, dk % 16 == 0,

@@ -40,3 +40,36 @@ def test_long_step(gpu_device, H, G, dk, dv, pad, dtype):
     unused = torch.ones(pages * PAGE, dtype=torch.bool)
     unused[slots.long()] = False
     assert (k_pool.cpu().transpose(1, 2).reshape(pages * PAGE, -1)[unused] == 7).all()
+
+
+# heads of one and two halves of a wave's channels; rows on both sides of a slab block; values of one block and more
+@pytest.mark.parametrize("T,S,H,G,dk,dv", [(1, 1, 4, 2, 64, 64), (24, 4, 32, 4, 64, 64), (33, 3, 3, 1, 130, 18), (70, 8, 6, 3, 72, 512), (256, 2, 5, 5, 256, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("blend", [False, True])
+def test_of_partial_sums(gpu_device, T, S, H, G, dk, dv, dtype, blend):
+    """The projection left as partial sums: the bits of their sum, added in order and rounded, and then normed and written."""
+    from tgis_amd import native
+
+    N, PAGE = (H + G) * dk + G * dv, 32
+    g = torch.Generator().manual_seed(T + S)
+    ld, blocks = -N // 32 * -32, -T // 32 * -1
+    slabs = torch.randn(blocks, S, 32, ld, generator=g).to(gpu_device)
+    part = native.Partial(slabs, S, ld, T, N, None)
+    part.dtype = dtype
+    total = slabs[:, 0]
+    for s in range(1, S):
+        total = total + slabs[:, s]
+    whole = total.reshape(-1, ld)[:T, :N].to(dtype).contiguous()
+    qw, kw = (torch.rand(dk, generator=g) + 0.5).to(gpu_device), (torch.rand(dk, generator=g) + 0.5).to(gpu_device)
+    pages = T // PAGE + 3
+    slots, pos = torch.randperm(pages * PAGE, generator=g)[:T].int().to(gpu_device), torch.randint(0, 5000, (T,), generator=g).int().to(gpu_device)
+    first = torch.randn(T, G * dv, generator=g).to(dtype).to(gpu_device) if blend else None
+    lam = torch.tensor([0.375], device=gpu_device) if blend else None
+
+    def run(x):
+        k_pool = torch.full((pages, G, PAGE, dk), 7.0, dtype=dtype, device=gpu_device)
+        v_pool = torch.full((pages, G, dv, PAGE), 7.0, dtype=dtype, device=gpu_device)
+        out = native.qk_norm_kv_write(x, pos, slots, qw, kw, 1e-5, 0.1, 1024, first, lam, k_pool, v_pool, H, G, dk, dv)
+        return out, k_pool, v_pool
+
+    assert all(torch.equal(a, b) for a, b in zip(run(part), run(whole)))

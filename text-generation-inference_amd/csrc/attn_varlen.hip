@@ -191,6 +191,81 @@ __global__ __launch_bounds__(256) void qk_norm_kv_write_kernel(
     for (int d = lane; d < dk; d += 64) dst[d] = (T)(ldf(p + d) * rinv * w[d]);
 }
 
+// The same on a projection that was left as S partial sums (tgis_dense_gemm_partial): each is added here, in the order and with the rounding
+// of the launch that would add them, and q, the values and k as it came land in qkv as from there.  Short steps are launches that wait: 24
+// rows of 36 heads of 64 were 4.8 us to add and 4.7 to norm, 3.8 together.
+template <typename T>
+__global__ __launch_bounds__(256) void qk_norm_kv_sum_kernel(
+    const float* __restrict__ slabs, int S, int64_t sld, T* __restrict__ qkv, int64_t ld, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ slots, const float* __restrict__ qw, const float* __restrict__ kw, float eps, float gain_coef, int gain_every,
+    const T* __restrict__ v_first, int64_t ld_vf, const float* __restrict__ lambda_ptr, T* __restrict__ k_pool, T* __restrict__ v_pool, int H,
+    int G, int dk, int dv) {
+    using V2 = typename VecT<T>::x2;
+    const int64_t t = blockIdx.x;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int slot = slots[t];
+    const int64_t page = slot / PAGE;
+    const int off = slot % PAGE;
+    T* row = qkv + t * ld;
+    const float* src = slabs + ((t >> 5) * S * 32 + (t & 31)) * sld;
+    const int64_t next = 32 * sld;
+    const int head_blocks = (H + G + 3) / 4;
+    if ((int)blockIdx.y >= head_blocks) {
+        const float lam = (v_first && lambda_ptr) ? *lambda_ptr : 0.f;
+        const int c0 = (H + G) * dk, i0 = ((int)blockIdx.y - head_blocks) * 1024, i1 = min(i0 + 1024, G * dv);
+        for (int i = i0 + threadIdx.x; i < i1; i += 256) {
+            float sum = 0.f;
+#pragma unroll 4
+            for (int s = 0; s < S; ++s) sum += src[s * next + c0 + i];
+            const T own = (T)sum;
+            row[c0 + i] = own;
+            float v = (float)own;
+            if (v_first) v = (1.f - lam) * v + lam * ldf(v_first + t * ld_vf + i);
+            const int g = i / dv, c = i - g * dv;
+            v_pool[((page * G + g) * dv + c) * PAGE + off] = (T)v;
+        }
+        return;
+    }
+    const int h = blockIdx.y * 4 + wave;
+    if (h >= H + G) return;
+    const bool is_q = h < H;
+    float gain = 1.f;
+    if (is_q && gain_every > 0) gain = 1.f + gain_coef * logf((float)((positions[t] + 1) / gain_every) + 1.f);
+    T* p = row + (int64_t)h * dk;
+    T* dst = is_q ? p : k_pool + ((page * G + (h - H)) * PAGE + off) * dk;
+    const float* w = is_q ? qw : kw;
+    float v[4];
+    float ss = 0.f;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int d = lane * 2 + it * 128;
+        f32x2 sum = {0.f, 0.f};
+        if (d < dk) {
+#pragma unroll 4
+            for (int s = 0; s < S; ++s) sum += *reinterpret_cast<const f32x2*>(src + s * next + h * dk + d);
+        }
+        V2 x;
+        x[0] = (T)sum[0];
+        x[1] = (T)sum[1];
+        if (!is_q && d < dk) *reinterpret_cast<V2*>(p + d) = x;
+        v[it * 2] = (float)x[0];
+        v[it * 2 + 1] = (float)x[1];
+        ss += v[it * 2] * v[it * 2] + v[it * 2 + 1] * v[it * 2 + 1];
+    }
+    ss = wave_sum(ss);
+    const float rinv = 1.0f / sqrtf(ss / (float)dk + eps) * gain;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int d = lane * 2 + it * 128;
+        if (d < dk) {
+            V2 y;
+            y[0] = (T)(v[it * 2] * rinv * w[d]);
+            y[1] = (T)(v[it * 2 + 1] * rinv * w[d + 1]);
+            *reinterpret_cast<V2*>(dst + d) = y;
+        }
+    }
+}
+
 // The norm of q and k alone, for long steps of two-byte models: L lanes take one head of up to 8 L channels with one 16-byte load each, so
 // a wave has 64 / L heads in flight.  Bound by its bytes; with a wave per head (above) a head of 64 was one 128-byte load and a six-step
 // sum per wave, 147 thousand waves for 4096 tokens of 36 heads.  us, with the values' launch, before / now: 512, 1024, 4096 tokens of 36 heads
@@ -1470,6 +1545,32 @@ extern "C" int tgis_qk_norm_kv_write(void* qkv, int64_t ld, const int32_t* posit
         launch_prep<bf16>(qkv, ld, positions, slots, q_gain, k_gain, eps, gain_coef, gain_every, v_first, ld_v_first, v_lambda, k_pool, v_pool, T, H, G, dk, dv, st);
     else
         launch_prep<float>(qkv, ld, positions, slots, q_gain, k_gain, eps, gain_coef, gain_every, v_first, ld_v_first, v_lambda, k_pool, v_pool, T, H, G, dk, dv, st);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+extern "C" int tgis_qk_norm_kv_write_partial(const float* slabs, int num_slabs, int64_t slab_ld, void* qkv, int64_t ld, const int32_t* positions,
+                                             const int32_t* slots, const float* q_gain, const float* k_gain, float eps, float gain_coef,
+                                             int gain_every, const void* v_first, int64_t ld_v_first, const float* v_lambda, void* k_pool,
+                                             void* v_pool, int64_t T, int H, int G, int dk, int dv, int dtype, void* stream) {
+    TGIS_CHECK_ARG(slabs && qkv && positions && slots && q_gain && k_gain && k_pool && v_pool, "tgis_qk_norm_kv_write_partial: null tensor");
+    TGIS_CHECK_ARG(H >= 1 && G >= 1 && H % G == 0 && dk >= 2 && dk <= 256 && dk % 2 == 0 && dv >= 1 &&
+                       ld >= (int64_t)(H + G) * dk + (int64_t)G * dv && ld % 2 == 0 && (uintptr_t)qkv % 4 == 0,
+                   "tgis_qk_norm_kv_write_partial: bad head geometry (H %d, G %d, dk %d, dv %d, ld %ld)", H, G, dk, dv, (long)ld);
+    TGIS_CHECK_ARG(num_slabs >= 1 && slab_ld >= (int64_t)(H + G) * dk + (int64_t)G * dv && slab_ld % 4 == 0 && (uintptr_t)slabs % 8 == 0,
+                   "tgis_qk_norm_kv_write_partial: bad slab geometry");
+    TGIS_CHECK_ARG(!v_first || (v_lambda && ld_v_first >= (int64_t)G * dv), "tgis_qk_norm_kv_write_partial: blending needs lambda and a row stride");
+    TGIS_CHECK_ARG(dtype == TGIS_F16 || dtype == TGIS_BF16, "tgis_qk_norm_kv_write_partial: bad dtype");
+    if (T == 0) return TGIS_OK;
+    const hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_ROPE_KV, st);
+    const dim3 grid((unsigned)T, (unsigned)((H + G + 3) / 4 + cdiv64((int64_t)G * dv, 1024)));
+#define TGIS_NORM_SUM(TT)                                                                                                                      hipLaunchKernelGGL(qk_norm_kv_sum_kernel<TT>, grid, dim3(256), 0, st, slabs, num_slabs, slab_ld, (TT*)qkv, ld, positions, slots, q_gain,                        k_gain, eps, gain_coef, gain_every, (const TT*)v_first, ld_v_first, v_lambda, (TT*)k_pool, (TT*)v_pool, H, G, dk, dv)
+    if (dtype == TGIS_F16)
+        TGIS_NORM_SUM(f16);
+    else
+        TGIS_NORM_SUM(bf16);
+#undef TGIS_NORM_SUM
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }

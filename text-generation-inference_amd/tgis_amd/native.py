@@ -112,6 +112,8 @@ SIGNATURES = {
     "tgis_glu": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_int, _c_f, _c_f, _c_int, _vp]),
     "tgis_qk_norm_kv_write": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _c_f, _c_f, _c_int, _vp, _c_i64, _vp, _vp, _vp, _c_i64,
                                        _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
+    "tgis_qk_norm_kv_write_partial": (_c_int, [_vp, _c_int, _c_i64, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_f, _c_f, _c_int, _vp, _c_i64, _vp, _vp,
+                                               _vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tgis_attn_varlen": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64,
                                   _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_int, _vp]),
     "tgis_token_shift_mix": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_int, _vp, _c_i64, _c_i64, _c_int, _vp]),
@@ -1221,14 +1223,23 @@ def glu(gate_up: torch.Tensor, I: int, mode: int = 0, alpha: float = 1.0, limit:
 
 def qk_norm_kv_write(qkv, positions, slots, q_gain, k_gain, eps: float, gain_coef: float, gain_every: int, v_first, v_lambda,
                      k_pool, v_pool, H: int, G: int, dk: int, dv: int):
+    """qkv may be a Partial without a bias (two-byte dtypes, dk even, up to 256); -> the tensor with q normed in place."""
+    part = qkv if isinstance(qkv, Partial) else None
+    T = qkv.shape[0]
+    if part is not None:
+        assert part.bias is None and part.N == (H + G) * dk + G * dv
+        qkv = torch.empty((T, part.N), dtype=part.dtype, device=part.device)
     assert qkv.dim() == 2 and qkv.stride(1) == 1 and k_pool.dtype == qkv.dtype and v_pool.dtype == qkv.dtype
-    assert positions.shape[0] == qkv.shape[0] and slots.shape[0] == qkv.shape[0]
-    assert v_first is None or (v_first.dtype == qkv.dtype and v_first.stride(1) == 1 and v_first.shape == (qkv.shape[0], G * dv))
-    _check(load_library().tgis_qk_norm_kv_write(
-        _ptr(qkv), qkv.stride(0), _i32(positions, "positions"), _i32(slots, "slots"), _f32(q_gain, "q_gain"),
-        _f32(k_gain, "k_gain"), float(eps), float(gain_coef), int(gain_every), _ptr(v_first),
-        v_first.stride(0) if v_first is not None else 0, _f32(v_lambda, "v_lambda") if v_first is not None else None,
-        _ptr(k_pool), _ptr(v_pool), qkv.shape[0], H, G, dk, dv, dtype_code3(qkv.dtype), _stream()), "tgis_qk_norm_kv_write")
+    assert positions.shape[0] == T and slots.shape[0] == T
+    assert v_first is None or (v_first.dtype == qkv.dtype and v_first.stride(1) == 1 and v_first.shape == (T, G * dv))
+    args = (_ptr(qkv), qkv.stride(0), _i32(positions, "positions"), _i32(slots, "slots"), _f32(q_gain, "q_gain"), _f32(k_gain, "k_gain"), float(eps),
+            float(gain_coef), int(gain_every), _ptr(v_first), v_first.stride(0) if v_first is not None else 0,
+            _f32(v_lambda, "v_lambda") if v_first is not None else None, _ptr(k_pool), _ptr(v_pool), T, H, G, dk, dv, dtype_code3(qkv.dtype), _stream())
+    if part is not None:
+        _check(load_library().tgis_qk_norm_kv_write_partial(_ptr(part.slabs), part.S, part.ld, *args), "tgis_qk_norm_kv_write_partial")
+    else:
+        _check(load_library().tgis_qk_norm_kv_write(*args), "tgis_qk_norm_kv_write")
+    return qkv
 
 
 def attn_varlen(q, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_q, H: int, G: int, dk: int, dv: int, scale: float,

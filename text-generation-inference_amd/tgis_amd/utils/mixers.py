@@ -99,6 +99,8 @@ class NormedQKAttention:
         # blend: v <- (1 - lambda) v + lambda v_other, lambda a learned scalar kept on the device
         self.v_lambda = _f32(weights.get_tensor(f"{prefix}.vmix")).reshape(1) if blend else None
         self.defer = can_defer(self.o)
+        # short steps: the launch that norms q and k adds the projection's split-K sums
+        self.defer_qkv = self.qkv.streams and dim % 2 == 0 and dim <= 256 and self.qkv.out_features % 2 == 0
 
     def values_of(self, qkv: torch.Tensor) -> torch.Tensor:
         """The value columns of a projected step (what another layer blends with)."""
@@ -107,12 +109,12 @@ class NormedQKAttention:
     def forward(self, h: torch.Tensor, position_ids, step, v_other: Optional[torch.Tensor] = None, ends: Optional[torch.Tensor] = None):
         """h [T, W] -> (out [T, W], qkv [T, H dk + G dk + G dv] with q normed in place).  ends: out for these rows alone, each the last token of a
         sequence of the step."""
-        qkv = self.qkv(h)
+        qkv = self.qkv(h, partial=self.defer_qkv)
         cache = step.cache
         k_pool, v_pool = cache.k_pool(self.layer_id), cache.v_pool(self.layer_id)
-        native.qk_norm_kv_write(qkv, position_ids, step.slots, self.q_gain, self.k_gain, self.eps, self.gain_coef,
-                                self.gain_every, v_other if self.v_lambda is not None else None, self.v_lambda, k_pool, v_pool,
-                                self.H, self.G, self.dk, self.dv)
+        qkv = native.qk_norm_kv_write(qkv, position_ids, step.slots, self.q_gain, self.k_gain, self.eps, self.gain_coef,
+                                      self.gain_every, v_other if self.v_lambda is not None else None, self.v_lambda, k_pool, v_pool,
+                                      self.H, self.G, self.dk, self.dv)
         q, cu_q, longest = qkv, step.cu_seqlens_q, step.max_q_len
         if ends is not None:
             q, longest = qkv.index_select(0, ends), 1
