@@ -4,7 +4,7 @@ Mirrors utils/layers.py of the reference: `FastLinear` (:104-111), the `get_line
 (:172-203), `TensorParallelHead` (:215-277), `TensorParallelColumnLinear` (:280-297),
 `TensorParallelRowLinear` (all-reduce, :300-322), `TensorParallelEmbedding` (:325-357) and
 `PositionRotaryEmbedding` (:406-490); `Ex4bitLinearV2` mirrors utils/gptq/exllamav2.py:100-144.
-Every forward runs a kernel of libtgis_hip.so (decode-sized M) or, for prefill-sized M, a library GEMM
+Every forward runs a kernel of libtgis_hip.so or, for prefill-sized M where that is faster, a library GEMM
 on the same device; there is no CPU path."""
 import copy
 import math
