@@ -133,3 +133,10 @@ def test_rows_it_cannot_read(pad, first):
     lin = FastLinear(w.cuda(), bias.cuda())
     assert lin.tall(view) == -1 and lin.tall(x.cuda()) >= 0
     _check(lin(view), _expect(z, acc, torch.float16, 0))
+
+
+# behind a whole turn of the ring of four buffers: one, two and three steps, and none; behind none, and in the parts of a split
+@pytest.mark.parametrize("steps,S", [(1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (11, 1), (14, 2)])
+@pytest.mark.parametrize("tile", ["2,1", "2,2", "3,1", "3,2", "4,1", "4,2"])
+def test_tails_of_the_ring(tile, steps, S, monkeypatch):
+    _run(290, 64 * steps, 264, torch.bfloat16, 0, f"{tile},{S}", monkeypatch)

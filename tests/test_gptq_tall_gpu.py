@@ -46,6 +46,23 @@ def test_every_plan(gpu_device, K, N, groupsize, M, act, monkeypatch):
             assert (wide[:, cols:] == 7.0).all()
 
 
+# behind a whole turn of the ring of four buffers: one, two and three steps, and none; behind none, and in the parts of a split
+@pytest.mark.parametrize("steps,S", [(1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (11, 1), (14, 2)])
+def test_tails_of_the_ring(gpu_device, steps, S, monkeypatch):
+    from tgis_amd import native
+
+    K, N, M = 64 * steps, 288, 290
+    qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, 64, seed=steps)
+    w = native.GptqWeight(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), 4, 64)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(steps)).half()
+    want = x.double() @ ops_ref.gptq_dequant(qw, qz, sc, gi, 64).half().double()
+    ws = native.Workspace(64 << 20, gpu_device)
+    for tile in ("2,1", "2,2", "3,1", "3,2", "4,1", "4,2"):
+        monkeypatch.setenv("TGIS_TALL_PLAN", f"{tile},{S}")
+        got = native.gptq_gemm(x.to(gpu_device), w, ws).double().cpu()
+        assert ((got - want).abs() <= 2.0 ** -10 * want.abs() + 1e-5).all(), tile  # (as in test_every_plan)
+
+
 def test_linear_takes_whole_sums_past_128_rows(gpu_device):
     """129 .. 256 rows: the linear returns a finished tensor where 64-row passes left slabs to the consumer."""
     from tgis_amd import native

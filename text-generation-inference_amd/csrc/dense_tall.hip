@@ -14,9 +14,9 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <algorithm>
-#include <type_traits>
 #include "common.h"
 #include "dense_gemm_body.h"
+#include "tall_ring.h"
 
 namespace {
 
@@ -39,7 +39,7 @@ struct DTallArgs {
     float* scratch;
 };
 
-constexpr int X_RING = 4;  // buffers of x
+constexpr int X_RING = tall::RING;  // buffers of x
 
 template <typename T> __device__ __forceinline__ float act2_of(const DTallArgs& a, float gate, float up) {
     if (a.glu_limit > 0.f) {
@@ -129,10 +129,12 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
         for (int rb = 0; rb < BMR; ++rb) dst[rb] = ld16<V8>(smem + buf * (BM * 128) + rb * 4096 + apos[i]);
     };
     read_a(av[0], 0, 0);
-    auto step = [&](int s, auto slot_) {
+    auto step = [&](int s, auto slot_, auto tail_) {
         constexpr int SL = decltype(slot_)::value;
+        constexpr bool TAIL = decltype(tail_)::value;  // (at most RING - 1 steps, the first at slot 0)
         constexpr int NX = (SL + 1) % X_RING, WS = SL % WR;
-        x_load(s + 3, (SL + 3) % X_RING);  // everyone is done with that buffer since the barrier of the step before
+        constexpr bool REFILL = !TAIL || SL + WR < X_RING - 1;
+        if constexpr (!TAIL) x_load(s + 3, (SL + 3) % X_RING);  // everyone is done with that buffer since the barrier of the step before
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             read_a(av[(i + 1) & 1], i < 3 ? SL : NX, (i + 1) & 3);
@@ -141,32 +143,16 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
             for (int rb = 0; rb < BMR; ++rb)
 #pragma unroll
                 for (int t = 0; t < TW; ++t) acc[t][rb] = mfma32(av[i & 1][rb], wq[WS][t][i], acc[t][rb]);
+            if constexpr (REFILL) {
 #pragma unroll
-            for (int t = 0; t < TW; ++t) wq[WS][t][i] = w_at(t, ks0 + s + WR, i);
+                for (int t = 0; t < TW; ++t) wq[WS][t][i] = w_at(t, ks0 + s + WR, i);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // the x loads of step s + 2 were issued a step ago: behind them are that step's weights and everything of this step
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BMR + 8 * TW) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        // the x loads of step s + 2 were issued a step ago: behind them are that step's weights and, in whole turns, everything of this step
+        tall::meet<TAIL ? 0 : BMR + 8 * TW>();
     };
-    // whole turns of the ring, then what is left: with a way out behind every step the compiler sees ways back to the first one from each of
-    // them, and waits there for every load there is
-    using std::integral_constant;
-    int s = 0;
-    for (; s + X_RING <= n; s += X_RING) {
-        step(s, integral_constant<int, 0>{});
-        step(s + 1, integral_constant<int, 1>{});
-        step(s + 2, integral_constant<int, 2>{});
-        step(s + 3, integral_constant<int, 3>{});
-    }
-    if (s < n) {
-        step(s, integral_constant<int, 0>{});
-        if (s + 1 < n) {
-            step(s + 1, integral_constant<int, 1>{});
-            if (s + 2 < n) step(s + 2, integral_constant<int, 2>{});
-        }
-    }
+    tall::ring_steps(n, step);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
 
     const int c = lane & 31;

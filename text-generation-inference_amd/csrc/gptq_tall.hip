@@ -17,10 +17,10 @@
 // o 36 -> 32, gate_up 145 -> 138, down 81 -> 74 us with the loop in whole turns of its ring (below); 300 rows 41 -> 38, 28 -> 23, 72, 45 -> 42.
 #include <stdlib.h>
 #include <algorithm>
-#include <type_traits>
 #include "common.h"
 #include "gptq_gemm_body.h"
 #include "gptq_tall.h"
+#include "tall_ring.h"
 
 namespace {
 
@@ -43,7 +43,7 @@ struct TallArgs {
     float* scratch;
 };
 
-constexpr int TALL_RING = 4;  // k64-steps of weights in flight per wave, and buffers of x
+constexpr int TALL_RING = tall::RING;  // k64-steps of weights in flight per wave, and buffers of x
 
 // Tiles are walked in groups of 8 row blocks, each XCD its own run of them, so that its L2 serves a tile of weights to 8 blocks.  us, columns
 // fastest over the whole chip / this: 4096 x 22016 with SiLU at 300, 765, 6000 rows 74.9 / 69.4, 148.6 / 146.2, 989 / 961; 8192 x 57344 with SiLU at
@@ -155,19 +155,22 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     };
     read_a(av[0], 0, 0);
     dequant(b[0], wq[0], szr[0], 0);
-    auto step = [&](int s, auto slot_) {
+    auto step = [&](int s, auto slot_, auto tail_) {
         constexpr int SL = decltype(slot_)::value;
+        constexpr bool TAIL = decltype(tail_)::value;  // (at most RING - 1 steps: their weights are there)
         constexpr int NX = (SL + 1) % TALL_RING;
-        x_load(s + 3, (SL + 3) % TALL_RING);  // everyone is done with that buffer since the barrier of the step before
+        if constexpr (!TAIL) x_load(s + 3, (SL + 3) % TALL_RING);  // everyone is done with that buffer since the barrier of the step before
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             read_a(av[(i + 1) & 1], i < 3 ? SL : NX, (i + 1) & 3);
             __builtin_amdgcn_sched_barrier(0);
             if (i == 3) {
+                if constexpr (!TAIL) {
 #pragma unroll
-                for (int t = 0; t < TW; ++t) {
-                    wq[SL][t] = w_at(t, ks0 + s + TALL_RING);
-                    szr[SL][t] = sz_at(t, ks0 + s + TALL_RING);
+                    for (int t = 0; t < TW; ++t) {
+                        wq[SL][t] = w_at(t, ks0 + s + TALL_RING);
+                        szr[SL][t] = sz_at(t, ks0 + s + TALL_RING);
+                    }
                 }
                 dequant(b[0], wq[NX], szr[NX], 0);
             } else {
@@ -186,28 +189,10 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         }
         // the x loads of step s + 2 were issued a step ago: behind them this wave has asked for that step's 2 TW weights and scales
-        // and for everything of this step
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BMR + 4 * TW) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        // and, in whole turns, for everything of this step
+        tall::meet<TAIL ? 0 : BMR + 4 * TW>();
     };
-    // whole turns of the ring, then what is left: with a way out behind every step the compiler sees ways back to the first one from each of
-    // them, and waits there for every load there is
-    using std::integral_constant;
-    int s = 0;
-    for (; s + TALL_RING <= n; s += TALL_RING) {
-        step(s, integral_constant<int, 0>{});
-        step(s + 1, integral_constant<int, 1>{});
-        step(s + 2, integral_constant<int, 2>{});
-        step(s + 3, integral_constant<int, 3>{});
-    }
-    if (s < n) {
-        step(s, integral_constant<int, 0>{});
-        if (s + 1 < n) {
-            step(s + 1, integral_constant<int, 1>{});
-            if (s + 2 < n) step(s + 2, integral_constant<int, 2>{});
-        }
-    }
+    tall::ring_steps(n, step);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
 
     // ---- epilogue: lane holds rows m = 32 rb + (r & 3) + 8 (r >> 2) + 4 (lane >> 5) of column nt * 32 + (lane & 31) -----------

@@ -1,0 +1,42 @@
+// The k loop of the GEMMs of prefills (gptq_tall.hip, dense_tall.hip): a ring of four LDS buffers of x, filled by direct loads three steps ahead.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <type_traits>
+
+namespace tall {
+
+constexpr int RING = 4;
+
+// The end of a step: the buffer that step s + 2 reads is whole for every wave, with BEHIND vector loads issued behind its own.  The count holds
+// only where each of these loads is sure to be issued: a load that nothing reads any more is dropped by the compiler, and the count then lets
+// the one that it is meant for through.
+template <int BEHIND> __device__ __forceinline__ void meet() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// step(s, slot s % RING, tail) for s = 0 .. n - 1: whole turns of the ring, then what is left: with a way out behind every step the compiler sees
+// ways back to the first one from each of them, and waits there for every load there is.  In the tail nothing is fetched that no step
+// is left to read, and a step ends with meet<0>, which counts on no load.
+template <typename F> __device__ __forceinline__ void ring_steps(int n, F&& step) {
+    using std::integral_constant;
+    using std::false_type;
+    using std::true_type;
+    int s = 0;
+    for (; s + RING <= n; s += RING) {
+        step(s, integral_constant<int, 0>{}, false_type{});
+        step(s + 1, integral_constant<int, 1>{}, false_type{});
+        step(s + 2, integral_constant<int, 2>{}, false_type{});
+        step(s + 3, integral_constant<int, 3>{}, false_type{});
+    }
+    if (s < n) {
+        step(s, integral_constant<int, 0>{}, true_type{});
+        if (s + 1 < n) {
+            step(s + 1, integral_constant<int, 1>{}, true_type{});
+            if (s + 2 < n) step(s + 2, integral_constant<int, 2>{}, true_type{});
+        }
+    }
+}
+
+}  // namespace tall
