@@ -70,6 +70,21 @@ def test_dense_tall(M, K, N, act, pays):
     assert (native.load_library().tgis_dense_tall_bytes(M, K, N, act) >= 0) == bool(pays)
 
 
+def test_dense_tall_operands():
+    """What the library's linear takes and the kernel does not read is not its to serve: one dimension, three, columns or rows out of step."""
+    import types
+
+    import torch
+
+    from tgis_amd import native
+
+    w = types.SimpleNamespace(K=512, N=2048, plans={})
+    serves = lambda x: native.dense_tall_bytes(x, w) >= 0
+    x = torch.zeros(300, 512, dtype=torch.float16)
+    assert serves(x)
+    assert not any(map(serves, (x.flatten()[:512], x.view(300, 1, 512), x.view(100, 3, 512).transpose(1, 2), x.t().contiguous().t(), x.view(-1)[4:4 + 299 * 512].view(299, 512))))
+
+
 def test_dense_tall_scratch():
     """Its scratch fits the workspace that projections share, which captured graphs hold the address of."""
     from tgis_amd import native

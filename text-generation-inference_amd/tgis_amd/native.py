@@ -696,7 +696,7 @@ def dense_tall_serves(M: int, K: int, N: int, act: int = 0) -> bool:
 def dense_tall_bytes(x: torch.Tensor, w: DenseWeight, act: int = 0) -> int:
     """The scratch of dense_tall where it is the faster way to x @ w^T, -1 where it is not or x is not as it reads it (a size query)."""
     M, ld = x.shape[0], x.stride(0)
-    if M < DENSE_TALL_MIN_M or x.stride(1) != 1 or ld % 8 or not w.K <= ld < 1 << 22 or x.data_ptr() % 16:
+    if x.dim() != 2 or M < DENSE_TALL_MIN_M or x.stride(1) != 1 or ld % 8 or not w.K <= ld < 1 << 22 or x.data_ptr() % 16:
         return -1
     if M > PARTIAL_MAX_M:
         return load_library().tgis_dense_tall_bytes(M, w.K, w.N, act)
