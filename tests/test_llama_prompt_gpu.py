@@ -71,3 +71,28 @@ def test_one_by_one(gpu_device, monkeypatch, kw, lens):
     with lm.context_manager():
         logits = lm.ragged_forward(torch.full((sum(lens),), 5).cuda(), pages, [0] * len(lens), lens)
     assert bool(torch.isfinite(logits).all())
+
+
+def test_no_split_sums_where_they_are_off(gpu_device, monkeypatch):
+    """TGIS_DEFER_REDUCE=0: prompts of up to 256 rows go layer by layer, and no product leaves its sum to a norm."""
+    from tgis_amd import native
+    from tgis_amd.models.custom_modeling import flash_llama_modeling
+    from tgis_amd.utils import layers
+
+    lm, cfg = model(torch.bfloat16)
+    served, run = [], native.llama_prompt
+    monkeypatch.setattr(native, "llama_prompt", lambda got, x, *a, **k: served.append(x.shape[0]) or run(got, x, *a, **k))
+    prompts = ([47], [70], [200, 56], [257])
+    want = [steps(lm, cfg.vocab_size, lens)[0] for lens in prompts]
+    assert {47, 70, 256, 257} == set(served)
+    del served[:]
+    monkeypatch.setattr(flash_llama_modeling, "DEFER_REDUCE", False)
+    monkeypatch.setattr(layers, "DEFER_REDUCE", False)
+    for name in ("dense_tall_partial", "dense_gemm_partial"):
+        monkeypatch.setattr(native, name, lambda *a, **k: pytest.fail("left its sum"))
+    got = [steps(lm, cfg.vocab_size, lens)[0] for lens in prompts]
+    assert set(served) == {257}
+    # every product is rounded to the model dtype in front of the norm either way: what differs is the order of the fp32 sums, and with it here and
+    # there a rounding (a step of 2 ** -8), which three layers carry on: below four steps in the norm of all logits
+    for a, b in zip(got, want):
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 4 * 2.0 ** -8

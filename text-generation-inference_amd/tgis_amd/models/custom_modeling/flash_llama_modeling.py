@@ -369,7 +369,9 @@ class FlashLlamaModel:
         shapes = {"qkv": ((H + 2 * Hkv) * D, hidden), "o": (hidden, H * D), "gate_up": (2 * inner, hidden), "down": (hidden, inner)}
         if tall and not all(native.dense_tall_serves(rows, K, N, 2 if name == "gate_up" else 0) for name, (N, K) in shapes.items()):
             return []
-        if not tall and not (DEFER_REDUCE and rows <= SKINNY_MAX_M):
+        if rows <= native.PARTIAL_MAX_M and not DEFER_REDUCE:  # (the launches of such steps leave split sums to the norms)
+            return []
+        if not tall and rows > SKINNY_MAX_M:
             return []
         got = []
         for layer in self.layers[:count]:
