@@ -140,3 +140,25 @@ def test_rows_it_cannot_read(pad, first):
 @pytest.mark.parametrize("tile", ["2,1", "2,2", "3,1", "3,2", "4,1", "4,2"])
 def test_tails_of_the_ring(tile, steps, S, monkeypatch):
     _run(290, 64 * steps, 264, torch.bfloat16, 0, f"{tile},{S}", monkeypatch)
+
+
+def test_rows_that_the_user_divides(monkeypatch):
+    """TGIS_SKINNY_MAX_M: the streaming kernel up to that many rows, the library above, nothing else."""
+    from tgis_amd import native
+    from tgis_amd.utils import layers
+
+    K, N = 512, 1024
+    monkeypatch.setattr(layers, "DENSE_TALL", False)
+    monkeypatch.setattr(layers, "SKINNY_MAX_M", 128)
+    for name in ("dense_tall", "dense_tall_partial"):
+        monkeypatch.setattr(native, name, lambda *a, **k: pytest.fail("the prefill kernel"))
+    streamed, run = [], native.dense_gemm
+    monkeypatch.setattr(native, "dense_gemm", lambda x, *a, **k: streamed.append(x.shape[0]) or run(x, *a, **k))
+    for M in (65, 128, 129, 300):
+        x, w, bias, z, acc = _case(M, K, N, torch.float16, seed=6)
+        lin = layers.FastLinear(w.cuda(), bias.cuda())
+        _check(lin(x.cuda()), _expect(z, acc, torch.float16, 0))
+        _check(lin(x.cuda(), gelu=False), _expect(z, acc, torch.float16, 4))
+        lin.gate_up = True
+        _check(lin(x.cuda()), _expect(z, acc, torch.float16, 2))
+    assert streamed == [65] * 3 + [128] * 3

@@ -96,3 +96,20 @@ def test_no_split_sums_where_they_are_off(gpu_device, monkeypatch):
     # there a rounding (a step of 2 ** -8), which three layers carry on: below four steps in the norm of all logits
     for a, b in zip(got, want):
         assert float((a.double() - b.double()).norm() / b.double().norm()) < 4 * 2.0 ** -8
+
+
+def test_rows_that_the_user_divides(gpu_device, monkeypatch):
+    """TGIS_SKINNY_MAX_M: dense linears are the streaming kernel and the library alone, in whole prompts and in the steps of a few rows as well."""
+    from tgis_amd import native
+    from tgis_amd.models.custom_modeling import flash_llama_modeling
+    from tgis_amd.utils import layers
+
+    lm, cfg = model(torch.float16)
+    for module in (flash_llama_modeling, layers):
+        monkeypatch.setattr(module, "DENSE_TALL", False)
+        monkeypatch.setattr(module, "SKINNY_MAX_M", 2)
+    for name in ("llama_prompt", "dense_tall", "dense_tall_partial"):
+        monkeypatch.setattr(native, name, lambda *a, **k: pytest.fail("served"))
+    for lens in ([20], [70], [300]):
+        assert bool(torch.isfinite(steps(lm, cfg.vocab_size, lens)[0]).all())
+    assert [lm.model.rows_path(rows) for rows in (1, 2, 3, 4)] == [True, True, False, False]

@@ -20,6 +20,7 @@ import torch
 from tgis_amd import native
 from tgis_amd.utils.layers import (
     DEFER_REDUCE,
+    DENSE_TALL,
     SKINNY_MAX_M,
     FastLinear,
     PositionRotaryEmbedding,
@@ -371,7 +372,7 @@ class FlashLlamaModel:
             return []
         if rows <= native.PARTIAL_MAX_M and not DEFER_REDUCE:  # (the launches of such steps leave split sums to the norms)
             return []
-        if not tall and rows > SKINNY_MAX_M:
+        if not DENSE_TALL if tall else rows > SKINNY_MAX_M:
             return []
         got = []
         for layer in self.layers[:count]:
@@ -443,7 +444,7 @@ class FlashLlamaForCausalLM:
         """Whether a decode step of `rows` rows runs on the launches that norm their operand themselves (FlashLlamaModel.forward_rows)."""
         got = self._rows_path.get(rows)
         if got is None:
-            got = self._rows_path[rows] = rows <= native.DENSE_ROWS_MAX_M and self._serves_rows(rows)
+            got = self._rows_path[rows] = rows <= min(native.DENSE_ROWS_MAX_M, SKINNY_MAX_M) and self._serves_rows(rows)
         return got
 
     def _serves_rows(self, rows: int) -> bool:

@@ -24,6 +24,7 @@ import os
 # GPTQ linears ask the library how far its fused kernels reach (GptqWeight.fused_rows: 64-row streaming passes
 # to 256 rows, the tall kernel from 65 / 129 rows to 8192 where it is faster; else dequantise once + hipBLASLt, exllamav2.py:87).
 SKINNY_MAX_M = int(os.getenv("TGIS_SKINNY_MAX_M", "256"))
+DENSE_TALL = os.getenv("TGIS_SKINNY_MAX_M") is None  # with the variable set, dense linears are the streaming kernel and the library alone
 # fuse the split-K reduce of decode-sized GPTQ GEMMs into the consumer kernel (rmsnorm / rope+KV write)
 DEFER_REDUCE = os.getenv("TGIS_DEFER_REDUCE", "true").lower() not in ("0", "false")
 # steps of up to 64 rows, prompts where that pays (native.rope_gemm_pays_for_prompts): rotary embedding + cache write in the epilogue of the qkv
@@ -41,6 +42,12 @@ def workspace(device) -> native.Workspace:
     if ws is None:
         ws = _WORKSPACES[key] = native.Workspace(64 << 20, device)
     return ws
+
+
+def tall_bytes(x: torch.Tensor, image: native.DenseWeight, act: int = 0) -> int:
+    """The scratch of the prefill kernel on this image where it serves the step, and sooner than the weight-streaming kernel or the library GEMM
+    would; else -1."""
+    return native.dense_tall_bytes(x, image, act) if x.shape[0] >= native.DENSE_TALL_MIN_M and DENSE_TALL else -1
 
 
 class FastLinear:
@@ -95,9 +102,7 @@ class FastLinear:
                 self.rope_handle = native.DenseWeight(self.weight, rope=(D, H + Hkv))
 
     def tall(self, x: torch.Tensor, act: int = 0) -> int:
-        """The scratch of the prefill kernel on the image where it serves this step, and sooner than the weight-streaming kernel or the library
-        GEMM would; else -1."""
-        return native.dense_tall_bytes(x, self.prepared, act) if x.shape[0] >= native.DENSE_TALL_MIN_M and self.streams else -1
+        return tall_bytes(x, self.prepared, act) if self.streams else -1
 
     def forward(self, x: torch.Tensor, act: int = 0, out_f32: bool = False, partial: bool = False,
                 gelu: Optional[bool] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:

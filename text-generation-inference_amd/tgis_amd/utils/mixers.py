@@ -55,7 +55,7 @@ from typing import Optional
 import torch
 
 from tgis_amd import native
-from tgis_amd.utils.layers import SKINNY_MAX_M, FastLinear, workspace
+from tgis_amd.utils.layers import SKINNY_MAX_M, FastLinear, tall_bytes, workspace
 
 # rows up to which the clamped gated unit runs in the epilogue of the weight-streaming GEMM
 CLAMPED_EPILOGUE_MAX_M = SKINNY_MAX_M
@@ -202,7 +202,7 @@ class GatedUnit:
         partial = partial and can_defer(self.down)
         if self.fused:
             return self.down(self.gate_up(h), partial=partial)
-        tall = native.dense_tall_bytes(h, self.clamped_image, 2) if self.clamped_image is not None else -1
+        tall = tall_bytes(h, self.clamped_image, 2) if self.clamped_image is not None else -1
         if tall >= 0:
             act = native.dense_tall(h, self.clamped_image, workspace(h.device), tall, bias=self.gate_up.bias, act=2, alpha=self.alpha, limit=self.limit)
             return self.down(act, partial=partial)
