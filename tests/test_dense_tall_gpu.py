@@ -90,6 +90,20 @@ def test_fp32_sums(plan, M, monkeypatch):
     _check(lin(x.cuda(), out_f32=True), (z, acc))
 
 
+def test_parts_of_the_plan_that_ran(monkeypatch):
+    """One projection whose plan is changed between two calls: the number of parts is that of the launch, not the first call's."""
+    from tgis_amd.utils.layers import FastLinear
+
+    x, w, bias, z, acc = _case(130, 576, 1100, torch.float16, seed=7)
+    lin = FastLinear(w.cuda(), bias.cuda())
+    for plan in ("2,1,3", "4,2,2", "3,1,1", "2,1,3"):
+        monkeypatch.setenv("TGIS_DTALL_PLAN", plan)
+        part = lin(x.cuda(), partial=True)
+        assert part.S == int(plan[4])
+        sums = part.slabs[:160 * part.S * part.ld].view(-1, part.S, 32, part.ld).sum(1, dtype=torch.float64).flatten(0, 1)
+        _check(sums[:130, :1100], (z - bias.double(), acc))
+
+
 @pytest.mark.parametrize("plan", ["2,1,1", "2,2,2", "3,1,3", "3,2,1", "4,1,2", "4,2,1"])
 @pytest.mark.parametrize("act", [2, 3, 4, 5])
 def test_activations(plan, act, monkeypatch):

@@ -725,15 +725,13 @@ def dense_tall_partial(x: torch.Tensor, w: DenseWeight, bias=None) -> Partial:
     assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K and not w.flags
     lib, M = load_library(), x.shape[0]
     plan = w.plans.get(("tall slabs", M))
-    nbytes = plan[0] if plan is not None else lib.tgis_dense_tall_partial_bytes(M, w.K, w.N)
-    slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
-    S, ld = (None, None) if plan is not None else (_c_int(), _c_i64())
-    _check(lib.tgis_dense_tall_partial(_ptr(x), x.stride(0), _ptr(w.image), M, w.K, w.N, dtype_code(w.dtype), _ptr(slabs), nbytes,
-                                       None if S is None else ctypes.byref(S), None if ld is None else ctypes.byref(ld), _stream()),
-           "tgis_dense_tall_partial")
     if plan is None:
-        plan = w.plans[("tall slabs", M)] = (nbytes, S.value, ld.value)
-    p = Partial(slabs, plan[1], plan[2], M, w.N, bias)
+        plan = w.plans[("tall slabs", M)] = (lib.tgis_dense_tall_partial_bytes(M, w.K, w.N), _c_int(), _c_i64())
+    nbytes, S, ld = plan  # (S and ld are of the plan that this launch runs, which TGIS_DTALL_PLAN may have changed)
+    slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+    _check(lib.tgis_dense_tall_partial(_ptr(x), x.stride(0), _ptr(w.image), M, w.K, w.N, dtype_code(w.dtype), _ptr(slabs), nbytes,
+                                       ctypes.byref(S), ctypes.byref(ld), _stream()), "tgis_dense_tall_partial")
+    p = Partial(slabs, S.value, ld.value, M, w.N, bias)
     p.dtype = w.dtype
     return p
 
