@@ -1,5 +1,6 @@
 // The layers of a dense Llama model on the rows of prompts, launched from here: the launches that the model's own forward makes one by one,
-// with the same arguments and the same results, without its way back to Python between them.  A layer of a short prompt is six launches of 4 to
+// with the same arguments and the same results, without its way back to Python between them.  (One exception: where `fresh` is not set, qkv of
+// TGIS_DENSE_TALL_MIN_M to 256 rows is finished here, and left in parts to the rotary launch there: another order of its fp32 sums.)  A layer of a short prompt is six launches of 4 to
 // 16 us, each of which took 9 us of host time to prepare; here it is 2 - 3 us.  47 tokens through 22 layers of 2048: 1820 -> 1540 us.
 #include "common.h"
 
