@@ -20,6 +20,23 @@ def close(got, want, K, dtype, roundings, turned=0.0):
     assert (err <= tol).all(), float((err / tol).max())
 
 
+def refused(dev, M, K, dtype, norm):
+    """More rows than fit LDS, or than are served at this width: an error in front of any launch, and outputs as they were."""
+    from tgis_amd import native
+
+    N, stream = 64, torch.full((M, K if norm else 64), 3.0, device=dev)
+    image, w = native.DenseWeight(torch.zeros(N, K, dtype=dtype, device=dev)), torch.ones(K, dtype=dtype, device=dev)
+    with pytest.raises(RuntimeError, match="up to 4 rows"):
+        if norm:
+            native.dense_rows_head(stream, w, 1e-5, image)
+        else:
+            native.dense_rows_residual(torch.ones(M, K, dtype=dtype, device=dev), image, stream)
+    if norm:
+        with pytest.raises(RuntimeError, match="up to 4 rows"):
+            native.dense_rows_silu(stream, w, 1e-5, native.DenseWeight(torch.zeros(N, K, dtype=dtype, device=dev), gate_up=True))
+    assert bool((stream == 3.0).all())
+
+
 # K: one step of 64, fewer steps than waves, every depth at its edge and past it; N: not a multiple of a tile, of a workgroup's columns
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("K,N", [(64, 40), (448, 72), (2048, 2048), (2112, 96), (4096, 32), (4160, 100), (5632, 256), (6208, 40), (12288, 32)])
@@ -28,7 +45,7 @@ def test_residual(gpu_device, M, K, N, dtype):
     from tgis_amd import native
 
     if not native.dense_rows_ok(M, K, False):
-        pytest.skip("rows that do not fit LDS")
+        return refused(gpu_device, M, K, dtype, norm=False)
     g = torch.Generator().manual_seed(M + K)
     x, w = torch.randn(M, K + 8, generator=g).to(dtype), (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype)
     h = torch.randn(M, N, generator=g)
@@ -48,7 +65,7 @@ def test_norm_silu_and_head(gpu_device, M, K, ff, vocab, dtype):
     from tgis_amd import native
 
     if not native.dense_rows_ok(M, K, True):
-        pytest.skip("more rows than are served at this width")
+        return refused(gpu_device, M, K, dtype, norm=True)
     g = torch.Generator().manual_seed(M + K)
     h, nw = torch.randn(M, K, generator=g) * 3, (torch.rand(K, generator=g) + 0.5).to(dtype)
     wg, wh = ((torch.randn(n, K, generator=g) * K ** -0.5).to(dtype) for n in (2 * ff, vocab))
@@ -69,7 +86,7 @@ def test_norm_rope(gpu_device, M, K, H, Hkv, D, bias, dtype):
     from tgis_amd import native
 
     if not native.dense_rows_ok(M, K, True):
-        pytest.skip("more rows than are served at this width")
+        return refused(gpu_device, M, K, dtype, norm=True)
     g = torch.Generator().manual_seed(M + K)
     N, pages = (H + 2 * Hkv) * D, 3
     h, nw = torch.randn(M, K, generator=g) * 2, (torch.rand(K, generator=g) + 0.5).to(dtype)
