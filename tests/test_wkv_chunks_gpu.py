@@ -292,3 +292,28 @@ def test_scan_in_segments(gpu_device, d, longest, dtype):
     assert ((got - want).abs() <= tol).all(), float(((got - want).abs() / size).max())
     assert (got_st - want_st).abs().max() <= 2e-5 * want_st.abs().max()
     assert torch.equal(got_sh, want_sh) and torch.equal(spare, state[3])
+
+
+def test_scan_entries_without_segments(gpu_device):
+    """tgis_wkv_scan and tgis_wkv_scan_runs: the launches of a step that is not cut, with the hint 0 and with one, bit for bit."""
+    from tgis_amd import native
+
+    lib, H, W, d, eps = native.load_library(), 3, 8, 64, 1e-4
+    lens = [5, 1, 33, 60]
+    T, B = sum(lens), len(lens)
+    g = torch.Generator().manual_seed(1)
+    rkvg = [torch.randn(T, H * d, generator=g).to(torch.bfloat16).to(gpu_device) for _ in range(4)]
+    logw, u, gain, state, h = (t.to(gpu_device) for t in (-torch.rand(T, H * d, generator=g), torch.rand(H * d, generator=g), torch.rand(H * d, generator=g),
+                                                          torch.randn(B, H, d, d, generator=g), torch.randn(T, W, generator=g)))
+    slots, pos = torch.arange(B).int().to(gpu_device), torch.cat([torch.arange(n) for n in lens]).int().to(gpu_device) + 3
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(gpu_device)
+    ptr = lambda t: t.data_ptr()
+    for name, hint in (("tgis_wkv_scan", 0), ("tgis_wkv_scan_runs", 60)):
+        st, sh = state.clone(), torch.zeros(B, W, device=gpu_device)
+        want = native.wkv_scan(*rkvg, logw, u, gain, st, sh, h, slots, cu, pos, H, d, eps, max_q_len=hint)
+        st2, sh2, out = state.clone(), torch.zeros(B, W, device=gpu_device), torch.zeros_like(want)
+        rest = (eps, hint, native.dtype_code3(out.dtype)) if hint else (eps, native.dtype_code3(out.dtype))
+        assert lib.tgis_wkv_scan_workspace(B, H, d, hint) == 0
+        assert getattr(lib, name)(*map(ptr, rkvg), H * d, ptr(logw), ptr(u), ptr(gain), ptr(st2), ptr(sh2), ptr(h), W, ptr(slots), ptr(cu), ptr(pos), ptr(out),
+                                  H * d, B, H, d, *rest, torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(out, want) and torch.equal(st2, st) and torch.equal(sh2, sh)
