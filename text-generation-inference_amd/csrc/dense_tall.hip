@@ -344,7 +344,10 @@ TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
 }
 
 // ... where the consumer adds the parts: every tile in the same number of them, and no launch behind: completions of two prompts of 54 tokens, 8 hybrid layers
-// of 2048, 2360 -> 2250 us (2145 with the plans kept, below).
+// of 2048, 2360 -> 2250 us (2145 with the plans kept, below).  Past a whole round of 256 blocks the rest costs what it costs in make_plan_tall: priced
+// by its share alone, 257 - 320 blocks looked best and were the slower way.  us with the norm behind, the passes of 64 rows / by the share / now: 6144 x
+// 6144 at 100, 128 rows 33.8 / 35.9 / 26.0, 34.6 / 38.2 / 30.2; 24576 x 6144 at 65, 160 119 / 90 / 69, 203 / 126 / 87; 11008 x 4096 at 256 55 / 60 / 41; 28672 x
+// 8192 at 128 120 / 134 / 108; 13824 x 5120 at 193 119 / 65 / 50; 8192 x 10240 in front of a q / k norm at 192 66 / 74 / 58.
 TallPlan make_plan_parts(int64_t M, int64_t K, int64_t N) {
     const int64_t steps = K / 64, NT = cdiv64(N, 32);
     TallPlan best{};
@@ -357,9 +360,11 @@ TallPlan make_plan_parts(int64_t M, int64_t K, int64_t N) {
                 const int64_t per = cdiv64(steps, S);
                 if (S > 1 && per < 4) break;
                 if ((S - 1) * per >= steps) continue;
-                const double fill = (double)(tiles * S) / CUS, alone = 1.6 + per * c.alone, busy = 1.8 + per * c.busy;
-                const double us = (fill <= 1.0 ? alone + std::max(0.0, busy - alone) * fill : std::max(alone, busy * fill)) + 0.3 * (S - 1) +
-                                  2.0 * S * M * N * 4 / 3.5e6;
+                const int64_t blocks = tiles * S, rounds = blocks / CUS, rest = blocks % CUS;
+                const double alone = 1.6 + per * c.alone, busy = 1.8 + per * c.busy, share = (double)rest / CUS;
+                const double us = (blocks <= CUS ? alone + std::max(0.0, busy - alone) * blocks / CUS
+                                                 : std::max(alone, rounds * busy + (rest ? busy * (0.51 + 0.49 * share) : 0.0))) +
+                                  0.3 * (S - 1) + 2.0 * S * M * N * 4 / 3.5e6;
                 if (us < best_us) {
                     best_us = us;
                     best = {BMR, TW, (int)cb, (int)tiles, 0, S, (int)per, us};
