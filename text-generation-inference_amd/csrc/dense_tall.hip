@@ -14,6 +14,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <algorithm>
+#include <cmath>
 #include "common.h"
 #include "dense_gemm_body.h"
 #include "tall_ring.h"
@@ -300,13 +301,22 @@ struct TallPlan {
     int S, per;
     double us;
 };
-// us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip.  These and the constants of plan_tall are fitted to
-// 300 products of 65 to 4096 rows and 1024 x 1024 to 24576 x 6144, each with up to 42 plans: the estimates are 10 % off, the plans that they
-// pick 1.1 % behind the best.
+// us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip.  These and the constants of walk_us, launch_us and the two
+// plan makers are fitted to 280 products of 65 to 8000 rows and 1024 x 1024 to 57344 x 8192, each with up to 48 plans, weights cold (the copies of
+// a matrix that take turns are more than the caches hold): the estimates are 5 % off, the plans that they pick 0.9 % behind the best, at most 9.
 struct TallCost {
     double alone, busy;
 };
-constexpr TallCost TALL_COST[3][2] = {{{0.310, 0.415}, {0.538, 0.795}}, {{0.389, 0.451}, {0.612, 0.840}}, {{0.643, 0.556}, {0.711, 0.988}}};
+constexpr TallCost TALL_COST[3][2] = {{{0.262, 0.356}, {0.609, 0.599}}, {{0.347, 0.411}, {0.659, 0.705}}, {{0.420, 0.508}, {0.692, 0.853}}};
+// Blocks that walk `per` steps each: a last round that is not full costs more than three quarters of a whole one
+double walk_us(int64_t blocks, int64_t per, const TallCost& c) {
+    const int64_t rounds = blocks / CUS, rest = blocks % CUS;
+    const double alone = per * c.alone, busy = per * c.busy, share = (double)rest / CUS;
+    if (rounds == 0) return alone + std::max(0.0, busy - alone) * share;
+    return std::max(alone, rounds * busy + (rest ? busy * (0.77 + 0.23 * share) : 0.0));
+}
+// ... with the weights' way from HBM, which hides behind the walk as far as one of the two is short
+double launch_us(double walk, int64_t K, int64_t N) { return 5.55 + std::hypot(walk, 2.0 * K * N / 6.33e6); }
 constexpr int MAX_PARTS = 384;  // blocks of the split launch: 48 MiB of fp32 tiles
 
 // Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k: 256 rows of 24576 x 6144 are 48 tiles of 128 x
@@ -319,20 +329,16 @@ TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
         for (int TW = 1; TW <= 2; ++TW) {
             const TallCost c = TALL_COST[BMR - 2][TW - 1];
             const int64_t cb = cdiv64(NT, 4 * TW), tiles = cb * cdiv64(M, 32 * BMR), rounds = tiles / CUS, rest = tiles % CUS;
-            const double alone = 1.6 + steps * c.alone, busy = 1.8 + steps * c.busy, share = (double)rest / CUS;
             for (int S = 1; S <= 12; ++S) {
                 const int64_t per = cdiv64(steps, S);
                 if (S > 1 && (rest == 0 || rest * S > MAX_PARTS || per < 4)) break;
                 if ((S - 1) * per >= steps) continue;
-                double us = rounds * busy;
-                if (S > 1) {
-                    const double fill = (double)(rest * S) / CUS, part = 1.6 + per * c.alone;
-                    us += fill <= 1.0 ? part : std::max(part, (1.8 + per * c.busy) * fill);
-                    us += 4.4 + 2.0 * rest * S * (32 * BMR) * (128 * TW) * 4 / 3.5e6;  // the finish launch, the partial tiles at 3.5 TB/s
-                } else if (rounds == 0) {
-                    us = alone + std::max(0.0, busy - alone) * share;
+                double us;
+                if (S > 1) {  // the finish launch and the partial tiles; behind whole rounds, a launch of its own
+                    us = launch_us(rounds * steps * c.busy + walk_us(rest * S, per, c), K, N) + 1.0 + 0.27 * (S - 1) + (rounds ? 6.7 : 0.0) +
+                         2.0 * rest * S * (32 * BMR) * (128 * TW) * 4 / 8.9e6;
                 } else {
-                    us = std::max(alone, us + (rest ? busy * (0.51 + 0.49 * share) : 0.0));
+                    us = launch_us(walk_us(tiles, steps, c), K, N);
                 }
                 if (us < best_us) {
                     best_us = us;
@@ -360,11 +366,7 @@ TallPlan make_plan_parts(int64_t M, int64_t K, int64_t N) {
                 const int64_t per = cdiv64(steps, S);
                 if (S > 1 && per < 4) break;
                 if ((S - 1) * per >= steps) continue;
-                const int64_t blocks = tiles * S, rounds = blocks / CUS, rest = blocks % CUS;
-                const double alone = 1.6 + per * c.alone, busy = 1.8 + per * c.busy, share = (double)rest / CUS;
-                const double us = (blocks <= CUS ? alone + std::max(0.0, busy - alone) * blocks / CUS
-                                                 : std::max(alone, rounds * busy + (rest ? busy * (0.51 + 0.49 * share) : 0.0))) +
-                                  0.3 * (S - 1) + 2.0 * S * M * N * 4 / 3.5e6;
+                const double us = launch_us(walk_us(tiles * S, per, c), K, N) + 0.06 * (S - 1) + 2.0 * S * M * N * 4 / 4.8e6;
                 if (us < best_us) {
                     best_us = us;
                     best = {BMR, TW, (int)cb, (int)tiles, 0, S, (int)per, us};
