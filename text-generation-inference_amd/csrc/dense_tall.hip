@@ -321,6 +321,9 @@ constexpr int MAX_PARTS = 384;  // blocks of the split launch: 48 MiB of fp32 ti
 
 // Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k: 256 rows of 24576 x 6144 are 48 tiles of 128 x
 // 256 that walk 384 steps each (264 us; 95 split in four), 765 rows of 2048 x 11264 352 tiles of 96 x 128 (44 us; 52 in tiles of 128 x 128).
+// GELU: in the unsplit launch each thread evaluates it 16 BMR TW times, one call behind the other, 0.18 us each; the finish launch has a thread for
+// every four (1024 x 1024 at 65 - 256 rows +5.7 us / +0.9).
+template <bool GELU>
 TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
     const int64_t steps = K / 64, NT = cdiv64(N, 32);
     TallPlan best{};
@@ -340,6 +343,7 @@ TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
                 } else {
                     us = launch_us(walk_us(tiles, steps, c), K, N);
                 }
+                if (GELU && (S == 1 || rounds)) us += 0.18 * 16 * BMR * TW;
                 if (us < best_us) {
                     best_us = us;
                     best = {BMR, TW, (int)cb, (int)tiles, (int)(S > 1 ? tiles - rest : tiles), S, (int)per, us};
@@ -400,9 +404,10 @@ TallPlan kept_plan(int64_t M, int64_t K, int64_t N) {
     return e.plan;
 }
 
-TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
+TallPlan plan_tall(int64_t M, int64_t K, int64_t N, int act) {
     TallPlan p;
-    return plan_from_env(M, K, N, false, p) ? p : kept_plan<make_plan_tall>(M, K, N);
+    if (plan_from_env(M, K, N, false, p)) return p;
+    return act == 4 || act == 5 ? kept_plan<make_plan_tall<true>>(M, K, N) : kept_plan<make_plan_tall<false>>(M, K, N);
 }
 
 TallPlan plan_parts(int64_t M, int64_t K, int64_t N) {
@@ -501,7 +506,7 @@ static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act) {
 // Bytes of scratch of tgis_dense_tall where it is the faster way to this product, -1 where it is not.
 extern "C" int64_t tgis_dense_tall_bytes(int64_t M, int64_t K, int64_t N, int act) {
     if (M < 1 || K < 64 || N < 1 || !(act == 0 || act == 2 || act == 4 || act == 5) || !dense_tall_pays(M, K, N, act)) return -1;
-    return plan_scratch(plan_tall(M, K, N));
+    return plan_scratch(plan_tall(M, K, N, act));
 }
 
 static bool rows_ok(const void* x, int64_t ldx, int64_t K) {  // (a tile's rows are addressed with 31 bits)
@@ -532,7 +537,7 @@ extern "C" int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared,
     TGIS_CHECK_ARG(act != 2 || N % 32 == 0, "tgis_dense_tall: act 2 needs a gate|up image (N / 2 a multiple of 16)");
     TGIS_CHECK_ARG(rows_ok(x, ldx, K), "tgis_dense_tall: x rows must be 16-byte aligned and less than 2^22 elements apart");
     if (M == 0) return TGIS_OK;
-    const TallPlan p = plan_tall(M, K, N);
+    const TallPlan p = plan_tall(M, K, N, act);
     TGIS_CHECK_ARG(plan_scratch(p) == 0 || (workspace && workspace_bytes >= plan_scratch(p)), "tgis_dense_tall: workspace too small");
     DTallArgs a = tall_args(x, ldx, prepared, M, K, N, workspace);
     a.bias = bias;
