@@ -184,7 +184,7 @@ int tgis_dense_tall_partial(const void* x, int64_t ldx, const void* prepared, in
 
 /* The layers of a dense Llama model (no biases but qkv's, one rank) on T rows of prompts: the launches of its forward, one call.  Images as
  * tgis_dense_prepare makes them; qkv_rope is the rope image, for T < TGIS_DENSE_TALL_MIN_M, where tgis_dense_rope_ok must hold; qkv the plain
- * one, for more rows, where tgis_dense_tall_bytes of the four products must not be negative. */
+ * one, for more rows.  There tgis_dense_tall_bytes of gate_up, past 256 rows of all four products, must not be negative. */
 typedef struct {
     const void *input_norm, *qkv, *qkv_rope, *qkv_bias, *o, *post_norm, *gate_up, *down;
     void *k_pool, *v_pool;
@@ -198,7 +198,7 @@ typedef struct {
     const void *cos, *sin;
     void *y, *res[2];      /* [T][hidden]; the residual stream is left in res[0] */
     void *qkv, *att, *act; /* [T][(H + 2 Hkv) D], [T][H D], [T][inner] */
-    float* slabs;          /* up to 256 rows: the last product is left here, num_slabs partial sums (tgis_rmsnorm_residual_partial) */
+    float* slabs;          /* up to 256 rows: products are left here, the last one as num_slabs partial sums (tgis_rmsnorm_residual_partial) */
     int64_t slabs_bytes;
     void* out;             /* more rows: [T][hidden], the last product (slabs NULL) */
     void* workspace;

@@ -58,10 +58,12 @@ def test_int4_library(M, K, N, act, pays):
     assert lib.tgis_gptq_gemm_fused_pays(256, K, N, K // 64, 1, act) == 1
 
 
-# the dense prefill kernel: from 65 rows on, past 256 where the library's tiles would leave the chip idle or an activation launch is saved
+# the dense prefill kernel: from 65 rows on where the streaming kernel's passes are more than one short round, past 256 where the library's tiles would
+# leave the chip idle or an activation launch is saved
 @pytest.mark.parametrize("M,K,N,act,pays", [
-    (64, 2048, 2048, 0, 0), (65, 2048, 2048, 0, 1), (256, 6144, 24576, 4, 1), (257, 6144, 24576, 4, 0), (1400, 2048, 2048, 0, 1), (1401, 2048, 2048, 0, 0),
-    (500, 2048, 6144, 0, 1), (501, 2048, 6144, 0, 0), (100, 2040, 2048, 0, 0), (100, 2048, 1024, 0, 1), (100, 2048, 1023, 0, 0), (300, 448, 2048, 0, 0), (200, 64, 2048, 0, 1), (512, 4096, 22016, 2, 0), (513, 4096, 22016, 2, 1), (300, 2048, 11264, 2, 1),
+    (64, 2048, 2048, 0, 0), (65, 2048, 2048, 0, 0), (65, 4096, 4096, 0, 1), (256, 6144, 24576, 4, 1), (257, 6144, 24576, 4, 0), (1400, 2048, 2048, 0, 1), (1401, 2048, 2048, 0, 0),
+    (500, 2048, 6144, 0, 1), (501, 2048, 6144, 0, 0), (100, 2040, 2048, 0, 0), (100, 2048, 1024, 0, 0), (100, 8192, 1024, 0, 1), (100, 8192, 1023, 0, 0), (300, 448, 2048, 0, 0), (200, 64, 2048, 0, 1), (512, 4096, 22016, 2, 0), (513, 4096, 22016, 2, 1), (300, 2048, 11264, 2, 1),
+    (65, 320, 1280, 0, 1), (65, 320, 1280, 5, 0), (896, 3072, 5120, 0, 0), (700, 3072, 5120, 0, 1), (900, 24576, 6144, 0, 1), (600, 28672, 8192, 0, 0), (600, 4096, 28672, 2, 0),
     (8192, 2048, 11264, 2, 1), (8193, 2048, 11264, 2, 0), (100, 2048, 2048, 1, 0), (0, 2048, 2048, 0, 0),
 ])
 def test_dense_tall(M, K, N, act, pays):
@@ -94,9 +96,18 @@ def test_dense_tall_scratch():
 
 
 # split sums of the dense prefill kernel: a second block on some CUs costs more than three quarters of a round, so the parts end within a whole one
-@pytest.mark.parametrize("M,K,N,parts", [(128, 6144, 6144, 4), (100, 6144, 6144, 5), (160, 8192, 10240, 3), (256, 11008, 4096, 4), (65, 24576, 6144, 5), (128, 2048, 2048, 4)])
+@pytest.mark.parametrize("M,K,N,parts", [(128, 6144, 6144, 4), (100, 6144, 6144, 5), (160, 8192, 10240, 3), (256, 11008, 4096, 4), (65, 24576, 6144, 5), (128, 4096, 4096, 4)])
 def test_dense_tall_parts(M, K, N, parts):
     from tgis_amd import native
 
     rows = -(-M // 32) * 32
     assert native.load_library().tgis_dense_tall_partial_bytes(M, K, N) == rows * N * 4 * parts
+
+
+# ... and stay parts of the streaming kernel where its passes are one round of short blocks, more than half full
+@pytest.mark.parametrize("M,K,N,serves", [(64, 4096, 4096, 0), (65, 2048, 2048, 0), (256, 2048, 2560, 1), (192, 2048, 2560, 0), (128, 1024, 1024, 1), (256, 1024, 1024, 0), (128, 4096, 1024, 1),
+                                          (128, 2560, 1024, 0), (257, 4096, 4096, 0), (100, 4096, 1000, 0)])
+def test_dense_tall_parts_or_passes(M, K, N, serves):
+    from tgis_amd import native
+
+    assert (native.load_library().tgis_dense_tall_partial_bytes(M, K, N) >= 0) == bool(serves)

@@ -66,7 +66,7 @@ def test_same_bits(gpu_device, monkeypatch, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_cache_writes_token_by_token(gpu_device, monkeypatch, dtype):
-    """TGIS_PREFILL_KV=0: the same bits, but for the order of the sums of 65 - 256 rows' queries, keys and values."""
+    """TGIS_PREFILL_KV=0: the same bits."""
     from tgis_amd import native
     from tgis_amd.models import flash_causal_lm
     from tgis_amd.models.custom_modeling.flash_llama_modeling import FlashLlamaModel
@@ -83,13 +83,7 @@ def test_cache_writes_token_by_token(gpu_device, monkeypatch, dtype):
         with monkeypatch.context() as m:
             m.setattr(FlashLlamaModel, "plain_layers", lambda self, *a: [])
             want = steps(lm, cfg.vocab_size, lens)
-        for a, b in zip(got, want):
-            if 65 <= sum(lens) <= 256:
-                # what differs is here and there a rounding to the model dtype, which three layers carry on: below four steps in the norm of all
-                a, b, step = a.double(), b.double(), 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-                assert float((a - b).norm() / b.norm()) < 4 * step
-            else:
-                assert torch.equal(a, b)
+        assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want)), lens
 
 
 @pytest.mark.parametrize("kw,lens", [(dict(quantize="gptq"), [20]), (dict(hidden_size=256, num_attention_heads=4), [70]),

@@ -482,30 +482,48 @@ int run_tall(const TallPlan& p, DTallArgs& a, int act, hipStream_t st) {
 }
 }  // namespace
 
-// Is this kernel the faster way?  us, the alternative / this kernel, weights cold, launches back to back.
+// Is this kernel the faster way?  us, the alternative / this kernel, weights cold, launches back to back; of 480 products on either side of 256 rows the
+// choice is 0.5 and 2.6 % behind the better of the two, with GELU 0.4 and 0.6, as parts 0.3, with SiLU 0.3 and 0.9.
 // Up to 256 rows the alternative is the weight-streaming kernel, which goes over the weights once per 64 rows (a product below 65 rows stays there):
-//   65 / 128 / 140 / 256 rows: 2048 x 2048 9.9 / 8.9, 10.7 / 9.6, 11.4 / 9.9, 12.4 / 10.9; 1024 x 1024 8.0 / 7.8, 8.2 / 7.9, 8.3 / 7.9, 8.7 / 8.0; 5632 x
-//   2048 14.8 / 12.2, 15.5 / 12.6, 20 / 13.6, 21 / 15; 2048 x 11264 with SiLU 18.6 / 16.3, 18.8 / 18.4, 30 / 20, 36 / 24; 4096 x 12288 33 / 26, 32 / 30,
-//   55 / 34, 65 / 42; 6144 x 24576 98 / 63, 106 / 76, 157 / 88, 195 / 99; 24576 x 6144 109 / 66, 110 / 68, 203 / 84, 219 / 95
-// Above, it is the library, with a launch of its own for the activation.  Its 256 x 256 tiles at 1.2 - 1.45 PFLOP/s win wherever they fill the chip:
-//   act 0 / GELU, 300 / 600 / 1024 / 1400 / 2048 rows: 2048 x 2048 10.7 / 11.6, 13.8 / 12.5, 15.9 / 13.6, 19.0 / 18.2, 21.6 / 23.6; 5632 x 2048 24 / 16, 30 /
-//   25, 37 / 32, 45 / 40, 54 / 54; 6144 x 6400 44 / 42, 64 / 59, 92 / 85, 101 / 115, 139 / 155; 24576 x 6144 200 / 123, 278 / 180, 405 / 320, 621 / 380, 468 /
-//   530; 4096 x 12288 53 / 52, 66 / 68, 93 / 115; 6144 x 24576 118 / 130, 202 / 180, 267 / 264, 386 / 379, 463 / 497; 2048 x 6144 15.6 / 13.8, 22 / 23,
-//   29 / 36: hence bounds on rows x columns, against the depth and at 6.3 million, and on the rows
-//   act 2, 300 / 433 / 600 / 1024 / 2048 / 4096 / 8186 / 16128 rows: 1024 x 5632 14 / 8.4, 17 / 11, 20 / 13, 26 / 18, 44 / 31, 69 / 54; 2048 x 11264 32 / 28, 37 /
-//   30, 39 / 35, 60 / 54, 100 / 90, 187 / 170, 410 / 316, 626 / 620; 4096 x 22016 78 / 86, 95 / 97, 140 / 117, 190 / 177, 440 / 335, 720 / 627, 1260 / 1249,
-//   2294 / 2500
+//   65 / 128 / 192 / 256 rows: 4096 x 4096 17.1 / 14.9, 17.8 / 16.1, 24.6 / 18.3, 25.4 / 21; 5632 x 2048 15.3 / 14.8, 15.4 / 15.0, 20.2 / 16.1, 20.8 / 17.5; 4096 x
+//   12288 37.6 / 28.4, 33.2 / 31.1, 60.5 / 38, 64.5 / 42; 6144 x 24576 106 / 68, 113 / 78, 166 / 95, 198 / 100; 24576 x 6144 120 / 68, 115 / 73, 218 / 87, 216 /
+//   95; with SiLU 1024 x 5632 9.5 / 8.9, 9.8 / 10, 17 / 10, 17 / 10; 2048 x 11264 21 / 17, 21 / 19, 34 / 23, 40 / 25
+// It stays where its passes are one round of two-tile blocks of up to 1024 k that split k: 2048 x 2048 10.1 / 10.2, 10.9 / 11.3, 12.0 / 12.6, 12.5 / 13.9; 1536
+// x 1536 8.9 / 9.4, 9.3 / 10.0, 10.1 / 10.8, 11.7 / 10.8; 2048 x 1024 8.9 / 9.6, 9.3 / 10.2, 9.8 / 10.6, 10.5 / 10.9; as parts in front of a norm from 128 such
+// blocks of up to 2560 k on (2048 x 2048 9.7 / 9.8, 10.7 / 11.2, 11.9 / 12.3, 12.5 / 13.1; but 1024 x 1024 7.9 / 7.5, 8.0 / 7.8 and 4096 x 1024 10.9 / 9.9,
+// 11.1 / 11.2).  GELU of fewer than eight steps, which have no split: 320 x 1280 10.1 / 11.2.
+// Above, it is the library, with a launch of its own for the activation.
+//   act 0 / GELU: it wins where its tiles of 128 x 256 fill more than half the chip (4096 x 6144 at 800, 1024 rows 47 / 56, 52 / 61; 3072 x 5120 at 900, 1400 40 / 44,
+//   49 / 50; 28672 x 8192 at 600 259 / 346; layers of 3072, 8192 at 1390 rows 394 / 371 us with it, of 4096, 14336 at 900 494 / 467), but not on narrow products of
+//   long k (24576 x 6144 at 700, 1024 rows 298 / 278, 408 / 349; 13824 x 5120 at 1200 1.7).  Below that the two are close (300, 512, 1024 rows: 2048 x
+//   2560 13.3 / 14.8, 15.3 / 16.6, 22.9 / 19.7; 4096 x 4096 26.2 / 25.6, 30 / 31, 41.9 / 42.7; 5632 x 2048 26 / 22.5, 26.7 / 23.6, 40 / 35; 6144 x 6400 44.7 / 43.5,
+//   67 / 60, 91 / 88), and inside a model this kernel is the faster one also where it is not alone: 22 layers of 2048, 5632 at 257, 400 rows 2781 / 2466,
+//   2810 / 2669 us, both launched one by one
+//   act 2: up to 32 Mi weights always (300, 1024, 4096, 8192 rows: 1024 x 5632 0.60, 0.77, 0.91, 0.82 of the library and the activation; 2048 x 11264 0.86, 0.93,
+//   0.94, 0.83); larger ones from 513 rows on, but for widths of whole 4096s, on which the library is at its best (600, 1400, 2048, 8192 rows: 4096 x 22016
+//   0.90, 0.79, 0.82, 0.99; 5120 x 27648 0.98, 0.92, 0.94, 0.98; 3072 x 16384 1.14, 0.97, 1.06, 1.07; 4096 x 28672 0.95, 0.99, 1.03, 1.11; 8192 x 57344 0.97,
+//   1.08, 1.16, 1.16)
 // Narrow and shallow ones stay where they were: 2048 x 512 at 128 / 300 rows 8.6 / 9.2, 8.2 / 9.0; 64 x 2048 at 600, 1400 rows 4.4 / 5.1, 5.2 / 6.8.
-static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act) {
-    if (M < TGIS_DENSE_TALL_MIN_M || K % 64 != 0 || N < 1024) return false;
-    if (M <= 256) return true;
-    if (act == 2) return M <= 8192 && (M > 512 || K * N <= (32 << 20));
-    return M <= 1400 && K >= 512 && M * N <= std::min<int64_t>(1500 * K, 6300000);
+static bool passes_in_a_round(int64_t M, int64_t K, int64_t N, int64_t from_blocks) {
+    const dense::DensePlan pass = dense::plan_dense(K, N, M);
+    const int64_t blocks = cdiv64(cdiv64(N, 32), pass.TN) * cdiv64(M, 64) * pass.S;
+    return pass.TN == 2 && pass.S > 1 && pass.KR <= 1024 && blocks >= from_blocks && blocks <= CUS;
+}
+static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act, bool parts) {
+    if (M < TGIS_DENSE_TALL_MIN_M || K < 64 || K % 64 != 0 || N < 1024) return false;
+    TallPlan forced;
+    if (plan_from_env(M, K, N, parts, forced)) return true;
+    const bool gelu = act == 4 || act == 5;
+    if (parts) return M <= 256 && !(K <= 2560 && passes_in_a_round(M, K, N, 128));
+    if (M <= 256) return act == 2 || (!passes_in_a_round(M, K, N, 0) && !(gelu && K < 512));
+    if (act == 2) return M <= 8192 && (K * N <= (32 << 20) || (M > 512 && N % 4096 != 0));
+    if (M > 1400 || K < 512 || M * N > std::min<int64_t>(1500 * K, 6300000)) return false;
+    return cdiv64(M, 128) * cdiv64(N, 256) <= CUS / 2 || (K > 9600 && N < 8192);
 }
 
 // Bytes of scratch of tgis_dense_tall where it is the faster way to this product, -1 where it is not.
 extern "C" int64_t tgis_dense_tall_bytes(int64_t M, int64_t K, int64_t N, int act) {
-    if (M < 1 || K < 64 || N < 1 || !(act == 0 || act == 2 || act == 4 || act == 5) || !dense_tall_pays(M, K, N, act)) return -1;
+    if (!(act == 0 || act == 2 || act == 4 || act == 5) || !dense_tall_pays(M, K, N, act, false)) return -1;
     return plan_scratch(plan_tall(M, K, N, act));
 }
 
@@ -556,7 +574,7 @@ extern "C" int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared,
 
 // The product as fp32 partial sums for the consumers of tgis_dense_gemm_partial's, in the same layout; up to 256 rows.
 extern "C" int64_t tgis_dense_tall_partial_bytes(int64_t M, int64_t K, int64_t N) {
-    if (M > 256 || tgis_dense_tall_bytes(M, K, N, 0) < 0) return -1;
+    if (!dense_tall_pays(M, K, N, 0, true)) return -1;
     return cdiv64(M, 32) * 32 * cdiv64(N, 32) * 32 * 4 * plan_parts(M, K, N).S;
 }
 

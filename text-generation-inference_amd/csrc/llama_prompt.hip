@@ -1,6 +1,5 @@
 // The layers of a dense Llama model on the rows of prompts, launched from here: the launches that the model's own forward makes one by one,
-// with the same arguments and the same results, without its way back to Python between them.  (One exception: where `fresh` is not set, qkv of
-// TGIS_DENSE_TALL_MIN_M to 256 rows is finished here, and left in parts to the rotary launch there: another order of its fp32 sums.)  A layer of a short prompt is six launches of 4 to
+// with the same arguments and the same results, without its way back to Python between them.  A layer of a short prompt is six launches of 4 to
 // 16 us, each of which took 9 us of host time to prepare; here it is 2 - 3 us.  47 tokens through 22 layers of 2048: 1820 -> 1540 us.
 #include "common.h"
 
@@ -37,15 +36,22 @@ extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, Tgi
         }
         return TGIS_OK;
     };
-    auto product = [&](const void* in, const void* image, int64_t K) -> int {  // [T, hidden], summed by the norm behind it
-        if (tall && p->slabs)
-            return tgis_dense_tall_partial(in, K, image, T, K, p->hidden, p->dtype, p->slabs, p->slabs_bytes, &S, &ld, stream);
-        if (tall) {
+    // which of the two kernels leaves a product in parts, and whether qkv is left so
+    const bool left = p->slabs != nullptr;
+    auto tall_parts = [&](int64_t K, int64_t N) { return tall && left && tgis_dense_tall_partial_bytes(T, K, N) >= 0; };
+    const bool qkv_tall = tall_parts(p->hidden, QKV), o_tall = tall_parts(HD, p->hidden), down_tall = tall_parts(p->inner, p->hidden);
+    const bool qkv_whole = tall && (!left || (p->fresh && tgis_dense_tall_bytes(T, p->hidden, QKV, 0) >= 0));
+    auto parts = [&](bool by_tall, const void* in, const void* image, int64_t K, int64_t N, int* slabs, int64_t* row) -> int {
+        if (by_tall) return tgis_dense_tall_partial(in, K, image, T, K, N, p->dtype, p->slabs, p->slabs_bytes, slabs, row, stream);
+        return tgis_dense_gemm_partial(in, K, image, T, K, N, p->dtype, 0, p->slabs, p->slabs_bytes, slabs, row, stream);
+    };
+    auto product = [&](bool by_tall, const void* in, const void* image, int64_t K) -> int {  // [T, hidden], summed by the norm behind it
+        if (!left) {
             x0 = p->out;
             return tgis_dense_tall(in, K, image, nullptr, p->out, p->hidden, T, K, p->hidden, p->dtype, 0, 0, 0.f, 0.f, ws + 4096,
                                    p->workspace_bytes - 4096, stream);
         }
-        return tgis_dense_gemm_partial(in, K, image, T, K, p->hidden, p->dtype, 0, p->slabs, p->slabs_bytes, &S, &ld, stream);
+        return parts(by_tall, in, image, K, p->hidden, &S, &ld);
     };
     for (int i = 0; i < n_layers; ++i) {
         const TgisLlamaLayer& l = layers[i];
@@ -53,6 +59,12 @@ extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, Tgi
         if (!tall) {
             TRY(tgis_dense_gemm_rope(p->y, p->hidden, l.qkv_rope, l.qkv_bias, p->positions, p->slots, p->cos, p->sin, p->qkv, QKV, l.k_pool, l.v_pool,
                                      T, p->hidden, QKV, p->H, p->Hkv, p->D, p->dtype, stream));
+        } else if (!qkv_whole) {
+            int qkv_slabs = 0;
+            int64_t row = 0;
+            TRY(parts(qkv_tall, p->y, l.qkv, p->hidden, QKV, &qkv_slabs, &row));
+            TRY(tgis_rope_kv_write_partial(p->slabs, qkv_slabs, row, l.qkv_bias, p->qkv, QKV, p->cos, p->sin, p->positions, p->slots, l.k_pool, l.v_pool, T,
+                                           p->H, p->Hkv, p->D, p->D, p->dtype, stream));
         } else {
             TRY(tgis_dense_tall(p->y, p->hidden, l.qkv, l.qkv_bias, p->qkv, QKV, T, p->hidden, QKV, p->dtype, 0, 0, 0.f, 0.f, ws + 4096,
                                 p->workspace_bytes - 4096, stream));
@@ -65,7 +77,7 @@ extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, Tgi
         }
         TRY(tgis_attn_paged(p->qkv, QKV, l.k_pool, l.v_pool, p->block_tables, p->max_pages, p->ctx_lens, p->cu_seqlens, p->att, HD, p->B, p->H,
                             p->Hkv, p->D, p->max_q_len, p->max_ctx, p->scale, p->dtype, 1, nullptr, 0, stream));
-        TRY(product(p->att, l.o, HD));
+        TRY(product(o_tall, p->att, l.o, HD));
         TRY(norm(l.post_norm, p->eps));
         if (tall)
             TRY(tgis_dense_tall(p->y, p->hidden, l.gate_up, nullptr, p->act, p->inner, T, p->hidden, 2 * p->inner, p->dtype, 0, 2, 0.f, 0.f, ws + 4096,
@@ -73,7 +85,7 @@ extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, Tgi
         else
             TRY(tgis_dense_gemm(p->y, p->hidden, l.gate_up, nullptr, p->act, p->inner, T, p->hidden, 2 * p->inner, p->dtype, 0, 2, ws,
                                 p->workspace_bytes, stream));
-        TRY(product(p->act, l.down, p->inner));
+        TRY(product(down_tall, p->act, l.down, p->inner));
     }
     p->num_slabs = S;
     p->slab_ld = ld;

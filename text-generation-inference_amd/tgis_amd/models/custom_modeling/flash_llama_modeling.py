@@ -368,7 +368,11 @@ class FlashLlamaModel:
             return []
         tall = rows >= native.DENSE_TALL_MIN_M
         shapes = {"qkv": ((H + 2 * Hkv) * D, hidden), "o": (hidden, H * D), "gate_up": (2 * inner, hidden), "down": (hidden, inner)}
-        if tall and not all(native.dense_tall_serves(rows, K, N, 2 if name == "gate_up" else 0) for name, (N, K) in shapes.items()):
+        if tall and any(K % 64 or N < native.DENSE_TALL_MIN_N for N, K in shapes.values()):
+            return []
+        # past the rows whose products may be left in parts, by either kernel, all four are the prefill kernel's
+        if tall and not all(native.dense_tall_serves(rows, K, N, 2 if name == "gate_up" else 0) for name, (N, K) in shapes.items()
+                            if rows > native.PARTIAL_MAX_M or name == "gate_up"):
             return []
         if rows <= native.PARTIAL_MAX_M and not DEFER_REDUCE:  # (the launches of such steps leave split sums to the norms)
             return []

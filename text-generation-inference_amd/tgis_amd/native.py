@@ -687,6 +687,7 @@ def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f3
 
 
 DENSE_TALL_MIN_M = 65  # TGIS_DENSE_TALL_MIN_M
+DENSE_TALL_MIN_N = 1024  # columns from which dense_tall is ever the faster way
 
 
 def dense_tall_serves(M: int, K: int, N: int, act: int = 0) -> bool:
@@ -706,6 +707,19 @@ def dense_tall_bytes(x: torch.Tensor, w: DenseWeight, act: int = 0) -> int:
     return got
 
 
+def _tall_slabs(M: int, w: DenseWeight):
+    got = w.plans[("tall slabs", M)] = (load_library().tgis_dense_tall_partial_bytes(M, w.K, w.N), _c_int(), _c_i64())
+    return got
+
+
+def dense_tall_partial_bytes(x: torch.Tensor, w: DenseWeight) -> int:
+    """The slabs of dense_tall_partial where it is the faster way to leave x @ w^T to a consumer and x is as it reads it, else -1."""
+    M, ld = x.shape[0], x.stride(0)
+    if x.dim() != 2 or not DENSE_TALL_MIN_M <= M <= PARTIAL_MAX_M or x.stride(1) != 1 or ld % 8 or not w.K <= ld < 1 << 22 or x.data_ptr() % 16:
+        return -1
+    return (w.plans.get(("tall slabs", M)) or _tall_slabs(M, w))[0]
+
+
 def dense_tall(x: torch.Tensor, w: DenseWeight, ws: Workspace, nbytes: int, bias=None, act: int = 0, alpha: float = 0.0, limit: float = 0.0,
                out=None, out_f32: bool = False) -> torch.Tensor:
     """dense_gemm of a prefill's rows (nbytes: dense_tall_bytes); act 0, 4, 5 or 2 (limit > 0: the clamped unit of dense_gemm_clamped_glu)."""
@@ -721,16 +735,14 @@ def dense_tall(x: torch.Tensor, w: DenseWeight, ws: Workspace, nbytes: int, bias
 
 
 def dense_tall_partial(x: torch.Tensor, w: DenseWeight, bias=None) -> Partial:
-    """dense_gemm_partial of up to PARTIAL_MAX_M rows, where dense_tall_bytes says so."""
+    """dense_gemm_partial of up to PARTIAL_MAX_M rows, where dense_tall_partial_bytes is not negative."""
     assert x.dim() == 2 and x.stride(1) == 1 and x.dtype == w.dtype and x.shape[1] == w.K and not w.flags
-    lib, M = load_library(), x.shape[0]
-    plan = w.plans.get(("tall slabs", M))
-    if plan is None:
-        plan = w.plans[("tall slabs", M)] = (lib.tgis_dense_tall_partial_bytes(M, w.K, w.N), _c_int(), _c_i64())
-    nbytes, S, ld = plan  # (S and ld are of the plan that this launch runs, which TGIS_DTALL_PLAN may have changed)
+    M = x.shape[0]
+    nbytes, S, ld = w.plans.get(("tall slabs", M)) or _tall_slabs(M, w)
     slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
-    _check(lib.tgis_dense_tall_partial(_ptr(x), x.stride(0), _ptr(w.image), M, w.K, w.N, dtype_code(w.dtype), _ptr(slabs), nbytes,
-                                       ctypes.byref(S), ctypes.byref(ld), _stream()), "tgis_dense_tall_partial")
+    # (S and ld: of the plan that this launch runs, which TGIS_DTALL_PLAN may have changed)
+    _check(load_library().tgis_dense_tall_partial(_ptr(x), x.stride(0), _ptr(w.image), M, w.K, w.N, dtype_code(w.dtype), _ptr(slabs), nbytes,
+                                                  ctypes.byref(S), ctypes.byref(ld), _stream()), "tgis_dense_tall_partial")
     p = Partial(slabs, S.value, ld.value, M, w.N, bias)
     p.dtype = w.dtype
     return p
@@ -846,15 +858,16 @@ def llama_prompt(layers, x, ws: Workspace, positions, slots, cu_seqlens, block_t
     y, res0, res1, qkv, att, act = new(hidden), new(hidden), new(hidden), new(qkv_cols), new(H * D), new(inner)
     out = slabs = None
     nbytes = 0
+    if T <= PARTIAL_MAX_M:
+        for K, N in ((hidden, qkv_cols), (H * D, hidden), (inner, hidden)):
+            got = lib.tgis_dense_tall_partial_bytes(T, K, N)
+            nbytes = max(nbytes, got if got >= 0 else lib.tgis_dense_gemm_partial_bytes(T, K, N))
+    else:
+        out = new(hidden)
     if tall:
-        if T <= PARTIAL_MAX_M:
-            nbytes = max(lib.tgis_dense_tall_partial_bytes(T, K, hidden) for K in (H * D, inner))
-        else:
-            out = new(hidden)
         ws.ensure(4096 + max(lib.tgis_dense_tall_bytes(T, K, N, a) for K, N, a in
                              ((hidden, qkv_cols, 0), (H * D, hidden, 0), (hidden, 2 * inner, 2), (inner, hidden, 0))))
     else:
-        nbytes = max(lib.tgis_dense_gemm_partial_bytes(T, K, hidden) for K in (H * D, inner))
         ws.ensure(lib.tgis_dense_gemm_workspace_bytes(T, hidden, 2 * inner))
     if out is None:
         slabs = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)

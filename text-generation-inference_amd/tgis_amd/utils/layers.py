@@ -144,10 +144,10 @@ class FastLinear:
                 return native.dense_gemm(x, self.prepared, workspace(x.device), bias=self.bias, act=2)
             return native.act_mul(F.linear(x, self.weight, self.bias), self.out_features // 2)
         defers = partial and x.shape[0] <= native.PARTIAL_MAX_M and DEFER_REDUCE and not out_f32
-        tall = self.tall(x) if not act and (not out_f32 or x.shape[0] <= SKINNY_MAX_M) else -1
+        if defers and not act and DENSE_TALL and native.dense_tall_partial_bytes(x, self.prepared) >= 0:
+            return native.dense_tall_partial(x, self.prepared, bias=self.bias)
+        tall = self.tall(x) if not act and not defers and (not out_f32 or x.shape[0] <= SKINNY_MAX_M) else -1
         if tall >= 0:
-            if defers:
-                return native.dense_tall_partial(x, self.prepared, bias=self.bias)
             return native.dense_tall(x, self.prepared, workspace(x.device), tall, bias=self.bias, out_f32=out_f32)
         if defers:
             # the split-K sum (and the bias) is finished by the consumer kernel (add+norm / rope): no reduce launch
