@@ -306,8 +306,8 @@ struct TallPlan {
 };
 
 // us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip (several blocks on each; clocks drop under
-// the matrix cores' load).  Fitted to launches of 23 - 400 us at the 7B shapes; over nine matrices and ten row counts from 140 to 3000 the
-// plans that the model picks are 0.6 % behind the best of up to 24 that were timed at each size.
+// the matrix cores' load).  Fitted to launches of 23 - 400 us at the 7B shapes; over 21 matrices and 16 row counts from 65 to 6000, weights
+// cold, the plans that the model picks are 1.1 % up to 256 rows, 0.6 above behind the best of up to 48 that were timed at each size.
 struct TallCost {
     double alone, busy;
 };
@@ -315,7 +315,9 @@ constexpr TallCost TALL_COST[3][2] = {{{0.33, 0.286}, {0.42, 0.50}}, {{0.41, 0.3
 
 // Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k.  One size does not do: 765 rows of
 // a 7B gate_up are 516 tiles of 128 x 256, two rounds and four tiles, which take a third round (187 us; 161 with the four split in
-// eight); a 7B qkv at that size is 768 tiles of 96 x 128, three whole rounds (86 us against 101 for 288 of 128 x 256).
+// eight); a 7B qkv at that size is 768 tiles of 96 x 128, three whole rounds (86 us against 101 for 288 of 128 x 256).  (With 12 us for a split
+// behind no whole round, where it costs 7, 3072 x 3072 at 129 - 192 rows was 96 unsplit tiles of 18.6 us, 14.7 in three parts; 5120 x 5120 at 256
+// 30.6 / 26.7, 8192 x 3072 at 600 51 / 47, 5632 x 2048 at 765 34 / 30.)
 TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
     const int64_t steps = K / 64, NT = cdiv64(N, 32);
     TallPlan best{};
@@ -330,8 +332,8 @@ TallPlan plan_tall(int64_t M, int64_t K, int64_t N) {
                 if (S > 1 && (rest == 0 || rest * S > CUS || per < 4)) break;
                 if ((S - 1) * per >= steps) continue;  // an empty last split
                 double us = rounds * busy;
-                if (S > 1)  // the splits, their fp32 tiles written and read, and the launch that adds them
-                    us += 4.0 + per * c.alone + 8.0 + 2.0 * rest * S * (32 * BMR) * (128 * TW) * 4 / 4e6;
+                if (S > 1)  // the splits, their fp32 tiles written and read, and the launch that adds them; behind whole rounds, a launch of its own
+                    us += 7.0 + (rounds ? 5.0 : 0.0) + per * c.alone + 2.0 * rest * S * (32 * BMR) * (128 * TW) * 4 / 4e6;
                 else if (rounds == 0)
                     us = alone + std::max(0.0, busy - alone) * share;
                 else
@@ -461,17 +463,14 @@ bool gptq::tall_before_library(int64_t M, int64_t K, int64_t N, int act) {
 //           10240 49.1 / 45.5, 88.9 / 56.2; 28672 x 8192 146 / 98, 162 / 126
 //   act 2:  2048 x 11264 at 65 / 128 / 129 / 256 rows 15.1 / 15.8, 15.1 / 13.7, 26.1 / 17.7, 28.3 / 19.7; 4096 x 22016 45.5 / 31.0, 46.7 / 34.9,
 //           67.5 / 44.9, 74.0 / 55.7; 8192 x 57344 185 / 92, 185 / 121, 272 / 177, 348 / 225; 1024 x 8192 11.9 / 11.4, 13.6 / 9.2, 10.7 / 8.7, 11.3 / 9.0
-// The passes' time is that of their rounds of 256 blocks, each its chunks of 256 k per k-part (fitted to 30 shapes, within 8 %); of the 63
-// (matrix, rows) that were timed three go the slower way by more than 7 %, by up to 2.4 us (4096 x 4096 at 129
-// rows; 2048 x 11264 with SiLU at 96 and 128).
+// The passes' time is that of their rounds of 256 blocks, each its chunks of 256 k per k-part (fitted to 30 shapes, within 8 %).
 static bool pays_below_257_rows(int64_t M, int64_t K, int64_t N, int act) {
     const gptq::GemmPlan pass = gptq::plan_gemm(K, N, act, M);
     const double rounds = (double)cdiv64(cdiv64(cdiv64(N, 32), pass.TN) * cdiv64(M, 64) * pass.S, CUS), chunks = pass.KR / 256 / pass.WK;
     const double passes = act == 2 ? 2.0 + rounds * (2.0 + chunks * (pass.TN == 4 ? 2.65 : 1.9))
                                    : 5.0 + rounds * (3.0 + chunks * (pass.TN == 4 ? 2.45 : 1.65));
     const TallPlan p = plan_tall(M, K, N);
-    const bool split = p.whole < p.tiles;  // (the model is 4 us above split plans)
-    return (split ? p.us - (act == 2 ? 4.0 : 3.5) : act == 2 ? 1.1 * p.us - 1.0 : 1.1 * p.us + 1.0) <= passes;
+    return (act == 2 ? 1.1 * p.us - 1.0 : 1.1 * p.us + 1.0) <= passes;
 }
 bool gptq::tall_ok(int64_t M, int64_t K, int64_t N, int64_t groups, bool act_order, int act) {
     if (M < tall_min_m(act) || !tall_serves(K, groups, act_order, act)) return false;
