@@ -76,3 +76,15 @@ def test_prefill_of_the_ends(gpu_device, monkeypatch, case):
     size = want.double().square().mean(-1, keepdim=True).sqrt()
     assert ((got - want).abs() <= TOL[dtype] * size).all(), float(((got - want).abs() / size).max())
     assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(left, want_left))
+
+
+@pytest.mark.parametrize("lens,recurrent,cut", [([128], False, True), ([127], False, False), ([128], True, True), ([16] * 8, True, False), ([16] * 8, False, True),
+                                                ([24] * 8, True, True), ([2] * 64, False, True), ([1] * 192, True, False), ([32] * 4, True, True)])
+def test_rows_that_are_cut(gpu_device, lens, recurrent, cut):
+    from tgis_amd.models.custom_modeling.flash_llama_modeling import KVArgs
+
+    kv = KVArgs(cache=None, block_tables=None, ctx_lens=None, slots=None, max_q_len=max(lens), max_ctx=max(lens), num_splits=1,
+                ends=torch.tensor(lens, device=gpu_device).cumsum(0) - 1)
+    assert kv.cuts_to_ends(sum(lens), recurrent) == cut
+    kv.residual_trace = []
+    assert not kv.cuts_to_ends(sum(lens), recurrent)

@@ -118,7 +118,7 @@ class FlashLenisunModel:
         n = len(self.layers)
         for i, layer in enumerate(self.layers):
             # the last layer of a prefill of which only the last tokens' logits are wanted
-            ends = kv.ends if i + 1 == n and kv.cuts_to_ends(x.shape[0]) else None
+            ends = kv.ends if i + 1 == n and kv.cuts_to_ends(x.shape[0], recurrent=True) else None
             if layer.kind == "attention":
                 y, qkv = layer.mixer.forward(h, position_ids, kv, v_first, ends=ends)
                 if i == self.first_blender:
@@ -161,7 +161,7 @@ class FlashLenisunForCausalLM:
                 lm_head_indices: Optional[torch.Tensor] = None):
         """fp32 logits [T or len(lm_head_indices), vocab]."""
         hidden = self.model(input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv)
-        if lm_head_indices is not None and not kv.cuts_to_ends(position_ids.shape[0]):
+        if lm_head_indices is not None and not kv.cuts_to_ends(position_ids.shape[0], recurrent=True):
             hidden = hidden.index_select(0, lm_head_indices)
         # fp32 logits from the weight-streaming kernel's fp32 accumulators, 256 rows at a time (the library GEMM above
         # that size would round them to the serving dtype first)
