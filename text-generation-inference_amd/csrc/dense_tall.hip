@@ -51,18 +51,9 @@ template <typename T> __device__ __forceinline__ float act2_of(const DTallArgs& 
     return to_f32(from_f32<T>(sl)) * up;
 }
 
-constexpr int GROUP_ROWS = 8;  // 4 against 8 row blocks: 4096 x 22016 at 4096 rows 634 / 627 us, 6144 x 6400 at 300 45 / 43
-// Block bid of a launch of n -> its tile: XCD x (blocks x, x + 8, ...) takes a run of neighbouring tiles
-__device__ __forceinline__ int xcd_run(int bid, int n) {
-    const int x = bid & 7, q = n >> 3, rem = n & 7;
-    return x * q + min(x, rem) + (bid >> 3);
-}
-// Tile t of rows x cols blocks: groups of GROUP_ROWS row blocks, rows fastest
-__device__ __forceinline__ void tile_at(int t, int rows, int cols, int& row, int& col) {
-    const int per = GROUP_ROWS * cols, g = t / per, in = t - g * per, h = min(GROUP_ROWS, rows - g * GROUP_ROWS);
-    row = g * GROUP_ROWS + in % h;
-    col = in / h;
-}
+// (groups of 4 against 8 row blocks: 4096 x 22016 at 4096 rows 634 / 627 us, 6144 x 6400 at 300 45 / 43)
+using tall::tile_at;
+using tall::xcd_run;
 
 template <typename T, int BMR, int ACT, int TW>
 __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {

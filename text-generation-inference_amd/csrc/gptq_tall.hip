@@ -45,22 +45,12 @@ struct TallArgs {
 
 constexpr int TALL_RING = tall::RING;  // k64-steps of weights in flight per wave, and buffers of x
 
-// Tiles are walked in groups of 8 row blocks, each XCD its own run of them, so that its L2 serves a tile of weights to 8 blocks.  us, columns
+// The order of tiles (tall_ring.h).  us, columns
 // fastest over the whole chip / this: 4096 x 22016 with SiLU at 300, 765, 6000 rows 74.9 / 69.4, 148.6 / 146.2, 989 / 961; 8192 x 57344 with SiLU at
 // 300, 3000 rows 345 / 324, 2611 / 2456; 11008 x 4096 at 140, 300, 765 rows 33.3 / 30.3, 41.3 / 42.6, 79.4 / 79.1; 4096 x 4096 at 433 25.3 / 25.9.
 // (Groups of 4: alike, 69, 145, 955; 327, 2432; 30.2, 44.4, 78.0; 26.8.)
-constexpr int GROUP_ROWS = 8;
-// Block bid of a launch of n -> its tile: XCD x (blocks x, x + 8, ...) takes a run of neighbouring tiles
-__device__ __forceinline__ int xcd_run(int bid, int n) {
-    const int x = bid & 7, q = n >> 3, rem = n & 7;
-    return x * q + min(x, rem) + (bid >> 3);
-}
-// Tile t of rows x cols blocks: groups of GROUP_ROWS row blocks, rows fastest
-__device__ __forceinline__ void tile_at(int t, int rows, int cols, int& row, int& col) {
-    const int per = GROUP_ROWS * cols, g = t / per, in = t - g * per, h = min(GROUP_ROWS, rows - g * GROUP_ROWS);
-    row = g * GROUP_ROWS + in % h;
-    col = in / h;
-}
+using tall::tile_at;
+using tall::xcd_run;
 
 template <int BMR, int ACT, int TW>
 __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {

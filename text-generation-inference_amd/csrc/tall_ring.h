@@ -1,9 +1,24 @@
-// The k loop of the GEMMs of prefills (gptq_tall.hip, dense_tall.hip): a ring of four LDS buffers of x, filled by direct loads three steps ahead.
+// What the GEMMs of prefills (gptq_tall.hip, dense_tall.hip) share: the order of their tiles, and their k loop over a ring of four LDS buffers of x,
+// filled by direct loads three steps ahead.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <type_traits>
 
 namespace tall {
+
+// Tiles are walked in groups of GROUP_ROWS row blocks, each XCD its own run of them, so that its L2 serves a tile of weights to 8 blocks.
+constexpr int GROUP_ROWS = 8;
+// Block bid of a launch of n -> its tile: XCD x (blocks x, x + 8, ...) takes a run of neighbouring tiles
+__device__ __forceinline__ int xcd_run(int bid, int n) {
+    const int x = bid & 7, q = n >> 3, rem = n & 7;
+    return x * q + min(x, rem) + (bid >> 3);
+}
+// Tile t of rows x cols blocks: groups of GROUP_ROWS row blocks, rows fastest
+__device__ __forceinline__ void tile_at(int t, int rows, int cols, int& row, int& col) {
+    const int per = GROUP_ROWS * cols, g = t / per, in = t - g * per, h = min(GROUP_ROWS, rows - g * GROUP_ROWS);
+    row = g * GROUP_ROWS + in % h;
+    col = in / h;
+}
 
 constexpr int RING = 4;
 
