@@ -45,10 +45,9 @@ struct TallArgs {
 
 constexpr int TALL_RING = tall::RING;  // k64-steps of weights in flight per wave, and buffers of x
 
-// The order of tiles (tall_ring.h).  us, columns
-// fastest over the whole chip / this: 4096 x 22016 with SiLU at 300, 765, 6000 rows 74.9 / 69.4, 148.6 / 146.2, 989 / 961; 8192 x 57344 with SiLU at
-// 300, 3000 rows 345 / 324, 2611 / 2456; 11008 x 4096 at 140, 300, 765 rows 33.3 / 30.3, 41.3 / 42.6, 79.4 / 79.1; 4096 x 4096 at 433 25.3 / 25.9.
-// (Groups of 4: alike, 69, 145, 955; 327, 2432; 30.2, 44.4, 78.0; 26.8.)
+// The order of tiles (tall_ring.h).  us, columns fastest over the whole chip / this: 4096 x 22016 with SiLU at 300, 765, 6000 rows 74.9 / 69.4, 148.6 /
+// 146.2, 989 / 961; 8192 x 57344 with SiLU at 300, 3000 rows 345 / 324, 2611 / 2456; 11008 x 4096 at 140, 300, 765 rows 33.3 / 30.3, 41.3 / 42.6,
+// 79.4 / 79.1; 4096 x 4096 at 433 25.3 / 25.9.  (Groups of 4: alike, 69, 145, 955; 327, 2432; 30.2, 44.4, 78.0; 26.8.)
 using tall::tile_at;
 using tall::xcd_run;
 

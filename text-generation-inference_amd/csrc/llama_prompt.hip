@@ -1,6 +1,6 @@
 // The layers of a dense Llama model on the rows of prompts, launched from here: the launches that the model's own forward makes one by one,
-// with the same arguments and the same results, without its way back to Python between them.  A layer of a short prompt is six launches of 4 to
-// 16 us, each of which took 9 us of host time to prepare; here it is 2 - 3 us.  47 tokens through 22 layers of 2048: 1820 -> 1540 us.
+// with the same arguments and the same results, without its way back to Python between them.  A layer of a short prompt is seven launches of 4 to
+// 17 us, each of which took 9 us of host time to prepare; here it is 2 - 3 us.  47 tokens through 22 layers of 2048: 1820 -> 1540 us.
 #include "common.h"
 
 #define TRY(call)                          \

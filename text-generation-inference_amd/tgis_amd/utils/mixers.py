@@ -99,7 +99,9 @@ class NormedQKAttention:
         # blend: v <- (1 - lambda) v + lambda v_other, lambda a learned scalar kept on the device
         self.v_lambda = _f32(weights.get_tensor(f"{prefix}.vmix")).reshape(1) if blend else None
         self.defer = can_defer(self.o)
-        # short steps: the launch that norms q and k adds the projection's split-K sums
+        # short steps: the launch that norms q and k adds the projection's split-K sums (us, added by a launch of their own / there, 1, 24, 64, 128, 256
+        # rows: 2048 x 2560 9.6 / 7.3, 10.7 / 7.9, 13.0 / 10.2, 14.8 / 12.4, 18.2 / 15.7; 4096 x 6144 16.9 / 16.0, 18.3 / 17.5, 22.1 / 20.6, 24.7 / 24.1, 33.6 / 31.7;
+        # 8192 x 10240 31 / 31.6, 36.3 / 36.5, 41.6 / 40.1, 46.5 / 45.4, 67.6 / 65.0; 512 x 768 5.8 / 5.9, 7.4 / 6.5, 9.6 / 7.9, 9.9 / 8.4, 10.2 / 8.8)
         self.defer_qkv = self.qkv.streams and dim % 2 == 0 and dim <= 256 and self.qkv.out_features % 2 == 0
 
     def values_of(self, qkv: torch.Tensor) -> torch.Tensor:
