@@ -92,7 +92,7 @@ int tgis_gptq_prepare(const int32_t* qweight, const int32_t* qzeros, const void*
 /* Workspace for split-K partial sums + arrival counters of one gemm call. The counter region
  * (first 4096 bytes) must be zero before the first call; the kernel leaves it zero. */
 /* Largest M for which tgis_gptq_gemm_f16 is a fused dequantise + MFMA kernel worth calling (above it the caller
- * dequantises once with tgis_gptq_dequant_f16 and uses a library GEMM, exllamav2.py:87 "M > 50"): M <= 64 streams the
+ * dequantises once with tgis_gptq_dequant_t_f16 and uses a library GEMM, exllamav2.py:87 "M > 50"): M <= 64 streams the
  * weights once per pass, 64 < M <= 256 in 64-row passes, and — for K % 64 == 0, group size 64 * 2^n, no act-order, act != 1 —
  * a tall kernel (one dequantisation per 64 - 128 rows, 0.5 - 1.0 PFLOP/s at 500 - 1000 rows of a 7B matrix, 1.0 - 1.1 from 2000, no scratch copy of W) takes over up to
  * 8192 rows: from 257, and from 129 (act 2: 65) where it is done before the passes.  tgis_gptq_gemm_whole_sums: 1 where it does.
@@ -168,6 +168,10 @@ int tgis_dense_gemm_rope(const void* x, int64_t ldx, const void* prepared, const
  * uses for M > 50 before a library GEMM (exllamav2.py:65-66,87). */
 int tgis_gptq_dequant_f16(const void* prepared, void* w_out, int64_t K, int64_t N, int64_t groups,
                           int flags, void* stream);
+/* The same values as [N,K] (row-major, 16-byte aligned), the layout of a torch-Linear weight: library products of many rows take
+ * 10 - 15 % less time with it. */
+int tgis_gptq_dequant_t_f16(const void* prepared, void* w_out, int64_t K, int64_t N, int64_t groups,
+                            int flags, void* stream);
 
 /* Dense products of prefills on the image of tgis_dense_prepare: out = act(x W^T + bias) in the model dtype or, act 0, in fp32; K a multiple of 64, x rows 16-byte aligned.  act 0 none, 4 / 5 GELU (erf / tanh) of the rounded sum, 2 SiLU(gate) * up of the gate|up image ([M][N / 2]; glu_limit > 0: the
  * clamped unit of tgis_dense_gemm_clamped_glu instead).

@@ -102,11 +102,11 @@ def test_deferred_sums_at_any_row_count(gpu_device):
 
 # K: half a k64-step, whole ones, a ragged last; N: one tile, a block of eight and ragged ones; groups shorter than a step
 # (and a matrix on each side of the 768 blocks of eight tiles)
-@pytest.mark.parametrize("K,N,groupsize", [(32, 32, 32), (96, 288, 32), (256, 256, 128), (320, 544, 64), (160, 1024, 160), (2016, 6112, 32),
+@pytest.mark.parametrize("K,N,groupsize", [(32, 32, 32), (96, 288, 32), (256, 256, 128), (320, 544, 64), (160, 1024, 160), (512, 64, 128), (544, 96, 32), (2016, 6112, 32),
                                            (2048, 5888, 128)])
 @pytest.mark.parametrize("image", ["plain", "gate_up", "rope"])
 def test_dequant_bits(gpu_device, K, N, groupsize, image):
-    """The image back to [K, N]: the bits of the reference formula, from each column order, into aligned and unaligned memory."""
+    """The image back to [K, N]: the bits of the reference formula, from each column order, into aligned and unaligned memory; and to [N, K]."""
     from tgis_amd import native
 
     qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, groupsize, seed=K + N)
@@ -114,6 +114,8 @@ def test_dequant_bits(gpu_device, K, N, groupsize, image):
     w = native.GptqWeight(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), 4, groupsize, **kind)
     want = ops_ref.gptq_dequant(qw, qz, sc, gi, groupsize).half()
     assert torch.equal(native.gptq_dequant(w).cpu(), want)
+    buf = torch.full((K * N + 16,), 7.0, dtype=torch.float16, device=gpu_device)
+    assert torch.equal(native.gptq_dequant_t(w, buf[8:-8].view(N, K)).t().cpu(), want) and (buf[:8] == 7.0).all() and (buf[-8:] == 7.0).all()
     buf = torch.full((K * N + 2,), 7.0, dtype=torch.float16, device=gpu_device)
     lib = native.load_library()
     assert lib.tgis_gptq_dequant_f16(w.image.data_ptr(), buf.data_ptr() + 2, K, N, w.groups, w.flags, torch.cuda.current_stream().cuda_stream) == 0

@@ -227,6 +227,39 @@ __global__ __launch_bounds__(256) void gptq_dequant_kernel(const uint8_t* __rest
     }
 }
 
+// The same as [N][K], a column's k together: the operand that the library's products of large M are at their best with (TN).  f16, us, the product alone with
+// [K][N] / [N][K]: 16128 rows of 4096 x 12288 1272 / 1105, 4096 x 4096 423 / 363, 4096 x 22016 2333 / 2053, 11008 x 4096 1108 / 969; 16 prompts of 1008
+// tokens through 32 int4 layers of 4096, 11008 193.6 / 172.3 ms.  (Of the sizes that go to the library one is the other way round: 13824 x 5120 at 6000 rows
+// 945 / 982 with the expansion.)  A workgroup takes 512 k of a tile: 8 KiB of the image, 32 k of a column per lane, and through LDS, so that a column leaves
+// in a KiB without a gap.  Bound by the bytes: 4096 x 12288 30.4 / 25.4, 4096 x 22016 47.2 / 37.8, 8192 x 57344 238 / 203, 4096 x 4096 11.0 / 9.1.
+constexpr int DQT_K = 512;
+__global__ __launch_bounds__(256) void gptq_dequant_t_kernel(const uint8_t* __restrict__ prep, int64_t offB, f16* __restrict__ wout, int K, int N,
+                                                             int G, int gs, int KS, int flags) {
+    constexpr int ROW = DQT_K + 8;
+    __shared__ __attribute__((aligned(16))) f16 tile[32 * ROW];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int parts = (K + DQT_K - 1) / DQT_K, nt = blockIdx.x / parts, k0 = blockIdx.x % parts * DQT_K;
+    const int steps = min(DQT_K / 64, (K - k0 + 63) >> 6);  // (of a last half step the first 32 rows are stored)
+    const uint32_t* sz = reinterpret_cast<const uint32_t*>(prep + offB) + (int64_t)nt * G * 32 + (lane & 31);
+    for (int s = w; s < steps; s += 4) {
+        const u32x4 q = *reinterpret_cast<const u32x4*>(prep + (((int64_t)nt * KS + (k0 >> 6) + s) * 64 + lane) * 16);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int kk = s * 64 + (lane >> 5) * 32 + i * 8;
+            const f16x2 szh = __builtin_bit_cast(f16x2, sz[min((k0 + kk) / gs, G - 1) * 32]);
+            const f16 zd = (f16)960.f - szh[1];
+            st16(tile + (lane & 31) * ROW + kk,
+                 gptq::dequant8(q[i], f16x2{szh[1], szh[1]}, f16x2{zd, zd}, f16x2{szh[0], szh[0]}, 0x64006400u, 0x000F000Fu, 0x00F000F0u));
+        }
+    }
+    __syncthreads();
+    const int pieces = min(DQT_K, K - k0) >> 3;
+    for (int p = tid; p < 32 * (DQT_K / 8); p += 256) {
+        const int c = p / (DQT_K / 8), j = p % (DQT_K / 8);
+        if (j < pieces) st16(wout + col_src(nt, c, N, flags) * K + k0 + j * 8, ld16<f16x8>(tile + c * ROW + j * 8));
+    }
+}
+
 }  // namespace
 
 extern "C" int64_t tgis_gptq_prepared_bytes(int64_t K, int64_t N, int64_t groups) {
@@ -700,6 +733,18 @@ extern "C" int tgis_gptq_dequant_f16(const void* prepared, void* w_out, int64_t 
                        (const uint8_t*)prepared, p.offB, (f16*)w_out, (int)K, (int)N, (int)groups, (int)(K / groups), (int)p.NT, (int)p.KS, flags, vec)
     if (blocks < 768) TGIS_DEQUANT(2); else TGIS_DEQUANT(8);
 #undef TGIS_DEQUANT
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+extern "C" int tgis_gptq_dequant_t_f16(const void* prepared, void* w_out, int64_t K, int64_t N, int64_t groups, int flags, void* stream) {
+    TGIS_CHECK_ARG(prepared && w_out && K > 0 && N > 0 && K % 32 == 0 && N % 32 == 0 && groups > 0 && K % groups == 0 && K / groups % 8 == 0,
+                   "tgis_gptq_dequant_t_f16: bad arguments");
+    TGIS_CHECK_ARG((uintptr_t)w_out % 16 == 0, "tgis_gptq_dequant_t_f16: the matrix must be 16-byte aligned");
+    const PrepLayout p = prep_layout(K, N, groups);
+    TGIS_CHECK_ARG(p.NT * cdiv64(K, DQT_K) <= 2147483647LL, "tgis_gptq_dequant_t_f16: matrix too large");
+    hipLaunchKernelGGL(gptq_dequant_t_kernel, dim3((unsigned)(p.NT * cdiv64(K, DQT_K))), dim3(256), 0, (hipStream_t)stream,
+                       (const uint8_t*)prepared, p.offB, (f16*)w_out, (int)K, (int)N, (int)groups, (int)(K / groups), (int)p.KS, flags);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }

@@ -414,7 +414,10 @@ TallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, 
 
 // Rows from which it may replace the 64-row streaming passes, and up to which it replaces dequantise + library GEMM: (library with its
 // dequantisation / tall, us, the four GEMMs of a 7B layer) 4096 rows 1547 / 1400, 6000 rows 2288 / 2121, 8192 rows 2829 / 2851; at 16128 rows
-// hipBLASLt's 256 x 256 tiles, free of dequantisation, run at 1.35 PFLOP/s against 1.12 - 1.25.
+// hipBLASLt's 256 x 256 tiles, free of dequantisation, run at 1.35 PFLOP/s against 1.12 - 1.25.  (These and the figures below are with the expansion to [K][N]; with
+// tgis_gptq_dequant_t_f16's [N][K] the library's side takes 10 - 15 % less: 4096 x 12288 at 3500, 4096, 7168, 8190 rows 286 / 330, 309 / 355, 553 / 624, 588 / 695, but
+// 581 / 513 at 6000; 11008 x 4096 at 5225, 7168 664 / 428, 557 / 563; 8192 x 10240 at 4096 716 / 573; 28672 x 8192 at 5225, 7168 2487 / 2009, 3217 / 2823.  Which of its
+// kernels the library takes there follows no rule of sizes, so the line stays where its tiles fill their rounds.)
 int64_t gptq::tall_min_m(int act) {
     static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 0;
     return v ? v : act == 2 ? 65 : 129;

@@ -51,6 +51,7 @@ SIGNATURES = {
     "tgis_gptq_gemm_f16_partial": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64,
                                             ctypes.POINTER(_c_int), ctypes.POINTER(_c_i64), _vp]),
     "tgis_gptq_dequant_f16": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_gptq_dequant_t_f16": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_rope": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64,
                                       _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_gptq_rope_ok": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_i64]),
@@ -615,6 +616,16 @@ def gptq_dequant(w: GptqWeight) -> torch.Tensor:
     out = torch.empty((w.K, w.N), dtype=torch.float16, device=w.image.device)
     _check(load_library().tgis_gptq_dequant_f16(_ptr(w.image), _ptr(out), w.K, w.N, w.groups, w.flags, _stream()),
            "tgis_gptq_dequant_f16")
+    return out
+
+
+def gptq_dequant_t(w: GptqWeight, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The same values as [N,K]."""
+    if out is None:
+        out = torch.empty((w.N, w.K), dtype=torch.float16, device=w.image.device)
+    assert out.shape == (w.N, w.K) and out.dtype == torch.float16 and out.is_contiguous()
+    _check(load_library().tgis_gptq_dequant_t_f16(_ptr(w.image), _ptr(out), w.K, w.N, w.groups, w.flags, _stream()),
+           "tgis_gptq_dequant_t_f16")
     return out
 
 

@@ -261,7 +261,7 @@ class Ex4bitLinearV2:
         buf = Ex4bitLinearV2._temp_dq.get(key)
         if buf is None:
             Ex4bitLinearV2._temp_dq.clear()  # one scratch at a time, like exllama's temp_dq
-            buf = Ex4bitLinearV2._temp_dq[key] = torch.empty((self.height, self.width), dtype=torch.float16,
+            buf = Ex4bitLinearV2._temp_dq[key] = torch.empty((self.width, self.height), dtype=torch.float16,
                                                              device=self.device)
         return buf
 
@@ -309,11 +309,7 @@ class Ex4bitLinearV2:
 
     def _large_m(self, x: torch.Tensor) -> torch.Tensor:
         """prefill-sized M: dequantise once into scratch, then a library GEMM (exllamav2.py:87 "M > 50"); x in image order."""
-        w = self._dequant_scratch()
-        native._check(native.load_library().tgis_gptq_dequant_f16(
-            self.ordered.image.data_ptr(), w.data_ptr(), self.height, self.width, self.ordered.groups,
-            self.ordered.flags, native._stream()), "tgis_gptq_dequant_f16")
-        out = torch.matmul(x, w)
+        out = torch.matmul(x, native.gptq_dequant_t(self.ordered, self._dequant_scratch()).t())
         if self.bias is not None:
             out.add_(self.bias)
         return out
