@@ -809,6 +809,10 @@ int tgis_dense_gemm_whole_operand(int64_t M, int64_t K, int64_t N, int act);
  * M <= 64, K a multiple of 64, N_group of 32, x_group of 8. */
 int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo, int64_t out_group,
                            int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups, int dtype, void* stream);
+/* The same for the rows of a prefill: any M; x rows 16-byte aligned, less than 2^22 elements apart.  ..._pays: 1 where it is the faster way (a size query). */
+int tgis_dense_tall_groups_pays(int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups);
+int tgis_dense_tall_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo, int64_t out_group,
+                           int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups, int dtype, void* stream);
 /* Matrix memory with exponential gates per (sequence, head), tokens in order (the running maximum m starts at 0):
  *   i = cap tanh((z_i + i_bias) / cap);  f = ln sigmoid(cap tanh((z_f + f_bias) / cap));  m' = max(f + m, i);
  *   S <- e^(f + m - m') S + e^(i - m') k v^T;  n likewise with k;  o = c S^T q / (max(|c n . q|, e^-m') + read_eps), c = q_scale;

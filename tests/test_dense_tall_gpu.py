@@ -176,3 +176,40 @@ def test_rows_that_the_user_divides(monkeypatch):
         lin.gate_up = True
         _check(lin(x.cuda()), _expect(z, acc, torch.float16, 2))
     assert streamed == [65] * 3 + [128] * 3
+
+
+# one launch of several products: one, several with a last one that is whole / part of a tile / a narrow one ahead of the others (from 2049 rows on)
+@pytest.mark.parametrize("M,K,n_group,N,G,plans", [
+    (65, 64, 32, 20, 1, "234"), (129, 448, 96, 288, 3, "234"), (97, 576, 64, 150, 3, "2"), (300, 2048, 512, 2048 + 64, 5, "234"), (257, 128, 160, 470, 3, "4"),
+    (2049, 192, 256, 256 + 128, 2, "234"), (2050, 64, 288, 4 * 288 + 33, 5, "234"), (2049, 128, 256, 256 + 129, 2, "3"), (2111, 320, 32, 64, 2, "4"),
+])
+@pytest.mark.parametrize("width", [1, 2])
+def test_groups(M, K, n_group, N, G, plans, width, monkeypatch):
+    from tgis_amd import native
+
+    dtype = torch.bfloat16 if M & 1 else torch.float16
+    g = torch.Generator().manual_seed(K + N + M)
+    x, wt = torch.randn(G, M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype)
+    image, xd = native.DenseWeight(wt.cuda()), x.cuda()
+    want = [_expect(x[i].double() @ wt[i * n_group:(i + 1) * n_group].double().t(),
+                    K * 2.0 ** -24 * (x[i].double().abs() @ wt[i * n_group:(i + 1) * n_group].double().abs().t()), dtype, 0) for i in range(G)]
+    for rows in [None, *plans]:
+        if rows:
+            monkeypatch.setenv("TGIS_DTALL_PLAN", f"{rows},{width},1")
+        out = torch.full((G, M, n_group + (8 if M & 2 else 1)), 7.0, dtype=dtype, device="cuda")
+        native.dense_tall_groups(xd, image, n_group, out)
+        for i in range(G):
+            cols = min(n_group, N - i * n_group)
+            _check(out[i, :, :cols], want[i])
+            assert bool((out[i, :, cols:] == 7.0).all())
+
+
+def test_groups_rule():
+    from tgis_amd import native
+
+    pays = lambda *a: native.load_library().tgis_dense_tall_groups_pays(*a)
+    assert pays(65, 2048, 2048, 4 * 2048 + 64, 5) and pays(4096, 2048, 2048, 4 * 2048 + 64, 5) and not pays(4097, 2048, 2048, 4 * 2048 + 64, 5)
+    assert not pays(64, 2048, 2048, 4 * 2048 + 64, 5) and not pays(300, 96, 2048, 4 * 2048 + 64, 5) and not pays(300, 2048, 2048, 4 * 2048, 5)
+    wide = native.DenseWeight(torch.zeros(96, 72, dtype=torch.float16, device="cuda"))
+    with pytest.raises(RuntimeError, match="bad arguments"):
+        native.dense_tall_groups(torch.zeros(3, 70, 72, dtype=torch.float16, device="cuda"), wide, 32, torch.zeros(3, 70, 32, dtype=torch.float16, device="cuda"))

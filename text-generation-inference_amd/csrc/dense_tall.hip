@@ -55,8 +55,7 @@ template <typename T> __device__ __forceinline__ float act2_of(const DTallArgs& 
 using tall::tile_at;
 using tall::xcd_run;
 
-template <typename T, int BMR, int ACT, int TW>
-__global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
+template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void dense_tall_tile(const DTallArgs& a, int tile, int split) {
     using V8 = typename VecT<T>::x8;
     constexpr int BM = 32 * BMR;
     constexpr int WR = TW == 2 ? 2 : 4;  // k64-steps of weights in flight per wave
@@ -64,10 +63,9 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int row_block, col_block;
-    tile_at(a.tile0 + xcd_run(blockIdx.x, gridDim.x), (a.M + BM - 1) / BM, a.col_blocks, row_block, col_block);
+    tile_at(tile, (a.M + BM - 1) / BM, a.col_blocks, row_block, col_block);
     const int m0 = row_block * BM;
     const int mrows = min(BM, a.M - m0);
-    const int split = blockIdx.y;
     const int nt_raw0 = (col_block * 4 + w) * TW;
     const int ksteps = a.K >> 6;                                         // K % 64 == 0 (host)
     const int ks0 = split * a.per, n = min(ksteps, ks0 + a.per) - ks0;   // n >= 1 (host)
@@ -151,7 +149,7 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
     auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
     constexpr int BN = 128 * TW;
     if (a.part == 1) {
-        float* dst = a.scratch + ((int64_t)xcd_run(blockIdx.x, gridDim.x) * a.S + split) * (BM * BN) + w * (32 * TW) + c;
+        float* dst = a.scratch + ((int64_t)(tile - a.tile0) * a.S + split) * (BM * BN) + w * (32 * TW) + c;
 #pragma unroll
         for (int t = 0; t < TW; ++t)
 #pragma unroll
@@ -239,6 +237,38 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
             for (int e = 0; e < 8; ++e)
                 if (n0 + col + e < n_out) o[e] = v[e];
         }
+    }
+}
+
+template <typename T, int BMR, int ACT, int TW>
+__global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
+    dense_tall_tile<T, BMR, ACT, TW>(a, a.tile0 + xcd_run(blockIdx.x, gridDim.x), blockIdx.y);
+}
+
+// Several products in one launch, each of its own operand, on neighbouring tiles of one image: the tiles of the first, then those of the second, ...
+// NARROW: a last product of up to 128 columns goes first, in tiles of 64 x 128.  (Four 2048 x 2048 and one 2048 x 64, bf16, us, whole tiles behind the others, where
+// they are a round of their own / this: 4096 rows 147 / 140, 3000 118 / 110; below, where the rounds are short, 2045 rows 76.5 / 78.7, 300 22.7 / 25.8.)
+struct TallGroups {
+    int n, tiles, narrow;        // products; 32-column tiles of the image to each but the last, which has the rest; blocks of a narrow last product
+    int64_t x_group, out_group;  // elements between their operands, their outputs
+};
+template <typename T, int BMR, int TW, bool NARROW>
+__global__ __launch_bounds__(256, 2) void dense_tall_groups_kernel(DTallArgs a, TallGroups g) {
+    const bool narrow = NARROW && (int)blockIdx.x < g.narrow;
+    const int each = (a.M + 32 * BMR - 1) / (32 * BMR) * a.col_blocks;
+    const int tile = narrow ? blockIdx.x : xcd_run(blockIdx.x - g.narrow, gridDim.x - g.narrow);
+    const int i = narrow ? g.n - 1 : min(tile / each, g.n - 1), first = i * g.tiles;
+    a.x = reinterpret_cast<const T*>(a.x) + i * g.x_group;
+    a.out = reinterpret_cast<T*>(a.out) + i * g.out_group;
+    a.prep += (int64_t)first * (a.K >> 6) * 4096;
+    a.N = i + 1 < g.n ? g.tiles * 32 : a.N - first * 32;
+    a.NT = (a.N + 31) >> 5;
+    if (NARROW && narrow) {
+        a.col_blocks = 1;
+        dense_tall_tile<T, 2, 0, 1>(a, tile, 0);
+    } else {
+        a.col_blocks = (a.NT + 4 * TW - 1) / (4 * TW);
+        dense_tall_tile<T, BMR, 0, TW>(a, tile - i * each, 0);
     }
 }
 
@@ -561,6 +591,91 @@ extern "C" int tgis_dense_tall(const void* x, int64_t ldx, const void* prepared,
     const hipStream_t st = (hipStream_t)stream;
     TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
     return dtype == TGIS_F16 ? run_tall<f16>(p, a, act == 2 ? 2 : 0, st) : run_tall<bf16>(p, a, act == 2 ? 2 : 0, st);
+}
+
+// Several products in one launch (TallGroups), unsplit: the tile of the least walk.
+struct GroupsPlan {
+    int BMR, TW, col_blocks, tiles, narrow;
+};
+static GroupsPlan plan_groups(int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups) {
+    const int64_t last = N - (groups - 1) * N_group;
+    const bool narrow = groups > 1 && last <= 128 && M > 2048;
+    GroupsPlan best{};
+    double best_us = 1e30;
+    TallPlan forced;
+    const bool fixed = plan_from_env(M, K, N, false, forced);
+    for (int BMR = 2; BMR <= 4; ++BMR)
+        for (int TW = narrow ? 2 : 1; TW <= 2; ++TW) {
+            if (fixed && (BMR != forced.BMR || TW != std::max(forced.TW, narrow ? 2 : 1))) continue;
+            const int64_t cb = cdiv64(N_group, 128 * TW);
+            const int64_t tiles = cdiv64(M, 32 * BMR) * (cb * (groups - 1) + (narrow ? 0 : cdiv64(last, 128 * TW)));
+            const double us = launch_us(walk_us(tiles, K / 64, TALL_COST[BMR - 2][TW - 1]), K, N);
+            if (us < best_us) {
+                best_us = us;
+                best = {BMR, TW, (int)cb, (int)tiles, narrow ? (int)cdiv64(M, 64) : 0};
+            }
+        }
+    return best;
+}
+
+template <typename T, int BMR, int TW, bool NARROW> static int launch_groups(const GroupsPlan& p, const DTallArgs& a, const TallGroups& g, hipStream_t st) {
+    constexpr size_t ring = (size_t)X_RING * (32 * BMR) * 128, rows = (size_t)(32 * BMR) * (128 * TW + 8) * 2;
+    constexpr size_t lds = ring > rows ? ring : rows;
+    static const hipError_t attr = hipFuncSetAttribute((const void*)dense_tall_groups_kernel<T, BMR, TW, NARROW>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    TGIS_CHECK_HIP(attr);
+    hipLaunchKernelGGL((dense_tall_groups_kernel<T, BMR, TW, NARROW>), dim3((unsigned)(p.narrow + p.tiles)), dim3(256), lds, st, a, g);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+template <typename T> static int launch_groups_shape(const GroupsPlan& p, const DTallArgs& a, const TallGroups& g, hipStream_t st) {
+    switch (p.BMR * 10 + p.TW + (p.narrow ? 100 : 0)) {
+        case 21: return launch_groups<T, 2, 1, false>(p, a, g, st);
+        case 22: return launch_groups<T, 2, 2, false>(p, a, g, st);
+        case 31: return launch_groups<T, 3, 1, false>(p, a, g, st);
+        case 32: return launch_groups<T, 3, 2, false>(p, a, g, st);
+        case 41: return launch_groups<T, 4, 1, false>(p, a, g, st);
+        case 42: return launch_groups<T, 4, 2, false>(p, a, g, st);
+        case 122: return launch_groups<T, 2, 2, true>(p, a, g, st);
+        case 132: return launch_groups<T, 3, 2, true>(p, a, g, st);
+        default: return launch_groups<T, 4, 2, true>(p, a, g, st);
+    }
+}
+
+// Is one launch the faster way than the products one by one?  Up to where 256 x 256 tiles of one of them fill half the chip, which is where the library's begin to
+// be ahead by more than four launches' ends.  Four products and a narrow one, bf16, weights cold, us, one by one / together:
+//   2048 x 2048, 64: 65 rows 54 / 17, 300 68 / 23, 1024 77 / 47, 1393 92 / 57, 2045 109 / 77, 3000 128 / 110, 4096 152 / 140 (128 tiles; 6000 194 / 198, 8190 224 / 271)
+//   4096 x 4096, 128: 65 72 / 39, 512 132 / 98, 1024 182 / 143, 2045 265 / 261 (128 tiles; 3000 358 / 380, 4096 414 / 508)
+//   2560 x 2560, 160: 300 72 / 30, 1393 129 / 82, 3000 184 / 162 (120 tiles; 4096 235 / 214, 6000 267 / 308);  1024 x 1024, 64: 8190 105 / 85 (128 tiles)
+// Prompts through 8 layers of 2048 of which every other takes such a launch: 1 x 70 tokens 1144 / 937 us, 2 x 150 1163 / 978, 4 x 333 ragged 1862 / 1714, 4 x 1024 4402 /
+// 4370; 24 prompts and eight tokens each 6978 / 6845.
+extern "C" int tgis_dense_tall_groups_pays(int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups) {
+    if (M < TGIS_DENSE_TALL_MIN_M || K < 64 || K % 64 != 0 || N_group <= 0 || N_group % 32 != 0 || groups < 2 || N <= (groups - 1) * N_group || N > groups * N_group)
+        return 0;
+    return cdiv64(M, 256) * cdiv64(N_group, 256) <= CUS / 2 ? 1 : 0;
+}
+
+extern "C" int tgis_dense_tall_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo, int64_t out_group,
+                                      int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups, int dtype, void* stream) {
+    TGIS_CHECK_ARG(x && prepared && out && M >= 0 && K >= 64 && K % 64 == 0, "tgis_dense_tall_groups: bad arguments");
+    TGIS_CHECK_ARG(dtype == TGIS_F16 || dtype == TGIS_BF16, "tgis_dense_tall_groups: bad dtype");
+    TGIS_CHECK_ARG(rows_ok(x, ldx, K) && x_group % 8 == 0, "tgis_dense_tall_groups: x rows must be 16-byte aligned and less than 2^22 elements apart");
+    TGIS_CHECK_ARG(N_group > 0 && N_group % 32 == 0 && groups >= 1 && N > (groups - 1) * N_group && N <= groups * N_group && ldo >= std::min(N, N_group),
+                   "tgis_dense_tall_groups: %ld columns do not make %ld groups of up to %ld", (long)N, (long)groups, (long)N_group);
+    TGIS_CHECK_ARG(cdiv64(M, 64) * (cdiv64(N, 128) + groups) <= 2147483647LL, "tgis_dense_tall_groups: too many tiles");
+    if (M == 0) return TGIS_OK;
+    const GroupsPlan p = plan_groups(M, K, N_group, N, groups);
+    DTallArgs a = tall_args(x, ldx, prepared, M, K, N, nullptr);
+    a.out = out;
+    a.ldo = ldo;
+    a.vec = ldo % 8 == 0 && (uintptr_t)out % 16 == 0 && out_group % 8 == 0;
+    a.col_blocks = p.col_blocks;
+    a.per = (int)(K / 64);
+    a.S = 1;
+    const TallGroups g{(int)groups, (int)(N_group / 32), p.narrow, x_group, out_group};
+    const hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
+    return dtype == TGIS_F16 ? launch_groups_shape<f16>(p, a, g, st) : launch_groups_shape<bf16>(p, a, g, st);
 }
 
 // The product as fp32 partial sums for the consumers of tgis_dense_gemm_partial's, in the same layout; up to 256 rows.

@@ -210,6 +210,8 @@ SIGNATURES = {
     "tgis_llama_prompt": (_c_int, [_vp, _c_int, _vp, _vp]),
     "tgis_dense_gemm_whole_operand": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_tall_groups_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
+    "tgis_dense_tall_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
     "tgis_matrix_memory": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _vp, _c_i64, _vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp,
                                     _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_f, _c_f, _c_f, _c_int, _c_int, _vp]),
@@ -678,6 +680,21 @@ def dense_gemm_groups(x: torch.Tensor, w: DenseWeight, n_group: int, out: torch.
     _check(load_library().tgis_dense_gemm_groups(_ptr(x), x.stride(1), x.stride(0), _ptr(w.image), _ptr(out), out.stride(1), out.stride(0), M, K,
                                                  n_group, w.N, G, dtype_code(w.dtype), _stream()), "tgis_dense_gemm_groups")
     return out
+
+
+def dense_tall_groups(x: torch.Tensor, w: DenseWeight, n_group: int, out: torch.Tensor) -> torch.Tensor:
+    """dense_gemm_groups of a prefill's rows."""
+    G, M, K = x.shape
+    assert x.dtype == w.dtype == out.dtype and not w.flags and K == w.K and x.stride(2) == out.stride(2) == 1
+    assert out.shape[:2] == (G, M) and out.shape[2] >= n_group and (G - 1) * n_group < w.N <= G * n_group
+    _check(load_library().tgis_dense_tall_groups(_ptr(x), x.stride(1), x.stride(0), _ptr(w.image), _ptr(out), out.stride(1), out.stride(0), M, K,
+                                                 n_group, w.N, G, dtype_code(w.dtype), _stream()), "tgis_dense_tall_groups")
+    return out
+
+
+def dense_tall_groups_pays(M: int, w: DenseWeight, n_group: int, groups: int) -> bool:
+    """Whether that is the faster way than the products one by one (a size query)."""
+    return bool(load_library().tgis_dense_tall_groups_pays(M, w.K, n_group, w.N, groups))
 
 
 def dense_gemm(x: torch.Tensor, w: DenseWeight, ws: Workspace, bias=None, out_f32: bool = False, act: int = 0,

@@ -55,7 +55,7 @@ from typing import Optional
 import torch
 
 from tgis_amd import native
-from tgis_amd.utils.layers import SKINNY_MAX_M, FastLinear, tall_bytes, workspace
+from tgis_amd.utils.layers import DENSE_TALL, SKINNY_MAX_M, FastLinear, tall_bytes, workspace
 
 # rows up to which the clamped gated unit runs in the epilogue of the weight-streaming GEMM
 CLAMPED_EPILOGUE_MAX_M = SKINNY_MAX_M
@@ -134,7 +134,7 @@ class WkvMixer:
         self.H, self.d, self.eps = heads, dim, float(eps)
         self.mu = torch.stack([_f32(weights.get_tensor(f"{prefix}.mu.{s}")) for s in self.MIXES]).contiguous()
         names, HD, rank = [f"{prefix}.{s}" for s in ("r", "k", "v", "g", "w1")], heads * dim, weights.get_tensor(f"{prefix}.w1").shape[0]
-        # decode-sized steps take the five projections, each of its own mix, in one launch on one stacked image
+        # the five projections, each of its own mix, in one launch on one stacked image: decode-sized steps, and prefills up to where that is slower
         self.stacked = None
         if HD % 32 == 0 and rank <= HD:
             stacked = load_stacked_linear(weights, names)
@@ -160,6 +160,9 @@ class WkvMixer:
         rkvg = torch.empty((5, T, HD), dtype=dtype, device=h32.device)
         if self.stacked is not None and T <= native.GROUPS_MAX_M:
             native.dense_gemm_groups(mixes, self.stacked, HD, rkvg)
+            low = rkvg[4, :, :self.w1.out_features]
+        elif self.stacked is not None and DENSE_TALL and native.dense_tall_groups_pays(T, self.stacked, HD, 5):
+            native.dense_tall_groups(mixes, self.stacked, HD, rkvg)
             low = rkvg[4, :, :self.w1.out_features]
         else:
             for i, lin in enumerate(self.proj):
