@@ -4,13 +4,20 @@
 //
 // A block of 4 waves owns a tile of 64, 96 or 128 rows x 128 or 256 columns; wave w its columns, TW tiles of 32, whose fragments it loads
 // straight from the image into registers, WR k64-steps ahead: no other wave reads them, so they need no LDS.  x, which all four read, goes to
-// LDS with direct loads, a ring of four k64-steps of 128-byte rows whose 16-byte pieces are permuted (piece ^ row mod 8) so that the fragment
-// reads fill all banks.  One barrier a step; while slice i is multiplied the A fragments of slice i + 1 are read.
+// LDS with direct loads, a ring of four k64-steps of 128-byte rows whose 16-byte pieces are permuted (piece ^ row / 2 mod 8) so that the fragment
+// reads of 16 rows fill all banks.  One barrier a step, which is two slices of 32 k in two halves of the rows; while one half is multiplied the A fragments of
+// the next are read.
 //
-// Bound: the matrix cores from about 1000 rows on (1.05 - 1.2 PFLOP/s), before that the weights' way from HBM and the latency of the blocks'
-// serial chains: hence the choice of tiles, and the split of a last round's tiles over k (plan_tall).  Tiles are walked in groups of 8 row
+// Products by the 16x16x32 instruction: under the card's power limit it does more than 32x32x16 (bare loops on random values, PFLOP/s: bf16 2.10 against 1.77, f16
+// 1.95, 1.71).  us, 32x32x16 / now: 2048 x 11264 with SiLU at 1024, 1393, 4096 rows 55.9 / 53.2, 65.2 / 60.8, 173 / 160; 4096 x 22016 with SiLU at 2048 327 / 305;
+// 6144 x 24576 at 400 165 / 156; where a SIMD has one wave, twice the products to issue cost 2 - 6 % of tiles of 256 columns (24576 x 6144 at 128 rows 307 / 321),
+// which no plan takes there.
+//
+// Bound: the matrix cores and their power from about 1000 rows on (1.15 - 1.35 PFLOP/s; with nothing to load 1.55 - 1.9, with the weights in L1 1.3 - 1.6, with no x
+// 1.25 - 1.5), before that the weights' way from HBM and the latency of the blocks' serial chains: hence the choice of tiles, and the split of a last round's tiles
+// over k (plan_tall).  (Tiles of 256 x 256 by eight waves, the weights shared in L1: 2 - 8 % slower.)  Tiles are walked in groups of 8 row
 // blocks, each XCD its own run of them, so that its L2 serves a tile of weights to 8 blocks: with columns fastest over the whole chip 4096 x
-// 22016 at 4096 rows took 844 us, now 627.
+// 22016 at 4096 rows took 844 us, 627 so (and 551 by the other instruction).
 #include <stdio.h>
 #include <stdlib.h>
 #include <algorithm>
@@ -70,20 +77,29 @@ template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void 
     const int ksteps = a.K >> 6;                                         // K % 64 == 0 (host)
     const int ks0 = split * a.per, n = min(ksteps, ks0 + a.per) - ks0;   // n >= 1 (host)
 
-    const char* wtile[TW];
+    const uint8_t* wtile[TW];
 #pragma unroll
-    for (int t = 0; t < TW; ++t) wtile[t] = reinterpret_cast<const char*>(a.prep) + (int64_t)min(nt_raw0 + t, a.NT - 1) * ksteps * 4096;
-    const uint32_t woff = lane * 16;
-    auto w_at = [&](int t, int ks, int i) -> V8 {
-        const char* p = wtile[t] + (int64_t)min(ks, ksteps - 1) * 4096 + i * 1024;
-        PIN_SGPR(p);
-        return *(const GLOBAL_AS V8*)(p + woff);
+    for (int t = 0; t < TW; ++t) wtile[t] = a.prep + (int64_t)min(nt_raw0 + t, a.NT - 1) * ksteps * 4096;
+    // lane (c, q) of B fragment 2 m + h of a tile holds column 16 h + c and eight k of slice m: piece `chunk(m)` of the step's eight, which lies in the image's
+    // fragment chunk % 4, half chunk / 4 (four runs of 256 bytes a load, the lines of a whole KiB)
+    const int c = lane & 15, q = lane >> 4;
+    auto chunk = [&](int m) { return (q >> 1) * 4 + m * 2 + (q & 1); };
+    const uint32_t woff = (q & 1) * 1024 + (q >> 1) * 512 + c * 16;
+    auto w_at = [&](int t, int ks, int f) -> V8 {
+        const int at = min(ks, ksteps - 1) * 4096, in = (f >> 1) * 2048 + (f & 1) * 256;
+        if constexpr (BMR == 4 && TW == 2) {  // (no registers to spare for addresses; the smaller tiles are a little faster without: gptq_tall.hip)
+            return __builtin_bit_cast(V8, tall::buffer_piece<0>(wtile[t], ksteps * 4096, woff + in, at));
+        } else {
+            const uint8_t* p = wtile[t] + at + in;
+            PIN_SGPR(p);
+            return *(const GLOBAL_AS V8*)(p + woff);
+        }
     };
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
     uint32_t rowoff[BMR];
 #pragma unroll
     for (int j = 0; j < BMR; ++j)
-        rowoff[j] = (uint32_t)(min(8 * (4 * j + w) + (lane >> 3), mrows - 1) * (int)a.ldx * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+        rowoff[j] = (uint32_t)(min(8 * (4 * j + w) + (lane >> 3), mrows - 1) * (int)a.ldx * 2 + ((lane & 7) ^ (4 * (w & 1) + (lane >> 4))) * 16);
     const char* xbase = reinterpret_cast<const char*>(a.x) + (int64_t)m0 * a.ldx * 2;
     auto x_load = [&](int step, int buf) {
         const char* xb = xbase + (int64_t)min(ks0 + step, ksteps - 1) * 128;
@@ -92,14 +108,16 @@ template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void 
         for (int j = 0; j < BMR; ++j)
             kib_to_lds(xb, rowoff[j], __builtin_amdgcn_readfirstlane(lds0 + buf * (BM * 128) + (4 * j + w) * 1024));
     };
-    f32x16 acc[TW][BMR];
+    f32x4 acc[TW][2][2 * BMR];  // [tile][its left, right columns][rows 16 i .. + 15]
 #pragma unroll
     for (int t = 0; t < TW; ++t)
 #pragma unroll
-        for (int rb = 0; rb < BMR; ++rb) acc[t][rb] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t apos[4];
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) apos[i] = (uint32_t)((lane & 31) * 128 + ((i + 4 * (lane >> 5)) ^ (lane & 7)) * 16);
+            for (int rf = 0; rf < 2 * BMR; ++rf) acc[t][h][rf] = f32x4{0, 0, 0, 0};
+    uint32_t apos[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) apos[m] = (uint32_t)(c * 128 + (chunk(m) ^ (c >> 1)) * 16);
 
     x_load(0, 0);
     x_load(1, 1);
@@ -116,7 +134,7 @@ template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void 
     V8 av[2][BMR];
     auto read_a = [&](V8 (&dst)[BMR], int buf, int i) {
 #pragma unroll
-        for (int rb = 0; rb < BMR; ++rb) dst[rb] = ld16<V8>(smem + buf * (BM * 128) + rb * 4096 + apos[i]);
+        for (int rb = 0; rb < BMR; ++rb) dst[rb] = ld16<V8>(smem + buf * (BM * 128) + ((i & 1) * BMR + rb) * 2048 + apos[i >> 1]);
     };
     read_a(av[0], 0, 0);
     auto step = [&](int s, auto slot_, auto tail_) {
@@ -132,10 +150,15 @@ template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void 
 #pragma unroll
             for (int rb = 0; rb < BMR; ++rb)
 #pragma unroll
-                for (int t = 0; t < TW; ++t) acc[t][rb] = mfma32(av[i & 1][rb], wq[WS][t][i], acc[t][rb]);
+                for (int f = 0; f < 2 * TW; ++f) {
+                    f32x4& sum = acc[f >> 1][f & 1][(i & 1) * BMR + rb];
+                    sum = mfma16(av[i & 1][rb], wq[WS][f >> 1][(i & 2) + (f & 1)], sum);
+                }
             if constexpr (REFILL) {
+                if (i & 1) {
 #pragma unroll
-                for (int t = 0; t < TW; ++t) wq[WS][t][i] = w_at(t, ks0 + s + WR, i);
+                    for (int f = 0; f < 2 * TW; ++f) wq[WS][f >> 1][(i & 2) + (f & 1)] = w_at(f >> 1, ks0 + s + WR, (i & 2) + (f & 1));
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -145,49 +168,47 @@ template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void 
     tall::ring_steps(n, step);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
 
-    const int c = lane & 31;
-    auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
+    auto row_of = [&](int rf, int r) { return rf * 16 + 4 * q + r; };
     constexpr int BN = 128 * TW;
     if (a.part == 1) {
         float* dst = a.scratch + ((int64_t)(tile - a.tile0) * a.S + split) * (BM * BN) + w * (32 * TW) + c;
 #pragma unroll
-        for (int t = 0; t < TW; ++t)
+        for (int f = 0; f < 2 * TW; ++f)
 #pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
+            for (int rf = 0; rf < 2 * BMR; ++rf)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(rb, r) * BN + t * 32] = acc[t][rb][r];
+                for (int r = 0; r < 4; ++r) dst[(int64_t)row_of(rf, r) * BN + f * 16] = acc[f >> 1][f & 1][rf][r];
         return;
     }
     if (ACT == 0 && a.part == 2) {
         const int ld = a.NT * 32, blocks = (a.M + 31) >> 5;
 #pragma unroll
-        for (int t = 0; t < TW; ++t) {
-            if (nt_raw0 + t >= a.NT) continue;
+        for (int f = 0; f < 2 * TW; ++f) {
+            if (nt_raw0 + (f >> 1) >= a.NT) continue;
 #pragma unroll
-            for (int rb = 0; rb < BMR; ++rb) {
-                const int block = row_block * BMR + rb;
+            for (int rf = 0; rf < 2 * BMR; ++rf) {
+                const int block = row_block * BMR + (rf >> 1);
                 if (block >= blocks) continue;
-                float* dst = a.scratch + ((int64_t)block * a.S + split) * 32 * ld + (nt_raw0 + t) * 32 + c;
+                float* dst = a.scratch + ((int64_t)block * a.S + split) * 32 * ld + nt_raw0 * 32 + f * 16 + c;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(0, r) * ld] = acc[t][rb][r];
+                for (int r = 0; r < 4; ++r) dst[(int64_t)row_of(rf & 1, r) * ld] = acc[f >> 1][f & 1][rf][r];
             }
         }
         return;
     }
     if (ACT == 0 && a.out_f32) {
-        const int m_lane = m0 + 4 * (lane >> 5);
 #pragma unroll
-        for (int t = 0; t < TW; ++t) {
-            const int n = (nt_raw0 + t) * 32 + c;
+        for (int f = 0; f < 2 * TW; ++f) {
+            const int n = nt_raw0 * 32 + f * 16 + c;
             if (n >= a.N) continue;
             const float bv = a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[n]) : 0.f;
             float* dst = reinterpret_cast<float*>(a.out) + n;
 #pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
+            for (int rf = 0; rf < 2 * BMR; ++rf)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m_lane + rb * 32 + (r & 3) + 8 * (r >> 2);
-                    if (m < a.M) dst[(int64_t)m * a.ldo] = acc[t][rb][r] + bv;
+                for (int r = 0; r < 4; ++r) {
+                    const int m = m0 + row_of(rf, r);
+                    if (m < a.M) dst[(int64_t)m * a.ldo] = acc[f >> 1][f & 1][rf][r] + bv;
                 }
         }
         return;
@@ -197,30 +218,29 @@ template <typename T, int BMR, int ACT, int TW> __device__ __forceinline__ void 
     __syncthreads();
     T* tile_out = reinterpret_cast<T*>(smem);  // [BM][OS]
     const T* bias = reinterpret_cast<const T*>(a.bias);
+    if (ACT == 2) {  // a tile's left columns are those of the gate, the right ones the same of up
 #pragma unroll
-    for (int t = 0; t < TW; ++t) {
-        const int nt = min(nt_raw0 + t, a.NT - 1);
-        if (ACT == 2) {
-            const int half = a.N >> 1, j = nt * 16 + (c & 15);
-            const float bv = bias ? to_f32(bias[c < 16 ? j : half + j]) : 0.f;
+        for (int t = 0; t < TW; ++t) {
+            const int j = min(nt_raw0 + t, a.NT - 1) * 16 + c;
+            const float bg = bias ? to_f32(bias[j]) : 0.f, bu = bias ? to_f32(bias[(a.N >> 1) + j]) : 0.f;
 #pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
+            for (int rf = 0; rf < 2 * BMR; ++rf)
 #pragma unroll
-                for (int r = 0; r < 16; r += 2) {
-                    const uint32_t v0 = __builtin_bit_cast(uint32_t, to_f32(from_f32<T>(acc[t][rb][r] + bv)));
-                    const uint32_t v1 = __builtin_bit_cast(uint32_t, to_f32(from_f32<T>(acc[t][rb][r + 1] + bv)));
-                    const auto p = __builtin_amdgcn_permlane16_swap(v0, v1, false, false);
-                    const uint32_t g0 = p[0], u0 = p[1];
-                    const float gate = __builtin_bit_cast(float, g0), up = __builtin_bit_cast(float, u0);
-                    tile_out[(row_of(rb, r) + (c >> 4)) * OS + (w * TW + t) * 16 + (c & 15)] = from_f32<T>(act2_of<T>(a, gate, up));
+                for (int r = 0; r < 4; ++r) {
+                    const float gate = to_f32(from_f32<T>(acc[t][0][rf][r] + bg)), up = to_f32(from_f32<T>(acc[t][1][rf][r] + bu));
+                    tile_out[row_of(rf, r) * OS + (w * TW + t) * 16 + c] = from_f32<T>(act2_of<T>(a, gate, up));
                 }
-        } else {
-            const float bv = bias && nt * 32 + c < a.N ? to_f32(bias[nt * 32 + c]) : 0.f;
+        }
+    } else {
 #pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
+        for (int f = 0; f < 2 * TW; ++f) {
+            const int n = nt_raw0 * 32 + f * 16 + c;
+            const float bv = bias && n < a.N ? to_f32(bias[n]) : 0.f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    tile_out[row_of(rb, r) * OS + (w * TW + t) * 32 + c] = dense::finish_out<T>(acc[t][rb][r] + bv, a.gelu);
+            for (int rf = 0; rf < 2 * BMR; ++rf)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    tile_out[row_of(rf, r) * OS + w * (32 * TW) + f * 16 + c] = dense::finish_out<T>(acc[f >> 1][f & 1][rf][r] + bv, a.gelu);
         }
     }
     __syncthreads();
@@ -324,7 +344,8 @@ struct TallPlan {
 };
 // us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip.  These and the constants of walk_us, launch_us and the two
 // plan makers are fitted to 280 products of 65 to 8000 rows and 1024 x 1024 to 57344 x 8192, each with up to 48 plans, weights cold (the copies of
-// a matrix that take turns are more than the caches hold): the estimates are 5 % off, the plans that they pick 0.9 % behind the best, at most 9.
+// a matrix that take turns are more than the caches hold): the estimates are 5 % off, the plans that they pick 0.9 % behind the best, at most 9.  (Of the 32x32x16 form; with 16x16x32
+// they are 13 % off, mostly above, and the plans still 1.0 % behind the best of 57 products, at most 13.)
 struct TallCost {
     double alone, busy;
 };

@@ -20,6 +20,15 @@ __device__ __forceinline__ void tile_at(int t, int rows, int cols, int& row, int
     col = in / h;
 }
 
+// 16 (4) bytes at base + at + off, base and at the same for the wave: the buffer form, which takes no 64-bit address per lane.  bytes: the range past which it reads
+// zeros.  NT: 2 for a line that is read once.
+template <int NT> __device__ __forceinline__ auto buffer_piece(const uint8_t* base, int bytes, uint32_t off, int at) {
+    return __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00020000), off, at, NT);
+}
+__device__ __forceinline__ uint32_t buffer_word(const uint8_t* base, int bytes, uint32_t off, int at) {
+    return __builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, bytes, 0x00020000), off, at, 0);
+}
+
 constexpr int RING = 4;
 
 // The end of a step: the buffer that step s + 2 reads is whole for every wave, with BEHIND vector loads issued behind its own.  The count holds
