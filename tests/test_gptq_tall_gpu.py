@@ -8,9 +8,9 @@ pytestmark = pytest.mark.gpu
 
 
 # K: one step, fewer and more steps than the ring of buffers, a whole number of rings; N: one tile, ragged and several column blocks; the last
-# size has more tiles than the 256 of a whole round, so that a split plan launches whole tiles and split ones behind them
+# sizes have more tiles than the 256 of a whole round, so that a split plan launches whole tiles and split ones behind them: of the smallest tile, of each
 @pytest.mark.parametrize("K,N,groupsize,M", [(*shape, M) for shape in [(64, 32, 64), (192, 288, 64), (320, 512, 64), (1024, 1120, 128), (1152, 96, 1152)]
-                                             for M in (129, 161, 300)] + [(320, 4128, 64, 700)])
+                                             for M in (129, 161, 300)] + [(320, 4128, 64, 700), (320, 4128, 64, 2100)])
 @pytest.mark.parametrize("act", [0, 2])
 def test_every_plan(gpu_device, K, N, groupsize, M, act, monkeypatch):
     from tgis_amd import native
@@ -47,11 +47,13 @@ def test_every_plan(gpu_device, K, N, groupsize, M, act, monkeypatch):
 
 
 # behind a whole turn of the ring of four buffers: one, two and three steps, and none; behind none, and in the parts of a split
+# (the larger product has more than 256 tiles of each size, which take the other shape of the matrix instruction)
 @pytest.mark.parametrize("steps,S", [(1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (6, 1), (7, 1), (11, 1), (14, 2)])
-def test_tails_of_the_ring(gpu_device, steps, S, monkeypatch):
+@pytest.mark.parametrize("N,M", [(288, 290), (4128, 2100)])
+def test_tails_of_the_ring(gpu_device, steps, S, N, M, monkeypatch):
     from tgis_amd import native
 
-    K, N, M = 64 * steps, 288, 290
+    K = 64 * steps
     qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, 64, seed=steps)
     w = native.GptqWeight(*(torch.from_numpy(t).to(gpu_device) for t in (qw, qz, sc)), torch.from_numpy(gi), 4, 64)
     x = torch.randn(M, K, generator=torch.Generator().manual_seed(steps)).half()

@@ -6,17 +6,18 @@
 // applies them to all BMR row blocks.  No scratch copy of W, no second pass over the weights, SiLU * up in the epilogue.
 //
 // Rows of x go to LDS by direct loads, 64 k at a time, three steps ahead, into a ring of four buffers: no registers, no stores, and one
-// barrier per step (32 MFMAs per wave at TW 2), behind which the NEXT step's x is complete too, so that its first fragments are read
-// before the barrier.  A buffer row is 128 bytes; its 16-byte pieces are stored at piece ^ (row & 7) (each lane of the load asks for the
-// piece that belongs at its place), so that fragment reads of 32 rows meet no bank twice.  Inside a step the four 16-k slices are
-// pipelined: while slice i is multiplied, slice i + 1 is dequantised and its A fragments are read.
+// barrier per step, behind which the NEXT step's x is complete too, so that its first fragments are read
+// before the barrier.  A buffer row is 128 bytes; its 16-byte pieces are stored at piece ^ (row / 2 & 7) (each lane of the load asks for the
+// piece that belongs at its place), so that fragment reads of 16 rows meet no bank twice.  Inside a step the slices are
+// pipelined: while one is multiplied, the next is dequantised and its A fragments are read.
 //
-// Bound: the matrix cores, which this card's power holds to about 1.5 PFLOP/s on random data whatever feeds them (a bare MFMA loop), and
+// Bound: the matrix cores, which this card's power holds to 1.7 (32x32x16) and 1.95 PFLOP/s (16x16x32) on random data in a bare loop, and
 // the dequantisation's share of that power.  A 128 x 256 tile of 4096 k takes 45 us alone on a CU, 56 on a full chip (1.2 PFLOP/s); several
-// blocks on a CU only share its matrix cores, so that the plan below weighs whole rounds of 256 CUs.  7B layer, 765 rows: qkv 79 -> 77,
-// o 36 -> 32, gate_up 145 -> 138, down 81 -> 74 us with the loop in whole turns of its ring (below); 300 rows 41 -> 38, 28 -> 23, 72, 45 -> 42.
+// blocks on a CU only share its matrix cores, so that the plan below weighs whole rounds of 256 CUs.  7B layer, 765 rows, us, with the loop in whole turns of its
+// ring (below) / and the 16x16x32 form: qkv 79 -> 77 -> 73, o 36 -> 32, gate_up 145 -> 138 -> 130, down 81 -> 74; 300 rows 41 -> 38, 28 -> 23, 72 -> 68, 45 -> 42.
 #include <stdlib.h>
 #include <algorithm>
+#include <type_traits>
 #include "common.h"
 #include "gptq_gemm_body.h"
 #include "gptq_tall.h"
@@ -43,7 +44,7 @@ struct TallArgs {
     float* scratch;
 };
 
-constexpr int TALL_RING = tall::RING;  // k64-steps of weights in flight per wave, and buffers of x
+constexpr int TALL_RING = tall::RING;  // buffers of x
 
 // The order of tiles (tall_ring.h).  us, columns fastest over the whole chip / this: 4096 x 22016 with SiLU at 300, 765, 6000 rows 74.9 / 69.4, 148.6 /
 // 146.2, 989 / 961; 8192 x 57344 with SiLU at 300, 3000 rows 345 / 324, 2611 / 2456; 11008 x 4096 at 140, 300, 765 rows 33.3 / 30.3, 41.3 / 42.6,
@@ -51,7 +52,73 @@ constexpr int TALL_RING = tall::RING;  // k64-steps of weights in flight per wav
 using tall::tile_at;
 using tall::xcd_run;
 
-template <int BMR, int ACT, int TW>
+// A wave's sums, 32 BMR rows of TW tiles, as the two shapes of the matrix instruction leave them in its lanes.  each: f(row, column of the tile, sum); pairs: the
+// same of a gate | up tile, f(row, j, rounded gate, rounded up) of its columns j and 16 + j, given their biases.
+template <int BMR, int TW> struct Sums16 {
+    f32x4 v[TW][2][2 * BMR];  // 16x16x32: [tile][its left, right columns][rows 16 i .. + 15]
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int rf = 0; rf < 2 * BMR; ++rf) v[t][h][rf] = f32x4{0, 0, 0, 0};
+    }
+    template <typename F> __device__ __forceinline__ void each(int t, int lane, F f) const {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int rf = 0; rf < 2 * BMR; ++rf)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) f(rf * 16 + 4 * (lane >> 4) + r, h * 16 + (lane & 15), v[t][h][rf][r]);
+    }
+    template <typename F> __device__ __forceinline__ void pairs(int t, int lane, float bias_gate, float bias_up, F f) const {
+#pragma unroll
+        for (int rf = 0; rf < 2 * BMR; ++rf)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                f(rf * 16 + 4 * (lane >> 4) + r, lane & 15, (float)(f16)(v[t][0][rf][r] + bias_gate), (float)(f16)(v[t][1][rf][r] + bias_up));
+    }
+};
+template <int BMR, int TW> struct Sums32 {
+    f32x16 v[TW][BMR];  // 32x32x16: [tile][rows 32 i .. + 31]
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int rb = 0; rb < BMR; ++rb) v[t][rb] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    static __device__ __forceinline__ int row_of(int lane, int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); }
+    template <typename F> __device__ __forceinline__ void each(int t, int lane, F f) const {
+#pragma unroll
+        for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) f(row_of(lane, rb, r), lane & 31, v[t][rb][r]);
+    }
+    // Lanes 0 - 15 of a half wave hold gate columns, 16 - 31 the matching up columns.  Swapping those rows of lanes between two
+    // accumulator rows gives every lane a (gate, up) pair: the lower lanes that of row r, the upper ones that of row r + 1.
+    template <typename F> __device__ __forceinline__ void pairs(int t, int lane, float bias_gate, float bias_up, F f) const {
+        const int c = lane & 31;
+        const float bv = c < 16 ? bias_gate : bias_up;
+#pragma unroll
+        for (int rb = 0; rb < BMR; ++rb)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const uint32_t v0 = __builtin_bit_cast(uint32_t, (float)(f16)(v[t][rb][r] + bv));
+                const uint32_t v1 = __builtin_bit_cast(uint32_t, (float)(f16)(v[t][rb][r + 1] + bv));
+                const auto p = __builtin_amdgcn_permlane16_swap(v0, v1, false, false);
+                const uint32_t g0 = p[0], u0 = p[1];  // (a bit cast of a vector's element itself reads element 0)
+                f(row_of(lane, rb, r) + (c >> 4), c & 15, __builtin_bit_cast(float, g0), __builtin_bit_cast(float, u0));
+            }
+    }
+};
+
+// M16: products by the 16x16x32 instruction instead of 32x32x16.  Under the card's power limit it does more: bare loops on random f16 1.95 against 1.71 PFLOP/s
+// (bf16 2.10, 1.77).  Where a SIMD has one wave it is the slower one: twice the products to issue, and 19 TW register moves between the lanes' halves a step.
+// us, 32x32x16 / 16x16x32, tiles of 96 x 128, 96 x 256, 128 x 256: 4096 x 22016 with SiLU at 2045 rows 370 / 352, 362 / 339, 340 / 316; 4096 x 12288 at 1500 152 /
+// 146, 143 / 139, 161 / 155; of up to 256 blocks 4096 x 4096 at 763 33.1 / 34.2, 41.5 / 49.6, 46.7 / 57.1; 11008 x 4096 at 2045 (128 x 256) 164 / 172.
+// Tiles of 64 rows have too few products to a dequantised fragment for either to matter (4096 x 12288 at 763 rows 92 / 91, 94 / 94).
+template <int BMR, int ACT, int TW, bool M16>
 __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     constexpr int BM = 32 * BMR;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // [TALL_RING][BM][128 bytes]
@@ -66,24 +133,35 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     const int ksteps = a.K >> 6;                                         // K % 64 == 0 (host)
     const int ks0 = split * a.per, n = min(ksteps, ks0 + a.per) - ks0;   // n >= 1 (host)
 
-    const char* wtile[TW];
-    const char* sztile[TW];
+    const uint8_t *wtile[TW], *sztile[TW];
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
         const int nt = min(nt_raw0 + t, a.NT - 1);
-        wtile[t] = reinterpret_cast<const char*>(a.prep) + (int64_t)nt * a.KS * 1024;
-        sztile[t] = reinterpret_cast<const char*>(a.prep + a.offB) + (int64_t)nt * a.G * 128;
+        wtile[t] = a.prep + (int64_t)nt * a.KS * 1024;
+        sztile[t] = a.prep + a.offB + (int64_t)nt * a.G * 128;
     }
     const uint32_t woff = lane * 16, szoff = (lane & 31) * 4;
+    // (M16 has no registers to spare for addresses; where a wave is waited for, the loads that need none are the slower ones: 4096 x 4096 at 300 rows in tiles of
+    // 64 x 128 24.2 / 25.8 us)
     auto sz_at = [&](int t, int ks) -> uint32_t {
-        const char* p = sztile[t] + (int64_t)min(ks >> a.spg_shift, a.G - 1) * 128;
-        PIN_SGPR(p);
-        return *(const GLOBAL_AS uint32_t*)(p + szoff);
+        const int at = min(ks >> a.spg_shift, a.G - 1) * 128;
+        if constexpr (M16) {
+            return tall::buffer_word(sztile[t], a.G * 128, szoff, at);
+        } else {
+            const uint8_t* p = sztile[t] + at;
+            PIN_SGPR(p);
+            return *(const GLOBAL_AS uint32_t*)(p + szoff);
+        }
     };
     auto w_at = [&](int t, int ks) -> u32x4 {
-        const char* p = wtile[t] + (int64_t)min(ks, ksteps - 1) * 1024;
-        PIN_SGPR(p);
-        return __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(p + woff));
+        const int at = min(ks, ksteps - 1) * 1024;
+        if constexpr (M16) {
+            return __builtin_bit_cast(u32x4, tall::buffer_piece<2>(wtile[t], a.KS * 1024, woff, at));
+        } else {
+            const uint8_t* p = wtile[t] + at;
+            PIN_SGPR(p);
+            return __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(p + woff));
+        }
     };
 
     // x: load j of wave w brings rows 8 (4 j + w) .. + 7 (rows past M: the last one, never stored)
@@ -91,7 +169,7 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     uint32_t rowoff[BMR];
 #pragma unroll
     for (int j = 0; j < BMR; ++j)
-        rowoff[j] = (uint32_t)(min(8 * (4 * j + w) + (lane >> 3), mrows - 1) * (int)a.ldx * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+        rowoff[j] = (uint32_t)(min(8 * (4 * j + w) + (lane >> 3), mrows - 1) * (int)a.ldx * 2 + ((lane & 7) ^ (4 * (w & 1) + (lane >> 4))) * 16);
     const char* xbase = reinterpret_cast<const char*>(a.x + (int64_t)m0 * a.ldx);
     auto x_load = [&](int step, int buf) {
         const char* xb = xbase + (int64_t)min(ks0 + step, ksteps - 1) * 128;
@@ -104,23 +182,29 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     uint32_t EXr = 0x64006400u, M0r = 0x000F000Fu, M1r = 0x00F000F0u;
     asm volatile("" : "+v"(EXr));
     asm volatile("" : "+s"(M0r), "+s"(M1r));
-    f32x16 acc[TW][BMR];
+    std::conditional_t<M16, Sums16<BMR, TW>, Sums32<BMR, TW>> acc;
+    acc.clear();
+    // A fragments.  M16: lane (c, q) has row c of its sixteen, and of the 32 k of slice m the step's piece 4 (q / 2) + 2 m + q % 2, as the swap in `halves` leaves
+    // those of the weights.  Else: slice i, row lane % 32, piece i + 4 (lane / 32).
+    const int c = lane & 15, q = lane >> 4;
+    constexpr int SLICES = M16 ? 2 : 4, FRAGS = M16 ? 2 * BMR : BMR;
+    uint32_t apos[SLICES];
 #pragma unroll
-    for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int rb = 0; rb < BMR; ++rb) acc[t][rb] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // A fragment of slice i, row block rb: row 32 rb + lane % 32, piece i + 4 (lane / 32)
-    uint32_t apos[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) apos[i] = (uint32_t)((lane & 31) * 128 + ((i + 4 * (lane >> 5)) ^ (lane & 7)) * 16);
+    for (int i = 0; i < SLICES; ++i) {
+        const int row = M16 ? c : lane & 31, piece = M16 ? (q >> 1) * 4 + i * 2 + (q & 1) : i + 4 * (lane >> 5);
+        apos[i] = (uint32_t)(row * 128 + (piece ^ ((row >> 1) & 7)) * 16);
+    }
 
     x_load(0, 0);
     x_load(1, 1);
     x_load(2, 2);
-    u32x4 wq[TALL_RING][TW];
-    uint32_t szr[TALL_RING][TW];
+    // k64-steps of weights in flight per wave, slices of x in registers: the 16x16x32 form of the larger tiles has room for less
+    constexpr bool LEAN = M16 && TW == 2;
+    constexpr int WR = LEAN && BMR == 4 ? 2 : 4, AS = LEAN ? 1 : 2;
+    u32x4 wq[WR][TW];
+    uint32_t szr[WR][TW];
 #pragma unroll
-    for (int s = 0; s < TALL_RING; ++s)
+    for (int s = 0; s < WR; ++s)
 #pragma unroll
         for (int t = 0; t < TW; ++t) {
             szr[s][t] = sz_at(t, ks0 + s);
@@ -129,53 +213,106 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
-    f16x8 b[2][TW], av[2][BMR];
-    auto dequant = [&](f16x8 (&dst)[TW], const u32x4 (&q)[TW], const uint32_t (&sz)[TW], int i) {
-#pragma unroll
-        for (int t = 0; t < TW; ++t) {
-            const f16x2 szh = __builtin_bit_cast(f16x2, sz[t]);
-            const f16 zd1 = (f16)960.f - szh[1];
-            dst[t] = gptq::dequant8(q[t][i], f16x2{szh[1], szh[1]}, f16x2{zd1, zd1}, f16x2{szh[0], szh[0]}, EXr, M0r, M1r);
-        }
+    f16x8 b[2][TW], av[AS][FRAGS];
+    uint32_t scale[TW][2];
+    // A register of the image holds a tile's left columns in the first and third row of lanes, its right ones in the others: swapping the second row of one
+    // with the first of the next, and the fourth with the third, leaves the left columns of both in one register, the right ones in the other.
+    auto halves = [&](uint32_t& l, uint32_t& r) {
+        const auto p = __builtin_amdgcn_permlane16_swap(l, r, false, false);
+        l = p[0];
+        r = p[1];
     };
-    auto read_a = [&](f16x8 (&dst)[BMR], int buf, int i) {
-#pragma unroll
-        for (int rb = 0; rb < BMR; ++rb) dst[rb] = ld16<f16x8>(smem + buf * (BM * 128) + rb * 4096 + apos[i]);
+    auto words = [&](u32x4 (&wr)[TW], int t, int m) {
+        if (!M16) return;
+        uint32_t l = wr[t][2 * m], r = wr[t][2 * m + 1];
+        halves(l, r);
+        wr[t][2 * m] = l;
+        wr[t][2 * m + 1] = r;
     };
-    read_a(av[0], 0, 0);
-    dequant(b[0], wq[0], szr[0], 0);
+    auto scales = [&](const uint32_t (&sz)[TW], int t) {
+        scale[t][0] = scale[t][1] = sz[t];
+        if (M16) halves(scale[t][0], scale[t][1]);
+    };
+    auto dequant = [&](f16x8& dst, const u32x4 (&wr)[TW], int t, int u) {  // word u of a step: M16 half u % 2 of slice u / 2, else slice u
+        const f16x2 szh = __builtin_bit_cast(f16x2, scale[t][M16 ? u & 1 : 0]);
+        const f16 zd1 = (f16)960.f - szh[1];
+        dst = gptq::dequant8(wr[t][u], f16x2{szh[1], szh[1]}, f16x2{zd1, zd1}, f16x2{szh[0], szh[0]}, EXr, M0r, M1r);
+    };
+    auto read_a = [&](int rf, int buf, int i) { av[i % AS][rf] = ld16<f16x8>(smem + buf * (BM * 128) + rf * (BM * 128 / FRAGS) + apos[i]); };
+#pragma unroll
+    for (int rf = 0; rf < FRAGS; ++rf) read_a(rf, 0, 0);
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+        scales(szr[0], t);
+        words(wq[0], t, 0);
+        dequant(b[0][t], wq[0], t, 0);
+    }
     auto step = [&](int s, auto slot_, auto tail_) {
         constexpr int SL = decltype(slot_)::value;
-        constexpr bool TAIL = decltype(tail_)::value;  // (at most RING - 1 steps: their weights are there)
-        constexpr int NX = (SL + 1) % TALL_RING;
+        constexpr bool TAIL = decltype(tail_)::value;  // (at most RING - 1 steps, the first at slot 0)
+        constexpr int NX = (SL + 1) % TALL_RING, WS = SL % WR, WN = (SL + 1) % WR;
+        constexpr bool REFILL = !TAIL || SL + WR < TALL_RING - 1;
         if constexpr (!TAIL) x_load(s + 3, (SL + 3) % TALL_RING);  // everyone is done with that buffer since the barrier of the step before
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            read_a(av[(i + 1) & 1], i < 3 ? SL : NX, (i + 1) & 3);
+        for (int u = 0; u < 4; ++u) {
             __builtin_amdgcn_sched_barrier(0);
-            if (i == 3) {
-                if constexpr (!TAIL) {
+            auto refill = [&]() {
+                if constexpr (REFILL) {
+                    if (u < 3) return;
 #pragma unroll
                     for (int t = 0; t < TW; ++t) {
-                        wq[SL][t] = w_at(t, ks0 + s + TALL_RING);
-                        szr[SL][t] = sz_at(t, ks0 + s + TALL_RING);
+                        wq[WS][t] = w_at(t, ks0 + s + WR);
+                        szr[WS][t] = sz_at(t, ks0 + s + WR);
                     }
                 }
-                dequant(b[0], wq[NX], szr[NX], 0);
+            };
+            auto dequant_next = [&](int t) {
+                if (u == 3) scales(szr[WN], t);
+                if (u & 1) words(wq[u == 3 ? WN : WS], t, u == 1);
+                dequant(b[(u + 1) & 1][t], wq[u == 3 ? WN : WS], t, (u + 1) & 3);
+            };
+            if constexpr (LEAN) {
+                refill();
+                // rows in turn, in this order: a slice's are read again, for the next slice, behind their last product, and the next fragment of each tile is
+                // dequantised between two of them
+#pragma unroll
+                for (int rf = 0; rf < 2 * BMR; ++rf) {
+#pragma unroll
+                    for (int t = 0; t < TW; ++t) acc.v[t][u & 1][rf] = mfma16(av[0][rf], b[u & 1][t], acc.v[t][u & 1][rf]);
+                    if (u & 1) read_a(rf, u == 1 ? SL : NX, (u >> 1) ^ 1);
+#pragma unroll
+                    for (int t = 0; t < TW; ++t)
+                        if (rf == (2 * BMR * t) / TW) dequant_next(t);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             } else {
-                dequant(b[(i + 1) & 1], wq[SL], szr[SL], i + 1);
+                if (!M16 || !(u & 1)) {
+                    const int next = M16 ? (u >> 1) ^ 1 : (u + 1) & 3;
+#pragma unroll
+                    for (int rf = 0; rf < FRAGS; ++rf) read_a(rf, next ? SL : NX, next);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                refill();
+#pragma unroll
+                for (int t = 0; t < TW; ++t) dequant_next(t);
+#pragma unroll
+                for (int rf = 0; rf < FRAGS; ++rf)
+#pragma unroll
+                    for (int t = 0; t < TW; ++t) {
+                        if constexpr (M16)
+                            acc.v[t][u & 1][rf] = mfma16(av[u >> 1][rf], b[u & 1][t], acc.v[t][u & 1][rf]);
+                        else
+                            acc.v[t][rf] = mfma32(av[u & 1][rf], b[u & 1][t], acc.v[t][rf]);
+                    }
+                // the dequantisation's 13 TW instructions, and the swaps in front, between the products
+                constexpr int PRODUCTS = FRAGS * TW;
+#pragma unroll
+                for (int g = 0; g < PRODUCTS; ++g) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, ((M16 ? 16 : 13) * TW + PRODUCTS - 1) / PRODUCTS, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
-#pragma unroll
-                for (int t = 0; t < TW; ++t) acc[t][rb] = mfma32(av[i & 1][rb], b[i & 1][t], acc[t][rb]);
-            // a slice's 13 TW dequantisation instructions between its BMR TW products
-#pragma unroll
-            for (int g = 0; g < BMR * TW; ++g) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, (13 * TW + BMR * TW - 1) / (BMR * TW), 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
         }
         // the x loads of step s + 2 were issued a step ago: behind them this wave has asked for that step's 2 TW weights and scales
         // and, in whole turns, for everything of this step
@@ -184,18 +321,11 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     tall::ring_steps(n, step);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way to LDS when the block ends
 
-    // ---- epilogue: lane holds rows m = 32 rb + (r & 3) + 8 (r >> 2) + 4 (lane >> 5) of column nt * 32 + (lane & 31) -----------
-    const int c = lane & 31;
-    auto row_of = [&](int rb, int r) { return rb * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5); };
     constexpr int BN = 128 * TW;
     if (a.part) {
-        float* dst = a.scratch + ((int64_t)xcd_run(blockIdx.x, gridDim.x) * a.S + split) * (BM * BN) + w * (32 * TW) + c;
+        float* dst = a.scratch + ((int64_t)xcd_run(blockIdx.x, gridDim.x) * a.S + split) * (BM * BN) + w * (32 * TW);
 #pragma unroll
-        for (int t = 0; t < TW; ++t)
-#pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) dst[(int64_t)row_of(rb, r) * BN + t * 32] = acc[t][rb][r];
+        for (int t = 0; t < TW; ++t) acc.each(t, lane, [&](int row, int col, float sum) { dst[(int64_t)row * BN + t * 32 + col] = sum; });
         return;
     }
     // finished: the tile goes through LDS so that rows leave in 16-byte pieces, 512 (256 with SiLU * up) contiguous bytes a row
@@ -207,28 +337,16 @@ __global__ __launch_bounds__(256, 2) void gptq_gemm_tall_kernel(TallArgs a) {
     for (int t = 0; t < TW; ++t) {
         const int nt = min(nt_raw0 + t, a.NT - 1);
         if (ACT == 2) {
-            // Lanes 0 - 15 of a half wave hold gate columns, 16 - 31 the matching up columns.  Swapping those rows of lanes between two
-            // accumulator rows gives every lane a (gate, up) pair: the lower lanes that of row r, the upper ones that of row r + 1.
-            const int half = a.N >> 1, j = nt * 16 + (c & 15);
-            const float bv = a.bias ? (float)a.bias[c < 16 ? j : half + j] : 0.f;
-#pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
-#pragma unroll
-                for (int r = 0; r < 16; r += 2) {
-                    const uint32_t v0 = __builtin_bit_cast(uint32_t, (float)(f16)(acc[t][rb][r] + bv));
-                    const uint32_t v1 = __builtin_bit_cast(uint32_t, (float)(f16)(acc[t][rb][r + 1] + bv));
-                    const auto p = __builtin_amdgcn_permlane16_swap(v0, v1, false, false);
-                    const uint32_t g0 = p[0], u0 = p[1];  // (a bit cast of a vector's element itself reads element 0)
-                    const float gate = __builtin_bit_cast(float, g0), up = __builtin_bit_cast(float, u0);
-                    const float sl = gate / (1.f + __expf(-gate));
-                    tile_out[(row_of(rb, r) + (c >> 4)) * OS + (w * TW + t) * 16 + (c & 15)] = (f16)((float)(f16)sl * up);
-                }
+            const int j = nt * 16 + c;
+            acc.pairs(t, lane, a.bias ? (float)a.bias[j] : 0.f, a.bias ? (float)a.bias[(a.N >> 1) + j] : 0.f, [&](int row, int col, float gate, float up) {
+                const float sl = gate / (1.f + __expf(-gate));
+                tile_out[row * OS + (w * TW + t) * 16 + col] = (f16)((float)(f16)sl * up);
+            });
         } else {
-            const float bv = a.bias ? (float)a.bias[nt * 32 + c] : 0.f;
-#pragma unroll
-            for (int rb = 0; rb < BMR; ++rb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) tile_out[row_of(rb, r) * OS + (w * TW + t) * 32 + c] = (f16)(acc[t][rb][r] + bv);
+            const float left = a.bias ? (float)a.bias[nt * 32 + (M16 ? c : lane & 31)] : 0.f, right = M16 && a.bias ? (float)a.bias[nt * 32 + 16 + c] : left;
+            acc.each(t, lane, [&](int row, int col, float sum) {
+                tile_out[row * OS + (w * TW + t) * 32 + col] = (f16)(sum + (M16 && col >= 16 ? right : left));
+            });
         }
     }
     __syncthreads();
@@ -296,7 +414,8 @@ struct TallPlan {
 
 // us per k64-step of a block that has its CU to itself, and of a CU's share of a full chip (several blocks on each; clocks drop under
 // the matrix cores' load).  Fitted to launches of 23 - 400 us at the 7B shapes; over 21 matrices and 16 row counts from 65 to 6000, weights
-// cold, the plans that the model picks are 1.1 % up to 256 rows, 0.6 above behind the best of up to 48 that were timed at each size.
+// cold, the plans that the model picks are 1.1 % up to 256 rows, 0.6 above behind the best of up to 48 that were timed at each size (with the 16x16x32 form 0.5 %
+// over 53 products, at most 9).
 struct TallCost {
     double alone, busy;
 };
@@ -347,18 +466,24 @@ int64_t plan_scratch(const TallPlan& p) {
     return p.whole < p.tiles ? (int64_t)(p.tiles - p.whole) * p.S * (32 * p.BMR) * (128 * p.TW) * 4 : 0;
 }
 
-template <int BMR, int ACT, int TW>
-int launch_blocks(const TallArgs& a, int tiles, int S, hipStream_t st) {
+template <int BMR, int ACT, int TW, bool M16>
+int launch_form(const TallArgs& a, int tiles, int S, hipStream_t st) {
     constexpr size_t ring = (size_t)TALL_RING * (32 * BMR) * 128, rows = (size_t)(32 * BMR) * ((ACT == 2 ? 64 : 128) * TW + 8) * 2;
     constexpr size_t lds = ring > rows ? ring : rows;
-    static const hipError_t attr = hipFuncSetAttribute((const void*)gptq_gemm_tall_kernel<BMR, ACT, TW>,
+    static const hipError_t attr = hipFuncSetAttribute((const void*)gptq_gemm_tall_kernel<BMR, ACT, TW, M16>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     TGIS_CHECK_HIP(attr);
-    hipLaunchKernelGGL((gptq_gemm_tall_kernel<BMR, ACT, TW>), dim3((unsigned)tiles, (unsigned)S), dim3(256), lds, st, a);
+    hipLaunchKernelGGL((gptq_gemm_tall_kernel<BMR, ACT, TW, M16>), dim3((unsigned)tiles, (unsigned)S), dim3(256), lds, st, a);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
-
+// (M16: where CUs have two blocks, and tiles of more than 64 rows)
+template <int BMR, int ACT, int TW>
+int launch_blocks(const TallArgs& a, int tiles, int S, hipStream_t st) {
+    if constexpr (BMR > 2)
+        if ((int64_t)tiles * S > CUS) return launch_form<BMR, ACT, TW, true>(a, tiles, S, st);
+    return launch_form<BMR, ACT, TW, false>(a, tiles, S, st);
+}
 template <int ACT>
 int launch_shape(const TallPlan& p, const TallArgs& a, int tiles, int S, hipStream_t st) {
     switch (p.BMR * 10 + p.TW) {
