@@ -323,6 +323,11 @@ int tgis_rope_kv_write_prefill(void* qkv, int64_t ld_qkv, const void* cos, const
                                const int32_t* cu_seqlens, const int32_t* block_tables, int64_t max_pages, void* k_pool,
                                void* v_pool, int64_t B, int64_t T, int64_t max_len, int H, int Hkv, int D, int rot_dim,
                                int dtype, void* stream);
+/* ... with q left as it came, for tgis_attn_paged_rope. */
+int tgis_rope_k_write_prefill(const void* qkv, int64_t ld_qkv, const void* cos, const void* sin, const int32_t* positions,
+                              const int32_t* cu_seqlens, const int32_t* block_tables, int64_t max_pages, void* k_pool,
+                              void* v_pool, int64_t B, int64_t T, int64_t max_len, int H, int Hkv, int D, int rot_dim,
+                              int dtype, void* stream);
 
 /* ---- paged attention, prefill and decode (replaces flash_attn_2_cuda.varlen_fwd,
  *      utils/flash_attn.py:43-78) ---------------------------------------------------------------- */
@@ -342,6 +347,13 @@ int tgis_attn_paged(const void* q, int64_t ld_q, const void* k_pool, const void*
                     const int32_t* cu_seqlens_q, void* out, int64_t ld_out, int64_t B, int H, int Hkv, int D,
                     int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
                     void* workspace, int64_t workspace_bytes, void* stream);
+/* ... of long queries (tgis_attn_rotates_q: 1), with q rotated as it is read: cos / sin [positions][D / 2] in the model dtype, positions
+ * [total_q]; out [total_q, H * D] contiguous. */
+int tgis_attn_rotates_q(int H, int Hkv, int D, int64_t max_q_len);
+int tgis_attn_paged_rope(const void* q, int64_t ld_q, const void* cos, const void* sin, const int32_t* positions, const void* k_pool,
+                         const void* v_pool, const int32_t* block_tables, int64_t max_pages, const int32_t* ctx_lens,
+                         const int32_t* cu_seqlens_q, void* out, int64_t B, int H, int Hkv, int D, int64_t max_q_len,
+                         int64_t max_ctx, float scale, int dtype, void* stream);
 /* ... of a decode step (one token per sequence), written in fragment order with output column k at column out_cols[k] (a permutation of
  * 0 .. H * D - 1): the order an act-order matrix behind it wants its operand in. */
 int tgis_attn_paged_ordered(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,

@@ -109,3 +109,54 @@ def test_large_and_missing_scores(gpu_device, groups_per_wave, monkeypatch):
     # scores of ~300: an fp32 sum's error moves a probability by up to 300 * 64 * 2 ** -24 of it
     tol = (3 * 2.0 ** -11 + 2 * 300 * D * 2.0 ** -24) * size + 1e-6
     assert ((out.view(n, H, D).double().cpu() - want).abs() <= tol).all()
+
+
+# both head sizes, group widths, tile widths; positions from anywhere in the table; a row stride of its own
+@pytest.mark.parametrize("H,G,D,dtype", [(8, 8, 128, torch.float16), (6, 2, 64, torch.bfloat16), (16, 1, 128, torch.bfloat16), (20, 1, 64, torch.float16)])
+@pytest.mark.parametrize("groups_per_wave", ["1", "2"])
+@pytest.mark.parametrize("lens", [[65], [129, 1, 70], [300, 33]])
+def test_q_rotated_as_it_is_read(gpu_device, H, G, D, dtype, groups_per_wave, lens, monkeypatch):
+    """The bits of a q that is rotated in front of the attention; the same cache pages."""
+    from tgis_amd import native
+
+    monkeypatch.setenv("TGIS_PREFILL_CG", groups_per_wave)
+    g = torch.Generator().manual_seed(H + D + len(lens))
+    T, row = sum(lens), (H + 2 * G) * D
+    qkv = torch.randn(T, row + 8, generator=g).to(dtype).to(gpu_device)
+    angle = torch.rand(700, D // 2, generator=g) * 6.28
+    cos, sin = angle.cos().to(dtype).to(gpu_device), angle.sin().to(dtype).to(gpu_device)
+    pos = torch.randint(0, 700, (T,), generator=g, dtype=torch.int32).to(gpu_device)
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(gpu_device)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=gpu_device)
+    per = [(n + 31) // 32 for n in lens]
+    table = torch.full((len(lens), max(per)), sum(per), dtype=torch.int32)
+    for b, n in enumerate(per):
+        table[b, :n] = torch.arange(sum(per[:b]), sum(per[:b]) + n)
+    table = table.to(gpu_device)
+    assert native.attn_rotates_q(H, G, D, max(lens)) == (max(lens) * min(16, 1 << (H // G - 1).bit_length()) > 64)
+
+    def run(later):
+        x = qkv.clone()
+        kp, vp = (torch.zeros(sum(per) + 1, G, 32 * D, dtype=dtype, device=gpu_device) for _ in range(2))
+        native.rope_kv_write_prefill(x, cos, sin, pos, cu, table, kp, vp, max(lens), H, G, D, D, rotate_q=not later)
+        assert torch.equal(x, qkv) == later
+        out = torch.empty(T, H * D, dtype=dtype, device=gpu_device)
+        native.attn_paged(x, x.stride(0), kp, vp, table, ctx, cu, out, len(lens), H, G, D, max(lens), max(lens), D ** -0.5, 1, None,
+                          **({"rope": (cos, sin, pos)} if later else {}))
+        return out, kp, vp
+
+    for a, b in zip(run(False), run(True)):
+        assert torch.equal(a, b)
+
+
+def test_q_not_rotated_for_short_queries(gpu_device):
+    from tgis_amd import native
+
+    q = torch.zeros(4, 8 * 64, dtype=torch.float16, device=gpu_device)
+    one = torch.ones(1, dtype=torch.int32, device=gpu_device)
+    pool, table = torch.zeros(1, 8, 32 * 64, dtype=torch.float16, device=gpu_device), torch.zeros(1, 1, dtype=torch.int32, device=gpu_device)
+    tables = torch.zeros(8, 32, dtype=torch.float16, device=gpu_device)
+    assert not native.attn_rotates_q(8, 8, 64, 4) and not native.attn_rotates_q(8, 8, 96, 400)
+    with pytest.raises(RuntimeError, match="not for these heads"):
+        native.attn_paged(q, q.stride(0), pool, pool, table, 4 * one, torch.tensor([0, 4], dtype=torch.int32, device=gpu_device), torch.empty_like(q), 1, 8, 8, 64,
+                          4, 4, 0.1, 1, None, rope=(tables, tables, torch.zeros(4, dtype=torch.int32, device=gpu_device)))

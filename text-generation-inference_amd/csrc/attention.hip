@@ -778,11 +778,15 @@ struct CounterLease {  // gives the slot back when the launch is in its stream (
 };
 }  // namespace
 
+// long enough for blocks of 128 columns that stage each K / V page once in LDS (attention_prefill.hip)?
+static bool long_queries(int64_t max_q_len, const AttnGeom& g) { return max_q_len * g.Gp > 64 && !getenv("TGIS_ATTN_NO_PREFILL_KERNEL"); }
+
 static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool,
                            const int32_t* block_tables, int64_t max_pages, const int32_t* ctx_lens,
                            const int32_t* cu_seqlens_q, void* out, int64_t ld_out, const int32_t* out_cols, int64_t B, int H, int Hkv,
                            int D, int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
-                           void* workspace, int64_t workspace_bytes, void* stream) {
+                           void* workspace, int64_t workspace_bytes, void* stream, const void* cos = nullptr, const void* sin = nullptr,
+                           const int32_t* positions = nullptr) {
     TGIS_CHECK_ARG(q && k_pool && v_pool && block_tables && ctx_lens && cu_seqlens_q && out,
                    "tgis_attn_paged: null tensor");
     TGIS_CHECK_ARG(H > 0 && Hkv > 0 && H % Hkv == 0, "tgis_attn_paged: H (%d) must be a multiple of Hkv (%d)", H, Hkv);
@@ -811,6 +815,9 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     a.cu_q = cu_seqlens_q;
     a.out = out;
     a.out_cols = out_cols;
+    a.cosb = cos;
+    a.sinb = sin;
+    a.positions = positions;
     a.out_frag = out_cols ? 2 : ld_out == TGIS_LD_FRAGMENTS;
     a.ld_out = (int64_t)H * D;
     attn_set_geom(a, H, Hkv, g);
@@ -840,7 +847,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
         }
     }
     // long q (prefill): blocks of 128 columns that stage each K/V page once in LDS (attention_prefill.hip)
-    if (num_splits == 1 && max_q_len * g.Gp > 64 && !getenv("TGIS_ATTN_NO_PREFILL_KERNEL")) {
+    if (num_splits == 1 && long_queries(max_q_len, g)) {
         TgisTimedScope timed(TGIS_OP_ATTN, st);
         return tgis_launch_attn_prefill(a, B, Hkv, D, max_q_len, dtype, false, st);
     }
@@ -880,6 +887,22 @@ extern "C" int tgis_attn_paged(const void* q, int64_t ld_q, const void* k_pool, 
                                void* workspace, int64_t workspace_bytes, void* stream) {
     return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, ld_out, nullptr, B, H, Hkv, D,
                            max_q_len, max_ctx, scale, dtype, num_splits, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tgis_attn_rotates_q(int H, int Hkv, int D, int64_t max_q_len) {
+    if (H <= 0 || Hkv <= 0 || H % Hkv != 0 || (D != 64 && D != 128) || max_q_len < 1) return 0;
+    return long_queries(max_q_len, attn_geom(H, Hkv)) ? 1 : 0;
+}
+
+extern "C" int tgis_attn_paged_rope(const void* q, int64_t ld_q, const void* cos, const void* sin, const int32_t* positions, const void* k_pool,
+                                    const void* v_pool, const int32_t* block_tables, int64_t max_pages, const int32_t* ctx_lens,
+                                    const int32_t* cu_seqlens_q, void* out, int64_t B, int H, int Hkv, int D, int64_t max_q_len, int64_t max_ctx,
+                                    float scale, int dtype, void* stream) {
+    TGIS_CHECK_ARG(cos && sin && positions, "tgis_attn_paged_rope: null rotary table");
+    TGIS_CHECK_ARG(tgis_attn_rotates_q(H, Hkv, D, max_q_len), "tgis_attn_paged_rope: not for these heads (%d, %d of %d) and %ld query tokens", H, Hkv, D,
+                   (long)max_q_len);
+    return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, 0, nullptr, B, H, Hkv, D, max_q_len, max_ctx,
+                           scale, dtype, 1, nullptr, 0, stream, cos, sin, positions);
 }
 
 extern "C" int tgis_attn_paged_ordered(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,

@@ -23,6 +23,8 @@ struct AttnArgs {
     unsigned* counters;  // fused combine: per-group arrival counters (zero between launches), or nullptr
     int64_t ld_out;  // prefill kernel: elements between two tokens' rows of `out`
     const int32_t* out_cols;  // out_frag 2: output column k is stored as column out_cols[k] (a permutation)
+    const void *cosb, *sinb;  // prefill kernel: q is rotated as it is read, by these tables [position][D / 2] (or nullptr: it is as it is to be)
+    const int32_t* positions;  // of the q tokens
 };
 
 constexpr float NEG_BIG = -1.0e30f;

@@ -41,6 +41,7 @@ extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, Tgi
     auto tall_parts = [&](int64_t K, int64_t N) { return tall && left && tgis_dense_tall_partial_bytes(T, K, N) >= 0; };
     const bool qkv_tall = tall_parts(p->hidden, QKV), o_tall = tall_parts(HD, p->hidden), down_tall = tall_parts(p->inner, p->hidden);
     const bool qkv_whole = tall && (!left || (p->fresh && tgis_dense_tall_bytes(T, p->hidden, QKV, 0) >= 0));
+    const bool q_later = tgis_attn_rotates_q(p->H, p->Hkv, p->D, p->max_q_len);  // the attention rotates q as it reads it
     auto parts = [&](bool by_tall, const void* in, const void* image, int64_t K, int64_t N, int* slabs, int64_t* row) -> int {
         if (by_tall) return tgis_dense_tall_partial(in, K, image, T, K, N, p->dtype, p->slabs, p->slabs_bytes, slabs, row, stream);
         return tgis_dense_gemm_partial(in, K, image, T, K, N, p->dtype, 0, p->slabs, p->slabs_bytes, slabs, row, stream);
@@ -68,15 +69,22 @@ extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, Tgi
         } else {
             TRY(tgis_dense_tall(p->y, p->hidden, l.qkv, l.qkv_bias, p->qkv, QKV, T, p->hidden, QKV, p->dtype, 0, 0, 0.f, 0.f, ws + 4096,
                                 p->workspace_bytes - 4096, stream));
-            if (p->fresh)
+            if (p->fresh && q_later)
+                TRY(tgis_rope_k_write_prefill(p->qkv, QKV, p->cos, p->sin, p->positions, p->cu_seqlens, p->block_tables, p->max_pages, l.k_pool,
+                                              l.v_pool, p->B, T, p->max_q_len, p->H, p->Hkv, p->D, p->D, p->dtype, stream));
+            else if (p->fresh)
                 TRY(tgis_rope_kv_write_prefill(p->qkv, QKV, p->cos, p->sin, p->positions, p->cu_seqlens, p->block_tables, p->max_pages, l.k_pool,
                                                l.v_pool, p->B, T, p->max_q_len, p->H, p->Hkv, p->D, p->D, p->dtype, stream));
             else
                 TRY(tgis_rope_kv_write(p->qkv, QKV, p->cos, p->sin, p->positions, p->slots, l.k_pool, l.v_pool, T, p->H, p->Hkv, p->D, p->D,
                                        p->dtype, stream));
         }
-        TRY(tgis_attn_paged(p->qkv, QKV, l.k_pool, l.v_pool, p->block_tables, p->max_pages, p->ctx_lens, p->cu_seqlens, p->att, HD, p->B, p->H,
-                            p->Hkv, p->D, p->max_q_len, p->max_ctx, p->scale, p->dtype, 1, nullptr, 0, stream));
+        if (qkv_whole && p->fresh && q_later)
+            TRY(tgis_attn_paged_rope(p->qkv, QKV, p->cos, p->sin, p->positions, l.k_pool, l.v_pool, p->block_tables, p->max_pages, p->ctx_lens, p->cu_seqlens,
+                                     p->att, p->B, p->H, p->Hkv, p->D, p->max_q_len, p->max_ctx, p->scale, p->dtype, stream));
+        else
+            TRY(tgis_attn_paged(p->qkv, QKV, l.k_pool, l.v_pool, p->block_tables, p->max_pages, p->ctx_lens, p->cu_seqlens, p->att, HD, p->B, p->H,
+                                p->Hkv, p->D, p->max_q_len, p->max_ctx, p->scale, p->dtype, 1, nullptr, 0, stream));
         TRY(product(o_tall, p->att, l.o, HD));
         TRY(norm(l.post_norm, p->eps));
         if (tall)

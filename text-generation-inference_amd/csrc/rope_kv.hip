@@ -206,11 +206,9 @@ extern "C" int tgis_rope_kv_write_partial(const float* slabs, int num_slabs, int
                        stream, slabs, num_slabs, slab_ld, bias);
 }
 
-extern "C" int tgis_rope_kv_write_prefill(void* qkv, int64_t ld_qkv, const void* cos, const void* sin,
-                                          const int32_t* positions, const int32_t* cu_seqlens,
-                                          const int32_t* block_tables, int64_t max_pages, void* k_pool, void* v_pool,
-                                          int64_t B, int64_t T, int64_t max_len, int H, int Hkv, int D, int rot_dim,
-                                          int dtype, void* stream) {
+static int write_pages(void* qkv, int64_t ld_qkv, const void* cos, const void* sin, const int32_t* positions, const int32_t* cu_seqlens,
+                       const int32_t* block_tables, int64_t max_pages, void* k_pool, void* v_pool, int64_t B, int64_t T, int64_t max_len, int H, int Hkv,
+                       int D, int rot_dim, int dtype, void* stream, bool rotate_q) {
     TGIS_CHECK_ARG(qkv && cu_seqlens && block_tables && k_pool && v_pool, "tgis_rope_kv_write_prefill: null tensor");
     TGIS_CHECK_ARG(B >= 0 && T >= 0 && max_len >= 0 && max_pages > 0, "tgis_rope_kv_write_prefill: bad sizes");
     TGIS_CHECK_ARG(H > 0 && Hkv > 0 && D > 0 && D % 16 == 0, "tgis_rope_kv_write_prefill: head_dim must be a multiple of 16");
@@ -219,10 +217,13 @@ extern "C" int tgis_rope_kv_write_prefill(void* qkv, int64_t ld_qkv, const void*
                    "tgis_rope_kv_write_prefill: rot_dim must be a multiple of 16 and <= head_dim");
     TGIS_CHECK_ARG(dtype == TGIS_F16 || dtype == TGIS_BF16, "tgis_rope_kv_write_prefill: bad dtype");
     if (B == 0 || T == 0) return TGIS_OK;
-    // q heads: rotated in place by the per-token kernel (no cache traffic: Hkv = 0, no pools)
-    int rc = rope_launch(qkv, ld_qkv, cos, sin, positions, nullptr, nullptr, nullptr, T, H, 0, D, rot_dim, dtype, stream,
-                         nullptr, 0, 0, nullptr);
-    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(ld_qkv % 8 == 0 && ld_qkv >= (int64_t)H * D, "tgis_rope_kv_write_prefill: bad row stride");
+    // q heads: rotated in place by the per-token kernel (no cache traffic: Hkv = 0, no pools).  Without rotary embedding there is nothing to do (it read q for
+    // nothing: 8186 rows of 48 heads of 128 24 us).
+    if (rotate_q && cos) {
+        const int rc = rope_launch(qkv, ld_qkv, cos, sin, positions, nullptr, nullptr, nullptr, T, H, 0, D, rot_dim, dtype, stream, nullptr, 0, 0, nullptr);
+        if (rc != TGIS_OK) return rc;
+    }
     hipStream_t st = (hipStream_t)stream;
     const int pps = (int)cdiv64(max_len, 32);
     TGIS_CHECK_ARG(pps <= max_pages && B * pps <= 2147483647LL && Hkv <= 65535, "tgis_rope_kv_write_prefill: grid too large");
@@ -239,4 +240,20 @@ extern "C" int tgis_rope_kv_write_prefill(void* qkv, int64_t ld_qkv, const void*
                            (bf16*)k_pool, (bf16*)v_pool, H, Hkv, D, rot_dim, pps);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
+}
+
+extern "C" int tgis_rope_kv_write_prefill(void* qkv, int64_t ld_qkv, const void* cos, const void* sin,
+                                          const int32_t* positions, const int32_t* cu_seqlens,
+                                          const int32_t* block_tables, int64_t max_pages, void* k_pool, void* v_pool,
+                                          int64_t B, int64_t T, int64_t max_len, int H, int Hkv, int D, int rot_dim,
+                                          int dtype, void* stream) {
+    return write_pages(qkv, ld_qkv, cos, sin, positions, cu_seqlens, block_tables, max_pages, k_pool, v_pool, B, T, max_len, H, Hkv, D, rot_dim, dtype,
+                       stream, true);
+}
+
+extern "C" int tgis_rope_k_write_prefill(const void* qkv, int64_t ld_qkv, const void* cos, const void* sin, const int32_t* positions,
+                                         const int32_t* cu_seqlens, const int32_t* block_tables, int64_t max_pages, void* k_pool, void* v_pool, int64_t B,
+                                         int64_t T, int64_t max_len, int H, int Hkv, int D, int rot_dim, int dtype, void* stream) {
+    return write_pages(const_cast<void*>(qkv), ld_qkv, cos, sin, positions, cu_seqlens, block_tables, max_pages, k_pool, v_pool, B, T, max_len, H, Hkv, D,
+                       rot_dim, dtype, stream, false);
 }

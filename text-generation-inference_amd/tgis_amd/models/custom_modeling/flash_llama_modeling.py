@@ -180,9 +180,11 @@ class FlashLlamaAttention:
             self.query_key_value.linear.rope_heads = (self.num_heads, self.num_key_value_heads, self.head_size)
         self.out_places: Optional[torch.Tensor] = None  # an act-order o_proj's order of the attention's output columns (post_init)
 
-    def project_qkv(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False):
-        """qkv GEMM, rotation of q and k in place, k and v scattered to their page slots (reference :251-268,282).
-        gathered: hidden_states' columns are in the order of an act-order qkv weight."""
+    def project_qkv(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False,
+                    attended: bool = False):
+        """qkv GEMM, rotation of q and k in place, k and v scattered to their page slots (reference :251-268,282): the qkv rows, and what `attend`
+        is to rotate q by (None: it is rotated).
+        gathered: hidden_states' columns are in the order of an act-order qkv weight.  attended: all rows' q go to `attend`, which may rotate it."""
         H, Hkv, D = self.num_heads, self.num_key_value_heads, self.head_size
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         lin = self.query_key_value.linear
@@ -195,24 +197,26 @@ class FlashLlamaAttention:
                 and (decode or native.rope_gemm_pays_for_prompts(hidden_states.shape[0], rope_w))):
             # one launch: GEMM + rotary embedding + cache write (native.gptq_gemm_rope / native.dense_gemm_rope)
             fused = native.gptq_gemm_rope if isinstance(rope_w, native.GptqWeight) else native.dense_gemm_rope
-            return fused(hidden_states, rope_w, lin.bias, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D)
+            return fused(hidden_states, rope_w, lin.bias, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D), None
         # [T, (H + 2 Hkv) D]; at decode sizes the split-K sum of the GPTQ GEMM is finished inside the rope kernel; whole prompts on the dense
         # prefill kernel take the finished sum, and with it the page-wise cache writes
         whole = kv.fresh_prefill and isinstance(lin, FastLinear) and lin.tall(hidden_states) >= 0
         qkv = self.query_key_value(hidden_states, partial=not whole, **({"gathered": True} if gathered else {}))
         if kv.fresh_prefill and not isinstance(qkv, native.Partial):
-            return native.rope_kv_write_prefill(qkv, cos, sin, position_ids, cu_seqlens_q, kv.block_tables, k_pool, v_pool,
-                                                kv.max_q_len, H, Hkv, D, D)
-        return native.rope_kv_write(qkv, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D, D)
+            pages = (qkv, cos, sin, position_ids, cu_seqlens_q, kv.block_tables, k_pool, v_pool, kv.max_q_len, H, Hkv, D, D)
+            if attended and qkv.is_cuda and kv.num_splits == 1 and cos.shape[1] * 2 == D and native.attn_rotates_q(H, Hkv, D, kv.max_q_len):
+                return native.rope_kv_write_prefill(*pages, rotate_q=False), (cos, sin, position_ids)
+            return native.rope_kv_write_prefill(*pages), None
+        return native.rope_kv_write(qkv, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D, D), None
 
-    def attend(self, qkv, cu_seqlens_q, layer_id: int, kv: KVArgs):
-        """Attention of the rotated q over the layer's cache pages (reference :271-295): [T, H D]."""
+    def attend(self, qkv, cu_seqlens_q, layer_id: int, kv: KVArgs, rope=None):
+        """Attention of q (rotated, or to be rotated by `rope`) over the layer's cache pages (reference :271-295): [T, H D]."""
         H, Hkv, D = self.num_heads, self.num_key_value_heads, self.head_size
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         T = qkv.shape[0]
         B = kv.block_tables.shape[0]
         # decode: the o_proj GEMM reads its operand in fragment order, an act-order one with its columns in its own
-        places = {}
+        places = {} if rope is None else {"rope": rope}
         if frag_rows(self.o_proj.linear, T, kv, gathers=self.out_places is not None):
             if self.out_places is not None:
                 places = {"out_cols": self.out_places}
@@ -229,8 +233,8 @@ class FlashLlamaAttention:
         return attn_output
 
     def forward(self, hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id: int, kv: KVArgs, gathered: bool = False):
-        qkv = self.project_qkv(hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id, kv, gathered)
-        attn_output = self.attend(qkv, cu_seqlens_q, layer_id, kv)
+        qkv, rope = self.project_qkv(hidden_states, cos, sin, position_ids, cu_seqlens_q, layer_id, kv, gathered, attended=True)
+        attn_output = self.attend(qkv, cu_seqlens_q, layer_id, kv, rope)
         # may be a native.Partial: the following fused add+RMSNorm finishes the split-K sum
         return self.o_proj(attn_output, partial=True)
 
@@ -316,7 +320,7 @@ class FlashLlamaLayer:
         att = self.self_attn
         qkv_perm = getattr(att.query_key_value.linear, "perm", None)
         normed_hidden_states, res = self.input_layernorm(hidden_states, residual, perm=qkv_perm)
-        qkv = att.project_qkv(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv, qkv_perm is not None)
+        qkv, _ = att.project_qkv(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv, qkv_perm is not None)
         step = kv.at_ends(att.num_heads, att.num_key_value_heads)
         attn_output = att.o_proj(att.attend(qkv.index_select(0, kv.ends), step.cu_seqlens_q, self.layer_id, step), partial=True)
         return self.feed_forward(attn_output, res.index_select(0, kv.ends), step)

@@ -82,6 +82,8 @@ SIGNATURES = {
                                             _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tgis_rope_kv_write_prefill": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64,
                                             _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
+    "tgis_rope_k_write_prefill": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64,
+                                            _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tgis_attn_num_splits": (_c_int, [_c_i64, _c_int, _c_int, _c_i64, _c_i64]),
     "tgis_attn_workspace_bytes": (_c_i64, [_c_i64, _c_int, _c_int, _c_int, _c_int]),
     "tgis_dense_rows_ok": (_c_int, [_c_i64, _c_i64, _c_int]),
@@ -92,6 +94,9 @@ SIGNATURES = {
     "tgis_dense_rows_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_attn_paged": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int,
                                  _c_int, _c_i64, _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
+    "tgis_attn_rotates_q": (_c_int, [_c_int, _c_int, _c_int, _c_i64]),
+    "tgis_attn_paged_rope": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int, _c_i64, _c_i64, _c_f,
+                                      _c_int, _vp]),
     "tgis_attn_paged_ordered": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int,
                                          _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
     "tgis_act_mul": (_c_int, [_vp, _vp, _c_i64, _c_i64, _c_int, _c_int, _vp]),
@@ -1017,16 +1022,16 @@ def rope_kv_write(qkv, cos, sin, positions, slots, k_pool, v_pool, H: int, Hkv: 
 
 
 def rope_kv_write_prefill(qkv, cos, sin, positions, cu_seqlens, block_tables, k_pool, v_pool, max_len: int, H: int,
-                          Hkv: int, D: int, rot_dim: int):
-    """rope_kv_write for a fresh prefill (token i of a sequence = cache position i): page-wise cache writes."""
+                          Hkv: int, D: int, rot_dim: int, rotate_q: bool = True):
+    """rope_kv_write for a fresh prefill (token i of a sequence = cache position i): page-wise cache writes.  rotate_q=False leaves q as it came, for
+    attn_paged with `rope`."""
     assert qkv.dim() == 2 and qkv.stride(1) == 1 and block_tables.is_contiguous()
     B = block_tables.shape[0]
-    _check(
-        load_library().tgis_rope_kv_write_prefill(_ptr(qkv), qkv.stride(0), _ptr(cos), _ptr(sin), _ptr(positions),
-                                                  _ptr(cu_seqlens), _ptr(block_tables), block_tables.shape[1],
-                                                  _ptr(k_pool), _ptr(v_pool), B, qkv.shape[0], max_len, H, Hkv, D,
-                                                  rot_dim, dtype_code(qkv.dtype), _stream()),
-        "tgis_rope_kv_write_prefill")
+    lib = load_library()
+    launch = lib.tgis_rope_kv_write_prefill if rotate_q else lib.tgis_rope_k_write_prefill
+    _check(launch(_ptr(qkv), qkv.stride(0), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(cu_seqlens), _ptr(block_tables), block_tables.shape[1],
+                  _ptr(k_pool), _ptr(v_pool), B, qkv.shape[0], max_len, H, Hkv, D, rot_dim, dtype_code(qkv.dtype), _stream()),
+           "tgis_rope_kv_write_prefill")
     return qkv
 
 
@@ -1038,11 +1043,17 @@ def attn_workspace_bytes(total_q: int, H: int, Hkv: int, D: int, num_splits: int
     return load_library().tgis_attn_workspace_bytes(total_q, H, Hkv, D, num_splits)
 
 
+def attn_rotates_q(H: int, Hkv: int, D: int, max_q_len: int) -> bool:
+    """Whether attn_paged of such queries takes `rope`."""
+    return bool(load_library().tgis_attn_rotates_q(H, Hkv, D, max_q_len))
+
+
 def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_q, out, B: int, H: int, Hkv: int,
                D: int, max_q_len: int, max_ctx: int, scale: float, num_splits: int, ws: Optional[Workspace],
-               out_cols: Optional[torch.Tensor] = None):
+               out_cols: Optional[torch.Tensor] = None, rope: Optional[tuple] = None):
     """q is a (view into a) [T, *] activation whose row stride is ld_q elements; out [T, H*D], or (decode, B <= 32) a
-    FragAct of that shape for the o_proj GEMM, with out_cols (int32, a permutation) with its columns at those places."""
+    FragAct of that shape for the o_proj GEMM, with out_cols (int32, a permutation) with its columns at those places.
+    rope (where attn_rotates_q): (cos, sin, positions) of a q that is not rotated yet."""
     assert block_tables.dtype == torch.int32 and ctx_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
     assert block_tables.is_contiguous()
     if isinstance(out, FragAct):
@@ -1052,6 +1063,14 @@ def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_
         assert out.is_contiguous()
         optr, ldo = _ptr(out), H * D
     wptr, wbytes = (ws.ptr, ws.nbytes) if ws is not None else (None, 0)
+    if rope is not None:
+        cos, sin, positions = rope
+        assert out_cols is None and ldo == H * D and num_splits == 1 and cos.shape[1] * 2 == D and cos.dtype == sin.dtype == q.dtype
+        assert positions.dtype == torch.int32 and positions.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
+        _check(load_library().tgis_attn_paged_rope(_ptr(q), ld_q, _ptr(cos), _ptr(sin), _ptr(positions), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
+                                                   block_tables.shape[1], _ptr(ctx_lens), _ptr(cu_seqlens_q), optr, B, H, Hkv, D, max_q_len, max_ctx,
+                                                   float(scale), dtype_code(q.dtype), _stream()), "tgis_attn_paged_rope")
+        return out
     if out_cols is not None:
         assert ldo == LD_FRAGMENTS and out_cols.dtype == torch.int32 and out_cols.is_contiguous() and out_cols.numel() == H * D
         _check(load_library().tgis_attn_paged_ordered(_ptr(q), ld_q, _ptr(k_pool), _ptr(v_pool), _ptr(block_tables), block_tables.shape[1],
