@@ -159,12 +159,17 @@ __host__ __device__ __forceinline__ int64_t xf_off(int64_t m, int64_t k, int64_t
 }
 
 // GELU on an fp32 value (exact erf form, or the tanh approximation): ONE function for tgis_gelu and for the GEMM epilogues
-// that apply it to their rounded output.  Not inlined: inside a caller the compiler contracts the expression (and the
-// library's erf / tanh polynomials) with whatever surrounds it, and the two forms then differ in the last bit.
-__device__ __attribute__((noinline)) inline float gelu_f32(float f, bool tanh_approx) {
-    if (tanh_approx) {
-        float inner = 0.7978845608028654f * (f + 0.044715f * f * f * f);
-        return 0.5f * f * (1.f + tanhf(inner));
-    }
-    return 0.5f * f * (1.f + erff(f * 0.7071067811865476f));
+// that apply it to their rounded output, which leave the same bits.
+// The erf form is not inlined: inside a caller the compiler contracts the expression (and the library's polynomial) with whatever surrounds it, and the two then
+// differ in the last bit.
+__device__ __attribute__((noinline)) inline float gelu_erf_f32(float f) { return 0.5f * f * (1.f + erff(f * 0.7071067811865476f)); }
+// f (1 + tanh u) / 2 = f / (1 + e^-2u), u = sqrt(2 / pi) (f + 0.044715 f^3): an exponential and a reciprocal of the hardware's, in operations that leave nothing
+// to contract.  Against float64 no worse than with the library's tanh, whose 1 + tanh u loses its digits below zero (largest error over the values of bf16 in
+// -8 .. 8, of the value: 4e-6, before the value itself).  us, the library's tanh / this: 8186 x 24576 bf16 through tgis_gelu 178 / 131; at the end of a launch of
+// tiles of 128 x 256 +23 / +5.
+__device__ __forceinline__ float gelu_tanh_f32(float f) {
+    constexpr float K = -2.302208198f;  // -2 sqrt(2 / pi) log2 e
+    const float e = __builtin_amdgcn_exp2f(f * __builtin_fmaf(f * f, 0.044715f * K, K));
+    return f * __builtin_amdgcn_rcpf(1.f + e);
 }
+__device__ __forceinline__ float gelu_f32(float f, bool tanh_approx) { return tanh_approx ? gelu_tanh_f32(f) : gelu_erf_f32(f); }

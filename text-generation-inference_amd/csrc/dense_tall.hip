@@ -363,9 +363,9 @@ constexpr int MAX_PARTS = 384;  // blocks of the split launch: 48 MiB of fp32 ti
 
 // Rows x columns of a tile, and whether the tiles past the last whole round of 256 are split over k: 256 rows of 24576 x 6144 are 48 tiles of 128 x
 // 256 that walk 384 steps each (264 us; 95 split in four), 765 rows of 2048 x 11264 352 tiles of 96 x 128 (44 us; 52 in tiles of 128 x 128).
-// GELU: in the unsplit launch each thread evaluates it 16 BMR TW times, one call behind the other, 0.18 us each; the finish launch has a thread for
-// every four (1024 x 1024 at 65 - 256 rows +5.7 us / +0.9).
-template <bool GELU>
+// GELU: in the unsplit launch each thread evaluates it 16 BMR TW times, one behind the other, GELU_NS each (erf 180, a call; tanh 40): the finish launch has a thread
+// for every four (1024 x 1024 at 65 - 256 rows, tiles of 64 x 128, 128 x 256: erf +6.4, +25 us, tanh +1.3, +5; behind a split +0.9).
+template <int GELU_NS>
 TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
     const int64_t steps = K / 64, NT = cdiv64(N, 32);
     TallPlan best{};
@@ -385,7 +385,7 @@ TallPlan make_plan_tall(int64_t M, int64_t K, int64_t N) {
                 } else {
                     us = launch_us(walk_us(tiles, steps, c), K, N);
                 }
-                if (GELU && (S == 1 || rounds)) us += 0.18 * 16 * BMR * TW;
+                if (GELU_NS && (S == 1 || rounds)) us += GELU_NS * 1e-3 * 16 * BMR * TW;
                 if (us < best_us) {
                     best_us = us;
                     best = {BMR, TW, (int)cb, (int)tiles, (int)(S > 1 ? tiles - rest : tiles), S, (int)per, us};
@@ -449,7 +449,7 @@ TallPlan kept_plan(int64_t M, int64_t K, int64_t N) {
 TallPlan plan_tall(int64_t M, int64_t K, int64_t N, int act) {
     TallPlan p;
     if (plan_from_env(M, K, N, false, p)) return p;
-    return act == 4 || act == 5 ? kept_plan<make_plan_tall<true>>(M, K, N) : kept_plan<make_plan_tall<false>>(M, K, N);
+    return act == 4 ? kept_plan<make_plan_tall<180>>(M, K, N) : act == 5 ? kept_plan<make_plan_tall<40>>(M, K, N) : kept_plan<make_plan_tall<0>>(M, K, N);
 }
 
 TallPlan plan_parts(int64_t M, int64_t K, int64_t N) {
