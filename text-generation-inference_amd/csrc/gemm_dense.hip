@@ -445,9 +445,15 @@ static int launch_groups(const DenseArgs& a, int groups, int tiles, int64_t x_gr
 }
 template <typename T>
 static int launch_groups_rows(const DenseArgs& a, int groups, int tiles, int64_t x_group, int64_t out_group, hipStream_t st) {
-    if (a.M <= 16) return launch_groups<T, 1, true, 4>(a, groups, tiles, x_group, out_group, st);
-    return a.M <= 32 ? launch_groups<T, 1, false, 2>(a, groups, tiles, x_group, out_group, st)
-                     : launch_groups<T, 2, false, 1>(a, groups, tiles, x_group, out_group, st);
+    if (a.M > 32) return launch_groups<T, 2, false, 1>(a, groups, tiles, x_group, out_group, st);
+    // The longest phases of x that leave room for two blocks on a CU: with one, tiles past the 256th are a round of their own (258 tiles of 2048 k, us, phases of
+    // 1024 / 512 k: 21 rows 13.5 / 12.3, 32 14.4 / 13.5; 514 of 4096 34.6 / 32.0, 37.1 / 33.9; of 2048 / 1024 k at 16 rows 32.1 / 29.0)
+    auto fits = [&](bool r16, int q) { return dense::wide_lds_bytes(a.M, a.K, 1, 1, r16, q) <= 80 * 1024; };
+    if (a.M <= 16)
+        return fits(true, 4) ? launch_groups<T, 1, true, 4>(a, groups, tiles, x_group, out_group, st)
+                             : launch_groups<T, 1, true, 2>(a, groups, tiles, x_group, out_group, st);
+    return fits(false, 2) ? launch_groups<T, 1, false, 2>(a, groups, tiles, x_group, out_group, st)
+                          : launch_groups<T, 1, false, 1>(a, groups, tiles, x_group, out_group, st);
 }
 
 extern "C" int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo,
