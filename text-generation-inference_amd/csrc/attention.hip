@@ -533,9 +533,29 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     }
 }
 
-// Decode with fewer than 256 (sequence, kv head) groups: blocks of 8 waves that share one group's keys page by page
-// (and merge through LDS) instead of more key splits merged across blocks.
-static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && groups < 256; }
+// Decode with up to 256 (sequence, kv head) groups: blocks of 8 waves that share one group's keys page by page
+// (and merge through LDS) instead of more key splits merged across blocks.  256 groups, a block for each CU: one block of 8
+// waves against two splits of 4, us, D 128 at ctx 130, 600, 1400, 4096 8.0 / 10.2, 16.1 / 18.4, 30.6 / 32.3, 80.2 / 82.2, sequences of a quarter of that to
+// all of it 6.9 / 9.4, 13.2 / 15.5, 23.7 / 26.8, 61.3 / 62.8; D 64 at 600, 1400 10.4 / 12.8, 17.7 / 20.2.
+static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && groups <= 256; }
+
+// Waves of a decode block of one chunk.  What is resident decides: of D 128 (three waves per SIMD) 256 blocks of 8 waves, 768 of 4, 1536 of 2; of D 64 twice that
+// and more.  us, waves:
+//   257 - 511 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600, 2048:
+//     14.2 / 13.9, 35.9 / 34.7, ragged 12.8 / 11.7, 32.3 / 26.5; at 130 8.0 / 8.3)
+//   769 - 1023 of D 128: 8, since 4 leave a second round (992 at 300, 1024, 3000 4 / 8: 29.7 / 27.7, 85.6 / 79.0, 257.7 / 231.8, ragged 20.6 / 20.3, 55.6 / 52.9, 150.8 /
+//     146.6; 800 76.2 / 69.5, ragged 45.2 / 45.9; 2 waves take 8 - 14 % longer than 4 where 800 sequences are ragged)
+//   1024 - 2047: 2, which halve the page-count imbalance between a block's waves (33 pages over 4 waves = 9/8/8/8; over 2 = 17/16); of D 128 past 1536, a second round
+//     of these, 8 (1600 at 300, 1024, 3000 2 / 8: 47.5 / 43.8, 147 / 133, 430 / 383, ragged 32.2 / 30.6, 92.0 / 86.2, 257 / 249)
+//   from 2048 on 4: past that the dispatch rate, 7 ns per workgroup, costs more than the imbalance
+static int decode_waves(int64_t blocks, int num_splits, int ch, int D, int64_t pages) {
+    if (wide_decode_blocks(blocks / num_splits, ch)) return 8;
+    if (ch == 1 && num_splits == 1) {
+        if (D == 64 && blocks < 512 && pages >= 8) return 8;
+        if (D == 128 && ((blocks > 768 && blocks < 1024) || (blocks > 1536 && blocks < 2048))) return 8;
+    }
+    return blocks >= 1024 && blocks < 2048 ? 2 : 4;
+}
 
 // 16-head chunks one decode block serves (register budget: 3 sets of O accumulators at D = 128)
 static int chunks_per_block(int HC, int64_t max_q_len) {
@@ -615,8 +635,6 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
     const int ch = chunks_per_block(g.HC, max_q_len);
     int64_t base = B * Hkv * cdiv64(g.HC, ch) * q_tiles;
     int64_t pages = cdiv64(std::max<int64_t>(max_ctx, 1), 32);
-    // single-chunk blocks, many groups: ~512 blocks fill 256 CUs twice; more, thinner blocks lose to the dispatch ramp
-    // and the merge
     int64_t ns;
     if (wide_decode_blocks(base, ch)) {
         // few (sequence, kv head) groups: 8-wave blocks, one round of <= 256 of them, >= 2 pages per wave
@@ -645,8 +663,11 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
         // 6 (23.9 vs 24.2, profiles/r06_mqa_variants.log)
         ns = std::min<int64_t>(cdiv64(256, base), pages / 16);
     } else {
-        ns = cdiv64(512, base);
-        ns = std::min<int64_t>(ns, cdiv64(pages, 4));  // at least one page per wave
+        // single-chunk blocks, many groups: two splits only where the second half of the chip's waves gives more than the merge takes: up to 384 groups (768 blocks of
+        // 4 waves are resident at D 128) from 48 pages on.  us, 1 / 2 splits: 352 groups of D 128 at ctx 600, 1024, 1400 21.2 / 23.2, 32.5 / 33.5, 42.3 / 42.8, ragged 16.6 /
+        // 18.3, 25.3 / 25.2, 32.0 / 32.8, but at 2048, 4096 61.0 / 59.2, 117.6 / 113.1, ragged 44.8 / 44.3, 84.6 / 81.6; 320 at 1400, 2048 41.5 / 41.5, 59.0 / 56.3; 448 at 1024, 3000 36.6 /
+        // 45.4, 103.8 / 127.4, ragged 30.2 / 34.0, 80.1 / 82.1; D 64, 448 at 600, 2048 14.9 / 18.4, 37.8 / 42.4
+        ns = base <= 384 && pages >= 48 ? 2 : 1;
     }
     ns = std::max<int64_t>(1, std::min<int64_t>(ns, 64));
     return (int)ns;
@@ -800,7 +821,6 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
                    "tgis_attn_paged: out is [tokens, H * D] contiguous (ld_out = 0 or H * D), or — decode, <= 64 sequences — in "
                    "fragment order (ld_out = TGIS_LD_FRAGMENTS)");
     TGIS_CHECK_ARG(!out_cols || ld_out == TGIS_LD_FRAGMENTS, "tgis_attn_paged: columns are re-ordered in fragment order only");
-    (void)max_ctx;
     if (B == 0) return TGIS_OK;
     hipStream_t st = (hipStream_t)stream;
     AttnGeom g = attn_geom(H, Hkv);
@@ -859,12 +879,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
         static const bool xcd_off = getenv("TGIS_ATTN_XCD") && atoi(getenv("TGIS_ATTN_XCD")) == 0;  // A/B hook
         a.xcd_remap = (!xcd_off && max_q_len == 1 && q_tiles == 1 && a.HCB > 1 && (B * num_splits * Hkv) % 8 == 0) ? 1 : 0;
     }
-    // waves per block: with >= 1024 (sequence, kv head) blocks the chip is full either way and 2-wave blocks halve
-    // the page-count imbalance between a block's waves (33 pages over 4 waves = 9/8/8/8; over 2 = 17/16)
-    const int64_t nblocks = (int64_t)grid.x * grid.y * grid.z;
-    // (past ~2k blocks the dispatch rate, 7 ns per workgroup, costs more than the imbalance)
-    int nw = (max_q_len == 1 && nblocks >= 1024 && nblocks < 2048) ? 2 : 4;
-    if (max_q_len == 1 && wide_decode_blocks(nblocks / num_splits, ch)) nw = 8;
+    int nw = max_q_len == 1 ? decode_waves((int64_t)grid.x * grid.y * grid.z, num_splits, ch, D, cdiv64(max_ctx, 32)) : 4;
     if (const char* e = getenv("TGIS_ATTN_NW")) {
         const int v = atoi(e);
         nw = (v == 1 || v == 2 || v == 3 || v == 8) ? v : 4;
