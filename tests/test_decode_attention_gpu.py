@@ -21,7 +21,7 @@ def test_splits(B, Hkv, ctx, splits):
 # and D 64 2
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Hkv,G,D,longest", [
-    (128, 2, 1, 128, 300), (257, 1, 2, 128, 300), (96, 4, 1, 128, 1505), (97, 4, 1, 128, 1505), (511, 1, 1, 64, 225), (511, 1, 1, 64, 224), (128, 3, 4, 64, 1504),
+    (128, 2, 1, 128, 300), (257, 1, 2, 128, 300), (96, 4, 1, 128, 1505), (97, 4, 1, 128, 1505), (511, 1, 1, 64, 225), (512, 1, 1, 64, 225), (513, 1, 1, 64, 225), (511, 1, 1, 64, 224), (128, 3, 4, 64, 1504),
     (128, 3, 4, 64, 1505), (769, 1, 1, 128, 130), (1023, 1, 1, 128, 130), (1024, 1, 1, 128, 130), (1537, 1, 1, 128, 70), (1537, 1, 1, 64, 70), (2047, 1, 1, 128, 33),
 ])
 def test_groups(gpu_device, B, Hkv, G, D, longest):

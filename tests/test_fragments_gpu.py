@@ -83,6 +83,29 @@ def test_fragment_gemm_matches_the_oracle_and_the_row_major_launch(nat, gpu_devi
     assert float(dd.max()) <= 2.0 ** -9 * float(want.abs().max()) + 1e-3
 
 
+@pytest.mark.parametrize("plan", ["1,1", "2,3", "3,1", "4,2"])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 49])
+def test_fragment_gemm_row_blocks(nat, gpu_device, monkeypatch, M, plan):
+    """Both sides of each count of 16-row blocks (one and three take another instruction than two and four), at every width of a wave's column group, on eleven tiles
+    and eleven k64-steps, with and without the SiLU epilogue; rows past M hold NaN."""
+    K, N, gs = 704, 352, 64
+    monkeypatch.setenv("TGIS_GPTQ_WIDE_PLAN", plan)
+    g = torch.Generator().manual_seed(M)
+    x = (torch.randn(M, K, generator=g) * 0.5).half()
+    for act in (0, 2):
+        (qw, qz, sc, gi), w = _weight(nat, gpu_device, K, N, gs, seed=M + act, gate_up=act == 2)
+        ws = nat.Workspace(w.workspace_bytes(M), gpu_device)
+        xf = nat.FragAct.from_rows(x.to(gpu_device))
+        if M % 32:
+            xf.buf.view((M + 31) // 32, -1, 2, 32, 8)[-1][:, :, M % 32:].fill_(float("nan"))
+        want = ops_ref.gptq_linear(x, qw, qz, sc, gi, gs, None)
+        if act == 2:
+            want = ops_ref.silu_mul(want.half().view(M, N), N // 2).float()
+        got = nat.gptq_gemm(xf, w, ws, act=act).float().cpu()
+        err = (got - want).abs()  # the tolerances of the tests around this one
+        assert bool((err <= 2e-3 * want.abs() + 2e-3 * float(want.abs().mean()) + 1e-4).all()) if act == 0 else float(err.max()) <= 6e-3 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("order", [(16, 48), (48, 16)])
 def test_deferred_reduce_plan_follows_the_row_class(nat, gpu_device, order):
     """One GptqWeight serving a <= 32-row and then a 33 - 64-row decode batch (continuous batching: concatenate / prune move a

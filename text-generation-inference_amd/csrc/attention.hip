@@ -539,10 +539,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
 // all of it 6.9 / 9.4, 13.2 / 15.5, 23.7 / 26.8, 61.3 / 62.8; D 64 at 600, 1400 10.4 / 12.8, 17.7 / 20.2.
 static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && groups <= 256; }
 
-// Waves of a decode block of one chunk.  What is resident decides: of D 128 (three waves per SIMD) 256 blocks of 8 waves, 768 of 4, 1536 of 2; of D 64 twice that
-// and more.  us, waves:
-//   257 - 511 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600, 2048:
-//     14.2 / 13.9, 35.9 / 34.7, ragged 12.8 / 11.7, 32.3 / 26.5; at 130 8.0 / 8.3)
+// Waves of a decode block of one chunk.  What is resident decides: of D 128 768 blocks of 4 waves, 1536 of 2 (three waves per SIMD), 512 of 8 (four: their bound on
+// registers), of D 64 more.  (Four waves per SIMD for the smaller blocks as well: equal sequences 7 - 10 % faster at 992 groups, but ragged ones 3 - 7 % slower and
+// 1 - 2 % at 1024, since blocks that wait for a place level what is ragged.  16 waves: 0 - 2 us slower on up to 256 groups.)  us, waves:
+//   257 - 512 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600, 2048:
+//     14.2 / 13.9, 35.9 / 34.7, ragged 12.8 / 11.7, 32.3 / 26.5; 512 at 700, 4000 17.8 / 18.1, 78.9 / 80.4, ragged 15.2 / 14.3, 63.6 / 55.9; 384 at 130 8.0 / 8.3)
 //   769 - 1023 of D 128: 8, since 4 leave a second round (992 at 300, 1024, 3000 4 / 8: 29.7 / 27.7, 85.6 / 79.0, 257.7 / 231.8, ragged 20.6 / 20.3, 55.6 / 52.9, 150.8 /
 //     146.6; 800 76.2 / 69.5, ragged 45.2 / 45.9; 2 waves take 8 - 14 % longer than 4 where 800 sequences are ragged)
 //   1024 - 2047: 2, which halve the page-count imbalance between a block's waves (33 pages over 4 waves = 9/8/8/8; over 2 = 17/16); of D 128 past 1536, a second round
@@ -551,7 +552,7 @@ static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && group
 static int decode_waves(int64_t blocks, int num_splits, int ch, int D, int64_t pages) {
     if (wide_decode_blocks(blocks / num_splits, ch)) return 8;
     if (ch == 1 && num_splits == 1) {
-        if (D == 64 && blocks < 512 && pages >= 8) return 8;
+        if (D == 64 && blocks <= 512 && pages >= 8) return 8;
         if (D == 128 && ((blocks > 768 && blocks < 1024) || (blocks > 1536 && blocks < 2048))) return 8;
     }
     return blocks >= 1024 && blocks < 2048 ? 2 : 4;

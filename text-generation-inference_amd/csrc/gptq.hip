@@ -105,12 +105,12 @@ __global__ __launch_bounds__(64 * TN * WK) void gptq_gemm_kernel(GemmArgs a) {
     gptq::gptq_gemm_unit<TN, WK, ACT, GROUP64, PERM, MR>(a, blockIdx.x, blockIdx.y, blockIdx.z, smem);
 }
 
-// Decode batches of up to 32 rows whose activation is in fragment order (gptq_wide_body.h).  8 waves; CT = 4 holds 2 waves
+// Decode batches of up to 64 rows whose activation is in fragment order (gptq_wide_body.h).  8 waves; CT = 4 holds 2 waves
 // per SIMD (one block per CU), CT = 2 / 3 leave room for more.
-template <int CT, int ACT, bool OUTF, int MR>
+template <int CT, int ACT, bool OUTF, int RB>
 __global__ __launch_bounds__(64 * gptq::WIDE_WK) void gptq_wide_kernel(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gptq::gptq_wide_unit<CT, ACT, OUTF, MR>(a, smem);
+    gptq::gptq_wide_unit<CT, ACT, OUTF, RB>(a, smem);
 }
 
 // Sum the S split-K slabs in fixed order (deterministic) and emit f16 (+bias): thread = (row, 4 columns).
@@ -374,21 +374,23 @@ struct RopeEpi {
     int H, Hkv, D;
 };
 
-template <int CT, int ACT, bool OUTF, int MR>
-static int launch_wide_mr(dim3 grid, hipStream_t st, const GemmArgs& a) {
-    const size_t lds = gptq::wide_lds_bytes(CT);
+template <int CT, int ACT, bool OUTF, int RB>
+static int launch_wide_rows(dim3 grid, hipStream_t st, const GemmArgs& a) {
+    const size_t lds = gptq::wide_lds_bytes(CT, RB);
     static bool attr_done = false;
     if (!attr_done) {
-        TGIS_CHECK_HIP(hipFuncSetAttribute((const void*)gptq_wide_kernel<CT, ACT, OUTF, MR>,
+        TGIS_CHECK_HIP(hipFuncSetAttribute((const void*)gptq_wide_kernel<CT, ACT, OUTF, RB>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         attr_done = true;
     }
-    hipLaunchKernelGGL((gptq_wide_kernel<CT, ACT, OUTF, MR>), grid, dim3(64 * gptq::WIDE_WK), lds, st, a);
+    hipLaunchKernelGGL((gptq_wide_kernel<CT, ACT, OUTF, RB>), grid, dim3(64 * gptq::WIDE_WK), lds, st, a);
     return TGIS_OK;
 }
 template <int CT, int ACT, bool OUTF>
 static int launch_wide_one(dim3 grid, hipStream_t st, const GemmArgs& a) {
-    return a.M > 32 ? launch_wide_mr<CT, ACT, OUTF, 2>(grid, st, a) : launch_wide_mr<CT, ACT, OUTF, 1>(grid, st, a);
+    if (a.M <= 16) return launch_wide_rows<CT, ACT, OUTF, 1>(grid, st, a);
+    if (a.M <= 32) return launch_wide_rows<CT, ACT, OUTF, 2>(grid, st, a);
+    return a.M <= 48 ? launch_wide_rows<CT, ACT, OUTF, 3>(grid, st, a) : launch_wide_rows<CT, ACT, OUTF, 4>(grid, st, a);
 }
 
 static int launch_gptq(const void* x, int64_t ldx, const void* prepared, const void* bias, const int32_t* perm,

@@ -30,7 +30,7 @@ namespace gptq {
 constexpr int WIDE_WK = 8;      // k-parts (waves) per block
 constexpr int WIDE_DEPTH = 2;   // k64-steps in flight per wave
 constexpr int WIDE_TG(int ct) { return ct < 4 ? ct : 4; }   // tiles per round of the k-part exchange
-static inline size_t wide_lds_bytes(int ct) { return (size_t)WIDE_WK * WIDE_TG(ct) * 4096; }
+static inline size_t wide_lds_bytes(int ct, int rb) { return (size_t)WIDE_WK * WIDE_TG(ct) * (rb == 1 ? 2048 : 4096); }
 
 struct WidePlan {
     int CT, S;  // column tiles per wave (= per block), global k splits
@@ -95,12 +95,25 @@ static inline int wide_max_splits(int64_t K, int64_t N) {
                     std::max(plan_wide(K, N, 0, 32, true).S, plan_wide(K, N, 0, 64, true).S));
 }
 
+// rows 1, 3 of 16 lanes of x against rows 0, 2 of y
+__device__ __forceinline__ void swap_rows(uint32_t x, uint32_t y, uint32_t (&out)[2]) {
+    const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    out[0] = p[0];
+    out[1] = p[1];
+}
+
 // OUTF: the act = 2 output (the operand of the down projection) leaves in fragment order as well.
-// MR = 32-row blocks of the activation (1: M <= 32; 2: M <= 64 — every dequantised B fragment then feeds two MFMAs, the
-// "two tiles per wave on one activation" of the 64-row passes, with the activation in registers instead of LDS).
-template <int CT, int ACT, bool OUTF, int MR>
+// RB = 16-row blocks of the activation; every dequantised B fragment feeds them all.  Two and four are one and two operands of the 32x32x16 instruction.
+// One and three take 16x16x32: half of x and of the matrix work up to 16 rows, three quarters at 33 - 48, for a row swap of the weights per two words.
+// us, 32x32x16 / 16x16x32 (qkv + rotary, o, gate | up, down): 4096, 11008 at 16 rows 12.4 / 10.9, 5.4 / 4.9, 15.5 / 13.2, 8.8 / 8.1; at 48 17.7 / 16.5, 7.1 / 7.4, 19.6 / 18.6,
+// 12.3 / 11.5; 8192, 28672 at 16 17.9 / 14.8, 11.2 / 10.7, 59.6 / 52.7, 33.6 / 25.9; at 48 26.4 / 23.5, 15.3 / 14.3, 77.9 / 74.6, 38.2 / 35.8.  At an even count there is
+// nothing to leave out and the swaps cost 3 - 14 % (gate | up at 32 rows 15.9 / 17.2, 64 20.6 / 23.1).  More k64-steps in flight, with the registers that sixteen rows
+// leave, are slower (three, four: gate | up 13.7 / 14.4 / 14.6, 61.0 for 55.6).
+template <int CT, int ACT, bool OUTF, int RB>
 __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char* smem) {
-    constexpr int WK = WIDE_WK, DEPTH = WIDE_DEPTH, NR = 16 / WK;
+    constexpr bool R16 = RB & 1;
+    constexpr int WK = WIDE_WK, DEPTH = WIDE_DEPTH, MR = (RB + 1) / 2, NR = RB == 1 ? 1 : 2;
+    constexpr int XB = R16 ? RB : MR, XN = R16 ? 2 : 4;  // row blocks of the instruction, fragments of a k64-step in each
     {   // every cache line of the argument block is requested at entry: one scalar round trip instead of three dependent
         // ones before the first weight request (tools/floor/wide.hip `pre`: 0.1 - 0.25 us per launch)
         const int64_t l0 = a.ldo;
@@ -119,7 +132,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
     // the younger half and deeper weight rings: the block finishes when its CU has moved its bytes, however they are dealt;
     // tools/floor/wide.hip `kb` / `pb` / `prio` / `DW`, profiles/r05_wide_kbias*.log, r05_wide_plans.log.)
     const int s0 = sb + (len * wk) / WK, s1 = sb + (len * (wk + 1)) / WK;
-    const int mrows = a.M;  // 1 .. 32 MR
+    const int mrows = a.M;  // 1 .. 16 RB
 
     const char* wt[CT];
     const char* st[CT];
@@ -130,13 +143,14 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
         st[t] = reinterpret_cast<const char*>(a.prep + a.offB) + (int64_t)nt * a.G * 128;
     }
     const uint32_t woff = lane * 16, szoff = (lane & 31) * 4;
+    const uint32_t xoff = R16 ? ((lane >> 4) & 1) * 1024 + ((lane & 32) + (lane & 15)) * 16 : woff;
     const int sclamp = max(s1 - 1, s0);  // loads past the wave's steps re-read its last one (a cache hit), never consumed
     const char* xb = reinterpret_cast<const char*>(a.x);
     const int64_t xblk = (int64_t)a.K * 64;  // bytes between the 32-row blocks of the activation
 
     u32x4 wq[DEPTH][CT];
     uint32_t sz[DEPTH][CT];
-    f16x8 xa[DEPTH][MR][4];
+    f16x8 xa[DEPTH][XB][XN];
     auto load_step = [&](int d, int step) {
         const int sc = min(step, sclamp);
         const int g = min(sc >> a.spg_shift, a.G - 1);
@@ -153,16 +167,17 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
             wq[d][t] = __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(p + woff));
         }
 #pragma unroll
-        for (int mr = 0; mr < MR; ++mr) {
-            const char* p = xb + mr * xblk + (int64_t)sc * 4096;  // fragment order: four contiguous KiB per k64-step
+        for (int b = 0; b < XB; ++b) {
+            const char* p = xb + (R16 ? b >> 1 : b) * xblk + (int64_t)sc * 4096;  // fragment order: four contiguous KiB per k64-step and 32 rows
             PIN_SGPR(p);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) xa[d][mr][i] = *(const GLOBAL_AS f16x8*)(p + woff + i * 1024);
+            for (int i = 0; i < XN; ++i) xa[d][b][i] = *(const GLOBAL_AS f16x8*)(p + xoff + (R16 ? (b & 1) * 256 : 0) + i * (4096 / XN));
         }
     };
 
-    // the rows this wave finishes: accumulator registers [wk NR, (wk + 1) NR) of every tile and row block
+    // the rows this wave finishes: accumulator registers [wk NR, (wk + 1) NR) of every tile and row block; two rows of each block of sixteen
     auto row_of = [&](int mr, int j) {
+        if (R16) return mr * 32 + j * 16 + 2 * wk + (lane >> 5);
         const int r = wk * NR + j;
         return mr * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
     };
@@ -182,11 +197,15 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
     uint32_t EXr = 0x64006400u, M0r = 0x000F000Fu, M1r = 0x00F000F0u;
     asm volatile("" : "+v"(EXr));
     asm volatile("" : "+s"(M0r), "+s"(M1r));
-    f32x16 acc[MR][CT];
+    using Acc = std::conditional_t<R16, f32x4, f32x16>;
+    constexpr int CH = R16 ? 2 : 1;  // parts of a tile's columns: 0 - 15 and 16 - 31
+    Acc acc[XB][CT][CH];
 #pragma unroll
-    for (int mr = 0; mr < MR; ++mr)
+    for (int b = 0; b < XB; ++b)
 #pragma unroll
-        for (int t = 0; t < CT; ++t) acc[mr][t] = f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int h = 0; h < CH; ++h) acc[b][t][h] = Acc{0};
 
     WIDE_STAMP(0);
 #pragma unroll
@@ -196,15 +215,29 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
     auto consume = [&](int d) {
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
-            const f16x2 szh = __builtin_bit_cast(f16x2, sz[d][t]);
-            const f16 zc1 = szh[1];
-            const f16 zd1 = (f16)960.f - zc1;  // -(64 + z + 1), exact
-            const f16x2 zc = {zc1, zc1}, zd = {zd1, zd1}, sc = {szh[0], szh[0]};
+            // 16x16x32: word i of a lane is a column's k chunk 4 (lane / 32) + i; with rows of lanes swapped between words 2 i and 2 i + 1 it is, of columns c and
+            // 16 + c each, chunk 4 (lane / 32) + 2 i + (lane / 16 & 1): the operand against x read the same way
+            uint32_t z[CH] = {sz[d][t]};
+            if constexpr (R16) swap_rows(sz[d][t], sz[d][t], z);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const f16x8 b = dequant8(wq[d][t][i], zc, zd, sc, EXr, M0r, M1r);
+            for (int i = 0; i < XN; ++i) {
+                uint32_t q[CH] = {wq[d][t][i]};
+                if constexpr (R16) swap_rows(wq[d][t][2 * i], wq[d][t][2 * i + 1], q);
 #pragma unroll
-                for (int mr = 0; mr < MR; ++mr) acc[mr][t] = mfma32(xa[d][mr][i], b, acc[mr][t]);
+                for (int h = 0; h < CH; ++h) {
+                    const f16x2 szh = __builtin_bit_cast(f16x2, z[h]);
+                    const f16 zc1 = szh[1];
+                    const f16 zd1 = (f16)960.f - zc1;  // -(64 + z + 1), exact
+                    const f16x2 zc = {zc1, zc1}, zd = {zd1, zd1}, sc = {szh[0], szh[0]};
+                    const f16x8 w = dequant8(q[h], zc, zd, sc, EXr, M0r, M1r);
+#pragma unroll
+                    for (int b = 0; b < XB; ++b) {
+                        if constexpr (R16)
+                            acc[b][t][h] = mfma16(xa[d][b][i], w, acc[b][t][h]);
+                        else
+                            acc[b][t][h] = mfma32(xa[d][b][i], w, acc[b][t][h]);
+                    }
+                }
             }
         }
     };
@@ -261,22 +294,44 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
         // ds_write_b64 and the two registers a wave finishes come back as one ds_read_b64 per k-part and tile: the exchange
         // moves 2 x 8 waves x CT x 4 KiB through an LDS that takes 64 B/clk of 4-byte stores and gives 128 B/clk of 4-byte
         // loads, ~2.3 k clocks at CT 3; 8-byte accesses take 85 and 256 B/clk.  Same values, same order of the sum.)
-        static_assert(NR == 2, "the pair layout is for eight k-parts");
-#pragma unroll
-        for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
-            f32x2* dst = reinterpret_cast<f32x2*>(red + ((wk * TG + (t - tg0)) << 10)) + lane;
-#pragma unroll
-            for (int rp = 0; rp < 8; ++rp) dst[rp << 6] = f32x2{acc[mr][t][2 * rp], acc[mr][t][2 * rp + 1]};
-        }
-        __syncthreads();
+        // Blocks of sixteen rows: [k-part][tile][block][column half][lane][4 rows], a lane's four sums in one store; a wave finishes a value per lane and block.
+        static_assert(WK == 8, "the layouts are for eight k-parts");
         float fin[CT][NR];
+        if constexpr (R16) {
 #pragma unroll
-        for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
+            for (int t = tg0; t < tg0 + TG && t < CT; ++t)
 #pragma unroll
-            for (int k2 = 0; k2 < WK; ++k2) {
-                const f32x2 v = (reinterpret_cast<const f32x2*>(red + ((k2 * TG + (t - tg0)) << 10)) + (wk << 6))[lane];
+                for (int j = 0; j < NR && mr * 2 + j < RB; ++j)
 #pragma unroll
-                for (int j = 0; j < NR; ++j) fin[t][j] = k2 == 0 ? v[j] : fin[t][j] + v[j];
+                    for (int h = 0; h < 2; ++h)
+                        *reinterpret_cast<f32x4*>(red + ((wk * TG + (t - tg0)) * NR + j) * 512 + h * 256 + lane * 4) = acc[mr * 2 + j][t][h];
+            __syncthreads();
+            const float* src = red + ((lane >> 4) & 1) * 256 + ((wk >> 1) * 16 + (lane & 15)) * 4 + (wk & 1) * 2 + (lane >> 5);
+#pragma unroll
+            for (int t = tg0; t < tg0 + TG && t < CT; ++t)
+#pragma unroll
+                for (int j = 0; j < NR && mr * 2 + j < RB; ++j)
+#pragma unroll
+                    for (int k2 = 0; k2 < WK; ++k2) {
+                        const float v = src[((k2 * TG + (t - tg0)) * NR + j) * 512];
+                        fin[t][j] = k2 == 0 ? v : fin[t][j] + v;
+                    }
+        } else {
+#pragma unroll
+            for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
+                f32x2* dst = reinterpret_cast<f32x2*>(red + ((wk * TG + (t - tg0)) << 10)) + lane;
+#pragma unroll
+                for (int rp = 0; rp < 8; ++rp) dst[rp << 6] = f32x2{acc[mr][t][0][2 * rp], acc[mr][t][0][2 * rp + 1]};
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
+#pragma unroll
+                for (int k2 = 0; k2 < WK; ++k2) {
+                    const f32x2 v = (reinterpret_cast<const f32x2*>(red + ((k2 * TG + (t - tg0)) << 10)) + (wk << 6))[lane];
+#pragma unroll
+                    for (int j = 0; j < NR; ++j) fin[t][j] = k2 == 0 ? v[j] : fin[t][j] + v[j];
+                }
             }
         }
 #pragma unroll
@@ -292,7 +347,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
                 const int col = head * a.rD + d;
                 const float bv = a.bias ? (float)a.bias[col] : 0.f;
 #pragma unroll
-                for (int j = 0; j < NR; ++j) {
+                for (int j = 0; j < NR && mr * 2 + j < RB; ++j) {
                     const int m = row_of(mr, j);
                     const float mine = (float)(f16)(fin[t][j] + bv);
                     float o = mine;
@@ -324,7 +379,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
                 const int nsrc = (c < 16) ? j2 : half + j2;
                 const float bv = (a.bias && j2 < half) ? (float)a.bias[nsrc] : 0.f;
 #pragma unroll
-                for (int j = 0; j < NR; ++j) {
+                for (int j = 0; j < NR && mr * 2 + j < RB; ++j) {
                     const float mine = (float)(f16)(fin[t][j] + bv);
                     const float other = __shfl_xor(mine, 16, 64);
                     const int m = row_of(mr, j);
@@ -343,7 +398,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
                 const float bv = (a.bias && n < a.N) ? (float)a.bias[n] : 0.f;
                 if (n < a.N) {
 #pragma unroll
-                    for (int j = 0; j < NR; ++j) {
+                    for (int j = 0; j < NR && mr * 2 + j < RB; ++j) {
                         const int m = row_of(mr, j);
                         if (m < mrows) a.out[(int64_t)m * a.ldo + n] = (f16)(fin[t][j] + bv);
                     }
@@ -352,7 +407,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
                 // slabs in 32-row units: [row block][split][32][ld]
                 float* sl = a.slabs + ((int64_t)(mr * a.S + split) * 32) * (a.NT * 32) + n;
 #pragma unroll
-                for (int j = 0; j < NR; ++j) sl[(int64_t)(row_of(mr, j) & 31) * (a.NT * 32)] = fin[t][j];
+                for (int j = 0; j < NR && mr * 2 + j < RB; ++j) sl[(int64_t)(row_of(mr, j) & 31) * (a.NT * 32)] = fin[t][j];
             }
         }
       }

@@ -28,7 +28,7 @@ static __device__ long long* g_wide_trace = nullptr;   // [blocks][8 waves][8]
 template <int CT, int ACT, bool OUTF, int MR>
 __global__ __launch_bounds__(64 * gptq::WIDE_WK) void unit_kernel(gptq::GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gptq::gptq_wide_unit<CT, ACT, OUTF, MR>(a, smem);
+    gptq::gptq_wide_unit<CT, ACT, OUTF, 2 * MR>(a, smem);
 }
 
 static uint64_t rng_state = 0x1234567ull;
@@ -67,7 +67,7 @@ static void run(const char* name, int K, int N, int S, int M) {
     a.G = im.G; a.gs = 128; a.S = S; a.NT = im.NT; a.KS = im.KS; a.slabs = dslabs; a.partial = S > 1;
     a.spg_shift = 1;
     const int cgs = (im.NT + CT - 1) / CT;
-    const size_t lds = gptq::wide_lds_bytes(CT);
+    const size_t lds = gptq::wide_lds_bytes(CT, 2 * MR);
     auto kern = unit_kernel<CT, ACT, false, MR>;
     CK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     dim3 grid(cgs, S);
