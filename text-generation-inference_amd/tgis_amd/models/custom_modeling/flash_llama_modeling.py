@@ -114,11 +114,10 @@ class KVArgs:
 # measured slower than the launches they replace: experiments/README.md is their ledger.)
 
 
-def frag_rows(linear, rows: int, kv: "KVArgs", act: int = 0, gathers: bool = False) -> bool:
-    """Decode step of <= 64 rows in front of an int4 linear that takes its operand in fragment order (native.FragAct); gathers: the
+def frag_rows(linear, rows: int, act: int = 0, gathers: bool = False) -> bool:
+    """Up to 64 rows in front of an int4 linear that takes its operand in fragment order (native.FragAct); gathers: the
     producer can write an act-order matrix's column order."""
-    return (kv.max_q_len == 1 and not kv.fresh_prefill and rows <= 64 and hasattr(linear, "wants_fragments")
-            and linear.wants_fragments(rows, act, gathers))
+    return rows <= 64 and hasattr(linear, "wants_fragments") and linear.wants_fragments(rows, act, gathers)
 
 
 class LlamaRMSNorm:
@@ -217,7 +216,8 @@ class FlashLlamaAttention:
         B = kv.block_tables.shape[0]
         # decode: the o_proj GEMM reads its operand in fragment order, an act-order one with its columns in its own
         places = {} if rope is None else {"rope": rope}
-        if frag_rows(self.o_proj.linear, T, kv, gathers=self.out_places is not None):
+        decode = kv.max_q_len == 1 and not kv.fresh_prefill
+        if decode and frag_rows(self.o_proj.linear, T, gathers=self.out_places is not None):
             if self.out_places is not None:
                 places = {"out_cols": self.out_places}
             attn_output = native.FragAct.empty(T, H * D, qkv.device)
@@ -272,7 +272,7 @@ class LlamaMLP:
     def forward(self, hidden_states, gathered: bool = False):
         kw = {"gathered": True} if gathered else {}
         if self.fused_epilogue:
-            if isinstance(hidden_states, native.FragAct):  # decode: SiLU * up leaves in the layout down_proj reads
+            if isinstance(hidden_states, native.FragAct):  # SiLU * up leaves in the layout down_proj reads
                 rows = hidden_states.shape[0]
                 act = self.gate_up_proj(hidden_states, out_frag=self.down_proj.linear.wants_fragments(rows))
                 return self.down_proj(act, partial=True)
@@ -295,14 +295,22 @@ class FlashLlamaLayer:
         self.post_attention_layernorm = LlamaRMSNorm(prefix=f"{prefix}.post_attention_layernorm", weights=weights,
                                                      eps=config.rms_norm_eps)
 
+    def hands_fragments(self, rows: int, kv: KVArgs) -> bool:
+        """Whether the norms may hand the int4 GEMMs of up to 64 rows their operands in fragment order (native.FragAct): decode steps, and prompts but
+        for those whose row-major fused qkv launch pays.  us, rows / fragments: a 7B model's prompts of 40 rows 3000 / 2660, two of 32 3223 / 2866, 60 in
+        act order 3130 / 2822, four 70B layers' of 12, 48 868 / 801, 1069 / 1001; but a 7B model's of 16, 30 rows, the host's time either way, 2647 / 2668,
+        2652 / 2692."""
+        return ((kv.max_q_len == 1 and not kv.fresh_prefill)
+                or not native.rope_gemm_pays_for_prompts(rows, getattr(self.self_attn.query_key_value.linear, "rope_handle", None)))
+
     def forward(self, hidden_states, residual, cos, sin, position_ids, cu_seqlens_q, kv: KVArgs):
         rows = hidden_states.shape[0]
         att = self.self_attn
-        # decode steps of <= 64 rows hand the int4 GEMMs their operands in fragment order (native.FragAct): the qkv + rotary
-        # launch when it serves the step, the MLP when the SiLU * up epilogue does; the norms gather for act-order weights
+        # the qkv + rotary launch takes its operand in fragment order when it serves the rows, the MLP when the SiLU * up epilogue does; the norms
+        # gather for act-order weights
         qkv_perm = getattr(att.query_key_value.linear, "perm", None)
-        qkv_frag = (kv.slots is not None and cos.shape[1] * 2 == att.head_size
-                    and frag_rows(att.query_key_value.linear, rows, kv, act=3, gathers=True))
+        qkv_frag = (kv.slots is not None and cos.shape[1] * 2 == att.head_size and self.hands_fragments(rows, kv)
+                    and frag_rows(att.query_key_value.linear, rows, act=3, gathers=True))
         normed_hidden_states, res = self.input_layernorm(hidden_states, residual, frag=qkv_frag, perm=qkv_perm)
         attn_output = att(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv, qkv_perm is not None)
         return self.feed_forward(attn_output, res, kv)
@@ -310,7 +318,8 @@ class FlashLlamaLayer:
     def feed_forward(self, attn_output, res, kv: KVArgs):
         rows = attn_output.shape[0]
         mlp_perm = getattr(self.mlp.gate_up_proj.linear, "perm", None)
-        mlp_frag = self.mlp.fused_epilogue and frag_rows(self.mlp.gate_up_proj.linear, rows, kv, act=2, gathers=True)
+        mlp_frag = (self.mlp.fused_epilogue and self.hands_fragments(rows, kv)
+                    and frag_rows(self.mlp.gate_up_proj.linear, rows, act=2, gathers=True))
         normed_attn_res_output, attn_res = self.post_attention_layernorm(attn_output, res, frag=mlp_frag, perm=mlp_perm)
         mlp_output = self.mlp(normed_attn_res_output, mlp_perm is not None)
         return mlp_output, attn_res
