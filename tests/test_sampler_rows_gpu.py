@@ -48,3 +48,19 @@ def test_top_p_removes_all_that_fits_the_cut(gpu_device, V, top_p):
         assert removed <= cut + slack
         if low < x[b].max():
             assert removed + p[b][x[b] == low].sum() > cut - slack
+
+
+@pytest.mark.parametrize("V", [255, 1025, 32768])
+@pytest.mark.parametrize("k", [1, 4, 50, 254, 256, 257])
+def test_top_p_behind_top_k(gpu_device, V, k):
+    """One launch for both removes, to the bit, what a top-k and a top-p of its scores remove: rows with ties past the list and past a thread's four places among them."""
+    from tgis_amd import native
+
+    x = torch.cat([_rows(V, V + k), torch.randn(1, V, generator=torch.Generator().manual_seed(k))]).to(gpu_device)
+    top_k, cut = torch.full((4,), k, dtype=torch.int32, device=gpu_device), torch.full((4,), 0.1, device=gpu_device)
+    first = native.warp_sample(x, top_k=top_k)[3]
+    ids, logprob, lse, want = native.warp_sample(first.clone(), top_p_cut=cut)
+    got = native.warp_sample(x, top_k=top_k, top_p_cut=cut)
+    assert torch.equal(got[3], want) and torch.equal(got[0], ids) and torch.equal(got[1], logprob) and torch.equal(got[2], lse)
+    kept = torch.isfinite(want).sum(dim=1)
+    assert int(kept.min()) >= 1 and (k >= V or int(kept[3]) <= k)

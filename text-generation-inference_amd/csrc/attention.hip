@@ -119,7 +119,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
     const int pbeg = split * pps, pend = min(pages, pbeg + pps);
     ATTN_STAMP(1);  // (the sequence's lengths are in: the stamp macro waits for scalar loads)
     // The first fully visible page's table entry is asked for HERE — as soon as the lengths are in, in front of the q loads and
-    // of the partly visible pages: behind them it was a scalar round trip with nothing of this wave in flight (round 5 timeline,
+    // of the partly visible pages: behind them it was a scalar round trip with nothing of this wave in flight (timeline,
     // profiles/r05_attn_timeline.log: multi-chunk blocks had their first entry 4.8 k ticks after entry, 3.5 k after the lengths).
     const int pg_first = a.NS == 1 ? pg_spec : ((pbeg + w < pend) ? btrow[pbeg + w] : 0);
 
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
             }
         }
     }
-    // (Rotary embedding + cache write of the new token in this prologue was built in round 2, bit-exact, and measured slower
+    // (Rotary embedding + cache write of the new token in this prologue was built, bit-exact, and measured slower
     // than the launch in front: cfg3 104 vs 93 us — experiments/README.md.)
 
     f32x4 o[CH][NB];
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) vf[nb] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(vb + nb * 128));
     };
-    // The page a sequence is still filling: only the part its nv written tokens occupy is requested (round 5: the launch
+    // The page a sequence is still filling: only the part its nv written tokens occupy is requested (the launch
     // cost one whole page per started page — bench.py's steps got 0.1 ms slower the moment the batch crossed a page
     // boundary, and the counters saw 1.016 x the algorithmic bytes).  K: the second 16-token tile is requested only once the
     // sequence has reached it — until then its registers repeat the first tile (finite values, scores masked); a scalar base,
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
     const int kfull = ctx - q_len + t0 + 1;
     int p = pbeg + w;
     ATTN_STAMP(2);  // q requested, first table entry in
-    // The partly visible pages of this wave (decode: the sequence's last page) go FIRST (round 4): the softmax is order-
+    // The partly visible pages of this wave (decode: the sequence's last page) go FIRST: the softmax is order-
     // independent, and their masked body is a second copy of the page code that each wave runs once — at the end of the
     // launch its instruction fetch and its un-overlapped load were part of every block's tail (ctx 1023 vs 1024: +2.6 us
     // per launch before, +1.7 after); at the start both hide under the first pages' latency.
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
             // (row d = nb 16 + c 4 + r sits at nb 16 + r 4 + c: the four 16-lane groups of a store then hit four different
-            // groups of 16 banks instead of the same one — round 5: the [d][16] order was a 4-way conflict on every access)
+            // groups of 16 banks instead of the same one: the [d][16] order was a 4-way conflict on every access)
             for (int r = 0; r < 4; ++r) so[((ch * NW + w) * D + nb * 16 + r * 4 + c) * 16 + col] = o[ch][nb][r];
         if (c == 0) {
             sml[((ch * NW + w) * 2 + 0) * 16 + col] = m[ch];
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
 
 // out[tok][head][:] = sum_s O_s * 2^(m_s - m*) / sum_s l_s * 2^(m_s - m*);  one wave per (tok, head), four per workgroup.
 // MAXS > 0 (NS <= MAXS): every record of the row — {m, l} and the O slice of each split — is requested before the first use,
-// so the launch is ONE round trip to the records instead of two dependent passes over them (round 6: the MQA launch pair
+// so the launch is ONE round trip to the records instead of two dependent passes over them (the MQA launch pair
 // spends 4.5 of its 26 us here); MAXS == 0: any NS, the two-pass loop.  Same expressions in the same order either way.
 template <typename T, int D, int MAXS>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restrict__ ws_o,
@@ -642,14 +642,14 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
         // (tools/attn_nw.py, us: B=16 GQA 8:1 D=64 ctx 512: 6.8 unsplit vs 8.5 at 4 splits of 4 waves;
         //  B=1 MHA D=128 ctx 2048: 14.1 at 8 splits vs 17.7 at 16; B=4 GQA 4:1 ctx 4096: 19.0 at 8 vs 24.0 at 16)
         ns = std::min<int64_t>(cdiv64(256, base), pages / 16);
-        // Round 6 (profiles/r06_attn_fewgroups.log, first column = the rule above): from 32 pages on, up to 8 splits of >= 8
+        // (profiles/r06_attn_fewgroups.log, first column = the rule above)  From 32 pages on, up to 8 splits of >= 8
         // pages pay as long as every block still gets a CU of its own — B 1 MHA ctx 1024 11.6 -> 9.5 us (2 -> 8 splits), B 4
         // GQA 8:1 12.3 -> 10.4, B 8 GQA 8:1 D 64 9.4 -> 8.3, B 2 MHA 12.9 -> 11.8; 96 groups keep 2 (3 would be 288 blocks:
         // 16.4 vs 14.3), 16 pages keep 1 (8.7 vs 10.2), long contexts keep the rule above (>= 16 pages per block).
         if (pages >= 32) ns = std::max<int64_t>(ns, std::min<int64_t>(std::min<int64_t>(256 / base, pages / 8), 8));
         // From 128 groups on the merge costs more than the second half of the CUs gives while the context is short (a 7B rank at
         // TP = 8, B 32 x 4 heads, ctx 1024: 16.0 us unsplit, 16.5 at 2 splits; 64 groups, ctx 2048: 24.0 / 19.2 / 17.7 at
-        // 1 / 2 / 4 — profiles/r05_attn_tp8.log).  Round 6 swept it over the context (profiles/r06_attn_base128.log): exactly
+        // 1 / 2 / 4 — profiles/r05_attn_tp8.log).  Over the context (profiles/r06_attn_base128.log): exactly
         // 128 groups take 2 splits from ctx 2048 on (26.9 vs 29.1 us, 46.0 vs 51.7 at 4096, 166.6 vs 194.8 at 16384: the page
         // walk grows, the merge does not); 129 - 255 groups never do (2 splits would be a second round of blocks: 192 groups
         // 41.2 vs 34.9 at 2048, 272.8 vs 243.5 at 16384).
@@ -660,7 +660,7 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
         // not in the launch (a last-arriving block reads NS x 24 KB through ONE CU: 2.7 us at 4 splits, 5.4 at 8).
         // 48 q heads on 1 kv head, B=32 ctx 4096, us (kernel + combine): 26.7 at 4 splits, 25.1 at 6, 25.3 at 8
         // (in-launch merge: 28.1 / 28.6 / 30.2)
-        // round 6: with the combine launch down to one round trip (24.1 vs 25.3 us at 6 splits) 8 splits = 256 blocks edge out
+        // with the combine launch down to one round trip (24.1 vs 25.3 us at 6 splits) 8 splits = 256 blocks edge out
         // 6 (23.9 vs 24.2, profiles/r06_mqa_variants.log)
         ns = std::min<int64_t>(cdiv64(256, base), pages / 16);
     } else {

@@ -476,7 +476,7 @@ extern "C" int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_grou
 
 // ---- qkv projection with the rotary embedding and the cache write in its epilogue (dense weights) ---------------------
 // The unsplit plan of the fused qkv + rotary launch: plan_dense's SiLU plan, with ONE tile per k-part group where two would
-// leave fewer than 128 blocks (round 5: TinyLlama's 80 tiles ran as 40 blocks of 262 KB each — one CU takes in ~50 GB/s).
+// leave fewer than 128 blocks (TinyLlama's 80 tiles ran as 40 blocks of 262 KB each — one CU takes in ~50 GB/s).
 static DensePlan plan_dense_rope(int64_t K, int64_t N, int64_t M) {
     DensePlan pl = plan_dense(K, N, M, 2);
     const int64_t tiles = cdiv64(N, 32);

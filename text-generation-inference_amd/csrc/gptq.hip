@@ -5,7 +5,7 @@
 // utils/gptq/exllamav2.py:14-62,124-144.  Normative arithmetic (utils/gptq/quant_linear.py:130-138,
 // 184-194):  W[k,n] = (q[k,n] - (z[g(k),n] + 1)) * s[g(k),n];  y = x @ W, fp32 accumulate, f16 out.
 //
-// Prepared image (DESIGN.md §3), NT = ceil(N/32) column tiles, KS = ceil(K/64) k-steps, G groups:
+// Prepared image, NT = ceil(N/32) column tiles, KS = ceil(K/64) k-steps, G groups:
 //   A: wq [NT][KS][64 lanes][4] int32 — lane l word i = the 8 nibbles of rows
 //        k = (ks*8 + (l>>5)*4 + i)*8 + {0,2,4,6,1,3,5,7} of column n = nt*32 + (l&31): one KiB per wave
 //        load, and (after dequant8) exactly the B-operand fragment of v_mfma_f32_32x32x16_f16
@@ -619,7 +619,7 @@ extern "C" int tgis_gptq_rope_ok(int64_t M, int64_t K, int64_t N, int64_t groups
     // The epilogue needs the whole k range in one block (no split-K): worth it only while that plan still covers the chip
     // (measured: 7B qkv at 32 rows, 192 blocks: 14.9 vs 17.2 us for the pair; 70B qkv at 64 rows, 80 blocks of 42 MB: +5 % on
     // the step; a TP = 8 shard of the 7B qkv, 24 blocks: +2 % on the rank-step; TinyLlama dense, 40 blocks: +-0).
-    // Round 6: counted in blocks of the kernel that will run it (the fragment-order kernel gives a wave ONE tile where two would
+    // counted in blocks of the kernel that will run it (the fragment-order kernel gives a wave ONE tile where two would
     // leave fewer than 128 blocks), and up to 32 rows it pays from 48 blocks on — one rank of cfg3 at TP 8 / 4 / 2 (48 / 96 / 192
     // one-tile blocks) 1.838 / 2.110 / 3.000 -> 1.815 / 2.072 / 2.903 ms per step; at 64 rows every block takes in twice the
     // activation and the bar stays at 128 (a cfg4 rank at TP 8, 40 blocks: 6.45 -> 7.10 ms).  profiles/r06_tp_rope_blocks.log
@@ -671,7 +671,7 @@ extern "C" int tgis_gptq_fragments_ok(int64_t M, int64_t K, int64_t N, int64_t g
     if (off) return 0;
     static const int64_t max_rows = getenv("TGIS_GPTQ_FRAGMENTS_MAX_ROWS") ? atoll(getenv("TGIS_GPTQ_FRAGMENTS_MAX_ROWS")) : 64;
     if (M > max_rows) return 0;
-    // SiLU * up: from 64 blocks on (round 5, a 7B gate_up shard at TP = 8, 86 one-tile blocks: 8.2 us against 6.3 + 4.7 for
+    // SiLU * up: from 64 blocks on (a 7B gate_up shard at TP = 8, 86 one-tile blocks: 8.2 us against 6.3 + 4.7 for
     // the split streaming kernel + its reduce, profiles/r05_tp8_variants.log)
     static const int64_t min_blocks_silu = getenv("TGIS_SILU_MIN_BLOCKS") ? atoll(getenv("TGIS_SILU_MIN_BLOCKS")) : 64;
     if (act == 3 && gptq::wide_blocks(K, N, act, M) < rope_min_blocks(M)) return 0;

@@ -1,8 +1,8 @@
-// The int4 GPTQ GEMM for decode batches of up to 32 rows whose activation arrives in MFMA-fragment order (round 4).
+// The int4 GPTQ GEMM for decode batches and prompts of up to 64 rows whose activation arrives in MFMA-fragment order.
 //
 // Replaces exllamav2_kernels.gemm_half_q_half (utils/gptq/exllamav2.py:139-144) on the decode step, like the streaming
 // kernel of gptq_gemm_body.h, on the same prepared image.  What is different, and why (tools/floor/wide.hip measured every
-// step on the cfg3 shapes, profiles/r04_wide_*.log):
+// step at 4096, 11008, profiles/r04_wide_*.log):
 //   * the activation is not staged through LDS chunk by chunk.  Its producer (add + RMSNorm, the attention epilogue, the
 //     SiLU * up epilogue of this kernel) writes it in FRAGMENT ORDER — xf[k64-step][i][lane][8 halves], lane = 32 (k / 32 % 2)
 //     + row, i = k / 8 % 4 (xf_off in common.h) — so the A operand of the four MFMAs of a k64-step is four contiguous
@@ -15,8 +15,8 @@
 //     2.3 us of a 10 us launch) — and every wave finishes two of the sixteen accumulator rows of each tile (fixed order);
 //   * two k64-steps of weights + scales + activation in flight per wave, refilled in place; the last steps are taken by
 //     wave-uniform branches, so no wave dequantises padding.
-// cfg3 shapes, 32 rows, us per launch (streaming kernel -> this one): qkv + rope epilogue 16.9 -> 12.x, o 6.0 -> 5.3,
-// gate_up + SiLU 16.8 -> 14.x, down 10.5 -> 9.2.
+// 4096, 11008 at 32 rows, us per launch (streaming kernel -> this one): qkv + rope epilogue 16.9 -> 12.0, o 6.0 -> 5.4,
+// gate_up + SiLU 16.8 -> 15.9, down 10.5 -> 8.9; at 16 rows 10.9, 4.9, 13.2, 8.2.
 #pragma once
 #include "gptq_gemm_body.h"
 
@@ -50,7 +50,7 @@ static inline bool wide_serves(int64_t M, int64_t K, int64_t N, int64_t groups, 
 // One block per CU where the shape allows it: column groups first (a wider group re-uses an A fragment more often), then
 // global k splits (fp32 slabs that the consumer sums) until ~256 blocks; at least one k64-step per wave.
 // act 2 / 3 (SiLU * up, rotary + cache write) finish their outputs in the epilogue: no split.
-// Round 5 (tensor-parallel shard shapes): CT 1 where two tiles per wave would leave fewer than 128 blocks on an unsplit plan
+// Tensor-parallel shard shapes: CT 1 where two tiles per wave would leave fewer than 128 blocks on an unsplit plan
 // (a shard's gate_up: 224 tiles = 112 blocks of two tiles, each taking in its whole M x K activation — 1 MB at 64 rows —
 // through one CU), and `finished` (the caller needs the f16 output, not slabs: row-parallel linears in front of an
 // all-reduce): unsplit whenever that still gives >= 128 blocks, because a split plan costs a reduce launch on top.
@@ -127,7 +127,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
     const int sp_len = (steps + a.S - 1) / a.S;
     const int sb = split * sp_len, se = min(steps, sb + sp_len);
     const int len = max(se - sb, 0);
-    // This wave's k64-steps (may be empty).  (Round 5 measured an uneven split — the four waves a CU launches first run ~2 steps
+    // This wave's k64-steps (may be empty).  (Measured: an uneven split — the four waves a CU launches first run ~2 steps
     // ahead of the younger four, which queue behind them in the address path — and a prologue barrier, a raised priority for
     // the younger half and deeper weight rings: the block finishes when its CU has moved its bytes, however they are dealt;
     // tools/floor/wide.hip `kb` / `pb` / `prio` / `DW`, profiles/r05_wide_kbias*.log, r05_wide_plans.log.)
@@ -290,7 +290,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
 #pragma unroll
       for (int tg0 = 0; tg0 < CT; tg0 += TG) {
         if (mr > 0 || tg0 > 0) __syncthreads();  // the previous group's sums have been read
-        // (round 5: register PAIRS — [k-part][tile][register / 2][lane][2] — so that the sixteen registers leave as eight
+        // (register PAIRS — [k-part][tile][register / 2][lane][2] — so that the sixteen registers leave as eight
         // ds_write_b64 and the two registers a wave finishes come back as one ds_read_b64 per k-part and tile: the exchange
         // moves 2 x 8 waves x CT x 4 KiB through an LDS that takes 64 B/clk of 4-byte stores and gives 128 B/clk of 4-byte
         // loads, ~2.3 k clocks at CT 3; 8-byte accesses take 85 and 256 B/clk.  Same values, same order of the sum.)

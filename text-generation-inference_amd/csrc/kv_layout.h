@@ -1,4 +1,4 @@
-// KV page block layout for one (page, kv head), 32 tokens x D elements (DESIGN.md §3), and the "partial input" form of
+// KV page block layout for one (page, kv head), 32 tokens x D elements, and the "partial input" form of
 // the qkv activation (fp32 split-K slabs of the qkv GEMM that the consumer sums itself).  Shared by rope_kv.hip (the
 // stand-alone rotary + cache-write kernels) and attention.hip (the decode kernel that does both in its prologue).
 //   K: [tile=tok>>4][D/8][16 tokens][8]      -> MFMA 16x16x32 A-fragments are 1 KiB contiguous loads

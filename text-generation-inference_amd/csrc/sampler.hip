@@ -356,15 +356,20 @@ __global__ __launch_bounds__(NT) void warp_sample_kernel(SampleArgs a) {
 // registers; the probabilities of the top-p / typical-p searches are computed once per search instead of once per bit.
 // Same per-thread element order, same expressions, same block reductions: bit-identical to warp_sample_kernel, which stays
 // for larger vocabularies.  (The global form re-read the 128 KB row from L2 ~80 times: 0.4 ms per step at V = 32000.)
-// One CU per row, so bound by its vector units and by the chain of reductions.  V = 32000, us, with 32 row masks and keys made anew for
-// every bit (82 registers in memory) and the histogram read bin by bin / now: greedy 26 / 17, a draw 51 / 38, top-k 50 64 / 37, top-p 0.9
-// 89 / 54, both and a draw 132 / 78, repetition penalty 36 / 21, everything 190 / 129.
+// One CU per row, so bound by its vector units and by the chain of reductions: a bit of a search over 32 elements a thread is 1.0 us, of
+// which the two barriers and the sum of 16 partials are half.  V = 32000, us, with 32 row masks and keys made anew for every bit (82 registers in memory), the histogram read
+// bin by bin / all elements in each pass of the top-k and bit of the top-p / now: greedy 26 / 17 / 17, a draw 51 / 38 / 37, top-k 50 64 / 35 / 26, top-p 0.9
+// 89 / 50 / 48, both and a draw 132 / 73 / 53, repetition penalty 36 / 21 / 21.  (Waves that hold no key the bits to come could tell apart keeping their sum: 53 for 50 us
+// at top-p 0.9, since the reductions stay.)
 template <int NPT>
 __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
     __shared__ float fbuf[NW];
     __shared__ int ibuf[NW];
     __shared__ int hist[256];
     __shared__ uint32_t bc[2];
+    constexpr int LIST = 2 * NT, FEW_K = NT / 4;
+    __shared__ uint32_t list[LIST];
+    __shared__ int listed;
     const int b = blockIdx.x, tid = threadIdx.x, V = a.V;
     Block blk{fbuf, ibuf, tid & 63, tid >> 6};
     const float* in = a.logits + (int64_t)b * a.ld_logits;
@@ -428,28 +433,67 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
     // ---- top-k ----------------------------------------------------------------------------------------------------
     int k = a.top_k ? a.top_k[b] : 0;
     if (k > 0 && k < V) {
-        uint32_t prefix = 0, known = 0;
-        int want = k;
-#pragma unroll 1
-        for (int shift = 24; shift >= 0; shift -= 8) {
+        // eight more bits of the `want`-th key from above, of the keys that `count` puts into the histogram
+        auto narrow = [&](int shift, uint32_t& prefix, int& want, auto&& count) {
             for (int i = tid; i < 256; i += NT) hist[i] = 0;
             __syncthreads();
-            const int own4 = own_count();
-#pragma unroll
-            for (int j = 0; j < NPT; ++j) {
-                if (j < own4) {
-                    uint32_t key = order_key(x[j]);
-                    if ((key & known) == prefix) atomicAdd(&hist[(key >> shift) & 255], 1);
-                }
-            }
+            count(shift, prefix, ~(0xFFFFFFFFu >> (24 - shift)));
             __syncthreads();
             if (tid < 64) bin_from_above(hist, want, tid, bc);
             __syncthreads();
             prefix |= bc[0] << shift;
-            known |= 255u << shift;
             want = (int)bc[1];
             __syncthreads();
+        };
+        // Few of the row: the k-th of the threads' largest keys is no larger than the k-th of all, so that two bytes of it tell nearly all other elements
+        // off, and the passes go over a list of those that are left.  (With all elements in each pass the first of them is a queue at the few exponents
+        // that logits have: top-k 50 of 32000 20 us.)
+        uint32_t prefix = 0;
+        int n = LIST + 1;
+        if (k <= FEW_K) {  // us, all elements / the list: k 50, 200, 256 35 / 26, 35 / 27, 35 / 27, but 900 35 / 41
+            uint32_t largest = 0, low = 0;
+            const int own4 = own_count();
+#pragma unroll
+            for (int j = 0; j < NPT; ++j)
+                if (j < own4) largest = max(largest, order_key(x[j]));
+            int want = k;
+#pragma unroll 1
+            for (int shift = 24; shift >= 16; shift -= 8)
+                narrow(shift, low, want, [&](int sh, uint32_t pre, uint32_t known) {
+                    if ((largest & known) == pre) atomicAdd(&hist[(largest >> sh) & 255], 1);
+                });
+            if (tid == 0) listed = 0;
+            __syncthreads();
+            const int own5 = own_count();
+#pragma unroll
+            for (int j = 0; j < NPT; ++j) {
+                const uint32_t key = order_key(x[j]);
+                if (j < own5 && key >= low) {
+                    const int at = atomicAdd(&listed, 1);
+                    if (at < LIST) list[at] = key;
+                }
+            }
+            __syncthreads();
+            n = listed;
         }
+        int want = k;
+#pragma unroll 1
+        for (int shift = 24; shift >= 0; shift -= 8)
+            narrow(shift, prefix, want, [&](int sh, uint32_t pre, uint32_t known) {
+                if (n <= LIST) {
+                    for (int i = tid; i < n; i += NT)
+                        if ((list[i] & known) == pre) atomicAdd(&hist[(list[i] >> sh) & 255], 1);
+                    return;
+                }
+                const int own6 = own_count();
+#pragma unroll
+                for (int j = 0; j < NPT; ++j) {
+                    if (j < own6) {
+                        uint32_t key = order_key(x[j]);
+                        if ((key & known) == pre) atomicAdd(&hist[(key >> sh) & 255], 1);
+                    }
+                }
+            });
 #pragma unroll
         for (int j = 0; j < NPT; ++j)
             if (order_key(x[j]) < prefix) x[j] = NEG_INF;
@@ -478,13 +522,38 @@ __global__ __launch_bounds__(NT) void warp_sample_reg_kernel(SampleArgs a) {
             key[j] = order_key(x[j]);
             asm volatile("" : "+v"(key[j]));  // (kept, not made again from x for every bit)
         }
+        // Behind a top-k, a thread's few elements of any mass go into four places of their own: the same sums with what adds nothing left out.
+        constexpr int FEW = 4;
+        float q[FEW] = {};
+        uint32_t q_key[FEW] = {};
+        bool few = k > 0 && k <= FEW_K;
+        if (few) {
+            int c = 0;
+#pragma unroll
+            for (int j = 0; j < NPT; ++j) {
+                const bool some = !(p[j] == 0.f);
+#pragma unroll
+                for (int r = 0; r < FEW; ++r)
+                    if (some && c == r) {
+                        q[r] = p[j];
+                        q_key[r] = key[j];
+                    }
+                c += some;
+            }
+            few = blk.max((float)c) <= (float)FEW;
+        }
         uint32_t t = 0;
 #pragma unroll 1
         for (int bit = 31; bit >= 0; --bit) {
             const uint32_t cand = t | (1u << bit);
             float acc = 0.f;
+            if (few) {
 #pragma unroll
-            for (int j = 0; j < NPT; ++j) acc += key[j] <= cand ? p[j] : 0.f;  // p is 0 beyond the row
+                for (int r = 0; r < FEW; ++r) acc += q_key[r] <= cand ? q[r] : 0.f;
+            } else {
+#pragma unroll
+                for (int j = 0; j < NPT; ++j) acc += key[j] <= cand ? p[j] : 0.f;  // p is 0 beyond the row
+            }
             if (blk.sum(acc) <= cut) t = cand;
         }
         const uint32_t top = order_key(m);  // min_tokens_to_keep = 1
