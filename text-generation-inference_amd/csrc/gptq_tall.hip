@@ -538,11 +538,8 @@ TallArgs tall_args(const void* x, int64_t ldx, const void* prepared, int64_t M, 
 }  // namespace
 
 // Rows from which it may replace the 64-row streaming passes, and up to which it replaces dequantise + library GEMM: (library with its
-// dequantisation / tall, us, the four GEMMs of a 7B layer) 4096 rows 1547 / 1400, 6000 rows 2288 / 2121, 8192 rows 2829 / 2851; at 16128 rows
-// hipBLASLt's 256 x 256 tiles, free of dequantisation, run at 1.35 PFLOP/s against 1.12 - 1.25.  (These and the figures below are with the expansion to [K][N]; with
-// tgis_gptq_dequant_t_f16's [N][K] the library's side takes 10 - 15 % less: 4096 x 12288 at 3500, 4096, 7168, 8190 rows 286 / 330, 309 / 355, 553 / 624, 588 / 695, but
-// 581 / 513 at 6000; 11008 x 4096 at 5225, 7168 664 / 428, 557 / 563; 8192 x 10240 at 4096 716 / 573; 28672 x 8192 at 5225, 7168 2487 / 2009, 3217 / 2823.  Which of its
-// kernels the library takes there follows no rule of sizes, so the line stays where its tiles fill their rounds.)
+// dequantisation / tall, us, the four GEMMs of a 7B layer) 4096 rows 1428 / 1360, 6000 rows 2169 / 2011, 8190 rows 2595 / 2693; at 16128 rows
+// hipBLASLt's 256 x 256 tiles, free of dequantisation, run at 1.4 PFLOP/s against 1.2 - 1.25.
 int64_t gptq::tall_min_m(int act) {
     static const int64_t v = getenv("TGIS_TALL_MIN_M") ? atoll(getenv("TGIS_TALL_MIN_M")) : 0;
     return v ? v : act == 2 ? 65 : 129;
@@ -557,16 +554,18 @@ bool gptq::tall_serves(int64_t K, int64_t groups, bool act_order, int act) {
     return groups == 1 || (gs % 64 == 0 && (spg & (spg - 1)) == 0);
 }
 // Between 3072 and tall_max_m() rows it depends on how full the library's 256 x 256 tiles leave their rounds of 256.  act 0, us, dequantise
-// and library / this kernel, weights cold:
-//   93 % full and more:  5120 x 15360 at 5000, 6000, 8192 655 / 681, 785 / 804, 1043 / 1096; 11008 x 4096 at 4096, 8192 298 / 300, 561 / 590; 8192 x
-//                        10240 at 6000, 8192 822 / 834, 1060 / 1093; 5120 x 15360 at 4096 543 / 540 (but 4096 x 12288 at 4096 367 / 342, 13824 x
-//                        5120 at 6000 926 / 707)
-//   less:                4096 x 12288 at 6000, 7168 609 / 499, 637 / 596; 11008 x 4096 at 7168 732 / 545; 8192 x 10240 at 4096, 5000 744 / 550, 778 /
-//                        704; 13824 x 5120 at 4096, 5000 574 / 491, 838 / 600
-//   one round, from three fifths on, of long k:  5632 x 2048 at 5000, 7168 111 / 112, 143 / 146; 8192 x 3072 at 4096, 5000 183 / 197, 210 / 216
-//                        (4096 x 4096 at 3500 109 / 106; 5632 x 2048 at 4096, half a round, 97 / 87)
-// With SiLU * up this kernel is in front of the library and its activation launch (4096 x 22016 at 4096, 8192 rows 764 / 641, 1389 / 1365; 2048 x
-// 11264 198 / 178, 421 / 333).
+// ([N][K]) and library / this kernel, weights cold:
+//   93 % full and more:  5120 x 15360 at 4096, 6000, 8190 487 / 534, 713 / 768, 945 / 1029; 11008 x 4096 at 4096, 8190 269 / 298, 514 / 591; 8192 x
+//                        10240 at 6000, 8190 739 / 819, 957 / 1067; 4096 x 12288 at 4096, 5225, 8190 310 / 335, 410 / 432, 589 / 665 (but 13824 x 5120
+//                        at 6000 984 / 706)
+//   less:                4096 x 12288 at 6000 602 / 494; 11008 x 4096 at 5225, 7168 663 / 417, 561 / 546; 8192 x 10240 at 3500, 4096, 5225, 7168 629 / 491,
+//                        717 / 545, 833 / 722, 999 / 951; 13824 x 5120 at 3500, 5225, 8190 775 / 419, 897 / 620, 1067 / 917; 28672 x 8192 at 5225,
+//                        7168 2504 / 1990, 3224 / 2712; but also 4096 x 12288 at 3500 295 / 317, 4096 x 4096 at 7168 185 / 212, 8192 x 8192 at 5225,
+//                        7168 542 / 573, 705 / 757: which of its kernels the library takes there follows no rule of sizes
+//   one round, from three fifths on, of long k:  11008 x 4096 at 3500 248 / 277; 8192 x 3072 at 4096, 5000 183 / 197, 210 / 216 (5632 x 2048 at 4096,
+//                        half a round, 97 / 87)
+// With SiLU * up this kernel is in front of the library and its activation launch (4096 x 22016 at 4096, 8190 rows 740 / 611, 1291 / 1207; 2048 x
+// 11264 198 / 178, 421 / 333; 8192 x 57344 at 2045, 3500 1598 / 1514, 2666 / 2662, but at 4096, 8190 2889 / 3027, 5632 / 6084).
 bool gptq::tall_before_library(int64_t M, int64_t K, int64_t N, int act) {
     if (M <= 3072 || act == 2 || getenv("TGIS_TALL_MAX_M")) return M <= tall_max_m();
     const int64_t tiles = cdiv64(M, 256) * cdiv64(N, 256), slots = cdiv64(tiles, CUS) * CUS;
