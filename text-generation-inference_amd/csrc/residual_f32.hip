@@ -393,7 +393,8 @@ __global__ void unary_rows_vec_kernel(const T* __restrict__ in, int64_t ld_in, c
     }
 }
 
-// out[t][c] = gelu_tanh(gate[t][c]) * table[ids[t]][col0 + c]: a slice of a second token embedding, gated
+// out[t][c] = gelu_tanh(gate[t][c]) * table[ids[t]][col0 + c]: a slice of a second token embedding, gated.  The same function of the gate as where a projection's
+// epilogue applies it (dense_gemm_body.h), so that a token's bits do not depend on how many rows its step had.
 template <typename T>
 __global__ void gelu_gated_lookup_kernel(const T* __restrict__ gate, int64_t ld_gate, const int64_t* __restrict__ ids,
                                          const T* __restrict__ table, int64_t ld_table, int64_t col0, int64_t vocab,
@@ -403,9 +404,7 @@ __global__ void gelu_gated_lookup_kernel(const T* __restrict__ gate, int64_t ld_
         const int64_t t = idx / C, c = idx - t * C;
         const int64_t id = ids[t];
         const float e = (id >= 0 && id < vocab) ? Elem<T>::ld(table + id * ld_table + col0 + c) : 0.f;
-        const float z = Elem<T>::ld(gate + t * ld_gate + c);
-        const float inner = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-        out[t * ld_out + c] = cvt_out<T>(0.5f * z * (1.f + tanhf(inner)) * e);
+        out[t * ld_out + c] = cvt_out<T>(gelu_f32(Elem<T>::ld(gate + t * ld_gate + c), true) * e);
     }
 }
 
