@@ -821,6 +821,8 @@ int tgis_dense_gemm_whole_operand(int64_t M, int64_t K, int64_t N, int act);
  * M <= 64, K a multiple of 64, N_group of 32, x_group of 8. */
 int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo, int64_t out_group,
                            int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups, int dtype, void* stream);
+/* The k of its inputs that a workgroup keeps on the chip at a time (a host-side query). */
+int tgis_dense_gemm_groups_phase(int64_t M, int64_t K, int64_t N);
 /* The same for the rows of a prefill: any M; x rows 16-byte aligned, less than 2^22 elements apart.  ..._pays: 1 where it is the faster way (a size query). */
 int tgis_dense_tall_groups_pays(int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups);
 int tgis_dense_tall_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo, int64_t out_group,

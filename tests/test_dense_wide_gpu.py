@@ -92,8 +92,8 @@ def test_rope(gpu_device, K, H, Hkv, D, M):
         assert float(diff.max()) <= scale and float((diff > 0).float().mean()) < 0.05
 
 
-# groups: one, and several with a last one that is whole / one ragged tile / several tiles
-@pytest.mark.parametrize("K,n_group,N,G", [(64, 32, 20, 1), (448, 96, 288, 3), (576, 64, 150, 3), (2048, 512, 2048 + 64, 5), (4160, 64, 4 * 64 + 33, 5)])
+# groups: one, and several with a last one that is whole / one ragged tile / several tiles; the last has more tiles than there are CUs, whose phases of x are shorter
+@pytest.mark.parametrize("K,n_group,N,G", [(64, 32, 20, 1), (448, 96, 288, 3), (576, 64, 150, 3), (2048, 512, 2048 + 64, 5), (4160, 64, 4 * 64 + 33, 5), (2112, 2080, 4 * 2080 + 33, 5)])
 @pytest.mark.parametrize("M", [1, 8, 15, 16, 17, 32, 33, 64])
 def test_groups(gpu_device, K, n_group, N, G, M):
     from tgis_amd import native

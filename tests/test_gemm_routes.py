@@ -111,3 +111,14 @@ def test_dense_tall_parts_or_passes(M, K, N, serves):
     from tgis_amd import native
 
     assert (native.load_library().tgis_dense_tall_partial_bytes(M, K, N) >= 0) == bool(serves)
+
+
+# phases of the x of several products in one launch: halved where that lets a CU take a second of more tiles than there are CUs
+@pytest.mark.parametrize("M,K,N,k", [
+    (21, 2048, 256 * 32, 1024), (21, 2048, 256 * 32 + 1, 512), (32, 4096, 130 * 32, 1024), (32, 4096, 516 * 32, 512), (17, 2048, 258 * 32, 1024), (21, 1024, 516 * 32, 1024),
+    (16, 8192, 97 * 32, 2048), (16, 4096, 516 * 32, 1024), (8, 4096, 516 * 32, 2048), (16, 2048, 516 * 32, 2048), (33, 4096, 516 * 32, 512), (64, 512, 32, 512),
+])
+def test_dense_groups_phase(M, K, N, k):
+    from tgis_amd import native
+
+    assert native.load_library().tgis_dense_gemm_groups_phase(M, K, N) == k

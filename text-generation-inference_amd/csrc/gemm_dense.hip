@@ -443,17 +443,26 @@ static int launch_groups(const DenseArgs& a, int groups, int tiles, int64_t x_gr
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
+// k of a phase of x: the longest (up to 16 rows 2048, to 32 1024, above 512), and where there are more tiles than CUs half of that if it leaves room for two blocks on a
+// CU: with one, the tiles past the 256th are a round of their own.  us, longest / half: 258 tiles of 2048 k at 21, 32 rows 13.4 / 12.1, 14.2 / 13.3; 325 of 2560 at 16, 21,
+// 32 16.8 / 14.8, 17.9 / 15.8, 19.7 / 17.0; 516 of 4096 32.3 / 28.6, 34.5 / 31.6, 36.6 / 33.7; but 66 of 2048 at 21, 32 6.6 / 7.0, 7.0 / 7.4, 130 of 4096 11.1 / 12.1, 12.5 /
+// 12.7, 250 of 2048 8.8 / 9.2, 9.3 / 9.7, of 4096 14.4 / 15.3, 15.5 / 15.9
+extern "C" int tgis_dense_gemm_groups_phase(int64_t M, int64_t K, int64_t N) {
+    if (M < 1 || K < 64 || N < 1 || M > 32) return 512;
+    const bool r16 = M <= 16;
+    const int q = r16 ? 4 : 2;
+    const bool halved = cdiv64(N, 32) > 256 && dense::wide_lds_bytes(M, K, 1, 1, r16, q) > 80 * 1024;
+    return 512 * (halved ? q / 2 : q);
+}
 template <typename T>
 static int launch_groups_rows(const DenseArgs& a, int groups, int tiles, int64_t x_group, int64_t out_group, hipStream_t st) {
+    const int phase = tgis_dense_gemm_groups_phase(a.M, a.K, a.N);
     if (a.M > 32) return launch_groups<T, 2, false, 1>(a, groups, tiles, x_group, out_group, st);
-    // The longest phases of x that leave room for two blocks on a CU: with one, tiles past the 256th are a round of their own (258 tiles of 2048 k, us, phases of
-    // 1024 / 512 k: 21 rows 13.5 / 12.3, 32 14.4 / 13.5; 514 of 4096 34.6 / 32.0, 37.1 / 33.9; of 2048 / 1024 k at 16 rows 32.1 / 29.0)
-    auto fits = [&](bool r16, int q) { return dense::wide_lds_bytes(a.M, a.K, 1, 1, r16, q) <= 80 * 1024; };
-    if (a.M <= 16)
-        return fits(true, 4) ? launch_groups<T, 1, true, 4>(a, groups, tiles, x_group, out_group, st)
-                             : launch_groups<T, 1, true, 2>(a, groups, tiles, x_group, out_group, st);
-    return fits(false, 2) ? launch_groups<T, 1, false, 2>(a, groups, tiles, x_group, out_group, st)
-                          : launch_groups<T, 1, false, 1>(a, groups, tiles, x_group, out_group, st);
+    if (a.M > 16)
+        return phase == 1024 ? launch_groups<T, 1, false, 2>(a, groups, tiles, x_group, out_group, st)
+                             : launch_groups<T, 1, false, 1>(a, groups, tiles, x_group, out_group, st);
+    return phase == 2048 ? launch_groups<T, 1, true, 4>(a, groups, tiles, x_group, out_group, st)
+                         : launch_groups<T, 1, true, 2>(a, groups, tiles, x_group, out_group, st);
 }
 
 extern "C" int tgis_dense_gemm_groups(const void* x, int64_t ldx, int64_t x_group, const void* prepared, void* out, int64_t ldo,

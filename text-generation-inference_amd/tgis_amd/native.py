@@ -215,6 +215,7 @@ SIGNATURES = {
     "tgis_llama_prompt": (_c_int, [_vp, _c_int, _vp, _vp]),
     "tgis_dense_gemm_whole_operand": (_c_int, [_c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_dense_gemm_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_gemm_groups_phase": (_c_int, [_c_i64, _c_i64, _c_i64]),
     "tgis_dense_tall_groups_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
     "tgis_dense_tall_groups": (_c_int, [_vp, _c_i64, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_gemm_relu2": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp, _c_i64, _vp]),
