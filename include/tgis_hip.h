@@ -116,6 +116,8 @@ int64_t tgis_gptq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
  * faster with it (1 <= M <= 64, no act-order, groups of 64 * 2^n rows; act 2 / 3 additionally >= 128 workgroups). */
 #define TGIS_LD_FRAGMENTS ((int64_t)-32)
 int tgis_gptq_fragments_ok(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act);
+/* ... and the rows that the launch computes (a multiple of 16, at least M; a host-side query). */
+int tgis_gptq_fragment_rows(int64_t M, int64_t K, int64_t N, int act);
 
 /* out[M,N] f16 = x[M,K] f16 @ dequant(W)[K,N] (+ bias[N] f16 if non-NULL); fp32 accumulate.
  * Fused int4-dequant MFMA kernel for any M (rows are processed in slabs of 32).

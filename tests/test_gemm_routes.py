@@ -122,3 +122,14 @@ def test_dense_groups_phase(M, K, N, k):
     from tgis_amd import native
 
     assert native.load_library().tgis_dense_gemm_groups_phase(M, K, N) == k
+
+
+# int4 launches in fragment order: blocks of 16 rows, but four for three where a wave walks one or two k64-steps of two tiles
+@pytest.mark.parametrize("M,K,N,act,rows", [
+    (1, 2048, 2048, 0, 16), (16, 2048, 2048, 0, 16), (17, 2048, 2048, 0, 32), (33, 2048, 2048, 0, 64), (48, 1024, 3072, 0, 64), (48, 4096, 4096, 0, 64), (33, 6144, 4096, 0, 48),
+    (33, 4160, 4096, 0, 48), (48, 5632, 2048, 0, 64), (48, 4096, 12288, 0, 48), (48, 4096, 22016, 2, 48), (48, 1024, 8192, 2, 64), (48, 1024, 4096, 2, 48), (49, 4096, 12288, 0, 64), (64, 2048, 2048, 0, 64),
+])
+def test_int4_fragment_rows(M, K, N, act, rows):
+    from tgis_amd import native
+
+    assert native.load_library().tgis_gptq_fragment_rows(M, K, N, act) == rows

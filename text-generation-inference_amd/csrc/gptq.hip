@@ -388,9 +388,12 @@ static int launch_wide_rows(dim3 grid, hipStream_t st, const GemmArgs& a) {
 }
 template <int CT, int ACT, bool OUTF>
 static int launch_wide_one(dim3 grid, hipStream_t st, const GemmArgs& a) {
-    if (a.M <= 16) return launch_wide_rows<CT, ACT, OUTF, 1>(grid, st, a);
-    if (a.M <= 32) return launch_wide_rows<CT, ACT, OUTF, 2>(grid, st, a);
-    return a.M <= 48 ? launch_wide_rows<CT, ACT, OUTF, 3>(grid, st, a) : launch_wide_rows<CT, ACT, OUTF, 4>(grid, st, a);
+    switch (gptq::wide_row_blocks(a.M, a.K, CT, a.S)) {
+        case 1: return launch_wide_rows<CT, ACT, OUTF, 1>(grid, st, a);
+        case 2: return launch_wide_rows<CT, ACT, OUTF, 2>(grid, st, a);
+        case 3: return launch_wide_rows<CT, ACT, OUTF, 3>(grid, st, a);
+        default: return launch_wide_rows<CT, ACT, OUTF, 4>(grid, st, a);
+    }
 }
 
 static int launch_gptq(const void* x, int64_t ldx, const void* prepared, const void* bias, const int32_t* perm,
@@ -677,6 +680,12 @@ extern "C" int tgis_gptq_fragments_ok(int64_t M, int64_t K, int64_t N, int64_t g
     if (act == 3 && gptq::wide_blocks(K, N, act, M) < rope_min_blocks(M)) return 0;
     if (act == 2 && gptq::wide_blocks(K, N, act, M, true) < min_blocks_silu) return 0;
     return 1;
+}
+
+extern "C" int tgis_gptq_fragment_rows(int64_t M, int64_t K, int64_t N, int act) {
+    if (M < 1 || M > 64 || K < 64 || K % 64 != 0 || N < 1) return 0;
+    const gptq::WidePlan p = gptq::plan_wide(K, N, act, M);
+    return 16 * gptq::wide_row_blocks(M, K, p.CT, p.S);
 }
 
 extern "C" int tgis_gptq_gemm_f16_partial(const void* x, int64_t ldx, const void* prepared, const int32_t* perm,

@@ -95,6 +95,15 @@ static inline int wide_max_splits(int64_t K, int64_t N) {
                     std::max(plan_wide(K, N, 0, 32, true).S, plan_wide(K, N, 0, 64, true).S));
 }
 
+// 16-row blocks that a launch works on (gptq_wide_unit's RB): those of its rows, but four for three where a wave walks no more than two k64-steps of two tiles and the
+// launch is over before the row swaps pay.  us, three / four at 33 - 48 rows: 1024 x 3072 (one step) 5.7 / 5.5, 2048 x 2048 (one) 5.9 / 5.7, 5632 x 2048 (one to two) 6.9 / 6.8, 4096 x
+// 4096 (two) 7.1 / 7.0; 5632 x 2048 and 4096 x 4096 cut so that it is three 7.9 / 7.8, 8.1 / 8.1; 6144 x 4096 (three) 8.9 / 9.3.  Two steps of three tiles or four: 2048 x 12288 9.6 /
+// 10.7, 4096 x 8192 12.4 / 13.6, of one tile 2048 x 2048 4.9 / 5.1.
+static inline int wide_row_blocks(int64_t M, int64_t K, int CT, int S) {
+    const int rb = (int)cdiv64(M, 16);
+    return rb == 3 && CT == 2 && cdiv64(K / 64, S) <= 2 * WIDE_WK ? 4 : rb;
+}
+
 // rows 1, 3 of 16 lanes of x against rows 0, 2 of y
 __device__ __forceinline__ void swap_rows(uint32_t x, uint32_t y, uint32_t (&out)[2]) {
     const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false);
