@@ -335,6 +335,8 @@ int tgis_rope_k_write_prefill(const void* qkv, int64_t ld_qkv, const void* cos, 
  *      utils/flash_attn.py:43-78) ---------------------------------------------------------------- */
 /* Number of key-range splits the launcher will use for this shape (so callers can size workspace). */
 int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len, int64_t max_ctx);
+/* ... and the waves of a workgroup of a decode step that takes that many (a host-side query). */
+int tgis_attn_decode_waves(int64_t B, int Hkv, int H, int D, int64_t max_ctx);
 int64_t tgis_attn_workspace_bytes(int64_t total_q_tokens, int H, int Hkv, int D, int num_splits);
 /* Causal softmax(q k^T * scale) v over the paged cache.
  *   q: [total_q, H, D] with token stride ld_q (elements); out: [total_q, H*D] contiguous (ld_out = 0 or

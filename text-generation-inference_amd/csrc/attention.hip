@@ -544,16 +544,19 @@ static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && group
 // 1 - 2 % at 1024, since blocks that wait for a place level what is ragged.  16 waves: 0 - 2 us slower on up to 256 groups.)  us, waves:
 //   257 - 512 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600, 2048:
 //     14.2 / 13.9, 35.9 / 34.7, ragged 12.8 / 11.7, 32.3 / 26.5; 512 at 700, 4000 17.8 / 18.1, 78.9 / 80.4, ragged 15.2 / 14.3, 63.6 / 55.9; 384 at 130 8.0 / 8.3)
-//   769 - 1023 of D 128: 8, since 4 leave a second round (992 at 300, 1024, 3000 4 / 8: 29.7 / 27.7, 85.6 / 79.0, 257.7 / 231.8, ragged 20.6 / 20.3, 55.6 / 52.9, 150.8 /
-//     146.6; 800 76.2 / 69.5, ragged 45.2 / 45.9; 2 waves take 8 - 14 % longer than 4 where 800 sequences are ragged)
+//   896 - 1023 of D 128: 8 from 12 pages on, since 4 leave a second round.  4 / 8, and the mean of five ragged draws: 896 at 200, 256, 400, 1000, 3500 18.0 / 18.0, 20.5 / 20.5, 35.4 /
+//     31.0, 78.7 / 70.2, 293 / 242, ragged 14.1 / 15.1, 15.8 / 16.5, 23.3 / 22.6, 50.5 / 48.5, 168.0 / 165.4; 992 at 200, 400, 3500 20.3 / 19.4, 37.4 / 32.6, 316 / 266, ragged 15.2 / 15.6, 25.3 /
+//     24.3, 183 / 179.  Below, blocks that wait for a place level what is ragged: 832 at 400, 1700, 3500 33.7 / 30.1, 130 / 118, 272 / 237, but ragged 19.7 / 21.0, 75.7 / 76.4, 160 / 164 (2
+//     waves take 8 - 14 % longer than 4 where 800 sequences are ragged)
 //   1024 - 2047: 2, which halve the page-count imbalance between a block's waves (33 pages over 4 waves = 9/8/8/8; over 2 = 17/16); of D 128 past 1536, a second round
-//     of these, 8 (1600 at 300, 1024, 3000 2 / 8: 47.5 / 43.8, 147 / 133, 430 / 383, ragged 32.2 / 30.6, 92.0 / 86.2, 257 / 249)
+//     of these, 8 from 12 pages on (2 / 8: 1600 at 200, 256, 400, 1000, 3500 32.4 / 30.1, 37.7 / 34.8, 59.7 / 52.4, 143.5 / 126.9, 522 / 457, ragged 19.5 / 22.0, 25.3 / 25.5, 37.0 / 35.4, 86.7 /
+//     81.7, 298 / 286; 2000 at 130, 200, 400 28.2 / 30.1, 38.9 / 36.7, 68.7 / 63.2, ragged 19.7 / 22.1, 24.9 / 27.1, 46.8 / 43.1)
 //   from 2048 on 4: past that the dispatch rate, 7 ns per workgroup, costs more than the imbalance
 static int decode_waves(int64_t blocks, int num_splits, int ch, int D, int64_t pages) {
     if (wide_decode_blocks(blocks / num_splits, ch)) return 8;
     if (ch == 1 && num_splits == 1) {
         if (D == 64 && blocks <= 512 && pages >= 8) return 8;
-        if (D == 128 && ((blocks > 768 && blocks < 1024) || (blocks > 1536 && blocks < 2048))) return 8;
+        if (D == 128 && pages >= 12 && ((blocks >= 896 && blocks < 1024) || (blocks > 1536 && blocks < 2048))) return 8;
     }
     return blocks >= 1024 && blocks < 2048 ? 2 : 4;
 }
@@ -667,11 +670,17 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
         // single-chunk blocks, many groups: two splits only where the second half of the chip's waves gives more than the merge takes: up to 384 groups (768 blocks of
         // 4 waves are resident at D 128) from 48 pages on.  us, 1 / 2 splits: 352 groups of D 128 at ctx 600, 1024, 1400 21.2 / 23.2, 32.5 / 33.5, 42.3 / 42.8, ragged 16.6 /
         // 18.3, 25.3 / 25.2, 32.0 / 32.8, but at 2048, 4096 61.0 / 59.2, 117.6 / 113.1, ragged 44.8 / 44.3, 84.6 / 81.6; 320 at 1400, 2048 41.5 / 41.5, 59.0 / 56.3; 448 at 1024, 3000 36.6 /
-        // 45.4, 103.8 / 127.4, ragged 30.2 / 34.0, 80.1 / 82.1; D 64, 448 at 600, 2048 14.9 / 18.4, 37.8 / 42.4
+        // 45.4, 103.8 / 127.4, ragged 30.2 / 34.0, 80.1 / 82.1 (416 at 3500 111 / 137, but the mean of ten ragged draws 87 / 84); D 64, 448 at 600, 2048 14.9 / 18.4, 37.8 / 42.4
         ns = base <= 384 && pages >= 48 ? 2 : 1;
     }
     ns = std::max<int64_t>(1, std::min<int64_t>(ns, 64));
     return (int)ns;
+}
+
+extern "C" int tgis_attn_decode_waves(int64_t B, int Hkv, int H, int D, int64_t max_ctx) {
+    if (B <= 0 || Hkv <= 0 || H <= 0 || H % Hkv != 0 || (D != 64 && D != 128)) return 0;
+    const int HC = attn_geom(H, Hkv).HC, ch = chunks_per_block(HC, 1), ns = tgis_attn_num_splits(B, Hkv, H, 1, max_ctx);
+    return decode_waves(B * Hkv * cdiv64(HC, ch) * ns, ns, ch, D, cdiv64(max_ctx, 32));
 }
 
 // records of the fused combine: [group = (sequence, kv head, chunk block)][chunk][16 columns][split]

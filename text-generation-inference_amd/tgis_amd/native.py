@@ -86,6 +86,7 @@ SIGNATURES = {
     "tgis_rope_k_write_prefill": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64,
                                             _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tgis_attn_num_splits": (_c_int, [_c_i64, _c_int, _c_int, _c_i64, _c_i64]),
+    "tgis_attn_decode_waves": (_c_int, [_c_i64, _c_int, _c_int, _c_int, _c_i64]),
     "tgis_attn_workspace_bytes": (_c_i64, [_c_i64, _c_int, _c_int, _c_int, _c_int]),
     "tgis_dense_rows_ok": (_c_int, [_c_i64, _c_i64, _c_int]),
     "tgis_dense_rows_norm_rope": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64,
