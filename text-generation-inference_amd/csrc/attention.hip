@@ -542,8 +542,8 @@ static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && group
 // Waves of a decode block of one chunk.  What is resident decides: of D 128 768 blocks of 4 waves, 1536 of 2 (three waves per SIMD), 512 of 8 (four: their bound on
 // registers), of D 64 more.  (Four waves per SIMD for the smaller blocks as well: equal sequences 7 - 10 % faster at 992 groups, but ragged ones 3 - 7 % slower and
 // 1 - 2 % at 1024, since blocks that wait for a place level what is ragged.  16 waves: 0 - 2 us slower on up to 256 groups.)  us, waves:
-//   257 - 512 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600, 2048:
-//     14.2 / 13.9, 35.9 / 34.7, ragged 12.8 / 11.7, 32.3 / 26.5; 512 at 700, 4000 17.8 / 18.1, 78.9 / 80.4, ragged 15.2 / 14.3, 63.6 / 55.9; 384 at 130 8.0 / 8.3)
+//   257 - 512 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600
+//     14.2 / 13.9, ragged 12.8 / 11.7; 512 at 700, 4000 17.8 / 18.1, 78.9 / 80.4, ragged 15.2 / 14.3, 63.6 / 55.9; 384 at 130 8.0 / 8.3); two splits, below, are of 4 waves
 //   896 - 1023 of D 128: 8 from 12 pages on, since 4 leave a second round.  4 / 8, and the mean of five ragged draws: 896 at 200, 256, 400, 1000, 3500 18.0 / 18.0, 20.5 / 20.5, 35.4 /
 //     31.0, 78.7 / 70.2, 293 / 242, ragged 14.1 / 15.1, 15.8 / 16.5, 23.3 / 22.6, 50.5 / 48.5, 168.0 / 165.4; 992 at 200, 400, 3500 20.3 / 19.4, 37.4 / 32.6, 316 / 266, ragged 15.2 / 15.6, 25.3 /
 //     24.3, 183 / 179.  Below, blocks that wait for a place level what is ragged: 832 at 400, 1700, 3500 33.7 / 30.1, 130 / 118, 272 / 237, but ragged 19.7 / 21.0, 75.7 / 76.4, 160 / 164 (2
@@ -670,7 +670,9 @@ extern "C" int tgis_attn_num_splits(int64_t B, int Hkv, int H, int64_t max_q_len
         // single-chunk blocks, many groups: two splits only where the second half of the chip's waves gives more than the merge takes: up to 384 groups (768 blocks of
         // 4 waves are resident at D 128) from 48 pages on.  us, 1 / 2 splits: 352 groups of D 128 at ctx 600, 1024, 1400 21.2 / 23.2, 32.5 / 33.5, 42.3 / 42.8, ragged 16.6 /
         // 18.3, 25.3 / 25.2, 32.0 / 32.8, but at 2048, 4096 61.0 / 59.2, 117.6 / 113.1, ragged 44.8 / 44.3, 84.6 / 81.6; 320 at 1400, 2048 41.5 / 41.5, 59.0 / 56.3; 448 at 1024, 3000 36.6 /
-        // 45.4, 103.8 / 127.4, ragged 30.2 / 34.0, 80.1 / 82.1 (416 at 3500 111 / 137, but the mean of ten ragged draws 87 / 84); D 64, 448 at 600, 2048 14.9 / 18.4, 37.8 / 42.4
+        // 45.4, 103.8 / 127.4, ragged 30.2 / 34.0, 80.1 / 82.1 (416 at 3500 111 / 137, but the mean of ten ragged draws 87 / 84); D 64, 448 at 600, 2048 14.9 / 18.4, 37.8 / 42.4,
+        // but one of 8 waves against two of 4 at 288 groups, 1536, 3500 22.8 / 21.8, 47.6 / 43.8, ragged 19.0 / 18.6, 36.8 / 34.5, at 352 24.4 / 24.3, 51.9 / 50.6, ragged 18.9 / 19.1, 40.8 / 39.7, at 384,
+        // 2048, 8000 32.8 / 33.6, 119.9 / 119.3, ragged 26.0 / 26.1, 91.9 / 89.3
         ns = base <= 384 && pages >= 48 ? 2 : 1;
     }
     ns = std::max<int64_t>(1, std::min<int64_t>(ns, 64));
