@@ -63,7 +63,7 @@ def test_int4_library(M, K, N, act, pays):
 @pytest.mark.parametrize("M,K,N,act,pays", [
     (64, 2048, 2048, 0, 0), (65, 2048, 2048, 0, 0), (65, 4096, 4096, 0, 1), (256, 6144, 24576, 4, 1), (257, 6144, 24576, 4, 0), (1400, 2048, 2048, 0, 1), (1401, 2048, 2048, 0, 0),
     (500, 2048, 6144, 0, 1), (501, 2048, 6144, 0, 0), (100, 2040, 2048, 0, 0), (100, 2048, 1024, 0, 0), (100, 8192, 1024, 0, 1), (100, 8192, 1023, 0, 0), (300, 448, 2048, 0, 0), (200, 64, 2048, 0, 1), (512, 4096, 22016, 2, 0), (513, 4096, 22016, 2, 1), (300, 2048, 11264, 2, 1),
-    (65, 320, 1280, 0, 1), (65, 320, 1280, 5, 0), (896, 3072, 5120, 0, 0), (700, 3072, 5120, 0, 1), (900, 24576, 6144, 0, 1), (1708, 24576, 6144, 0, 1), (1709, 24576, 6144, 0, 0), (2048, 18944, 3584, 0, 1), (1793, 20480, 5120, 0, 0), (1401, 11008, 4096, 0, 0), (600, 28672, 8192, 0, 0), (600, 4096, 28672, 2, 0),
+    (65, 320, 1280, 0, 1), (65, 320, 1280, 5, 0), (896, 3072, 5120, 0, 0), (700, 3072, 5120, 0, 1), (900, 24576, 6144, 0, 1), (1708, 24576, 6144, 0, 1), (1709, 24576, 6144, 0, 0), (2048, 18944, 3584, 0, 1), (1793, 20480, 5120, 0, 0), (1408, 28672, 7168, 0, 0), (1032, 28672, 7168, 4, 1), (1033, 28672, 7168, 4, 0), (1024, 24576, 7200, 0, 0), (1448, 24576, 6144, 5, 1), (1449, 24576, 6144, 5, 0), (1600, 24576, 6144, 0, 0), (1601, 24576, 6144, 0, 1), (1650, 24576, 5888, 0, 0), (1738, 28672, 5120, 0, 1), (1739, 28672, 5120, 0, 0), (2048, 24576, 4096, 0, 1), (2049, 24576, 4096, 0, 0), (1401, 24640, 4096, 0, 0), (1400, 24640, 4096, 0, 1), (2048, 32768, 2048, 0, 1), (1401, 32768, 2080, 0, 0), (1401, 16384, 2048, 0, 0), (1401, 11008, 4096, 0, 0), (600, 28672, 8192, 0, 0), (600, 4096, 28672, 2, 0),
     (8192, 2048, 11264, 2, 1), (8193, 2048, 11264, 2, 0), (100, 2048, 2048, 1, 0), (0, 2048, 2048, 0, 0),
 ])
 def test_dense_tall(M, K, N, act, pays):

@@ -537,10 +537,7 @@ int run_tall(const TallPlan& p, DTallArgs& a, int act, hipStream_t st) {
 // Above, it is the library, with a launch of its own for the activation.
 //   act 0 / GELU: it wins where its tiles of 128 x 256 fill more than half the chip (4096 x 6144 at 800, 1024 rows 47 / 56, 52 / 61; 3072 x 5120 at 900, 1400 40 / 44,
 //   49 / 50; 28672 x 8192 at 600 259 / 346; layers of 3072, 8192 at 1390 rows 394 / 371 us with it, of 4096, 14336 at 900 494 / 467), but not on narrow products of
-//   long k (11008 x 4096 at 1024, 1400 rows 102 / 85, 133 / 124; 13824 x 5120 at 1200 1.7), and past k of 16384 up to 1792 rows, where the library is 1.2 to 1.9 times
-//   as long (24576 x 6144 at 700, 1024, 1393, 1700 298 / 259, 405 / 327, 621 / 363, 677 / 449, at 2045 445 / 517; 20480 x 5120 at 1280, 1536, 1700 346 / 253, 426 / 275,
-//   532 / 304, at 1900 315 / 342; 28672 x 7168 at 1024, 1280 501 / 382, 731 / 447, at 1408 430 / 500), and up to 2048 where half a round of tiles covers it (18944 x 3584 at
-//   1900, 2048 344 / 221, 356 / 224): 8 layers of 6144, 24576 at 1300, 1700 rows 9.39 -> 7.65, 10.90 -> 9.23 ms.  Between k of 9600 and 16384 more rows give as much as they take
+//   long k (11008 x 4096 at 1024, 1400 rows 102 / 85, 133 / 124; 13824 x 5120 at 1200 1.7), nor past k of 16384 (below).  Between k of 9600 and 16384 more rows give as much as they take
 //   (1700 rows: 11008 x 4096 152 / 135, 10240 x 2560 104 / 114, 14336 x 7168 246 / 298).  Below that the two are close (300, 512, 1024 rows: 2048 x
 //   2560 13.3 / 14.8, 15.3 / 16.6, 22.9 / 19.7; 4096 x 4096 26.2 / 25.6, 30 / 31, 41.9 / 42.7; 5632 x 2048 26 / 22.5, 26.7 / 23.6, 40 / 35; 6144 x 6400 44.7 / 43.5,
 //   67 / 60, 91 / 88), and inside a model this kernel is the faster one also where it is not alone: 22 layers of 2048, 5632 at 257, 400 rows 2781 / 2466,
@@ -555,6 +552,20 @@ static bool passes_in_a_round(int64_t M, int64_t K, int64_t N, int64_t from_bloc
     const int64_t blocks = cdiv64(cdiv64(N, 32), pass.TN) * cdiv64(M, 64) * pass.S;
     return pass.TN == 2 && pass.S > 1 && pass.KR <= 1024 && blocks >= from_blocks && blocks <= CUS;
 }
+// Past k of 16384, up to 2048 rows and 7168 columns.  The library's time goes in steps of up to twice, by a choice of kernels that follows no rule of sizes; drawn here
+// is where it was the longer one, of 1938 products (k 16448 - 36864, 1024 - 7168 columns, 900 - 2048 rows; this kernel takes 0.70 of its time) but for one in 140.  us, library / this:
+//   up to 4096 columns  24576 x 4096 at 1408, 1700, 2048 rows 420 / 274, 428 / 315, 490 / 350; 18432 x 3584 219 / 204 - 336 / 239; 16448 x 1024 169 / 64 (18496 x 3456 at 1760 208 / 246); past k of
+//                       24576 up to 2048 (28672 x 2048 at 2048 325 / 205, but x 4096 at 1408 298 / 323, x 3072 at 2048 293 / 397, 34944 x 2304 at 1969 308 / 374)
+//   up to 6144 columns  as far as 8.9 M outputs: 24576 x 5120 at 1280, 1700 403 / 330, 616 / 378; x 6144 at 1152, 1393 373 / 355, 628 / 375; but at 1464, 1536 385 / 400, 388 / 416, x 5120 at 1792 382 /
+//                       394, x 5723 at 1676 395 / 434.  From 1601 rows of 24 columns of 256 tiles on again: 24576 x 6144 at 1650, 1700 669 / 444, 675 / 459 (23424 x 6144 at 1599 367 / 398)
+//   up to 7168          as far as 7.4 M: 28672 x 7168 at 900, 1024 485 / 391, 503 / 393, but at 1152, 1344, 1408 413 / 438, 463 / 505, 466 / 525 (at 1280 738 / 465); x 8128 at 850 369 / 438
+// 8 layers of 6144, 24576 at 1300, 1700 rows 9.39 -> 7.65, 10.90 -> 9.23 ms.
+static bool pays_past_16k(int64_t M, int64_t K, int64_t N) {
+    if (K <= 16384 || M > 2048) return false;
+    if (N <= (K <= 24576 ? 4096 : 2048)) return true;
+    if (N > 7168 || M > 1792 || (K > 24576 && N <= 4096)) return false;
+    return M * N <= (N <= 6144 ? 8900000 : 7400000) || (M > 1600 && N > 23 * 256 && N <= 6144 && M * N <= 10500000);
+}
 static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act, bool parts) {
     if (M < TGIS_DENSE_TALL_MIN_M || K < 64 || K % 64 != 0 || N < 1024) return false;
     TallPlan forced;
@@ -563,7 +574,7 @@ static bool dense_tall_pays(int64_t M, int64_t K, int64_t N, int act, bool parts
     if (parts) return M <= 256 && !(K <= 2560 && passes_in_a_round(M, K, N, 128));
     if (M <= 256) return act == 2 || (!passes_in_a_round(M, K, N, 0) && !(gelu && K < 512));
     if (act == 2) return M <= 8192 && (K * N <= (32 << 20) || (M > 512 && N % 4096 != 0));
-    if (K > 16384 && N < 8192 && M <= 2048) return M <= 1792 ? M * N <= 10500000 : cdiv64(M, 256) * cdiv64(N, 256) <= CUS / 2;
+    if (pays_past_16k(M, K, N)) return true;
     if (M > 1400 || K < 512 || M * N > std::min<int64_t>(1500 * K, 6300000)) return false;
     return cdiv64(M, 128) * cdiv64(N, 256) <= CUS / 2 || (K > 9600 && N < 8192);
 }
