@@ -178,10 +178,11 @@ def test_rows_that_the_user_divides(monkeypatch):
     assert streamed == [65] * 3 + [128] * 3
 
 
-# one launch of several products: one, several with a last one that is whole / part of a tile / a narrow one ahead of the others (from 2049 rows on)
+# one launch of several products: one, several with a last one that is whole / part of a tile / a narrow one ahead of the others (past 5000 rows, or 6 M of their outputs)
 @pytest.mark.parametrize("M,K,n_group,N,G,plans", [
     (65, 64, 32, 20, 1, "234"), (129, 448, 96, 288, 3, "234"), (97, 576, 64, 150, 3, "2"), (300, 2048, 512, 2048 + 64, 5, "234"), (257, 128, 160, 470, 3, "4"),
     (2049, 192, 256, 256 + 128, 2, "234"), (2050, 64, 288, 4 * 288 + 33, 5, "234"), (2049, 128, 256, 256 + 129, 2, "3"), (2111, 320, 32, 64, 2, "4"),
+    (5001, 192, 256, 256 + 128, 2, "234"), (5002, 64, 288, 4 * 288 + 33, 5, "234"), (2100, 64, 2880, 2880 + 40, 2, "3"),
 ])
 @pytest.mark.parametrize("width", [1, 2])
 def test_groups(M, K, n_group, N, G, plans, width, monkeypatch):

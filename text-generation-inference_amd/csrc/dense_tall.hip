@@ -266,8 +266,11 @@ __global__ __launch_bounds__(256, 2) void dense_tall_kernel(DTallArgs a) {
 }
 
 // Several products in one launch, each of its own operand, on neighbouring tiles of one image: the tiles of the first, then those of the second, ...
-// NARROW: a last product of up to 128 columns goes first, in tiles of 64 x 128.  (Four 2048 x 2048 and one 2048 x 64, bf16, us, whole tiles behind the others, where
-// they are a round of their own / this: 4096 rows 147 / 140, 3000 118 / 110; below, where the rounds are short, 2045 rows 76.5 / 78.7, 300 22.7 / 25.8.)
+// NARROW: a last product of up to 128 columns goes first, in tiles of 64 x 128: where rows times width make several rounds, a column of whole tiles for it tends to be a
+// round of its own; where they are few it takes the slots of larger tiles.  Four of a width and one of 64, bf16, us, whole tiles behind the others / this: 2048 at 2100, 2500,
+// 3000, 4096 rows 72 / 79, 89 / 95, 111 / 103, 138 / 133; 1024 (of 2048 k) at 2500, 4096, 6000, 8190 48 / 49, 71 / 73, 112 / 104, 140 / 130; 1536 at 3000, 4096 74 / 68, 91 / 86; 512 at 2500, 4096, 8190,
+// 16000 15.5 / 16.4, 18.3 / 24.2, 49 / 35, 76 / 64; 256 at 5000, 16000 11.4 / 15.6, 44 / 32; 65 - 700 rows of any 5 - 70 % slower.  (It follows the rounds no closer than that: over 125 products the
+// line leaves 1.2 % to the better of the two, at most 20.)
 struct TallGroups {
     int n, tiles, narrow;        // products; 32-column tiles of the image to each but the last, which has the rest; blocks of a narrow last product
     int64_t x_group, out_group;  // elements between their operands, their outputs
@@ -636,7 +639,7 @@ struct GroupsPlan {
 };
 static GroupsPlan plan_groups(int64_t M, int64_t K, int64_t N_group, int64_t N, int64_t groups) {
     const int64_t last = N - (groups - 1) * N_group;
-    const bool narrow = groups > 1 && last <= 128 && M > 2048;
+    const bool narrow = groups > 1 && last <= 128 && (M > 5000 || M * N_group > 6000000);
     GroupsPlan best{};
     double best_us = 1e30;
     TallPlan forced;
