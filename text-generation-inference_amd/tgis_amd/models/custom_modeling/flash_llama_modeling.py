@@ -309,8 +309,8 @@ class FlashLlamaLayer:
         # the qkv + rotary launch takes its operand in fragment order when it serves the rows, the MLP when the SiLU * up epilogue does; the norms
         # gather for act-order weights
         qkv_perm = getattr(att.query_key_value.linear, "perm", None)
-        qkv_frag = (kv.slots is not None and cos.shape[1] * 2 == att.head_size and self.hands_fragments(rows, kv)
-                    and frag_rows(att.query_key_value.linear, rows, act=3, gathers=True))
+        qkv_frag = (kv.slots is not None and cos.shape[1] * 2 == att.head_size
+                    and frag_rows(att.query_key_value.linear, rows, act=3, gathers=True) and self.hands_fragments(rows, kv))
         normed_hidden_states, res = self.input_layernorm(hidden_states, residual, frag=qkv_frag, perm=qkv_perm)
         attn_output = att(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv, qkv_perm is not None)
         return self.feed_forward(attn_output, res, kv)
@@ -318,8 +318,8 @@ class FlashLlamaLayer:
     def feed_forward(self, attn_output, res, kv: KVArgs):
         rows = attn_output.shape[0]
         mlp_perm = getattr(self.mlp.gate_up_proj.linear, "perm", None)
-        mlp_frag = (self.mlp.fused_epilogue and self.hands_fragments(rows, kv)
-                    and frag_rows(self.mlp.gate_up_proj.linear, rows, act=2, gathers=True))
+        mlp_frag = (self.mlp.fused_epilogue and frag_rows(self.mlp.gate_up_proj.linear, rows, act=2, gathers=True)
+                    and self.hands_fragments(rows, kv))
         normed_attn_res_output, attn_res = self.post_attention_layernorm(attn_output, res, frag=mlp_frag, perm=mlp_perm)
         mlp_output = self.mlp(normed_attn_res_output, mlp_perm is not None)
         return mlp_output, attn_res
