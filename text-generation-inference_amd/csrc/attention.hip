@@ -847,9 +847,6 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     a.cu_q = cu_seqlens_q;
     a.out = out;
     a.out_cols = out_cols;
-    a.cosb = cos;
-    a.sinb = sin;
-    a.positions = positions;
     a.out_frag = out_cols ? 2 : ld_out == TGIS_LD_FRAGMENTS;
     a.ld_out = (int64_t)H * D;
     attn_set_geom(a, H, Hkv, g);
@@ -881,7 +878,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     // long q (prefill): blocks of 128 columns that stage each K/V page once in LDS (attention_prefill.hip)
     if (num_splits == 1 && long_queries(max_q_len, g)) {
         TgisTimedScope timed(TGIS_OP_ATTN, st);
-        return tgis_launch_attn_prefill(a, B, Hkv, D, max_q_len, dtype, false, st);
+        return tgis_launch_attn_prefill(a, B, Hkv, D, max_q_len, dtype, false, st, cos, sin, positions);
     }
     int64_t q_tiles = cdiv64(max_q_len, g.TQ);
     TGIS_CHECK_ARG(q_tiles <= 2147483647LL && (int64_t)Hkv * a.HCB <= 65535 && B * num_splits <= 65535,

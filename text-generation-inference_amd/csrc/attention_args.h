@@ -23,7 +23,10 @@ struct AttnArgs {
     unsigned* counters;  // fused combine: per-group arrival counters (zero between launches), or nullptr
     int64_t ld_out;  // prefill kernel: elements between two tokens' rows of `out`
     const int32_t* out_cols;  // out_frag 2: output column k is stored as column out_cols[k] (a permutation)
-    const void *cosb, *sinb;  // prefill kernel: q is rotated as it is read, by these tables [position][D / 2] (or nullptr: it is as it is to be)
+};
+// The prefill kernel's.  (Three more fields of its own in AttnArgs cost every launch of the decode kernel 0.05 us: 8 heads of 64 on one at ctx 137 3.94 / 3.99.)
+struct AttnPrefillArgs : AttnArgs {
+    const void *cosb, *sinb;   // q is rotated as it is read, by these tables [position][D / 2] (or nullptr: it is as it is to be)
     const int32_t* positions;  // of the q tokens
 };
 
@@ -55,5 +58,6 @@ static inline void attn_set_geom(AttnArgs& a, int H, int Hkv, const AttnGeom& g)
 }
 
 // prefill kernel launcher (attention_prefill.hip): q, pools, tables, out, scale and geometry of `a`; D 64 or 128; rows: the page layout
-// of attn_varlen.hip
-int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st);
+// of attn_varlen.hip; cos, sin, positions: AttnPrefillArgs
+int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st, const void* cos = nullptr,
+                             const void* sin = nullptr, const int32_t* positions = nullptr);

@@ -47,7 +47,7 @@ constexpr int PREFILL_RING = 4;  // pages in LDS
 // that a score row stands for is chosen so that the probabilities a lane holds are eight neighbours of a value row.
 // CG: 16-column groups per wave (2; 1 where that leaves the chip idle, see the launcher).
 template <typename T, int D, bool ROWS, int CG>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a) {
     using V8 = typename VecT<T>::x8;
     constexpr int KS = D / 32;  // k-steps of the QK^T MFMA
     constexpr int NB = D / 16;  // 16-row blocks of O^T
@@ -335,7 +335,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnArgs a) {
 
 }  // namespace
 
-int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st) {
+int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64_t max_q_len, int dtype, bool rows, hipStream_t st, const void* cos,
+                             const void* sin, const int32_t* positions) {
     TGIS_CHECK_ARG(cdiv64(max_q_len, a.TQ * 4) <= 2147483647LL && (int64_t)Hkv * a.HC <= 65535 && B <= 65535, "tgis_attn_paged: grid too large");
     const int64_t groups = (int64_t)Hkv * a.HC * B;
     // Tiles of 128 columns, or of 64 where those would leave part of the chip idle: of the 512 blocks that are resident at once a quarter may
@@ -346,7 +347,7 @@ int tgis_launch_attn_prefill(const AttnArgs& a, int64_t B, int Hkv, int D, int64
     int cg = groups * cdiv64(max_q_len, a.TQ * 8) < (D == 128 ? 384 : 512) ? 1 : 2;
     if (const char* e = getenv("TGIS_PREFILL_CG")) cg = atoi(e) == 1 ? 1 : 2;  // tuning and test hook
     const int64_t q_tiles = cdiv64(max_q_len, a.TQ * 4 * cg);
-    AttnArgs dealt = a;
+    AttnPrefillArgs dealt{a, cos, sin, positions};
     dealt.xcd_remap = groups % 8 == 0 && (double)q_tiles * groups <= 2147483647.0;
     dim3 grid((unsigned)q_tiles, (unsigned)(Hkv * a.HC), (unsigned)B);
     const size_t lds = (size_t)PREFILL_RING * 2 * 32 * D * 2;  // buffers of (K page + V page)
