@@ -18,7 +18,7 @@ def test_splits(B, Hkv, ctx, splits):
 
 
 @pytest.mark.parametrize("B,Hkv,D,ctx,waves", [
-    (8, 32, 128, 33, 8), (8, 32, 64, 33, 8), (257, 1, 128, 4096, 4), (512, 1, 64, 224, 4), (512, 1, 64, 225, 8), (513, 1, 64, 4096, 4), (769, 1, 128, 4096, 4), (800, 1, 128, 4096, 4),
+    (255, 1, 128, 33, 8), (8, 32, 128, 33, 4), (8, 32, 64, 128, 4), (8, 32, 128, 129, 8), (128, 2, 64, 129, 8), (32, 4, 128, 4096, 8), (257, 1, 128, 4096, 4), (512, 1, 64, 224, 4), (512, 1, 64, 225, 8), (513, 1, 64, 4096, 4), (769, 1, 128, 4096, 4), (800, 1, 128, 4096, 4),
     (895, 1, 128, 4096, 4), (896, 1, 128, 352, 4), (896, 1, 128, 353, 8), (1023, 1, 128, 353, 8), (1023, 1, 128, 200, 4), (1024, 1, 128, 353, 2), (896, 1, 64, 4096, 4), (1536, 1, 128, 4096, 2),
     (1537, 1, 128, 352, 2), (1537, 1, 128, 353, 8), (2047, 1, 128, 353, 8), (2047, 1, 128, 130, 2), (2047, 1, 64, 353, 2), (2048, 1, 128, 353, 4),
 ])
@@ -26,11 +26,11 @@ def test_waves(B, Hkv, D, ctx, waves):
     assert native.load_library().tgis_attn_decode_waves(B, Hkv, Hkv, D, ctx) == waves
 
 
-# B x Hkv groups: 8 waves up to 256; 4 (D 64 from 8 pages on: 8) up to 511, two splits from 48 pages on up to 384; D 128 from 12 pages on 8 at 896 - 1023 and 1537 - 2047,
+# B x Hkv groups: 8 waves up to 256 (256 of up to 4 pages: 4); 4 (D 64 from 8 pages on: 8) up to 511, two splits from 48 pages on up to 384; D 128 from 12 pages on 8 at 896 - 1023 and 1537 - 2047,
 # between and D 64 2
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Hkv,G,D,longest", [
-    (128, 2, 1, 128, 300), (257, 1, 2, 128, 300), (96, 4, 1, 128, 1505), (97, 4, 1, 128, 1505), (511, 1, 1, 64, 225), (512, 1, 1, 64, 225), (513, 1, 1, 64, 225), (511, 1, 1, 64, 224), (128, 3, 4, 64, 1504),
+    (128, 2, 1, 128, 128), (128, 2, 4, 64, 129), (128, 2, 1, 128, 300), (257, 1, 2, 128, 300), (96, 4, 1, 128, 1505), (97, 4, 1, 128, 1505), (511, 1, 1, 64, 225), (512, 1, 1, 64, 225), (513, 1, 1, 64, 225), (511, 1, 1, 64, 224), (128, 3, 4, 64, 1504),
     (128, 3, 4, 64, 1505), (769, 1, 1, 128, 130), (1023, 1, 1, 128, 130), (1024, 1, 1, 128, 130), (1537, 1, 1, 128, 70), (1537, 1, 1, 64, 70), (2047, 1, 1, 128, 33),
     (896, 1, 1, 128, 353), (1023, 1, 1, 128, 353), (1537, 1, 1, 128, 353), (2047, 1, 1, 128, 353),
 ])

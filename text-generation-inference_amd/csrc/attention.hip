@@ -542,6 +542,8 @@ static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && group
 // Waves of a decode block of one chunk.  What is resident decides: of D 128 768 blocks of 4 waves, 1536 of 2 (three waves per SIMD), 512 of 8 (four: their bound on
 // registers), of D 64 more.  (Four waves per SIMD for the smaller blocks as well: equal sequences 7 - 10 % faster at 992 groups, but ragged ones 3 - 7 % slower and
 // 1 - 2 % at 1024, since blocks that wait for a place level what is ragged.  16 waves: 0 - 2 us slower on up to 256 groups.)  us, waves:
+//   256 groups: 8, but 4 up to 4 pages, one each (32 x 8 of D 128, 8 heads on one, at 33, 64, 128, 160 4 / 8: 4.13 / 4.46, 4.03 / 4.31, 4.41 / 4.48, 4.87 / 4.61; 64 x 4 of D 64 at 128, 160
+//     3.76 / 3.99, 5.27 / 4.54; 8 x 32 of D 64 3.85 / 4.16, 4.38 / 4.33)
 //   257 - 512 groups: D 128 4 (352 at ctx 1400 4 / 8: 42.3 / 45.1, ragged 32.0 / 32.8); D 64 8 from 8 pages on, where they share a longer sequence (384 at 600
 //     14.2 / 13.9, ragged 12.8 / 11.7; 512 at 700, 4000 17.8 / 18.1, 78.9 / 80.4, ragged 15.2 / 14.3, 63.6 / 55.9; 384 at 130 8.0 / 8.3); two splits, below, are of 4 waves
 //   896 - 1023 of D 128: 8 from 12 pages on, since 4 leave a second round.  4 / 8, and the mean of five ragged draws: 896 at 200, 256, 400, 1000, 3500 18.0 / 18.0, 20.5 / 20.5, 35.4 /
@@ -553,7 +555,7 @@ static bool wide_decode_blocks(int64_t groups, int ch) { return ch == 1 && group
 //     81.7, 298 / 286; 2000 at 130, 200, 400 28.2 / 30.1, 38.9 / 36.7, 68.7 / 63.2, ragged 19.7 / 22.1, 24.9 / 27.1, 46.8 / 43.1)
 //   from 2048 on 4: past that the dispatch rate, 7 ns per workgroup, costs more than the imbalance
 static int decode_waves(int64_t blocks, int num_splits, int ch, int D, int64_t pages) {
-    if (wide_decode_blocks(blocks / num_splits, ch)) return 8;
+    if (wide_decode_blocks(blocks / num_splits, ch)) return blocks == 256 && num_splits == 1 && pages <= 4 ? 4 : 8;
     if (ch == 1 && num_splits == 1) {
         if (D == 64 && blocks <= 512 && pages >= 8) return 8;
         if (D == 128 && pages >= 12 && ((blocks >= 896 && blocks < 1024) || (blocks > 1536 && blocks < 2048))) return 8;
