@@ -1,5 +1,5 @@
-// Round 4: the PRODUCT's fragment-order int4 GEMM unit (csrc/gptq_wide_body.h, included as is) on arbitrary shapes, with
-// per-wave s_memtime stamps: where does a launch of the 64-row form (MR = 2) spend its time at the Llama-2-70B shapes?
+// The PRODUCT's fragment-order int4 GEMM unit (csrc/gptq_wide_body.h, included as is) on arbitrary shapes and in each of its forms (RB blocks
+// of 16 rows), with per-wave s_memtime stamps: where does a launch spend its time at the Llama-2 shapes?
 //   hipcc --offload-arch=gfx950 -O3 -std=c++17 [-DWIDE_TRACE] -I text-generation-inference_amd/csrc -o tools/floor/wide_unit tools/floor/wide_unit.hip
 //   tools/floor/wide_unit            (random images: timing and timeline only; parity is tests/test_fragments_gpu.py's job)
 #include <hip/hip_runtime.h>
@@ -25,10 +25,10 @@ static __device__ long long* g_wide_trace = nullptr;   // [blocks][8 waves][8]
 #include <string.h>
 #define CK(x) do { hipError_t e = (x); if (e != hipSuccess) { printf("%s: %s\n", #x, hipGetErrorString(e)); exit(1);} } while (0)
 
-template <int CT, int ACT, bool OUTF, int MR>
+template <int CT, int ACT, bool OUTF, int RB>
 __global__ __launch_bounds__(64 * gptq::WIDE_WK) void unit_kernel(gptq::GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gptq::gptq_wide_unit<CT, ACT, OUTF, 2 * MR>(a, smem);
+    gptq::gptq_wide_unit<CT, ACT, OUTF, RB>(a, smem);
 }
 
 static uint64_t rng_state = 0x1234567ull;
@@ -42,8 +42,9 @@ static Image layout(int K, int N, int gs) {
     return im;
 }
 
-template <int CT, int ACT, int MR>
-static void run(const char* name, int K, int N, int S, int M) {
+template <int CT, int ACT, int RB>
+static void run(const char* name, int K, int N, int S, int M = 16 * RB) {
+    constexpr int MR = (RB + 1) / 2;  // 32-row blocks of the operand and of the slabs
     const Image im = layout(K, N, 128);
     const int nsets = (int)std::max<int64_t>(2, (900ll << 20) / im.total);
     std::vector<uint8_t> host(im.total);
@@ -67,8 +68,8 @@ static void run(const char* name, int K, int N, int S, int M) {
     a.G = im.G; a.gs = 128; a.S = S; a.NT = im.NT; a.KS = im.KS; a.slabs = dslabs; a.partial = S > 1;
     a.spg_shift = 1;
     const int cgs = (im.NT + CT - 1) / CT;
-    const size_t lds = gptq::wide_lds_bytes(CT, 2 * MR);
-    auto kern = unit_kernel<CT, ACT, false, MR>;
+    const size_t lds = gptq::wide_lds_bytes(CT, RB);
+    auto kern = unit_kernel<CT, ACT, false, RB>;
     CK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     dim3 grid(cgs, S);
     hipEvent_t e0, e1; CK(hipEventCreate(&e0)); CK(hipEventCreate(&e1));
@@ -109,16 +110,24 @@ static void run(const char* name, int K, int N, int S, int M) {
 }
 
 int main() {
-    run<4, 2, 2>("70B gate_up", 8192, 57344, 1, 64);
-    run<7, 2, 2>("70B gate_up", 8192, 57344, 1, 64);
-    run<8, 2, 2>("70B gate_up", 8192, 57344, 1, 64);
-    run<2, 0, 2>("70B o", 8192, 8192, 2, 64);
-    run<4, 0, 2>("70B o", 8192, 8192, 4, 64);
-    run<2, 0, 2>("70B down", 28672, 8192, 2, 64);
-    run<4, 0, 2>("70B down", 28672, 8192, 4, 64);
-    run<8, 0, 2>("70B down", 28672, 8192, 8, 64);
-    run<3, 2, 2>("7B gate_up", 4096, 22016, 1, 64);
-    run<2, 0, 2>("7B down", 11008, 4096, 4, 64);
-    run<4, 0, 2>("7B down", 11008, 4096, 8, 64);
+    run<4, 2, 4>("70B gate_up", 8192, 57344, 1);
+    run<7, 2, 4>("70B gate_up", 8192, 57344, 1);
+    run<8, 2, 4>("70B gate_up", 8192, 57344, 1);
+    run<2, 0, 4>("70B o", 8192, 8192, 2);
+    run<4, 0, 4>("70B o", 8192, 8192, 4);
+    run<2, 0, 4>("70B down", 28672, 8192, 2);
+    run<4, 0, 4>("70B down", 28672, 8192, 4);
+    run<8, 0, 4>("70B down", 28672, 8192, 8);
+    run<3, 2, 4>("7B gate_up", 4096, 22016, 1);
+    run<2, 0, 4>("7B down", 11008, 4096, 4);
+    run<4, 0, 4>("7B down", 11008, 4096, 8);
+    run<3, 2, 1>("7B gate_up", 4096, 22016, 1);
+    run<3, 2, 2>("7B gate_up", 4096, 22016, 1);
+    run<3, 2, 3>("7B gate_up", 4096, 22016, 1);
+    run<2, 0, 1>("7B o", 4096, 4096, 4);
+    run<2, 0, 2>("7B o", 4096, 4096, 4);
+    run<2, 0, 3>("7B o", 4096, 4096, 4);
+    run<2, 0, 1>("7B down", 11008, 4096, 4);
+    run<2, 0, 3>("7B down", 11008, 4096, 4);
     return 0;
 }
