@@ -2,7 +2,7 @@
  * tgis_hip.h — C ABI of libtgis_hip.so, the MI355X (gfx950) native-kernel library that sits
  * where the reference's CUDA extension modules sit on the batched-decode hot path.
  *
- * Boundary: SURVEY.md §8(b) row #5.  The reference calls pybind/torch-extension functions with
+ * Boundary: the reference calls pybind/torch-extension functions with
  * at::Tensor arguments (flash_attn_2_cuda, dropout_layer_norm, rotary_emb, exllamav2_kernels);
  * this library exposes the same operations behind a plain C ABI: raw device pointers, int64
  * sizes/strides, float scalars and a hipStream_t passed as void*.  No torch types, no allocation
@@ -34,7 +34,7 @@ extern "C" {
 #define TGIS_BF16 1
 #define TGIS_F32 2 /* only where an entry point says so (the fp32-residual / ragged-step family at the end) */
 
-/* KV page geometry (DESIGN.md §3): 32 tokens per page; per (page, k|v, kv_head) one
+/* KV page geometry: 32 tokens per page; per (page, k|v, kv_head) one
  * 32*head_dim element block in an MFMA-fragment-ready order. */
 #define TGIS_KV_PAGE_TOKENS 32
 
@@ -74,7 +74,7 @@ int tgis_timing_read(int op, int64_t* count, double* total_ms);
 /* Bytes of the prepared (repacked) weight image for a [K,N] 4-bit matrix with `groups` groups. */
 int64_t tgis_gptq_prepared_bytes(int64_t K, int64_t N, int64_t groups);
 
-/* Repack GPTQ tensors into the kernel layout (DESIGN.md §3).  One-time, at load
+/* Repack GPTQ tensors into the kernel layout.  One-time, at load
  * (the reference does this in Ex4bitLinearV2.post_init, exllamav2.py:124-137).
  *   qweight [K/8, N] int32, qzeros [groups, N/8] int32, scales [groups, N] f16,
  *   g_idx [K] int32 or NULL (NULL = trivial k / groupsize), perm_out [K] int32 or NULL:
@@ -94,7 +94,7 @@ int tgis_gptq_prepare(const int32_t* qweight, const int32_t* qzeros, const void*
 /* Largest M for which tgis_gptq_gemm_f16 is a fused dequantise + MFMA kernel worth calling (above it the caller
  * dequantises once with tgis_gptq_dequant_t_f16 and uses a library GEMM, exllamav2.py:87 "M > 50"): M <= 64 streams the
  * weights once per pass, 64 < M <= 256 in 64-row passes, and — for K % 64 == 0, group size 64 * 2^n, no act-order, act != 1 —
- * a tall kernel (one dequantisation per 64 - 128 rows, 0.5 - 1.0 PFLOP/s at 500 - 1000 rows of a 7B matrix, 1.0 - 1.1 from 2000, no scratch copy of W) takes over up to
+ * a tall kernel (one dequantisation per 64 - 128 rows, 0.5 - 1.1 PFLOP/s at 500 - 1000 rows of a 7B matrix, 1.1 - 1.25 from 2000, no scratch copy of W) takes over up to
  * 8192 rows: from 257, and from 129 (act 2: 65) where it is done before the passes.  tgis_gptq_gemm_whole_sums: 1 where it does.
  * tgis_gptq_gemm_fused_pays: 0 at row counts up to that largest one where dequantising and a library GEMM is the faster way all the same
  * (some between 3072 and 8192, where 256 x 256 tiles fill their rounds). */
@@ -103,7 +103,7 @@ int tgis_gptq_gemm_whole_sums(int64_t M, int64_t K, int64_t N, int64_t groups, i
 int tgis_gptq_gemm_fused_pays(int64_t M, int64_t K, int64_t N, int64_t groups, int act_order, int act);
 int64_t tgis_gptq_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
 
-/* Activation layout between the decode step's own kernels (round 4).  A leading dimension of TGIS_LD_FRAGMENTS says that a
+/* Activation layout between the decode step's own kernels.  A leading dimension of TGIS_LD_FRAGMENTS says that a
  * [M <= 64, K] f16 activation (K % 64 == 0; the buffer holds ceil(M / 32) * 32 * K elements) is stored in the order the MFMA
  * reads it — [row block m/32][k64-step][i = k/8 % 4][lane = 32 (k/32 % 2) + m % 32][k % 8], i.e. element (m, k) at
  * (m/32) * 32 K + ((k/64 * 4 + k/8 % 4) * 64 + 32 (k/32 % 2) + m % 32) * 8 + k % 8 — instead of row-major.  Producers that can write it:
@@ -141,7 +141,7 @@ int tgis_gptq_gemm_f16_partial(const void* x, int64_t ldx, const void* prepared,
                                int64_t K, int64_t N, int64_t groups, int act, float* slabs, int64_t slabs_bytes,
                                int* num_slabs, int64_t* slab_ld, void* stream);
 
-/* ---- fused qkv projection + rotary embedding + cache write (decode, round 3) ------------------------------------------
+/* ---- fused qkv projection + rotary embedding + cache write (decode) ---------------------------------------------------
  * One launch for `qkv = query_key_value(x)`, `rotary_emb(q, k, cos, sin)` and `layer_past[slot] = (k, v)`
  * (flash_llama_modeling.py:251-268,282) at decode sizes: the GEMM keeps the whole k range in a block (no split-K slabs)
  * and its epilogue rounds the sum (+ bias) to f16, rotates q / k heads in fp32 (the arithmetic of tgis_rope_kv_write) and
@@ -303,7 +303,7 @@ int tgis_layernorm_residual_partial(const float* slabs, int num_slabs, int64_t s
  * (= page_id*32 + offset).  cos == NULL skips the rotation (learned-position models).
  * k_pool / v_pool: this layer's K and V page pools, [num_pages][Hkv][32*D] each.  Inside a (page, kv head) block of
  * 32 tokens x D: K as [token >> 4][D / 8][16 tokens][8], V as [4 column groups][D][8] with token t in column
- * (i >> 2) * 8 + (t >> 4) * 4 + (i & 3), i = t & 15 (csrc/kv_layout.h, DESIGN.md section 3: the orders in which the
+ * (i >> 2) * 8 + (t >> 4) * 4 + (i & 3), i = t & 15 (csrc/kv_layout.h: the orders in which the
  * attention kernels' MFMA fragments are whole cache lines).  The pools are opaque to callers; oracle/ops_ref.py's
  * kv_page_unpack reads them back for tests. */
 int tgis_rope_kv_write(void* qkv, int64_t ld_qkv, const void* cos, const void* sin,

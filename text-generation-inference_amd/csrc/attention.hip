@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * NW) void attn_paged_kernel(AttnArgs a) {
         }
     }
     // (Rotary embedding + cache write of the new token in this prologue was built, bit-exact, and measured slower
-    // than the launch in front: cfg3 104 vs 93 us — experiments/README.md.)
+    // than the launch in front: 32 rows, 32 heads of 128, ctx 1024 104 vs 93 us — experiments/README.md.)
 
     f32x4 o[CH][NB];
     float m[CH], lsum[CH];
@@ -728,7 +728,7 @@ std::mutex g_attn_counters_mu;
 std::map<int, CounterPool> g_attn_counters;
 
 // `slot` receives the index to give back with attn_counters_enqueued() once the launch that uses the array is in its
-// stream (ADVICE r04: between this call and the launch a second host thread could see the new owner's stream idle and take
+// stream (between this call and the launch a second host thread could see the new owner's stream idle and take
 // the same array).
 unsigned* attn_counters(hipStream_t st, int* dev_out, int* slot) {
     *slot = -1;

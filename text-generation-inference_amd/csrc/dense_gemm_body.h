@@ -1,5 +1,5 @@
 // The dense (f16 / bf16 weights) skinny GEMM as a device function (one workgroup = one unit) plus its launch planning; the
-// kernel that runs it is in gemm_dense.hip.  (The persistent decode-tail form of rounds 2 - 5 is gone: experiments/README.md.)
+// kernel that runs it is in gemm_dense.hip.  (A persistent decode-tail form was slower: experiments/README.md.)
 #pragma once
 #include "gptq_gemm_body.h"
 #include "kv_layout.h"
@@ -192,7 +192,7 @@ __device__ __forceinline__ void dense_finish(const DenseArgs& a, const float (&f
 // MR = 32-row blocks of x per pass (2 for M > 32: every weight fragment then feeds two MFMAs; needs WK = 2).
 // R16 (batches of up to 16 rows, MR == 1): only 16 rows of x are staged — half the requests through the CU's address path,
 // half the LDS stores and half the LDS footprint per chunk; lanes 16 - 31 of the A fragment re-read rows 0 - 15 (an LDS
-// broadcast), so accumulator rows 16 - 31 repeat rows 0 - 15 and are never stored.  Round 6: at TinyLlama's widths the
+// broadcast), so accumulator rows 16 - 31 repeat rows 0 - 15 and are never stored.  At TinyLlama's widths the
 // activation is a third to a half of what a block takes in, and rows 16 - 31 of a 16-sequence batch were clamped copies.
 template <typename T, int TN, int WK, int ACT, int MR, bool R16 = false>
 __device__ __forceinline__ void dense_gemm_unit(const DenseArgs& a, const int ntg, const int split, const int mslab,

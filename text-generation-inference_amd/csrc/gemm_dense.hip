@@ -165,7 +165,7 @@ static int launch_dense_variant(int mr, dim3 grid, size_t lds, hipStream_t st, c
         if (mr == 2) return launch_dense_one<T, TN, WK, ACT, 2>(grid, lds, st, a);
     }
     // batches of up to 16 rows stage 16 rows of x (dense_gemm_body.h, R16); the LDS request shrinks with them.  Same box,
-    // 32-row staging patched back in: cfg2 1.066 / 1.067 -> 1.038 / 1.044 ms per step (profiles/r06d_bench_cfg2_rows16_*.json)
+    // 32-row staging patched back in: a 1.1B model, 16 rows, 1.066 / 1.067 -> 1.038 / 1.044 ms per step (profiles/r06d_bench_cfg2_rows16_*.json)
     if (a.M <= 16)
         return launch_dense_one<T, TN, WK, ACT, 1, true>(grid, (size_t)WK * 2 * 16 * DRS * sizeof(T) + 64, st, a);
     return launch_dense_one<T, TN, WK, ACT, 1>(grid, lds, st, a);

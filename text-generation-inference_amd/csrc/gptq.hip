@@ -623,9 +623,9 @@ extern "C" int tgis_gptq_rope_ok(int64_t M, int64_t K, int64_t N, int64_t groups
     // (measured: 7B qkv at 32 rows, 192 blocks: 14.9 vs 17.2 us for the pair; 70B qkv at 64 rows, 80 blocks of 42 MB: +5 % on
     // the step; a TP = 8 shard of the 7B qkv, 24 blocks: +2 % on the rank-step; TinyLlama dense, 40 blocks: +-0).
     // counted in blocks of the kernel that will run it (the fragment-order kernel gives a wave ONE tile where two would
-    // leave fewer than 128 blocks), and up to 32 rows it pays from 48 blocks on — one rank of cfg3 at TP 8 / 4 / 2 (48 / 96 / 192
+    // leave fewer than 128 blocks), and up to 32 rows it pays from 48 blocks on — one rank of a 7B model, 32 rows, at TP 8 / 4 / 2 (48 / 96 / 192
     // one-tile blocks) 1.838 / 2.110 / 3.000 -> 1.815 / 2.072 / 2.903 ms per step; at 64 rows every block takes in twice the
-    // activation and the bar stays at 128 (a cfg4 rank at TP 8, 40 blocks: 6.45 -> 7.10 ms).  profiles/r06_tp_rope_blocks.log
+    // activation and the bar stays at 128 (a rank of a 70B model at TP 8, 40 blocks: 6.45 -> 7.10 ms).  profiles/r06_tp_rope_blocks.log
     const GemmPlan pl = plan_gemm(K, N, 2, M);
     const int64_t blocks = gptq::wide_serves(M, K, N, groups, false) ? gptq::wide_blocks(K, N, 3, M)
                                                                      : cdiv64(cdiv64(N, 32), pl.TN);

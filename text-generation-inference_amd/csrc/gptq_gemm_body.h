@@ -1,6 +1,6 @@
 // The int4 GPTQ streaming GEMM as a device function (one workgroup = one unit) plus its launch planning; the kernel that
-// runs it is in gptq.hip.  (Rounds 2 - 5 also ran this unit inside a persistent "decode tail" launch and with an add +
-// RMSNorm phase in front of it — both measured slower than separate launches and removed in round 6: experiments/README.md.)
+// runs it is in gptq.hip.  (It has also run inside a persistent "decode tail" launch and with an add +
+// RMSNorm phase in front of it — both measured slower than separate launches: experiments/README.md.)
 #pragma once
 #include <stdlib.h>
 #include <algorithm>
@@ -123,7 +123,7 @@ constexpr int RS = KC + 8;  // LDS row stride in halves (+16 B -> conflict-free 
 typedef __attribute__((address_space(3))) int lds_int;  // explicit LDS pointer: a generic one costs vmcnt(0) waits
 
 // A wave keeps RING = 4 one-KiB weight loads (one chunk) and the {scale, zero} words of their k64-steps in flight; a
-// two-chunk ring measured ~1 us SLOWER on every cfg3 shape (the first barrier waits for twice the prologue loads to issue).
+// two-chunk ring measured ~1 us SLOWER on every shape of a 7B layer (the first barrier waits for twice the prologue loads to issue).
 template <int TN, int WK, int ACT, bool GROUP64, bool PERM, int MR>
 __device__ __forceinline__ void gptq_gemm_unit(const GemmArgs& a, const int ntg, const int split, const int mslab,
                                                unsigned char* smem) {
@@ -252,7 +252,7 @@ __device__ __forceinline__ void gptq_gemm_unit(const GemmArgs& a, const int ntg,
     // two accumulators: consecutive MFMAs of a step alternate, halving the dependent-accumulator stalls
     // One accumulator: the ~15 dequantisation instructions between two MFMAs already cover the 32-cycle dependency of
     // consecutive MFMAs on it, and the 16 registers a second (alternating) accumulator took are worth more as occupancy
-    // (round 2, cfg3 decode: 4.93 -> 4.84 ms/step).
+    // (7B, 32 rows, ctx 1024: 4.93 -> 4.84 ms/step).
     constexpr int NACC = 1;
     f32x16 accs[MR][2];
 #pragma unroll

@@ -5,7 +5,7 @@
 //   V: [4 column groups][D][8], token tok in column v_col(tok) = (i>>2)*8 + tile*4 + (i&3), i = tok&15 (column group =
 //      v_col >> 3, slot = v_col & 7) -> a V^T A-fragment (16 rows d x 32 token columns) is four contiguous 256-byte runs of
 //      whole cache lines, and the d run of ONE token (a decode step's write) is 16-byte strided: 16 cache lines per head
-//      where the [D][32] order of rounds 1-3 touched 64 (round 4: the qkv + rotary launch 15.9 -> 12.6 us with cold pages)
+//      where a [D][32] order touches 64 (the qkv + rotary launch 15.9 -> 12.6 us with cold pages)
 #pragma once
 #include "common.h"
 

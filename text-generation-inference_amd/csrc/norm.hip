@@ -58,7 +58,7 @@ __global__ __launch_bounds__(NT) void norm_kernel(const T* x, const T* residual,
         if (c < nchunk) {
             wvs[it] = ld16<V8>(weight + c * 8);
             if (bias) bvs[it] = ld16<V8>(bias + c * 8);
-            // Round 5: the residual and the bias of the GEMM before are requested HERE, in front of the slabs.  Behind them (in
+            // The residual and the bias of the GEMM before are requested HERE, in front of the slabs.  Behind them (in
             // their own basic blocks, after the waits of the slab sum) they were a second and a third dependent round trip to
             // memory in a kernel that is nothing but one round trip.
             V8 b, bv;

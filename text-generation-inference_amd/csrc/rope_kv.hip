@@ -4,7 +4,7 @@
 // custom_modeling/flash_llama_modeling.py:262-263) and the cache writes `layer_past[...] = kv`
 // (flash_llama_modeling.py:268,282).
 //
-// KV page block layout for one (page, kv head), 32 tokens x D elements (DESIGN.md §3):
+// KV page block layout for one (page, kv head), 32 tokens x D elements:
 //   K: [tile=tok>>4][D/8][16 tokens][8]      -> MFMA 16x16x32 A-fragments are 1 KiB contiguous loads
 //   V: [4 column groups][D][8], token tok in column (i>>2)*8 + tile*4 + (i&3), i = tok&15 (kv_layout.h)
 #include <algorithm>

@@ -1,5 +1,5 @@
 """Engine plugin loader: `tgis_amd.inference_engine.<DEPLOYMENT_FRAMEWORK>` must export `InferenceEngine`
-(mirrors inference_engine/__init__.py:7-9 of the reference — drop-in boundary #3 of SURVEY.md §8b)."""
+(mirrors inference_engine/__init__.py:7-9 of the reference)."""
 import importlib
 
 

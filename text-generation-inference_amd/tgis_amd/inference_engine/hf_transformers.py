@@ -1,6 +1,6 @@
 """Engine plugin `hf_transformers`: the model is whatever `AutoModelForCausalLM.from_pretrained` builds from a local
 checkpoint directory, on the device of this rank (CPU when there is no GPU) — the engine behind the padded `CausalLM`
-path and BASELINE config 1 (mirrors inference_engine/hf_transformers.py:11-78 of the reference).
+path (mirrors inference_engine/hf_transformers.py:11-78 of the reference).
 
 Not offered here: `bitsandbytes` / AutoGPTQ loading (neither library is in the image; int4 GPTQ is served by the
 `tgis_native` engine on the HIP kernels) and the `hf_accelerate` device maps."""
@@ -16,7 +16,7 @@ class InferenceEngine(BaseInferenceEngine):
     def __init__(self, model_path: Optional[str], model_class, dtype: torch.dtype, quantize: Optional[str],
                  model_config: Optional[Any], max_sequence_length: Optional[int] = None, *, preloaded=None,
                  tokenizer=None) -> None:
-        """`preloaded` (an already constructed HF model) replaces the checkpoint read: tests and the cfg1 benchmark
+        """`preloaded` (an already constructed HF model) replaces the checkpoint read: tests and the GPT-2 benchmark
         build seeded random models in memory, there are no checkpoint files offline."""
         if preloaded is not None and model_config is None:
             model_config = preloaded.config

@@ -1,6 +1,6 @@
 """Engine for seeded synthetic checkpoints held in memory (benchmarks, smoke and parity tests): same model
 classes, same `Weights` interface and TP slicing as tgis_native, no files and no tokenizer download.
-The weight recipe is the one SURVEY.md §8(d) defines (N(0, 0.02) dense; GPTQ: random nibbles, random zero nibbles in 0..13,
+The weights are N(0, 0.02) (dense; GPTQ: random nibbles, random zero nibbles in 0..13,
 scales U(0.5,1.5)*2/15*0.02, g_idx = k // group) — there is no network for real checkpoints."""
 import os
 from typing import Any, Dict, Optional

@@ -1,6 +1,5 @@
 """The native engine: model type -> MI355X model class, process group, safetensors `Weights`, GPTQ params
-(mirrors inference_engine/tgis_native.py:23-139 of the reference; model families of the configs in
-llama, and gpt_bigcode when flash_santacoder_modeling is present)."""
+(mirrors inference_engine/tgis_native.py:23-139 of the reference; model families: llama, and gpt_bigcode when flash_santacoder_modeling is present)."""
 import os
 from typing import Any, Optional
 

@@ -5,7 +5,7 @@ models/__init__.py:31-166 that concern this build's two paths).
   visible and the model family has a flash implementation.  As in the reference (:81-114) it always runs on the
   `tgis_native` engine; another `deployment_framework` is overridden with a warning.
 * padded path (`CausalLM` on the engine plugin named by `deployment_framework`, e.g. `hf_transformers`): everything
-  else that HF can load as a causal LM — BASELINE config 1 and any CPU run."""
+  else that HF can load as a causal LM — GPT-2 on the CPU and any CPU run."""
 import json
 import os
 from typing import Optional

@@ -1,8 +1,8 @@
 """CausalLMBatch + CausalLM: the padded (rectangular) batch path on a HF `AutoModelForCausalLM`.
 
 This is the reference's plumbing path (models/causal_lm.py: batch fields :21-57, `from_pb` :65-216, `concatenate`
-:218-461, `prune` :463-526, `CausalLM.forward` :604-634, `generate_token` :636-739) — BASELINE config 1 (GPT-2 small,
-fp32, CPU) and the path the parity oracle was captured from.  It is host code around a library model, on whatever
+:218-461, `prune` :463-526, `CausalLM.forward` :604-634, `generate_token` :636-739) — GPT-2 small in fp32 on the
+CPU, and the path the parity oracle was captured from.  It is host code around a library model, on whatever
 device the engine chose; it is NOT a fallback of the flash path (FlashCausalLM still refuses to run without the HIP
 library).
 

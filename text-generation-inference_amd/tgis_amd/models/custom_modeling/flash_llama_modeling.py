@@ -110,7 +110,7 @@ class KVArgs:
                        cu_seqlens_q=torch.arange(B + 1, dtype=torch.int32, device=self.ends.device))
 
 
-# (The persistent decode tail, the rope-in-attention launch and the norm-as-a-GEMM-phase launches of rounds 2 and 3 were all
+# (The persistent decode tail, the rope-in-attention launch and the norm-as-a-GEMM-phase launches were all
 # measured slower than the launches they replace: experiments/README.md is their ledger.)
 
 

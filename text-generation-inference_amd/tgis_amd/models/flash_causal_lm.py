@@ -5,7 +5,7 @@ Mirrors models/flash_causal_lm.py of the reference: batch fields and `from_pb` (
 (:462-588).  Same names, same argument meaning, same returned tuple, same logical bookkeeping
 (`cu_seqlens`, `cu_seqlens_q`, `max_seqlen`, `position_ids`, `all_input_ids_tensor`, `input_lengths`).
 
-What is different by design (DESIGN.md §2):
+What is different by design:
   * `past_key_values` is always None: KV lives in the model's PagedKVCache and a batch owns a list of page
     ids per request.  The reference re-concatenates the whole KV tensor on every decode step for B > 1
     (:439-447) and on every concatenate/prune; here those are page-table edits.
@@ -368,7 +368,7 @@ class LiveSequence:
 FRESH_PREFILL_KV = os.getenv("TGIS_PREFILL_KV", "true").lower() not in ("0", "false")
 
 
-# A captured decode step serves every batch size of its BUCKET (round 6): the rows past the batch are inactive — position 0,
+# A captured decode step serves every batch size of its BUCKET: the rows past the batch are inactive — position 0,
 # every table entry the pool's null page (utils/kv_cache.py), their token written there and attended to alone, their ids
 # never read.  A router that lets a batch wander over 24..32 requests then replays ONE graph instead of capturing nine (a
 # capture is a warm-up step + the capture itself: tens of ms in the middle of serving; bench.py --churn reports them).

@@ -1,6 +1,6 @@
 """ctypes binding of libtgis_hip.so (include/tgis_hip.h) for torch tensors on an MI355X.
 
-This is the drop-in boundary #5 of SURVEY.md §8(b): where the reference imports CUDA extension modules
+This stands where the reference imports CUDA extension modules
 (`flash_attn_2_cuda`, `dropout_layer_norm`, `rotary_emb`, `exllamav2_kernels`; utils/flash_attn.py:23,
 utils/layers.py:361,403-404, utils/gptq/exllamav2.py:7) this module loads one C-ABI shared library and
 passes raw device pointers, sizes and the current HIP stream.  There is no CPU or eager-torch fallback:

@@ -1,4 +1,4 @@
-"""Prompt-prefix ("soft prompt") cache for decoder-only models: SURVEY.md §8(f) row 4.
+"""Prompt-prefix ("soft prompt") cache for decoder-only models.
 
 Behaviour follows the reference's `prompt_cache.py:145-462` as seen by `FlashCausalLMBatch.from_pb`
 (`flash_causal_lm.py:97-107,157-168`) and the `PrefixLookup` RPC (`server.py:86-103`):
@@ -14,7 +14,7 @@ Behaviour follows the reference's `prompt_cache.py:145-462` as seen by `FlashCau
 * `return_zero` (ranks > 0 of a tensor-parallel embedding that reduces later) yields a zero tensor of the same shape
   so that the all-reduce adds the prefix once — `models/model.py:76-82`, `prompt_cache.py:332-347`.
 
-Encoder-decoder prefixes (`encoder.pt`) are outside the hot path (SURVEY.md §8: decoder-only flash models) and are
+Encoder-decoder prefixes (`encoder.pt`) are outside the hot path (decoder-only flash models) and are
 rejected.  The LRU is an `OrderedDict` guarded by one lock; loads from disk happen outside the lock, as in the
 reference, so a slow disk never blocks lookups of cached ids."""
 import logging

@@ -1,5 +1,5 @@
 """The shard: gRPC `generate.v1.TextGenerationService` on `unix://{uds_path}-{rank}`, driven by the unmodified Rust
-router (drop-in boundary #1).  Mirrors server.py:65-231,251-460 of the reference:
+router.  Mirrors server.py:65-231,251-460 of the reference:
 
 * Prefill: prune `to_prune` batches, build the batch with `batch_type.from_pb`, `generate_token(first=True,
   for_concat=len(cache) > 0)`, cache it unless it is the healthcheck batch (id 2^64-1);

@@ -10,12 +10,12 @@ Design cue for paging: models/paged_causal_lm.py:300-348 (block size 16 there; 3
 Where a sequence's pages sit in the pool.  The decode attention's blocks walk their sequences' pages in step, so what the
 chip reads at one instant is "page p of every sequence of the batch".  The pool hands out its LOWEST free ids and a batch deals
 what it takes PAGE-MAJOR over its sequences (FlashCausalLMBatch.allocate_pages): on a pristine pool those rows are dense runs
-(cfg3: 80.7 us per launch against 82.6 for a random order and 88-92 for a sequence's pages side by side,
+(32 rows, 32 heads of 128, ctx 1024: 80.7 us per launch against 82.6 for a random order and 88-92 for a sequence's pages side by side,
 profiles/r05_attn_page_order.log), and a finished sequence's column of ids is the next one out, so the request that replaces
-it inherits it.  Round 6 measured what churn does to that (bench.py --churn, profiles/r06_churn_cfg3.json: requests leaving
+it inherits it.  What churn does to that (bench.py --churn, profiles/r06_churn_cfg3.json: requests leaving
 and joining every 4-8 steps on a pool aged by random allocations and frees): decode p50 4.149 ms against 4.144 ms on the
 pristine pool — lowest-id-first dealing over the holes of an aged pool is still mostly dense.  A channel-aware free list
-(one heap per page-id residue class, page p of sequence b from class (b + p) mod C — VERDICT r05 item 2a) was built and
+(one heap per page-id residue class, page p of sequence b from class (b + p) mod C) was built and
 measured on aged pools for C = 2 .. 128 at five shapes: never better than this one, 1-4 % worse for several C
 (profiles/r06_page_classes.log; the allocator lives on in tools/attn_page_order.py), so it is not here.
 """
