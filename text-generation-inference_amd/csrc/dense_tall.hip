@@ -10,8 +10,8 @@
 //
 // Products by the 16x16x32 instruction: under the card's power limit it does more than 32x32x16 (bare loops on random values, PFLOP/s: bf16 2.10 against 1.77, f16
 // 1.95, 1.71).  us, 32x32x16 / now: 2048 x 11264 with SiLU at 1024, 1393, 4096 rows 55.9 / 53.2, 65.2 / 60.8, 173 / 160; 4096 x 22016 with SiLU at 2048 327 / 305;
-// 6144 x 24576 at 400 165 / 156; where a SIMD has one wave, twice the products to issue cost 2 - 6 % of tiles of 256 columns (24576 x 6144 at 128 rows 307 / 321),
-// which no plan takes there.
+// 6144 x 24576 at 400 165 / 156; where a SIMD has one wave, twice the products to issue cost 2 - 6 % of tiles of 256 columns (24576 x 6144 at 128 rows 307 / 321):
+// of the plans those of 193 - 256 rows of some 20000 columns and more (4096 x 22016 with SiLU at 256, 172 tiles, 63.0 / 64.0; 4096 x 28672 at 224 72.2 / 74.2).
 //
 // Bound: the matrix cores and their power from about 1000 rows on (1.15 - 1.35 PFLOP/s; with nothing to load 1.55 - 1.9, with the weights in L1 1.3 - 1.6, with no x
 // 1.25 - 1.5), before that the weights' way from HBM and the latency of the blocks' serial chains: hence the choice of tiles, and the split of a last round's tiles
