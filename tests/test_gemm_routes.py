@@ -43,11 +43,13 @@ def test_int4_tall(M, K, N, act, whole):
     assert lib.tgis_gptq_gemm_whole_sums(M, K, N, K // 32, 0, act) == 0   # groups shorter than a k64-step
 
 
-# past 3072 rows: row counts at which 256 x 256 tiles fill their rounds of 256, or most of a single one over a long k, and others
+# past 3072 rows: row counts at which 256 x 256 tiles fill their rounds of 256 and are dealt evenly, or most of a single one over a long k, and others
 @pytest.mark.parametrize("M,K,N,act,pays", [
     (257, 4096, 12288, 0, 1), (3072, 11008, 4096, 0, 1), (4096, 11008, 4096, 0, 0), (4097, 11008, 4096, 0, 1), (8192, 4096, 12288, 0, 0), (6000, 4096, 12288, 0, 1),
     (3841, 4096, 4096, 0, 0), (3840, 4096, 4096, 0, 0), (3584, 4096, 4096, 0, 1), (7168, 11008, 4096, 0, 1), (8192, 13824, 5120, 0, 1), (5120, 5632, 2048, 0, 0),
     (4864, 5632, 2048, 0, 1), (4865, 5632, 2048, 0, 0), (5120, 5056, 2048, 0, 1), (8192, 4096, 22016, 2, 1), (8193, 4096, 22016, 2, 0), (8193, 4096, 4000, 0, 0),
+    (4800, 8192, 10240, 0, 1), (4376, 8192, 10240, 0, 0), (5700, 8192, 8192, 0, 1), (6500, 7168, 7168, 0, 1), (6700, 7168, 7168, 0, 0), (7203, 5120, 15360, 0, 1), (6000, 13824, 5120, 0, 1),
+    (6264, 13824, 5120, 0, 0), (7459, 14336, 4096, 0, 1), (7459, 11008, 4096, 0, 0), (6000, 5120, 5120, 0, 0),
 ])
 def test_int4_library(M, K, N, act, pays):
     from tgis_amd import native

@@ -229,8 +229,8 @@ __global__ __launch_bounds__(256) void gptq_dequant_kernel(const uint8_t* __rest
 
 // The same as [N][K], a column's k together: the operand that the library's products of large M are at their best with (TN).  f16, us, the product alone with
 // [K][N] / [N][K]: 16128 rows of 4096 x 12288 1272 / 1105, 4096 x 4096 423 / 363, 4096 x 22016 2333 / 2053, 11008 x 4096 1108 / 969; 16 prompts of 1008
-// tokens through 32 int4 layers of 4096, 11008 193.6 / 172.3 ms.  (Of the sizes that go to the library one is the other way round: 13824 x 5120 at 6000 rows
-// 945 / 982 with the expansion.)  A workgroup takes 512 k of a tile: 8 KiB of the image, 32 k of a column per lane, and through LDS, so that a column leaves
+// tokens through 32 int4 layers of 4096, 11008 193.6 / 172.3 ms.  (Where blocks of the library's have not as many of its tiles each, [N][K] is up to 20 %
+// the slower one, and up to 8192 rows the kernel of gptq_tall.hip before both.)  A workgroup takes 512 k of a tile: 8 KiB of the image, 32 k of a column per lane, and through LDS, so that a column leaves
 // in a KiB without a gap.  Bound by the bytes: 4096 x 12288 30.4 / 25.4, 4096 x 22016 47.2 / 37.8, 8192 x 57344 238 / 203, 4096 x 4096 11.0 / 9.1.
 constexpr int DQT_K = 512;
 __global__ __launch_bounds__(256) void gptq_dequant_t_kernel(const uint8_t* __restrict__ prep, int64_t offB, f16* __restrict__ wout, int K, int N,

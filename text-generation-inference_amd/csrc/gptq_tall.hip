@@ -554,24 +554,28 @@ bool gptq::tall_serves(int64_t K, int64_t groups, bool act_order, int act) {
     const int64_t gs = K / groups, spg = gs / 64;
     return groups == 1 || (gs % 64 == 0 && (spg & (spg - 1)) == 0);
 }
-// Between 3072 and tall_max_m() rows it depends on how full the library's 256 x 256 tiles leave their rounds of 256.  act 0, us, dequantise
-// ([N][K]) and library / this kernel, weights cold:
-//   93 % full and more:  5120 x 15360 at 4096, 6000, 8190 487 / 534, 713 / 768, 945 / 1029; 11008 x 4096 at 4096, 8190 269 / 298, 514 / 591; 8192 x
-//                        10240 at 6000, 8190 739 / 819, 957 / 1067; 4096 x 12288 at 4096, 5225, 8190 310 / 335, 410 / 432, 589 / 665 (but 13824 x 5120
-//                        at 6000 984 / 706)
-//   less:                4096 x 12288 at 6000 602 / 494; 11008 x 4096 at 5225, 7168 663 / 417, 561 / 546; 8192 x 10240 at 3500, 4096, 5225, 7168 629 / 491,
-//                        717 / 545, 833 / 722, 999 / 951; 13824 x 5120 at 3500, 5225, 8190 775 / 419, 897 / 620, 1067 / 917; 28672 x 8192 at 5225,
-//                        7168 2504 / 1990, 3224 / 2712; but also 4096 x 12288 at 3500 295 / 317, 4096 x 4096 at 7168 185 / 212, 8192 x 8192 at 5225,
-//                        7168 542 / 573, 705 / 757: which of its kernels the library takes there follows no rule of sizes
-//   one round, from three fifths on, of long k:  11008 x 4096 at 3500 248 / 277; 8192 x 3072 at 4096, 5000 183 / 197, 210 / 216 (5632 x 2048 at 4096,
-//                        half a round, 97 / 87)
+// Between 3072 and tall_max_m() rows it depends on the library's 256 x 256 tiles: whether they fill their rounds of 256, and each block has as many of them (rounds that
+// do not divide the tiles, up to ten, send the library to kernels that take 1.2 to 1.5 times as long).  act 0, us, dequantise ([N][K]) and library / this kernel, weights cold:
+//   93 % full and dealt evenly:  5120 x 15360 at 4096, 6000, 8190 481 / 529, 704 / 769, 936 / 1021; 11008 x 4096 at 4096, 7476, 8190 262 / 299, 476 / 545, 498 / 587; 8192 x 10240 at 4376, 6000,
+//                        8190 544 / 602, 729 / 806, 933 / 1072; 4096 x 12288 at 4096, 5225, 8190 297 / 332, 401 / 430, 572 / 656; 7168 x 7168 at 6711 (756 tiles) 486 / 554; 13824 x 5120 at 6264
+//                        (500) 620 / 697
+//   93 % full, not evenly:  8192 x 10240 at 4728 (760 tiles) 827 / 614; 8192 x 8192 at 5683 (736) 758 / 604; 7168 x 7168 at 6409 (728) 684 / 530; 17920 x 6656 at 7206 (754) 1687 / 1368; 5120 x
+//                        15360 at 7203 (1740) 972 / 884.  Of 1640 drawn products this kernel takes 0.86 of the time, at three rounds 0.78, and 79 are more than 2 % behind, at most 10
+//   two rounds 93 - 95 % full past k of 13056:  13824 x 5120 at 6000 976 / 681; 14336 x 4096 at 7459 1028 / 714; 28672 x 8192 at 3625 1728 / 1404 (291 drawn: 0.75)
+//   less:                4096 x 12288 at 6000 580 / 482; 11008 x 4096 at 5225 672 / 402; 8192 x 10240 at 3500, 4096, 5225 623 / 490, 716 / 530, 813 / 714; 13824 x 5120 at 3500, 5225, 8190 772 /
+//                        417, 891 / 601, 1060 / 898; 28672 x 8192 at 5225, 7168 2499 / 1964, 3247 / 2706; but also 4096 x 12288 at 3500 279 / 306, 4096 x 4096 at 7168 183 / 206, 8192 x 8192 at 5225,
+//                        7168 537 / 572, 705 / 746, which are dealt evenly too (672, 448, 672, 896 tiles)
+//   one round, from three fifths on, of long k:  11008 x 4096 at 3500 245 / 273; 8192 x 3072 at 4096, 5000 169 / 199, 180 / 207 (5632 x 2048 at 4096,
+//                        half a round, 86 / 87)
 // With SiLU * up this kernel is in front of the library and its activation launch (4096 x 22016 at 4096, 8190 rows 740 / 611, 1291 / 1207; 2048 x
 // 11264 198 / 178, 421 / 333; 8192 x 57344 at 2045, 3500 1598 / 1514, 2666 / 2662, but at 4096, 8190 2889 / 3027, 5632 / 6084).
 bool gptq::tall_before_library(int64_t M, int64_t K, int64_t N, int act) {
     if (M <= 3072 || act == 2 || getenv("TGIS_TALL_MAX_M")) return M <= tall_max_m();
     const int64_t tiles = cdiv64(M, 256) * cdiv64(N, 256), slots = cdiv64(tiles, CUS) * CUS;
-    const bool full = 100 * tiles >= 93 * slots, long_round = tiles <= CUS && 10 * tiles > 6 * CUS && K >= 5120;
-    return M <= tall_max_m() && !full && !long_round;
+    const int64_t rounds = slots / CUS;
+    const bool evenly = (tiles % rounds == 0 || rounds > 10) && !(rounds == 2 && 100 * tiles < 95 * slots && K > 13056);
+    const bool long_round = tiles <= CUS && 10 * tiles > 6 * CUS && K >= 5120;
+    return M <= tall_max_m() && !(evenly && 100 * tiles >= 93 * slots) && !long_round;
 }
 // Up to 256 rows the passes take k in parallel (k-parts, splits) where a tile here walks it alone, so it depends on the matrix which of
 // the two is done first.  us, the passes with the launch that adds their slabs / this kernel with a norm behind it (act 2: either alone):
