@@ -294,14 +294,17 @@ class FlashLlamaLayer:
                                             eps=config.rms_norm_eps)
         self.post_attention_layernorm = LlamaRMSNorm(prefix=f"{prefix}.post_attention_layernorm", weights=weights,
                                                      eps=config.rms_norm_eps)
+        self.int4 = hasattr(self.self_attn.query_key_value.linear, "wants_fragments")
 
     def hands_fragments(self, rows: int, kv: KVArgs) -> bool:
         """Whether the norms may hand the int4 GEMMs of up to 64 rows their operands in fragment order (native.FragAct): decode steps, and prompts but
         for those whose row-major fused qkv launch pays.  us, rows / fragments: a 7B model's prompts of 40 rows 3000 / 2660, two of 32 3223 / 2866, 60 in
         act order 3130 / 2822, four 70B layers' of 12, 48 868 / 801, 1069 / 1001; but a 7B model's of 16, 30 rows, the host's time either way, 2647 / 2668,
         2652 / 2692."""
+        if rows > 64 or not self.int4:
+            return False
         return ((kv.max_q_len == 1 and not kv.fresh_prefill)
-                or not native.rope_gemm_pays_for_prompts(rows, getattr(self.self_attn.query_key_value.linear, "rope_handle", None)))
+                or not native.rope_gemm_pays_for_prompts(rows, self.self_attn.query_key_value.linear.rope_handle))
 
     def forward(self, hidden_states, residual, cos, sin, position_ids, cu_seqlens_q, kv: KVArgs):
         rows = hidden_states.shape[0]
@@ -309,8 +312,8 @@ class FlashLlamaLayer:
         # the qkv + rotary launch takes its operand in fragment order when it serves the rows, the MLP when the SiLU * up epilogue does; the norms
         # gather for act-order weights
         qkv_perm = getattr(att.query_key_value.linear, "perm", None)
-        qkv_frag = (kv.slots is not None and cos.shape[1] * 2 == att.head_size
-                    and frag_rows(att.query_key_value.linear, rows, act=3, gathers=True) and self.hands_fragments(rows, kv))
+        qkv_frag = (self.hands_fragments(rows, kv) and kv.slots is not None and cos.shape[1] * 2 == att.head_size
+                    and frag_rows(att.query_key_value.linear, rows, act=3, gathers=True))
         normed_hidden_states, res = self.input_layernorm(hidden_states, residual, frag=qkv_frag, perm=qkv_perm)
         attn_output = att(normed_hidden_states, cos, sin, position_ids, cu_seqlens_q, self.layer_id, kv, qkv_perm is not None)
         return self.feed_forward(attn_output, res, kv)
@@ -318,8 +321,8 @@ class FlashLlamaLayer:
     def feed_forward(self, attn_output, res, kv: KVArgs):
         rows = attn_output.shape[0]
         mlp_perm = getattr(self.mlp.gate_up_proj.linear, "perm", None)
-        mlp_frag = (self.mlp.fused_epilogue and frag_rows(self.mlp.gate_up_proj.linear, rows, act=2, gathers=True)
-                    and self.hands_fragments(rows, kv))
+        mlp_frag = (self.hands_fragments(rows, kv) and self.mlp.fused_epilogue
+                    and frag_rows(self.mlp.gate_up_proj.linear, rows, act=2, gathers=True))
         normed_attn_res_output, attn_res = self.post_attention_layernorm(attn_output, res, frag=mlp_frag, perm=mlp_perm)
         mlp_output = self.mlp(normed_attn_res_output, mlp_perm is not None)
         return mlp_output, attn_res
