@@ -233,6 +233,24 @@ int tgis_dense_rows_norm_silu(const float* h, const void* norm_w, float eps, con
                               int64_t K, int64_t N, int dtype, void* stream);
 int tgis_dense_rows_norm_head(const float* h, const void* norm_w, float eps, const void* prepared, float* out, int64_t ldo, int64_t M,
                               int64_t K, int64_t N, int dtype, void* stream);
+/* The same for up to 32 rows in bf16, by the matrix instruction, K up to 12288, where it norms 4096 (up to 16 rows) or 2048.  The stream between the launches is T(h),
+ * T(h * norm_w) of the norm weight that is next, and sums: the sums of h^2 of eight columns each, h in fp32, as [width / 32][32 rows][4].  These, x of `residual` and
+ * the output of `norm_silu` are in 32-row fragment order (TGIS_LD_FRAGMENTS); rows past M are left alone.
+ *   tgis_dense_rows16_embed       the stream of M tokens (zeros for an id outside the vocabulary)
+ *   tgis_dense_rows16_residual    h = T(x W^T) + T(h), norm_w that of the norm behind it; N (the width) a multiple of 64
+ *   tgis_dense_rows16_norm_*      of T(h * norm_w) and its sums: products times rsqrt(mean h^2 + eps), from there as above; norm_silu: N / 2 a multiple of 64 */
+int tgis_dense_rows16_ok(int64_t M, int64_t K, int norm);
+int tgis_dense_rows16_embed(const int64_t* ids, const void* table, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
+                            int64_t vocab, void* stream);
+int tgis_dense_rows16_residual(const void* x, const void* prepared, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
+                               int64_t N, void* stream);
+int tgis_dense_rows16_norm_rope(const void* hw, const float* sums, float eps, const void* prepared, const void* bias, const int32_t* positions,
+                                const int32_t* slots, const void* cos, const void* sin, void* q_out, int64_t ldq, void* k_pool, void* v_pool,
+                                int64_t M, int64_t K, int64_t H, int64_t Hkv, int64_t D, void* stream);
+int tgis_dense_rows16_norm_silu(const void* hw, const float* sums, float eps, const void* prepared, void* out, int64_t M, int64_t K, int64_t N,
+                                void* stream);
+int tgis_dense_rows16_norm_head(const void* hw, const float* sums, float eps, const void* prepared, float* out, int64_t ldo, int64_t M, int64_t K,
+                                int64_t N, void* stream);
 
 /* ---- dense skinny GEMM (replaces F.linear / torch.mm at decode sizes, utils/layers.py:110-111,
  *      lm_head utils/layers.py:261) -------------------------------------------------------------- */

@@ -1,4 +1,4 @@
-// Dense products of a decode step of a few rows (up to 4) with the norm in front of them and the residual add behind them.
+// Dense products of a decode step of a few rows (up to 4; in bf16 up to 32, below) with the norm in front of them and the residual add behind them.
 //
 // A layer of a small model at one row is seven dependent launches of 3.5 - 11 us for 88 MB of weights, 14 us at the rate of a large copy: split sums
 // that a norm launch adds up, norms of one row on one CU, and projections of 64 column tiles that leave three quarters of the chip idle.  For
@@ -12,6 +12,7 @@
 // The values and their roundings are those of the launches replaced (norm.hip, dense_finish in dense_gemm_body.h); sums are fp32 in another order.
 #include <algorithm>
 #include "common.h"
+#include "gptq_gemm_body.h"
 #include "kv_layout.h"
 
 namespace {
@@ -39,8 +40,8 @@ struct RowsArgs {
     int H, Hkv, D;
 };
 
-// v summed over the lanes with the same lane % 8, in every one of them
-__device__ __forceinline__ float sum_of_eighths(float v) {
+// v summed over the lanes with the same lane % 16, in every one of them
+__device__ __forceinline__ float sum_of_quarters(float v) {
     const uint32_t x = __builtin_bit_cast(uint32_t, v);
     const auto a = __builtin_amdgcn_permlane32_swap(x, x, false, false);
     const uint32_t a0 = a[0], a1 = a[1];
@@ -48,7 +49,11 @@ __device__ __forceinline__ float sum_of_eighths(float v) {
     const uint32_t y = __builtin_bit_cast(uint32_t, v);
     const auto b = __builtin_amdgcn_permlane16_swap(y, y, false, false);
     const uint32_t b0 = b[0], b1 = b[1];
-    v = __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
+    return __builtin_bit_cast(float, b0) + __builtin_bit_cast(float, b1);
+}
+// v summed over the lanes with the same lane % 8, in every one of them
+__device__ __forceinline__ float sum_of_eighths(float v) {
+    v = sum_of_quarters(v);
     return v + row_moved<0x128>(v);
 }
 
@@ -284,6 +289,323 @@ int launch_rows(const RowsArgs& a, int dtype, hipStream_t st) {
 #undef TGIS_ROWS
 }
 
+// ---- up to 16 RB rows in bf16, on the matrix instruction ----
+// The same five launches with v_mfma_f32_16x16x32: sixteen weight columns are its rows, the batch its columns.  A unit is sixteen columns c0 .. +7 and c0 + 16 .. +23 of
+// a tile (ROPE, SILU, HEAD), or eight columns whose two halves of a k64-step lie beside each other (RESIDUAL: each half is multiplied by its own x, and the halves that met
+// the other's x are never read).  Nobody shares x: the waves of a workgroup split the k range, and a wave reads x of its own k64-steps straight into the operand's registers;
+// a workgroup keeps it and takes units in turn.
+// What bounds these launches is each workgroup's own copy of x beside its share of the weights, so
+//   * x is 16 bits: behind a sum of the stream h (fp32 in registers) RESIDUAL leaves T(h), which the next sum adds to, T(h w) of the norm weight
+//     behind it, and the sums of h^2 of its eight columns.  The norm's 1 / rms is a factor of the finished sums; an operand is rounded once either way.  (h itself in
+//     fp32, normed by each workgroup: 16 rows of a 1.1B model 890 us a step for 850 at two units on their way.)
+//   * x is in fragment order (xf_off): a load is four runs of 256 bytes.  From rows of x, whose cache lines the same loads take by halves, that step took
+//     1056 us in the place of 890;
+//   * a wave has one unit, or one k64-step of RESIDUAL, on its way, not more: gate | up of 2048 x 11264 at 16 rows with one, two, three units 9.9 / 11.2 / 11.1 us (the other
+//     waves of the CU ask meanwhile), the residual products with one, two, four steps 6.2 / 6.4 / 7.2.  Fewer units a workgroup than fill one round of 256 take x in more often: one
+//     11.1, two 11.5, three 9.9.
+// bf16 only: T(h w) has its range.
+constexpr int STREAM_ROWS = 32;
+struct Rows16Args {
+    const bf16* x;       // T(h w) or an activation, fragment order
+    const float* sums;   // [K / 32][32 rows][4]: sums of h^2 of eight columns each
+    float eps;
+    const uint8_t* prep;
+    int M, K, N, NT;
+    void* out;
+    int64_t ldo;
+    // RESIDUAL: the stream behind it
+    const bf16* norm_w;
+    bf16 *h, *hw;        // T(h), T(h w), fragment order
+    float* sums_out;
+    // ROPE (as tgis_dense_gemm_rope)
+    const bf16* bias;
+    const int32_t *positions, *slots;
+    const bf16 *cosb, *sinb;
+    bf16 *kpool, *vpool;
+    int H, Hkv, D;
+};
+__device__ __forceinline__ int64_t sums_off(int m, int k) { return ((int64_t)(k >> 5) * STREAM_ROWS + m) * 4 + ((k >> 3) & 3); }
+
+__global__ __launch_bounds__(256) void rows16_embed_kernel(const int64_t* __restrict__ ids, const bf16* __restrict__ table, const bf16* __restrict__ norm_w,
+                                                           bf16* __restrict__ h, bf16* __restrict__ hw, float* __restrict__ sums, int M, int K, int64_t vocab) {
+    const int at = blockIdx.x * 256 + threadIdx.x, m = at % STREAM_ROWS, k = at / STREAM_ROWS * 8;
+    if (m >= M || k >= K) return;
+    const int64_t id = ids[m];
+    bf16x8 v{}, y;
+    if (id >= 0 && id < vocab) v = ld16<bf16x8>(table + id * K + k);
+    const bf16x8 nw = ld16<bf16x8>(norm_w + k);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        ss += to_f32(v[e]) * to_f32(v[e]);
+        y[e] = (bf16)(to_f32(v[e]) * to_f32(nw[e]));
+    }
+    st16(h + xf_off(m, k, K), v);
+    st16(hw + xf_off(m, k, K), y);
+    sums[sums_off(m, k)] = ss;
+}
+
+// SPW: k64-steps of a wave at most
+template <int KIND, int SPW, int RB>
+__global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int units, int per) {
+    constexpr int W = 8;
+    static_assert(KIND != ROWS_RESIDUAL && RB <= 2, "the kernel below");
+    __shared__ __attribute__((aligned(16))) float red[2][W][RB][64 * 4];
+    __shared__ float part[W][16 * RB];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int K = a.K, steps = K >> 6, mine = (steps - w + W - 1) / W;  // k64-steps w, w + 8, ..
+    const int m = lane & 15, kq = lane >> 4;
+    const int u0 = blockIdx.x * per, n = min(per, units - u0);
+
+    // the block of rows whose outputs this wave finishes (unit i: waves 2 i and 2 i + 1 mod 8)
+    const int fb = w & 1, frow = fb * 16 + m;
+    int32_t pos = 0, slot = 0;
+    if (KIND == ROWS_ROPE) {
+        pos = a.positions[min(frow, a.M - 1)];
+        slot = a.slots[min(frow, a.M - 1)];
+    }
+    bf16x8 x[RB][SPW][2];
+    uint32_t xoff[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) xoff[b] = kq * 1024 + min(b * 16 + m, a.M - 1) * 16;
+#pragma unroll
+    for (int j = 0; j < SPW; ++j) {
+        const char* xp = reinterpret_cast<const char*>(a.x) + (int64_t)min(w + W * j, steps - 1) * 4096;
+        PIN_SGPR(xp);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int b = 0; b < RB; ++b) x[b][j][h] = *(const GLOBAL_AS bf16x8*)(xp + xoff[b] + h * 512);
+    }
+    const uint32_t woff = kq * 1024 + ((lane & 7) + ((lane >> 3) & 1) * 16) * 16;
+    bf16x8 wq[SPW][2];
+    auto ask = [&](int u) {
+        const char* base = reinterpret_cast<const char*>(a.prep) + (int64_t)(u >> 1) * steps * 4096 + (u & 1) * 128;
+#pragma unroll
+        for (int j = 0; j < SPW; ++j) {
+            const char* p = base + (int64_t)min(w + W * j, steps - 1) * 4096;
+            PIN_SGPR(p);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) wq[j][h] = __builtin_nontemporal_load((const GLOBAL_AS bf16x8*)(p + h * 512 + woff));
+        }
+    };
+    ask(u0);
+    // the sums of h^2: SPW / 2 groups of 4 x 32 columns a wave
+    constexpr int SG = (SPW + 1) / 2;
+    f32x4 sq[RB][SG];
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int t = 0; t < SG; ++t)
+            sq[b][t] = *reinterpret_cast<const f32x4*>(a.sums + sums_off(min(b * 16 + m, a.M - 1), min((t * W + w) * 4 + kq, (K >> 5) - 1) * 32));
+    // ROPE: what unit u's outputs are rotated by, and the bias; asked for early for the first unit that this wave finishes
+    const bool second = kq >= 2;  // this lane's columns are of the tile's second half
+    bf16x4 cf{}, sf{}, bv{};
+    int head = 0, dim = 0;
+    auto rope_inputs = [&](int u) {
+        const int tile = u >> 1, c = (u & 1) * 8 + (kq & 1) * 4, per_head = a.D >> 5, tt = tile % per_head;
+        head = tile / per_head;
+        const bool roth = head < a.H + a.Hkv;
+        dim = roth ? (second ? (a.D >> 1) : 0) + 16 * tt + c : 32 * tt + c + (second ? 16 : 0);
+        const int64_t at = (int64_t)pos * (a.D >> 1) + 16 * tt + c;
+        if (roth) {
+            cf = *reinterpret_cast<const bf16x4*>(a.cosb + at);
+            sf = *reinterpret_cast<const bf16x4*>(a.sinb + at);
+        }
+        if (a.bias) bv = *reinterpret_cast<const bf16x4*>(a.bias + head * a.D + dim);
+    };
+    if (KIND == ROWS_ROPE) rope_inputs(u0 + min(w >> 1, n - 1));
+
+    auto unit = [&](int i, bool more) {
+        f32x4 acc[RB];
+#pragma unroll
+        for (int b = 0; b < RB; ++b) acc[b] = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < SPW; ++j)
+            if (j < mine) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int b = 0; b < RB; ++b) acc[b] = mfma16(wq[j][h], x[b][j][h], acc[b]);
+            }
+        if (more) ask(u0 + i + 1);
+        const int r = i & 1;
+#pragma unroll
+        for (int b = 0; b < RB; ++b) *reinterpret_cast<f32x4*>(&red[r][w][b][lane * 4]) = acc[b];
+        if (i == 0) {
+#pragma unroll
+            for (int b = 0; b < RB; ++b) {
+                float ss = 0.f;
+#pragma unroll
+                for (int t = 0; t < SG; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ss += (t * W + w) * 4 + kq < (K >> 5) ? sq[b][t][e] : 0.f;
+                ss = sum_of_quarters(ss);
+                if (kq == 0) part[w][b * 16 + m] = ss;
+            }
+        }
+        __syncthreads();  // (the sums of the unit that had this buffer before were read in front of a barrier since)
+        if (((w - 2 * i) & (W - 1)) >= RB) return;
+        float tot = 0.f;
+#pragma unroll
+        for (int k = 0; k < W; ++k) tot += part[k][frow];
+        const float rstd = rsqrtf(tot / K + a.eps);
+        f32x4 v = *reinterpret_cast<const f32x4*>(&red[r][0][fb][lane * 4]);
+#pragma unroll
+        for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[r][k][fb][lane * 4]);
+        v *= rstd;
+        // v[e]: row frow, column c + e of its half of the tile
+        const int u = u0 + i, tile = u >> 1, c = (u & 1) * 8 + (kq & 1) * 4;
+        const bool live = frow < a.M;
+        if (KIND == ROWS_HEAD) {
+            const int col = tile * 32 + c + (second ? 16 : 0);
+            float* o = reinterpret_cast<float*>(a.out) + (int64_t)frow * a.ldo + col;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (live && col + e < a.N) o[e] = v[e];
+        } else if (KIND == ROWS_SILU) {
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float own = to_f32((bf16)v[e]), up = __shfl_xor(own, 32, 64);
+                const float sl = own / (1.f + __expf(-own));
+                o[e] = (bf16)(to_f32((bf16)sl) * up);
+            }
+            if (live && !second) *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.out) + xf_off(frow, tile * 16 + c, a.N >> 1)) = o;
+        } else {
+            if (i >= W / 2) rope_inputs(u);
+            const bool roth = head < a.H + a.Hkv;
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float own = to_f32((bf16)(v[e] + to_f32(bv[e]))), other = __shfl_xor(own, 32, 64);
+                const float co = to_f32(cf[e]), si = to_f32(sf[e]);
+                o[e] = (bf16)(!roth ? own : second ? other * si + own * co : own * co - other * si);
+            }
+            if (!live) return;
+            const int64_t page = slot >> 5;
+            const int tok = slot & 31;
+            if (head < a.H) {
+                *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.out) + (int64_t)frow * a.ldo + head * a.D + dim) = o;
+            } else if (roth) {
+                *reinterpret_cast<bf16x4*>(a.kpool + (page * a.Hkv + (head - a.H)) * 32 * a.D + k_off(tok, dim, a.D)) = o;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a.vpool[(page * a.Hkv + (head - a.H - a.Hkv)) * 32 * a.D + v_off(tok, dim + e, a.D)] = o[e];
+            }
+        }
+    };
+    for (int i = 0; i + 1 < n; ++i) unit(i, true);
+    unit(n - 1, false);
+}
+
+template <int RB>
+__global__ __launch_bounds__(1024) void dense_rows16_residual_kernel(Rows16Args a) {
+    constexpr int W = 16;
+    __shared__ __attribute__((aligned(16))) float red[W][RB][64 * 4];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int steps = a.K >> 6;  // this wave's: w, w + 16, ..
+    const int m = lane & 15, kq = lane >> 4, tile = blockIdx.x >> 2, c0 = (blockIdx.x & 3) * 8;
+    const char* wbase = reinterpret_cast<const char*>(a.prep) + (int64_t)tile * steps * 4096;
+    const uint32_t woff = kq * 1024 + ((lane >> 3) & 1) * 512 + (c0 + (lane & 7)) * 16;
+    uint32_t xoff[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) xoff[b] = kq * 1024 + min(b * 16 + m, a.M - 1) * 16;
+    bf16x8 wq, x[RB][2];
+    auto ask = [&](int s) {
+        const char *p = wbase + (int64_t)s * 4096, *xp = reinterpret_cast<const char*>(a.x) + (int64_t)s * 4096;
+        PIN_SGPR(p);
+        PIN_SGPR(xp);
+        wq = __builtin_nontemporal_load((const GLOBAL_AS bf16x8*)(p + woff));
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[b][h] = *(const GLOBAL_AS bf16x8*)(xp + xoff[b] + h * 512);
+    };
+    ask(min(w, steps - 1));
+    const int frow = w * 16 + m, col = tile * 32 + c0 + (kq & 1) * 4;
+    const int64_t at = xf_off(min(frow, a.M - 1), col, a.N);
+    bf16x4 res{}, nw{};
+    if (w < RB) {
+        res = *reinterpret_cast<const bf16x4*>(a.h + at);
+        nw = *reinterpret_cast<const bf16x4*>(a.norm_w + col);
+    }
+    f32x4 acc[RB][2];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) acc[b][0] = acc[b][1] = f32x4{0, 0, 0, 0};
+    for (int s = w; s < steps; s += W) {
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) acc[b][h] = mfma16(wq, x[b][h], acc[b][h]);
+        if (s + W < steps) ask(s + W);
+    }
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = kq < 2 ? acc[b][0][e] : acc[b][1][e];
+        *reinterpret_cast<f32x4*>(&red[w][b][lane * 4]) = v;
+    }
+    __syncthreads();
+    if (w >= RB) return;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][w][lane * 4]);
+#pragma unroll
+    for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[k][w][lane * 4]);
+    bf16x4 h, hw;
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float f = to_f32((bf16)(v[e] + __shfl_xor(v[e], 32, 64))) + to_f32(res[e]);
+        ss += f * f;
+        h[e] = (bf16)f;
+        hw[e] = (bf16)(f * to_f32(nw[e]));
+    }
+    ss += __shfl_xor(ss, 16, 64);
+    if (kq >= 2 || frow >= a.M) return;
+    *reinterpret_cast<bf16x4*>(a.h + at) = h;
+    *reinterpret_cast<bf16x4*>(a.hw + at) = hw;
+    if (kq == 0) a.sums_out[sums_off(frow, col)] = ss;
+}
+
+// Whole steps, us, the other launches of a layer / these (2048 wide, inner 5632, 22 layers; ctx 137): 3, 4 rows 881 / 746 (the launches of up to four rows), 8 rows 964 / 761, 16
+// 990 / 814, 24 1053 / 917, 32 1077 / 970; 768, 2048, 12 layers, 8, 16, 32 rows: 461 / 302, 479 / 318, 541 / 397; 1024, 2816, 16 layers: 568 / 453, 589 / 484, 658 / 595;
+// 1536, 4096, 16 layers: 673 / 542, 701 / 581, 816 / 732.  Wider ones, 4, 8, 16 rows: 2560, 6912, 8 layers 504 / 471, 531 / 480, 569 / 540; 3072,
+// 8192: 543 / 542, 574 / 548, 597 / 585; 4096, 11008, 6 layers 664 / 617, 705 / 630, 748 / 695; there 32 rows 635 / 767, 654 / 776, 828 / 915 by more x than weights.  One and two rows: 716 / 744, 754 / 745, narrower ones 4 -
+// 10 % behind the launches of up to four rows, which keep them.
+bool rows16_fits(int64_t M, int64_t K, bool norm) {
+    return M >= 1 && M <= STREAM_ROWS && K >= 64 && K % 64 == 0 && K <= (!norm ? 12288 : M <= 16 ? 4096 : 2048);
+}
+
+template <int KIND, int RB, int SPW>
+void launch_rows16_k(const Rows16Args& a, hipStream_t st) {
+    const int units = a.NT * 2, per = (units + 255) / 256;
+    hipLaunchKernelGGL((dense_rows16_kernel<KIND, SPW, RB>), dim3((unsigned)((units + per - 1) / per)), dim3(512), 0, st, a, units, per);
+}
+template <int KIND, int RB>
+void launch_rows16_rb(const Rows16Args& a, hipStream_t st) {
+    if constexpr (KIND == ROWS_RESIDUAL) {
+        hipLaunchKernelGGL((dense_rows16_residual_kernel<RB>), dim3((unsigned)(a.NT * 4)), dim3(1024), 0, st, a);
+    } else {
+        const int spw = (a.K + 511) / 512;
+        if (spw <= 2) return launch_rows16_k<KIND, RB, 2>(a, st);
+        if (spw == 3) return launch_rows16_k<KIND, RB, 3>(a, st);
+        if constexpr (RB == 1) {
+            if (spw == 5) return launch_rows16_k<KIND, RB, 5>(a, st);
+            if (spw == 6) return launch_rows16_k<KIND, RB, 6>(a, st);
+            if (spw > 6) return launch_rows16_k<KIND, RB, 8>(a, st);
+        }
+        launch_rows16_k<KIND, RB, 4>(a, st);
+    }
+}
+template <int KIND>
+int launch_rows16(const Rows16Args& a, hipStream_t st) {
+    TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
+    a.M <= 16 ? launch_rows16_rb<KIND, 1>(a, st) : launch_rows16_rb<KIND, 2>(a, st);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
 int64_t rows_height(int64_t M) { return M <= 2 ? M : 4; }
 
 // Whole steps, us, seven launches a layer / these: 2048 wide, inner 5632, 22 layers: 1, 2, 3, 4 rows 920 / 729, 945 / 769, 980 / 948, 1008 / 981;
@@ -374,4 +696,99 @@ extern "C" int tgis_dense_rows_norm_rope(const float* h, const void* norm_w, flo
     a.Hkv = (int)Hkv;
     a.D = (int)D;
     return launch_rows<ROWS_ROPE>(a, dtype, (hipStream_t)stream);
+}
+
+// ---- the launches of up to 32 rows ----
+
+extern "C" int tgis_dense_rows16_ok(int64_t M, int64_t K, int norm) { return rows16_fits(M, K, norm != 0) ? 1 : 0; }
+
+namespace {
+
+int rows16_check(const char* what, int64_t M, int64_t K, int64_t N, bool norm, const void* x, const void* prepared, const void* other) {
+    TGIS_CHECK_ARG(x && prepared && other && N > 0 && N < (1ll << 31), "%s: null tensor or bad shape", what);
+    TGIS_CHECK_ARG(rows16_fits(M, K, norm), "%s: up to %d rows, K a multiple of 64 up to %d (M=%ld K=%ld)", what, STREAM_ROWS,
+                   !norm ? 12288 : M <= 16 ? 4096 : 2048, (long)M, (long)K);
+    TGIS_CHECK_ARG(((uintptr_t)x | (uintptr_t)prepared | (uintptr_t)other) % 16 == 0, "%s: operands must be 16-byte aligned", what);
+    return TGIS_OK;
+}
+Rows16Args rows16_args(const void* x, const float* sums, float eps, const void* prepared, int64_t M, int64_t K, int64_t N, void* out, int64_t ldo) {
+    Rows16Args a{};
+    a.x = (const bf16*)x;
+    a.sums = sums;
+    a.eps = eps;
+    a.prep = (const uint8_t*)prepared;
+    a.M = (int)M;
+    a.K = (int)K;
+    a.N = (int)N;
+    a.NT = (int)cdiv64(N, 32);
+    a.out = out;
+    a.ldo = ldo;
+    return a;
+}
+
+}  // namespace
+
+extern "C" int tgis_dense_rows16_embed(const int64_t* ids, const void* table, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
+                                       int64_t vocab, void* stream) {
+    const int rc = rows16_check("tgis_dense_rows16_embed", M, K, vocab, true, table, norm_w, h);
+    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(ids && hw && sums && ((uintptr_t)hw | (uintptr_t)sums) % 16 == 0, "tgis_dense_rows16_embed: null or unaligned tensor");
+    hipLaunchKernelGGL(rows16_embed_kernel, dim3((unsigned)(K / 8 * STREAM_ROWS / 256)), dim3(256), 0, (hipStream_t)stream, ids, (const bf16*)table,
+                       (const bf16*)norm_w, (bf16*)h, (bf16*)hw, sums, (int)M, (int)K, vocab);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+extern "C" int tgis_dense_rows16_residual(const void* x, const void* prepared, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
+                                          int64_t N, void* stream) {
+    const int rc = rows16_check("tgis_dense_rows16_residual", M, K, N, false, x, prepared, h);
+    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(norm_w && hw && sums && ((uintptr_t)norm_w | (uintptr_t)hw | (uintptr_t)sums) % 16 == 0 && N % 64 == 0,
+                   "tgis_dense_rows16_residual: null or unaligned tensor, or a width that is no multiple of 64");
+    Rows16Args a = rows16_args(x, nullptr, 0.f, prepared, M, K, N, nullptr, 0);
+    a.norm_w = (const bf16*)norm_w;
+    a.h = (bf16*)h;
+    a.hw = (bf16*)hw;
+    a.sums_out = sums;
+    return launch_rows16<ROWS_RESIDUAL>(a, (hipStream_t)stream);
+}
+
+extern "C" int tgis_dense_rows16_norm_head(const void* hw, const float* sums, float eps, const void* prepared, float* out, int64_t ldo, int64_t M, int64_t K,
+                                           int64_t N, void* stream) {
+    const int rc = rows16_check("tgis_dense_rows16_norm_head", M, K, N, true, hw, prepared, sums);
+    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(out && ldo >= N, "tgis_dense_rows16_norm_head: bad output");
+    return launch_rows16<ROWS_HEAD>(rows16_args(hw, sums, eps, prepared, M, K, N, out, ldo), (hipStream_t)stream);
+}
+
+extern "C" int tgis_dense_rows16_norm_silu(const void* hw, const float* sums, float eps, const void* prepared, void* out, int64_t M, int64_t K, int64_t N,
+                                           void* stream) {
+    const int rc = rows16_check("tgis_dense_rows16_norm_silu", M, K, N, true, hw, prepared, sums);
+    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(out && (uintptr_t)out % 16 == 0 && N % 128 == 0, "tgis_dense_rows16_norm_silu: needs a gate|up image (N / 2 a multiple of 64) and its output");
+    return launch_rows16<ROWS_SILU>(rows16_args(hw, sums, eps, prepared, M, K, N, out, 0), (hipStream_t)stream);
+}
+
+extern "C" int tgis_dense_rows16_norm_rope(const void* hw, const float* sums, float eps, const void* prepared, const void* bias, const int32_t* positions,
+                                           const int32_t* slots, const void* cos, const void* sin, void* q_out, int64_t ldq, void* k_pool, void* v_pool,
+                                           int64_t M, int64_t K, int64_t H, int64_t Hkv, int64_t D, void* stream) {
+    const int64_t N = (H + 2 * Hkv) * D;
+    const int rc = rows16_check("tgis_dense_rows16_norm_rope", M, K, N, true, hw, prepared, sums);
+    if (rc != TGIS_OK) return rc;
+    TGIS_CHECK_ARG(positions && slots && cos && sin && q_out && k_pool && v_pool, "tgis_dense_rows16_norm_rope: null tensor");
+    TGIS_CHECK_ARG(H >= 1 && Hkv >= 1 && D >= 32 && D % 32 == 0 && ldq >= H * D, "tgis_dense_rows16_norm_rope: bad head geometry");
+    TGIS_CHECK_ARG(ldq % 4 == 0 && ((uintptr_t)q_out | (uintptr_t)cos | (uintptr_t)sin | (uintptr_t)bias | (uintptr_t)k_pool) % 8 == 0,
+                   "tgis_dense_rows16_norm_rope: q, its rows, bias, tables and pages must be 8-byte aligned");
+    Rows16Args a = rows16_args(hw, sums, eps, prepared, M, K, N, q_out, ldq);
+    a.bias = (const bf16*)bias;
+    a.positions = positions;
+    a.slots = slots;
+    a.cosb = (const bf16*)cos;
+    a.sinb = (const bf16*)sin;
+    a.kpool = (bf16*)k_pool;
+    a.vpool = (bf16*)v_pool;
+    a.H = (int)H;
+    a.Hkv = (int)Hkv;
+    a.D = (int)D;
+    return launch_rows16<ROWS_ROPE>(a, (hipStream_t)stream);
 }

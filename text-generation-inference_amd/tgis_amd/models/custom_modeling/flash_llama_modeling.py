@@ -208,8 +208,9 @@ class FlashLlamaAttention:
             return native.rope_kv_write_prefill(*pages), None
         return native.rope_kv_write(qkv, cos, sin, position_ids, kv.slots, k_pool, v_pool, H, Hkv, D, D), None
 
-    def attend(self, qkv, cu_seqlens_q, layer_id: int, kv: KVArgs, rope=None):
-        """Attention of q (rotated, or to be rotated by `rope`) over the layer's cache pages (reference :271-295): [T, H D]."""
+    def attend(self, qkv, cu_seqlens_q, layer_id: int, kv: KVArgs, rope=None, frag: bool = False):
+        """Attention of q (rotated, or to be rotated by `rope`) over the layer's cache pages (reference :271-295): [T, H D], a native.FragAct where the
+        o_proj GEMM reads that, or with `frag` (a decode step)."""
         H, Hkv, D = self.num_heads, self.num_key_value_heads, self.head_size
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         T = qkv.shape[0]
@@ -221,6 +222,8 @@ class FlashLlamaAttention:
             if self.out_places is not None:
                 places = {"out_cols": self.out_places}
             attn_output = native.FragAct.empty(T, H * D, qkv.device)
+        elif frag:
+            attn_output = native.FragAct.empty(T, H * D, qkv.device, qkv.dtype)
         else:
             attn_output = torch.empty((T, H * D), dtype=qkv.dtype, device=qkv.device)
         ws = None
@@ -362,9 +365,11 @@ class FlashLlamaModel:
             self.max_positions = max(max_s, 2 * self.max_positions, declared, 2048)
         return self.layers[0].self_attn.rotary_emb.tables(dtype, device, self.max_positions)
 
-    def forward_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
+    def forward_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs, matrix: bool = False):
         """A decode step of a few rows on the launches of csrc/dense_rows.hip: the residual stream (fp32, [rows, hidden]) in front of the final
-        norm.  Five launches a layer; the values are those of `forward` but for the order of the sums."""
+        norm.  Five launches a layer; the values are those of `forward` but for the order of the sums.  matrix: `forward_rows16`."""
+        if matrix:
+            return self.forward_rows16(input_ids, position_ids, cu_seqlens_q, max_s, kv)
         h = native.embedding_scaled_f32(input_ids, self.embed_tokens.weight, 1.0)
         cos, sin = self.rope_tables(self.embed_tokens.weight.dtype, h.device, max_s)
         for layer in self.layers:
@@ -377,6 +382,21 @@ class FlashLlamaModel:
             act = native.dense_rows_silu(h, layer.post_attention_layernorm.weight, layer.post_attention_layernorm.variance_epsilon,
                                          mlp.gate_up_proj.linear.prepared)
             native.dense_rows_residual(act, mlp.down_proj.linear.prepared, h)
+        return h
+
+    def forward_rows16(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
+        """The same for more rows, in bf16, on the launches there that take the matrix instruction: a native.RowsStream."""
+        norms = [n for layer in self.layers for n in (layer.input_layernorm, layer.post_attention_layernorm)] + [self.norm]
+        h = native.RowsStream.embed(input_ids, self.embed_tokens.weight, norms[0].weight)
+        cos, sin = self.rope_tables(self.embed_tokens.weight.dtype, h.device, max_s)
+        for i, layer in enumerate(self.layers):
+            att, mlp = layer.self_attn, layer.mlp
+            qkv = native.dense_rows16_rope(h, norms[2 * i].variance_epsilon, att.query_key_value.linear.rope_handle, att.query_key_value.linear.bias, cos, sin,
+                                           position_ids, kv.slots, kv.cache.k_pool(layer.layer_id), kv.cache.v_pool(layer.layer_id), att.num_heads,
+                                           att.num_key_value_heads, att.head_size)
+            native.dense_rows16_residual(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv, frag=True), att.o_proj.linear.prepared, h, norms[2 * i + 1].weight)
+            act = native.dense_rows16_silu(h, norms[2 * i + 1].variance_epsilon, mlp.gate_up_proj.linear.prepared)
+            native.dense_rows16_residual(act, mlp.down_proj.linear.prepared, h, norms[2 * i + 2].weight)
         return h
 
     def plain_layers(self, count: int, x, cos, kv: KVArgs) -> list:
@@ -446,7 +466,7 @@ class FlashLlamaForCausalLM:
         self.config = config
         self.model = FlashLlamaModel(config, weights)
         self.lm_head = TensorParallelHead.load(config, prefix="lm_head", weights=weights)
-        self._rows_path = {}
+        self._rows_path, self._rows16_path = {}, {}
         self.gptq_linears: List = []
         for layer in self.model.layers:
             for lin in (layer.self_attn.query_key_value.linear, layer.self_attn.o_proj.linear,
@@ -473,16 +493,25 @@ class FlashLlamaForCausalLM:
             got = self._rows_path[rows] = rows <= min(native.DENSE_ROWS_MAX_M, SKINNY_MAX_M) and self._serves_rows(rows)
         return got
 
-    def _serves_rows(self, rows: int) -> bool:
-        cfg = self.config
+    def rows16_path(self, rows: int) -> bool:
+        """The same of the launches for more rows (FlashLlamaModel.forward_rows16)."""
+        got = self._rows16_path.get(rows)
+        if got is None:
+            got = self._rows16_path[rows] = (native.DENSE_ROWS16_MIN_M <= rows <= min(native.DENSE_ROWS16_MAX_M, SKINNY_MAX_M)
+                                             and self.model.embed_tokens.weight.dtype == torch.bfloat16
+                                             and self._serves_rows(rows, native.dense_rows16_ok))
+        return got
+
+    def _serves_rows(self, rows: int, ok=None) -> bool:
+        cfg, ok = self.config, ok or native.dense_rows_ok
         plain = lambda lin: isinstance(lin, FastLinear) and lin.streams and lin.bias is None
-        if self.model.tp_world_size != 1 or not plain(self.lm_head.linear) or not native.dense_rows_ok(rows, cfg.hidden_size, True):
+        if self.model.tp_world_size != 1 or not plain(self.lm_head.linear) or not ok(rows, cfg.hidden_size, True):
             return False
         for layer in self.model.layers:
             qkv, o = layer.self_attn.query_key_value.linear, layer.self_attn.o_proj.linear
             gate_up, down = layer.mlp.gate_up_proj.linear, layer.mlp.down_proj.linear
             if not (isinstance(qkv, FastLinear) and qkv.rope_handle is not None and plain(o) and plain(gate_up) and gate_up.gate_up and plain(down)
-                    and native.dense_rows_ok(rows, o.in_features, False) and native.dense_rows_ok(rows, down.in_features, False)):
+                    and ok(rows, o.in_features, False) and ok(rows, down.in_features, False)):
                 return False
         return True
 
@@ -496,10 +525,18 @@ class FlashLlamaForCausalLM:
     def forward(self, input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds=None, kv: KVArgs = None,
                 lm_head_indices: Optional[torch.Tensor] = None):
         """position_ids int32 [T]; returns fp32 logits [T or len(lm_head_indices), vocab]."""
-        if (kv.max_q_len == 1 and not kv.fresh_prefill and inputs_embeds is None and lm_head_indices is None and kv.slots is not None
-                and self.rows_path(input_ids.shape[0])):
-            h = self.model.forward_rows(input_ids, position_ids, cu_seqlens_q, max_s, kv)
-            return native.dense_rows_head(h, self.model.norm.weight, self.model.norm.variance_epsilon, self.lm_head.linear.prepared)
+        if kv.max_q_len == 1 and not kv.fresh_prefill and inputs_embeds is None and lm_head_indices is None and kv.slots is not None:
+            rows, h = input_ids.shape[0], None
+            step = (input_ids, position_ids, cu_seqlens_q, max_s, kv)
+            if self.rows_path(rows):
+                h = self.model.forward_rows(*step, self.rows16_path(rows))
+            elif self.rows16_path(rows):
+                h = self.model.forward_rows16(*step)
+            norm, head = self.model.norm, self.lm_head.linear
+            if isinstance(h, native.RowsStream):
+                return native.dense_rows16_head(h, norm.variance_epsilon, head.prepared)
+            if h is not None:
+                return native.dense_rows_head(h, norm.weight, norm.variance_epsilon, head.prepared)
         hidden_states = self.model(input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv)
         if lm_head_indices is not None and not kv.cuts_to_ends(position_ids.shape[0]):
             hidden_states = hidden_states.index_select(0, lm_head_indices)

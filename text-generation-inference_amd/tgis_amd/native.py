@@ -94,6 +94,13 @@ SIGNATURES = {
     "tgis_dense_rows_residual": (_c_int, [_vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_rows_norm_silu": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_dense_rows_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _vp]),
+    "tgis_dense_rows16_ok": (_c_int, [_c_i64, _c_i64, _c_int]),
+    "tgis_dense_rows16_embed": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_dense_rows16_norm_rope": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64,
+                                             _c_i64, _vp]),
+    "tgis_dense_rows16_residual": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_dense_rows16_norm_silu": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_dense_rows16_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_attn_paged": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int,
                                  _c_int, _c_i64, _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
     "tgis_attn_rotates_q": (_c_int, [_c_int, _c_int, _c_int, _c_i64]),
@@ -348,11 +355,11 @@ LD_FRAGMENTS = -32
 
 
 class FragAct:
-    """A [M <= 64, K] f16 activation stored in fragment order (include/tgis_hip.h, TGIS_LD_FRAGMENTS): what the decode
+    """A [M <= 64, K] activation (f16 in front of int4 GEMMs) stored in fragment order (include/tgis_hip.h, TGIS_LD_FRAGMENTS): what the decode
     step's norm / attention / SiLU epilogue hand to the int4 GEMM behind them.  `buf` holds ceil(M / 32) * 32 * K elements."""
 
     def __init__(self, buf: torch.Tensor, M: int, K: int):
-        assert 1 <= M <= 64 and K % 64 == 0 and buf.dtype == torch.float16 and buf.numel() == (M + 31) // 32 * 32 * K
+        assert 1 <= M <= 64 and K % 64 == 0 and buf.dtype in (torch.float16, torch.bfloat16) and buf.numel() == (M + 31) // 32 * 32 * K
         self.buf, self.M, self.K = buf, M, K
         self.dtype, self.device = buf.dtype, buf.device
 
@@ -361,8 +368,8 @@ class FragAct:
         return (self.M, self.K)
 
     @staticmethod
-    def empty(M: int, K: int, device) -> "FragAct":
-        return FragAct(torch.empty((M + 31) // 32 * 32 * K, dtype=torch.float16, device=device), M, K)
+    def empty(M: int, K: int, device, dtype=torch.float16) -> "FragAct":
+        return FragAct(torch.empty((M + 31) // 32 * 32 * K, dtype=dtype, device=device), M, K)
 
     @staticmethod
     def from_rows(x: torch.Tensor) -> "FragAct":
@@ -822,10 +829,15 @@ def dense_gemm_rope(x: torch.Tensor, w: DenseWeight, bias, cos, sin, positions, 
 
 
 DENSE_ROWS_MAX_M = 4
+DENSE_ROWS16_MIN_M, DENSE_ROWS16_MAX_M = 3, 32  # (one and two rows are sooner done by the launches for a few)
 
 
 def dense_rows_ok(M: int, K: int, norm: bool) -> bool:
     return bool(load_library().tgis_dense_rows_ok(M, K, int(norm)))
+
+
+def dense_rows16_ok(M: int, K: int, norm: bool) -> bool:
+    return bool(load_library().tgis_dense_rows16_ok(M, K, int(norm)))
 
 
 def _rows_stream(h: torch.Tensor, width: int):
@@ -865,6 +877,58 @@ def dense_rows_head(h, norm_w, eps: float, w: DenseWeight) -> torch.Tensor:
     out = torch.empty((h.shape[0], w.N), dtype=torch.float32, device=h.device)
     _check(load_library().tgis_dense_rows_norm_head(_rows_stream(h, w.K), _ptr(norm_w), float(eps), _ptr(w.image), _ptr(out), out.stride(0),
                                                     h.shape[0], w.K, w.N, dtype_code(w.dtype), _stream()), "tgis_dense_rows_norm_head")
+    return out
+
+
+class RowsStream:
+    """The residual stream of up to DENSE_ROWS16_MAX_M rows in front of a norm: T(h), T(h * norm weight) and the sums of h^2 of eight columns each, in
+    the order that the launches below read them in (include/tgis_hip.h)."""
+
+    def __init__(self, M: int, width: int, device):
+        self.M, self.width, self.device = M, width, device
+        self.h, self.hw = FragAct.empty(M, width, device, torch.bfloat16), FragAct.empty(M, width, device, torch.bfloat16)
+        self.sums = torch.empty(width // 8 * DENSE_ROWS16_MAX_M, dtype=torch.float32, device=device)
+
+    @staticmethod
+    def embed(ids: torch.Tensor, table: torch.Tensor, norm_w: torch.Tensor) -> "RowsStream":
+        assert ids.dtype == torch.int64 and ids.dim() == 1 and ids.is_contiguous() and table.dim() == 2 and table.is_contiguous()
+        assert table.dtype == norm_w.dtype == torch.bfloat16 and norm_w.numel() == table.shape[1]
+        h = RowsStream(ids.shape[0], table.shape[1], table.device)
+        _check(load_library().tgis_dense_rows16_embed(_ptr(ids), _ptr(table), _ptr(norm_w), _ptr(h.h.buf), _ptr(h.hw.buf), _ptr(h.sums), h.M, h.width,
+                                                      table.shape[0], _stream()), "tgis_dense_rows16_embed")
+        return h
+
+
+def dense_rows16_rope(h: RowsStream, eps: float, w: DenseWeight, bias, cos, sin, positions, slots, k_pool, v_pool, H: int, Hkv: int, D: int) -> torch.Tensor:
+    assert w.flags & 2 and w.N == (H + 2 * Hkv) * D and w.K == h.width and cos.dtype == w.dtype == torch.bfloat16 and cos.shape[1] * 2 == D
+    assert positions.dtype == torch.int32 and slots.dtype == torch.int32
+    out = torch.empty((h.M, w.N), dtype=w.dtype, device=h.device)
+    _check(load_library().tgis_dense_rows16_norm_rope(
+        _ptr(h.hw.buf), _ptr(h.sums), float(eps), _ptr(w.image), _ptr(bias), _ptr(positions), _ptr(slots), _ptr(cos), _ptr(sin), _ptr(out), out.stride(0),
+        _ptr(k_pool), _ptr(v_pool), h.M, w.K, H, Hkv, D, _stream()), "tgis_dense_rows16_norm_rope")
+    return out
+
+
+def dense_rows16_residual(x: FragAct, w: DenseWeight, h: RowsStream, norm_w) -> None:
+    """h += x @ w^T, both rounded first, in front of the norm of weight norm_w."""
+    assert x.dtype == w.dtype == norm_w.dtype == torch.bfloat16 and x.K == w.K and not w.flags and x.M == h.M and w.N == h.width == norm_w.numel()
+    _check(load_library().tgis_dense_rows16_residual(_ptr(x.buf), _ptr(w.image), _ptr(norm_w), _ptr(h.h.buf), _ptr(h.hw.buf), _ptr(h.sums), h.M, w.K, w.N,
+                                                     _stream()), "tgis_dense_rows16_residual")
+
+
+def dense_rows16_silu(h: RowsStream, eps: float, w: DenseWeight) -> FragAct:
+    assert w.flags & 1 and w.dtype == torch.bfloat16 and w.K == h.width
+    out = FragAct.empty(h.M, w.N // 2, h.device, w.dtype)
+    _check(load_library().tgis_dense_rows16_norm_silu(_ptr(h.hw.buf), _ptr(h.sums), float(eps), _ptr(w.image), _ptr(out.buf), h.M, w.K, w.N, _stream()),
+           "tgis_dense_rows16_norm_silu")
+    return out
+
+
+def dense_rows16_head(h: RowsStream, eps: float, w: DenseWeight) -> torch.Tensor:
+    assert not w.flags and w.dtype == torch.bfloat16 and w.K == h.width
+    out = torch.empty((h.M, w.N), dtype=torch.float32, device=h.device)
+    _check(load_library().tgis_dense_rows16_norm_head(_ptr(h.hw.buf), _ptr(h.sums), float(eps), _ptr(w.image), _ptr(out), out.stride(0), h.M, w.K, w.N,
+                                                      _stream()), "tgis_dense_rows16_norm_head")
     return out
 
 
@@ -1060,7 +1124,7 @@ def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_
     assert block_tables.dtype == torch.int32 and ctx_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
     assert block_tables.is_contiguous()
     if isinstance(out, FragAct):
-        assert max_q_len == 1 and out.K == H * D and out.M == B
+        assert max_q_len == 1 and out.K == H * D and out.M == B and out.dtype == q.dtype
         optr, ldo = _ptr(out.buf), LD_FRAGMENTS
     else:
         assert out.is_contiguous()
