@@ -211,6 +211,10 @@ typedef struct {
     int64_t workspace_bytes;
     int64_t slab_ld;       /* set by the call */
     int num_slabs;
+    /* not NULL (up to 64 rows in bf16 that tgis_dense_rows16_ok): the launches tgis_dense_rows16_*, with their buffers of that stream.  att and act are in fragment
+     * order then, slabs their scratch, and the last product is left in `last` as one slab of rows */
+    void *h, *hw;
+    float *sums, *last;
 } TgisLlamaPrompt;
 int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, TgisLlamaPrompt* prompt, void* stream);
 
@@ -233,17 +237,21 @@ int tgis_dense_rows_norm_silu(const float* h, const void* norm_w, float eps, con
                               int64_t K, int64_t N, int dtype, void* stream);
 int tgis_dense_rows_norm_head(const float* h, const void* norm_w, float eps, const void* prepared, float* out, int64_t ldo, int64_t M,
                               int64_t K, int64_t N, int dtype, void* stream);
-/* The same for up to 32 rows in bf16, by the matrix instruction, K up to 12288, where it norms 4096 (up to 16 rows) or 2048.  The stream between the launches is T(h),
- * T(h * norm_w) of the norm weight that is next, and sums: the sums of h^2 of eight columns each, h in fp32, as [width / 32][32 rows][4].  These, x of `residual` and
+/* The same for up to 64 rows in bf16, by the matrix instruction, K up to 12288, where it norms 4096 (up to 16 rows) or 2048.  The stream between the launches is T(h),
+ * T(h * norm_w) of the norm weight that is next, and sums: the sums of h^2 of eight columns each, h in fp32, as [width / 32][64 rows][4].  These, x of `residual` and
  * the output of `norm_silu` are in 32-row fragment order (TGIS_LD_FRAGMENTS); rows past M are left alone.
- *   tgis_dense_rows16_embed       the stream of M tokens (zeros for an id outside the vocabulary)
- *   tgis_dense_rows16_residual    h = T(x W^T) + T(h), norm_w that of the norm behind it; N (the width) a multiple of 64
+ *   tgis_dense_rows16_embed       the stream of M tokens (x the table; zeros for an id outside the vocabulary), or of the rows x [M][K] (ids null)
+ *   tgis_dense_rows16_residual    h = T(x W^T) + T(h), norm_w that of the norm behind it; N (the width) a multiple of 64; slabs: tgis_dense_rows16_slab_bytes of scratch
+ *   tgis_dense_rows16_leave       behind the last layer: x W^T in fp32 as one slab of rows ([32-row block][32][N], tgis_rmsnorm_residual_partial) and T(h) as rows
  *   tgis_dense_rows16_norm_*      of T(h * norm_w) and its sums: products times rsqrt(mean h^2 + eps), from there as above; norm_silu: N / 2 a multiple of 64 */
 int tgis_dense_rows16_ok(int64_t M, int64_t K, int norm);
-int tgis_dense_rows16_embed(const int64_t* ids, const void* table, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
+int tgis_dense_rows16_embed(const int64_t* ids, const void* x, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
                             int64_t vocab, void* stream);
-int tgis_dense_rows16_residual(const void* x, const void* prepared, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
-                               int64_t N, void* stream);
+int64_t tgis_dense_rows16_slab_bytes(int64_t M, int64_t K, int64_t N, int leave);
+int tgis_dense_rows16_residual(const void* x, const void* prepared, const void* norm_w, void* h, void* hw, float* sums, float* slabs,
+                               int64_t slabs_bytes, int64_t M, int64_t K, int64_t N, void* stream);
+int tgis_dense_rows16_leave(const void* x, const void* prepared, const void* h, void* h_rows, float* sum_rows, float* slabs, int64_t slabs_bytes,
+                            int64_t M, int64_t K, int64_t N, void* stream);
 int tgis_dense_rows16_norm_rope(const void* hw, const float* sums, float eps, const void* prepared, const void* bias, const int32_t* positions,
                                 const int32_t* slots, const void* cos, const void* sin, void* q_out, int64_t ldq, void* k_pool, void* v_pool,
                                 int64_t M, int64_t K, int64_t H, int64_t Hkv, int64_t D, void* stream);
@@ -376,6 +384,10 @@ int tgis_attn_paged_rope(const void* q, int64_t ld_q, const void* cos, const voi
                          const void* v_pool, const int32_t* block_tables, int64_t max_pages, const int32_t* ctx_lens,
                          const int32_t* cu_seqlens_q, void* out, int64_t B, int H, int Hkv, int D, int64_t max_q_len,
                          int64_t max_ctx, float scale, int dtype, void* stream);
+/* tgis_attn_paged of prompts (any max_q_len, no key splits) whose output leaves in 32-row fragment order: ceil(tokens / 32) blocks, H * D a multiple of 64. */
+int tgis_attn_paged_fragments(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables, int64_t max_pages,
+                              const int32_t* ctx_lens, const int32_t* cu_seqlens_q, void* out, int64_t B, int H, int Hkv, int D, int64_t max_q_len,
+                              int64_t max_ctx, float scale, int dtype, void* stream);
 /* ... of a decode step (one token per sequence), written in fragment order with output column k at column out_cols[k] (a permutation of
  * 0 .. H * D - 1): the order an act-order matrix behind it wants its operand in. */
 int tgis_attn_paged_ordered(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,

@@ -15,17 +15,17 @@ def to_stream(h, nw, dev):
 
     (M, width), dtype = h.shape, torch.bfloat16
     stream = native.RowsStream(M, width, dev)
-    full = torch.full((32, width), float("nan"))
+    full = torch.full((64, width), float("nan"))
     for act, value in ((stream.h, h), (stream.hw, h * nw.float())):
         full[:M] = value
-        act.buf.copy_(native.FragAct.from_rows(full.to(dtype)).buf)
+        act.buf.copy_(native.FragAct.from_rows(full.to(dtype)).buf[:act.buf.numel()])
     full[:M] = h
-    stream.sums.copy_((full * full).view(32, -1, 4, 8).sum(-1).transpose(0, 1).reshape(-1))
+    stream.sums.copy_((full * full).view(64, -1, 4, 8).sum(-1).transpose(0, 1).reshape(-1))
     return stream
 
 
 # K: one step of 64, fewer steps than waves, one more than a round of them, more than are asked for at once
-@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("K,N", [(64, 64), (1088, 192), (2112, 2048), (6208, 64), (12288, 64)])
 def test_residual(gpu_device, M, K, N):
     from tgis_amd import native
@@ -36,8 +36,8 @@ def test_residual(gpu_device, M, K, N):
     h, nw = torch.randn(M, N, generator=g), (torch.rand(N, generator=g) + 0.5).to(dtype)
     stream = to_stream(h, nw, gpu_device)
     native.dense_rows16_residual(native.FragAct.from_rows(x.to(gpu_device)), native.DenseWeight(w.to(gpu_device)), stream, nw.to(gpu_device))
-    rows = lambda act: native.FragAct(act.buf, 32, N).to_rows().cpu().double()
-    sums = stream.sums.cpu().view(-1, 32, 4).transpose(0, 1).reshape(32, -1).double()
+    rows = lambda act: native.FragAct(act.buf, act.buf.numel() // N, N).to_rows().cpu().double()
+    sums = stream.sums.cpu().view(-1, 64, 4).transpose(0, 1).reshape(64, -1).double()
     y = x.double() @ w.double().t()
     want = y.to(dtype).double() + h.to(dtype).double()
     u = 2.0 ** -8
@@ -50,14 +50,14 @@ def test_residual(gpu_device, M, K, N):
 
 
 # ff, vocab: one unit, an odd number of units a workgroup, tiles that end within four columns
-@pytest.mark.parametrize("M", [5, 16, 17, 32])
+@pytest.mark.parametrize("M", [5, 16, 17, 48, 64])
 @pytest.mark.parametrize("K,ff,vocab", [(64, 64, 50), (1088, 4160, 8203), (2048, 5632, 40), (2560, 64, 40), (3072, 64, 40), (4096, 128, 72)])
 def test_norm_silu_and_head(gpu_device, M, K, ff, vocab):
     from tgis_amd import native
 
     dtype = torch.bfloat16
     if not native.dense_rows16_ok(M, K, True):
-        with pytest.raises(RuntimeError, match="up to 32 rows"):
+        with pytest.raises(RuntimeError, match="up to 64 rows"):
             native.dense_rows16_head(native.RowsStream(M, K, gpu_device), 1e-5, native.DenseWeight(torch.zeros(64, K, dtype=dtype, device=gpu_device)))
         return
     g = torch.Generator().manual_seed(M + K)
@@ -72,7 +72,7 @@ def test_norm_silu_and_head(gpu_device, M, K, ff, vocab):
     close(logits, x @ wh.double().t(), K, dtype, 0)
 
 
-@pytest.mark.parametrize("M", [5, 16, 31])
+@pytest.mark.parametrize("M", [5, 31, 47, 64])
 @pytest.mark.parametrize("K,H,Hkv,D,bias", [(2048, 32, 4, 64, False), (448, 3, 1, 32, True), (1984, 32, 16, 128, True)])
 def test_norm_rope(gpu_device, M, K, H, Hkv, D, bias):
     """The same launch as norm + dense_gemm_rope: q, and the pages that it wrote, element for element within roundings."""
@@ -119,3 +119,18 @@ def test_same_steps(gpu_device, monkeypatch, rows):
     for a, b in zip(got[1:] + pages, want[1:] + pages_want):
         a, b = a.double(), b.double()
         assert a.shape == b.shape and float((a - b).norm() / b.norm()) < 4 * step
+
+
+@pytest.mark.parametrize("lens", [[3], [30, 1, 33], [47], [64]])
+def test_prompts(gpu_device, monkeypatch, lens):
+    """Prompts of up to 64 rows: every token's logits and the pages, against the launches of `forward`."""
+    from tests.test_llama_prompt_gpu import steps
+    from tgis_amd.models.custom_modeling.flash_llama_modeling import FlashLlamaModel
+
+    lm, cfg = model(torch.bfloat16)
+    got = steps(lm, cfg.vocab_size, lens)
+    monkeypatch.setattr(FlashLlamaModel, "serves_rows16", lambda self, rows: False)
+    want = steps(lm, cfg.vocab_size, lens)
+    assert len(got) == len(want) and not torch.equal(got[0], want[0])
+    for a, b in zip(got, want):  # (as above)
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 4 * 2.0 ** -8

@@ -821,7 +821,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
                            const int32_t* cu_seqlens_q, void* out, int64_t ld_out, const int32_t* out_cols, int64_t B, int H, int Hkv,
                            int D, int64_t max_q_len, int64_t max_ctx, float scale, int dtype, int num_splits,
                            void* workspace, int64_t workspace_bytes, void* stream, const void* cos = nullptr, const void* sin = nullptr,
-                           const int32_t* positions = nullptr) {
+                           const int32_t* positions = nullptr, bool prompts = false) {
     TGIS_CHECK_ARG(q && k_pool && v_pool && block_tables && ctx_lens && cu_seqlens_q && out,
                    "tgis_attn_paged: null tensor");
     TGIS_CHECK_ARG(H > 0 && Hkv > 0 && H % Hkv == 0, "tgis_attn_paged: H (%d) must be a multiple of Hkv (%d)", H, Hkv);
@@ -831,7 +831,7 @@ static int attn_paged_impl(const void* q, int64_t ld_q, const void* k_pool, cons
     TGIS_CHECK_ARG(max_q_len > 0 && max_pages > 0 && num_splits >= 1, "tgis_attn_paged: bad launch bounds");
     TGIS_CHECK_ARG(num_splits == 1 || max_q_len == 1, "tgis_attn_paged: key splits are for decode (max_q_len == 1)");
     TGIS_CHECK_ARG(ld_out == 0 || ld_out == (int64_t)H * D ||
-                       (ld_out == TGIS_LD_FRAGMENTS && max_q_len == 1 && B <= 64 && ((int64_t)H * D) % 64 == 0),
+                       (ld_out == TGIS_LD_FRAGMENTS && (prompts || (max_q_len == 1 && B <= 64)) && ((int64_t)H * D) % 64 == 0),
                    "tgis_attn_paged: out is [tokens, H * D] contiguous (ld_out = 0 or H * D), or — decode, <= 64 sequences — in "
                    "fragment order (ld_out = TGIS_LD_FRAGMENTS)");
     TGIS_CHECK_ARG(!out_cols || ld_out == TGIS_LD_FRAGMENTS, "tgis_attn_paged: columns are re-ordered in fragment order only");
@@ -929,6 +929,13 @@ extern "C" int tgis_attn_paged_rope(const void* q, int64_t ld_q, const void* cos
                    (long)max_q_len);
     return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, 0, nullptr, B, H, Hkv, D, max_q_len, max_ctx,
                            scale, dtype, 1, nullptr, 0, stream, cos, sin, positions);
+}
+
+extern "C" int tgis_attn_paged_fragments(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,
+                                         int64_t max_pages, const int32_t* ctx_lens, const int32_t* cu_seqlens_q, void* out, int64_t B, int H, int Hkv,
+                                         int D, int64_t max_q_len, int64_t max_ctx, float scale, int dtype, void* stream) {
+    return attn_paged_impl(q, ld_q, k_pool, v_pool, block_tables, max_pages, ctx_lens, cu_seqlens_q, out, TGIS_LD_FRAGMENTS, nullptr, B, H, Hkv, D,
+                           max_q_len, max_ctx, scale, dtype, 1, nullptr, 0, stream, nullptr, nullptr, nullptr, true);
 }
 
 extern "C" int tgis_attn_paged_ordered(const void* q, int64_t ld_q, const void* k_pool, const void* v_pool, const int32_t* block_tables,

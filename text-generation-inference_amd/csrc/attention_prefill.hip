@@ -322,13 +322,17 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(AttnPrefillArgs a)
         if (!col_valid[cg]) continue;
         const float ls = total[cg][0];  // every lane of a column holds the column's normaliser
         const float inv = ls > 0.f ? 1.f / ls : 0.f;
-        T* dst = reinterpret_cast<T*>(a.out) + (int64_t)(q0 + t0 + tq[cg]) * a.ld_out + head * D + c * 4;
+        const int64_t tok = q0 + t0 + tq[cg];
+        T* dst = reinterpret_cast<T*>(a.out) + tok * a.ld_out + head * D + c * 4;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             V4 v;
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = from_f32<T>(o[cg][nb][r] * inv);
-            *reinterpret_cast<V4*>(dst + nb * 16) = v;
+            if (a.out_frag)
+                *reinterpret_cast<V4*>(reinterpret_cast<T*>(a.out) + xf_off(tok, head * D + c * 4 + nb * 16, a.ld_out)) = v;
+            else
+                *reinterpret_cast<V4*>(dst + nb * 16) = v;
         }
     }
 }

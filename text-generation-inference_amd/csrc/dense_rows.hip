@@ -1,4 +1,4 @@
-// Dense products of a decode step of a few rows (up to 4; in bf16 up to 32, below) with the norm in front of them and the residual add behind them.
+// Dense products of a decode step of a few rows (up to 4; in bf16 up to 64, below) with the norm in front of them and the residual add behind them.
 //
 // A layer of a small model at one row is seven dependent launches of 3.5 - 11 us for 88 MB of weights, 14 us at the rate of a large copy: split sums
 // that a norm launch adds up, norms of one row on one CU, and projections of 64 column tiles that leave three quarters of the chip idle.  For
@@ -304,10 +304,10 @@ int launch_rows(const RowsArgs& a, int dtype, hipStream_t st) {
 //     waves of the CU ask meanwhile), the residual products with one, two, four steps 6.2 / 6.4 / 7.2.  Fewer units a workgroup than fill one round of 256 take x in more often: one
 //     11.1, two 11.5, three 9.9.
 // bf16 only: T(h w) has its range.
-constexpr int STREAM_ROWS = 32;
+constexpr int STREAM_ROWS = 64;
 struct Rows16Args {
     const bf16* x;       // T(h w) or an activation, fragment order
-    const float* sums;   // [K / 32][32 rows][4]: sums of h^2 of eight columns each
+    const float* sums;   // [K / 32][64 rows][4]: sums of h^2 of eight columns each
     float eps;
     const uint8_t* prep;
     int M, K, N, NT;
@@ -324,41 +324,54 @@ struct Rows16Args {
     bf16 *kpool, *vpool;
     int H, Hkv, D;
 };
+// byte offset of a lane's piece of row `row` (chunk kq of the first 32 k) within a k64-step in fragment order of an operand of K columns
+__device__ __forceinline__ uint32_t frag_lane(int row, int kq, int K) { return (uint32_t)(row >> 5) * 64 * K + kq * 1024 + (row & 31) * 16; }
 __device__ __forceinline__ int64_t sums_off(int m, int k) { return ((int64_t)(k >> 5) * STREAM_ROWS + m) * 4 + ((k >> 3) & 3); }
 
-__global__ __launch_bounds__(256) void rows16_embed_kernel(const int64_t* __restrict__ ids, const bf16* __restrict__ table, const bf16* __restrict__ norm_w,
-                                                           bf16* __restrict__ h, bf16* __restrict__ hw, float* __restrict__ sums, int M, int K, int64_t vocab) {
-    const int at = blockIdx.x * 256 + threadIdx.x, m = at % STREAM_ROWS, k = at / STREAM_ROWS * 8;
-    if (m >= M || k >= K) return;
-    const int64_t id = ids[m];
-    bf16x8 v{}, y;
-    if (id >= 0 && id < vocab) v = ld16<bf16x8>(table + id * K + k);
+// What is left of eight columns k .. k + 7 of row m of h = f: T(h), T(h w) and the sum of h^2
+__device__ __forceinline__ void leave_stream(const float (&f)[8], int m, int k, int K, const bf16* norm_w, bf16* h, bf16* hw, float* sums) {
     const bf16x8 nw = ld16<bf16x8>(norm_w + k);
+    bf16x8 v, y;
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        ss += to_f32(v[e]) * to_f32(v[e]);
-        y[e] = (bf16)(to_f32(v[e]) * to_f32(nw[e]));
+        ss += f[e] * f[e];
+        v[e] = (bf16)f[e];
+        y[e] = (bf16)(f[e] * to_f32(nw[e]));
     }
     st16(h + xf_off(m, k, K), v);
     st16(hw + xf_off(m, k, K), y);
     sums[sums_off(m, k)] = ss;
+}
+// the stream of tokens (ids), or of rows x [M][K] (ids null); R: M rounded up to sixteen
+__global__ __launch_bounds__(256) void rows16_embed_kernel(const int64_t* __restrict__ ids, const bf16* __restrict__ x, const bf16* __restrict__ norm_w,
+                                                           bf16* __restrict__ h, bf16* __restrict__ hw, float* __restrict__ sums, int M, int K, int64_t vocab, int R) {
+    const int at = blockIdx.x * 256 + threadIdx.x, m = at % R, k = at / R * 8;
+    if (m >= M || k >= K) return;
+    const int64_t id = ids ? ids[m] : m;
+    bf16x8 v{};
+    if (id >= 0 && id < vocab) v = ld16<bf16x8>(x + id * K + k);
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = to_f32(v[e]);
+    leave_stream(f, m, k, K, norm_w, h, hw, sums);
 }
 
 // SPW: k64-steps of a wave at most
 template <int KIND, int SPW, int RB>
 __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int units, int per) {
     constexpr int W = 8;
-    static_assert(KIND != ROWS_RESIDUAL && RB <= 2, "the kernel below");
-    __shared__ __attribute__((aligned(16))) float red[2][W][RB][64 * 4];
+    static_assert(KIND != ROWS_RESIDUAL && RB <= 4, "the kernels below");
+    constexpr int BUFS = RB <= 2 ? 2 : 1;                 // of the waves' sums
+    constexpr int FW = RB == 1 ? 1 : RB == 2 ? 2 : 4;     // a unit's outputs are finished by FW waves, unit i's by the (i mod 8 / FW)-th FW
+    __shared__ __attribute__((aligned(16))) float red[BUFS][W][RB][64 * 4];
     __shared__ float part[W][16 * RB];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int K = a.K, steps = K >> 6, mine = (steps - w + W - 1) / W;  // k64-steps w, w + 8, ..
     const int m = lane & 15, kq = lane >> 4;
     const int u0 = blockIdx.x * per, n = min(per, units - u0);
 
-    // the block of rows whose outputs this wave finishes (unit i: waves 2 i and 2 i + 1 mod 8)
-    const int fb = w & 1, frow = fb * 16 + m;
+    const int fb = w & (FW - 1), frow = fb * 16 + m;  // the block of rows whose outputs this wave finishes (RB 3: the fourth wave none)
     int32_t pos = 0, slot = 0;
     if (KIND == ROWS_ROPE) {
         pos = a.positions[min(frow, a.M - 1)];
@@ -367,7 +380,7 @@ __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int uni
     bf16x8 x[RB][SPW][2];
     uint32_t xoff[RB];
 #pragma unroll
-    for (int b = 0; b < RB; ++b) xoff[b] = kq * 1024 + min(b * 16 + m, a.M - 1) * 16;
+    for (int b = 0; b < RB; ++b) xoff[b] = frag_lane(min(b * 16 + m, a.M - 1), kq, a.K);
 #pragma unroll
     for (int j = 0; j < SPW; ++j) {
         const char* xp = reinterpret_cast<const char*>(a.x) + (int64_t)min(w + W * j, steps - 1) * 4096;
@@ -377,6 +390,14 @@ __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int uni
 #pragma unroll
             for (int b = 0; b < RB; ++b) x[b][j][h] = *(const GLOBAL_AS bf16x8*)(xp + xoff[b] + h * 512);
     }
+    // the sums of h^2: SPW / 2 groups of 4 x 32 columns a wave
+    constexpr int SG = (SPW + 1) / 2;
+    f32x4 sq[RB][SG];
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int t = 0; t < SG; ++t)
+            sq[b][t] = *reinterpret_cast<const f32x4*>(a.sums + sums_off(min(b * 16 + m, a.M - 1), min((t * W + w) * 4 + kq, (K >> 5) - 1) * 32));
     const uint32_t woff = kq * 1024 + ((lane & 7) + ((lane >> 3) & 1) * 16) * 16;
     bf16x8 wq[SPW][2];
     auto ask = [&](int u) {
@@ -390,14 +411,6 @@ __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int uni
         }
     };
     ask(u0);
-    // the sums of h^2: SPW / 2 groups of 4 x 32 columns a wave
-    constexpr int SG = (SPW + 1) / 2;
-    f32x4 sq[RB][SG];
-#pragma unroll
-    for (int b = 0; b < RB; ++b)
-#pragma unroll
-        for (int t = 0; t < SG; ++t)
-            sq[b][t] = *reinterpret_cast<const f32x4*>(a.sums + sums_off(min(b * 16 + m, a.M - 1), min((t * W + w) * 4 + kq, (K >> 5) - 1) * 32));
     // ROPE: what unit u's outputs are rotated by, and the bias; asked for early for the first unit that this wave finishes
     const bool second = kq >= 2;  // this lane's columns are of the tile's second half
     bf16x4 cf{}, sf{}, bv{};
@@ -414,7 +427,18 @@ __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int uni
         }
         if (a.bias) bv = *reinterpret_cast<const bf16x4*>(a.bias + head * a.D + dim);
     };
-    if (KIND == ROWS_ROPE) rope_inputs(u0 + min(w >> 1, n - 1));
+    if (KIND == ROWS_ROPE) rope_inputs(u0 + min(w / FW, n - 1));
+
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+        float ss = 0.f;
+#pragma unroll
+        for (int t = 0; t < SG; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss += (t * W + w) * 4 + kq < (K >> 5) ? sq[b][t][e] : 0.f;
+        ss = sum_of_quarters(ss);
+        if (kq == 0) part[w][b * 16 + m] = ss;  // (read behind the first unit's barrier)
+    }
 
     auto unit = [&](int i, bool more) {
         f32x4 acc[RB];
@@ -429,23 +453,12 @@ __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int uni
                     for (int b = 0; b < RB; ++b) acc[b] = mfma16(wq[j][h], x[b][j][h], acc[b]);
             }
         if (more) ask(u0 + i + 1);
-        const int r = i & 1;
+        const int r = i & (BUFS - 1);
+        if (BUFS == 1 && i > 0) __syncthreads();  // the unit before has been read
 #pragma unroll
         for (int b = 0; b < RB; ++b) *reinterpret_cast<f32x4*>(&red[r][w][b][lane * 4]) = acc[b];
-        if (i == 0) {
-#pragma unroll
-            for (int b = 0; b < RB; ++b) {
-                float ss = 0.f;
-#pragma unroll
-                for (int t = 0; t < SG; ++t)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) ss += (t * W + w) * 4 + kq < (K >> 5) ? sq[b][t][e] : 0.f;
-                ss = sum_of_quarters(ss);
-                if (kq == 0) part[w][b * 16 + m] = ss;
-            }
-        }
-        __syncthreads();  // (the sums of the unit that had this buffer before were read in front of a barrier since)
-        if (((w - 2 * i) & (W - 1)) >= RB) return;
+        __syncthreads();  // (two buffers: the one before last was read in front of a barrier since)
+        if (w / FW != i % (W / FW) || fb >= RB) return;
         float tot = 0.f;
 #pragma unroll
         for (int k = 0; k < W; ++k) tot += part[k][frow];
@@ -473,7 +486,7 @@ __global__ __launch_bounds__(512) void dense_rows16_kernel(Rows16Args a, int uni
             }
             if (live && !second) *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.out) + xf_off(frow, tile * 16 + c, a.N >> 1)) = o;
         } else {
-            if (i >= W / 2) rope_inputs(u);
+            if (i >= W / FW) rope_inputs(u);
             const bool roth = head < a.H + a.Hkv;
             bf16x4 o;
 #pragma unroll
@@ -510,7 +523,7 @@ __global__ __launch_bounds__(1024) void dense_rows16_residual_kernel(Rows16Args 
     const uint32_t woff = kq * 1024 + ((lane >> 3) & 1) * 512 + (c0 + (lane & 7)) * 16;
     uint32_t xoff[RB];
 #pragma unroll
-    for (int b = 0; b < RB; ++b) xoff[b] = kq * 1024 + min(b * 16 + m, a.M - 1) * 16;
+    for (int b = 0; b < RB; ++b) xoff[b] = frag_lane(min(b * 16 + m, a.M - 1), kq, a.K);
     bf16x8 wq, x[RB][2];
     auto ask = [&](int s) {
         const char *p = wbase + (int64_t)s * 4096, *xp = reinterpret_cast<const char*>(a.x) + (int64_t)s * 4096;
@@ -568,14 +581,112 @@ __global__ __launch_bounds__(1024) void dense_rows16_residual_kernel(Rows16Args 
     if (kq == 0) a.sums_out[sums_off(frow, col)] = ss;
 }
 
+// RESIDUAL with the k range split over S workgroups a tile, for as many rows as make x of a whole range the larger part of what a workgroup takes in: a tile of 32 columns
+// a workgroup, sums left as slabs [S][N / 4][64 rows][4], which the launch behind adds up: T(x W^T) + T(h) as above, or (`leave`, behind the last layer) the
+// sum as one slab of rows and T(h) as rows for a norm of its own.
+template <int RB>
+__global__ __launch_bounds__(512) void dense_rows16_parts_kernel(Rows16Args a, int S, float* slabs) {
+    constexpr int W = 8;
+    __shared__ __attribute__((aligned(16))) float red[W][2 * RB][64 * 4];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int steps = a.K >> 6, tile = blockIdx.x, split = blockIdx.y, sb = steps * split / S, se = steps * (split + 1) / S;
+    const int m = lane & 15, kq = lane >> 4;
+    const char* wbase = reinterpret_cast<const char*>(a.prep) + (int64_t)tile * steps * 4096;
+    const uint32_t woff = kq * 1024 + m * 16;
+    uint32_t xoff[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) xoff[b] = frag_lane(min(b * 16 + m, a.M - 1), kq, a.K);
+    bf16x8 wq[2][2], x[RB][2];
+    auto ask = [&](int s) {
+        const char *p = wbase + (int64_t)s * 4096, *xp = reinterpret_cast<const char*>(a.x) + (int64_t)s * 4096;
+        PIN_SGPR(p);
+        PIN_SGPR(xp);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) wq[u][h] = __builtin_nontemporal_load((const GLOBAL_AS bf16x8*)(p + woff + h * 512 + u * 256));
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[b][h] = *(const GLOBAL_AS bf16x8*)(xp + xoff[b] + h * 512);
+    };
+    ask(min(sb + w, steps - 1));
+    f32x4 acc[2][RB];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int b = 0; b < RB; ++b) acc[u][b] = f32x4{0, 0, 0, 0};
+    for (int s = sb + w; s < se; s += W) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int b = 0; b < RB; ++b) acc[u][b] = mfma16(wq[u][h], x[b][h], acc[u][b]);
+        if (s + W < se) ask(s + W);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int b = 0; b < RB; ++b) *reinterpret_cast<f32x4*>(&red[w][u * RB + b][lane * 4]) = acc[u][b];
+    __syncthreads();
+    const int u = w / RB, b = w % RB, row = b * 16 + m;
+    if (u >= 2 || row >= a.M) return;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][w][lane * 4]);
+#pragma unroll
+    for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[k][w][lane * 4]);
+    *reinterpret_cast<f32x4*>(slabs + (((int64_t)split * (a.N >> 2) + tile * 8 + u * 4 + kq) * STREAM_ROWS + row) * 4) = v;
+}
+template <int SB, bool LEAVE>
+__global__ __launch_bounds__(256) void rows16_sum_kernel(const float* __restrict__ slabs, int S, const bf16* __restrict__ norm_w, bf16* __restrict__ h, bf16* __restrict__ hw,
+                                                         float* __restrict__ sums, int M, int N, int R) {
+    const int at = blockIdx.x * 256 + threadIdx.x, m = at % R, k = at / R * 8;
+    if (m >= M || k >= N) return;
+    const bf16x8 res = ld16<bf16x8>(h + xf_off(m, k, N));
+    f32x4 lo[SB], hi[SB];
+#pragma unroll
+    for (int s = 0; s < SB; ++s) {
+        const float* p = slabs + (((int64_t)min(s, S - 1) * (N >> 2) + (k >> 2)) * STREAM_ROWS + m) * 4;
+        lo[s] = *reinterpret_cast<const f32x4*>(p);
+        hi[s] = *reinterpret_cast<const f32x4*>(p + STREAM_ROWS * 4);
+    }
+#pragma unroll
+    for (int s = 1; s < SB; ++s)
+        if (s < S) {
+            lo[0] += lo[s];
+            hi[0] += hi[s];
+        }
+    if (LEAVE) {  // hw: rows of T(h); sums: [32-row block][32][N]
+        st16(hw + (int64_t)m * N + k, res);
+        float* o = sums + (int64_t)m * N + k;
+        *reinterpret_cast<f32x4*>(o) = lo[0];
+        *reinterpret_cast<f32x4*>(o + 4) = hi[0];
+    } else {
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = to_f32((bf16)(e < 4 ? lo[0][e & 3] : hi[0][e & 3])) + to_f32(res[e]);
+        leave_stream(f, m, k, N, norm_w, h, hw, sums);
+    }
+}
+
 // Whole steps, us, the other launches of a layer / these (2048 wide, inner 5632, 22 layers; ctx 137): 3, 4 rows 881 / 746 (the launches of up to four rows), 8 rows 964 / 761, 16
-// 990 / 814, 24 1053 / 917, 32 1077 / 970; 768, 2048, 12 layers, 8, 16, 32 rows: 461 / 302, 479 / 318, 541 / 397; 1024, 2816, 16 layers: 568 / 453, 589 / 484, 658 / 595;
-// 1536, 4096, 16 layers: 673 / 542, 701 / 581, 816 / 732.  Wider ones, 4, 8, 16 rows: 2560, 6912, 8 layers 504 / 471, 531 / 480, 569 / 540; 3072,
-// 8192: 543 / 542, 574 / 548, 597 / 585; 4096, 11008, 6 layers 664 / 617, 705 / 630, 748 / 695; there 32 rows 635 / 767, 654 / 776, 828 / 915 by more x than weights.  One and two rows: 716 / 744, 754 / 745, narrower ones 4 -
+// 990 / 814, 24 1053 / 906, 32 1077 / 965, 48 1284 / 1059, 64 1355 / 1135; 768, 2048, 12 layers, 8, 16, 32, 48, 64 rows: 461 / 302, 479 / 318, 541 / 397, 653 /
+// 453, 679 / 503; 1024, 2816, 16 layers: 568 / 453, 589 / 484, 658 / 595;
+// 1536, 4096, 16 layers: 673 / 520, 701 / 564, 816 / 706, 977 / 826, 1052 / 897.  Wider ones, 4, 8, 16 rows: 2560, 6912, 8 layers 504 / 471, 531 / 480, 569 / 540; 3072,
+// 8192: 543 / 542, 574 / 548, 597 / 585; 4096, 11008, 6 layers 664 / 617, 705 / 615, 748 / 676; there 32 rows 635 / 767, 654 / 776, 828 / 915 by more x than weights.  One and two rows: 716 / 744, 754 / 745, narrower ones 4 -
 // 10 % behind the launches of up to four rows, which keep them.
 bool rows16_fits(int64_t M, int64_t K, bool norm) {
     return M >= 1 && M <= STREAM_ROWS && K >= 64 && K % 64 == 0 && K <= (!norm ? 12288 : M <= 16 ? 4096 : 2048);
 }
+// Splits of a residual product's k range: as many as fill the chip with a tile a workgroup, a step for each wave of it; none where x of the whole range is less than 320 KiB.  Whole
+// steps, us, unsplit / these products split: down of 5632 x 2048 at 32, 48, 64 rows 978 / 965, 1094 / 1059, 1211 / 1135, at 24 906 / 909; o of 2048 x 2048 besides at 48, 64 rows 1059 / 1084,
+// 1135 / 1139; down of 4096 x 1536 at 24, 32 rows 659 / 673, 706 / 718, at 48 845 / 826; of 11008 x 4096 at 8, 16 rows 614 / 615, 700 / 676.  `must`: whatever the rows.
+int rows16_splits(int64_t M, int64_t K, int64_t N, bool must) {
+    if (!must && M * K < 160 * 1024) return 0;
+    const int64_t tiles = N / 32;
+    return (int)std::max<int64_t>(1, std::min<int64_t>({(256 + tiles / 2) / tiles, K / 512, 8}));
+}
+int64_t rows16_slab_bytes(int64_t N, int S) { return (int64_t)S * N * STREAM_ROWS * 4; }
 
 template <int KIND, int RB, int SPW>
 void launch_rows16_k(const Rows16Args& a, hipStream_t st) {
@@ -601,7 +712,30 @@ void launch_rows16_rb(const Rows16Args& a, hipStream_t st) {
 template <int KIND>
 int launch_rows16(const Rows16Args& a, hipStream_t st) {
     TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
-    a.M <= 16 ? launch_rows16_rb<KIND, 1>(a, st) : launch_rows16_rb<KIND, 2>(a, st);
+    if (a.M <= 16)
+        launch_rows16_rb<KIND, 1>(a, st);
+    else if (a.M <= 32)
+        launch_rows16_rb<KIND, 2>(a, st);
+    else if (a.M <= 48)
+        launch_rows16_rb<KIND, 3>(a, st);
+    else
+        launch_rows16_rb<KIND, 4>(a, st);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+template <bool LEAVE>
+int launch_rows16_split(const Rows16Args& a, int S, float* slabs, hipStream_t st) {
+    TgisTimedScope timed(TGIS_OP_DENSE_GEMM, st);
+    const dim3 grid((unsigned)a.NT, (unsigned)S);
+    const int R = (a.M + 15) / 16 * 16;
+    const auto parts = R == 16 ? dense_rows16_parts_kernel<1> : R == 32 ? dense_rows16_parts_kernel<2> : R == 48 ? dense_rows16_parts_kernel<3> : dense_rows16_parts_kernel<4>;
+    hipLaunchKernelGGL(parts, grid, dim3(512), 0, st, a, S, slabs);
+    TGIS_CHECK_LAUNCH();
+    const dim3 sgrid((unsigned)cdiv64((int64_t)R * (a.N >> 3), 256));
+    if (S <= 4)
+        hipLaunchKernelGGL((rows16_sum_kernel<4, LEAVE>), sgrid, dim3(256), 0, st, slabs, S, a.norm_w, a.h, a.hw, a.sums_out, a.M, a.N, R);
+    else
+        hipLaunchKernelGGL((rows16_sum_kernel<8, LEAVE>), sgrid, dim3(256), 0, st, slabs, S, a.norm_w, a.h, a.hw, a.sums_out, a.M, a.N, R);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
@@ -698,7 +832,7 @@ extern "C" int tgis_dense_rows_norm_rope(const float* h, const void* norm_w, flo
     return launch_rows<ROWS_ROPE>(a, dtype, (hipStream_t)stream);
 }
 
-// ---- the launches of up to 32 rows ----
+// ---- the launches of up to 64 rows ----
 
 extern "C" int tgis_dense_rows16_ok(int64_t M, int64_t K, int norm) { return rows16_fits(M, K, norm != 0) ? 1 : 0; }
 
@@ -728,29 +862,54 @@ Rows16Args rows16_args(const void* x, const float* sums, float eps, const void* 
 
 }  // namespace
 
-extern "C" int tgis_dense_rows16_embed(const int64_t* ids, const void* table, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
+extern "C" int tgis_dense_rows16_embed(const int64_t* ids, const void* x, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
                                        int64_t vocab, void* stream) {
-    const int rc = rows16_check("tgis_dense_rows16_embed", M, K, vocab, true, table, norm_w, h);
+    const int rc = rows16_check("tgis_dense_rows16_embed", M, K, ids ? vocab : M, true, x, norm_w, h);
     if (rc != TGIS_OK) return rc;
-    TGIS_CHECK_ARG(ids && hw && sums && ((uintptr_t)hw | (uintptr_t)sums) % 16 == 0, "tgis_dense_rows16_embed: null or unaligned tensor");
-    hipLaunchKernelGGL(rows16_embed_kernel, dim3((unsigned)(K / 8 * STREAM_ROWS / 256)), dim3(256), 0, (hipStream_t)stream, ids, (const bf16*)table,
-                       (const bf16*)norm_w, (bf16*)h, (bf16*)hw, sums, (int)M, (int)K, vocab);
+    TGIS_CHECK_ARG(hw && sums && ((uintptr_t)hw | (uintptr_t)sums) % 16 == 0, "tgis_dense_rows16_embed: null or unaligned tensor");
+    const int R = ((int)M + 15) / 16 * 16;
+    hipLaunchKernelGGL(rows16_embed_kernel, dim3((unsigned)cdiv64(K / 8 * R, 256)), dim3(256), 0, (hipStream_t)stream, ids, (const bf16*)x,
+                       (const bf16*)norm_w, (bf16*)h, (bf16*)hw, sums, (int)M, (int)K, ids ? vocab : M, R);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
 
-extern "C" int tgis_dense_rows16_residual(const void* x, const void* prepared, const void* norm_w, void* h, void* hw, float* sums, int64_t M, int64_t K,
-                                          int64_t N, void* stream) {
-    const int rc = rows16_check("tgis_dense_rows16_residual", M, K, N, false, x, prepared, h);
+extern "C" int64_t tgis_dense_rows16_slab_bytes(int64_t M, int64_t K, int64_t N, int leave) {
+    return rows16_slab_bytes(N, rows16_splits(M, K, N, leave != 0));
+}
+
+extern "C" int tgis_dense_rows16_residual(const void* x, const void* prepared, const void* norm_w, void* h, void* hw, float* sums, float* slabs,
+                                          int64_t slabs_bytes, int64_t M, int64_t K, int64_t N, void* stream) {
+    const char* what = "tgis_dense_rows16_residual";
+    const int rc = rows16_check(what, M, K, N, false, x, prepared, h);
     if (rc != TGIS_OK) return rc;
     TGIS_CHECK_ARG(norm_w && hw && sums && ((uintptr_t)norm_w | (uintptr_t)hw | (uintptr_t)sums) % 16 == 0 && N % 64 == 0,
-                   "tgis_dense_rows16_residual: null or unaligned tensor, or a width that is no multiple of 64");
+                   "%s: null or unaligned tensor, or a width that is no multiple of 64", what);
     Rows16Args a = rows16_args(x, nullptr, 0.f, prepared, M, K, N, nullptr, 0);
     a.norm_w = (const bf16*)norm_w;
     a.h = (bf16*)h;
     a.hw = (bf16*)hw;
     a.sums_out = sums;
-    return launch_rows16<ROWS_RESIDUAL>(a, (hipStream_t)stream);
+    const int S = rows16_splits(M, K, N, false);
+    if (S == 0) return launch_rows16<ROWS_RESIDUAL>(a, (hipStream_t)stream);
+    TGIS_CHECK_ARG(slabs && (uintptr_t)slabs % 16 == 0 && slabs_bytes >= rows16_slab_bytes(N, S), "%s: no room for %d partial sums", what, S);
+    return launch_rows16_split<false>(a, S, slabs, (hipStream_t)stream);
+}
+
+extern "C" int tgis_dense_rows16_leave(const void* x, const void* prepared, const void* h, void* h_rows, float* sum_rows, float* slabs, int64_t slabs_bytes,
+                                       int64_t M, int64_t K, int64_t N, void* stream) {
+    const char* what = "tgis_dense_rows16_leave";
+    const int rc = rows16_check(what, M, K, N, false, x, prepared, h);
+    if (rc != TGIS_OK) return rc;
+    const int S = rows16_splits(M, K, N, true);
+    TGIS_CHECK_ARG(h_rows && sum_rows && ((uintptr_t)h_rows | (uintptr_t)sum_rows) % 16 == 0 && N % 64 == 0 && slabs && (uintptr_t)slabs % 16 == 0 &&
+                       slabs_bytes >= rows16_slab_bytes(N, S),
+                   "%s: null or unaligned tensor, a width that is no multiple of 64, or no room for %d partial sums", what, S);
+    Rows16Args a = rows16_args(x, nullptr, 0.f, prepared, M, K, N, nullptr, 0);
+    a.h = const_cast<bf16*>((const bf16*)h);
+    a.hw = (bf16*)h_rows;
+    a.sums_out = sum_rows;
+    return launch_rows16_split<true>(a, S, slabs, (hipStream_t)stream);
 }
 
 extern "C" int tgis_dense_rows16_norm_head(const void* hw, const float* sums, float eps, const void* prepared, float* out, int64_t ldo, int64_t M, int64_t K,

@@ -9,8 +9,35 @@
         if (rc_ != TGIS_OK) return rc_;    \
     } while (0)
 
+// Up to 64 rows in bf16: the launches of dense_rows.hip, six or seven a layer.  A prefill of 47 tokens through 22 layers of 2048, us, the launches below / these:
+// 1519 / 1305 (a layer 54.5 / 43.6: qkv 11.0 / 7.1, o and the norm 10.2 / 7.0, gate | up 16.0 / 12.8, down and the norm 13.0 / 11.9).
+static int rows16_prompt(const TgisLlamaLayer* layers, int n_layers, TgisLlamaPrompt* p, void* stream) {
+    TGIS_CHECK_ARG(p->x && p->hw && p->sums && p->last && p->qkv && p->att && p->act && p->res[0] && p->slabs && p->dtype == TGIS_BF16,
+                   "tgis_llama_prompt: null buffer, or rows that are not bf16");
+    const int64_t T = p->T, HD = (int64_t)p->H * p->D, QKV = HD + 2 * (int64_t)p->Hkv * p->D;
+    TRY(tgis_dense_rows16_embed(nullptr, p->x, layers[0].input_norm, p->h, p->hw, p->sums, T, p->hidden, 0, stream));
+    for (int i = 0; i < n_layers; ++i) {
+        const TgisLlamaLayer& l = layers[i];
+        TRY(tgis_dense_rows16_norm_rope(p->hw, p->sums, p->eps, l.qkv_rope, l.qkv_bias, p->positions, p->slots, p->cos, p->sin, p->qkv, QKV, l.k_pool,
+                                        l.v_pool, T, p->hidden, p->H, p->Hkv, p->D, stream));
+        TRY(tgis_attn_paged_fragments(p->qkv, QKV, l.k_pool, l.v_pool, p->block_tables, p->max_pages, p->ctx_lens, p->cu_seqlens, p->att, p->B, p->H,
+                                      p->Hkv, p->D, p->max_q_len, p->max_ctx, p->scale, p->dtype, stream));
+        TRY(tgis_dense_rows16_residual(p->att, l.o, l.post_norm, p->h, p->hw, p->sums, p->slabs, p->slabs_bytes, T, HD, p->hidden, stream));
+        TRY(tgis_dense_rows16_norm_silu(p->hw, p->sums, p->eps, l.gate_up, p->act, T, p->hidden, 2 * p->inner, stream));
+        if (i + 1 < n_layers)
+            TRY(tgis_dense_rows16_residual(p->act, l.down, layers[i + 1].input_norm, p->h, p->hw, p->sums, p->slabs, p->slabs_bytes, T, p->inner, p->hidden,
+                                           stream));
+        else
+            TRY(tgis_dense_rows16_leave(p->act, l.down, p->h, p->res[0], p->last, p->slabs, p->slabs_bytes, T, p->inner, p->hidden, stream));
+    }
+    p->num_slabs = 1;
+    p->slab_ld = p->hidden;
+    return TGIS_OK;
+}
+
 extern "C" int tgis_llama_prompt(const TgisLlamaLayer* layers, int n_layers, TgisLlamaPrompt* p, void* stream) {
     TGIS_CHECK_ARG(layers && n_layers >= 1 && p && p->T >= 1, "tgis_llama_prompt: bad arguments");
+    if (p->h) return rows16_prompt(layers, n_layers, p, stream);
     TGIS_CHECK_ARG(p->x && p->y && p->qkv && p->att && p->act && p->res[0] && p->res[1] && p->workspace && p->workspace_bytes >= 4096,
                    "tgis_llama_prompt: null buffer");
     const bool tall = p->T >= TGIS_DENSE_TALL_MIN_M;

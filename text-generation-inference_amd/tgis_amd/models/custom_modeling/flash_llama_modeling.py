@@ -356,6 +356,8 @@ class FlashLlamaModel:
         self.num_heads = self.layers[0].self_attn.num_heads
         self.num_key_value_heads = config.num_key_value_heads // process_group.size()
         self.max_positions = 0
+        self._rows16 = {}  # rows -> serves_rows16
+
     def rope_tables(self, dtype, device, max_s: int):
         # Sized once for the model's whole position range, so the tables normally never move.  A longer request
         # still works: PositionRotaryEmbedding keeps the replaced tables allocated, because decode graphs captured
@@ -386,18 +388,51 @@ class FlashLlamaModel:
 
     def forward_rows16(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
         """The same for more rows, in bf16, on the launches there that take the matrix instruction: a native.RowsStream."""
-        norms = [n for layer in self.layers for n in (layer.input_layernorm, layer.post_attention_layernorm)] + [self.norm]
-        h = native.RowsStream.embed(input_ids, self.embed_tokens.weight, norms[0].weight)
+        h = native.RowsStream.embed(input_ids, self.embed_tokens.weight, self.layers[0].input_layernorm.weight)
         cos, sin = self.rope_tables(self.embed_tokens.weight.dtype, h.device, max_s)
+        down = self._rows16_layers(h, cos, sin, position_ids, cu_seqlens_q, kv)
+        native.dense_rows16_residual(*down, h, self.norm.weight)
+        return h
+
+    def _rows16_layers(self, h, cos, sin, position_ids, cu_seqlens_q, kv: KVArgs):
+        """All layers but for the last one's down projection, whose operands it returns."""
         for i, layer in enumerate(self.layers):
             att, mlp = layer.self_attn, layer.mlp
-            qkv = native.dense_rows16_rope(h, norms[2 * i].variance_epsilon, att.query_key_value.linear.rope_handle, att.query_key_value.linear.bias, cos, sin,
-                                           position_ids, kv.slots, kv.cache.k_pool(layer.layer_id), kv.cache.v_pool(layer.layer_id), att.num_heads,
-                                           att.num_key_value_heads, att.head_size)
-            native.dense_rows16_residual(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv, frag=True), att.o_proj.linear.prepared, h, norms[2 * i + 1].weight)
-            act = native.dense_rows16_silu(h, norms[2 * i + 1].variance_epsilon, mlp.gate_up_proj.linear.prepared)
-            native.dense_rows16_residual(act, mlp.down_proj.linear.prepared, h, norms[2 * i + 2].weight)
-        return h
+            if i > 0:
+                native.dense_rows16_residual(*down, h, layer.input_layernorm.weight)
+            qkv = native.dense_rows16_rope(h, layer.input_layernorm.variance_epsilon, att.query_key_value.linear.rope_handle,
+                                           att.query_key_value.linear.bias, cos, sin, position_ids, kv.slots, kv.cache.k_pool(layer.layer_id),
+                                           kv.cache.v_pool(layer.layer_id), att.num_heads, att.num_key_value_heads, att.head_size)
+            native.dense_rows16_residual(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv, frag=True), att.o_proj.linear.prepared, h,
+                                         layer.post_attention_layernorm.weight)
+            down = (native.dense_rows16_silu(h, layer.post_attention_layernorm.variance_epsilon, mlp.gate_up_proj.linear.prepared),
+                    mlp.down_proj.linear.prepared)
+        return down
+
+    def prompt_rows16(self, x, cos, kv: KVArgs) -> bool:
+        """Whether a step of x's rows is a prompt's that the launches of `forward_rows16` serve."""
+        return (DEFER_REDUCE and native.DENSE_ROWS16_MIN_M <= x.shape[0] <= min(native.DENSE_ROWS16_MAX_M, SKINNY_MAX_M) and kv.num_splits == 1
+                and not (kv.max_q_len == 1 and not kv.fresh_prefill) and kv.slots is not None and kv.residual_trace is None
+                and cos.shape[1] * 2 == self.head_size and x.is_contiguous() and self.serves_rows16(x.shape[0]))
+
+    def serves_rows16(self, rows: int) -> bool:
+        got = self._rows16.get(rows)
+        if got is None:
+            got = self._rows16[rows] = self.embed_tokens.weight.dtype == torch.bfloat16 and self.serves_rows(rows, native.dense_rows16_ok)
+        return got
+
+    def serves_rows(self, rows: int, ok) -> bool:
+        """Whether all layers are dense, of one rank, and of shapes that `ok` says are served."""
+        plain = lambda lin: isinstance(lin, FastLinear) and lin.streams and lin.bias is None
+        if self.tp_world_size != 1 or not ok(rows, self.config.hidden_size, True):
+            return False
+        for layer in self.layers:
+            qkv, o = layer.self_attn.query_key_value.linear, layer.self_attn.o_proj.linear
+            gate_up, down = layer.mlp.gate_up_proj.linear, layer.mlp.down_proj.linear
+            if not (isinstance(qkv, FastLinear) and qkv.rope_handle is not None and plain(o) and plain(gate_up) and gate_up.gate_up and plain(down)
+                    and ok(rows, o.in_features, False) and ok(rows, down.in_features, False)):
+                return False
+        return True
 
     def plain_layers(self, count: int, x, cos, kv: KVArgs) -> list:
         """The weights and cache pages of the first `count` layers, as native.llama_prompt takes them, if a step of x's rows is a prompt's and
@@ -445,12 +480,18 @@ class FlashLlamaModel:
         residual = None
         whole = len(self.layers) - kv.cuts_to_ends(hidden_states.shape[0])
         plain = self.plain_layers(whole, hidden_states, cos, kv)
+        rows16 = whole == len(self.layers) and self.prompt_rows16(hidden_states, cos, kv)
         if plain:
             att = self.layers[0].self_attn
             hidden_states, residual = native.llama_prompt(
                 plain, hidden_states, workspace(hidden_states.device), position_ids, kv.slots, cu_seqlens_q, kv.block_tables, kv.ctx_lens, cos, sin,
                 att.num_heads, att.num_key_value_heads, att.head_size, self.layers[0].mlp.intermediate_size, kv.max_q_len, kv.max_ctx,
-                kv.fresh_prefill, self.layers[0].input_layernorm.variance_epsilon, att.softmax_scale)
+                kv.fresh_prefill, self.layers[0].input_layernorm.variance_epsilon, att.softmax_scale, rows16)
+        elif rows16:
+            h = native.RowsStream.of_rows(hidden_states, self.layers[0].input_layernorm.weight)
+            down = self._rows16_layers(h, cos, sin, position_ids, cu_seqlens_q, kv)
+            hidden_states, residual = native.dense_rows16_leave(*down, h)
+            plain = self.layers
         for layer in self.layers[len(plain):whole]:
             hidden_states, residual = layer(hidden_states, residual, cos, sin, position_ids, cu_seqlens_q, kv)
         for layer in self.layers[whole:]:
@@ -498,22 +539,15 @@ class FlashLlamaForCausalLM:
         got = self._rows16_path.get(rows)
         if got is None:
             got = self._rows16_path[rows] = (native.DENSE_ROWS16_MIN_M <= rows <= min(native.DENSE_ROWS16_MAX_M, SKINNY_MAX_M)
-                                             and self.model.embed_tokens.weight.dtype == torch.bfloat16
-                                             and self._serves_rows(rows, native.dense_rows16_ok))
+                                             and self._plain_head() and self.model.serves_rows16(rows))
         return got
 
-    def _serves_rows(self, rows: int, ok=None) -> bool:
-        cfg, ok = self.config, ok or native.dense_rows_ok
-        plain = lambda lin: isinstance(lin, FastLinear) and lin.streams and lin.bias is None
-        if self.model.tp_world_size != 1 or not plain(self.lm_head.linear) or not ok(rows, cfg.hidden_size, True):
-            return False
-        for layer in self.model.layers:
-            qkv, o = layer.self_attn.query_key_value.linear, layer.self_attn.o_proj.linear
-            gate_up, down = layer.mlp.gate_up_proj.linear, layer.mlp.down_proj.linear
-            if not (isinstance(qkv, FastLinear) and qkv.rope_handle is not None and plain(o) and plain(gate_up) and gate_up.gate_up and plain(down)
-                    and ok(rows, o.in_features, False) and ok(rows, down.in_features, False)):
-                return False
-        return True
+    def _serves_rows(self, rows: int) -> bool:
+        return self._plain_head() and self.model.serves_rows(rows, native.dense_rows_ok)
+
+    def _plain_head(self) -> bool:
+        head = self.lm_head.linear
+        return isinstance(head, FastLinear) and head.streams and head.bias is None
 
     def get_input_embeddings(self):
         return self.model.embed_tokens

@@ -98,9 +98,13 @@ SIGNATURES = {
     "tgis_dense_rows16_embed": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_dense_rows16_norm_rope": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64,
                                              _c_i64, _vp]),
-    "tgis_dense_rows16_residual": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_dense_rows16_slab_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_int]),
+    "tgis_dense_rows16_residual": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_dense_rows16_leave": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_dense_rows16_norm_silu": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_dense_rows16_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_attn_paged_fragments": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int, _c_i64, _c_i64, _c_f,
+                                           _c_int, _vp]),
     "tgis_attn_paged": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int,
                                  _c_int, _c_i64, _c_i64, _c_f, _c_int, _c_int, _vp, _c_i64, _vp]),
     "tgis_attn_rotates_q": (_c_int, [_c_int, _c_int, _c_int, _c_i64]),
@@ -829,7 +833,7 @@ def dense_gemm_rope(x: torch.Tensor, w: DenseWeight, bias, cos, sin, positions, 
 
 
 DENSE_ROWS_MAX_M = 4
-DENSE_ROWS16_MIN_M, DENSE_ROWS16_MAX_M = 3, 32  # (one and two rows are sooner done by the launches for a few)
+DENSE_ROWS16_MIN_M, DENSE_ROWS16_MAX_M = 3, 64  # (one and two rows are sooner done by the launches for a few)
 
 
 def dense_rows_ok(M: int, K: int, norm: bool) -> bool:
@@ -888,14 +892,31 @@ class RowsStream:
         self.M, self.width, self.device = M, width, device
         self.h, self.hw = FragAct.empty(M, width, device, torch.bfloat16), FragAct.empty(M, width, device, torch.bfloat16)
         self.sums = torch.empty(width // 8 * DENSE_ROWS16_MAX_M, dtype=torch.float32, device=device)
+        self.slabs = None
+
+    def scratch(self, K: int, leave: bool = False):
+        """(pointer, bytes) of room for the split sums of a product of K columns."""
+        need = load_library().tgis_dense_rows16_slab_bytes(self.M, K, self.width, int(leave))
+        if need and (self.slabs is None or self.slabs.numel() * 4 < need):
+            self.slabs = torch.empty(need // 4, dtype=torch.float32, device=self.device)
+        return _ptr(self.slabs), 0 if self.slabs is None else self.slabs.numel() * 4
 
     @staticmethod
     def embed(ids: torch.Tensor, table: torch.Tensor, norm_w: torch.Tensor) -> "RowsStream":
         assert ids.dtype == torch.int64 and ids.dim() == 1 and ids.is_contiguous() and table.dim() == 2 and table.is_contiguous()
-        assert table.dtype == norm_w.dtype == torch.bfloat16 and norm_w.numel() == table.shape[1]
-        h = RowsStream(ids.shape[0], table.shape[1], table.device)
-        _check(load_library().tgis_dense_rows16_embed(_ptr(ids), _ptr(table), _ptr(norm_w), _ptr(h.h.buf), _ptr(h.hw.buf), _ptr(h.sums), h.M, h.width,
-                                                      table.shape[0], _stream()), "tgis_dense_rows16_embed")
+        return RowsStream._from(ids, table, norm_w, ids.shape[0])
+
+    @staticmethod
+    def of_rows(x: torch.Tensor, norm_w: torch.Tensor) -> "RowsStream":
+        assert x.dim() == 2 and x.is_contiguous()
+        return RowsStream._from(None, x, norm_w, x.shape[0])
+
+    @staticmethod
+    def _from(ids, x, norm_w, M: int) -> "RowsStream":
+        assert x.dtype == norm_w.dtype == torch.bfloat16 and norm_w.numel() == x.shape[1]
+        h = RowsStream(M, x.shape[1], x.device)
+        _check(load_library().tgis_dense_rows16_embed(_ptr(ids), _ptr(x), _ptr(norm_w), _ptr(h.h.buf), _ptr(h.hw.buf), _ptr(h.sums), M, h.width,
+                                                      x.shape[0], _stream()), "tgis_dense_rows16_embed")
         return h
 
 
@@ -912,8 +933,24 @@ def dense_rows16_rope(h: RowsStream, eps: float, w: DenseWeight, bias, cos, sin,
 def dense_rows16_residual(x: FragAct, w: DenseWeight, h: RowsStream, norm_w) -> None:
     """h += x @ w^T, both rounded first, in front of the norm of weight norm_w."""
     assert x.dtype == w.dtype == norm_w.dtype == torch.bfloat16 and x.K == w.K and not w.flags and x.M == h.M and w.N == h.width == norm_w.numel()
-    _check(load_library().tgis_dense_rows16_residual(_ptr(x.buf), _ptr(w.image), _ptr(norm_w), _ptr(h.h.buf), _ptr(h.hw.buf), _ptr(h.sums), h.M, w.K, w.N,
-                                                     _stream()), "tgis_dense_rows16_residual")
+    _check(load_library().tgis_dense_rows16_residual(_ptr(x.buf), _ptr(w.image), _ptr(norm_w), _ptr(h.h.buf), _ptr(h.hw.buf), _ptr(h.sums), *h.scratch(w.K),
+                                                     h.M, w.K, w.N, _stream()), "tgis_dense_rows16_residual")
+
+
+def dense_rows16_leave(x: FragAct, w: DenseWeight, h: RowsStream):
+    """What the add + norm behind the last layer takes: x @ w^T as a Partial, and the stream in front of it as rows."""
+    assert x.dtype == w.dtype == torch.bfloat16 and x.K == w.K and not w.flags and x.M == h.M and w.N == h.width
+    res = torch.empty((h.M, h.width), dtype=w.dtype, device=h.device)
+    rows = torch.empty((h.M + 31) // 32 * 32 * h.width, dtype=torch.float32, device=h.device)
+    _check(load_library().tgis_dense_rows16_leave(_ptr(x.buf), _ptr(w.image), _ptr(h.h.buf), _ptr(res), _ptr(rows), *h.scratch(w.K, True), h.M, w.K, w.N,
+                                                  _stream()), "tgis_dense_rows16_leave")
+    return _partial_rows(rows, h.M, h.width, w.dtype), res
+
+
+def _partial_rows(slab: torch.Tensor, M: int, N: int, dtype) -> "Partial":
+    got = Partial(slab, 1, N, M, N, None)
+    got.dtype = dtype
+    return got
 
 
 def dense_rows16_silu(h: RowsStream, eps: float, w: DenseWeight) -> FragAct:
@@ -939,12 +976,13 @@ class _LlamaPrompt(ctypes.Structure):
     _fields_ = ([(n, _c_i64) for n in ("T", "hidden", "inner", "B", "max_pages", "max_q_len", "max_ctx")]
                 + [(n, _c_int) for n in ("H", "Hkv", "D", "dtype", "fresh")] + [("eps", _c_f), ("scale", _c_f), ("x", _vp)]
                 + [(n, _vp) for n in ("positions", "slots", "cu_seqlens", "block_tables", "ctx_lens", "cos", "sin", "y", "res0", "res1", "qkv", "att", "act", "slabs")]
-                + [("slabs_bytes", _c_i64), ("out", _vp), ("workspace", _vp), ("workspace_bytes", _c_i64), ("slab_ld", _c_i64), ("num_slabs", _c_int)])
+                + [("slabs_bytes", _c_i64), ("out", _vp), ("workspace", _vp), ("workspace_bytes", _c_i64), ("slab_ld", _c_i64), ("num_slabs", _c_int)]
+                + [(n, _vp) for n in ("h", "hw", "sums", "last")])
 
 
 def llama_prompt(layers, x, ws: Workspace, positions, slots, cu_seqlens, block_tables, ctx_lens, cos, sin, H: int, Hkv: int, D: int, inner: int,
-                 max_q_len: int, max_ctx: int, fresh: bool, eps: float, scale: float):
-    """The layers of a dense Llama model on a prompt's rows in one call; layers: LLAMA_LAYER_POINTERS of each (DenseWeight images, tensors or
+                 max_q_len: int, max_ctx: int, fresh: bool, eps: float, scale: float, rows16: bool = False):
+    """rows16: on the launches of dense_rows16_*.  The layers of a dense Llama model on a prompt's rows in one call; layers: LLAMA_LAYER_POINTERS of each (DenseWeight images, tensors or
     None).  Returns what the last layer returns: (hidden states, a Partial up to PARTIAL_MAX_M rows, and the residual stream)."""
     lib = load_library()
     T, hidden = x.shape
@@ -955,6 +993,19 @@ def llama_prompt(layers, x, ws: Workspace, positions, slots, cu_seqlens, block_t
     tall = T >= DENSE_TALL_MIN_M
     qkv_cols = (H + 2 * Hkv) * D
     new = lambda cols: torch.empty((T, cols), dtype=x.dtype, device=x.device)
+    if rows16:
+        h = RowsStream(T, hidden, x.device)
+        qkv, res0, att, act = new(qkv_cols), new(hidden), FragAct.empty(T, H * D, x.device, x.dtype), FragAct.empty(T, inner, x.device, x.dtype)
+        last = torch.empty((T + 31) // 32 * 32 * hidden, dtype=torch.float32, device=x.device)
+        h.scratch(H * D)
+        h.scratch(inner)
+        slabs, nbytes = h.scratch(inner, leave=True)
+        p = _LlamaPrompt(T, hidden, inner, block_tables.shape[0], block_tables.shape[1], max_q_len, max_ctx, H, Hkv, D, dtype_code(x.dtype), int(fresh),
+                         eps, scale, _ptr(x), _ptr(positions), _ptr(slots), _ptr(cu_seqlens), _ptr(block_tables), _ptr(ctx_lens), _ptr(cos), _ptr(sin),
+                         None, _ptr(res0), None, _ptr(qkv), _ptr(att.buf), _ptr(act.buf), slabs, nbytes, None, None, 0, 0, 0, _ptr(h.h.buf),
+                         _ptr(h.hw.buf), _ptr(h.sums), _ptr(last))
+        _check(lib.tgis_llama_prompt(table, len(layers), ctypes.byref(p), _stream()), "tgis_llama_prompt")
+        return _partial_rows(last, T, hidden, x.dtype), res0
     y, res0, res1, qkv, att, act = new(hidden), new(hidden), new(hidden), new(qkv_cols), new(H * D), new(inner)
     out = slabs = None
     nbytes = 0
@@ -1124,7 +1175,14 @@ def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_
     assert block_tables.dtype == torch.int32 and ctx_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
     assert block_tables.is_contiguous()
     if isinstance(out, FragAct):
-        assert max_q_len == 1 and out.K == H * D and out.M == B and out.dtype == q.dtype
+        assert out.K == H * D and out.M == q.shape[0] and out.dtype == q.dtype
+        if max_q_len > 1:
+            assert num_splits == 1 and out_cols is None and rope is None
+            _check(load_library().tgis_attn_paged_fragments(
+                _ptr(q), ld_q, _ptr(k_pool), _ptr(v_pool), _ptr(block_tables), block_tables.shape[1], _ptr(ctx_lens), _ptr(cu_seqlens_q), _ptr(out.buf), B,
+                H, Hkv, D, max_q_len, max_ctx, float(scale), dtype_code(q.dtype), _stream()), "tgis_attn_paged_fragments")
+            return out
+        assert out.M == B
         optr, ldo = _ptr(out.buf), LD_FRAGMENTS
     else:
         assert out.is_contiguous()
