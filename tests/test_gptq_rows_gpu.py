@@ -1,0 +1,211 @@
+"""-m gpu: the int4 decode products of csrc/gptq_rows.hip against float64, and decode steps on them against `forward`."""
+import pytest
+import torch
+
+from oracle import ops_ref
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -11
+
+
+def weight(K, N, groupsize, dev, **kw):
+    """A prepared matrix and what it stands for, in the order of the checkpoint's rows, in float64."""
+    from tgis_amd import native
+
+    qw, qz, sc, gi = ops_ref.make_gptq_tensors(K, N, groupsize, seed=K + N, w_std=K ** -0.5)
+    dense = ops_ref.gptq_dequant(qw, qz, sc, gi, groupsize).half().double()
+    return native.GptqWeight(*(torch.from_numpy(t).to(dev) for t in (qw, qz, sc)), None, 4, groupsize, **kw), dense
+
+
+def norm_input(K, g, dev, shuffled, top=1.5):
+    from tgis_amd import native
+
+    w = ((torch.rand(K, generator=g) + 0.5) * top / 1.5).half()
+    places = torch.randperm(K, generator=g).int() if shuffled else None
+    return native.Int4NormInput(w.to(dev), None if places is None else places.to(dev)), w, places
+
+
+def in_places(x, places):
+    return x if places is None else torch.empty_like(x).index_copy_(1, places.long(), x)
+
+
+def to_stream(h, norm, w, places, dev):
+    """An fp32 stream [M, width] in front of `norm`; rows past M poisoned."""
+    from tgis_amd import native
+
+    M, width = h.shape
+    stream = native.Int4RowsStream(M, width, dev)
+    stream.unit = norm.unit
+    stream.h.copy_(h.half())
+    full = torch.full((32, width), float("nan"))
+    full[:M] = in_places(h * w.float() * norm.unit, places)
+    stream.hw.buf.copy_(native.FragAct.from_rows(full.half()).buf)
+    sums = torch.full((16, width // 16), float("nan"))
+    sums[:M] = (h * h).view(M, -1, 16).sum(-1)
+    stream.sums.copy_(sums.view(16, -1, 4).transpose(0, 1).reshape(-1))
+    return stream
+
+
+def check_stream(stream, want, slack, norm, w, places):
+    """T(h), T(h w unit) where it is wanted and the sums of h^2 of h = want up to slack; rows past M as they were."""
+    M, width = want.shape
+    assert ((stream.h.cpu().double() - want).abs() <= slack + U * want.abs()).all()
+    y, ys = (in_places(t * w.double() * norm.unit, places) for t in (want, slack))
+    rows = type(stream.hw)(stream.hw.buf, 32, width).to_rows().cpu().double()
+    assert ((rows[:M] - y).abs() <= ys + U * y.abs() + 2.0 ** -25).all() and bool(rows[M:].isnan().all())
+    sums = stream.sums.cpu().view(-1, 16, 4).transpose(0, 1).reshape(16, -1).double()
+    assert ((sums[:M] - (want * want).view(M, -1, 16).sum(-1)).abs() <= (2 * slack * want.abs() + slack * slack).view(M, -1, 16).sum(-1) + 1e-5).all()
+    assert bool(sums[M:].isnan().all())
+
+
+# the norm's weight below and above one; the width: steps of 64 that no wave shares evenly
+@pytest.mark.parametrize("M,shuffled,top", [(1, False, 0.06), (16, True, 1.5), (11, False, 30.0)])
+def test_embed(gpu_device, M, shuffled, top):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(M)
+    K, vocab = 1088, 50
+    norm, w, places = norm_input(K, g, gpu_device, shuffled, top)
+    assert 0.5 <= float(w.abs().max()) * norm.unit < 1.0
+    table, ids = torch.randn(vocab, K, generator=g).half(), torch.randint(0, vocab, (M,), generator=g)
+    ids[0] = vocab  # (zeros)
+    got = native.Int4RowsStream.embed(ids.to(gpu_device), table.to(gpu_device), norm)
+    want = table.double()[ids.clamp(max=vocab - 1)]
+    want[0] = 0.0
+    assert torch.equal(got.h.cpu().double(), want)
+    rows = got.hw.to_rows().cpu().double()
+    y = in_places(want * w.double() * norm.unit, places)
+    assert ((rows - y).abs() <= U * y.abs() + 2.0 ** -25).all()
+    sums = got.sums.cpu().view(-1, 16, 4).transpose(0, 1).reshape(16, -1)[:M].double()
+    assert ((sums - (want * want).view(M, -1, 16).sum(-1)).abs() <= 1e-5 * sums).all()
+
+
+# K: fewer steps of 128 than waves, one more than a round of them, every number of steps that a wave keeps; groups of one and of several steps of 64, and one group
+@pytest.mark.parametrize("M", [1, 11, 16])
+@pytest.mark.parametrize("K,N,groupsize", [(128, 64, 64), (1152, 192, 128), (2176, 2048, 128), (4096, 128, 4096), (6272, 64, 64), (8192, 64, 256), (12288, 64, 128)])
+def test_residual(gpu_device, M, K, N, groupsize):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(M + K)
+    image, dense = weight(K, N, groupsize, gpu_device)
+    norm, w, places = norm_input(N, g, gpu_device, M == 11)
+    x, h = torch.randn(M, K, generator=g).half(), torch.randn(M, N, generator=g)
+    y = x.double() @ dense
+    want = y.half().double() + h.half().double()
+    # the product's rounding may fall the other way (a step of it), and then the stream's
+    slack = 2 * U * y.abs() + 1e-5
+    stream = to_stream(h, norm, w, places, gpu_device)
+    frag = native.FragAct.from_rows(torch.cat([x, torch.full((32 - M, K), float("nan"), dtype=torch.float16)]).to(gpu_device))
+    native.gptq_rows_residual(native.FragAct(frag.buf, M, K), image, stream, norm)
+    check_stream(stream, want, slack, norm, w, places)
+    stream = to_stream(h, norm, w, places, gpu_device)
+    native.gptq_rows_sum(native.gptq_gemm_partial(native.FragAct(frag.buf, M, K), image), stream, norm)
+    check_stream(stream, want, slack, norm, w, places)
+
+
+# ff: turns of one, two and three units, a last workgroup that has fewer; K: the products of sixteen waves, and of steps that are left over
+@pytest.mark.parametrize("M", [1, 13, 16])
+@pytest.mark.parametrize("K,ff,groupsize", [(128, 64, 128), (1152, 2112, 128), (2048, 4160, 64), (4096, 6208, 128), (5120, 128, 128), (6272, 64, 128), (8192, 64, 128)])
+def test_norm_silu(gpu_device, M, K, ff, groupsize):
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(M + K)
+    image, dense = weight(K, 2 * ff, groupsize, gpu_device, gate_up=True)
+    norm, w, _ = norm_input(K, g, gpu_device, False, 0.1)
+    h = torch.randn(M, K, generator=g) * 3
+    x = (h * w.float() * norm.unit).half().double() / norm.unit / torch.sqrt((h.double() ** 2).mean(-1, keepdim=True) + 1e-5)  # (what the launch multiplies by)
+    gate, up = (x @ dense).split(ff, -1)
+    act = native.gptq_rows_silu(to_stream(h, norm, w, None, gpu_device), 1e-5, image).to_rows().cpu().double()
+    # a rounding that falls the other way for gate, SiLU(gate) (whose slope is below 1.1), up and the result; fp32 sums of K terms of size 0.1 K ** -0.5
+    s = torch.nn.functional.silu(gate)
+    tol = U * ((s * up).abs() * 4 + 1.1 * (gate * up).abs()) + 2e-5 * (1 + up.abs() + s.abs())
+    assert ((act - s * up).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("M", [1, 13, 16])
+@pytest.mark.parametrize("K,H,Hkv,D,bias", [(2048, 32, 4, 64, False), (384, 3, 1, 32, True), (4096, 32, 32, 128, True), (8192, 2, 1, 128, False), (128, 128, 16, 128, True), (256, 224, 16, 128, False)])
+def test_norm_rope(gpu_device, M, K, H, Hkv, D, bias):
+    """The same launch as norm + gptq_gemm_rope: q, and the pages that it wrote, element for element within roundings."""
+    from tgis_amd import native
+
+    dev = lambda t: None if t is None else t.to(gpu_device)
+    g = torch.Generator().manual_seed(M + K)
+    N, pages = (H + 2 * Hkv) * D, 3
+    image, _ = weight(K, N, 128, gpu_device, rope=(D, H + Hkv))
+    norm, w, _ = norm_input(K, g, gpu_device, False)
+    h, b = torch.randn(M, K, generator=g) * 2, torch.randn(N, generator=g).half() if bias else None
+    angle = torch.outer(torch.arange(100), 10000.0 ** (-torch.arange(0, D, 2) / D))
+    cos, sin = angle.cos().half(), angle.sin().half()
+    pos, slots = torch.randint(0, 100, (M,), generator=g).int(), torch.randperm(pages * 32, generator=g)[:M].int()
+    pools = [torch.full((pages, Hkv, 32 * D), 7.0, dtype=torch.float16, device=gpu_device) for _ in range(4)]
+    q = native.gptq_rows_rope(to_stream(h, norm, w, None, gpu_device), 1e-5, image, dev(b), dev(cos), dev(sin), dev(pos), dev(slots), pools[0], pools[1], H, Hkv, D)
+    hd = h.double()
+    x = (hd / torch.sqrt((hd * hd).mean(-1, keepdim=True) + 1e-5) * w.double()).half()
+    want = native.gptq_gemm_rope(dev(x), image, dev(b), dev(cos), dev(sin), dev(pos), dev(slots), pools[2], pools[3], H, Hkv, D)
+    # roundings of the result, of a pair of size up to 8 in front of its rotation, and of the operands in front of and behind the norm: K terms of at most 2 u times a
+    # weight of size K ** -0.5 each, six times their deviation
+    for got, ref in ((q[:, :H * D], want[:, :H * D]), (pools[0], pools[2]), (pools[1], pools[3])):
+        got, ref = got.cpu().double(), ref.cpu().double()
+        assert ((got - ref).abs() <= 2 * U * ref.abs() + 16 * U + 12 * U).all()
+
+
+def test_refusals(gpu_device):
+    from tgis_amd import native
+
+    image, _ = weight(128, 64, 64, gpu_device)
+    for M, K, N, groups, norm, ok in [(16, 128, 64, 2, True, True), (17, 128, 64, 2, True, False), (0, 128, 64, 2, True, False), (1, 192, 64, 3, True, False),
+                                      (1, 8320, 64, 65, True, False), (1, 8320, 64, 65, False, True), (1, 12416, 64, 97, False, False), (1, 384, 64, 2, True, False),
+                                      (1, 128, 40, 1, True, False)]:
+        assert native.load_library().tgis_gptq_rows_ok(M, K, N, groups, int(norm)) == int(ok), (M, K, N, groups, norm)
+    with pytest.raises(RuntimeError, match="up to 16 rows"):
+        stream = native.Int4RowsStream(17, 64, gpu_device)
+        native.gptq_rows_residual(native.FragAct.empty(17, 128, gpu_device), image, stream, native.Int4NormInput(torch.ones(64, dtype=torch.float16, device=gpu_device)))
+
+
+def decode(lm, cfg, rows, steps=4):
+    """Prompts of different lengths and forced tokens behind them: every step's logits."""
+    from tgis_amd.testing import SyntheticTokenizer, make_batch_pb
+
+    lens = [5 + 7 * i % 40 for i in range(rows)]
+    forced = torch.randint(3, cfg.vocab_size, (steps, rows), generator=torch.Generator().manual_seed(rows)).cuda()
+    taken, run = [], lm._process_new_tokens
+    lm._process_new_tokens = lambda batch, out, *a, **k: taken.append(out.clone()) or run(batch, out, *a, **k)
+    with lm.context_manager():
+        batch, errors = lm.batch_type.from_pb(make_batch_pb(lens, max_new=steps + 2), SyntheticTokenizer(cfg.vocab_size), lm.dtype, lm.device, lm.word_embeddings,
+                                              None, lm.use_position_ids)
+        assert not errors
+        lm.generate_token(batch, first=True)
+        for tokens in forced:
+            batch.input_ids = tokens
+            lm.generate_token(batch)
+    batch.release()
+    return taken
+
+
+@pytest.mark.parametrize("act_order", [False, True])
+@pytest.mark.parametrize("rows", [1, 5, 11])
+def test_same_steps(gpu_device, monkeypatch, rows, act_order):
+    from oracle.tiny_models import TinyLlamaConfig, tiny_llama_tensors
+    from tgis_amd.inference_engine.synthetic import InferenceEngine
+    from tgis_amd.models.custom_modeling.flash_llama_modeling import FlashLlamaModel, LlamaConfig
+    from tgis_amd.models.flash_causal_lm import FlashCausalLM
+    from tgis_amd.testing import SyntheticTokenizer
+
+    cfg = LlamaConfig(**TinyLlamaConfig(hidden_size=1024, intermediate_size=2048, num_attention_heads=16, num_key_value_heads=8, num_hidden_layers=3).to_dict())
+    tensors = tiny_llama_tensors(cfg, seed=3, quantize="gptq", groupsize=64, act_order=act_order)
+
+    def model():
+        eng = InferenceEngine({k: v.clone() for k, v in tensors.items()}, cfg, torch.float16, "gptq", tokenizer=SyntheticTokenizer(cfg.vocab_size), gptq_groupsize=64)
+        return FlashCausalLM("synthetic", None, "synthetic", torch.float16, "gptq", engine=eng, kv_cache_pages=64)
+
+    calls, run = [], FlashLlamaModel.forward_int4_rows
+    monkeypatch.setattr(FlashLlamaModel, "forward_int4_rows", lambda self, ids, *a: calls.append(ids.shape[0]) or run(self, ids, *a))
+    got = decode(model(), cfg, rows)
+    assert calls == [{1: 1, 5: 8, 11: 16}[rows]] * 2  # a warm-up and a capture, with the rows of the bucket
+    monkeypatch.setattr(FlashLlamaModel, "serves_int4_rows", lambda self, n: False)
+    want = decode(model(), cfg, rows)
+    assert len(calls) == 2 and len(got) == len(want) == 5 and torch.equal(got[0], want[0])
+    # sums in another order: here and there a value rounds to the other side (a step of the dtype), which three layers carry on: below eight steps in the norm of all
+    for a, b in zip(got[1:], want[1:]):
+        a, b = a.double(), b.double()
+        assert float((a - b).norm() / b.norm()) < 8 * U

@@ -22,6 +22,7 @@ from tgis_amd.utils.layers import (
     DEFER_REDUCE,
     DENSE_TALL,
     SKINNY_MAX_M,
+    Ex4bitLinearV2,
     FastLinear,
     PositionRotaryEmbedding,
     TensorParallelColumnLinear,
@@ -357,6 +358,7 @@ class FlashLlamaModel:
         self.num_key_value_heads = config.num_key_value_heads // process_group.size()
         self.max_positions = 0
         self._rows16 = {}  # rows -> serves_rows16
+        self.int4_norms, self._int4_rows = None, {}  # prepare_int4_rows; rows -> serves_int4_rows
 
     def rope_tables(self, dtype, device, max_s: int):
         # Sized once for the model's whole position range, so the tables normally never move.  A longer request
@@ -408,6 +410,56 @@ class FlashLlamaModel:
             down = (native.dense_rows16_silu(h, layer.post_attention_layernorm.variance_epsilon, mlp.gate_up_proj.linear.prepared),
                     mlp.down_proj.linear.prepared)
         return down
+
+    def forward_int4_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
+        """A decode step of up to 16 rows of an int4 model on the launches of csrc/gptq_rows.hip: the normed hidden states.  Five launches a layer; the values are those of
+        `forward` but for the order of the sums and where the norm's 1 / rms is multiplied in."""
+        qkv_norms, mlp_norms = self.int4_norms
+        table = self.embed_tokens.weight
+        h = native.Int4RowsStream.embed(input_ids, table, qkv_norms[0])
+        cos, sin = self.rope_tables(table.dtype, h.device, max_s)
+        for i, layer in enumerate(self.layers):
+            att, mlp = layer.self_attn, layer.mlp
+            if i > 0 and native.gptq_rows_ok(h.M, down.ordered, False):
+                native.gptq_rows_residual(act, down.ordered, h, qkv_norms[i])
+            elif i > 0:  # (a long k range is split over workgroups)
+                native.gptq_rows_sum(native.gptq_gemm_partial(act, down.ordered), h, qkv_norms[i])
+            qkv = native.gptq_rows_rope(h, layer.input_layernorm.variance_epsilon, att.query_key_value.linear.rope_handle, att.query_key_value.linear.bias, cos, sin,
+                                        position_ids, kv.slots, kv.cache.k_pool(layer.layer_id), kv.cache.v_pool(layer.layer_id), att.num_heads,
+                                        att.num_key_value_heads, att.head_size)
+            native.gptq_rows_residual(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv), att.o_proj.linear.ordered, h, mlp_norms[i])
+            act = native.gptq_rows_silu(h, layer.post_attention_layernorm.variance_epsilon, mlp.gate_up_proj.linear.ordered)
+            down = mlp.down_proj.linear
+        return self.norm(self.layers[-1].mlp.down_proj(act, partial=True), h.h)[0]
+
+    def prepare_int4_rows(self):
+        """Once the int4 matrices are prepared: the norms as `forward_int4_rows` takes them, if all layers are int4, of one rank, in f16 and without a bias but that of
+        qkv, and the orders of act-order matrices are ones that their operands' producers write."""
+        self.int4_norms, self._int4_rows = None, {}
+        if self.tp_world_size != 1 or self.embed_tokens.weight.dtype != torch.float16:
+            return
+        for layer in self.layers:
+            att, mlp = layer.self_attn, layer.mlp
+            qkv, o, gate_up, down = lins = (att.query_key_value.linear, att.o_proj.linear, mlp.gate_up_proj.linear, mlp.down_proj.linear)
+            if (not all(isinstance(lin, Ex4bitLinearV2) for lin in lins) or qkv.rope_handle is None or not gate_up.gate_up or down.perm is not None
+                    or any(lin.bias is not None for lin in lins[1:]) or any(lin.perm is not None and lin.places() is None for lin in lins[:3])):
+                return
+        self.int4_norms = ([native.Int4NormInput(layer.input_layernorm.weight, layer.self_attn.query_key_value.linear.places()) for layer in self.layers],
+                           [native.Int4NormInput(layer.post_attention_layernorm.weight, layer.mlp.gate_up_proj.linear.places()) for layer in self.layers])
+
+    def serves_int4_rows(self, rows: int) -> bool:
+        got = self._int4_rows.get(rows)
+        if got is None:
+            got = rows <= native.GPTQ_ROWS_MAX_M and self.int4_norms is not None
+            for layer in self.layers if got else ():
+                att, mlp = layer.self_attn, layer.mlp
+                o = att.o_proj.linear
+                got = (got and native.gptq_rows_ok(rows, att.query_key_value.linear.rope_handle, True) and native.gptq_rows_ok(rows, mlp.gate_up_proj.linear.ordered, True)
+                       and native.gptq_rows_ok(rows, o.ordered, False)
+                       and o.wants_fragments(rows, gathers=att.out_places is not None) and mlp.down_proj.linear.wants_fragments(rows)
+                       and mlp.intermediate_size % 64 == 0)
+            self._int4_rows[rows] = got
+        return got
 
     def prompt_rows16(self, x, cos, kv: KVArgs) -> bool:
         """Whether a step of x's rows is a prompt's that the launches of `forward_rows16` serve."""
@@ -526,6 +578,7 @@ class FlashLlamaForCausalLM:
             o_proj = layer.self_attn.o_proj.linear
             if hasattr(o_proj, "places"):
                 layer.self_attn.out_places = o_proj.places()
+        self.model.prepare_int4_rows()
 
     def rows_path(self, rows: int) -> bool:
         """Whether a decode step of `rows` rows runs on the launches that norm their operand themselves (FlashLlamaModel.forward_rows)."""
@@ -569,6 +622,8 @@ class FlashLlamaForCausalLM:
             norm, head = self.model.norm, self.lm_head.linear
             if isinstance(h, native.RowsStream):
                 return native.dense_rows16_head(h, norm.variance_epsilon, head.prepared)
+            if h is None and self.model.serves_int4_rows(rows) and DEFER_REDUCE:
+                return self.lm_head(self.model.forward_int4_rows(*step))
             if h is not None:
                 return native.dense_rows_head(h, norm.weight, norm.variance_epsilon, head.prepared)
         hidden_states = self.model(input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv)

@@ -8,6 +8,7 @@ if the library is missing or a call fails, an exception is raised.
 """
 import copy
 import ctypes
+import math
 import os
 from typing import Optional
 
@@ -103,6 +104,13 @@ SIGNATURES = {
     "tgis_dense_rows16_leave": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_dense_rows16_norm_silu": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_dense_rows16_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_gptq_rows_ok": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int]),
+    "tgis_gptq_rows_embed": (_c_int, [_vp, _vp, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_gptq_rows_residual": (_c_int, [_vp, _vp, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_gptq_rows_sum": (_c_int, [_vp, _c_int, _c_i64, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _vp]),
+    "tgis_gptq_rows_norm_silu": (_c_int, [_vp, _vp, _c_f, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_gptq_rows_norm_rope": (_c_int, [_vp, _vp, _c_f, _c_f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                          _c_i64, _vp]),
     "tgis_attn_paged_fragments": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_int, _c_int, _c_int, _c_i64, _c_i64, _c_f,
                                            _c_int, _vp]),
     "tgis_attn_paged": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_i64, _c_int, _c_int,
@@ -966,6 +974,79 @@ def dense_rows16_head(h: RowsStream, eps: float, w: DenseWeight) -> torch.Tensor
     out = torch.empty((h.M, w.N), dtype=torch.float32, device=h.device)
     _check(load_library().tgis_dense_rows16_norm_head(_ptr(h.hw.buf), _ptr(h.sums), float(eps), _ptr(w.image), _ptr(out), out.stride(0), h.M, w.K, w.N,
                                                       _stream()), "tgis_dense_rows16_norm_head")
+    return out
+
+
+GPTQ_ROWS_MAX_M = 16
+
+
+def gptq_rows_ok(M: int, w: GptqWeight, norm: bool) -> bool:
+    """Whether the launches below serve M rows of this int4 matrix (in the order of its image); norm: of one of those that norm."""
+    return bool(load_library().tgis_gptq_rows_ok(M, w.K, w.N, w.groups, int(norm)))
+
+
+class Int4NormInput:
+    """What a norm in front of an int4 product makes of the stream: its weight, the power of two by which that is at most one, and where the product wants its columns."""
+
+    def __init__(self, weight: torch.Tensor, places: Optional[torch.Tensor] = None):
+        top = float(weight.abs().max()) if weight.numel() else 0.0
+        self.weight, self.places = weight, places
+        self.unit = 2.0 ** -math.frexp(top)[1] if 0.0 < top < math.inf else 1.0
+
+
+class Int4RowsStream:
+    """The residual stream of up to GPTQ_ROWS_MAX_M rows in front of a norm and an int4 product (include/tgis_hip.h): T(h) as rows, the product's operand, sums of h^2."""
+
+    def __init__(self, M: int, width: int, device):
+        self.M, self.width, self.device = M, width, device
+        self.h = torch.empty((M, width), dtype=torch.float16, device=device)
+        self.hw = FragAct.empty(M, width, device)
+        self.sums = torch.empty(width // 16 * GPTQ_ROWS_MAX_M, dtype=torch.float32, device=device)
+        self.unit = 1.0
+
+    @staticmethod
+    def embed(ids: torch.Tensor, table: torch.Tensor, norm: Int4NormInput) -> "Int4RowsStream":
+        assert ids.dtype == torch.int64 and ids.dim() == 1 and ids.is_contiguous() and table.dim() == 2 and table.is_contiguous()
+        assert table.dtype == norm.weight.dtype == torch.float16 and norm.weight.numel() == table.shape[1]
+        h = Int4RowsStream(ids.shape[0], table.shape[1], table.device)
+        h.unit = norm.unit
+        _check(load_library().tgis_gptq_rows_embed(_ptr(ids), _ptr(table), _ptr(norm.weight), _ptr(norm.places), norm.unit, _ptr(h.h), _ptr(h.hw.buf), _ptr(h.sums),
+                                                   h.M, h.width, table.shape[0], _stream()), "tgis_gptq_rows_embed")
+        return h
+
+
+def gptq_rows_residual(x: FragAct, w: GptqWeight, h: Int4RowsStream, norm: Int4NormInput) -> None:
+    """h += x @ W, both rounded first, in front of `norm`."""
+    assert x.dtype == norm.weight.dtype == torch.float16 and x.K == w.K and not w.flags and x.M == h.M and w.N == h.width == norm.weight.numel()
+    h.unit = norm.unit
+    _check(load_library().tgis_gptq_rows_residual(_ptr(x.buf), _ptr(w.image), _ptr(norm.weight), _ptr(norm.places), norm.unit, _ptr(h.h), _ptr(h.hw.buf), _ptr(h.sums),
+                                                  h.M, w.K, w.N, w.groups, _stream()), "tgis_gptq_rows_residual")
+
+
+def gptq_rows_sum(part: "Partial", h: Int4RowsStream, norm: Int4NormInput) -> None:
+    """h += what a gptq_gemm_partial left, in front of `norm`."""
+    assert part.bias is None and part.M == h.M and part.N == h.width == norm.weight.numel()
+    h.unit = norm.unit
+    _check(load_library().tgis_gptq_rows_sum(_ptr(part.slabs), part.S, part.ld, _ptr(norm.weight), _ptr(norm.places), norm.unit, _ptr(h.h), _ptr(h.hw.buf), _ptr(h.sums),
+                                             h.M, h.width, _stream()), "tgis_gptq_rows_sum")
+
+
+def gptq_rows_silu(h: Int4RowsStream, eps: float, w: GptqWeight) -> FragAct:
+    assert w.flags == 1 and w.K == h.width
+    out = FragAct.empty(h.M, w.N // 2, h.device)
+    _check(load_library().tgis_gptq_rows_norm_silu(_ptr(h.hw.buf), _ptr(h.sums), float(eps), h.unit, _ptr(w.image), _ptr(out.buf), h.M, w.K, w.N, w.groups, _stream()),
+           "tgis_gptq_rows_norm_silu")
+    return out
+
+
+def gptq_rows_rope(h: Int4RowsStream, eps: float, w: GptqWeight, bias, cos, sin, positions, slots, k_pool, v_pool, H: int, Hkv: int, D: int) -> torch.Tensor:
+    """gptq_gemm_rope of the normed stream."""
+    assert w.flags & 2 and w.N == (H + 2 * Hkv) * D and w.K == h.width and cos.dtype == torch.float16 and cos.shape[1] * 2 == D
+    assert positions.dtype == torch.int32 and slots.dtype == torch.int32
+    out = torch.empty((h.M, w.N), dtype=torch.float16, device=h.device)
+    _check(load_library().tgis_gptq_rows_norm_rope(
+        _ptr(h.hw.buf), _ptr(h.sums), float(eps), h.unit, _ptr(w.image), _ptr(bias), _ptr(positions), _ptr(slots), _ptr(cos), _ptr(sin), _ptr(out), out.stride(0),
+        _ptr(k_pool), _ptr(v_pool), h.M, w.K, w.groups, H, Hkv, D, _stream()), "tgis_gptq_rows_norm_rope")
     return out
 
 
