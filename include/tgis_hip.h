@@ -259,9 +259,10 @@ int tgis_dense_rows16_norm_silu(const void* hw, const float* sums, float eps, co
                                 void* stream);
 int tgis_dense_rows16_norm_head(const void* hw, const float* sums, float eps, const void* prepared, float* out, int64_t ldo, int64_t M, int64_t K,
                                 int64_t N, void* stream);
-/* The same for int4 weights (the images of tgis_gptq_prepare) in f16: decode steps of up to 16 rows, K a multiple of 128 up to 12288, where it norms 8192, groups of 64 2^n rows.
+/* The same for int4 weights (the images of tgis_gptq_prepare) in f16: decode steps of up to 32 rows, K a multiple of 128 up to 12288, where it norms 8192 (up to
+ * 16 rows) or 4096, groups of 64 2^n rows.
  * The stream between the launches is T(h) as rows [M][width], T(h * norm_w * unit) of the norm weight that is next, in 32-row fragment order (TGIS_LD_FRAGMENTS) and its
- * columns where `places` (null: in their order) has them, and sums: the sums of h^2 of sixteen columns each, h in fp32, as [width / 64][16 rows][4].  unit: a power of two
+ * columns where `places` (null: in their order) has them, and sums: the sums of h^2 of sixteen columns each, h in fp32, as [width / 64][32 rows][4].  unit: a power of two
  * by which |norm_w| is at most one; that of the norm in front of the product in norm_silu and norm_rope.  x of `residual` and the output of `norm_silu` are in fragment order.
  *   tgis_gptq_rows_embed      the stream of M tokens (zeros for an id outside the vocabulary)
  *   tgis_gptq_rows_residual   h = T(x W) + T(h); N (the width) a multiple of 64

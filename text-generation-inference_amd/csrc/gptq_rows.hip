@@ -1,4 +1,4 @@
-// Int4 products of a decode step of up to 16 rows with the norm in front of them and the residual add behind them.
+// Int4 products of a decode step of up to 32 rows with the norm in front of them and the residual add behind them.
 // Replaces exllamav2_kernels.gemm_half_q_half (utils/gptq/exllamav2.py:139-144) and the add + RMSNorm launches (custom_modeling/flash_llama_modeling.py:132-152)
 // of such a step: five launches a layer, as csrc/dense_rows.hip does for dense weights, on the image of gptq_gemm_body.h.
 //
@@ -12,17 +12,20 @@
 // us a launch of 4096, 11008 at 16 rows, the other launches and the norm behind them / these: qkv 10.1 / 9.6, o 8.7 / 5.5, gate | up 13.8 / 12.9, down 12.5 / 10.0: 2.7 TB/s of
 // weights, bound by the launch's own ends and, of what is left, by the round trip of a turn's loads (weights of a turn ahead in registers of their own cost 0.7 us: x holds 64).
 // Whole steps at ctx 137, 1, 4, 16 rows: eight layers of 4096, 11008 484 / 449, 520 / 467, 579 / 522; of 2048, 5632 337 / 279, 341 / 282, 359 / 298; of 3072, 8192 394 / 361, 402 /
-// 367, 424 / 388; of 5120, 13824 607 / 598, 623 / 608, 705 / 696; four of 8192, 28672 623 / 565, 624 / 570, 646 / 600.
+// 367, 424 / 388; of 5120, 13824 607 / 598, 623 / 608, 705 / 696; four of 8192, 28672 623 / 565, 624 / 570, 646 / 600.  At 17 - 32 rows a weight feeds two instructions
+// and x of a whole k range takes as long as the weights: products as above at 32 rows 12.0 / 11.4, 9.9 / 6.7, 16.4 / 16.1, 13.3 / 13.3.
+// Steps at 24, 32 rows: 4096, 11008 679 / 634, 708 / 686; 2048, 5632 388 / 335, 399 / 357; 3072, 8192 468 / 451, 486 / 477; 5120, 13824, where it is 320 residual units and x
+// leaves the registers of one unit, 850 / 850, 858 / 869: not served.
 #include <algorithm>
 #include "gptq_gemm_body.h"
 
 namespace {
 
-constexpr int GROWS_M = 16;
+constexpr int GROWS_M = 32;
 enum { GROWS_ROPE, GROWS_SILU };
 struct GRowsArgs {
     const f16* x;       // T(h w unit) or an activation, fragment order (xf_off)
-    const float* sums;  // [K / 64][16 rows][4]: sums of h^2 of sixteen columns
+    const float* sums;  // [K / 64][32 rows][4]: sums of h^2 of sixteen columns
     float eps, unit;
     const uint8_t* prep;
     int64_t offB;
@@ -53,13 +56,18 @@ struct GRowsDequant {
         asm volatile("" : "+v"(EX));
         asm volatile("" : "+s"(M0), "+s"(M1));
     }
-    // acc += (a lane's 32 k of a column) x (x of the same)
-    __device__ __forceinline__ void mma(const u32x4& q, uint32_t sz, const f16x8 (&x)[4], f32x4& acc) const {
+    // acc += (a lane's 32 k of a column) x (x of the same, each block of sixteen rows)
+    template <int RB>
+    __device__ __forceinline__ void mma(const u32x4& q, uint32_t sz, const f16x8 (&x)[RB][4], f32x4 (&acc)[RB]) const {
         const f16x2 s = __builtin_bit_cast(f16x2, sz);
         const f16 zc1 = s[1], zd1 = (f16)960.f - zc1;
         const f16x2 zc = {zc1, zc1}, zd = {zd1, zd1}, sc = {s[0], s[0]};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc = mfma16(gptq::dequant8(q[i], zc, zd, sc, EX, M0, M1), x[i], acc);
+        for (int i = 0; i < 4; ++i) {
+            const f16x8 w = gptq::dequant8(q[i], zc, zd, sc, EX, M0, M1);
+#pragma unroll
+            for (int b = 0; b < RB; ++b) acc[b] = mfma16(w, x[b][i], acc[b]);
+        }
     }
 };
 
@@ -93,34 +101,43 @@ __global__ __launch_bounds__(256) void gptq_rows_embed_kernel(const int64_t* __r
 // Products of a normed operand.  A unit is columns c0 .. +7 and c0 + 16 .. +23 of a tile: the halves of a rotation, or gate and up.  DS: double k64-steps of a wave at most;
 // P: units a workgroup
 // takes at a time, with one exchange of its waves' sums.
-template <int KIND, int W, int DS, int P>
+template <int KIND, int W, int RB, int DS, int P>
 __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int units, int per) {
-    __shared__ __attribute__((aligned(16))) float red[2][P][W][64 * 4];
-    __shared__ float part[W][GROWS_M];
+    __shared__ __attribute__((aligned(16))) float red[2][P][RB][W][64 * 4];
+    __shared__ float part[W][16 * RB];
+    constexpr int FW = P * RB <= 4 ? 4 : 8;  // a turn's outputs are finished by FW waves, a unit's block of rows each
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int steps = a.K >> 7, mine = (steps - w + W - 1) / W;  // of 128 k: w, w + 8, ..
-    const int m = lane & 15, kq = lane >> 4, row = min(m, a.M - 1);
+    const int m = lane & 15, kq = lane >> 4;
+    const int fp = w % FW / RB, fb = w % RB, frow = fb * 16 + m;  // the unit of a turn and the row that this lane finishes
     const int u0 = blockIdx.x * per, n = min(per, units - u0);
 
     int32_t pos = 0, slot = 0;
     if (KIND == GROWS_ROPE) {
-        pos = a.positions[row];
-        slot = a.slots[row];
+        pos = a.positions[min(frow, a.M - 1)];
+        slot = a.slots[min(frow, a.M - 1)];
     }
-    f16x8 x[DS][4];
-    const uint32_t xoff = grows_x_off(kq, row);
+    f16x8 x[DS][RB][4];
+    uint32_t xoff[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) xoff[b] = grows_x_off(kq, min(b * 16 + m, a.M - 1));
 #pragma unroll
     for (int j = 0; j < DS; ++j) {
         const char* p = reinterpret_cast<const char*>(a.x) + (int64_t)min(w + W * j, steps - 1) * 8192;
         PIN_SGPR(p);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[j][i] = *(const GLOBAL_AS f16x8*)(p + xoff + i * 1024);
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[j][b][i] = *(const GLOBAL_AS f16x8*)(p + xoff[b] + i * 1024);
     }
     constexpr int SG = (DS + 1) / 2;  // groups of 4 x 16 columns of a lane
-    f32x4 sq[SG];
+    f32x4 sq[RB][SG];
     const int groups64 = a.K >> 6;
 #pragma unroll
-    for (int t = 0; t < SG; ++t) sq[t] = *reinterpret_cast<const f32x4*>(a.sums + ((int64_t)min((t * W + w) * 4 + kq, groups64 - 1) * GROWS_M + row) * 4);
+    for (int b = 0; b < RB; ++b)
+#pragma unroll
+        for (int t = 0; t < SG; ++t)
+            sq[b][t] = *reinterpret_cast<const f32x4*>(a.sums + ((int64_t)min((t * W + w) * 4 + kq, groups64 - 1) * GROWS_M + min(b * 16 + m, a.M - 1)) * 4);
 
     const int cl = (lane & 7) + ((lane >> 3) & 1) * 16;
     u32x4 wq[P][DS];
@@ -163,16 +180,19 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
         }
         if (a.bias) bv = *reinterpret_cast<const f16x4*>(a.bias + head * a.D + dim);
     };
-    if (KIND == GROWS_ROPE) rope_inputs(u0 + min(w / 4 * P + w % 4, n - 1));  // of the first unit that this wave finishes
+    if (KIND == GROWS_ROPE) rope_inputs(u0 + min(w / FW * P + fp, n - 1));  // of the first unit that this wave finishes
 
-    float ss = 0.f;
 #pragma unroll
-    for (int t = 0; t < SG; ++t)
+    for (int b = 0; b < RB; ++b) {
+        float ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ss += (t * W + w) * 4 + kq < groups64 ? sq[t][e] : 0.f;
-    ss += __shfl_xor(ss, 16, 64);
-    ss += __shfl_xor(ss, 32, 64);
-    if (kq == 0) part[w][m] = ss;  // (read behind the first unit's barrier)
+        for (int t = 0; t < SG; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss += (t * W + w) * 4 + kq < groups64 ? sq[b][t][e] : 0.f;
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        if (kq == 0) part[w][b * 16 + m] = ss;  // (read behind the first turn's barrier)
+    }
 
     const GRowsDequant dq;
     // P units from i on; what the next P take is asked for as each is done with
@@ -181,26 +201,27 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
         const int r = (i / P) & 1;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            f32x4 acc = {0, 0, 0, 0};
+            f32x4 acc[RB] = {};
 #pragma unroll
             for (int j = 0; j < DS; ++j) dq.mma(wq[p][j], sz[p][j], x[j], acc);
             if (MORE) ask(p, min(u0 + i + P + p, units - 1));
-            *reinterpret_cast<f32x4*>(&red[r][p][w][lane * 4]) = acc;
+#pragma unroll
+            for (int b = 0; b < RB; ++b) *reinterpret_cast<f32x4*>(&red[r][p][b][w][lane * 4]) = acc[b];
         }
         __syncthreads();  // (the buffer before last was read in front of a barrier since)
-        const int p = w % 4, at = i + p;
-        if (w / 4 != (i / P) % (W / 4) || p >= P || at >= n) return;
+        const int at = i + fp;
+        if (w / FW != (i / P) % (W / FW) || fp >= P || at >= n) return;
         float tot = 0.f;
 #pragma unroll
-        for (int k = 0; k < W; ++k) tot += part[k][m];
+        for (int k = 0; k < W; ++k) tot += part[k][frow];
         const float rstd = rsqrtf(tot / a.K + a.eps) / a.unit;
-        f32x4 v = *reinterpret_cast<const f32x4*>(&red[r][p][0][lane * 4]);
+        f32x4 v = *reinterpret_cast<const f32x4*>(&red[r][fp][fb][0][lane * 4]);
 #pragma unroll
-        for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[r][p][k][lane * 4]);
+        for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[r][fp][fb][k][lane * 4]);
         v *= rstd;
-        // v[e]: row m, column c + e of its half of the tile
+        // v[e]: row frow, column c + e of its half of the tile
         const int u = u0 + at, tile = u >> 1, c = (u & 1) * 8 + (kq & 1) * 4;
-        const bool live = m < a.M;
+        const bool live = frow < a.M;
         f16x4 o;
         if (KIND == GROWS_SILU) {
 #pragma unroll
@@ -209,9 +230,9 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
                 const float sl = own / (1.f + __expf(-own));
                 o[e] = (f16)((float)(f16)sl * up);
             }
-            if (live && !second) *reinterpret_cast<f16x4*>(a.out + xf_off(m, tile * 16 + c, a.N >> 1)) = o;
+            if (live && !second) *reinterpret_cast<f16x4*>(a.out + xf_off(frow, tile * 16 + c, a.N >> 1)) = o;
         } else {
-            if (i >= P * (W / 4)) rope_inputs(u);
+            if (i >= P * (W / FW)) rope_inputs(u);
             const bool roth = head < a.H + a.Hkv;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -223,7 +244,7 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
             const int64_t page = slot >> 5;
             const int tok = slot & 31;
             if (head < a.H) {
-                *reinterpret_cast<f16x4*>(a.out + (int64_t)m * a.ldo + head * a.D + dim) = o;
+                *reinterpret_cast<f16x4*>(a.out + (int64_t)frow * a.ldo + head * a.D + dim) = o;
             } else if (roth) {
                 *reinterpret_cast<f16x4*>(a.kpool + (page * a.Hkv + (head - a.H)) * 32 * a.D + k_off(tok, dim, a.D)) = o;
             } else {
@@ -239,25 +260,30 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
 
 // h += T(x W) and what the next norm's product needs of it; a unit of sixteen columns a workgroup.  DS: double k64-steps of a wave at most.  us at 16 rows, eight waves / sixteen: 4096
 // x 4096 5.5 / 5.8, 11008 x 4096 10.0 / 10.3, 2048 x 2048 3.7 / 4.6, 8192 x 8192 15.0 / 16.3; x asked for one, three, five steps ahead 10.0 / 10.3 / 10.5 (11008 x 4096).
-template <int DS>
+template <int RB, int DS>
 __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
     constexpr int W = 8;
-    __shared__ __attribute__((aligned(16))) float red[W][64 * 4];
+    __shared__ __attribute__((aligned(16))) float red[RB][W][64 * 4];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int steps = a.K >> 7, mine = (steps - w + W - 1) / W;
-    const int m = lane & 15, kq = lane >> 4, row = min(m, a.M - 1);
+    const int m = lane & 15, kq = lane >> 4;
     const int tile = blockIdx.x >> 1, c0 = (blockIdx.x & 1) * 16;
     const char* base = reinterpret_cast<const char*>(a.prep) + (int64_t)tile * a.KS * 1024;
     const char* sbase = reinterpret_cast<const char*>(a.prep + a.offB) + (int64_t)tile * a.G * 128;
     PIN_SGPR(sbase);
-    const uint32_t woff = grows_w_off(kq, c0 + m), xoff = grows_x_off(kq, row);
+    const uint32_t woff = grows_w_off(kq, c0 + m);
+    uint32_t xoff[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) xoff[b] = grows_x_off(kq, min(b * 16 + m, a.M - 1));
     auto step_at = [&](int j) { return min(w + W * j, steps - 1); };
-    f16x8 x[2][4];
-    auto ask_x = [&](int b, int j) {
+    f16x8 x[2][RB][4];
+    auto ask_x = [&](int d, int j) {
         const char* p = reinterpret_cast<const char*>(a.x) + (int64_t)step_at(j) * 8192;
         PIN_SGPR(p);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[b][i] = *(const GLOBAL_AS f16x8*)(p + xoff + i * 1024);
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[d][b][i] = *(const GLOBAL_AS f16x8*)(p + xoff[b] + i * 1024);
     };
     ask_x(0, 0);
     u32x4 wq[DS];
@@ -272,11 +298,12 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
         wq[j] = __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(p + woff));
     }
     if (DS > 1) ask_x(1, 1);
-    const int col = tile * 32 + c0 + kq * 4;  // .. + 3: what this lane of the first wave finishes, of row m
+    const int col = tile * 32 + c0 + kq * 4;  // .. + 3: what this lane of the first RB waves finishes, of its row
+    const int frow = w * 16 + m;
     f16x4 res{}, nw{};
     int32_t at[4] = {};
-    if (w == 0) {
-        res = *reinterpret_cast<const f16x4*>(a.h + (int64_t)row * a.N + col);
+    if (w < RB) {
+        res = *reinterpret_cast<const f16x4*>(a.h + (int64_t)min(frow, a.M - 1) * a.N + col);
         nw = *reinterpret_cast<const f16x4*>(a.norm_w + col);
         if (a.places) {
 #pragma unroll
@@ -284,18 +311,19 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
         }
     }
     const GRowsDequant dq;
-    f32x4 acc = {0, 0, 0, 0};
+    f32x4 acc[RB] = {};
 #pragma unroll
     for (int j = 0; j < DS; ++j) {
         dq.mma(wq[j], sz[j], x[j & 1], acc);
         if (j + 2 < DS) ask_x(j & 1, j + 2);
     }
-    *reinterpret_cast<f32x4*>(&red[w][lane * 4]) = acc;
-    __syncthreads();
-    if (w != 0) return;
-    f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][lane * 4]);
 #pragma unroll
-    for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[k][lane * 4]);
+    for (int b = 0; b < RB; ++b) *reinterpret_cast<f32x4*>(&red[b][w][lane * 4]) = acc[b];
+    __syncthreads();
+    if (w >= RB) return;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&red[w][0][lane * 4]);
+#pragma unroll
+    for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[w][k][lane * 4]);
     f16x4 h, hw;
     float ss = 0.f;
 #pragma unroll
@@ -307,15 +335,15 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
     }
     ss += __shfl_xor(ss, 16, 64);
     ss += __shfl_xor(ss, 32, 64);
-    if (m >= a.M) return;
-    *reinterpret_cast<f16x4*>(a.h + (int64_t)m * a.N + col) = h;
+    if (frow >= a.M) return;
+    *reinterpret_cast<f16x4*>(a.h + (int64_t)frow * a.N + col) = h;
     if (a.places) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a.hw[xf_off(m, at[e], a.N)] = hw[e];
+        for (int e = 0; e < 4; ++e) a.hw[xf_off(frow, at[e], a.N)] = hw[e];
     } else {
-        *reinterpret_cast<f16x4*>(a.hw + xf_off(m, col, a.N)) = hw;
+        *reinterpret_cast<f16x4*>(a.hw + xf_off(frow, col, a.N)) = hw;
     }
-    if (kq == 0) a.sums_out[sums16_off(m, col)] = ss;
+    if (kq == 0) a.sums_out[sums16_off(frow, col)] = ss;
 }
 
 // The same behind a product whose k range was split: S slabs [32][ld] of a tgis_gptq_gemm_partial, sixteen columns a thread
@@ -347,10 +375,11 @@ __global__ __launch_bounds__(64) void gptq_rows_sum_kernel(const float* __restri
     a.sums_out[sums16_off(m, k)] = ss;
 }
 
-// groups of 64 2^n rows, as gptq_wide_body.h; K of whole double steps, as many as a wave's registers hold of x, or of one unit's weights
+// groups of 64 2^n rows, as gptq_wide_body.h; K of whole double steps, as many as a wave's registers hold of x (or, where steps of 5120 columns and more
+// than 16 rows are no sooner done, 4096), or of one unit's weights
 bool grows_fits(int64_t M, int64_t K, int64_t N, int64_t groups, bool norm) {
     if (M < 1 || M > GROWS_M || K < 128 || K % 128 || N < 32 || N % 32 || N >= (1ll << 31) || groups < 1 || K % groups) return false;
-    if (K > (norm ? 8192 : 12288)) return false;
+    if (K > (!norm ? 12288 : M <= 16 ? 8192 : 4096)) return false;
     const int64_t spg = K / groups / 64;
     return groups == 1 || (K / groups % 64 == 0 && (spg & (spg - 1)) == 0);
 }
@@ -359,7 +388,7 @@ int grows_args(const char* what, GRowsArgs& a, const void* x, const float* sums,
                int64_t groups, bool norm) {
     TGIS_CHECK_ARG(x && prepared && sums && unit > 0.f, "%s: null tensor or bad factor", what);
     TGIS_CHECK_ARG(grows_fits(M, K, N, groups, norm), "%s: up to %d rows, K a multiple of 128 up to %d, groups of 64 2^n (M=%ld K=%ld N=%ld groups=%ld)", what, GROWS_M,
-                   norm ? 8192 : 12288, (long)M, (long)K, (long)N, (long)groups);
+                   !norm ? 12288 : M <= 16 ? 8192 : 4096, (long)M, (long)K, (long)N, (long)groups);
     TGIS_CHECK_ARG(((uintptr_t)x | (uintptr_t)prepared | (uintptr_t)sums) % 16 == 0, "%s: operands must be 16-byte aligned", what);
     const gptq::PrepLayout p = gptq::prep_layout(K, N, groups);
     a = GRowsArgs{};
@@ -380,16 +409,16 @@ int grows_args(const char* what, GRowsArgs& a, const void* x, const float* sums,
     return TGIS_OK;
 }
 
-template <int KIND, int W, int DS, int P>
+template <int KIND, int W, int RB, int DS, int P>
 void launch_grows_k(const GRowsArgs& a, int per, hipStream_t st) {
     const int units = a.N / 16;
-    hipLaunchKernelGGL((gptq_rows_kernel<KIND, W, DS, P>), dim3((unsigned)((units + per - 1) / per)), dim3(64 * W), 0, st, a, units, per);
+    hipLaunchKernelGGL((gptq_rows_kernel<KIND, W, RB, DS, P>), dim3((unsigned)((units + per - 1) / per)), dim3(64 * W), 0, st, a, units, per);
 }
-template <int KIND, int DS>
+template <int KIND, int RB, int DS>
 void launch_grows_p(const GRowsArgs& a, int per, hipStream_t st) {
-    if (per % 2 == 0) return launch_grows_k<KIND, 8, DS, 2>(a, per, st);
-    if (per % 3 == 0) return launch_grows_k<KIND, 8, DS, 3>(a, per, st);
-    launch_grows_k<KIND, 8, DS, 1>(a, per, st);
+    if (per % 2 == 0) return launch_grows_k<KIND, 8, RB, DS, 2>(a, per, st);
+    if (per % 3 == 0) return launch_grows_k<KIND, 8, RB, DS, 3>(a, per, st);
+    launch_grows_k<KIND, 8, RB, DS, 1>(a, per, st);
 }
 // One workgroup a CU.  us at 16 rows, turns of one, two, three units: gate | up of 4096 x 22016 (6 units a workgroup) 14.3 / 12.9 / 13.3, of 2048 x 11264 (3) 6.6 / 6.5 / 5.8; qkv of
 // 4096 x 12288 (3) 10.0 / 11.7 / 9.6; from K 5120 on x leaves the registers of one: 5120 x 27648 (7) 19.7 / 21.2 / 22.5.  Sixteen waves take less of x each: 8192 x 57344
@@ -398,18 +427,33 @@ template <int KIND>
 int launch_grows(const GRowsArgs& a, hipStream_t st) {
     TgisTimedScope timed(TGIS_OP_GPTQ_GEMM, st);
     const int units = a.N / 16, per = (units + 255) / 256, ds = (a.K + 1023) / 1024;
-    if (ds <= 2)
-        launch_grows_p<KIND, 2>(a, per, st);
+    if (a.M > 16) {
+        if (ds <= 2)
+            launch_grows_p<KIND, 2, 2>(a, per, st);
+        else
+            launch_grows_p<KIND, 2, 4>(a, per, st);
+    } else if (ds <= 2)
+        launch_grows_p<KIND, 1, 2>(a, per, st);
     else if (ds <= 4)
-        launch_grows_p<KIND, 4>(a, per, st);
+        launch_grows_p<KIND, 1, 4>(a, per, st);
     else if (ds == 5)
-        launch_grows_k<KIND, 8, 5, 1>(a, per, st);
+        launch_grows_k<KIND, 8, 1, 5, 1>(a, per, st);
     else if (KIND == GROWS_SILU)
-        launch_grows_k<GROWS_SILU, 16, 4, 1>(a, per, st);
+        launch_grows_k<GROWS_SILU, 16, 1, 4, 1>(a, per, st);
     else
-        launch_grows_k<KIND, 8, 8, 1>(a, per, st);
+        launch_grows_k<KIND, 8, 1, 8, 1>(a, per, st);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
+}
+template <int RB>
+void launch_grows_residual(const GRowsArgs& a, hipStream_t st) {
+    const int ds = (a.K + 1023) / 1024;
+    const auto kernel = ds <= 2   ? gptq_rows_residual_kernel<RB, 2>
+                        : ds <= 4 ? gptq_rows_residual_kernel<RB, 4>
+                        : ds <= 6 ? gptq_rows_residual_kernel<RB, 6>
+                        : ds <= 8 ? gptq_rows_residual_kernel<RB, 8>
+                                  : gptq_rows_residual_kernel<RB, 12>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(a.N / 16)), dim3(512), 0, st, a);
 }
 
 }  // namespace
@@ -449,13 +493,10 @@ extern "C" int tgis_gptq_rows_residual(const void* x, const void* prepared, cons
     a.hw = (f16*)hw;
     a.sums_out = sums;
     TgisTimedScope timed(TGIS_OP_GPTQ_GEMM, (hipStream_t)stream);
-    const int ds = (int)cdiv64(K, 1024);
-    const auto kernel = ds <= 2   ? gptq_rows_residual_kernel<2>
-                        : ds <= 4 ? gptq_rows_residual_kernel<4>
-                        : ds <= 6 ? gptq_rows_residual_kernel<6>
-                        : ds <= 8 ? gptq_rows_residual_kernel<8>
-                                  : gptq_rows_residual_kernel<12>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(N / 16)), dim3(512), 0, (hipStream_t)stream, a);
+    if (M <= 16)
+        launch_grows_residual<1>(a, (hipStream_t)stream);
+    else
+        launch_grows_residual<2>(a, (hipStream_t)stream);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }

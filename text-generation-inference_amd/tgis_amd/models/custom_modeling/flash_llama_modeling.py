@@ -412,22 +412,27 @@ class FlashLlamaModel:
         return down
 
     def forward_int4_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
-        """A decode step of up to 16 rows of an int4 model on the launches of csrc/gptq_rows.hip: the normed hidden states.  Five launches a layer; the values are those of
-        `forward` but for the order of the sums and where the norm's 1 / rms is multiplied in."""
+        """A decode step of up to 32 rows of an int4 model on the launches of csrc/gptq_rows.hip: the normed hidden states.  Five launches a layer, or one more for sums that are split; the values are
+        those of `forward` but for the order of the sums and where the norm's 1 / rms is multiplied in."""
         qkv_norms, mlp_norms = self.int4_norms
         table = self.embed_tokens.weight
         h = native.Int4RowsStream.embed(input_ids, table, qkv_norms[0])
         cos, sin = self.rope_tables(table.dtype, h.device, max_s)
+
+        def add(x, lin, h, norm):
+            if native.gptq_rows_ok(h.M, lin.ordered, False):
+                native.gptq_rows_residual(x, lin.ordered, h, norm)
+            else:
+                native.gptq_rows_sum(native.gptq_gemm_partial(x, lin.ordered), h, norm)
+
         for i, layer in enumerate(self.layers):
             att, mlp = layer.self_attn, layer.mlp
-            if i > 0 and native.gptq_rows_ok(h.M, down.ordered, False):
-                native.gptq_rows_residual(act, down.ordered, h, qkv_norms[i])
-            elif i > 0:  # (a long k range is split over workgroups)
-                native.gptq_rows_sum(native.gptq_gemm_partial(act, down.ordered), h, qkv_norms[i])
+            if i > 0:
+                add(act, down, h, qkv_norms[i])
             qkv = native.gptq_rows_rope(h, layer.input_layernorm.variance_epsilon, att.query_key_value.linear.rope_handle, att.query_key_value.linear.bias, cos, sin,
                                         position_ids, kv.slots, kv.cache.k_pool(layer.layer_id), kv.cache.v_pool(layer.layer_id), att.num_heads,
                                         att.num_key_value_heads, att.head_size)
-            native.gptq_rows_residual(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv), att.o_proj.linear.ordered, h, mlp_norms[i])
+            add(att.attend(qkv, cu_seqlens_q, layer.layer_id, kv), att.o_proj.linear, h, mlp_norms[i])
             act = native.gptq_rows_silu(h, layer.post_attention_layernorm.variance_epsilon, mlp.gate_up_proj.linear.ordered)
             down = mlp.down_proj.linear
         return self.norm(self.layers[-1].mlp.down_proj(act, partial=True), h.h)[0]
@@ -438,14 +443,18 @@ class FlashLlamaModel:
         self.int4_norms, self._int4_rows = None, {}
         if self.tp_world_size != 1 or self.embed_tokens.weight.dtype != torch.float16:
             return
+        norms = ([], [])
         for layer in self.layers:
             att, mlp = layer.self_attn, layer.mlp
             qkv, o, gate_up, down = lins = (att.query_key_value.linear, att.o_proj.linear, mlp.gate_up_proj.linear, mlp.down_proj.linear)
             if (not all(isinstance(lin, Ex4bitLinearV2) for lin in lins) or qkv.rope_handle is None or not gate_up.gate_up or down.perm is not None
-                    or any(lin.bias is not None for lin in lins[1:]) or any(lin.perm is not None and lin.places() is None for lin in lins[:3])):
+                    or any(lin.bias is not None for lin in lins[1:]) or (o.perm is not None and att.out_places is None)):
                 return
-        self.int4_norms = ([native.Int4NormInput(layer.input_layernorm.weight, layer.self_attn.query_key_value.linear.places()) for layer in self.layers],
-                           [native.Int4NormInput(layer.post_attention_layernorm.weight, layer.mlp.gate_up_proj.linear.places()) for layer in self.layers])
+            for lin, norm, inputs in ((qkv, layer.input_layernorm, norms[0]), (gate_up, layer.post_attention_layernorm, norms[1])):
+                inputs.append((norm.weight, lin.places()))
+                if lin.perm is not None and inputs[-1][1] is None:
+                    return
+        self.int4_norms = tuple(native.Int4NormInput.several(inputs) for inputs in norms)
 
     def serves_int4_rows(self, rows: int) -> bool:
         got = self._int4_rows.get(rows)
@@ -455,7 +464,6 @@ class FlashLlamaModel:
                 att, mlp = layer.self_attn, layer.mlp
                 o = att.o_proj.linear
                 got = (got and native.gptq_rows_ok(rows, att.query_key_value.linear.rope_handle, True) and native.gptq_rows_ok(rows, mlp.gate_up_proj.linear.ordered, True)
-                       and native.gptq_rows_ok(rows, o.ordered, False)
                        and o.wants_fragments(rows, gathers=att.out_places is not None) and mlp.down_proj.linear.wants_fragments(rows)
                        and mlp.intermediate_size % 64 == 0)
             self._int4_rows[rows] = got

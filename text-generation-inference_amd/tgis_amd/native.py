@@ -977,7 +977,7 @@ def dense_rows16_head(h: RowsStream, eps: float, w: DenseWeight) -> torch.Tensor
     return out
 
 
-GPTQ_ROWS_MAX_M = 16
+GPTQ_ROWS_MAX_M = 32
 
 
 def gptq_rows_ok(M: int, w: GptqWeight, norm: bool) -> bool:
@@ -988,10 +988,16 @@ def gptq_rows_ok(M: int, w: GptqWeight, norm: bool) -> bool:
 class Int4NormInput:
     """What a norm in front of an int4 product makes of the stream: its weight, the power of two by which that is at most one, and where the product wants its columns."""
 
-    def __init__(self, weight: torch.Tensor, places: Optional[torch.Tensor] = None):
-        top = float(weight.abs().max()) if weight.numel() else 0.0
+    def __init__(self, weight: torch.Tensor, places: Optional[torch.Tensor] = None, top: Optional[float] = None):
+        top = float(weight.abs().max()) if top is None else top
         self.weight, self.places = weight, places
         self.unit = 2.0 ** -math.frexp(top)[1] if 0.0 < top < math.inf else 1.0
+
+    @staticmethod
+    def several(inputs) -> list:
+        """Of (weight, places) each, with one wait for the device."""
+        tops = torch.stack([w.abs().max() for w, _ in inputs]).tolist()
+        return [Int4NormInput(w, places, top) for (w, places), top in zip(inputs, tops)]
 
 
 class Int4RowsStream:
