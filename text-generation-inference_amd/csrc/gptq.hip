@@ -107,10 +107,10 @@ __global__ __launch_bounds__(64 * TN * WK) void gptq_gemm_kernel(GemmArgs a) {
 
 // Decode batches of up to 64 rows whose activation is in fragment order (gptq_wide_body.h).  8 waves; CT = 4 holds 2 waves
 // per SIMD (one block per CU), CT = 2 / 3 leave room for more.
-template <int CT, int ACT, bool OUTF, int RB>
+template <int CT, int ACT, bool OUTF, int RB, int CG>
 __global__ __launch_bounds__(64 * gptq::WIDE_WK) void gptq_wide_kernel(GemmArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    gptq::gptq_wide_unit<CT, ACT, OUTF, RB>(a, smem);
+    gptq::gptq_wide_unit<CT, ACT, OUTF, RB, CG>(a, smem);
 }
 
 // Sum the S split-K slabs in fixed order (deterministic) and emit f16 (+bias): thread = (row, 4 columns).
@@ -374,16 +374,16 @@ struct RopeEpi {
     int H, Hkv, D;
 };
 
-template <int CT, int ACT, bool OUTF, int RB>
+template <int CT, int ACT, bool OUTF, int RB, int CG = 1>
 static int launch_wide_rows(dim3 grid, hipStream_t st, const GemmArgs& a) {
     const size_t lds = gptq::wide_lds_bytes(CT, RB);
     static bool attr_done = false;
     if (!attr_done) {
-        TGIS_CHECK_HIP(hipFuncSetAttribute((const void*)gptq_wide_kernel<CT, ACT, OUTF, RB>,
+        TGIS_CHECK_HIP(hipFuncSetAttribute((const void*)gptq_wide_kernel<CT, ACT, OUTF, RB, CG>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         attr_done = true;
     }
-    hipLaunchKernelGGL((gptq_wide_kernel<CT, ACT, OUTF, RB>), grid, dim3(64 * gptq::WIDE_WK), lds, st, a);
+    hipLaunchKernelGGL((gptq_wide_kernel<CT, ACT, OUTF, RB, CG>), grid, dim3(64 * gptq::WIDE_WK), lds, st, a);
     return TGIS_OK;
 }
 template <int CT, int ACT, bool OUTF>
@@ -393,6 +393,16 @@ static int launch_wide_one(dim3 grid, hipStream_t st, const GemmArgs& a) {
         case 2: return launch_wide_rows<CT, ACT, OUTF, 2>(grid, st, a);
         case 3: return launch_wide_rows<CT, ACT, OUTF, 3>(grid, st, a);
         default: return launch_wide_rows<CT, ACT, OUTF, 4>(grid, st, a);
+    }
+}
+
+template <bool OUTF>
+static int launch_wide_pair(dim3 grid, hipStream_t st, const GemmArgs& a) {
+    switch (gptq::wide_row_blocks(a.M, a.K, 4, a.S)) {
+        case 1: return launch_wide_rows<4, 2, OUTF, 1, 2>(grid, st, a);
+        case 2: return launch_wide_rows<4, 2, OUTF, 2, 2>(grid, st, a);
+        case 3: return launch_wide_rows<4, 2, OUTF, 3, 2>(grid, st, a);
+        default: return launch_wide_rows<4, 2, OUTF, 4, 2>(grid, st, a);
     }
 }
 
@@ -455,7 +465,10 @@ static int launch_gptq(const void* x, int64_t ldx, const void* prepared, const v
                              : launch_wide_one<CT, 0, false>(wgrid, st, a);                             \
         if (rc_ != TGIS_OK) return rc_;                                                                 \
     } while (0)
-        if (pl.TN == 4) TGIS_WIDE(4); else if (pl.TN == 3) TGIS_WIDE(3); else if (pl.TN == 1) TGIS_WIDE(1); else TGIS_WIDE(2);
+        if (pl.TN == 8) {  // act 2 alone
+            int rc_ = outf ? launch_wide_pair<true>(wgrid, st, a) : launch_wide_pair<false>(wgrid, st, a);
+            if (rc_ != TGIS_OK) return rc_;
+        } else if (pl.TN == 4) TGIS_WIDE(4); else if (pl.TN == 3) TGIS_WIDE(3); else if (pl.TN == 1) TGIS_WIDE(1); else TGIS_WIDE(2);
 #undef TGIS_WIDE
         TGIS_CHECK_LAUNCH();
         if (!partial && pl.S > 1) {

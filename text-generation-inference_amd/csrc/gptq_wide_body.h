@@ -33,7 +33,7 @@ constexpr int WIDE_TG(int ct) { return ct < 4 ? ct : 4; }   // tiles per round o
 static inline size_t wide_lds_bytes(int ct, int rb) { return (size_t)WIDE_WK * WIDE_TG(ct) * (rb == 1 ? 2048 : 4096); }
 
 struct WidePlan {
-    int CT, S;  // column tiles per wave (= per block), global k splits
+    int CT, S;  // column tiles per block (and wave; 8: two waves' four), global k splits
 };
 
 // Does the fragment-order kernel serve this GEMM at all?  (<= 64 rows, whole k64-steps, one {scale, zero} per k64-step and
@@ -57,12 +57,17 @@ static inline bool wide_serves(int64_t M, int64_t K, int64_t N, int64_t groups, 
 static inline WidePlan plan_wide(int64_t K, int64_t N, int act, int64_t M = 32, bool finished = false) {
     if (const char* ov = getenv("TGIS_GPTQ_WIDE_PLAN")) {  // tuning hook: "CT,S"
         int ct = 0, sp = 0;
-        if (sscanf(ov, "%d,%d", &ct, &sp) == 2 && ct >= 1 && ct <= 4 && sp >= 1 && (sp == 1 || (act != 2 && act != 3)))
+        if (sscanf(ov, "%d,%d", &ct, &sp) == 2 && ct >= 1 && (ct <= 4 || (ct == 8 && act == 2)) && sp >= 1 && (sp == 1 || (act != 2 && act != 3)))
             return {ct, sp};
     }
     const int64_t tiles = cdiv64(N, 32), steps = K / 64;
     int CT = 2;
     while (CT < 4 && cdiv64(tiles, CT) > 256) ++CT;
+    // SiLU * up past one round of four-tile blocks (one a CU): pairs of waves on four tiles of one k-part each, eight a block, take in x, in good part, once.  A round of them
+    // takes 1.75 times one of four tiles.  us, four / eight tiles at 32, 40, 64 rows: 8192 x 57344 (448 / 224 blocks) 67.9 / 64.2, 81.4 / 76.5, 89.6 / 86.5; 8192 x 36864 (288 / 144)
+    // 55.2 / 51.9, 68.7 / 62.0, 74.2 / 69.0; 5120 x 40960 (320 / 160) 38.4 / 33.4, 48.0 / 41.9, 51.7 / 46.3; at 16 rows there 31.0 / 32.0.
+    const int64_t rounds4 = cdiv64(cdiv64(tiles, 4), 256), rounds8 = cdiv64(cdiv64(tiles, 8), 256);
+    if (act == 2 && M > 16 && 7 * rounds8 < 4 * rounds4) return {8, 1};
     const bool unsplit = act == 2 || act == 3;
     // (SiLU * up of a 64-row shard with a long k range — 70B gate_up at TP = 8, 224 one-tile blocks that each take in a 1 MiB
     // activation, 20.3 us for 29 MB — was also run split over k with the activation in the reduce launch, CT x S = 1x2, 2x2,
@@ -112,16 +117,18 @@ __device__ __forceinline__ void swap_rows(uint32_t x, uint32_t y, uint32_t (&out
 }
 
 // OUTF: the act = 2 output (the operand of the down projection) leaves in fragment order as well.
+// CG: groups of CT tiles, a wave of each k-part for each.
 // RB = 16-row blocks of the activation; every dequantised B fragment feeds them all.  Two and four are one and two operands of the 32x32x16 instruction.
 // One and three take 16x16x32: half of x and of the matrix work up to 16 rows, three quarters at 33 - 48, for a row swap of the weights per two words.
 // us, 32x32x16 / 16x16x32 (qkv + rotary, o, gate | up, down): 4096, 11008 at 16 rows 12.4 / 10.9, 5.4 / 4.9, 15.5 / 13.2, 8.8 / 8.1; at 48 17.7 / 16.5, 7.1 / 7.4, 19.6 / 18.6,
 // 12.3 / 11.5; 8192, 28672 at 16 17.9 / 14.8, 11.2 / 10.7, 59.6 / 52.7, 33.6 / 25.9; at 48 26.4 / 23.5, 15.3 / 14.3, 77.9 / 74.6, 38.2 / 35.8.  At an even count there is
 // nothing to leave out and the swaps cost 3 - 14 % (gate | up at 32 rows 15.9 / 17.2, 64 20.6 / 23.1).  More k64-steps in flight, with the registers that sixteen rows
 // leave, are slower (three, four: gate | up 13.7 / 14.4 / 14.6, 61.0 for 55.6).
-template <int CT, int ACT, bool OUTF, int RB>
+template <int CT, int ACT, bool OUTF, int RB, int CG = 1>
 __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char* smem) {
     constexpr bool R16 = RB & 1;
-    constexpr int WK = WIDE_WK, DEPTH = WIDE_DEPTH, MR = (RB + 1) / 2, NR = RB == 1 ? 1 : 2;
+    static_assert(CG == 1 || ACT != 3, "the finishing rows' rotations are for one group of tiles");
+    constexpr int WK = WIDE_WK, KP = WK / CG, DEPTH = WIDE_DEPTH, MR = (RB + 1) / 2, NR = RB == 1 ? 1 : 2;
     constexpr int XB = R16 ? RB : MR, XN = R16 ? 2 : 4;  // row blocks of the instruction, fragments of a k64-step in each
     {   // every cache line of the argument block is requested at entry: one scalar round trip instead of three dependent
         // ones before the first weight request (tools/floor/wide.hip `pre`: 0.1 - 0.25 us per launch)
@@ -131,7 +138,8 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
     }
     const int lane = threadIdx.x & 63;
     const int wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int cg = blockIdx.x, split = blockIdx.y;
+    const int kp = wk / CG, gi = wk % CG;  // this wave's k-part and group of tiles
+    const int cg = blockIdx.x * CG, split = blockIdx.y;
     const int steps = a.K >> 6;
     const int sp_len = (steps + a.S - 1) / a.S;
     const int sb = split * sp_len, se = min(steps, sb + sp_len);
@@ -140,14 +148,14 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
     // ahead of the younger four, which queue behind them in the address path — and a prologue barrier, a raised priority for
     // the younger half and deeper weight rings: the block finishes when its CU has moved its bytes, however they are dealt;
     // tools/floor/wide.hip `kb` / `pb` / `prio` / `DW`, profiles/r05_wide_kbias*.log, r05_wide_plans.log.)
-    const int s0 = sb + (len * wk) / WK, s1 = sb + (len * (wk + 1)) / WK;
+    const int s0 = sb + (len * kp) / KP, s1 = sb + (len * (kp + 1)) / KP;
     const int mrows = a.M;  // 1 .. 16 RB
 
     const char* wt[CT];
     const char* st[CT];
 #pragma unroll
     for (int t = 0; t < CT; ++t) {
-        const int nt = min(cg * CT + t, a.NT - 1);  // a tile past the matrix re-reads the last one and is never stored
+        const int nt = min((cg + gi) * CT + t, a.NT - 1);  // a tile past the matrix re-reads the last one and is never stored
         wt[t] = reinterpret_cast<const char*>(a.prep) + (int64_t)nt * a.KS * 1024;
         st[t] = reinterpret_cast<const char*>(a.prep + a.offB) + (int64_t)nt * a.G * 128;
     }
@@ -305,7 +313,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
         // loads, ~2.3 k clocks at CT 3; 8-byte accesses take 85 and 256 B/clk.  Same values, same order of the sum.)
         // Blocks of sixteen rows: [k-part][tile][block][column half][lane][4 rows], a lane's four sums in one store; a wave finishes a value per lane and block.
         static_assert(WK == 8, "the layouts are for eight k-parts");
-        float fin[CT][NR];
+        float fin[CG][CT][NR];
         if constexpr (R16) {
 #pragma unroll
             for (int t = tg0; t < tg0 + TG && t < CT; ++t)
@@ -317,14 +325,16 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
             __syncthreads();
             const float* src = red + ((lane >> 4) & 1) * 256 + ((wk >> 1) * 16 + (lane & 15)) * 4 + (wk & 1) * 2 + (lane >> 5);
 #pragma unroll
-            for (int t = tg0; t < tg0 + TG && t < CT; ++t)
+            for (int g = 0; g < CG; ++g)
 #pragma unroll
-                for (int j = 0; j < NR && mr * 2 + j < RB; ++j)
+                for (int t = tg0; t < tg0 + TG && t < CT; ++t)
 #pragma unroll
-                    for (int k2 = 0; k2 < WK; ++k2) {
-                        const float v = src[((k2 * TG + (t - tg0)) * NR + j) * 512];
-                        fin[t][j] = k2 == 0 ? v : fin[t][j] + v;
-                    }
+                    for (int j = 0; j < NR && mr * 2 + j < RB; ++j)
+#pragma unroll
+                        for (int k2 = 0; k2 < KP; ++k2) {
+                            const float v = src[(((k2 * CG + g) * TG + (t - tg0)) * NR + j) * 512];
+                            fin[g][t][j] = k2 == 0 ? v : fin[g][t][j] + v;
+                        }
         } else {
 #pragma unroll
             for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
@@ -334,18 +344,22 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
             }
             __syncthreads();
 #pragma unroll
-            for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
+            for (int g = 0; g < CG; ++g)
 #pragma unroll
-                for (int k2 = 0; k2 < WK; ++k2) {
-                    const f32x2 v = (reinterpret_cast<const f32x2*>(red + ((k2 * TG + (t - tg0)) << 10)) + (wk << 6))[lane];
+                for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
 #pragma unroll
-                    for (int j = 0; j < NR; ++j) fin[t][j] = k2 == 0 ? v[j] : fin[t][j] + v[j];
+                    for (int k2 = 0; k2 < KP; ++k2) {
+                        const f32x2 v = (reinterpret_cast<const f32x2*>(red + (((k2 * CG + g) * TG + (t - tg0)) << 10)) + (wk << 6))[lane];
+#pragma unroll
+                        for (int j = 0; j < NR; ++j) fin[g][t][j] = k2 == 0 ? v[j] : fin[g][t][j] + v[j];
+                    }
                 }
-            }
         }
 #pragma unroll
+        for (int g = 0; g < CG; ++g)
+#pragma unroll
         for (int t = tg0; t < tg0 + TG && t < CT; ++t) {
-            const int nt = cg * CT + t;
+            const int nt = (cg + g) * CT + t;
             if (nt >= a.NT) break;
             if (ACT == 3) {
                 // rope image: see gptq_gemm_body.h (the same epilogue on the same image)
@@ -358,7 +372,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
 #pragma unroll
                 for (int j = 0; j < NR && mr * 2 + j < RB; ++j) {
                     const int m = row_of(mr, j);
-                    const float mine = (float)(f16)(fin[t][j] + bv);
+                    const float mine = (float)(f16)(fin[g][t][j] + bv);
                     float o = mine;
                     if (roth) {
                         const float other = __shfl_xor(mine, 16, 64);
@@ -389,7 +403,7 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
                 const float bv = (a.bias && j2 < half) ? (float)a.bias[nsrc] : 0.f;
 #pragma unroll
                 for (int j = 0; j < NR && mr * 2 + j < RB; ++j) {
-                    const float mine = (float)(f16)(fin[t][j] + bv);
+                    const float mine = (float)(f16)(fin[g][t][j] + bv);
                     const float other = __shfl_xor(mine, 16, 64);
                     const int m = row_of(mr, j);
                     if (c < 16 && j2 < half && m < mrows) {
@@ -409,14 +423,14 @@ __device__ __forceinline__ void gptq_wide_unit(const GemmArgs& a, unsigned char*
 #pragma unroll
                     for (int j = 0; j < NR && mr * 2 + j < RB; ++j) {
                         const int m = row_of(mr, j);
-                        if (m < mrows) a.out[(int64_t)m * a.ldo + n] = (f16)(fin[t][j] + bv);
+                        if (m < mrows) a.out[(int64_t)m * a.ldo + n] = (f16)(fin[g][t][j] + bv);
                     }
                 }
             } else {
                 // slabs in 32-row units: [row block][split][32][ld]
                 float* sl = a.slabs + ((int64_t)(mr * a.S + split) * 32) * (a.NT * 32) + n;
 #pragma unroll
-                for (int j = 0; j < NR && mr * 2 + j < RB; ++j) sl[(int64_t)(row_of(mr, j) & 31) * (a.NT * 32)] = fin[t][j];
+                for (int j = 0; j < NR && mr * 2 + j < RB; ++j) sl[(int64_t)(row_of(mr, j) & 31) * (a.NT * 32)] = fin[g][t][j];
             }
         }
       }
