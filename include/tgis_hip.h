@@ -536,6 +536,11 @@ int tgis_attn_varlen(const void* q, int64_t ldq, const void* k_pool, const void*
 int tgis_token_shift_mix(const float* h, const float* shift_state, const int32_t* state_slots, const int32_t* cu_seqlens_q,
                          const int32_t* positions, int64_t B, const float* mu, int num_mixes, void* out, int64_t T,
                          int64_t W, int dtype, void* stream);
+/* tgis_sandwich_norm_f32 (num_slabs 0) or tgis_sandwich_norm_f32_partial with an fp32 y of the width of shift_state, and the mixes of y as tgis_token_shift_mix leaves them,
+ * of steps whose every row is its sequence's one token: E a multiple of 4 up to 8192, five mixes of two bytes, delta of their dtype or fp32. */
+int tgis_sandwich_norm_shift(const float* x, const void* delta, int64_t ld_delta, int delta_dtype, int num_slabs, const float* post_w, float post_add, float* x_out,
+                             const float* pre_w, float pre_add, float* y, const float* shift_state, const int32_t* state_slots, const int32_t* positions, const float* mu,
+                             int num_mixes, void* mixes, int mix_dtype, int64_t rows, int64_t E, float eps, void* stream);
 /* logw[t][c] = -exp(w0[c] + sum_r tanh(a[t][r]) * w2t[r][c]) : the logarithm of a per-channel decay in (0, 1). */
 int tgis_wkv_decay(const void* a, int64_t ld_a, const float* w2t, const float* w0, float* logw, int64_t T, int rank,
                    int64_t C, int dtype, void* stream);

@@ -155,14 +155,32 @@ __global__ void glu_vec_kernel(const T* __restrict__ in, int64_t ld_in, T* __res
 // number of memory instructions in it is what counts.
 // delta may also arrive as the S fp32 split-K slabs of the GEMM that produced it ([row / 32][S][32][slab_ld], TD = float,
 // `delta` then points at the slabs): their sum is taken here instead of by a reduce launch of its own.
-template <typename TD, typename TY, int NV, bool SLABS>
-__global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, const TD* __restrict__ delta, int64_t ld_delta,
-                                                                const float* __restrict__ post_w, float post_add, float post_scale, float* x_out,
-                                                                const float* __restrict__ pre_w, float pre_add,
-                                                                TY* __restrict__ y, int64_t E, float eps, int S) {
+// SHIFT: each row is its sequence's one token, and the mixes of y with the token before it leave too (tgis_token_shift_mix).  That launch was 4.2 us of a step of 24 rows of 2048
+// for 24 x 48 KiB, behind this one's 4.4; a decode step of eight layers, four of them recurrent, 476 -> 468 us.
+constexpr int SHIFT_MIXES = 5;  // what a wkv mixer has
+template <typename TM> struct ShiftArgs {
+    const float* state;  // [slots][E], the token before
+    const int32_t *slots, *positions;
+    const float* mu;     // [5][E]
+    TM* mixes;           // [5][rows][E]
+};
+template <typename TD, typename TY, int NV, bool SLABS, bool SHIFT = false, typename TM = f16>
+__device__ __forceinline__ void sandwich_norm_row(const float* x, const TD* __restrict__ delta, int64_t ld_delta, const float* __restrict__ post_w, float post_add,
+                                                  float post_scale, float* x_out, const float* __restrict__ pre_w, float pre_add, TY* __restrict__ y, int64_t E, float eps,
+                                                  int S, const ShiftArgs<TM>& sh = {}) {
     __shared__ float red[16];
     const int64_t row = blockIdx.x;
     f32x4 xv[NV], dv[NV], pw[NV], qw[NV];
+    f32x4 mu[SHIFT ? NV : 1][SHIFT_MIXES], before[SHIFT ? NV : 1];
+    if constexpr (SHIFT) {
+        const int64_t slot = sh.slots[row];
+        const bool fresh = sh.positions[row] == 0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
+            before[i] = c < E && !fresh ? Vec4<float>::ld(sh.state + slot * E + c) : f32x4{};
+        }
+    }
     // everything is asked for at once: behind the slabs' sum, the residual and the gains were a second trip to memory
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -221,6 +239,14 @@ __global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, 
         else if (S - s0 == 1)
             add_slabs(s0, std::integral_constant<int, 1>{});
     }
+    if constexpr (SHIFT) {  // (on their way during the sums)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
+#pragma unroll
+            for (int k = 0; k < SHIFT_MIXES; ++k) mu[i][k] = c < E ? Vec4<float>::ld(sh.mu + (int64_t)k * E + c) : f32x4{};
+        }
+    }
     if (delta) {
         float rinv_d = post_scale;
         if (post_w) {
@@ -252,8 +278,30 @@ __global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, 
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int64_t c = ((int64_t)threadIdx.x + 512 * i) * 4;
-        if (c < E) Vec4<TY>::st(y + row * E + c, xv[i] * rinv * qw[i]);
+        f32x4 h = xv[i] * rinv * qw[i];
+        if (c < E) Vec4<TY>::st(y + row * E + c, h);
+        if constexpr (SHIFT) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(h[e]));  // (the rounded y, as a launch of its own reads it: no product inside the difference)
+            const f32x4 d = before[i] - h;
+#pragma unroll
+            for (int k = 0; k < SHIFT_MIXES; ++k)
+                if (c < E) Vec4<TM>::st(sh.mixes + ((int64_t)k * gridDim.x + row) * E + c, h + d * mu[i][k]);
+        }
     }
+}
+template <typename TD, typename TY, int NV, bool SLABS>
+__global__ __launch_bounds__(512) void sandwich_norm_vec_kernel(const float* x, const TD* __restrict__ delta, int64_t ld_delta,
+                                                                const float* __restrict__ post_w, float post_add, float post_scale, float* x_out,
+                                                                const float* __restrict__ pre_w, float pre_add,
+                                                                TY* __restrict__ y, int64_t E, float eps, int S) {
+    sandwich_norm_row<TD, TY, NV, SLABS>(x, delta, ld_delta, post_w, post_add, post_scale, x_out, pre_w, pre_add, y, E, eps, S);
+}
+template <typename TD, int NV, bool SLABS, typename TM>
+__global__ __launch_bounds__(512) void sandwich_norm_shift_kernel(const float* x, const TD* __restrict__ delta, int64_t ld_delta, const float* __restrict__ post_w,
+                                                                  float post_add, float* x_out, const float* __restrict__ pre_w, float pre_add, float* __restrict__ y,
+                                                                  int64_t E, float eps, int S, ShiftArgs<TM> sh) {
+    sandwich_norm_row<TD, float, NV, SLABS, true, TM>(x, delta, ld_delta, post_w, post_add, 1.f, x_out, pre_w, pre_add, y, E, eps, S, sh);
 }
 
 // out[t, i] = act(gate) * up' with gate = in[t, i], up = in[t, I + i]
@@ -653,6 +701,56 @@ extern "C" int tgis_sandwich_norm_f32(const float* x, const void* delta, int64_t
         dispatch_y<bf16>(y_dtype, x, delta, ld_delta, post_w, post_add, 1.f, x_out, pre_w, pre_add, y, rows, E, eps, st);
     else
         dispatch_y<float>(y_dtype, x, delta, ld_delta, post_w, post_add, 1.f, x_out, pre_w, pre_add, y, rows, E, eps, st);
+    TGIS_CHECK_LAUNCH();
+    return TGIS_OK;
+}
+
+namespace {
+
+template <typename TD, bool SLABS, typename TM>
+void launch_sandwich_shift(const float* x, const void* delta, int64_t ld_delta, const float* post_w, float post_add, float* x_out, const float* pre_w, float pre_add, float* y,
+                           int64_t rows, int64_t E, float eps, int S, const ShiftArgs<TM>& sh, hipStream_t st) {
+    const auto kernel = E <= 512 * 4 ? sandwich_norm_shift_kernel<TD, 1, SLABS, TM> : E <= 512 * 8 ? sandwich_norm_shift_kernel<TD, 2, SLABS, TM>
+                                                                                                  : sandwich_norm_shift_kernel<TD, 4, SLABS, TM>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(512), 0, st, x, (const TD*)delta, ld_delta, post_w, post_add, x_out, pre_w, pre_add, y, E, eps, S, sh);
+}
+template <typename T>
+void dispatch_sandwich_shift(const float* x, const void* delta, int64_t ld_delta, bool typed, const float* post_w, float post_add, float* x_out, const float* pre_w,
+                             float pre_add, float* y, int64_t rows, int64_t E, float eps, int S, const float* state, const int32_t* slots, const int32_t* positions,
+                             const float* mu, void* mixes, hipStream_t st) {
+    const ShiftArgs<T> sh{state, slots, positions, mu, (T*)mixes};
+    if (S > 0)
+        launch_sandwich_shift<float, true, T>(x, delta, ld_delta, post_w, post_add, x_out, pre_w, pre_add, y, rows, E, eps, S, sh, st);
+    else if (typed)
+        launch_sandwich_shift<T, false, T>(x, delta, ld_delta, post_w, post_add, x_out, pre_w, pre_add, y, rows, E, eps, 0, sh, st);
+    else
+        launch_sandwich_shift<float, false, T>(x, delta, ld_delta, post_w, post_add, x_out, pre_w, pre_add, y, rows, E, eps, 0, sh, st);
+}
+
+}  // namespace
+
+// tgis_sandwich_norm_f32 (num_slabs 0) or tgis_sandwich_norm_f32_partial with an fp32 y, and tgis_token_shift_mix of that y where every row is its sequence's one token
+extern "C" int tgis_sandwich_norm_shift(const float* x, const void* delta, int64_t ld_delta, int delta_dtype, int num_slabs, const float* post_w, float post_add, float* x_out,
+                                        const float* pre_w, float pre_add, float* y, const float* shift_state, const int32_t* state_slots, const int32_t* positions,
+                                        const float* mu, int num_mixes, void* mixes, int mix_dtype, int64_t rows, int64_t E, float eps, void* stream) {
+    const char* what = "tgis_sandwich_norm_shift";
+    TGIS_CHECK_ARG(x && x_out && pre_w && y && shift_state && state_slots && positions && mu && mixes && rows >= 0 && rows < (1ll << 31), "%s: null tensor", what);
+    TGIS_CHECK_ARG(E > 0 && E % 4 == 0 && E <= 512 * 16 && num_mixes == SHIFT_MIXES, "%s: widths of a multiple of 4 up to 8192 and %d mixes", what, SHIFT_MIXES);
+    TGIS_CHECK_ARG(mix_dtype == TGIS_F16 || mix_dtype == TGIS_BF16, "%s: mixes are of two bytes", what);
+    TGIS_CHECK_ARG(num_slabs >= 0 && (num_slabs == 0 || delta) &&
+                       (!delta || (post_w && ld_delta >= E && ld_delta % 4 == 0 && (num_slabs > 0 || delta_dtype == TGIS_F32 || delta_dtype == mix_dtype))),
+                   "%s: delta needs its gain, a row stride and the mixes' dtype, or fp32", what);
+    TGIS_CHECK_ARG(((uintptr_t)x | (uintptr_t)delta | (uintptr_t)post_w | (uintptr_t)x_out | (uintptr_t)pre_w | (uintptr_t)y | (uintptr_t)shift_state | (uintptr_t)mu |
+                    (uintptr_t)mixes) % 16 == 0,
+                   "%s: tensors must be 16-byte aligned", what);
+    if (rows == 0) return TGIS_OK;
+    hipStream_t st = (hipStream_t)stream;
+    TgisTimedScope timed(TGIS_OP_NORM, st);
+    const bool typed = delta && num_slabs == 0 && delta_dtype == mix_dtype;
+    if (mix_dtype == TGIS_F16)
+        dispatch_sandwich_shift<f16>(x, delta, ld_delta, typed, post_w, post_add, x_out, pre_w, pre_add, y, rows, E, eps, num_slabs, shift_state, state_slots, positions, mu, mixes, st);
+    else
+        dispatch_sandwich_shift<bf16>(x, delta, ld_delta, typed, post_w, post_add, x_out, pre_w, pre_add, y, rows, E, eps, num_slabs, shift_state, state_slots, positions, mu, mixes, st);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }

@@ -111,9 +111,18 @@ class FlashLenisunModel:
         cfg, dt = self.config, self.dtype
         kv.cu_seqlens_q = cu_seqlens_q
         x = native.embedding_scaled_f32(input_ids, self.embed, cfg.embedding_scale)
-        first = self.layers[0]
+
+        def normed_for(layer, y, post_gain):
+            """x += norm(y), and the mixer input of `layer` behind it; of a recurrent one in steps of a token each its mixes with the tokens before, too."""
+            if layer.kind != "wkv":
+                return native.sandwich_norm_f32(x, y, post_gain, layer.norm1, cfg.eps, dt), None
+            if layer.mixer.mixed_by_norm(*x.shape, kv, dt):
+                return native.sandwich_norm_shift(x, y, post_gain, layer.norm1, cfg.eps, kv.state.shift[layer.mixer.layer_id], kv.state_slots, position_ids,
+                                                  layer.mixer.mu, dt)
+            return native.sandwich_norm_f32(x, y, post_gain, layer.norm1, cfg.eps, torch.float32), None
+
         # the normed input of layer 0; afterwards every sublayer's output is normed, added and normed again in one launch
-        h = native.sandwich_norm_f32(x, None, None, first.norm1, cfg.eps, torch.float32 if first.kind == "wkv" else dt)
+        h, mixes = normed_for(self.layers[0], None, None)
         v_first = None
         n = len(self.layers)
         for i, layer in enumerate(self.layers):
@@ -124,18 +133,18 @@ class FlashLenisunModel:
                 if i == self.first_blender:
                     v_first = layer.mixer.values_of(qkv)
             else:
-                y = layer.mixer.forward(h, position_ids, kv, dt, ends=ends)
+                y = layer.mixer.forward(h, position_ids, kv, dt, ends=ends, mixes=mixes)
             if ends is not None:
                 x = x.index_select(0, ends)
-            nxt = self.layers[i + 1] if i + 1 < n else None
-            after_dtype = torch.float32 if (nxt is not None and nxt.kind == "wkv") else dt
-            after_gain = nxt.norm1 if nxt is not None else self.final_norm
+            post_gain = layer.norm1b
             if layer.ff is not None:
                 h = native.sandwich_norm_f32(x, y, layer.norm1b, layer.norm2, cfg.eps, dt)
                 y = layer.ff(h, partial=True) if layer.dense_ff else layer.ff(h)
-                h = native.sandwich_norm_f32(x, y, layer.norm2b, after_gain, cfg.eps, after_dtype)
+                post_gain = layer.norm2b
+            if i + 1 < n:
+                h, mixes = normed_for(self.layers[i + 1], y, post_gain)
             else:
-                h = native.sandwich_norm_f32(x, y, layer.norm1b, after_gain, cfg.eps, after_dtype)
+                h = native.sandwich_norm_f32(x, y, post_gain, self.final_norm, cfg.eps, dt)
             if kv.residual_trace is not None:
                 kv.residual_trace.append(x.clone())
         return h  # final-normed, in the serving dtype

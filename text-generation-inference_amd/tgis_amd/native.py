@@ -143,6 +143,8 @@ SIGNATURES = {
                                                _vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tgis_attn_varlen": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64, _c_i64,
                                   _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_int, _vp]),
+    "tgis_sandwich_norm_shift": (_c_int, [_vp, _vp, _c_i64, _c_int, _c_int, _vp, _c_f, _vp, _vp, _c_f, _vp, _vp, _vp, _vp, _vp, _c_int, _vp, _c_int, _c_i64, _c_i64, _c_f,
+                                          _vp]),
     "tgis_token_shift_mix": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_int, _vp, _c_i64, _c_i64, _c_int, _vp]),
     "tgis_wkv_decay": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _c_i64, _c_int, _c_i64, _c_int, _vp]),
     "tgis_wkv_step": (_c_int, [_vp, _vp, _vp, _vp, _vp, _c_i64, _c_i64, _vp, _vp, _c_int, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _vp, _vp,
@@ -1468,6 +1470,25 @@ def sandwich_norm_f32(x: torch.Tensor, delta: Optional[torch.Tensor], post_w: Op
         _f32(post_w, "post_w"), float(post_add), _ptr(x), _f32(pre_w, "pre_w"), float(pre_add), _ptr(y),
         dtype_code3(y_dtype) if y is not None else F32, rows, E, float(eps), _stream()), "tgis_sandwich_norm_f32")
     return y
+
+
+def sandwich_norm_shift(x: torch.Tensor, delta, post_w, pre_w, eps: float, shift_state, state_slots, positions, mu, out_dtype):
+    """sandwich_norm_f32 to an fp32 y, and token_shift_mix of y for a step whose every row is its sequence's one token: (y, mixes)."""
+    rows, E = x.shape
+    assert x.dtype == torch.float32 and x.is_contiguous() and shift_state.shape[-1] == E and state_slots.shape[0] == positions.shape[0] == rows
+    y = torch.empty_like(x)
+    mixes = torch.empty((mu.shape[0], rows, E), dtype=out_dtype, device=x.device)
+    if isinstance(delta, Partial):
+        assert delta.shape == (rows, E) and delta.bias is None
+        slabs, ld, code, S = delta.slabs, delta.ld, F32, delta.S
+    else:
+        assert delta is None or (delta.shape == x.shape and delta.stride(1) == 1)
+        slabs, ld, code, S = (delta, delta.stride(0), dtype_code3(delta.dtype), 0) if delta is not None else (None, 0, F32, 0)
+    _check(load_library().tgis_sandwich_norm_shift(
+        _ptr(x), _ptr(slabs), ld, code, S, _f32(post_w, "post_w"), 1.0, _ptr(x), _f32(pre_w, "pre_w"), 1.0, _ptr(y), _f32(shift_state, "shift_state"),
+        _i32(state_slots, "state_slots"), _i32(positions, "positions"), _f32(mu, "mu"), mu.shape[0], _ptr(mixes), dtype_code3(out_dtype), rows, E, float(eps), _stream()),
+        "tgis_sandwich_norm_shift")
+    return y, mixes
 
 
 def dense_gemm_clamped_glu(x: torch.Tensor, w: DenseWeight, ws: Workspace, alpha: float, limit: float) -> torch.Tensor:

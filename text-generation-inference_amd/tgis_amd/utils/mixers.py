@@ -150,11 +150,17 @@ class WkvMixer:
         self.o = load_linear(weights, f"{prefix}.o")
         self.defer = can_defer(self.o)
 
-    def forward(self, h32: torch.Tensor, position_ids, step, dtype, ends: Optional[torch.Tensor] = None):
-        """h32 [T, W] fp32 (the normed mixer input, kept in fp32 because it is also the shift state).  ends: the output of these rows alone."""
+    def mixed_by_norm(self, rows: int, width: int, step, dtype) -> bool:
+        """Whether the norm in front leaves the mixes of such a step as well (native.sandwich_norm_shift): steps of a token each."""
+        return step.max_q_len == 1 and rows == step.state_slots.shape[0] and width % 4 == 0 and width <= 8192 and dtype in (torch.float16, torch.bfloat16)
+
+    def forward(self, h32: torch.Tensor, position_ids, step, dtype, ends: Optional[torch.Tensor] = None, mixes: Optional[torch.Tensor] = None):
+        """h32 [T, W] fp32 (the normed mixer input, kept in fp32 because it is also the shift state).  ends: the output of these rows alone.  mixes: of
+        h32 with the tokens before, where the norm has left them."""
         st = step.state
         state, shift = st.state[self.layer_id], st.shift[self.layer_id]
-        mixes = native.token_shift_mix(h32, shift, step.state_slots, step.cu_seqlens_q, position_ids, self.mu, dtype)
+        if mixes is None:
+            mixes = native.token_shift_mix(h32, shift, step.state_slots, step.cu_seqlens_q, position_ids, self.mu, dtype)
         T = h32.shape[0]
         HD = self.H * self.d
         rkvg = torch.empty((5, T, HD), dtype=dtype, device=h32.device)
