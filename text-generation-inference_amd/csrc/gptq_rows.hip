@@ -417,11 +417,12 @@ void launch_grows_k(const GRowsArgs& a, int per, hipStream_t st) {
 template <int KIND, int RB, int DS>
 void launch_grows_p(const GRowsArgs& a, int per, hipStream_t st) {
     if (per % 2 == 0) return launch_grows_k<KIND, 8, RB, DS, 2>(a, per, st);
-    if (per % 3 == 0) return launch_grows_k<KIND, 8, RB, DS, 3>(a, per, st);
+    if constexpr (RB == 1 || DS <= 2)
+        if (per % 3 == 0) return launch_grows_k<KIND, 8, RB, DS, 3>(a, per, st);
     launch_grows_k<KIND, 8, RB, DS, 1>(a, per, st);
 }
 // One workgroup a CU.  us at 16 rows, turns of one, two, three units: gate | up of 4096 x 22016 (6 units a workgroup) 14.3 / 12.9 / 13.3, of 2048 x 11264 (3) 6.6 / 6.5 / 5.8; qkv of
-// 4096 x 12288 (3) 10.0 / 11.7 / 9.6; from K 5120 on x leaves the registers of one: 5120 x 27648 (7) 19.7 / 21.2 / 22.5.  Sixteen waves take less of x each: 8192 x 57344
+// 4096 x 12288 (3) 10.0 / 11.7 / 9.6, at 32 rows 11.5 / 13.4 / 12.0; from K 5120 on x leaves the registers of one: 5120 x 27648 (7) 19.7 / 21.2 / 22.5.  Sixteen waves take less of x each: 8192 x 57344
 // 54.2 -> 49.1, but 4096 x 22016 14.8 and, with what a rotation needs besides, 8192 x 10240 17.9 -> 36.5.
 template <int KIND>
 int launch_grows(const GRowsArgs& a, hipStream_t st) {
