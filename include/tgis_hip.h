@@ -261,24 +261,26 @@ int tgis_dense_rows16_norm_head(const void* hw, const float* sums, float eps, co
                                 int64_t N, void* stream);
 /* The same for int4 weights (the images of tgis_gptq_prepare) in f16: decode steps of up to 32 rows, K a multiple of 128 up to 12288, where it norms 8192 (up to
  * 16 rows) or 4096, groups of 64 2^n rows.
- * The stream between the launches is T(h) as rows [M][width], T(h * norm_w * unit) of the norm weight that is next, in 32-row fragment order (TGIS_LD_FRAGMENTS) and its
- * columns where `places` (null: in their order) has them, and sums: the sums of h^2 of sixteen columns each, h in fp32, as [width / 64][32 rows][4].  unit: a power of two
- * by which |norm_w| is at most one; that of the norm in front of the product in norm_silu and norm_rope.  x of `residual` and the output of `norm_silu` are in fragment order.
+ * The stream between the launches is T(h) as rows [M][width], T(h * norm_w * unit * p) of the norm weight that is next, p a power of two of each row, in 32-row fragment order
+ * (TGIS_LD_FRAGMENTS) and its columns where `places` (null: in their order) has them, and sums: the sums of h^2 of sixteen columns each, h in fp32, as [width / 64][32 rows][4],
+ * behind them the sums of h^2 of whole rows [32] and 1 / p [32].  unit: a power of two by which |norm_w| is at most one; that of the norm in front of the product in norm_silu and
+ * norm_rope.  p brings a bound on the row's |h| to 2^14 .. 2^15.  x of `residual` and the output of `norm_silu` are in fragment order.
  *   tgis_gptq_rows_embed      the stream of M tokens (zeros for an id outside the vocabulary)
- *   tgis_gptq_rows_residual   h = T(x W) + T(h); N (the width) a multiple of 64
+ *   tgis_gptq_rows_residual   h = T(x W) + T(h); N (the width) a multiple of 64; w_norm: at least the largest 2-norm of a column of W.  Takes the sums of whole rows that a norm_*
+ *                             of the same h has left: a step's launches alternate
  *   tgis_gptq_rows_sum        the same behind a product that tgis_gptq_gemm_partial left as slabs [num_slabs][32][ld]
- *   tgis_gptq_rows_norm_*     of T(h * norm_w * unit) and its sums: products times rsqrt(mean h^2 + eps) / unit, from there as tgis_gptq_gemm_f16 (act 2) and
+ *   tgis_gptq_rows_norm_*     of T(h * norm_w * unit * p) and its sums: products times rsqrt(mean h^2 + eps) / (unit p), from there as tgis_gptq_gemm_f16 (act 2) and
  *                             tgis_gptq_gemm_rope_f16; norm_silu: N / 2 a multiple of 64 */
 int tgis_gptq_rows_ok(int64_t M, int64_t K, int64_t N, int64_t groups, int norm);
 int tgis_gptq_rows_embed(const int64_t* ids, const void* table, const void* norm_w, const int32_t* places, float unit, void* h, void* hw, float* sums, int64_t M,
                          int64_t K, int64_t vocab, void* stream);
-int tgis_gptq_rows_residual(const void* x, const void* prepared, const void* norm_w, const int32_t* places, float unit, void* h, void* hw, float* sums, int64_t M,
-                            int64_t K, int64_t N, int64_t groups, void* stream);
+int tgis_gptq_rows_residual(const void* x, const void* prepared, float w_norm, const void* norm_w, const int32_t* places, float unit, void* h, void* hw, float* sums,
+                            int64_t M, int64_t K, int64_t N, int64_t groups, void* stream);
 int tgis_gptq_rows_sum(const float* slabs, int num_slabs, int64_t ld, const void* norm_w, const int32_t* places, float unit, void* h, void* hw, float* sums,
                        int64_t M, int64_t N, void* stream);
-int tgis_gptq_rows_norm_silu(const void* hw, const float* sums, float eps, float unit, const void* prepared, void* out, int64_t M, int64_t K, int64_t N, int64_t groups,
+int tgis_gptq_rows_norm_silu(const void* hw, float* sums, float eps, float unit, const void* prepared, void* out, int64_t M, int64_t K, int64_t N, int64_t groups,
                              void* stream);
-int tgis_gptq_rows_norm_rope(const void* hw, const float* sums, float eps, float unit, const void* prepared, const void* bias, const int32_t* positions,
+int tgis_gptq_rows_norm_rope(const void* hw, float* sums, float eps, float unit, const void* prepared, const void* bias, const int32_t* positions,
                              const int32_t* slots, const void* cos, const void* sin, void* q_out, int64_t ldq, void* k_pool, void* v_pool, int64_t M, int64_t K,
                              int64_t groups, int64_t H, int64_t Hkv, int64_t D, void* stream);
 

@@ -5,17 +5,22 @@
 // A layer of 4096, 11008 at 11 rows was seven launches: 38 us of products for 105 MB and two norm launches of 4.7 us, each a row on a CU and a boundary.  Here
 //   * a unit is sixteen columns and the whole k range, so that nothing is left to add up: 256 units for 4096 columns, one a workgroup; the stream's T(h), the norm's
 //     operand T(h w) and sums of h^2 leave from there, and 1 / rms is a factor of the next product's finished sums.  T(h w) is f16, which 1 / rms would bring into range:
-//     it is multiplied by a power of two (`unit`) that makes the largest |w| at most one, so that it holds what T(h) holds.  An operand is rounded once either way;
+//     two powers of two do, `unit`, which makes the largest |w| at most one, and one of each row, from a bound on the row's |h| that every workgroup of a launch
+//     knows: sqrt(sum h^2) in front of the add, which the norm's product has left, and |x| times the largest column of W behind it (Cauchy and Schwarz; |x|^2 is the
+//     diagonal of an instruction x x^T, which the matrix unit has time for).  The bound is set to 2^14 .. 2^15, and may be 2^10 above what a row holds: f16 is
+//     normal down to 2^-14.  An operand is rounded once either way.  (With `unit` alone rows of small h left f16's normal range: error of a product of 4096 columns, one weight
+//     of the norm 20 times the others, h of 1e-3 5.4e-4 and of 1e-4 6.4e-3, where the norm's own launch has 2e-4);
 //   * the product is v_mfma_f32_16x16x32 with the weights as rows.  A lane's sixteen bytes are 32 k of one column; lanes l / 16 hold the four halves of two k64-steps, so that word i of
 //     all of them is one operand against chunk i of x of the same halves: no rows of lanes to swap (gptq_wide_body.h), and 1 KiB of image to four instructions;
 //   * in front of a norm a wave keeps x of its k-steps in registers (16 VGPR each) and takes units in turn; behind, x is asked for a step ahead.
-// us a launch of 4096, 11008 at 16 rows, the other launches and the norm behind them / these: qkv 10.1 / 9.6, o 8.7 / 5.5, gate | up 13.8 / 12.9, down 12.5 / 10.0: 2.7 TB/s of
+// us a launch of 4096, 11008 at 16 rows, the other launches and the norm behind them / these: qkv 10.1 / 9.6, o 8.8 / 5.6, gate | up 13.8 / 13.3, down 11.7 / 10.7 (of these two x x^T
+// and the bound 0.2 and 0.6): 2.7 TB/s of
 // weights, bound by the launch's own ends and, of what is left, by the round trip of a turn's loads (weights of a turn ahead in registers of their own cost 0.7 us: x holds 64).
-// Whole steps at ctx 137, 1, 4, 16 rows: eight layers of 4096, 11008 484 / 449, 520 / 467, 579 / 522; of 2048, 5632 337 / 279, 341 / 282, 359 / 298; of 3072, 8192 394 / 361, 402 /
-// 367, 424 / 388; of 5120, 13824 607 / 598, 623 / 608, 705 / 696; four of 8192, 28672 623 / 565, 624 / 570, 646 / 600.  At 17 - 32 rows a weight feeds two instructions
-// and x of a whole k range takes as long as the weights: products as above at 32 rows 12.0 / 11.4, 9.9 / 6.7, 16.4 / 16.1, 13.3 / 13.3.
-// Steps at 24, 32 rows: 4096, 11008 679 / 634, 708 / 686; 2048, 5632 388 / 335, 399 / 357; 3072, 8192 468 / 451, 486 / 477; 5120, 13824, where it is 320 residual units and x
-// leaves the registers of one unit, 850 / 850, 858 / 869: not served.
+// Whole steps at ctx 137, 1, 4, 16 rows: eight layers of 4096, 11008 440 / 419, 471 / 424, 526 / 483; of 2048, 5632 294 / 238, 295 / 239, 308 / 253; of 3072, 8192 349 / 330, 365 /
+// 335, 379 / 349; of 5120, 13824 534 / 564, 574 / 572, 645 / 646; four of 8192, 28672 575 / 528, 577 / 533, 593 / 553.  At 17 - 32 rows a weight feeds two instructions
+// and x of a whole k range takes as long as the weights: products as above at 32 rows 12.0 / 11.8, 9.6 / 6.8, 16.4 / 16.1, 13.3 / 14.1.
+// Steps at 24, 32 rows: 4096, 11008 608 / 575, 634 / 617; 2048, 5632 334 / 284, 340 / 299; 3072, 8192 418 / 402, 429 / 421; 5120, 13824, where it is 320 residual units and x
+// leaves the registers of one unit, 782 / 783, 793 / 793: not served.
 #include <algorithm>
 #include "gptq_gemm_body.h"
 
@@ -25,7 +30,7 @@ constexpr int GROWS_M = 32;
 enum { GROWS_ROPE, GROWS_SILU };
 struct GRowsArgs {
     const f16* x;       // T(h w unit) or an activation, fragment order (xf_off)
-    const float* sums;  // [K / 64][32 rows][4]: sums of h^2 of sixteen columns
+    float* sums;        // [K / 64][32 rows][4]: sums of h^2 of sixteen columns; behind them of whole rows [32], and what a row's operand is to be multiplied by [32]
     float eps, unit;
     const uint8_t* prep;
     int64_t offB;
@@ -36,7 +41,7 @@ struct GRowsArgs {
     const f16* norm_w;
     const int32_t* places;  // where the next product wants column k of its operand (null: at k)
     f16 *h, *hw;            // T(h) [M][N]; T(h w unit), fragment order
-    float* sums_out;
+    float w_norm;           // at least the largest 2-norm of a column of W
     // ROPE (as tgis_gptq_gemm_rope_f16)
     const f16* bias;
     const int32_t *positions, *slots;
@@ -45,6 +50,15 @@ struct GRowsArgs {
     int H, Hkv, D;
 };
 __device__ __forceinline__ int64_t sums16_off(int m, int k) { return ((int64_t)(k >> 6) * GROWS_M + m) * 4 + ((k >> 4) & 3); }
+__device__ __forceinline__ float* row_sums(float* sums, int width) { return sums + (int64_t)(width >> 4) * GROWS_M; }
+__device__ __forceinline__ float* row_factors(float* sums, int width) { return row_sums(sums, width) + GROWS_M; }
+
+// c of the 2^c that brings a bound on a row's |h|, given by its square, to 2^14 .. 2^15 (squares that are zero, infinite or NaN: an end of a range whose powers fp32 holds)
+__device__ __forceinline__ int row_power(float square) {
+    const int e = (int)(__builtin_bit_cast(uint32_t, square) >> 23 & 255) - 127;
+    return min(max(14 - (e >> 1), -64), 64);
+}
+__device__ __forceinline__ f16 operand(float h, f16 w, float unit, int c) { return (f16)ldexpf(h * ((float)w * unit), c); }
 
 // byte offset of a lane's part (32 k of one column `col` of the tile) within the two k64-steps of a tile, and of x's (row m) within its two
 __device__ __forceinline__ uint32_t grows_w_off(int kq, int col) { return (kq >> 1) * 1024 + ((kq & 1) * 32 + col) * 16; }
@@ -71,31 +85,52 @@ struct GRowsDequant {
     }
 };
 
-// the stream of tokens: sixteen columns a thread
-__global__ __launch_bounds__(256) void gptq_rows_embed_kernel(const int64_t* __restrict__ ids, const f16* __restrict__ table, int64_t vocab, GRowsArgs a) {
-    const int at = blockIdx.x * 256 + threadIdx.x, m = at % GROWS_M, k = at / GROWS_M * 16;
-    if (m >= a.M || k >= a.K) return;
-    const int64_t id = ids[m];
-    float ss = 0.f;
+// the largest of v over a workgroup of T threads
+template <int T>
+__device__ __forceinline__ float block_max(float v, float (&red)[T / 64]) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        f16x8 v{}, y;
-        if (id >= 0 && id < vocab) v = ld16<f16x8>(table + id * a.K + k + p * 8);
-        const f16x8 w = ld16<f16x8>(a.norm_w + k + p * 8);
+    for (int d = 1; d < 64; d <<= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < T / 64; ++k) v = fmaxf(v, red[k]);
+    return v;
+}
+
+// the stream of tokens, a row a workgroup
+__global__ __launch_bounds__(256) void gptq_rows_embed_kernel(const int64_t* __restrict__ ids, const f16* __restrict__ table, int64_t vocab, GRowsArgs a) {
+    __shared__ float red[4];
+    const int m = blockIdx.x;
+    const int64_t id = ids[m];
+    const bool known = id >= 0 && id < vocab;
+    auto columns = [&](int k) { return known ? ld16<f16x8>(table + id * a.K + k) : f16x8{}; };
+    float top = 0.f;
+    for (int k = threadIdx.x * 8; k < a.K; k += 2048) {
+        const f16x8 v = columns(k);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf((float)v[e]));
+    }
+    const int c = row_power(block_max<256>(top * top, red));
+    for (int k = threadIdx.x * 8; k < a.K; k += 2048) {
+        const f16x8 v = columns(k), w = ld16<f16x8>(a.norm_w + k);
+        f16x8 y;
+        float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             ss += (float)v[e] * (float)v[e];
-            y[e] = (f16)((float)v[e] * ((float)w[e] * a.unit));
+            y[e] = operand((float)v[e], w[e], a.unit, c);
         }
-        st16(a.h + (int64_t)m * a.K + k + p * 8, v);
+        st16(a.h + (int64_t)m * a.K + k, v);
         if (a.places) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) a.hw[xf_off(m, a.places[k + p * 8 + e], a.K)] = y[e];
+            for (int e = 0; e < 8; ++e) a.hw[xf_off(m, a.places[k + e], a.K)] = y[e];
         } else {
-            st16(a.hw + xf_off(m, k + p * 8, a.K), y);
+            st16(a.hw + xf_off(m, k, a.K), y);
         }
+        ss += __shfl_xor(ss, 1, 64);
+        if ((threadIdx.x & 1) == 0) a.sums[sums16_off(m, k)] = ss;
     }
-    a.sums_out[sums16_off(m, k)] = ss;
+    if (threadIdx.x == 0) row_factors(a.sums, a.K)[m] = ldexpf(1.f, -c);
 }
 
 // Products of a normed operand.  A unit is columns c0 .. +7 and c0 + 16 .. +23 of a tile: the halves of a rotation, or gate and up.  DS: double k64-steps of a wave at most;
@@ -112,6 +147,7 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
     const int fp = w % FW / RB, fb = w % RB, frow = fb * 16 + m;  // the unit of a turn and the row that this lane finishes
     const int u0 = blockIdx.x * per, n = min(per, units - u0);
 
+    const float factor = row_factors(a.sums, a.K)[min(frow, a.M - 1)] / a.unit;
     int32_t pos = 0, slot = 0;
     if (KIND == GROWS_ROPE) {
         pos = a.positions[min(frow, a.M - 1)];
@@ -214,7 +250,8 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
         float tot = 0.f;
 #pragma unroll
         for (int k = 0; k < W; ++k) tot += part[k][frow];
-        const float rstd = rsqrtf(tot / a.K + a.eps) / a.unit;
+        if (blockIdx.x == 0 && at == 0 && kq == 0 && frow < a.M) row_sums(a.sums, a.K)[frow] = tot;  // (for the residual product behind)
+        const float rstd = rsqrtf(tot / a.K + a.eps) * factor;
         f32x4 v = *reinterpret_cast<const f32x4*>(&red[r][fp][fb][0][lane * 4]);
 #pragma unroll
         for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[r][fp][fb][k][lane * 4]);
@@ -258,12 +295,13 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
     turn(i, std::false_type{});
 }
 
-// h += T(x W) and what the next norm's product needs of it; a unit of sixteen columns a workgroup.  DS: double k64-steps of a wave at most.  us at 16 rows, eight waves / sixteen: 4096
+// h += T(x W) and what the next norm's product needs of it; a unit of sixteen columns a workgroup.  DS: double k64-steps of a wave at most.  us at 16 rows, eight waves / sixteen (without x x^T): 4096
 // x 4096 5.5 / 5.8, 11008 x 4096 10.0 / 10.3, 2048 x 2048 3.7 / 4.6, 8192 x 8192 15.0 / 16.3; x asked for one, three, five steps ahead 10.0 / 10.3 / 10.5 (11008 x 4096).
 template <int RB, int DS>
 __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
     constexpr int W = 8;
     __shared__ __attribute__((aligned(16))) float red[RB][W][64 * 4];
+    __shared__ __attribute__((aligned(16))) float squares[16 * RB][W];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int steps = a.K >> 7, mine = (steps - w + W - 1) / W;
     const int m = lane & 15, kq = lane >> 4;
@@ -302,7 +340,9 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
     const int frow = w * 16 + m;
     f16x4 res{}, nw{};
     int32_t at[4] = {};
+    float before = 0.f;
     if (w < RB) {
+        before = row_sums(a.sums, a.N)[min(frow, a.M - 1)];
         res = *reinterpret_cast<const f16x4*>(a.h + (int64_t)min(frow, a.M - 1) * a.N + col);
         nw = *reinterpret_cast<const f16x4*>(a.norm_w + col);
         if (a.places) {
@@ -311,16 +351,28 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
         }
     }
     const GRowsDequant dq;
-    f32x4 acc[RB] = {};
+    f32x4 acc[RB] = {}, gram[RB] = {};  // gram: rows by rows of x
 #pragma unroll
     for (int j = 0; j < DS; ++j) {
         dq.mma(wq[j], sz[j], x[j & 1], acc);
+#pragma unroll
+        for (int b = 0; b < RB; ++b)  // (of steps past this wave's last, too, which are another's: the bound is only higher)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) gram[b] = mfma16(x[j & 1][b][i], x[j & 1][b][i], gram[b]);
         if (j + 2 < DS) ask_x(j & 1, j + 2);
     }
 #pragma unroll
-    for (int b = 0; b < RB; ++b) *reinterpret_cast<f32x4*>(&red[b][w][lane * 4]) = acc[b];
+    for (int b = 0; b < RB; ++b) {
+        *reinterpret_cast<f32x4*>(&red[b][w][lane * 4]) = acc[b];
+        const float lo = m & 1 ? gram[b][1] : gram[b][0], hi = m & 1 ? gram[b][3] : gram[b][2];
+        if (kq == m >> 2) squares[b * 16 + m][w] = m & 2 ? hi : lo;
+    }
     __syncthreads();
     if (w >= RB) return;
+    float xx = 0.f;
+#pragma unroll
+    for (int k = 0; k < W; ++k) xx += squares[frow][k];
+    const int c = row_power(2.f * (before + xx * a.w_norm * a.w_norm));  // (a + b)^2 <= 2 (a^2 + b^2)
     f32x4 v = *reinterpret_cast<const f32x4*>(&red[w][0][lane * 4]);
 #pragma unroll
     for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4*>(&red[w][k][lane * 4]);
@@ -331,7 +383,7 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
         const float f = (float)(f16)v[e] + (float)res[e];
         ss += f * f;
         h[e] = (f16)f;
-        hw[e] = (f16)(f * ((float)nw[e] * a.unit));
+        hw[e] = operand(f, nw[e], a.unit, c);
     }
     ss += __shfl_xor(ss, 16, 64);
     ss += __shfl_xor(ss, 32, 64);
@@ -343,36 +395,58 @@ __global__ __launch_bounds__(512) void gptq_rows_residual_kernel(GRowsArgs a) {
     } else {
         *reinterpret_cast<f16x4*>(a.hw + xf_off(frow, col, a.N)) = hw;
     }
-    if (kq == 0) a.sums_out[sums16_off(frow, col)] = ss;
+    if (kq == 0) a.sums[sums16_off(frow, col)] = ss;
+    if (kq == 0 && blockIdx.x == 0) row_factors(a.sums, a.N)[frow] = ldexpf(1.f, -c);
 }
 
-// The same behind a product whose k range was split: S slabs [32][ld] of a tgis_gptq_gemm_partial, sixteen columns a thread
-__global__ __launch_bounds__(64) void gptq_rows_sum_kernel(const float* __restrict__ slabs, int S, int64_t ld, GRowsArgs a) {
-    const int per = a.N >> 4, at = blockIdx.x * 64 + threadIdx.x, m = at / per, k = at % per * 16;
-    if (m >= a.M) return;
-    float ss = 0.f;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const f16x8 res = ld16<f16x8>(a.h + (int64_t)m * a.N + k + p * 8), w = ld16<f16x8>(a.norm_w + k + p * 8);
-        f32x4 lo, hi;
-        sum_slabs8(slabs + (int64_t)m * ld + k + p * 8, 32 * ld, S, lo, hi);
-        f16x8 h, hw;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float f = (float)(f16)(e < 4 ? lo[e & 3] : hi[e & 3]) + (float)res[e];
-            ss += f * f;
-            h[e] = (f16)f;
-            hw[e] = (f16)(f * ((float)w[e] * a.unit));
-        }
-        st16(a.h + (int64_t)m * a.N + k + p * 8, h);
+// The same behind a product whose k range was split: S slabs [32][ld] of a tgis_gptq_gemm_partial.  A row a workgroup, which has its largest |h| then: 11 - 32 rows of 4096 3.6 - 3.9 us (a
+// thread per sixteen columns wherever it runs, which has not, 3.1).
+__global__ __launch_bounds__(1024) void gptq_rows_sum_kernel(const float* __restrict__ slabs, int S, int64_t ld, GRowsArgs a) {
+    __shared__ float red[16];
+    const int m = blockIdx.x;
+    float f[8];
+    f16x8 w;
+    int32_t at[8];
+    auto columns = [&](int k) {
+        const f16x8 res = ld16<f16x8>(a.h + (int64_t)m * a.N + k);
+        w = ld16<f16x8>(a.norm_w + k);
         if (a.places) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) a.hw[xf_off(m, a.places[k + p * 8 + e], a.N)] = hw[e];
-        } else {
-            st16(a.hw + xf_off(m, k + p * 8, a.N), hw);
+            for (int e = 0; e < 8; ++e) at[e] = a.places[k + e];
         }
+        f32x4 lo, hi;
+        sum_slabs8(slabs + (int64_t)m * ld + k, 32 * ld, S, lo, hi);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = (float)(f16)(e < 4 ? lo[e & 3] : hi[e & 3]) + (float)res[e];
+    };
+    float top = 0.f;
+    for (int k = threadIdx.x * 8; k < a.N; k += 8192) {
+        columns(k);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) top = fmaxf(top, fabsf(f[e]));
     }
-    a.sums_out[sums16_off(m, k)] = ss;
+    const int c = row_power(block_max<1024>(top * top, red));
+    for (int k = threadIdx.x * 8; k < a.N; k += 8192) {
+        if (a.N > 8192) columns(k);
+        f16x8 h, hw;
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            ss += f[e] * f[e];
+            h[e] = (f16)f[e];
+            hw[e] = operand(f[e], w[e], a.unit, c);
+        }
+        st16(a.h + (int64_t)m * a.N + k, h);
+        if (a.places) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) a.hw[xf_off(m, at[e], a.N)] = hw[e];
+        } else {
+            st16(a.hw + xf_off(m, k, a.N), hw);
+        }
+        ss += __shfl_xor(ss, 1, 64);
+        if ((threadIdx.x & 1) == 0) a.sums[sums16_off(m, k)] = ss;
+    }
+    if (threadIdx.x == 0) row_factors(a.sums, a.N)[m] = ldexpf(1.f, -c);
 }
 
 // groups of 64 2^n rows, as gptq_wide_body.h; K of whole double steps, as many as a wave's registers hold of x (or, where steps of 5120 columns and more
@@ -384,7 +458,7 @@ bool grows_fits(int64_t M, int64_t K, int64_t N, int64_t groups, bool norm) {
     return groups == 1 || (K / groups % 64 == 0 && (spg & (spg - 1)) == 0);
 }
 
-int grows_args(const char* what, GRowsArgs& a, const void* x, const float* sums, float eps, float unit, const void* prepared, int64_t M, int64_t K, int64_t N,
+int grows_args(const char* what, GRowsArgs& a, const void* x, float* sums, float eps, float unit, const void* prepared, int64_t M, int64_t K, int64_t N,
                int64_t groups, bool norm) {
     TGIS_CHECK_ARG(x && prepared && sums && unit > 0.f, "%s: null tensor or bad factor", what);
     TGIS_CHECK_ARG(grows_fits(M, K, N, groups, norm), "%s: up to %d rows, K a multiple of 128 up to %d, groups of 64 2^n (M=%ld K=%ld N=%ld groups=%ld)", what, GROWS_M,
@@ -474,25 +548,25 @@ extern "C" int tgis_gptq_rows_embed(const int64_t* ids, const void* table, const
     a.unit = unit;
     a.h = (f16*)h;
     a.hw = (f16*)hw;
-    a.sums_out = sums;
-    hipLaunchKernelGGL(gptq_rows_embed_kernel, dim3((unsigned)cdiv64(K / 16 * GROWS_M, 256)), dim3(256), 0, (hipStream_t)stream, ids, (const f16*)table, vocab, a);
+    a.sums = sums;
+    hipLaunchKernelGGL(gptq_rows_embed_kernel, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, ids, (const f16*)table, vocab, a);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
 
-extern "C" int tgis_gptq_rows_residual(const void* x, const void* prepared, const void* norm_w, const int32_t* places, float unit, void* h, void* hw, float* sums,
-                                       int64_t M, int64_t K, int64_t N, int64_t groups, void* stream) {
+extern "C" int tgis_gptq_rows_residual(const void* x, const void* prepared, float w_norm, const void* norm_w, const int32_t* places, float unit, void* h, void* hw,
+                                       float* sums, int64_t M, int64_t K, int64_t N, int64_t groups, void* stream) {
     const char* what = "tgis_gptq_rows_residual";
     GRowsArgs a;
     const int rc = grows_args(what, a, x, sums, 0.f, unit, prepared, M, K, N, groups, false);
     if (rc != TGIS_OK) return rc;
-    TGIS_CHECK_ARG(norm_w && h && hw && ((uintptr_t)norm_w | (uintptr_t)h | (uintptr_t)hw) % 16 == 0 && N % 64 == 0,
-                   "%s: null or unaligned tensor, or a width that is no multiple of 64", what);
+    TGIS_CHECK_ARG(norm_w && h && hw && ((uintptr_t)norm_w | (uintptr_t)h | (uintptr_t)hw) % 16 == 0 && N % 64 == 0 && w_norm >= 0.f,
+                   "%s: null or unaligned tensor, a width that is no multiple of 64, or no bound on the columns", what);
     a.norm_w = (const f16*)norm_w;
     a.places = places;
     a.h = (f16*)h;
     a.hw = (f16*)hw;
-    a.sums_out = sums;
+    a.w_norm = w_norm;
     TgisTimedScope timed(TGIS_OP_GPTQ_GEMM, (hipStream_t)stream);
     if (M <= 16)
         launch_grows_residual<1>(a, (hipStream_t)stream);
@@ -516,13 +590,13 @@ extern "C" int tgis_gptq_rows_sum(const float* slabs, int num_slabs, int64_t ld,
     a.unit = unit;
     a.h = (f16*)h;
     a.hw = (f16*)hw;
-    a.sums_out = sums;
-    hipLaunchKernelGGL(gptq_rows_sum_kernel, dim3((unsigned)cdiv64(M * (N / 16), 64)), dim3(64), 0, (hipStream_t)stream, slabs, num_slabs, ld, a);
+    a.sums = sums;
+    hipLaunchKernelGGL(gptq_rows_sum_kernel, dim3((unsigned)M), dim3(1024), 0, (hipStream_t)stream, slabs, num_slabs, ld, a);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }
 
-extern "C" int tgis_gptq_rows_norm_silu(const void* hw, const float* sums, float eps, float unit, const void* prepared, void* out, int64_t M, int64_t K, int64_t N,
+extern "C" int tgis_gptq_rows_norm_silu(const void* hw, float* sums, float eps, float unit, const void* prepared, void* out, int64_t M, int64_t K, int64_t N,
                                         int64_t groups, void* stream) {
     const char* what = "tgis_gptq_rows_norm_silu";
     GRowsArgs a;
@@ -533,7 +607,7 @@ extern "C" int tgis_gptq_rows_norm_silu(const void* hw, const float* sums, float
     return launch_grows<GROWS_SILU>(a, (hipStream_t)stream);
 }
 
-extern "C" int tgis_gptq_rows_norm_rope(const void* hw, const float* sums, float eps, float unit, const void* prepared, const void* bias, const int32_t* positions,
+extern "C" int tgis_gptq_rows_norm_rope(const void* hw, float* sums, float eps, float unit, const void* prepared, const void* bias, const int32_t* positions,
                                         const int32_t* slots, const void* cos, const void* sin, void* q_out, int64_t ldq, void* k_pool, void* v_pool, int64_t M,
                                         int64_t K, int64_t groups, int64_t H, int64_t Hkv, int64_t D, void* stream) {
     const char* what = "tgis_gptq_rows_norm_rope";

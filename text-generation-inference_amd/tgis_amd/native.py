@@ -106,7 +106,7 @@ SIGNATURES = {
     "tgis_dense_rows16_norm_head": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_gptq_rows_ok": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_int]),
     "tgis_gptq_rows_embed": (_c_int, [_vp, _vp, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _vp]),
-    "tgis_gptq_rows_residual": (_c_int, [_vp, _vp, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
+    "tgis_gptq_rows_residual": (_c_int, [_vp, _vp, _c_f, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_gptq_rows_sum": (_c_int, [_vp, _c_int, _c_i64, _vp, _vp, _c_f, _vp, _vp, _vp, _c_i64, _c_i64, _vp]),
     "tgis_gptq_rows_norm_silu": (_c_int, [_vp, _vp, _c_f, _c_f, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _vp]),
     "tgis_gptq_rows_norm_rope": (_c_int, [_vp, _vp, _c_f, _c_f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
@@ -462,6 +462,11 @@ class GptqWeight:
                 self.perm = perm_buf
         if explicit is not None:
             self.perm = explicit.to(dev, torch.int32).contiguous()
+        self.column_norm = None
+        if not self.flags:  # at least the largest 2-norm of a column (gptq_rows_residual): no value is further from its zero than the ends of the range
+            zeros = ((qzeros[:, :, None] >> (4 * torch.arange(8, dtype=torch.int32, device=dev))) & 15).view(self.groups, -1) + 1
+            reach = torch.maximum(zeros, 15 - zeros) * scales.float()
+            self.column_norm = float((self.K // self.groups * (reach * reach).sum(0).max()).sqrt()) * (1 + 2.0 ** -10)
         torch.cuda.current_stream().synchronize()  # qweight/qzeros/scales may be freed by the caller
 
     def in_order(self) -> "GptqWeight":
@@ -1009,7 +1014,7 @@ class Int4RowsStream:
         self.M, self.width, self.device = M, width, device
         self.h = torch.empty((M, width), dtype=torch.float16, device=device)
         self.hw = FragAct.empty(M, width, device)
-        self.sums = torch.empty(width // 16 * GPTQ_ROWS_MAX_M, dtype=torch.float32, device=device)
+        self.sums = torch.empty((width // 16 + 2) * GPTQ_ROWS_MAX_M, dtype=torch.float32, device=device)
         self.unit = 1.0
 
     @staticmethod
@@ -1024,11 +1029,11 @@ class Int4RowsStream:
 
 
 def gptq_rows_residual(x: FragAct, w: GptqWeight, h: Int4RowsStream, norm: Int4NormInput) -> None:
-    """h += x @ W, both rounded first, in front of `norm`."""
+    """h += x @ W, both rounded first, in front of `norm`; behind a product of the normed h."""
     assert x.dtype == norm.weight.dtype == torch.float16 and x.K == w.K and not w.flags and x.M == h.M and w.N == h.width == norm.weight.numel()
     h.unit = norm.unit
-    _check(load_library().tgis_gptq_rows_residual(_ptr(x.buf), _ptr(w.image), _ptr(norm.weight), _ptr(norm.places), norm.unit, _ptr(h.h), _ptr(h.hw.buf), _ptr(h.sums),
-                                                  h.M, w.K, w.N, w.groups, _stream()), "tgis_gptq_rows_residual")
+    _check(load_library().tgis_gptq_rows_residual(_ptr(x.buf), _ptr(w.image), w.column_norm, _ptr(norm.weight), _ptr(norm.places), norm.unit, _ptr(h.h), _ptr(h.hw.buf),
+                                                  _ptr(h.sums), h.M, w.K, w.N, w.groups, _stream()), "tgis_gptq_rows_residual")
 
 
 def gptq_rows_sum(part: "Partial", h: Int4RowsStream, norm: Int4NormInput) -> None:
