@@ -596,12 +596,12 @@ class FlashLlamaForCausalLM:
         return got
 
     def rows16_path(self, rows: int) -> bool:
-        """The same of the launches for more rows (FlashLlamaModel.forward_rows16)."""
+        """The same of the launches for more rows (FlashLlamaModel.forward_rows16), which may split their sums (TGIS_DEFER_REDUCE)."""
         got = self._rows16_path.get(rows)
         if got is None:
             got = self._rows16_path[rows] = (native.DENSE_ROWS16_MIN_M <= rows <= min(native.DENSE_ROWS16_MAX_M, SKINNY_MAX_M)
                                              and self._plain_head() and self.model.serves_rows16(rows))
-        return got
+        return got and DEFER_REDUCE
 
     def _serves_rows(self, rows: int) -> bool:
         return self._plain_head() and self.model.serves_rows(rows, native.dense_rows_ok)
