@@ -44,6 +44,8 @@ def test_same_steps(gpu_device, monkeypatch, dtype, graphs, rows):
 
     calls, run = [], FlashLlamaModel.forward_rows
     monkeypatch.setattr(FlashLlamaModel, "forward_rows", lambda self, ids, *a: calls.append(ids.shape[0]) or run(self, ids, *a))
+    # (three and four rows of bf16 are forward_rows16's, but for TGIS_DEFER_REDUCE=0)
+    monkeypatch.setattr(FlashLlamaForCausalLM, "rows16_path", lambda self, n: False)
     lm, cfg = model(dtype)
     got, pages = decode(lm, cfg.vocab_size, rows, graphs)
     # a warm-up and a capture, or every step; with the rows of its bucket
@@ -62,7 +64,7 @@ def test_same_steps(gpu_device, monkeypatch, dtype, graphs, rows):
 
 
 def test_other_steps(gpu_device, monkeypatch):
-    """Five rows, int4 layers and ranks of a group go through `forward`."""
+    """Five rows in f16, int4 layers and ranks of a group are not forward_rows's."""
     from tgis_amd.models.custom_modeling.flash_llama_modeling import FlashLlamaModel
 
     monkeypatch.setattr(FlashLlamaModel, "forward_rows", lambda *a: pytest.fail("served"))

@@ -746,6 +746,7 @@ int64_t rows_height(int64_t M) { return M <= 2 ? M : 4; }
 // 4096, 11008, 6 layers: 1, 2 rows 656 / 598, 663 / 626; 2560, 6912, 8 layers: 1, 2, 4 rows 489 / 462, 494 / 484, 500 / 622; 3072, 8192: 531 / 507, 543 /
 // 522, 545 / 735.  Beyond two rows of 2048 columns the vector unit and the reads of x from LDS outlast the weights.  Narrower ones, 1, 2, 4 rows: 768, 2048,
 // 12 layers 431 / 285, 445 / 302, 452 / 348; 1024, 2816, 16 layers 531 / 406, 540 / 427, 559 / 495; 1536, 4096, 16 layers 606 / 449, 621 / 470, 640 / 544.
+// Of bf16, steps of three and four rows are those of the launches of more rows, above; they come here where no product may split its sums (TGIS_DEFER_REDUCE=0).
 bool rows_fits(int64_t M, int64_t K, bool norm) {
     return M >= 1 && M <= 4 && K >= 64 && K % 64 == 0 && K <= (norm ? (M <= 2 ? 4096 : 2048) : 12288) && rows_height(M) * K * 4 <= ROWS_LDS;
 }

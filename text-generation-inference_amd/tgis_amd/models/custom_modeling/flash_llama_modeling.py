@@ -211,7 +211,7 @@ class FlashLlamaAttention:
 
     def attend(self, qkv, cu_seqlens_q, layer_id: int, kv: KVArgs, rope=None, frag: bool = False):
         """Attention of q (rotated, or to be rotated by `rope`) over the layer's cache pages (reference :271-295): [T, H D], a native.FragAct where the
-        o_proj GEMM reads that, or with `frag` (a decode step)."""
+        o_proj GEMM reads that, or with `frag`: decode steps, and prompts of up to 64 rows, on the launches of csrc/dense_rows.hip."""
         H, Hkv, D = self.num_heads, self.num_key_value_heads, self.head_size
         k_pool, v_pool = kv.cache.k_pool(layer_id), kv.cache.v_pool(layer_id)
         T = qkv.shape[0]
@@ -369,11 +369,9 @@ class FlashLlamaModel:
             self.max_positions = max(max_s, 2 * self.max_positions, declared, 2048)
         return self.layers[0].self_attn.rotary_emb.tables(dtype, device, self.max_positions)
 
-    def forward_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs, matrix: bool = False):
+    def forward_rows(self, input_ids, position_ids, cu_seqlens_q, max_s, kv: KVArgs):
         """A decode step of a few rows on the launches of csrc/dense_rows.hip: the residual stream (fp32, [rows, hidden]) in front of the final
-        norm.  Five launches a layer; the values are those of `forward` but for the order of the sums.  matrix: `forward_rows16`."""
-        if matrix:
-            return self.forward_rows16(input_ids, position_ids, cu_seqlens_q, max_s, kv)
+        norm.  Five launches a layer; the values are those of `forward` but for the order of the sums."""
         h = native.embedding_scaled_f32(input_ids, self.embed_tokens.weight, 1.0)
         cos, sin = self.rope_tables(self.embed_tokens.weight.dtype, h.device, max_s)
         for layer in self.layers:
@@ -621,19 +619,14 @@ class FlashLlamaForCausalLM:
                 lm_head_indices: Optional[torch.Tensor] = None):
         """position_ids int32 [T]; returns fp32 logits [T or len(lm_head_indices), vocab]."""
         if kv.max_q_len == 1 and not kv.fresh_prefill and inputs_embeds is None and lm_head_indices is None and kv.slots is not None:
-            rows, h = input_ids.shape[0], None
+            rows, norm, head = input_ids.shape[0], self.model.norm, self.lm_head.linear
             step = (input_ids, position_ids, cu_seqlens_q, max_s, kv)
+            if self.rows16_path(rows):
+                return native.dense_rows16_head(self.model.forward_rows16(*step), norm.variance_epsilon, head.prepared)
             if self.rows_path(rows):
-                h = self.model.forward_rows(*step, self.rows16_path(rows))
-            elif self.rows16_path(rows):
-                h = self.model.forward_rows16(*step)
-            norm, head = self.model.norm, self.lm_head.linear
-            if isinstance(h, native.RowsStream):
-                return native.dense_rows16_head(h, norm.variance_epsilon, head.prepared)
-            if h is None and self.model.serves_int4_rows(rows) and DEFER_REDUCE:
+                return native.dense_rows_head(self.model.forward_rows(*step), norm.weight, norm.variance_epsilon, head.prepared)
+            if DEFER_REDUCE and self.model.serves_int4_rows(rows):
                 return self.lm_head(self.model.forward_int4_rows(*step))
-            if h is not None:
-                return native.dense_rows_head(h, norm.weight, norm.variance_epsilon, head.prepared)
         hidden_states = self.model(input_ids, position_ids, cu_seqlens_q, max_s, inputs_embeds, kv)
         if lm_head_indices is not None and not kv.cuts_to_ends(position_ids.shape[0]):
             hidden_states = hidden_states.index_select(0, lm_head_indices)
