@@ -1,4 +1,6 @@
-"""Which launches a decode step of a Llama model takes, where a switch of the environment has a say."""
+"""Which launches a decode step of a Llama model takes."""
+from types import SimpleNamespace
+
 import pytest
 
 
@@ -12,3 +14,13 @@ def test_no_split_sums_where_they_are_off(monkeypatch, splits):
     lm._rows16_path, lm._rows_path = {n: True for n in range(3, 65)}, {n: n <= 4 for n in range(65)}
     assert [lm.rows16_path(n) for n in (3, 5, 64)] == [splits] * 3
     assert lm.rows_path(4) and not lm.rows_path(5)
+
+
+@pytest.mark.parametrize("width,served", [(512, True), (4096, True), (4608, False), (5120, False), (6144, True), (8192, True)])
+def test_int4_widths(width, served):
+    """Widths whose residual units are a little more than the chip has places stay with the other launches."""
+    from tgis_amd.models.custom_modeling import flash_llama_modeling as modeling
+
+    model = object.__new__(modeling.FlashLlamaModel)
+    model.config, model.layers, model.int4_norms, model._int4_rows = SimpleNamespace(hidden_size=width), [], ([], []), {}
+    assert model.serves_int4_rows(1) == served and not model.serves_int4_rows(33)

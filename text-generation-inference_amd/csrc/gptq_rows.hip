@@ -17,10 +17,11 @@
 // and the bound 0.2 and 0.6): 2.7 TB/s of
 // weights, bound by the launch's own ends and, of what is left, by the round trip of a turn's loads (weights of a turn ahead in registers of their own cost 0.7 us: x holds 64).
 // Whole steps at ctx 137, 1, 4, 16 rows: eight layers of 4096, 11008 440 / 419, 471 / 424, 526 / 483; of 2048, 5632 294 / 238, 295 / 239, 308 / 253; of 3072, 8192 349 / 330, 365 /
-// 335, 379 / 349; of 5120, 13824 534 / 564, 574 / 572, 645 / 646; four of 8192, 28672 575 / 528, 577 / 533, 593 / 553.  At 17 - 32 rows a weight feeds two instructions
+// 335, 379 / 349; of 1536, 4096 272 / 227, 279 / 231, 300 / 251; of 1024, 2816 230 / 204, 237 / 207, 246 / 214; of 768, 2048 224 / 190, 230 / 193, 244 / 203; of 512, 1536 209 / 184,
+// 214 / 186, 223 / 192; four of 8192, 28672 572 / 526, 569 / 518, 572 / 535; between 4096 and 6144 columns FlashLlamaModel.serves_int4_rows.  At 17 - 32 rows a weight feeds two instructions
 // and x of a whole k range takes as long as the weights: products as above at 32 rows 12.0 / 11.8, 9.6 / 6.8, 16.4 / 16.1, 13.3 / 14.1.
-// Steps at 24, 32 rows: 4096, 11008 608 / 575, 634 / 617; 2048, 5632 334 / 284, 340 / 299; 3072, 8192 418 / 402, 429 / 421; 5120, 13824, where it is 320 residual units and x
-// leaves the registers of one unit, 782 / 783, 793 / 793: not served.
+// Steps at 24, 32 rows: 4096, 11008 608 / 575, 634 / 617; 3072, 8192 418 / 402, 429 / 421; 2048, 5632 334 / 284, 340 / 299; 1536, 4096 345 / 301, 358 / 320; 1024, 2816 268 / 245, 276 /
+// 258; 768, 2048 280 / 236, 286 / 250; 512, 1536 241 / 214, 247 / 223.  Past 4096 columns x of two blocks leaves the registers of one unit: not served.
 #include <algorithm>
 #include "gptq_gemm_body.h"
 
@@ -511,8 +512,6 @@ int launch_grows(const GRowsArgs& a, hipStream_t st) {
         launch_grows_p<KIND, 1, 2>(a, per, st);
     else if (ds <= 4)
         launch_grows_p<KIND, 1, 4>(a, per, st);
-    else if (ds == 5)
-        launch_grows_k<KIND, 8, 1, 5, 1>(a, per, st);
     else if (KIND == GROWS_SILU)
         launch_grows_k<GROWS_SILU, 16, 1, 4, 1>(a, per, st);
     else

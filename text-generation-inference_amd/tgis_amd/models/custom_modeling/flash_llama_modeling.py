@@ -455,9 +455,14 @@ class FlashLlamaModel:
         self.int4_norms = tuple(native.Int4NormInput.several(inputs) for inputs in norms)
 
     def serves_int4_rows(self, rows: int) -> bool:
+        """Widths between 4096 and 6144 are 257 - 383 residual units, a second round of the chip that is mostly empty, and one unit at a time in front of a norm.  Whole
+        steps, us, the other launches / these (with a form for five double steps a wave, which is gone), at 1, 4, 11, 16 rows: 4608, inner 12288 541 / 546, 548 / 552, 593 / 609,
+        616 / 631; 5120, 12288 530 / 558, 540 / 563, 587 / 625, 609 / 645; 5120, 13824 563 / 564, 573 / 572, 622 / 626, 644 / 646, with eight kv heads 527 / 522, 535 / 524, 553 /
+        548, 554 / 550.  Served: 6144, 16384 537 / 536, 544 / 539, 558 / 563, 561 / 566; 6144, 12288 484 / 470, 489 / 471, 502 / 500, 505 / 501; 6656, 17920 671 / 620, 681 / 628,
+        733 / 687, 763 / 719; 7168, 20480 484 / 441, 487 / 442, 498 / 458, 499 / 460 (4 - 8 layers)."""
         got = self._int4_rows.get(rows)
         if got is None:
-            got = rows <= native.GPTQ_ROWS_MAX_M and self.int4_norms is not None
+            got = rows <= native.GPTQ_ROWS_MAX_M and self.int4_norms is not None and not 4096 < self.config.hidden_size < 6144
             for layer in self.layers if got else ():
                 att, mlp = layer.self_attn, layer.mlp
                 o = att.o_proj.linear
