@@ -396,10 +396,10 @@ static int launch_wide_one(dim3 grid, hipStream_t st, const GemmArgs& a) {
     }
 }
 
+// (more than sixteen rows, plan_wide)
 template <bool OUTF>
 static int launch_wide_pair(dim3 grid, hipStream_t st, const GemmArgs& a) {
     switch (gptq::wide_row_blocks(a.M, a.K, 4, a.S)) {
-        case 1: return launch_wide_rows<4, 2, OUTF, 1, 2>(grid, st, a);
         case 2: return launch_wide_rows<4, 2, OUTF, 2, 2>(grid, st, a);
         case 3: return launch_wide_rows<4, 2, OUTF, 3, 2>(grid, st, a);
         default: return launch_wide_rows<4, 2, OUTF, 4, 2>(grid, st, a);
@@ -553,7 +553,7 @@ static int check_gemm_args(const void* x, int64_t ldx, const void* prepared, int
     return TGIS_OK;
 }
 
-// the fragment-order kernel's plan in the GemmPlan that launch_gptq takes (TN = column tiles per wave, S = k splits)
+// the fragment-order kernel's plan in the GemmPlan that launch_gptq takes (TN = column tiles per block, S = k splits)
 static GemmPlan wide_plan_as_gemm_plan(int64_t K, int64_t N, int act, int64_t M, bool finished = false) {
     const gptq::WidePlan w = gptq::plan_wide(K, N, act, M, finished);
     return {0, w.S, gptq::WIDE_WK, w.CT, 1};

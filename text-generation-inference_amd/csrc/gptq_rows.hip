@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64 * W) void gptq_rows_kernel(GRowsArgs a, int unit
     __shared__ float part[W][16 * RB];
     constexpr int FW = P * RB <= 4 ? 4 : 8;  // a turn's outputs are finished by FW waves, a unit's block of rows each
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int steps = a.K >> 7, mine = (steps - w + W - 1) / W;  // of 128 k: w, w + 8, ..
+    const int steps = a.K >> 7, mine = (steps - w + W - 1) / W;  // of 128 k: w, w + W, ..
     const int m = lane & 15, kq = lane >> 4;
     const int fp = w % FW / RB, fb = w % RB, frow = fb * 16 + m;  // the unit of a turn and the row that this lane finishes
     const int u0 = blockIdx.x * per, n = min(per, units - u0);
@@ -512,10 +512,8 @@ int launch_grows(const GRowsArgs& a, hipStream_t st) {
         launch_grows_p<KIND, 1, 2>(a, per, st);
     else if (ds <= 4)
         launch_grows_p<KIND, 1, 4>(a, per, st);
-    else if (KIND == GROWS_SILU)
-        launch_grows_k<GROWS_SILU, 16, 1, 4, 1>(a, per, st);
     else
-        launch_grows_k<KIND, 8, 1, 8, 1>(a, per, st);
+        launch_grows_k<KIND, KIND == GROWS_SILU ? 16 : 8, 1, KIND == GROWS_SILU ? 4 : 8, 1>(a, per, st);
     TGIS_CHECK_LAUNCH();
     return TGIS_OK;
 }

@@ -57,7 +57,7 @@ static inline bool wide_serves(int64_t M, int64_t K, int64_t N, int64_t groups, 
 static inline WidePlan plan_wide(int64_t K, int64_t N, int act, int64_t M = 32, bool finished = false) {
     if (const char* ov = getenv("TGIS_GPTQ_WIDE_PLAN")) {  // tuning hook: "CT,S"
         int ct = 0, sp = 0;
-        if (sscanf(ov, "%d,%d", &ct, &sp) == 2 && ct >= 1 && (ct <= 4 || (ct == 8 && act == 2)) && sp >= 1 && (sp == 1 || (act != 2 && act != 3)))
+        if (sscanf(ov, "%d,%d", &ct, &sp) == 2 && ct >= 1 && (ct <= 4 || (ct == 8 && act == 2 && M > 16)) && sp >= 1 && (sp == 1 || (act != 2 && act != 3)))
             return {ct, sp};
     }
     const int64_t tiles = cdiv64(N, 32), steps = K / 64;
@@ -66,6 +66,8 @@ static inline WidePlan plan_wide(int64_t K, int64_t N, int act, int64_t M = 32, 
     // SiLU * up past one round of four-tile blocks (one a CU): pairs of waves on four tiles of one k-part each, eight a block, take in x, in good part, once.  A round of them
     // takes 1.75 times one of four tiles.  us, four / eight tiles at 32, 40, 64 rows: 8192 x 57344 (448 / 224 blocks) 67.9 / 64.2, 81.4 / 76.5, 89.6 / 86.5; 8192 x 36864 (288 / 144)
     // 55.2 / 51.9, 68.7 / 62.0, 74.2 / 69.0; 5120 x 40960 (320 / 160) 38.4 / 33.4, 48.0 / 41.9, 51.7 / 46.3; at 16 rows there 31.0 / 32.0.
+    // More rounds, four to two 8192 x 114688 120.2 / 117.5, 148.9 / 136.9, 162.0 / 155.6; 4096 x 114688 69.3 / 62.0, 88.7 / 78.0, 95.3 / 84.5; six to three 8192 x 196608 190 / 185, 233 /
+    // 218, 262 / 254; but three to two 8192 x 98304 98.5 / 106.5, 119 / 130, 136 / 144, five to three 8192 x 163840 160 / 165, 196 / 195, 216 / 225.
     const int64_t rounds4 = cdiv64(cdiv64(tiles, 4), 256), rounds8 = cdiv64(cdiv64(tiles, 8), 256);
     if (act == 2 && M > 16 && 7 * rounds8 < 4 * rounds4) return {8, 1};
     const bool unsplit = act == 2 || act == 3;
