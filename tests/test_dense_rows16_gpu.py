@@ -100,18 +100,21 @@ def test_norm_rope(gpu_device, M, K, H, Hkv, D, bias):
         assert ((got - ref).abs() <= 2 * u * ref.abs() + 8 * u + 5 * u).all()
 
 
-@pytest.mark.parametrize("rows", [3, 5])
-def test_same_steps(gpu_device, monkeypatch, rows):
+# two to four blocks of sixteen rows; the last two split the down projection
+@pytest.mark.parametrize("rows,inner", [(3, 1024), (5, 1024), (17, 1024), (40, 4096), (56, 4096)])
+def test_same_steps(gpu_device, monkeypatch, rows, inner):
+    from tgis_amd import native
     from tgis_amd.models.custom_modeling.flash_llama_modeling import FlashLlamaForCausalLM, FlashLlamaModel
 
     calls, run = [], FlashLlamaModel.forward_rows16
     monkeypatch.setattr(FlashLlamaModel, "forward_rows16", lambda self, ids, *a: calls.append(ids.shape[0]) or run(self, ids, *a))
-    lm, cfg = model(torch.bfloat16)
+    lm, cfg = model(torch.bfloat16, intermediate_size=inner)
     got, pages = decode(lm, cfg.vocab_size, rows, True)
-    assert calls == [4 if rows == 3 else 8] * 2  # a warm-up and a capture, with the rows of the bucket
+    assert calls == [{3: 4, 5: 8, 17: 24, 40: 40, 56: 56}[rows]] * 2  # a warm-up and a capture, with the rows of the bucket
+    assert (native.load_library().tgis_dense_rows16_slab_bytes(rows, inner, cfg.hidden_size, 0) > 0) == (rows >= 40)
     for path in ("rows_path", "rows16_path"):
         monkeypatch.setattr(FlashLlamaForCausalLM, path, lambda self, n: False)
-    lm, _ = model(torch.bfloat16)
+    lm, _ = model(torch.bfloat16, intermediate_size=inner)
     want, pages_want = decode(lm, cfg.vocab_size, rows, True)
     assert len(calls) == 2 and len(got) == len(want) == STEPS + 1 and torch.equal(got[0], want[0])
     # (as with fewer rows: sums in another order, which three layers carry on)
@@ -119,6 +122,30 @@ def test_same_steps(gpu_device, monkeypatch, rows):
     for a, b in zip(got[1:] + pages, want[1:] + pages_want):
         a, b = a.double(), b.double()
         assert a.shape == b.shape and float((a - b).norm() / b.norm()) < 4 * step
+
+
+# (query tokens, keys) of each sequence: prompts of few and of many query tokens, some behind a prefix, up to two blocks of rows; decode steps, whole and behind key splits
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,Hkv,D", [(32, 4, 64), (8, 8, 128), (16, 1, 128), (6, 2, 64)])
+@pytest.mark.parametrize("runs", [[(3, 3), (1, 40), (2, 2)], [(20, 20), (7, 100), (1, 1), (36, 36)], [(64, 64)], [(1, 700)] * 3, [(1, 5 + 9 * i) for i in range(40)]])
+def test_attention_in_fragment_order(gpu_device, dtype, H, Hkv, D, runs):
+    """The attention of the launches around it: the bits that the same launch leaves as rows."""
+    from tgis_amd import native
+
+    g = torch.Generator().manual_seed(len(runs) + D)
+    B, T, longest, ctx = len(runs), sum(n for n, _ in runs), max(n for n, _ in runs), max(k for _, k in runs)
+    per = (ctx + 31) // 32
+    pools = [(torch.randn(B * per + 1, Hkv, 32 * D, generator=g) * 0.5).to(dtype).to(gpu_device) for _ in range(2)]
+    table = torch.randperm(B * per, generator=g).int().view(B, per).to(gpu_device)
+    q = (torch.randn(T, (H + 2) * D, generator=g) * 0.5).to(dtype).to(gpu_device)
+    lens = torch.tensor([k for _, k in runs], dtype=torch.int32, device=gpu_device)
+    cu = torch.tensor([0] + [n for n, _ in runs], device=gpu_device).cumsum(0).int()
+    for splits in sorted({1, native.attn_num_splits(B, Hkv, H, longest, ctx)}):
+        ws = native.Workspace(native.attn_workspace_bytes(B, H, Hkv, D, splits), gpu_device) if splits > 1 else None
+        rows, frag = torch.empty((T, H * D), dtype=dtype, device=gpu_device), native.FragAct.empty(T, H * D, gpu_device, dtype)
+        for out in (rows, frag):
+            native.attn_paged(q, q.stride(0), *pools, table, lens, cu, out, B, H, Hkv, D, longest, ctx, D ** -0.5, splits, ws)
+        assert torch.equal(frag.to_rows(), rows), splits
 
 
 @pytest.mark.parametrize("lens", [[3], [30, 1, 33], [47], [64]])

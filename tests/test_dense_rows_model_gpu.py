@@ -15,7 +15,7 @@ def decode(lm, vocab, rows, graphs):
     from tgis_amd.testing import SyntheticTokenizer, make_batch_pb
 
     lm.use_graphs = graphs
-    lens = [30, 9, 47, 17, 5][:rows]
+    lens = ([30, 9, 47, 17, 5] + [3 + i % 20 for i in range(rows)])[:rows]
     forced = torch.randint(3, vocab, (STEPS, rows), generator=torch.Generator().manual_seed(rows)).cuda()
     taken, run = [], lm._process_new_tokens
     lm._process_new_tokens = lambda batch, out, *a, **k: taken.append(out.clone()) or run(batch, out, *a, **k)
