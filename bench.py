@@ -158,6 +158,17 @@ def cpu_baseline(cfg, quantize, B, ctx, groupsize=128):
                       f"extrapolated x{cfg.num_hidden_layers} layers + measured lm_head/greedy"}
 
 
+def decode_gemm_kernels(lm, quantize, B):
+    """The weight-streaming kernels of a decode step of B rows."""
+    model = getattr(lm.model, "model", None)
+    if quantize == "gptq":
+        rows = hasattr(model, "serves_int4_rows") and model.serves_int4_rows(B)
+        return "gptq_rows_kernel / gptq_rows_residual_kernel / gptq_wide_kernel" if rows else "gptq_wide_kernel / gptq_gemm_kernel"
+    if hasattr(lm.model, "rows16_path") and lm.model.rows16_path(B):
+        return "dense_rows16_kernel / dense_rows16_residual_kernel"
+    return "dense_rows_kernel" if hasattr(lm.model, "rows_path") and lm.model.rows_path(B) else "dense_gemm_kernel"
+
+
 def fused_rope_launches_per_step(lm):
     """Layers whose qkv projection runs the rotary embedding + cache write in its GEMM epilogue at this batch size."""
     n = 0
@@ -921,8 +932,7 @@ def main():
                 g_avg_s = ms_gemm * 1e-3 / n_gemm
                 g_bytes = gemm_bytes_step / max(per_step, 1)
                 g_traffic, g_traffic_src = pmc_gemm_traffic(args.config, B, ctx_mean) if tp == 1 else (None, None)
-                roofline_gemm = {"bound": "hbm", "kernel": ("gptq_wide_kernel / gptq_gemm_kernel" if quantize == "gptq"
-                                                            else "dense_gemm_kernel") + f" ({per_step:.0f} launches per step)",
+                roofline_gemm = {"bound": "hbm", "kernel": decode_gemm_kernels(lm, quantize, B) + f" ({per_step:.0f} launches per step)",
                                  "achieved": round(g_bytes / g_avg_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                  "frac": round(g_bytes / g_avg_s / 1e9 / HBM_PEAK_GBS, 4),
                                  "traffic": g_traffic,

@@ -1263,8 +1263,8 @@ def attn_rotates_q(H: int, Hkv: int, D: int, max_q_len: int) -> bool:
 def attn_paged(q, ld_q: int, k_pool, v_pool, block_tables, ctx_lens, cu_seqlens_q, out, B: int, H: int, Hkv: int,
                D: int, max_q_len: int, max_ctx: int, scale: float, num_splits: int, ws: Optional[Workspace],
                out_cols: Optional[torch.Tensor] = None, rope: Optional[tuple] = None):
-    """q is a (view into a) [T, *] activation whose row stride is ld_q elements; out [T, H*D], or (decode, B <= 32) a
-    FragAct of that shape for the o_proj GEMM, with out_cols (int32, a permutation) with its columns at those places.
+    """q is a (view into a) [T, *] activation whose row stride is ld_q elements; out [T, H*D], or (T <= 64) a
+    FragAct of that shape for the o_proj GEMM, of a decode step with out_cols (int32, a permutation) with its columns at those places.
     rope (where attn_rotates_q): (cos, sin, positions) of a q that is not rotated yet."""
     assert block_tables.dtype == torch.int32 and ctx_lens.dtype == torch.int32 and cu_seqlens_q.dtype == torch.int32
     assert block_tables.is_contiguous()
