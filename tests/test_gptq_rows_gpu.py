@@ -95,9 +95,10 @@ def test_embed(gpu_device, M, shuffled, top):
     assert ((sums - (want * want).view(M, -1, 16).sum(-1)).abs() <= 1e-5 * sums).all()
 
 
-# K: fewer steps of 128 than waves, one more than a round of them, every number of steps that a wave keeps; groups of one and of several steps of 64, and one group
+# K: fewer steps of 128 than waves, one more than a round of them, every number of steps that a wave keeps; groups of one and of several steps of 64, and one group; N: rows that
+# the sum's threads go over more than once
 @pytest.mark.parametrize("M", [1, 11, 16, 17, 32])
-@pytest.mark.parametrize("K,N,groupsize", [(128, 64, 64), (1152, 192, 128), (2176, 2048, 128), (4096, 128, 4096), (6272, 64, 64), (8192, 64, 256), (12288, 64, 128)])
+@pytest.mark.parametrize("K,N,groupsize", [(128, 64, 64), (1152, 192, 128), (2176, 2048, 128), (4096, 128, 4096), (6272, 64, 64), (8192, 64, 256), (12288, 64, 128), (128, 8256, 64)])
 def test_residual(gpu_device, M, K, N, groupsize):
     from tgis_amd import native
 
@@ -171,10 +172,10 @@ def test_norm_rope(gpu_device, M, K, H, Hkv, D, bias):
 
 
 # streams far below one, as in front of a trained model's first layers, and norms of which a few weights are far above the others: an operand that is not yet divided
-# by the row's size holds as many bits of them as the norm's own launch, behind the embedding, a residual product and a split one
-@pytest.mark.parametrize("size,spike", [(1e-4, 50.0), (1e-3, 1000.0), (2e-2, 100.0), (1e-5, 1.0), (100.0, 50.0)])
+# by the row's size holds as many bits of them as the norm's own launch, behind the embedding, a residual product and a split one; growth: what is added, by the stream's size
+@pytest.mark.parametrize("size,spike,growth", [(1e-4, 50.0, 1.0), (1e-3, 1000.0, 1.0), (2e-2, 100.0, 1.0), (1e-5, 1.0, 1.0), (100.0, 50.0, 1.0), (1e-4, 50.0, 1e6), (50.0, 50.0, 1e-5)])
 @pytest.mark.parametrize("M,shuffled", [(11, True), (19, False)])
-def test_small_streams(gpu_device, M, shuffled, size, spike):
+def test_small_streams(gpu_device, M, shuffled, size, spike, growth):
     from tgis_amd import native
 
     g = torch.Generator().manual_seed(M)
@@ -185,8 +186,7 @@ def test_small_streams(gpu_device, M, shuffled, size, spike):
     w[::64] = spike  # (as many as it takes that a row's error is not one rounding's)
     places = torch.randperm(K, generator=g).int() if shuffled else None
     norm = native.Int4NormInput(w.to(gpu_device), None if places is None else places.to(gpu_device))
-    table, x = (torch.randn(M, k, generator=g) * size for k in (K, 1024))
-    table, x = table.half(), x.half()
+    table, x = ((torch.randn(M, k, generator=g) * s).half() for k, s in ((K, size), (1024, size * growth)))
     stream = native.Int4RowsStream.embed(torch.arange(M).to(gpu_device), table.to(gpu_device), norm)
     frag = native.FragAct.from_rows(x.to(gpu_device))
     h, add = table.double(), (x.double() @ dense_o).half().double()
